@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define INFLLMV2_ABI_VERSION 11
+#define INFLLMV2_ABI_VERSION 12
 
 /* ---- library ------------------------------------------------------------------------------ */
 
@@ -133,6 +133,13 @@ int infllmv2_topk_select(void* stream, const void* pooled, int64_t row_stride, i
 int infllmv2_compress_keys(void* stream, const void* k, void* out, const int32_t* cu_seqlens_k,
                            int32_t* cu_seqlens_out, int batch, int max_seqlen_k, int num_heads_k, int head_dim,
                            int64_t k_row_stride, int64_t k_head_stride, int kernel_size, int stride, int first_row);
+
+/* Two sets of the same K in one launch: what two calls of infllmv2_compress_keys with first_row 0 give - the fine keys
+ * (kernel_size_a / stride_a) and the coarse ones of the log-sum-exp, say. */
+int infllmv2_compress_keys_pair(void* stream, const void* k, void* out_a, void* out_b, const int32_t* cu_seqlens_k,
+                                int32_t* cu_seqlens_out_a, int32_t* cu_seqlens_out_b, int batch, int max_seqlen_k,
+                                int num_heads_k, int head_dim, int64_t k_row_stride, int64_t k_head_stride,
+                                int kernel_size_a, int stride_a, int kernel_size_b, int stride_b);
 
 /* The same means for per-sequence key caches, as a batched decode loop keeps them: kcache (batch, capacity, Hk, d)
  * holds new_lens[b] keys of sequence b, out_cache (batch, rows capacity, Hk, d) its compressed keys; strides
@@ -354,6 +361,10 @@ int infllmv2_fwd_kvcache_static(void* stream, const void* q, void* kcache, void*
 int infllmv2_compress_keys_f16(void* stream, const void* k, void* out, const int32_t* cu_seqlens_k,
                                int32_t* cu_seqlens_out, int batch, int max_seqlen_k, int num_heads_k, int head_dim,
                                int64_t k_row_stride, int64_t k_head_stride, int kernel_size, int stride, int first_row);
+int infllmv2_compress_keys_pair_f16(void* stream, const void* k, void* out_a, void* out_b, const int32_t* cu_seqlens_k,
+                                    int32_t* cu_seqlens_out_a, int32_t* cu_seqlens_out_b, int batch, int max_seqlen_k,
+                                    int num_heads_k, int head_dim, int64_t k_row_stride, int64_t k_head_stride,
+                                    int kernel_size_a, int stride_a, int kernel_size_b, int stride_b);
 int infllmv2_compress_keys_cache_f16(void* stream, const void* kcache, void* out_cache, const int32_t* old_lens,
                                      const int32_t* new_lens, int32_t* out_lens, int batch, int max_new_rows,
                                      int num_heads_k, int head_dim, const int64_t* kcache_strides,

@@ -6,8 +6,9 @@
 // windows that fit entirely inside a sequence, mean over the window, result in the input dtype).
 // The mean is an fp32 sum taken in window order divided by kernel_size, rounded once to bf16.
 //
-// HBM-bound and small: K is read once from memory (the overlapping windows hit in cache) and
-// the output is 1/stride of its size.  A thread owns 8 contiguous d values (16 bytes) of one output row.
+// Small: K is read once from memory (the overlap of the windows hits in cache) and the output is 1/stride of its size, so
+// for prompts of a few thousand tokens what counts is latency: how many round trips to memory a workgroup makes, and
+// how many launches there are.
 #include "common.h"
 #include "infllmv2_hip.h"
 
@@ -17,65 +18,106 @@ __device__ __forceinline__ int compressed_rows(int len, int kernel_size, int str
     return len >= kernel_size ? (len - kernel_size) / stride + 1 : 0;
 }
 
-// cu_out[b] = rows of the sequences before b; one thread (batch is small)
-__global__ void compressed_cu_seqlens_kernel(const int* __restrict__ cu_k, int* __restrict__ cu_out, int batch,
-                                             int kernel_size, int stride) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    int acc = 0;
-    cu_out[0] = 0;
-    for (int b = 0; b < batch; ++b) {
-        acc += compressed_rows(cu_k[b + 1] - cu_k[b], kernel_size, stride);
-        cu_out[b + 1] = acc;
-    }
-}
-
+// One set of compressed keys of packed sequences.  (The host passes two where a caller wants two sets of one K.)
 struct CompressParams {
     const elem_bits* k;
     elem_bits* out;
     const int* cu_k;
-    const int* cu_out;
+    int* cu_out;
     int64_t k_row_stride, k_head_stride;
-    int units_per_row;               // num_heads * head_dim / 8
-    int units_per_head;              // head_dim / 8
+    int num_heads, units_per_head;   // 16-byte units of one head (head_dim / 8)
     int kernel_size, stride;
-    int first_row;                   // rows before this one are left alone (appending to a cache of compressed keys)
+    int first_row;                   // rows before this one are left alone (appending to a buffer of compressed keys)
+    int rows_per_wg;                 // output rows of one workgroup
 };
 
 constexpr int kCompressRowsPerWg = 8;
+constexpr int kCompressThreads = 256;
+constexpr int kCompressUnits = 16;           // units of one output row a workgroup works on: 128 elements
+constexpr int kCompressMaxLds = 49152;       // the K rows a workgroup stages: 192 rows of 256 bytes
 
-__global__ __launch_bounds__(256)
-void compress_keys_kernel(const CompressParams p) {
-    const int b = blockIdx.y;
+// A workgroup takes rows_per_wg consecutive output rows of one KV head (128 elements of it).  Their windows are one
+// stretch of (rows - 1) * stride + kernel_size K rows: it goes into LDS with every load in flight at once, and then
+// one thread per two output elements adds its columns in window order.  Summing straight from memory, a window walked
+// row by row is a chain of kernel_size round trips: 26 us for the two sets of 2048 tokens where this takes 5.
+// Windows longer than the LDS holds are added up in several such steps.
+__device__ __forceinline__ void compress_rows_of_head(const CompressParams& p, int wg, uint4* stage) {
+    const int b = blockIdx.y, head = blockIdx.z / ((p.units_per_head + kCompressUnits - 1) / kCompressUnits);
+    const int u0 = (blockIdx.z % ((p.units_per_head + kCompressUnits - 1) / kCompressUnits)) * kCompressUnits;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int k0 = p.cu_k[b];
     const int rows = compressed_rows(p.cu_k[b + 1] - k0, p.kernel_size, p.stride);
-    const int j0 = p.first_row + blockIdx.x * kCompressRowsPerWg;
-    for (int item = threadIdx.x; item < kCompressRowsPerWg * p.units_per_row; item += 256) {
-        const int j = j0 + item / p.units_per_row;
-        if (j >= rows) break;                                  // items are ordered by row
-        const int u = item % p.units_per_row;
-        const int head = u / p.units_per_head, piece = u % p.units_per_head;
-        const elem_bits* src = p.k + (static_cast<int64_t>(k0) + static_cast<int64_t>(j) * p.stride) * p.k_row_stride +
-                               head * p.k_head_stride + piece * 8;
-        float acc[8];
+    // rows of the sequences before this one, added up by every wavefront for itself
+    int before = 0;
+    for (int i = lane; i < b; i += 64) before += compressed_rows(p.cu_k[i + 1] - p.cu_k[i], p.kernel_size, p.stride);
+    if (b > 0) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] = 0.f;
-        for (int i = 0; i < p.kernel_size; ++i) {
-            const uint4 raw = *reinterpret_cast<const uint4*>(src + i * p.k_row_stride);
-            const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
+        for (int off = 32; off; off >>= 1) before += __shfl_xor(before, off);
+    }
+    if (wg == 0 && blockIdx.z == 0 && tid == 0) {
+        p.cu_out[b + 1] = before + rows;
+        if (b == 0) p.cu_out[0] = 0;
+    }
+    const int j0 = p.first_row + wg * p.rows_per_wg;
+    if (j0 >= rows) return;                                    // uniform per workgroup
+    const int nrows = rows - j0 < p.rows_per_wg ? rows - j0 : p.rows_per_wg;
+    const int nu = p.units_per_head - u0 < kCompressUnits ? p.units_per_head - u0 : kCompressUnits;
+    const elem_bits* src = p.k + (static_cast<int64_t>(k0) + static_cast<int64_t>(j0) * p.stride) * p.k_row_stride +
+                           head * p.k_head_stride + u0 * 8;
+    const int span = (nrows - 1) * p.stride + p.kernel_size;   // K rows the windows cover
+    const int step = kCompressMaxLds / (kCompressUnits * 16);  // K rows staged at a time
+    float acc[kCompressRowsPerWg / 4][2];                      // rows wave, wave + 4; elements 2 lane, 2 lane + 1
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                acc[2 * e] += elem_lo_to_f32(w[e]);
-                acc[2 * e + 1] += elem_hi_to_f32(w[e]);
+    for (int r = 0; r < kCompressRowsPerWg / 4; ++r) acc[r][0] = acc[r][1] = 0.f;
+    for (int base = 0; base < span; base += step) {
+        const int staged = span - base < step ? span - base : step;
+        if (base > 0) __syncthreads();
+#pragma unroll 4
+        for (int it = tid; it < staged * kCompressUnits; it += kCompressThreads) {
+            const int i = it / kCompressUnits, u = it % kCompressUnits;
+            if (u < nu) stage[it] = *reinterpret_cast<const uint4*>(src + (base + i) * p.k_row_stride + u * 8);
+        }
+        __syncthreads();
+        const uint32_t* words = reinterpret_cast<const uint32_t*>(stage) + lane;
+#pragma unroll
+        for (int r = 0; r < kCompressRowsPerWg / 4; ++r) {
+            const int row = wave + 4 * r;
+            if (row < nrows) {                                 // uniform per wavefront
+                int lo = row * p.stride - base, hi = lo + p.kernel_size;
+                lo = lo < 0 ? 0 : lo;
+                hi = hi < staged ? hi : staged;
+#pragma unroll 8
+                for (int i = lo; i < hi; ++i) {
+                    const uint32_t w = words[i * kCompressUnits * 4];
+                    acc[r][0] += elem_lo_to_f32(w);
+                    acc[r][1] += elem_hi_to_f32(w);
+                }
             }
         }
-        const float n = static_cast<float>(p.kernel_size);
-        uint4 o;
-        o.x = pack_elem2(acc[0] / n, acc[1] / n);
-        o.y = pack_elem2(acc[2] / n, acc[3] / n);
-        o.z = pack_elem2(acc[4] / n, acc[5] / n);
-        o.w = pack_elem2(acc[6] / n, acc[7] / n);
-        *reinterpret_cast<uint4*>(p.out + (static_cast<int64_t>(p.cu_out[b]) + j) * p.units_per_row * 8 + u * 8) = o;
     }
+    if (lane >= nu * 4) return;
+    const float n = static_cast<float>(p.kernel_size);
+#pragma unroll
+    for (int r = 0; r < kCompressRowsPerWg / 4; ++r) {
+        const int row = wave + 4 * r;
+        if (row < nrows) {
+            elem_bits* dst = p.out + ((static_cast<int64_t>(before) + j0 + row) * p.num_heads + head) * p.units_per_head * 8 + u0 * 8;
+            reinterpret_cast<uint32_t*>(dst)[lane] = pack_elem2(acc[r][0] / n, acc[r][1] / n);
+        }
+    }
+}
+
+__global__ __launch_bounds__(kCompressThreads)
+void compress_keys_kernel(const CompressParams p) {
+    extern __shared__ uint4 stage[];
+    compress_rows_of_head(p, blockIdx.x, stage);
+}
+// two sets of the same K in one launch: the first wgs_a workgroups of a sequence and head belong to set a
+__global__ __launch_bounds__(kCompressThreads)
+void compress_keys_pair_kernel(const CompressParams pa, const CompressParams pb, int wgs_a) {
+    extern __shared__ uint4 stage[];
+    if (static_cast<int>(blockIdx.x) < wgs_a) compress_rows_of_head(pa, blockIdx.x, stage);
+    else compress_rows_of_head(pb, blockIdx.x - wgs_a, stage);
 }
 
 // The same means for per-sequence key caches (decode): sequence b's keys are rows [0, new_lens[b]) of kcache[b]; the
@@ -201,32 +243,75 @@ void compress_keys_cache_append_pair_kernel(const CompressCacheParams pa, const 
 
 using namespace IV2_NS;
 
-extern "C" int IV2_ENTRY(infllmv2_compress_keys)(void* stream, const void* k, void* out, const int32_t* cu_seqlens_k,
-                                      int32_t* cu_seqlens_out, int batch, int max_seqlen_k, int num_heads_k,
-                                      int head_dim, int64_t k_row_stride, int64_t k_head_stride, int kernel_size,
-                                      int stride, int first_row) {
-    IV2_CHECK(batch > 0 && batch <= 65535 && max_seqlen_k >= 0, "compress_keys: bad batch or max_seqlen_k");
-    IV2_CHECK(kernel_size > 0 && stride > 0 && first_row >= 0, "compress_keys: kernel_size and stride must be positive");
-    IV2_CHECK(k && out && cu_seqlens_k && cu_seqlens_out, "compress_keys: null pointer");
-    IV2_CHECK(head_dim > 0 && head_dim % 8 == 0 && num_heads_k > 0, "compress_keys: head_dim must be a multiple of 8");
-    const int units = num_heads_k * head_dim / 8;
+namespace {
+
+// checks and parameters of one set of compressed keys of packed sequences; wgs: workgroups per sequence and head
+int packed_params(const char* who, CompressParams& p, int& wgs, const void* k, void* out, const int32_t* cu_seqlens_k,
+                  int32_t* cu_seqlens_out, int batch, int max_seqlen_k, int num_heads_k, int head_dim,
+                  int64_t k_row_stride, int64_t k_head_stride, int kernel_size, int stride, int first_row) {
+    IV2_CHECK(batch > 0 && batch <= 65535 && max_seqlen_k >= 0, "%s: bad batch or max_seqlen_k", who);
+    IV2_CHECK(kernel_size > 0 && stride > 0 && first_row >= 0, "%s: kernel_size and stride must be positive", who);
+    IV2_CHECK(k && out && cu_seqlens_k && cu_seqlens_out, "%s: null pointer", who);
+    IV2_CHECK(head_dim > 0 && head_dim % 8 == 0 && num_heads_k > 0, "%s: head_dim must be a multiple of 8", who);
+    IV2_CHECK(static_cast<int64_t>(num_heads_k) * ((head_dim + 127) / 128) <= 65535, "%s: too many heads", who);
     IV2_CHECK(reinterpret_cast<uintptr_t>(k) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-              k_row_stride % 8 == 0 && k_head_stride % 8 == 0, "compress_keys: k and out must be 16-byte aligned, strides multiples of 8");
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(compressed_cu_seqlens_kernel, dim3(1), dim3(64), 0, st, cu_seqlens_k, cu_seqlens_out, batch,
-                       kernel_size, stride);
-    IV2_LAUNCH_CHECK();
-    const int max_rows = max_seqlen_k >= kernel_size ? (max_seqlen_k - kernel_size) / stride + 1 : 0;
-    if (max_rows <= first_row) return 0;
-    CompressParams p{};
+              k_row_stride % 8 == 0 && k_head_stride % 8 == 0, "%s: k and out must be 16-byte aligned, strides multiples of 8", who);
+    p = CompressParams{};
     p.k = static_cast<const elem_bits*>(k);
     p.out = static_cast<elem_bits*>(out);
     p.cu_k = cu_seqlens_k; p.cu_out = cu_seqlens_out;
     p.k_row_stride = k_row_stride; p.k_head_stride = k_head_stride;
-    p.units_per_row = units; p.units_per_head = head_dim / 8;
+    p.num_heads = num_heads_k; p.units_per_head = head_dim / 8;
     p.kernel_size = kernel_size; p.stride = stride; p.first_row = first_row;
-    const dim3 grid((max_rows - first_row + kCompressRowsPerWg - 1) / kCompressRowsPerWg, batch);
-    hipLaunchKernelGGL(compress_keys_kernel, grid, dim3(256), 0, st, p);
+    // as many rows as fit the staging buffer together (8 at 32/16, 2 at 128/64), at least one
+    const int lds_rows = kCompressMaxLds / (kCompressUnits * 16);
+    int rows_per_wg = lds_rows > kernel_size ? (lds_rows - kernel_size) / stride + 1 : 1;
+    p.rows_per_wg = rows_per_wg < kCompressRowsPerWg ? rows_per_wg : kCompressRowsPerWg;
+    const int max_rows = max_seqlen_k >= kernel_size ? (max_seqlen_k - kernel_size) / stride + 1 : 0;
+    wgs = max_rows > first_row ? (max_rows - first_row + p.rows_per_wg - 1) / p.rows_per_wg : 1;   // one writes cu_out in any case
+    return 0;
+}
+size_t staging_bytes(const CompressParams& p) {
+    const int64_t rows = static_cast<int64_t>(p.rows_per_wg - 1) * p.stride + p.kernel_size;
+    const int64_t bytes = rows * kCompressUnits * 16;
+    return static_cast<size_t>(bytes < kCompressMaxLds ? bytes : kCompressMaxLds);
+}
+unsigned head_parts(const CompressParams& p) {
+    return static_cast<unsigned>(p.num_heads * ((p.units_per_head + kCompressUnits - 1) / kCompressUnits));
+}
+
+}  // namespace
+
+extern "C" int IV2_ENTRY(infllmv2_compress_keys)(void* stream, const void* k, void* out, const int32_t* cu_seqlens_k,
+                                      int32_t* cu_seqlens_out, int batch, int max_seqlen_k, int num_heads_k,
+                                      int head_dim, int64_t k_row_stride, int64_t k_head_stride, int kernel_size,
+                                      int stride, int first_row) {
+    CompressParams p;
+    int wgs;
+    if (int rc = packed_params("compress_keys", p, wgs, k, out, cu_seqlens_k, cu_seqlens_out, batch, max_seqlen_k, num_heads_k,
+                               head_dim, k_row_stride, k_head_stride, kernel_size, stride, first_row))
+        return rc;
+    hipLaunchKernelGGL(compress_keys_kernel, dim3(wgs, batch, head_parts(p)), dim3(kCompressThreads), staging_bytes(p),
+                       static_cast<hipStream_t>(stream), p);
+    IV2_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int IV2_ENTRY(infllmv2_compress_keys_pair)(void* stream, const void* k, void* out_a, void* out_b, const int32_t* cu_seqlens_k,
+                                           int32_t* cu_seqlens_out_a, int32_t* cu_seqlens_out_b, int batch, int max_seqlen_k,
+                                           int num_heads_k, int head_dim, int64_t k_row_stride, int64_t k_head_stride,
+                                           int kernel_size_a, int stride_a, int kernel_size_b, int stride_b) {
+    CompressParams pa, pb;
+    int wgs_a, wgs_b;
+    if (int rc = packed_params("compress_keys_pair", pa, wgs_a, k, out_a, cu_seqlens_k, cu_seqlens_out_a, batch, max_seqlen_k,
+                               num_heads_k, head_dim, k_row_stride, k_head_stride, kernel_size_a, stride_a, 0))
+        return rc;
+    if (int rc = packed_params("compress_keys_pair", pb, wgs_b, k, out_b, cu_seqlens_k, cu_seqlens_out_b, batch, max_seqlen_k,
+                               num_heads_k, head_dim, k_row_stride, k_head_stride, kernel_size_b, stride_b, 0))
+        return rc;
+    const size_t lds = staging_bytes(pa) > staging_bytes(pb) ? staging_bytes(pa) : staging_bytes(pb);
+    hipLaunchKernelGGL(compress_keys_pair_kernel, dim3(wgs_a + wgs_b, batch, head_parts(pa)), dim3(kCompressThreads), lds,
+                       static_cast<hipStream_t>(stream), pa, pb, wgs_a);
     IV2_LAUNCH_CHECK();
     return 0;
 }

@@ -43,6 +43,13 @@ def topk_blocks(pooled: torch.Tensor, k: int, *, return_mask: bool = False, by_i
     return (out, mask) if return_mask else out
 
 
+def _compressed_rows_bound(batch: int, total_k: int, max_seqlen_k: int, kernel_size: int, stride: int) -> int:
+    """Rows to allocate for compressed keys: their number for one sequence, an upper bound for a packed batch."""
+    if batch == 1:
+        return (max_seqlen_k - kernel_size) // stride + 1 if max_seqlen_k >= kernel_size else 0
+    return total_k // stride + 1
+
+
 def compress_keys(k: torch.Tensor, cu_seqlens_k: torch.Tensor, max_seqlen_k: int, kernel_size: int, stride: int,
                   out: torch.Tensor | None = None, first_row: int = 0):
     """Mean of ``k`` ``(total_k, nheads_k, d)`` bf16 over the full windows ``[stride*j, stride*j + kernel_size)`` of
@@ -63,10 +70,7 @@ def compress_keys(k: torch.Tensor, cu_seqlens_k: torch.Tensor, max_seqlen_k: int
         raise RuntimeError("cu_seqlens_k must be a contiguous int32 tensor")
     batch = cu_seqlens_k.numel() - 1
     total_k, Hk, d = k.shape
-    if batch == 1:
-        rows = (max_seqlen_k - kernel_size) // stride + 1 if max_seqlen_k >= kernel_size else 0
-    else:
-        rows = total_k // stride + 1
+    rows = _compressed_rows_bound(batch, total_k, max_seqlen_k, kernel_size, stride)
     if out is None:
         backing = torch.empty((max(rows, 1), Hk, d), dtype=k.dtype, device=k.device)      # never a null pointer
         out = backing[:rows]
@@ -79,6 +83,30 @@ def compress_keys(k: torch.Tensor, cu_seqlens_k: torch.Tensor, max_seqlen_k: int
         _lib.call_for(k.dtype, "infllmv2_compress_keys", stream_ptr(k.device), k.data_ptr(), backing.data_ptr(), cu_seqlens_k.data_ptr(),
                   cu_out.data_ptr(), batch, max_seqlen_k, Hk, d, k.stride(0), k.stride(1), kernel_size, stride, first_row)
     return out, cu_out
+
+
+def compress_keys_pair(k: torch.Tensor, cu_seqlens_k: torch.Tensor, max_seqlen_k: int, fine, coarse):
+    """Two :func:`compress_keys` calls on the same keys in one launch; ``fine`` and ``coarse`` are ``(kernel_size, stride)``.
+    Returns ``(k_fine, cu_fine, k_coarse, cu_coarse)``."""
+    require_gpu(k, "k")
+    if k.dtype not in (torch.float16, torch.bfloat16):
+        raise RuntimeError("FlashAttention only support fp16 and bf16 data type")
+    if k.dim() != 3 or k.stride(-1) != 1:
+        raise RuntimeError("k must have shape (total_k, num_heads_k, head_size) with a contiguous last dimension")
+    if cu_seqlens_k.dtype != torch.int32 or not cu_seqlens_k.is_contiguous():
+        raise RuntimeError("cu_seqlens_k must be a contiguous int32 tensor")
+    batch = cu_seqlens_k.numel() - 1
+    total_k, Hk, d = k.shape
+    backing, result = [], []
+    for ks, st in (fine, coarse):
+        rows = _compressed_rows_bound(batch, total_k, max_seqlen_k, ks, st)
+        backing.append(torch.empty((max(rows, 1), Hk, d), dtype=k.dtype, device=k.device))      # never a null pointer
+        result += [backing[-1][:rows], torch.empty(batch + 1, dtype=torch.int32, device=k.device)]
+    with torch.cuda.device(k.device):
+        _lib.call_for(k.dtype, "infllmv2_compress_keys_pair", stream_ptr(k.device), k.data_ptr(), backing[0].data_ptr(),
+                      backing[1].data_ptr(), cu_seqlens_k.data_ptr(), result[1].data_ptr(), result[3].data_ptr(), batch,
+                      max_seqlen_k, Hk, d, k.stride(0), k.stride(1), *fine, *coarse)
+    return tuple(result)
 
 
 def compress_keys_cache(k_cache: torch.Tensor, new_lens: torch.Tensor, kernel_size: int, stride: int, out: torch.Tensor,
@@ -176,11 +204,11 @@ def select_blocks(q: torch.Tensor, k: torch.Tensor, cu_seqlens_q: torch.Tensor, 
         if softmax_scale is None:
             softmax_scale = q.shape[-1] ** (-0.5)
         q, k = pad_head_dim(q, k)                              # the mean of zero columns is zero
-    kf, cu_f = compress_keys(k, cu_seqlens_k, max_seqlen_k, kernel_size, stride)
     if exact_lse:
+        kf, cu_f = compress_keys(k, cu_seqlens_k, max_seqlen_k, kernel_size, stride)
         kc, cu_c = kf, cu_f
     else:
-        kc, cu_c = compress_keys(k, cu_seqlens_k, max_seqlen_k, 4 * kernel_size, 4 * stride)
+        kf, cu_f, kc, cu_c = compress_keys_pair(k, cu_seqlens_k, max_seqlen_k, (kernel_size, stride), (4 * kernel_size, 4 * stride))
     max_lk = (max_seqlen_k - kernel_size) // stride + 1 if max_seqlen_k >= kernel_size else 0
     pooled = infllmv2_attn_stage1_pooled(q, kf, kc, cu_seqlens_q, cu_f, cu_c, max_seqlen_q, max_lk, local_blocks,
                                          init_blocks, cache_lens=cache_lens, max_cache_len=max_cache_len,
