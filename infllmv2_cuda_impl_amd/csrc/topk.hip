@@ -1,4 +1,5 @@
-// Deterministic top-k over rows of 16-bit scores (gfx950), one wavefront per row, with the uint64 block mask of
+// Deterministic top-k over rows of 16-bit scores (gfx950), one wavefront per row (one workgroup where there are few
+// rows), with the uint64 block mask of
 // the selection emitted by the same wavefront.
 //
 // Order contract: the first k entries of a stable descending sort of the row — larger value
@@ -305,6 +306,139 @@ void topk_rows_kernel(const TopkParams p) {
     }
 }
 
+// The same selection with a whole workgroup per row, for the few rows of a decode step: there a wavefront per row leaves
+// the chip idle and the kernel takes as long as one wavefront needs for one row (13 us at 2048 columns and 128 rows, 6.6 here; 8.0 and 5.9 at 1024).  Column
+// 512 e + 64 wave + lane sits in register e, so a wavefront's ballot is mask word 8 e + wave.  Two bits of the
+// threshold per round: three counts per wavefront, added up in LDS (a slot of its own per round: one barrier).
+constexpr int kTopkRowWaves = 8;
+
+template <int kItems>
+__global__ __launch_bounds__(kTopkRowWaves * 64)
+void topk_wide_kernel(const TopkParams p) {
+    extern __shared__ uint32_t sel[];                          // k survivors
+    __shared__ int counts[8][4];                               // per round: columns at or above each candidate
+    __shared__ uint32_t word_counts[kItems * kTopkRowWaves];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t row = blockIdx.x;
+    const int n = p.n, k = p.k;
+    const int k_sel = k < n ? k : n;
+    const uint16_t* src = p.x + row * p.row_stride;
+    uint32_t key[kItems];
+#pragma unroll
+    for (int e = 0; e < kItems; ++e) {
+        const int col = e * kTopkRowWaves * 64 + tid;
+        key[e] = col < n ? src[col] : 0;
+    }
+    if (tid < 32) counts[tid >> 2][tid & 3] = 0;
+#pragma unroll
+    for (int e = 0; e < kItems; ++e) key[e] = e * kTopkRowWaves * 64 + tid < n ? sortable16(key[e]) : 0u;
+    __syncthreads();
+    auto count_ge = [&](uint32_t cand) -> int {
+        int cnt = 0;
+#pragma unroll
+        for (int e = 0; e < kItems; ++e) cnt += __builtin_popcountll(__builtin_amdgcn_ballot_w64(key[e] >= cand));
+        return cnt;
+    };
+    // thr = largest candidate with count(key >= thr) >= k_sel (0 always satisfies it: every register counts)
+    uint32_t thr = 0;
+    for (int round = 0; round < 8; ++round) {
+        const uint32_t unit = 1u << (14 - 2 * round);
+        const int c1 = count_ge(thr + unit), c2 = count_ge(thr + 2 * unit), c3 = count_ge(thr + 3 * unit);
+        if (lane == 0) {
+            atomicAdd(&counts[round][0], c1);
+            atomicAdd(&counts[round][1], c2);
+            atomicAdd(&counts[round][2], c3);
+        }
+        __syncthreads();
+        const int s1 = counts[round][0], s2 = counts[round][1], s3 = counts[round][2];
+        thr += (s3 >= k_sel ? 3u : (s2 >= k_sel ? 2u : (s1 >= k_sel ? 1u : 0u))) * unit;
+    }
+    if (p.drop_neg_inf && thr <= p.neg_inf_key) thr = p.neg_inf_key;                 // scores above -inf only: none of those equal to thr
+    const bool no_equal = p.drop_neg_inf && thr == p.neg_inf_key;
+    if (k_sel == 0) thr = 0xffffffffu;
+    // per mask word: how many columns lie above the threshold (low half) and how many equal it (high half)
+#pragma unroll
+    for (int e = 0; e < kItems; ++e) {
+        const uint64_t above = __builtin_amdgcn_ballot_w64(key[e] > thr), equal = __builtin_amdgcn_ballot_w64(key[e] == thr);
+        if (lane == 0)
+            word_counts[e * kTopkRowWaves + wave] = __builtin_popcountll(above) | (no_equal ? 0 : __builtin_popcountll(equal) << 16);
+    }
+    __syncthreads();
+    // every wavefront scans the counts of all words for itself: lane w holds the columns of words 0 .. w (64 words at a time)
+    constexpr int kWords = kItems * kTopkRowWaves, kScans = (kWords + 63) / 64;
+    uint32_t upto[kScans], all = 0;
+#pragma unroll
+    for (int c = 0; c < kScans; ++c) {
+        uint32_t v = c * 64 + lane < kWords ? word_counts[c * 64 + lane] : 0u;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = __shfl_up(v, off);
+            v += lane >= off ? o : 0u;
+        }
+        upto[c] = v + all;
+        all = __builtin_amdgcn_readlane(upto[c], 63);
+    }
+    const int total_above = static_cast<int>(all & 0xffffu), total_equal = static_cast<int>(all >> 16);
+    const int ties = k_sel - total_above;                      // columns equal to the threshold that are taken, lowest first
+    const int taken = total_above + (total_equal < ties ? total_equal : ties);
+    uint64_t* mask_row = p.out_mask ? p.out_mask + row * p.n64 : nullptr;
+#pragma unroll
+    for (int e = 0; e < kItems; ++e) {
+        const int word = e * kTopkRowWaves + wave;
+        const uint32_t before = word == 0 ? 0u : __builtin_amdgcn_readlane(upto[(word - 1) >> 6], (word - 1) & 63);
+        const int above = static_cast<int>(before & 0xffffu), equal = static_cast<int>(before >> 16);
+        const uint64_t eq_mask = __builtin_amdgcn_ballot_w64(key[e] == thr);
+        const bool take = key[e] > thr || (!no_equal && key[e] == thr && equal + lanes_below(eq_mask, 0) < ties);
+        const uint64_t take_mask = __builtin_amdgcn_ballot_w64(take);
+        if (mask_row && lane == 0 && word < p.n64) mask_row[word] = take_mask;
+        if (take) {
+            const int col = word * 64 + lane;
+            const int slot = lanes_below(take_mask, above + (equal < ties ? equal : ties));
+            sel[slot] = p.by_index ? static_cast<uint32_t>(col) : (key[e] << 16) | (0xffffu - static_cast<uint32_t>(col));
+        }
+    }
+    if (mask_row)
+        for (int w = kItems * kTopkRowWaves + tid; w < p.n64; w += kTopkRowWaves * 64) mask_row[w] = 0ull;
+    __syncthreads();
+    int32_t* dst = p.out_idx + row * p.out_stride;
+    uint16_t* dst_val = p.out_val ? p.out_val + row * p.out_stride : nullptr;
+    if (!p.by_index && taken <= 64) {
+        if (wave == 0) {
+            const uint32_t mine = bitonic_sort_desc<64>(lane < taken ? sel[lane] : 0u);
+            if (lane < taken) {
+                const uint32_t col = 0xffffu - (mine & 0xffffu);
+                dst[lane] = static_cast<int32_t>(col);
+                if (dst_val) dst_val[lane] = src[col];
+            }
+        }
+    } else {
+        for (int i = tid; i < taken; i += kTopkRowWaves * 64) {
+            const uint32_t mine = sel[i];
+            int at = i;
+            if (!p.by_index) {                                 // rank among the survivors
+                at = 0;
+                for (int j = 0; j < taken; ++j) at += sel[j] > mine;
+            }
+            const uint32_t col = p.by_index ? mine : 0xffffu - (mine & 0xffffu);
+            dst[at] = static_cast<int32_t>(col);
+            if (dst_val) dst_val[at] = src[col];
+        }
+    }
+    for (int i = taken + tid; i < p.out_stride; i += kTopkRowWaves * 64) {
+        dst[i] = -1;
+        if (dst_val) dst_val[i] = 0;
+    }
+}
+
+template <int kItems>
+static int launch_topk_wide(void* stream, const TopkParams& p) {
+    hipLaunchKernelGGL(topk_wide_kernel<kItems>, dim3(static_cast<unsigned>(p.rows)), dim3(kTopkRowWaves * 64),
+                       sizeof(uint32_t) * (p.k > 0 ? p.k : 1), static_cast<hipStream_t>(stream), p);
+    IV2_LAUNCH_CHECK();
+    return 0;
+}
+
 template <int kItems>
 static int launch_topk(void* stream, const TopkParams& p) {
     const int64_t waves = (p.rows + p.rows_per_wave - 1) / p.rows_per_wave;
@@ -328,6 +462,8 @@ static int launch_topk(void* stream, const TopkParams& p) {
     return 0;
 }
 
+constexpr int kTopkWideRows = 512;
+
 static int topk_dispatch(void* stream, const uint16_t* x, int64_t row_stride, int32_t* idx, uint16_t* val,
                          uint64_t* mask, int n64, int out_stride, int64_t rows, int n, int k, int by_index,
                          int drop_neg_inf, int dtype) {
@@ -342,6 +478,14 @@ static int topk_dispatch(void* stream, const uint16_t* x, int64_t row_stride, in
     p.x = x; p.row_stride = row_stride; p.out_idx = idx; p.out_val = val; p.out_mask = mask;
     p.out_stride = out_stride; p.n64 = n64; p.rows = rows; p.n = n; p.k = k;
     p.by_index = by_index; p.drop_neg_inf = drop_neg_inf; p.neg_inf_key = dtype == 0 ? kKeyNegInfFp16 : kKeyNegInfBf16;
+    // few rows (two workgroups per CU at most): a workgroup per row.  Up to 512 columns one wavefront holds the row in
+    // eight registers and is done before a workgroup has met at its barriers (4.4 against 5.5 us at 512 columns).
+    if (rows <= kTopkWideRows && n > 512) {
+        if (n <= 1024) return launch_topk_wide<2>(stream, p);
+        if (n <= 2048) return launch_topk_wide<4>(stream, p);
+        if (n <= 4096) return launch_topk_wide<8>(stream, p);
+        return launch_topk_wide<16>(stream, p);
+    }
     // consecutive rows per wavefront (each search starts from the previous row's threshold), but never so many
     // that fewer than ~32 wavefronts per CU of a 256-CU device remain
     int rpw = 16;
