@@ -225,6 +225,26 @@ int infllmv2_stage1_decode(void* stream, const void* q, const void* k, const voi
                            int out_len, int kernel_size, int stride, int padding, int block_size, int local_blocks,
                            int init_blocks);
 
+/* Everything of a batched decode step in front of its top-k, in two launches (no counterpart in the reference, whose
+ * callers do it in Python): the new token's K/V rows (k_new, v_new: strides {batch, head}) are written to the caches
+ * (batch, capacity, Hk, 128; strides {batch, row, head}) at row lens[b] (host_len for every sequence when lens is null);
+ * where the token completes a window its compressed key is appended to fine_cache / coarse_cache (fine_rows, coarse_rows
+ * rows per sequence) as infllmv2_compress_keys_cache does with max_new_rows 1; new_lens (or null), fine_lens and
+ * coarse_lens (batch each) receive the lengths afterwards; and pooled (batch, Hk, out_len), dense, receives what
+ * infllmv2_stage1_decode gives for the query (batch; strides {batch, head-in-group, kv-head}) on those caches, non-causal, the
+ * query at position lens[b].  pooled null: no scores (q and workspace unused).  max_len bounds every length after the step;
+ * workspace: infllmv2_stage1_decode_workspace_bytes for the compressed rows that max_len tokens have. */
+int infllmv2_decode_step_scores(void* stream, const void* q, const void* k_new, const void* v_new, void* kcache,
+                                void* vcache, void* fine_cache, void* coarse_cache, const int32_t* lens, int host_len,
+                                int32_t* new_lens, int32_t* fine_lens, int32_t* coarse_lens, void* pooled,
+                                void* workspace, size_t workspace_bytes, int batch, int num_heads, int num_heads_k,
+                                int head_dim, int capacity, int fine_rows, int coarse_rows, int max_len,
+                                const int64_t* q_strides, const int64_t* knew_strides, const int64_t* vnew_strides,
+                                const int64_t* kcache_strides, const int64_t* vcache_strides,
+                                const int64_t* fine_strides, const int64_t* coarse_strides, int kernel_size_f,
+                                int stride_f, int kernel_size_c, int stride_c, float softmax_scale, int out_len,
+                                int local_blocks, int init_blocks);
+
 /* ---- Stage 2: block-sparse attention -------------------------------------------------------- */
 
 /* Scratch needed by infllmv2_varlen_fwd / _bwd for the fragment-major K/V block images. */
@@ -294,7 +314,7 @@ int infllmv2_varlen_bwd(void* stream, const void* dout, const void* q, const voi
 /* The split count infllmv2_fwd_kvcache will use: `requested` if > 0 (capped at 64), else a heuristic
  * (replaces num_splits_heuristic, csrc/flash_attn/flash_api.cpp:261-295). */
 int infllmv2_fwd_kvcache_num_splits(int batch, int num_heads_k, int requested);
-/* fp32 partial outputs and LSEs of the splits, plus room for the query turned by the rotary embedding. */
+/* fp32 partial outputs and LSEs of the splits. */
 size_t infllmv2_fwd_kvcache_workspace_bytes(int batch, int num_heads_k, int num_splits);
 
 /* csrc/entry.cu:18,214 `fwd_kvcache` = mha_fwd_kvcache (csrc/flash_attn/flash_api.cpp:1549-1843; kernels
@@ -328,9 +348,22 @@ int infllmv2_fwd_kvcache(void* stream, const void* q, void* kcache, void* vcache
                          int64_t block_table_batch_stride, int page_block_size, const void* rotary_cos,
                          const void* rotary_sin, int rotary_dim, int rotary_interleaved);
 
+/* infllmv2_fwd_kvcache with the selection as the index list itself, topk_idx (batch, Hk, k_idx) int32 (blocks in any
+ * order, -1 = unused slot, repeats count once): no packing launch. */
+int infllmv2_fwd_kvcache_topk(void* stream, const void* q, void* kcache, void* vcache, const void* k_new,
+                              const void* v_new, const int32_t* cache_seqlens, void* out, float* softmax_lse,
+                              const int32_t* topk_idx, int k_idx, void* workspace, size_t workspace_bytes, int batch,
+                              int seqlen_q, int num_heads, int num_heads_k, int head_dim, int cache_capacity,
+                              int seqlen_new, const int64_t* q_strides, const int64_t* kcache_strides,
+                              const int64_t* vcache_strides, const int64_t* knew_strides, const int64_t* vnew_strides,
+                              const int64_t* o_strides, int num_splits, float softmax_scale,
+                              const int32_t* cache_batch_idx, const int32_t* cache_leftpad, const int32_t* block_table,
+                              int64_t block_table_batch_stride, int page_block_size, const void* rotary_cos,
+                              const void* rotary_sin, int rotary_dim, int rotary_interleaved);
+
 /* No counterpart in the reference.  infllmv2_fwd_kvcache for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): the same kernels and arguments, without
- * the workspace pair.  The split partials and the turned query go to a buffer of INFLLMV2_STATIC_SCRATCH_BYTES that is
+ * the workspace pair.  The split partials go to a buffer of INFLLMV2_STATIC_SCRATCH_BYTES that is
  * part of the library's device code (one copy per GPU, held until the process ends); the call allocates and frees
  * nothing.  Sizes with infllmv2_fwd_kvcache_workspace_bytes(batch, num_heads_k, num_splits) above that limit are
  * rejected.  All calls on one GPU share the buffer: calls that overlap on one GPU (different streams or threads) race;
@@ -392,6 +425,16 @@ int infllmv2_varlen_fwd_stage1_pooled_f16(void* stream, const void* q, const voi
                                           const int64_t* k_strides, const int64_t* v_strides, int out_len,
                                           float softmax_scale, int is_causal, int kernel_size, int stride, int padding,
                                           int block_size, int local_blocks, int init_blocks);
+int infllmv2_decode_step_scores_f16(void* stream, const void* q, const void* k_new, const void* v_new, void* kcache,
+                                void* vcache, void* fine_cache, void* coarse_cache, const int32_t* lens, int host_len,
+                                int32_t* new_lens, int32_t* fine_lens, int32_t* coarse_lens, void* pooled,
+                                void* workspace, size_t workspace_bytes, int batch, int num_heads, int num_heads_k,
+                                int head_dim, int capacity, int fine_rows, int coarse_rows, int max_len,
+                                const int64_t* q_strides, const int64_t* knew_strides, const int64_t* vnew_strides,
+                                const int64_t* kcache_strides, const int64_t* vcache_strides,
+                                const int64_t* fine_strides, const int64_t* coarse_strides, int kernel_size_f,
+                                int stride_f, int kernel_size_c, int stride_c, float softmax_scale, int out_len,
+                                int local_blocks, int init_blocks);
 int infllmv2_stage1_decode_f16(void* stream, const void* q, const void* k, const void* v, void* out,
                                const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, const int32_t* k_lens,
                                const int32_t* cu_seqlens_v, const int32_t* v_lens, void* workspace,
@@ -419,6 +462,16 @@ int infllmv2_varlen_bwd_f16(void* stream, const void* dout, const void* q, const
                             const int64_t* do_strides, const int64_t* dq_strides, const int64_t* dk_strides,
                             const int64_t* dv_strides, const int64_t* lse_strides, int n_uint64_per_row,
                             float softmax_scale, int is_causal, int deterministic);
+int infllmv2_fwd_kvcache_topk_f16(void* stream, const void* q, void* kcache, void* vcache, const void* k_new,
+                                  const void* v_new, const int32_t* cache_seqlens, void* out, float* softmax_lse,
+                                  const int32_t* topk_idx, int k_idx, void* workspace, size_t workspace_bytes, int batch,
+                                  int seqlen_q, int num_heads, int num_heads_k, int head_dim, int cache_capacity,
+                                  int seqlen_new, const int64_t* q_strides, const int64_t* kcache_strides,
+                                  const int64_t* vcache_strides, const int64_t* knew_strides, const int64_t* vnew_strides,
+                                  const int64_t* o_strides, int num_splits, float softmax_scale,
+                                  const int32_t* cache_batch_idx, const int32_t* cache_leftpad, const int32_t* block_table,
+                                  int64_t block_table_batch_stride, int page_block_size, const void* rotary_cos,
+                                  const void* rotary_sin, int rotary_dim, int rotary_interleaved);
 int infllmv2_fwd_kvcache_f16(void* stream, const void* q, void* kcache, void* vcache, const void* k_new,
                              const void* v_new, const int32_t* cache_seqlens, void* out, float* softmax_lse,
                              const uint64_t* blockmask, void* workspace, size_t workspace_bytes, int batch,

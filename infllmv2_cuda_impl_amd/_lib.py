@@ -36,17 +36,19 @@ SIGNATURES = {
     "infllmv2_varlen_fwd_stage1": [_p, _p, _p, _p, _p, _p, _p, _p, _i, _i64, _i, _i, _i, _i, _i, _p, _p, _p, _i64, _i64, _f, _i],
     "infllmv2_varlen_fwd_stage1_pooled": [_p] * 9 + [_i, _i, _i64, _i, _i, _i, _i, _i, _p, _p, _p, _i, _f] + [_i] * 7,
     "infllmv2_stage1_decode": [_p] * 11 + [_sz] + [_i] * 6 + [_p] * 3 + [_i64, _i64, _f, _i, _i, _p] + [_i] * 8,
+    "infllmv2_decode_step_scores": [_p] * 9 + [_i] + [_p] * 5 + [_sz] + [_i] * 8 + [_p] * 7 + [_i] * 4 + [_f, _i, _i, _i],
     "infllmv2_varlen_fwd": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _i, _i, _i64, _i64, _i, _i, _i, _i, _i,
                             _p, _p, _p, _p, _p, _i, _f, _i],
     "infllmv2_varlen_bwd": [_p] * 14 + [_sz, _i, _i64, _i64, _i, _i, _i, _i, _i] + [_p] * 9 + [_i, _f, _i, _i],
     "infllmv2_fwd_kvcache": [_p] * 11 + [_sz] + [_i] * 7 + [_p] * 6 + [_i, _i, _f, _p, _p, _p, _i64, _i, _p, _p, _i, _i],
+    "infllmv2_fwd_kvcache_topk": [_p] * 10 + [_i, _p, _sz] + [_i] * 7 + [_p] * 6 + [_i, _f, _p, _p, _p, _i64, _i, _p, _p, _i, _i],
     "infllmv2_fwd_kvcache_static": [_p] * 10 + [_i] * 7 + [_p] * 6 + [_i, _i, _f, _p, _p, _p, _i64, _i, _p, _p, _i, _i],
     "infllmv2_pack_kv": [_p, _p, _p, _p, _p, _sz, _i, _i64, _i, _i, _i, _p, _p],
 }
 # entry points that exist once per element type: the plain name takes bfloat16, name + "_f16" IEEE half
 PER_ELEMENT_TYPE = ["infllmv2_compress_keys", "infllmv2_compress_keys_pair", "infllmv2_compress_keys_cache", "infllmv2_compress_keys_cache_pair", "infllmv2_varlen_fwd_stage1",
-                    "infllmv2_varlen_fwd_stage1_pooled", "infllmv2_stage1_decode", "infllmv2_varlen_fwd",
-                    "infllmv2_varlen_bwd", "infllmv2_fwd_kvcache"]
+                    "infllmv2_varlen_fwd_stage1_pooled", "infllmv2_stage1_decode", "infllmv2_decode_step_scores", "infllmv2_varlen_fwd",
+                    "infllmv2_varlen_bwd", "infllmv2_fwd_kvcache", "infllmv2_fwd_kvcache_topk"]
 for _name in PER_ELEMENT_TYPE:
     SIGNATURES[_name + "_f16"] = SIGNATURES[_name]
 OTHER = {

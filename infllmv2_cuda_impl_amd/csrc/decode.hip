@@ -35,6 +35,8 @@ struct DecodeParams {
     float* lse_part;                // (batch, Hk, splits, 16)
     const int* cache_seqlens;       // null: every sequence fills the whole cache
     const uint64_t* mask;           // (batch, Hk, n64) or null
+    const int* topk_idx;            // (batch, Hk, k_idx): the selection as an index list instead (-1: unused slot), or null
+    int k_idx;
     int64_t q_batch, q_head;        // element strides of q (batch, head); head dim dense
     int64_t o_batch, o_head;
     int64_t kc_batch, kc_row, kc_head, vc_batch, vc_row, vc_head;
@@ -52,7 +54,8 @@ struct DecodeParams {
     const elem_bits* rot_cos;       // (seqlen_ro, rotary_dim / 2)
     const elem_bits* rot_sin;
     int rotary_dim, rotary_interleaved;
-    elem_bits* q_rot;               // (batch, Hq, 128): the turned query, in the workspace
+    int slots;                      // block tiles of the split kernel's LDS ring: 1 or 2
+    int append_here;                // the split kernel itself writes the one new row per sequence (and sees it whatever the cache holds)
 };
 
 // element offset of cache row `row` of sequence b (head 0)
@@ -66,6 +69,20 @@ __device__ __forceinline__ int64_t cache_row_offset(const DecodeParams& p, int b
     return cb * batch_stride + static_cast<int64_t>(row) * row_stride;
 }
 
+// Eight table values from element index i on: one 16-byte load where the interleaved layout needs four of them, too
+// (the tables are only 2-byte aligned, which global loads do not mind; the last four may lie beyond the row, so they are
+// loaded only where they are used).
+__device__ __forceinline__ void rotary_values(float (&v)[8], const elem_bits* table, int i, bool eight) {
+    uint32_t w[4] = {0, 0, 0, 0};
+    if (eight) __builtin_memcpy(w, table + i, 16);
+    else __builtin_memcpy(w, table + i, 8);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[2 * e] = elem_lo_to_f32(w[e]);
+        v[2 * e + 1] = elem_hi_to_f32(w[e]);
+    }
+}
+
 // One 16-byte chunk (8 values, d = 8 chunk ...) of a head vector turned at position pos.  Interleaved: pairs
 // (2i, 2i+1) lie inside the chunk; contiguous: the partner of d is d +- rotary_dim / 2, in another chunk of the
 // same head vector.  (a, b) -> (a cos - b sin, a sin + b cos) in fp32, one rounding (rotary.h:57-62, 131-133).
@@ -74,7 +91,7 @@ __device__ __forceinline__ uint4 rotary_chunk(const DecodeParams& p, const elem_
     const int d0 = chunk * 8, half = p.rotary_dim >> 1;
     if (d0 >= p.rotary_dim) return raw;
     const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-    float x[8], y[8];
+    float x[8], y[8], c[8], s[8];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         x[2 * e] = elem_lo_to_f32(w[e]);
@@ -83,33 +100,33 @@ __device__ __forceinline__ uint4 rotary_chunk(const DecodeParams& p, const elem_
     const elem_bits* cs = p.rot_cos + static_cast<int64_t>(pos) * half;
     const elem_bits* sn = p.rot_sin + static_cast<int64_t>(pos) * half;
     if (p.rotary_interleaved) {
+        rotary_values(c, cs, d0 >> 1, false);
+        rotary_values(s, sn, d0 >> 1, false);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float c = elem_to_f32(cs[(d0 >> 1) + i]), s = elem_to_f32(sn[(d0 >> 1) + i]);
-            y[2 * i] = x[2 * i] * c - x[2 * i + 1] * s;
-            y[2 * i + 1] = x[2 * i] * s + x[2 * i + 1] * c;
+            y[2 * i] = x[2 * i] * c[i] - x[2 * i + 1] * s[i];
+            y[2 * i + 1] = x[2 * i] * s[i] + x[2 * i + 1] * c[i];
         }
     } else {
         const bool left = d0 < half;
         const uint4 oraw = *reinterpret_cast<const uint4*>(head_vec + (left ? d0 + half : d0 - half));
         const uint32_t ow[4] = {oraw.x, oraw.y, oraw.z, oraw.w};
         const int i0 = left ? d0 : d0 - half;
+        rotary_values(c, cs, i0, true);
+        rotary_values(s, sn, i0, true);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const float o = (e & 1) ? elem_hi_to_f32(ow[e >> 1]) : elem_lo_to_f32(ow[e >> 1]);
-            const float c = elem_to_f32(cs[i0 + e]), s = elem_to_f32(sn[i0 + e]);
-            y[e] = left ? x[e] * c - o * s : x[e] * c + o * s;
+            y[e] = left ? x[e] * c[e] - o * s[e] : x[e] * c[e] + o * s[e];
         }
     }
     return make_uint4(pack_elem2(y[0], y[1]), pack_elem2(y[2], y[3]), pack_elem2(y[4], y[5]), pack_elem2(y[6], y[7]));
 }
 
-constexpr int kVtPitch = kHeadDim + 16;                        // LDS row pitch (elements) of the V tile: rows 8 banks apart, so the
-                                                               // transposing reads of four rows at a time do not collide
-
+// Several new rows per sequence (one is written by the split kernel itself): one thread moves 16 bytes of one new row
+// of K and of V.
 __global__ __launch_bounds__(256)
 void decode_append_kernel(const DecodeParams p) {
-    // one thread moves 16 bytes of one new row of K and of V
     const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     const int64_t total = static_cast<int64_t>(p.batch) * p.seqlen_new * p.num_heads_k * 16;
     if (idx >= total) return;
@@ -127,20 +144,6 @@ void decode_append_kernel(const DecodeParams p) {
     *reinterpret_cast<uint4*>(p.vcache + cache_row_offset(p, b, pos, p.vc_batch, p.vc_row) + h * p.vc_head + chunk * 8) = vv;
 }
 
-// the query turned at the position of the first appended key (all 16 grouped heads of the single query token take
-// the same position: the non-causal rule of flash_fwd_kernel.h:899-901)
-__global__ __launch_bounds__(256)
-void decode_rotate_q_kernel(const DecodeParams p) {
-    const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    const int heads = p.num_heads_k * p.group;
-    if (idx >= static_cast<int64_t>(p.batch) * heads * 16) return;
-    const int chunk = static_cast<int>(idx & 15);
-    const int head = static_cast<int>((idx >> 4) % heads), b = static_cast<int>((idx >> 4) / heads);
-    const int pos = p.cache_seqlens ? p.cache_seqlens[b] : 0;
-    *reinterpret_cast<uint4*>(p.q_rot + (static_cast<int64_t>(b) * heads + head) * kHeadDim + chunk * 8) =
-        rotary_chunk(p, p.q + b * p.q_batch + head * p.q_head, chunk, pos);
-}
-
 typedef short short4d __attribute__((ext_vector_type(4)));
 // 16 lanes x 4 halfwords, transposed (ds_read_b64_tr_b16): lane 16 g + r receives element r % 4 of the four-halfword
 // rows offered by lanes 16 g + r / 4 + {0, 4, 8, 12}
@@ -148,108 +151,240 @@ __device__ __forceinline__ short4d lds_read_tr(const elem_bits* ptr) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4d*)(ptr));
 }
 
+__device__ __forceinline__ uint64_t decode_uniform64(uint64_t v) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
+    return (static_cast<uint64_t>(hi) << 32) | lo;
+}
+
+// A block's tile in LDS: 64 rows of 256 bytes (K, then V), filled by LDS-DMA.  A DMA instruction moves four whole rows
+// (lane 16 g + n: 16 bytes of row 4 u + g) and lands them in lane order, so the rows are unpadded, and the 16-byte
+// pieces of a row are stored XOR-ed with a function of the row instead: both the operand reads of K (16 rows, one piece
+// each) and the transposing reads of V (8 rows, two neighbouring pieces each) then touch every bank once.
+constexpr int kTileBytes = kBlockN * kHeadDim * 2;             // 16 KiB
+constexpr int kSlotBytes = 2 * kTileBytes;
+__device__ __forceinline__ int tile_swizzle(int row) { return ((row & 7) << 1) | ((row >> 3) & 1); }
+__device__ __forceinline__ uint32_t decode_lds_address(const void* ptr) {
+    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)ptr));
+}
+// 16 bytes per lane from base + lane_off to LDS at lds + 16 lane.  Non-temporal: the rows are read once per step.
+// The compiler does not see these loads: whoever reads the tile waits for them by hand.
+__device__ __forceinline__ void decode_dma16(const void* base, uint32_t lane_off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(lane_off), "s"(base), "s"(lds) : "memory", "m0");
+}
+
+// One wavefront per (sequence, KV head, split), bound by HBM: 16 KiB of K and of V per block, read once.  Whole rows go
+// to LDS by non-temporal DMA (269 MB of selected blocks: 45 us for the loads alone, against 51 us for the 16-row pieces
+// of 64 bytes that MFMA operands want straight from memory, and no faster with those marked non-temporal: their
+// 128-byte lines are then fetched twice), with as many blocks in flight as there are slots (p.slots: two, or one where a
+// split holds a single block and more workgroups per CU count).
+//
+// The set-up is a chain of round trips in front of the first block, which is most of the kernel when a split holds one
+// or two of them, so everything that does not depend on anything is requested together: the sequence's length, the mask
+// words (or the index list, OR-ed into words in LDS: no packing launch), the query and the new row.  The split's blocks
+// (64 at a time) and their pages are then looked up by the lanes in parallel and kept in registers: the walk itself
+// makes no loads but the DMA.
+//
+// append_here: the sequence's one new row is patched into its block's tile (turned by the rotary embedding where asked
+// for), so the row need not be in the cache before the launch: the last workgroup of each (sequence, KV head) writes
+// it there meanwhile, and what a reader of that row gets from memory does not matter.
 template <bool kDirect>
 __global__ __launch_bounds__(64)
 void decode_split_kernel(const DecodeParams p) {
-    __shared__ __attribute__((aligned(16))) elem_bits vt[kBlockN * kVtPitch];
+    extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+    __shared__ __attribute__((aligned(16))) elem_bits new_row[2 * kHeadDim];        // K, then V
+    __shared__ int list[64];                                   // the split's blocks
+    uint64_t* words = reinterpret_cast<uint64_t*>(smem + p.slots * kSlotBytes);     // the row's mask words, clipped to the sequence
     const int lane = threadIdx.x;
     const int n = lane & 15, g = lane >> 4;
     const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+    const int seqlen = p.cache_seqlens ? p.cache_seqlens[b] : p.capacity - p.seqlen_new;
     const int lp = p.leftpad ? p.leftpad[b] : 0;              // the sequence's key 0 is cache row lp
-    int L = (p.cache_seqlens ? p.cache_seqlens[b] : p.capacity - p.seqlen_new) + p.seqlen_new;
+    // position of the first appended key; a full cache takes no key, and the tables need not reach beyond it
+    const int rot_pos = !p.cache_seqlens ? 0 : (seqlen < p.capacity ? seqlen : p.capacity - 1);
+    if (p.append_here) {
+        // lanes 0..15: the new K row, lanes 16..31: the new V row, 16 bytes each
+        const int chunk = n;
+        uint4 val = make_uint4(0, 0, 0, 0);
+        if (g == 0) {
+            const elem_bits* kvec = p.knew + b * p.kn_batch + h * p.kn_head;
+            val = p.rotary_dim > 0 ? rotary_chunk(p, kvec, chunk, rot_pos) : *reinterpret_cast<const uint4*>(kvec + chunk * 8);
+        } else if (g == 1) {
+            val = *reinterpret_cast<const uint4*>(p.vnew + b * p.vn_batch + h * p.vn_head + chunk * 8);
+        }
+        if (split == p.splits) {                               // the workgroup that writes the cache
+            if (seqlen >= p.capacity) return;
+            if (g == 0) *reinterpret_cast<uint4*>(p.kcache + cache_row_offset(p, b, seqlen, p.kc_batch, p.kc_row) + h * p.kc_head + chunk * 8) = val;
+            else if (g == 1) *reinterpret_cast<uint4*>(p.vcache + cache_row_offset(p, b, seqlen, p.vc_batch, p.vc_row) + h * p.vc_head + chunk * 8) = val;
+            return;
+        }
+        if (g < 2) *reinterpret_cast<uint4*>(new_row + g * kHeadDim + chunk * 8) = val;    // read by other lanes after the fences below
+    }
+    int L = seqlen + p.seqlen_new;
     if (L > p.capacity) L = p.capacity;
     L -= lp;                                                   // keys of the sequence; mask block j = keys 64 j ..
+    const int new_key = (p.append_here && seqlen < p.capacity) ? seqlen - lp : -1;  // its index in the sequence
     const int last_blk = L <= 0 ? -1 : ((L - 1) >> 6);
-    const uint64_t* row = p.mask ? p.mask + (static_cast<int64_t>(b) * p.num_heads_k + h) * p.n64 : nullptr;
-    BlockWalker walk;
-    walk.init(row, p.n64, last_blk);
+    const bool listed = p.mask != nullptr || p.topk_idx != nullptr;                 // else: every block
+    int n_words = last_blk < 0 ? 0 : (last_blk >> 6) + 1;
+    if (listed && n_words > p.n64) n_words = p.n64;
 
-    // how many blocks does the row select, and which run of them is this split's
-    int total = 0;
-    for (int w = lane; w < walk.n_words; w += 64) {
-        uint64_t v = row ? row[w] : ~0ull;
-        if (w == (last_blk >> 6)) {
-            const int t = last_blk & 63;
-            v &= (t == 63) ? ~0ull : ((1ull << (t + 1)) - 1ull);
-        }
-        total += __builtin_popcountll(v);
-    }
+    elem8 qf[4];
+    {
+        const int qh = p.group * h + (n < p.group ? n : p.group - 1);      // rows beyond the group repeat its last head
+        const elem_bits* qp = p.q + b * p.q_batch + qh * p.q_head;
+        // the query is turned at the position of the first appended key (flash_fwd_kernel.h:899-901)
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) total += __shfl_xor(total, off);
-    total = __builtin_amdgcn_readfirstlane(total);
+        for (int c = 0; c < 4; ++c) {
+            if (p.rotary_dim > 0) {
+                const uint4 turned = rotary_chunk(p, qp, 4 * c + g, rot_pos);
+                __builtin_memcpy(&qf[c], &turned, 16);
+            } else {
+                qf[c] = *reinterpret_cast<const elem8*>(qp + 8 * g + 32 * c);
+            }
+        }
+    }
+
+    // ---- the selected blocks: words in LDS, how many there are, and which run of them is this split's ----
+    auto lds_fence = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
+    const uint64_t last_word_bits = (last_blk & 63) == 63 ? ~0ull : ((1ull << ((last_blk & 63) + 1)) - 1ull);
+    int total = 0;
+    if (!listed) {
+        total = last_blk + 1;
+        lds_fence();
+    } else {
+        const int64_t pair = static_cast<int64_t>(b) * p.num_heads_k + h;
+        if (p.mask != nullptr) {
+            for (int w = lane; w < n_words; w += 64) words[w] = p.mask[pair * p.n64 + w];
+        } else {
+            for (int w = lane; w < n_words; w += 64) words[w] = 0ull;
+            lds_fence();
+            for (int i = lane; i < p.k_idx; i += 64) {
+                const int j = p.topk_idx[pair * p.k_idx + i];
+                if (j >= 0 && j <= last_blk && (j >> 6) < n_words)
+                    atomicOr(reinterpret_cast<unsigned long long*>(&words[j >> 6]), 1ull << (j & 63));
+            }
+        }
+        lds_fence();
+        for (int w = lane; w < n_words; w += 64) {
+            uint64_t v = words[w];
+            if (w == (last_blk >> 6)) { v &= last_word_bits; words[w] = v; }
+            total += __builtin_popcountll(v);
+        }
+        lds_fence();
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) total += __shfl_xor(total, off);
+        total = __builtin_amdgcn_readfirstlane(total);
+    }
     const int per = (total + p.splits - 1) / p.splits;
     const int begin = split * per;
     int count = total - begin;
     if (count > per) count = per;
 
-    elem8 qf[4];
-    {
-        const int qh = p.group * h + (n < p.group ? n : p.group - 1);      // rows beyond the group repeat its last head
-        const elem_bits* qp = p.rotary_dim > 0
-            ? p.q_rot + (static_cast<int64_t>(b) * p.num_heads_k * p.group + qh) * kHeadDim + 8 * g
-            : p.q + b * p.q_batch + qh * p.q_head + 8 * g;
+    // Blocks [base, base + 64) of this split, one per lane, and the cache row (page) they lie in.
+    const int cache_row = p.block_table ? 0 : (p.cache_batch_idx ? p.cache_batch_idx[b] : b);
+    int my_block = 0, my_page = cache_row;
+    auto look_up = [&](int base) {
+        const int lo = begin + base, hi = begin + (count < base + 64 ? count : base + 64);   // ordinals of the row
+        if (!listed) {
+            my_block = lo + lane;
+        } else {
+            int passed = 0;                                    // set bits of the words looked at so far
+            for (int w0 = 0; passed < hi; w0 += 64) {          // hi <= total: some word holds the last one
+                uint64_t bits = w0 + lane < n_words ? words[w0 + lane] : 0ull;
+                const int c = __builtin_popcountll(bits);
+                int incl = c;                                  // inclusive prefix sum over the lanes
 #pragma unroll
-        for (int c = 0; c < 4; ++c) qf[c] = *reinterpret_cast<const elem8*>(qp + 32 * c);
-    }
+                for (int off = 1; off < 64; off <<= 1) {
+                    const int o = __shfl_up(incl, off);
+                    if (lane >= off) incl += o;
+                }
+                int ord = passed + incl - c;
+                if (ord + c > lo && ord < hi)
+                    for (; bits != 0ull && ord < hi; bits &= bits - 1ull, ++ord)
+                        if (ord >= lo) list[ord - lo] = (w0 + lane) * 64 + __builtin_ctzll(bits);
+                passed += __builtin_amdgcn_readlane(incl, 63);
+            }
+            lds_fence();
+            my_block = list[lane];
+            lds_fence();
+        }
+        if (p.block_table && base + lane < count) my_page = p.block_table[b * p.bt_batch + my_block * kBlockN / p.page_size];
+    };
+    if (count > 0) look_up(0);
+
     float m = -INFINITY, l = 0.f;
     floatx4 o[8];
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    int j = -1;
-    for (int skip = 0; skip <= begin && count > 0; ++skip) j = walk.next();   // ordinal `begin` of the row
-    // K rows as A operands and the V rows of block jb, requested together; rows past the end are clamped to a valid row
-    // (K is masked below, P is zero there).  A block never straddles two pages (page_size is a multiple of 64 and
-    // paged caches have no left padding).
-    elem8 kreg[16], vreg[16];
-    auto request = [&](int jb) {
+    // ---- block i of the split into slot i % slots ----
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(decode_lds_address(smem));
+    const int k_pitch = static_cast<int>(p.kc_row) * 2, v_pitch = static_cast<int>(p.vc_row) * 2;   // bytes
+    uint32_t k_off[4], v_off[4];                               // this lane's piece of rows g, 4 + g, 8 + g, 12 + g
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        k_off[u] = static_cast<uint32_t>((4 * u + g) * k_pitch + (n ^ tile_swizzle(4 * u + g)) * 16);
+        v_off[u] = static_cast<uint32_t>((4 * u + g) * v_pitch + (n ^ tile_swizzle(4 * u + g)) * 16);
+    }
+    // a block never straddles two pages (page_size is a multiple of 64 and paged caches have no left padding)
+    auto request = [&](int i) {
+        const int jb = __builtin_amdgcn_readlane(my_block, i & 63), page = __builtin_amdgcn_readlane(my_page, i & 63);
         const int key0 = jb * kBlockN;
-        const elem_bits* kbase = p.kcache + cache_row_offset(p, b, lp + key0, p.kc_batch, p.kc_row) + h * p.kc_head;
-        const elem_bits* vbase = p.vcache + cache_row_offset(p, b, lp + key0, p.vc_batch, p.vc_row) + h * p.vc_head;
+        const int64_t in_page = p.block_table ? key0 % p.page_size : lp + key0;
+        const elem_bits* kbase = p.kcache + page * p.kc_batch + in_page * p.kc_row + h * p.kc_head;
+        const elem_bits* vbase = p.vcache + page * p.vc_batch + in_page * p.vc_row + h * p.vc_head;
+        const uint32_t slot = lds0 + (p.slots == 2 ? i & 1 : 0) * kSlotBytes;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // the slot's previous tile has been read
+        const int last = L - 1 - key0;
+        if (last >= kBlockN - 1) {
 #pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-            int key = key0 + 16 * kt + n;
-            key = key < L ? key : L - 1;
-            const elem_bits* src = kbase + static_cast<int64_t>(key - key0) * p.kc_row + 8 * g;
+            for (int u = 0; u < 16; ++u) decode_dma16(kbase + (u >> 2) * 16 * p.kc_row, k_off[u & 3], slot + u * 1024);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) kreg[kt * 4 + c] = *reinterpret_cast<const elem8*>(src + 32 * c);
-        }
-#pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const int unit = lane + 64 * u;
-            int key = key0 + (unit >> 4);
-            key = key < L ? key : L - 1;
-            vreg[u] = *reinterpret_cast<const elem8*>(vbase + static_cast<int64_t>(key - key0) * p.vc_row + (unit & 15) * 8);
-        }
-    };
-    // One loop turn: S and the V tile of the block whose rows are in the registers (j), then - both register sets
-    // being free again - the request for the next block (j_req), then the softmax and P V of block j while those
-    // rows travel.  The first turn only requests.
-    int j_req = count > 0 ? j : -1, issued = 0;
-    j = -1;
-    for (;;) {
-        const int key0 = j * kBlockN;
-        floatx4 s[4];
-        if (j >= 0) {
-#pragma unroll
-            for (int kt = 0; kt < 4; ++kt) {
-                s[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    s[kt] = IV2_MFMA(kreg[kt * 4 + c], qf[c], s[kt], 0, 0, 0);
-            }
+            for (int u = 0; u < 16; ++u) decode_dma16(vbase + (u >> 2) * 16 * p.vc_row, v_off[u & 3], slot + kTileBytes + u * 1024);
+        } else {
+            // rows past the end are read from the last row (K is masked below, P is zero there)
 #pragma unroll
             for (int u = 0; u < 16; ++u) {
-                const int unit = lane + 64 * u;
-                *reinterpret_cast<elem8*>(&vt[(unit >> 4) * kVtPitch + (unit & 15) * 8]) = vreg[u];
+                int row = 4 * u + g;
+                row = row < last ? row : last;
+                decode_dma16(kbase, static_cast<uint32_t>(row * k_pitch + (n ^ tile_swizzle(4 * u + g)) * 16), slot + u * 1024);
+                decode_dma16(vbase, static_cast<uint32_t>(row * v_pitch + (n ^ tile_swizzle(4 * u + g)) * 16), slot + kTileBytes + u * 1024);
             }
         }
-        if (j_req >= 0) { request(j_req); ++issued; }
-        if (j < 0) {                                           // first turn: nothing to work on yet
-            if (j_req < 0) break;
-            j = j_req;
-            j_req = issued < count ? walk.next() : -1;
-            continue;
+    };
+    // every ordinary load so far has to be back before the waits below count DMA loads only
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(qf[c]));
+    asm volatile("" : "+v"(my_page));
+    if (count > 0) request(0);
+    if (count > 1 && p.slots == 2) request(1);
+    for (int i = 0; i < count; ++i) {
+        if (p.slots == 2 && i + 1 < count && (i & 63) != 63) asm volatile("s_waitcnt vmcnt(32)" ::: "memory");   // the block after this one is in flight
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const int j = __builtin_amdgcn_readlane(my_block, i & 63), key0 = j * kBlockN;
+        unsigned char* ktile = smem + (p.slots == 2 ? i & 1 : 0) * kSlotBytes;
+        if (new_key >= key0 && new_key < key0 + kBlockN) {     // uniform: the block of the row that is being appended
+            const int r = new_key - key0;
+            if (g < 2)
+                *reinterpret_cast<uint4*>(ktile + g * kTileBytes + r * 256 + (n ^ tile_swizzle(r)) * 16) =
+                    *reinterpret_cast<const uint4*>(new_row + g * kHeadDim + 8 * n);
+            lds_fence();
+        }
+        floatx4 s[4];
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            s[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const elem8 kf = *reinterpret_cast<const elem8*>(ktile + (16 * kt + n) * 256 + ((4 * c + g) ^ tile_swizzle(n)) * 16);
+                s[kt] = IV2_MFMA(kf, qf[c], s[kt], 0, 0, 0);
+            }
         }
         const int lim = L - 1 - key0;                           // in-block index of the last valid key
         if (lim < kBlockN - 1) {
@@ -289,31 +424,37 @@ void decode_split_kernel(const DecodeParams p) {
                 pf[cc][e] = static_cast<elem_t>(s[2 * cc][e]);
                 pf[cc][4 + e] = static_cast<elem_t>(s[2 * cc + 1][e]);
             }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_s_barrier();                          // single-wavefront workgroup: orders the LDS tile
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
         // A operand of O^T += V^T P^T: lane (n, g) needs V[32 cc + 4 g + {0..3}, 32 cc + 16 + 4 g + {0..3}][16 dt + n], the
         // keys in the order in which the lane holds P.  One transposing read hands a lane four rows' worth of one
         // column: within 16 lanes, lane i offers the four columns 16 dt + 4 (i % 4) .. of key 4 g + i / 4 (+ 32 cc),
         // and lane n receives column 16 dt + n of the keys 4 g + {0, 1, 2, 3}.
-        const elem_bits* tr_base = vt + (4 * g + (n >> 2)) * kVtPitch + 4 * (n & 3);
+        const int vrow = 4 * g + (n >> 2);                     // + 16, 32, 48: the same swizzle
+        const unsigned char* vtile = ktile + kTileBytes + vrow * 256 + (n & 1) * 8;
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt)
+        for (int dt = 0; dt < 8; ++dt) {
+            const int piece = ((2 * dt + ((n & 3) >> 1)) ^ tile_swizzle(vrow)) * 16;
 #pragma unroll
             for (int cc = 0; cc < 2; ++cc) {
-                const short4d lo = lds_read_tr(tr_base + (32 * cc) * kVtPitch + 16 * dt);
-                const short4d hi = lds_read_tr(tr_base + (32 * cc + 16) * kVtPitch + 16 * dt);
+                const short4d lo = lds_read_tr(reinterpret_cast<const elem_bits*>(vtile + (32 * cc) * 256 + piece));
+                const short4d hi = lds_read_tr(reinterpret_cast<const elem_bits*>(vtile + (32 * cc + 16) * 256 + piece));
                 elem8 vf;
                 __builtin_memcpy(&vf, &lo, 8);
                 __builtin_memcpy(reinterpret_cast<unsigned char*>(&vf) + 8, &hi, 8);
                 o[dt] = IV2_MFMA(vf, pf[cc], o[dt], 0, 0, 0);
             }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_s_barrier();                          // tile consumed before the next block overwrites it
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        if (j_req < 0) break;
-        j = j_req;
-        j_req = issued < count ? walk.next() : -1;
+        }
+        const int next = i + p.slots;                          // into the slot that has just been read
+        if ((i & 63) + p.slots >= 64 && i + 1 < count) {       // the looked-up blocks run out: drain, look up, start again
+            if ((i & 63) == 63) {
+                look_up(i + 1);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                asm volatile("" : "+v"(my_page));
+                request(i + 1);
+                if (p.slots == 2 && i + 2 < count) request(i + 2);
+            }
+        } else if (next < count) {
+            request(next);
+        }
     }
 
     const float l_tot = wave_sum_over_g(l);
@@ -332,73 +473,50 @@ void decode_split_kernel(const DecodeParams p) {
         if (g == 0) p.lse[static_cast<int64_t>(b) * p.num_heads_k * p.group + p.group * h + n] = lse;
     } else {
         const int64_t slot = (static_cast<int64_t>(b) * p.num_heads_k + h) * p.splits + split;
+        if (g == 0) p.lse_part[slot * 16 + n] = lse;
+        if (count <= 0) return;                                // LSE -inf: the combine kernel does not use the partial
         float* op = p.o_part + (slot * 16 + n) * kHeadDim + 4 * g;
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt)
             *reinterpret_cast<float4*>(op + 16 * dt) = make_float4(o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
-        if (g == 0) p.lse_part[slot * 16 + n] = lse;
     }
 }
 
-// merge the per-split partials: one workgroup per (sequence, KV head); thread t -> head t / 16, 8 columns.
-// kSplits > 0: the split count is known at compile time, so every partial is requested before the first is used
-// (one round trip to memory instead of one per split); 0: any count.
-template <int kSplits>
-__global__ __launch_bounds__(256)
+// Merge of the per-split partials: one wavefront per (sequence, query head), lane l holds columns 2 l and 2 l + 1 and,
+// for the weights, split l.  kMax >= splits: the loads are unrolled (beyond the last split the last one is read again),
+// so every partial is requested before the first is used.  A wavefront per head keeps the merge of 64 splits at one
+// round trip; one workgroup per KV head pulled 16 times as much through one CU.
+constexpr int kCombineWaves = 4;
+template <int kMax>
+__global__ __launch_bounds__(64 * kCombineWaves)
 void decode_combine_kernel(const DecodeParams p) {
-    const int h = blockIdx.x, b = blockIdx.y;
-    const int tid = threadIdx.x;
-    const int head = tid >> 4, d0 = (tid & 15) * 8;
+    const int lane = threadIdx.x & 63;
+    const int head = blockIdx.x * kCombineWaves + (threadIdx.x >> 6);
+    const int h = blockIdx.y, b = blockIdx.z;
     if (head >= p.group) return;                               // partial rows that only filled the MFMA tile
     const int64_t slot0 = (static_cast<int64_t>(b) * p.num_heads_k + h) * p.splits;
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float wsum = 0.f, mx = -INFINITY;
-    if constexpr (kSplits > 0) {
-        float ls[kSplits];
-        float4 a[kSplits], c[kSplits];
+    float2 part[kMax];
+    const float lse = lane < p.splits ? p.lse_part[(slot0 + lane) * 16 + head] : -INFINITY;
 #pragma unroll
-        for (int s = 0; s < kSplits; ++s) ls[s] = p.lse_part[(slot0 + s) * 16 + head];
+    for (int s = 0; s < kMax; ++s)
+        part[s] = *reinterpret_cast<const float2*>(p.o_part + ((slot0 + (s < p.splits ? s : p.splits - 1)) * 16 + head) * kHeadDim + 2 * lane);
+    float mx = lse;
 #pragma unroll
-        for (int s = 0; s < kSplits; ++s) {
-            const float* src = p.o_part + ((slot0 + s) * 16 + head) * kHeadDim + d0;
-            a[s] = *reinterpret_cast<const float4*>(src);
-            c[s] = *reinterpret_cast<const float4*>(src + 4);
-        }
+    for (int off = 1; off < 64; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+    const float w = lse == -INFINITY ? 0.f : expf(lse - mx);   // a split without blocks has no partial
+    float wsum = w;
 #pragma unroll
-        for (int s = 0; s < kSplits; ++s) mx = fmaxf(mx, ls[s]);
-        if (mx != -INFINITY) {
+    for (int off = 1; off < 64; off <<= 1) wsum += __shfl_xor(wsum, off);
+    float acc0 = 0.f, acc1 = 0.f;
 #pragma unroll
-            for (int s = 0; s < kSplits; ++s) {
-                const float w = ls[s] == -INFINITY ? 0.f : expf(ls[s] - mx);       // a split without blocks: zeros and -inf
-                wsum += w;
-                acc[0] += w * a[s].x; acc[1] += w * a[s].y; acc[2] += w * a[s].z; acc[3] += w * a[s].w;
-                acc[4] += w * c[s].x; acc[5] += w * c[s].y; acc[6] += w * c[s].z; acc[7] += w * c[s].w;
-            }
-        }
-    } else {
-        for (int s = 0; s < p.splits; ++s) mx = fmaxf(mx, p.lse_part[(slot0 + s) * 16 + head]);
-        if (mx != -INFINITY) {
-            for (int s = 0; s < p.splits; ++s) {
-                const float ls = p.lse_part[(slot0 + s) * 16 + head];
-                if (ls == -INFINITY) continue;
-                const float w = expf(ls - mx);
-                wsum += w;
-                const float* src = p.o_part + ((slot0 + s) * 16 + head) * kHeadDim + d0;
-                const float4 a = *reinterpret_cast<const float4*>(src);
-                const float4 c = *reinterpret_cast<const float4*>(src + 4);
-                acc[0] += w * a.x; acc[1] += w * a.y; acc[2] += w * a.z; acc[3] += w * a.w;
-                acc[4] += w * c.x; acc[5] += w * c.y; acc[6] += w * c.z; acc[7] += w * c.w;
-            }
-        }
+    for (int s = 0; s < kMax; ++s) {
+        const float ws = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(w), s));
+        acc0 += ws != 0.f ? ws * part[s].x : 0.f;              // what a split without blocks left in memory may be anything
+        acc1 += ws != 0.f ? ws * part[s].y : 0.f;
     }
     const float inv = wsum > 0.f ? 1.f / wsum : 0.f;
-    uint4 outv;
-    outv.x = pack_elem2(acc[0] * inv, acc[1] * inv);
-    outv.y = pack_elem2(acc[2] * inv, acc[3] * inv);
-    outv.z = pack_elem2(acc[4] * inv, acc[5] * inv);
-    outv.w = pack_elem2(acc[6] * inv, acc[7] * inv);
-    *reinterpret_cast<uint4*>(p.out + b * p.o_batch + (p.group * h + head) * p.o_head + d0) = outv;
-    if ((tid & 15) == 0)
+    reinterpret_cast<uint32_t*>(p.out + b * p.o_batch + (p.group * h + head) * p.o_head)[lane] = pack_elem2(acc0 * inv, acc1 * inv);
+    if (lane == 0)
         p.lse[static_cast<int64_t>(b) * p.num_heads_k * p.group + p.group * h + head] = wsum > 0.f ? mx + logf(wsum) : INFINITY;
 }
 
@@ -409,14 +527,14 @@ using namespace IV2_NS;
 #ifndef IV2_F16        // element-type independent: defined once
 extern "C" int infllmv2_fwd_kvcache_num_splits(int batch, int num_heads_k, int requested) {
     if (requested > 0) return requested > 64 ? 64 : requested;
-    // aim at two single-wavefront workgroups per CU of a 256-CU device (each keeps the next block's rows in flight, so
-    // longer runs beat more workgroups: 53 us with 4 splits against 55 with 8 at 128 pairs), rounded up to a power of
-    // two, for which the combine kernel is compiled
-    const int pairs = batch * num_heads_k;
-    const int want = (512 + pairs - 1) / (pairs > 0 ? pairs : 1);
-    int s = 1;
-    while (s < want && s < 16) s <<= 1;
-    return s;
+    // Two single-wavefront workgroups fit a CU (two 32 KiB tiles each): as many splits as fill 256 CUs once - one more
+    // and a second, nearly empty round follows (24 sequences x 2 heads, 64 blocks each: 27 us with 10 splits, 35 with
+    // 12).  Beyond 16 splits the merge costs more than the shorter runs gain, unless so few rows are there that most of
+    // the chip would idle (6 sequences: 15.8 us with 16 splits, 18 with 32; 1 sequence: 13.1 with 64, 14.3 with 32).
+    const int pairs = batch * num_heads_k > 0 ? batch * num_heads_k : 1;
+    const int fit = 512 / pairs;
+    if (fit <= 16) return fit > 1 ? fit : 1;
+    return pairs <= 4 ? 64 : 16;
 }
 #endif
 
@@ -427,15 +545,14 @@ static size_t decode_partials_bytes(int batch, int num_heads_k, int num_splits) 
 
 #ifndef IV2_F16        // both element types are 2 bytes wide: defined once
 extern "C" size_t infllmv2_fwd_kvcache_workspace_bytes(int batch, int num_heads_k, int num_splits) {
-    // per-split partial results, then room for the query turned by the rotary embedding
-    return decode_partials_bytes(batch, num_heads_k, num_splits) +
-           static_cast<size_t>(batch) * num_heads_k * 16 * kHeadDim * sizeof(elem_bits);
+    return decode_partials_bytes(batch, num_heads_k, num_splits);
 }
 #endif
 
 static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vcache, const void* k_new,
                                     const void* v_new, const int32_t* cache_seqlens, void* out, float* softmax_lse,
-                                    const uint64_t* blockmask, void* workspace, size_t workspace_bytes, int batch,
+                                    const uint64_t* blockmask, const int32_t* topk_idx, int k_idx, void* workspace,
+                                    size_t workspace_bytes, int batch,
                                     int seqlen_q, int num_heads, int num_heads_k, int head_dim, int cache_capacity,
                                     int seqlen_new, const int64_t* q_strides, const int64_t* kcache_strides,
                                     const int64_t* vcache_strides, const int64_t* knew_strides,
@@ -458,7 +575,9 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
     IV2_CHECK(num_splits >= 1 && num_splits <= 64, "fwd_kvcache: num_splits must be in [1, 64]");
     IV2_CHECK(workspace_bytes >= infllmv2_fwd_kvcache_workspace_bytes(batch, num_heads_k, num_splits),
               "fwd_kvcache: workspace too small");
-    IV2_CHECK(workspace != nullptr || (num_splits == 1 && rotary_cos == nullptr), "fwd_kvcache: split decode and rotary need a workspace");
+    IV2_CHECK(workspace != nullptr || num_splits == 1, "fwd_kvcache: split decode needs a workspace");
+    IV2_CHECK(blockmask == nullptr || topk_idx == nullptr, "fwd_kvcache: give the selection as a mask or as indices, not both");
+    IV2_CHECK(topk_idx == nullptr || k_idx >= 0, "fwd_kvcache: negative number of indices");
     IV2_CHECK(block_table == nullptr || cache_batch_idx == nullptr, "Paged KVcache does not support cache_batch_idx");
     IV2_CHECK(block_table == nullptr || cache_leftpad == nullptr,
               "We don't support Paged KV and leftpad_k running at the same time yet");
@@ -478,6 +597,9 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
     for (int s = 0; s < 3; ++s)
         IV2_CHECK(kcache_strides[s] % 8 == 0 && vcache_strides[s] % 8 == 0, "fwd_kvcache: cache strides must be multiples of 8 elements");
 
+    // a lane's offset inside a block is a 32-bit operand
+    IV2_CHECK(kcache_strides[1] >= 0 && kcache_strides[1] < (1 << 24) && vcache_strides[1] >= 0 && vcache_strides[1] < (1 << 24),
+              "fwd_kvcache: cache row strides must be below 2^24 elements");
     DecodeParams p{};
     p.q = static_cast<const elem_bits*>(q);
     p.kcache = static_cast<elem_bits*>(kcache);
@@ -501,7 +623,15 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
     p.block_table = block_table; p.bt_batch = block_table_batch_stride; p.page_size = block_table ? page_block_size : 1;
     p.rot_cos = static_cast<const elem_bits*>(rotary_cos); p.rot_sin = static_cast<const elem_bits*>(rotary_sin);
     p.rotary_dim = rotary_cos ? rotary_dim : 0; p.rotary_interleaved = rotary_interleaved;
-    p.q_rot = reinterpret_cast<elem_bits*>(static_cast<unsigned char*>(workspace) + decode_partials_bytes(batch, num_heads_k, num_splits));
+    p.topk_idx = topk_idx; p.k_idx = k_idx;
+    if (topk_idx != nullptr) p.n64 = ((cache_capacity + kBlockN - 1) / kBlockN + 63) / 64;
+    // mask words of one row, kept in LDS beside the V tile (18 KiB); 16384 words are 67 million tokens
+    // two tiles in flight per workgroup, two workgroups per CU; where a split holds about one block (64 of them: see
+    // infllmv2_fwd_kvcache_num_splits) a second tile would only keep workgroups off the CU
+    p.slots = num_splits >= 32 ? 1 : 2;
+    const size_t words = (blockmask || topk_idx) ? static_cast<size_t>(((cache_capacity + kBlockN - 1) / kBlockN + 63) / 64) : 0;
+    IV2_CHECK(words <= 8192, "fwd_kvcache: a cache of %d rows needs more mask words than the kernel holds", cache_capacity);
+    const size_t lds = static_cast<size_t>(p.slots) * kSlotBytes + words * sizeof(uint64_t);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (k_new != nullptr) {
         IV2_CHECK(reinterpret_cast<uintptr_t>(k_new) % 16 == 0 && reinterpret_cast<uintptr_t>(v_new) % 16 == 0,
@@ -510,33 +640,33 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
             IV2_CHECK(knew_strides[s] % 8 == 0 && vnew_strides[s] % 8 == 0, "fwd_kvcache: new k/v strides must be multiples of 8 elements");
         p.kn_batch = knew_strides[0]; p.kn_row = knew_strides[1]; p.kn_head = knew_strides[2];
         p.vn_batch = vnew_strides[0]; p.vn_row = vnew_strides[1]; p.vn_head = vnew_strides[2];
-        const int64_t total = static_cast<int64_t>(batch) * seqlen_new * num_heads_k * 16;
-        hipLaunchKernelGGL(decode_append_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, st, p);
-        IV2_LAUNCH_CHECK();
-        if (p.rotary_dim > 0) {
-            const int64_t units = static_cast<int64_t>(batch) * num_heads * 16;
-            hipLaunchKernelGGL(decode_rotate_q_kernel, dim3(static_cast<unsigned>((units + 255) / 256)), dim3(256), 0, st, p);
+        // one new row at a known place: the split kernel takes care of it (one launch less, and no wait for it)
+        p.append_here = seqlen_new == 1 && cache_seqlens != nullptr ? 1 : 0;
+        if (!p.append_here) {
+            const int64_t total = static_cast<int64_t>(batch) * seqlen_new * num_heads_k * 16;
+            hipLaunchKernelGGL(decode_append_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, st, p);
             IV2_LAUNCH_CHECK();
         }
     }
-    const dim3 grid(num_splits, num_heads_k, batch);
+    const void* fn = num_splits == 1 ? reinterpret_cast<const void*>(&decode_split_kernel<true>) : reinterpret_cast<const void*>(&decode_split_kernel<false>);
+    if (lds > 65536 - 2048) {
+        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+        IV2_CHECK(e == hipSuccess, "fwd_kvcache: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
+    }
+    const dim3 grid(num_splits + (p.append_here ? 1 : 0), num_heads_k, batch);
     if (num_splits == 1) {
-        hipLaunchKernelGGL(decode_split_kernel<true>, grid, dim3(64), 0, st, p);
+        hipLaunchKernelGGL(decode_split_kernel<true>, grid, dim3(64), lds, st, p);
         IV2_LAUNCH_CHECK();
     } else {
         float* ws = static_cast<float*>(workspace);
         p.o_part = ws;
         p.lse_part = ws + static_cast<size_t>(batch) * num_heads_k * num_splits * 16 * kHeadDim;
-        hipLaunchKernelGGL(decode_split_kernel<false>, grid, dim3(64), 0, st, p);
+        hipLaunchKernelGGL(decode_split_kernel<false>, grid, dim3(64), lds, st, p);
         IV2_LAUNCH_CHECK();
-        const dim3 cgrid(num_heads_k, batch);
-        switch (num_splits) {
-            case 2: hipLaunchKernelGGL(decode_combine_kernel<2>, cgrid, dim3(256), 0, st, p); break;
-            case 4: hipLaunchKernelGGL(decode_combine_kernel<4>, cgrid, dim3(256), 0, st, p); break;
-            case 8: hipLaunchKernelGGL(decode_combine_kernel<8>, cgrid, dim3(256), 0, st, p); break;
-            case 16: hipLaunchKernelGGL(decode_combine_kernel<16>, cgrid, dim3(256), 0, st, p); break;
-            default: hipLaunchKernelGGL(decode_combine_kernel<0>, cgrid, dim3(256), 0, st, p); break;
-        }
+        const dim3 cgrid((p.group + kCombineWaves - 1) / kCombineWaves, num_heads_k, batch), cblock(64 * kCombineWaves);
+        if (num_splits <= 4) hipLaunchKernelGGL(decode_combine_kernel<4>, cgrid, cblock, 0, st, p);
+        else if (num_splits <= 16) hipLaunchKernelGGL(decode_combine_kernel<16>, cgrid, cblock, 0, st, p);
+        else hipLaunchKernelGGL(decode_combine_kernel<64>, cgrid, cblock, 0, st, p);
         IV2_LAUNCH_CHECK();
     }
     return 0;
@@ -553,12 +683,31 @@ extern "C" int IV2_ENTRY(infllmv2_fwd_kvcache)(void* stream, const void* q, void
                                     const int32_t* cache_leftpad, const int32_t* block_table,
                                     int64_t block_table_batch_stride, int page_block_size, const void* rotary_cos,
                                     const void* rotary_sin, int rotary_dim, int rotary_interleaved) {
-    return fwd_kvcache_impl(stream, q, kcache, vcache, k_new, v_new, cache_seqlens, out, softmax_lse, blockmask, workspace,
-                            workspace_bytes, batch, seqlen_q, num_heads, num_heads_k, head_dim, cache_capacity, seqlen_new,
+    return fwd_kvcache_impl(stream, q, kcache, vcache, k_new, v_new, cache_seqlens, out, softmax_lse, blockmask, nullptr, 0,
+                            workspace, workspace_bytes, batch, seqlen_q, num_heads, num_heads_k, head_dim, cache_capacity, seqlen_new,
                             q_strides, kcache_strides, vcache_strides, knew_strides, vnew_strides, o_strides,
                             n_uint64_per_row, num_splits, softmax_scale, cache_batch_idx, cache_leftpad, block_table,
                             block_table_batch_stride, page_block_size, rotary_cos, rotary_sin, rotary_dim,
                             rotary_interleaved);
+}
+
+extern "C" int IV2_ENTRY(infllmv2_fwd_kvcache_topk)(void* stream, const void* q, void* kcache, void* vcache, const void* k_new,
+                                         const void* v_new, const int32_t* cache_seqlens, void* out, float* softmax_lse,
+                                         const int32_t* topk_idx, int k_idx, void* workspace, size_t workspace_bytes, int batch,
+                                         int seqlen_q, int num_heads, int num_heads_k, int head_dim, int cache_capacity,
+                                         int seqlen_new, const int64_t* q_strides, const int64_t* kcache_strides,
+                                         const int64_t* vcache_strides, const int64_t* knew_strides,
+                                         const int64_t* vnew_strides, const int64_t* o_strides,
+                                         int num_splits, float softmax_scale, const int32_t* cache_batch_idx,
+                                         const int32_t* cache_leftpad, const int32_t* block_table,
+                                         int64_t block_table_batch_stride, int page_block_size, const void* rotary_cos,
+                                         const void* rotary_sin, int rotary_dim, int rotary_interleaved) {
+    IV2_CHECK(topk_idx != nullptr, "fwd_kvcache_topk: null pointer");
+    return fwd_kvcache_impl(stream, q, kcache, vcache, k_new, v_new, cache_seqlens, out, softmax_lse, nullptr, topk_idx, k_idx,
+                            workspace, workspace_bytes, batch, seqlen_q, num_heads, num_heads_k, head_dim, cache_capacity,
+                            seqlen_new, q_strides, kcache_strides, vcache_strides, knew_strides, vnew_strides, o_strides, 0,
+                            num_splits, softmax_scale, cache_batch_idx, cache_leftpad, block_table, block_table_batch_stride,
+                            page_block_size, rotary_cos, rotary_sin, rotary_dim, rotary_interleaved);
 }
 
 #ifndef IV2_F16        // one such entry point in the library: bfloat16 only
@@ -620,7 +769,7 @@ extern "C" int infllmv2_fwd_kvcache_static(void* stream, const void* q, void* kc
         }
         ws = g_scratch_ptr[dev];
     }
-    return fwd_kvcache_impl(stream, q, kcache, vcache, k_new, v_new, cache_seqlens, out, softmax_lse, blockmask, ws,
+    return fwd_kvcache_impl(stream, q, kcache, vcache, k_new, v_new, cache_seqlens, out, softmax_lse, blockmask, nullptr, 0, ws,
                             static_cast<size_t>(INFLLMV2_STATIC_SCRATCH_BYTES), batch, seqlen_q, num_heads, num_heads_k,
                             head_dim, cache_capacity, seqlen_new, q_strides, kcache_strides, vcache_strides, knew_strides,
                             vnew_strides, o_strides, n_uint64_per_row, num_splits, softmax_scale, cache_batch_idx,

@@ -26,6 +26,7 @@
 #include "common.h"
 #include "infllmv2_hip.h"
 #include <math.h>
+#include <type_traits>
 
 namespace IV2_NS {
 
@@ -113,9 +114,11 @@ __device__ __forceinline__ void s1d_run_fixed(int tiles, int per, int split, int
     t1 = t1 < tiles ? t1 : tiles;
 }
 // (max, sum) in log2 units of head 4g + e over the coarse tiles [t0, t1) of one sequence and KV head, merged over the
-// 16 key-column lanes: every lane of row g returns the values of its four heads.
+// 16 key-column lanes: every lane of row g returns the values of its four heads.  patch(tile registers, tile) runs after
+// a tile is requested.
+template <typename Patch>
 __device__ __forceinline__ void s1d_lse_run(const S1DecodeParams& p, const S1DecodeSeq& sq, const elem8 (&qf)[4], int vis_c,
-                                            int t0, int t1, int n, int g, float (&m_out)[4], float (&l_out)[4]) {
+                                            int t0, int t1, int n, int g, float (&m_out)[4], float (&l_out)[4], Patch patch) {
     float m[4], l[4];                                          // head 4g + e over the keys == n (mod 16) of the run
 #pragma unroll
     for (int e = 0; e < 4; ++e) { m[e] = -INFINITY; l[e] = 0.f; }
@@ -150,14 +153,18 @@ __device__ __forceinline__ void s1d_lse_run(const S1DecodeParams& p, const S1Dec
     };
 
     elem8 ta[16], tb[16];
-    if (t0 < t1) s1d_load_tile(ta, sq.cbase, p.c_row_stride, t0 * 64, sq.Lc, n, g);
-    if (t0 + 1 < t1) s1d_load_tile(tb, sq.cbase, p.c_row_stride, (t0 + 1) * 64, sq.Lc, n, g);
+    auto load = [&](elem8 (&t)[16], int ti) {
+        s1d_load_tile(t, sq.cbase, p.c_row_stride, ti * 64, sq.Lc, n, g);
+        patch(t, ti);
+    };
+    if (t0 < t1) load(ta, t0);
+    if (t0 + 1 < t1) load(tb, t0 + 1);
     for (int ti = t0; ti < t1; ti += 2) {
         consume(ta, ti);
-        if (ti + 2 < t1) s1d_load_tile(ta, sq.cbase, p.c_row_stride, (ti + 2) * 64, sq.Lc, n, g);
+        if (ti + 2 < t1) load(ta, ti + 2);
         if (ti + 1 < t1) {
             consume(tb, ti + 1);
-            if (ti + 3 < t1) s1d_load_tile(tb, sq.cbase, p.c_row_stride, (ti + 3) * 64, sq.Lc, n, g);
+            if (ti + 3 < t1) load(tb, ti + 3);
         }
     }
     // merge the 16 key-column lanes of each head
@@ -235,6 +242,14 @@ __device__ __forceinline__ void s1d_merge_records(const S1DRecords& r, int count
     }
 }
 
+__device__ __forceinline__ void s1d_store_record(const S1DecodeParams& p, int b, int h, int split, const float (&m)[4], const float (&l)[4],
+                                                 int n, int g) {
+    float* slot = p.partial + ((static_cast<int64_t>(b) * gridDim.y + h) * p.splits_c + split) * 32;
+    if (n != 0) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { slot[4 * g + e] = m[e]; slot[16 + 4 * g + e] = l[e]; }
+}
+
 __global__ __launch_bounds__(64)
 void stage1_decode_lse_kernel(const S1DecodeParams p) {
     const int lane = threadIdx.x, n = lane & 15, g = lane >> 4;
@@ -249,12 +264,143 @@ void stage1_decode_lse_kernel(const S1DecodeParams p) {
     elem8 qf[4];
     s1d_load_q(qf, p, sq, h, n, g);
     float mm[4], ll[4];
-    s1d_lse_run(p, sq, qf, vis_c, t0, t1, n, g, mm, ll);
-    float* slot = p.partial + ((static_cast<int64_t>(b) * gridDim.y + h) * p.splits_c + split) * 32;
-    if (n == 0) {
+    s1d_lse_run(p, sq, qf, vis_c, t0, t1, n, g, mm, ll, [](elem8 (&)[16], int) {});
+    s1d_store_record(p, b, h, split, mm, ll, n, g);
+}
+
+// ---- the front of a decode step -------------------------------------------------------------------------------------
+// One launch appends the new token to the K/V caches, extends the two compressed-key caches where the token completes a
+// window, and leaves the log-sum-exp records of the coarse keys (the launch above).  Per (sequence, KV head): one
+// workgroup per coarse run, and one that keeps the caches.  Nothing waits for another workgroup: the run that holds a
+// coarse key completed by this very token computes it itself (128 rows of K, of which the newest comes from the
+// caller), writes it to its cache and uses it from LDS; the fine key is used by the next launch only.  As launches of their own
+// the lengths, the append, the compressed keys and the records were six.
+struct S1DecodeStep {
+    const elem_bits* knew;           // (batch, Hk, 128) with strides
+    const elem_bits* vnew;
+    elem_bits* kcache;
+    elem_bits* vcache;
+    elem_bits* fine;                 // the compressed caches (S1DecodeParams' k and c), to be written
+    elem_bits* coarse;
+    int64_t kn_batch, kn_head, vn_batch, vn_head;
+    int64_t kc_batch, kc_row, kc_head, vc_batch, vc_row, vc_head;
+    const int* lens;                 // tokens held before the step; null: host_len for every sequence
+    int host_len;
+    int* new_lens;                   // (batch) each: tokens and compressed keys held afterwards
+    int* fine_lens;
+    int* coarse_lens;
+    int capacity, fine_capacity, coarse_capacity;
+    int kernel_f, stride_f, kernel_c, stride_c;
+    int with_scores;                 // 0: no query, no records (a step that does not score)
+};
+
+__device__ __forceinline__ int s1d_windows(int len, int kernel_size, int stride) {
+    return len >= kernel_size ? (len - kernel_size) / stride + 1 : 0;
+}
+// rows a compressed cache holds after the step and the row this token completes (-1: none); the rules of
+// infllmv2_compress_keys_cache with max_new_rows = 1
+__device__ __forceinline__ int s1d_step_rows(int len, int capacity, int kernel_size, int stride, int out_capacity, int& added) {
+    const int first = s1d_windows(len, kernel_size, stride);
+    int rows = s1d_windows(len + 1 < capacity ? len + 1 : capacity, kernel_size, stride);
+    rows = rows < out_capacity ? rows : out_capacity;
+    rows = rows < first + 1 ? rows : first + 1;
+    added = rows > first ? first : -1;
+    return rows;
+}
+// Elements 2 lane and 2 lane + 1 of the mean of K rows [j stride, j stride + kernel_size) of one head: an fp32 sum in
+// window order divided by kernel_size, rounded once, as compress.hip computes it.  The window's last row is the new
+// token (that is why it is complete now) and comes from the caller.  Rows are requested 64 (32) at a time before they
+// are added up.
+__device__ __forceinline__ uint32_t s1d_window_mean(const S1DecodeStep& t, int b, int h, int j, int kernel_size, int stride, int lane) {
+    const elem_bits* row = t.kcache + b * t.kc_batch + static_cast<int64_t>(j) * stride * t.kc_row + h * t.kc_head + 2 * lane;
+    const uint32_t newest = *reinterpret_cast<const uint32_t*>(t.knew + b * t.kn_batch + h * t.kn_head + 2 * lane);
+    float lo = 0.f, hi = 0.f;
+    int left = kernel_size;
+    auto add = [&](uint32_t v) {
+        lo += elem_lo_to_f32(v);
+        hi += elem_hi_to_f32(v);
+    };
+    auto chunk = [&](auto size) {
+        constexpr int kRows = decltype(size)::value;
+        for (; left >= kRows; left -= kRows) {
+            uint32_t w[kRows];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) { slot[4 * g + e] = mm[e]; slot[16 + 4 * g + e] = ll[e]; }
+            for (int i = 0; i < kRows; ++i) {
+                w[i] = *reinterpret_cast<const uint32_t*>(row);
+                row += t.kc_row;
+                asm volatile("" : "+v"(row));                  // one running address, not one scalar pair per row
+            }
+            if (left == kRows) w[kRows - 1] = newest;
+#pragma unroll
+            for (int i = 0; i < kRows; ++i) add(w[i]);
+        }
+    };
+    chunk(std::integral_constant<int, 64>{});
+    chunk(std::integral_constant<int, 32>{});
+    chunk(std::integral_constant<int, 1>{});
+    const float n = static_cast<float>(kernel_size);
+    return pack_elem2(lo / n, hi / n);
+}
+
+__global__ __launch_bounds__(64)
+void stage1_decode_front_kernel(const S1DecodeParams p, const S1DecodeStep t) {
+    __shared__ __attribute__((aligned(16))) uint32_t newest_key[kHeadDim / 2];      // the coarse key this token completes
+    const int lane = threadIdx.x, n = lane & 15, g = lane >> 4;
+    const int split = static_cast<int>(blockIdx.x) - 1, h = blockIdx.y, b = blockIdx.z;
+    const int len = t.lens ? t.lens[b] : t.host_len;
+    int add_f, add_c;
+    const int rows_f = s1d_step_rows(len, t.capacity, t.kernel_f, t.stride_f, t.fine_capacity, add_f);
+    const int rows_c = s1d_step_rows(len, t.capacity, t.kernel_c, t.stride_c, t.coarse_capacity, add_c);
+    if (split < 0) {                                           // the caches' keeper
+        if (len < t.capacity && g < 2) {
+            const elem_bits* src = g == 0 ? t.knew + b * t.kn_batch + h * t.kn_head : t.vnew + b * t.vn_batch + h * t.vn_head;
+            elem_bits* dst = g == 0 ? t.kcache + b * t.kc_batch + len * t.kc_row + h * t.kc_head
+                                    : t.vcache + b * t.vc_batch + len * t.vc_row + h * t.vc_head;
+            *reinterpret_cast<uint4*>(dst + 8 * n) = *reinterpret_cast<const uint4*>(src + 8 * n);
+        }
+        if (h == 0 && lane == 0) {
+            if (t.new_lens) t.new_lens[b] = len + 1;
+            t.fine_lens[b] = rows_f;
+            t.coarse_lens[b] = rows_c;
+        }
+        if (add_f >= 0)
+            reinterpret_cast<uint32_t*>(t.fine + b * p.k_batch_stride + add_f * p.k_row_stride + h * p.k_head_stride)[lane] =
+                s1d_window_mean(t, b, h, add_f, t.kernel_f, t.stride_f, lane);
+        if (add_c >= 0 && !t.with_scores)
+            reinterpret_cast<uint32_t*>(t.coarse + b * p.c_batch_stride + add_c * p.c_row_stride + h * p.c_head_stride)[lane] =
+                s1d_window_mean(t, b, h, add_c, t.kernel_c, t.stride_c, lane);
+        return;
     }
+    int t0, t1;
+    s1d_run_fixed((rows_c + 63) >> 6, p.run_c, split, t0, t1);
+    if (t0 >= t1 && split > 0) return;                         // beyond this sequence's runs; run 0 always leaves a record
+    S1DecodeSeq sq;
+    sq.q_row = b; sq.Sq = 1; sq.Lk = rows_f; sq.Lc = rows_c;
+    sq.kbase = nullptr;
+    sq.cbase = p.c + b * p.c_batch_stride + h * p.c_head_stride;
+    elem8 qf[4];
+    s1d_load_q(qf, p, sq, h, n, g);
+    const bool adds = add_c >= 0 && add_c >= t0 * 64 && add_c < t1 * 64;            // uniform; add_c is the last key
+    if (adds) {
+        const uint32_t mean = s1d_window_mean(t, b, h, add_c, t.kernel_c, t.stride_c, lane);
+        reinterpret_cast<uint32_t*>(t.coarse + b * p.c_batch_stride + add_c * p.c_row_stride + h * p.c_head_stride)[lane] = mean;
+        newest_key[lane] = mean;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    }
+    float mm[4], ll[4];
+    s1d_lse_run(p, sq, qf, rows_c, t0, t1, n, g, mm, ll, [&](elem8 (&tile)[16], int ti) {
+        if (!adds || ti != add_c >> 6) return;
+        const elem_bits* key = reinterpret_cast<const elem_bits*>(newest_key);
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+            if (ti * 64 + 16 * kt + n >= add_c) {              // the last key, and the lanes beyond it that repeat it
+#pragma unroll
+                for (int c = 0; c < 4; ++c) tile[kt * 4 + c] = *reinterpret_cast<const elem8*>(key + 32 * c + 8 * g);
+            }
+    });
+    s1d_store_record(p, b, h, split, mm, ll, n, g);
 }
 
 __device__ __forceinline__ float s1d_fold_rows16(float x, float y) {
@@ -495,6 +641,82 @@ extern "C" int IV2_ENTRY(infllmv2_stage1_decode)(void* stream, const void* q, co
     const dim3 grid(p.splits_f, num_heads_k, batch);
     if (pooled) hipLaunchKernelGGL(stage1_decode_score_kernel<true>, grid, dim3(64), 0, st, p);
     else hipLaunchKernelGGL(stage1_decode_score_kernel<false>, grid, dim3(64), 0, st, p);
+    IV2_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int IV2_ENTRY(infllmv2_decode_step_scores)(void* stream, const void* q, const void* k_new, const void* v_new, void* kcache,
+                                           void* vcache, void* fine_cache, void* coarse_cache, const int32_t* lens, int host_len,
+                                           int32_t* new_lens, int32_t* fine_lens, int32_t* coarse_lens, void* pooled,
+                                           void* workspace, size_t workspace_bytes, int batch, int num_heads, int num_heads_k,
+                                           int head_dim, int capacity, int fine_rows, int coarse_rows, int max_len,
+                                           const int64_t* q_strides, const int64_t* knew_strides, const int64_t* vnew_strides,
+                                           const int64_t* kcache_strides, const int64_t* vcache_strides,
+                                           const int64_t* fine_strides, const int64_t* coarse_strides, int kernel_size_f,
+                                           int stride_f, int kernel_size_c, int stride_c, float softmax_scale, int out_len,
+                                           int local_blocks, int init_blocks) {
+    const char* who = "decode_step_scores";
+    IV2_CHECK(head_dim == kHeadDim, "%s: this build only supports head_dim 128 (got %d)", who, head_dim);
+    IV2_CHECK(valid_group(num_heads, num_heads_k),
+              "%s: requires num_heads == g * num_heads_k with g in {1, 2, 4, 8, 16} (got %d and %d)", who, num_heads, num_heads_k);
+    IV2_CHECK(batch > 0 && batch <= 65535 && num_heads_k <= 65535, "%s: batch and num_heads_k must be in [1, 65535]", who);
+    IV2_CHECK(capacity > 0 && fine_rows > 0 && coarse_rows > 0 && max_len > 0 && host_len >= 0 && out_len >= 0, "%s: bad sizes", who);
+    IV2_CHECK(kernel_size_f > 0 && stride_f > 0 && kernel_size_c > 0 && stride_c > 0, "%s: kernel_size and stride must be positive", who);
+    IV2_CHECK(k_new && v_new && kcache && vcache && fine_cache && coarse_cache && fine_lens && coarse_lens, "%s: null pointer", who);
+    IV2_CHECK(pooled == nullptr || (q != nullptr && workspace != nullptr), "%s: null pointer", who);
+    const void* aligned16[] = {q, k_new, v_new, kcache, vcache, fine_cache, coarse_cache, workspace};
+    for (const void* a : aligned16) IV2_CHECK(reinterpret_cast<uintptr_t>(a) % 16 == 0, "%s: tensors must be 16-byte aligned", who);
+    for (int s = 0; s < 3; ++s)
+        IV2_CHECK(kcache_strides[s] % 8 == 0 && vcache_strides[s] % 8 == 0 && fine_strides[s] % 8 == 0 && coarse_strides[s] % 8 == 0 &&
+                  (pooled == nullptr || q_strides[s] % 8 == 0), "%s: strides must be multiples of 8 elements", who);
+    IV2_CHECK(knew_strides[0] % 8 == 0 && knew_strides[1] % 8 == 0 && vnew_strides[0] % 8 == 0 && vnew_strides[1] % 8 == 0,
+              "%s: strides must be multiples of 8 elements", who);
+    S1DecodeParams p{};
+    S1DecodeStep t{};
+    // the compressed keys the longest sequence can hold after the step
+    auto windows = [&](int len, int ks, int st) { return len >= ks ? (len - ks) / st + 1 : 0; };
+    int max_f = windows(max_len, kernel_size_f, stride_f), max_c = windows(max_len, kernel_size_c, stride_c);
+    max_f = max_f < fine_rows ? max_f : fine_rows;
+    max_c = max_c < coarse_rows ? max_c : coarse_rows;
+    if (pooled) {
+        s1d_splits(batch, num_heads_k, max_f, max_c, p.splits_f, p.splits_c, p.run_f, p.run_c);
+        IV2_CHECK(workspace_bytes >= infllmv2_stage1_decode_workspace_bytes(batch, num_heads_k, max_f, max_c), "%s: workspace too small", who);
+    }
+    p.q = static_cast<const elem_bits*>(q);
+    p.k = static_cast<const elem_bits*>(fine_cache);
+    p.c = static_cast<const elem_bits*>(coarse_cache);
+    p.out = static_cast<elem_bits*>(pooled);
+    p.partial = static_cast<float*>(workspace);
+    p.k_lens = fine_lens; p.c_lens = coarse_lens;
+    if (pooled) { p.q_tok_stride = q_strides[0]; p.q_grp_stride = q_strides[1]; p.q_kvh_stride = q_strides[2]; }
+    p.k_batch_stride = fine_strides[0]; p.k_row_stride = fine_strides[1]; p.k_head_stride = fine_strides[2];
+    p.c_batch_stride = coarse_strides[0]; p.c_row_stride = coarse_strides[1]; p.c_head_stride = coarse_strides[2];
+    p.out_head_stride = out_len; p.out_row_stride = static_cast<int64_t>(num_heads_k) * out_len;
+    p.cols = fine_rows;
+    p.group = num_heads / num_heads_k;
+    p.scale_log2 = softmax_scale * 1.44269504088896340736f;
+    // the query sits at the position of the new token: its own block is lens[b] / 64
+    p.cache_lens = lens; p.cache_len = host_len; p.pool_len = out_len;
+    p.local_blocks = local_blocks; p.init_blocks = init_blocks;
+    t.knew = static_cast<const elem_bits*>(k_new);
+    t.vnew = static_cast<const elem_bits*>(v_new);
+    t.kcache = static_cast<elem_bits*>(kcache);
+    t.vcache = static_cast<elem_bits*>(vcache);
+    t.fine = static_cast<elem_bits*>(fine_cache);
+    t.coarse = static_cast<elem_bits*>(coarse_cache);
+    t.kn_batch = knew_strides[0]; t.kn_head = knew_strides[1]; t.vn_batch = vnew_strides[0]; t.vn_head = vnew_strides[1];
+    t.kc_batch = kcache_strides[0]; t.kc_row = kcache_strides[1]; t.kc_head = kcache_strides[2];
+    t.vc_batch = vcache_strides[0]; t.vc_row = vcache_strides[1]; t.vc_head = vcache_strides[2];
+    t.lens = lens; t.host_len = host_len;
+    t.new_lens = new_lens; t.fine_lens = fine_lens; t.coarse_lens = coarse_lens;
+    t.capacity = capacity; t.fine_capacity = fine_rows; t.coarse_capacity = coarse_rows;
+    t.kernel_f = kernel_size_f; t.stride_f = stride_f; t.kernel_c = kernel_size_c; t.stride_c = stride_c;
+    t.with_scores = pooled != nullptr ? 1 : 0;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    hipLaunchKernelGGL(stage1_decode_front_kernel, dim3(1 + p.splits_c, num_heads_k, batch), dim3(64), 0, st, p, t);
+    IV2_LAUNCH_CHECK();
+    if (pooled == nullptr || out_len == 0) return 0;
+    hipLaunchKernelGGL(stage1_decode_score_kernel<true>, dim3(p.splits_f, num_heads_k, batch), dim3(64), 0, st, p);
     IV2_LAUNCH_CHECK();
     return 0;
 }
