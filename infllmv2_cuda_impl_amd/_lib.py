@@ -88,6 +88,13 @@ def _load():
 
 lib = _load()
 
+try:
+    import torch  # noqa: F401  (the extension links against it)
+    from . import _host as host             # the operators' native host side (csrc/host_ops.cpp)
+except ImportError as e:
+    raise ImportError("infllmv2_cuda_impl_amd._host is missing or does not load: build it with "
+                      "`python infllmv2_cuda_impl_amd/csrc/build.py`. There is no fallback path.") from e
+
 
 def call(name: str, *args) -> None:
     """Call an int-returning entry point and raise RuntimeError with the library's message on failure."""

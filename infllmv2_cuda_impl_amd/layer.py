@@ -24,10 +24,10 @@ from dataclasses import dataclass
 
 import torch
 
-from .attention import (infllmv2_attn_stage1_kvcache, infllmv2_attn_stage1_pooled, infllmv2_attn_varlen_func,
-                        infllmv2_attn_with_kvcache)
+from . import _lib
+from .attention import HEAD_DIM, infllmv2_attn_varlen_func, infllmv2_attn_with_kvcache, pad_head_dim
 from .pooling import max_pooling_1d_varlen
-from .selection import compress_keys, compress_keys_cache, compress_keys_cache_pair, select_blocks, topk_blocks
+from .selection import compress_keys, compress_keys_cache, topk_blocks
 
 
 @dataclass
@@ -65,6 +65,10 @@ class BatchCache:
         i = lambda: torch.zeros(batch, dtype=torch.int32, device=device)
         return BatchCache(z(capacity), z(capacity), z(capacity // stride + 1), z(capacity // (4 * stride) + 1),
                           i(), i(), i(), 0)
+
+
+def _dense(x):
+    return x if x.stride(-1) == 1 else x.contiguous()
 
 
 class InfLLMv2Attention(torch.nn.Module):
@@ -111,13 +115,12 @@ class InfLLMv2Attention(torch.nn.Module):
             topk_idx, mask = self._window_blocks(k.shape[1], q.shape[0], cu_seqlens, torch.zeros(batch, dtype=torch.int32, device=q.device),
                                                  max_seqlen, 0, q.device)
         elif self.selection == "sparse" and max_seqlen > self.dense_len:
-            cache_lens = torch.zeros(batch, dtype=torch.int32, device=q.device) if batch > 1 else None
-            # the selection launch also writes the packed mask Stage 2 walks
-            topk_idx, mask = select_blocks(q.detach(), k.detach(), cu_seqlens, cu_seqlens, max_seqlen, max_seqlen,
-                                           self.topk, self.local_blocks, self.init_blocks, cache_lens=cache_lens,
-                                           max_cache_len=0, softmax_scale=self.softmax_scale, causal=True,
-                                           kernel_size=self.kernel_size, stride=self.stride,
-                                           block_size=self.block_size, return_mask=True)
+            # the selection launch also writes the packed mask Stage 2 walks; plain prefill: no cached tokens in any sequence
+            scale = q.shape[-1] ** (-0.5) if self.softmax_scale is None else self.softmax_scale
+            qs, ks = (q, k) if q.shape[-1] == HEAD_DIM else pad_head_dim(q, k)
+            topk_idx, mask = _lib.host.select_blocks(qs.detach(), ks.detach(), cu_seqlens, cu_seqlens, max_seqlen, max_seqlen, self.topk,
+                                                     self.local_blocks, self.init_blocks, None, 0, scale, True, self.kernel_size,
+                                                     self.stride, self.block_size, False, True, False, False)
         out = infllmv2_attn_varlen_func(q, k, v, cu_seqlens, cu_seqlens, max_seqlen, max_seqlen,
                                         softmax_scale=self.softmax_scale, causal=True, topk_idx=topk_idx,
                                         block_mask=mask)
@@ -142,36 +145,33 @@ class InfLLMv2Attention(torch.nn.Module):
                 compress_keys(cache.k[0, :n], cu, n, ks, st, out=buf, first_row=rows(old_length, ks, st))
 
     # ---- decode ----
+    def _step(self, q, k_new, v_new, k, v, k_fine, k_coarse, lens, host_len, fine_lens, coarse_lens, max_len):
+        """Append, compressed keys and (sparse branch) selection of one decode step: see :meth:`decode_batch`.  Returns the
+        lengths after the step (device) and the block mask ``(batch, nheads_k, 1, words)`` or None."""
+        scores = self.selection == "sparse" and max_len > self.dense_len
+        scale = q.shape[-1] ** (-0.5) if self.softmax_scale is None else self.softmax_scale
+        return _lib.host.decode_step(q, k_new, v_new, k, v, k_fine, k_coarse, lens, host_len, fine_lens, coarse_lens, max_len,
+                                     self.kernel_size, self.stride, self.block_size, self.topk if scores else 0, self.local_blocks,
+                                     self.init_blocks, scale)
+
     def decode(self, q, k_new, v_new, cache: SequenceCache):
         """One token of one sequence: q ``(1, 1, nheads, d)``, k_new/v_new ``(1, 1, nheads_k, d)``.  Appends the token
-        to the cache (K/V in the decode kernel itself, compressed keys when a window completes), selects blocks and
-        attends.  Returns ``(1, 1, nheads, d)``."""
-        dev = q.device
-        old = cache.length
-        pos = old                                              # position of the new token
-        # the selection needs the new token's key inside the compressed keys, so K goes into the cache first; the
-        # decode kernel's own append then rewrites the same row with the same bytes
-        cache.k[0, pos], cache.v[0, pos] = k_new[0, 0], v_new[0, 0]
-        cache.length = old + 1
-        self._extend_compressed(cache, old)
-        n = cache.length
-        lens = torch.tensor([old], dtype=torch.int32, device=dev)
-        topk_idx = None
+        to the cache (K/V, and the compressed keys when a window completes), selects blocks and attends.  Returns
+        ``(1, 1, nheads, d)``."""
+        pos = cache.length                                     # position of the new token
+        if pos >= cache.k.shape[1]:
+            raise IndexError(f"index {pos} is out of bounds: the K/V cache holds {cache.k.shape[1]} tokens")
+        n = pos + 1
+        q, k_new, v_new = _dense(q), _dense(k_new), _dense(v_new)
+        lens, mask = self._step(q, k_new, v_new, cache.k, cache.v, cache.k_fine.unsqueeze(0), cache.k_coarse.unsqueeze(0), None, pos,
+                                None, None, n)
+        cache.length = n
         if self.selection == "window" and n > self.dense_len:
-            topk_idx, _ = self._window_blocks(cache.k.shape[2], 1, torch.tensor([0, 1], dtype=torch.int32, device=dev), lens,
-                                              1, pos, dev)
-            topk_idx = topk_idx.unsqueeze(0)
-        elif self.selection == "sparse" and n > self.dense_len:
-            rows = lambda ks, st: (n - ks) // st + 1 if n >= ks else 0
-            lf, lc = rows(self.kernel_size, self.stride), rows(4 * self.kernel_size, 4 * self.stride)
-            one = lambda x: torch.tensor([0, x], dtype=torch.int32, device=dev)
-            pooled = infllmv2_attn_stage1_pooled(q[0], cache.k_fine[:lf], cache.k_coarse[:lc], one(1), one(lf), one(lc),
-                                                 1, lf, self.local_blocks, self.init_blocks, cache_len=pos,
-                                                 block_size=self.block_size, stride=self.stride,
-                                                 softmax_scale=self.softmax_scale, causal=False)
-            topk_idx = topk_blocks(pooled, self.topk).unsqueeze(0)                  # (Hk, 1, topk) -> (1, Hk, 1, topk)
-        return infllmv2_attn_with_kvcache(q, cache.k, cache.v, k=k_new, v=v_new, cache_seqlens=lens,
-                                          softmax_scale=self.softmax_scale, topk_idx=topk_idx)
+            dev = q.device
+            _, mask = self._window_blocks(cache.k.shape[2], 1, torch.tensor([0, 1], dtype=torch.int32, device=dev),
+                                          torch.tensor([pos], dtype=torch.int32, device=dev), 1, pos, dev)
+            mask = mask.transpose(0, 1).unsqueeze(2).contiguous()
+        return infllmv2_attn_with_kvcache(q, cache.k, cache.v, cache_seqlens=lens, softmax_scale=self.softmax_scale, block_mask=mask)
 
     # ---- batched decode ----
     def fill_cache(self, cache: BatchCache, k, v, seqlens):
@@ -198,27 +198,14 @@ class InfLLMv2Attention(torch.nn.Module):
         batch = q.shape[0]
         if cache.max_length + 1 > cache.k.shape[1]:
             raise RuntimeError("the K/V cache is full")
-        old = cache.lengths
-        new = old + 1
-        # the selection needs the new key inside the compressed keys; the decode kernel's own append rewrites the row
-        cache.k[torch.arange(batch, device=q.device), old.long()] = k_new[:, 0]
-        compress_keys_cache_pair(cache.k, new, (self.kernel_size, self.stride, cache.k_fine),
-                                 (4 * self.kernel_size, 4 * self.stride, cache.k_coarse), old_lens=old, max_new_rows=1,
-                                 out_lens=(cache.fine_lens, cache.coarse_lens))
-        mask = None
+        q, k_new, v_new = _dense(q), _dense(k_new), _dense(v_new)
+        new, mask = self._step(q, k_new, v_new, cache.k, cache.v, cache.k_fine, cache.k_coarse, cache.lengths, 0, cache.fine_lens,
+                               cache.coarse_lens, cache.max_length + 1)
         if self.selection == "window" and cache.max_length + 1 > self.dense_len:
             cu_one = torch.arange(batch + 1, dtype=torch.int32, device=q.device)
-            _, mask = self._window_blocks(cache.k.shape[2], batch, cu_one, old, 1, cache.max_length, q.device)
+            _, mask = self._window_blocks(cache.k.shape[2], batch, cu_one, cache.lengths, 1, cache.max_length, q.device)
             mask = mask.transpose(0, 1).unsqueeze(2).contiguous()                    # (Hk, batch, words) -> (batch, Hk, 1, words)
-        elif self.selection == "sparse" and cache.max_length + 1 > self.dense_len:
-            pooled = infllmv2_attn_stage1_kvcache(q, cache.k_fine, cache.k_coarse, cache.fine_lens, cache.coarse_lens,
-                                                  old, self.local_blocks, self.init_blocks,
-                                                  max_cache_len=cache.max_length, block_size=self.block_size,
-                                                  stride=self.stride, softmax_scale=self.softmax_scale, causal=False)
-            _, mask = topk_blocks(pooled, self.topk, return_mask=True, by_index=True)
-            mask = mask.unsqueeze(2)                                                 # (batch, Hk, 1, words)
-        out = infllmv2_attn_with_kvcache(q, cache.k, cache.v, k=k_new, v=v_new, cache_seqlens=old,
-                                         softmax_scale=self.softmax_scale, block_mask=mask)
+        out = infllmv2_attn_with_kvcache(q, cache.k, cache.v, cache_seqlens=new, softmax_scale=self.softmax_scale, block_mask=mask)
         cache.lengths = new
         cache.max_length += 1
         return out

@@ -27,20 +27,8 @@ def topk_to_uint64(topk_idx: torch.Tensor, max_seqlen_k: int, block_size: int,
     assert topk_idx.dtype == torch.int32
     if topk_idx.dim() not in (3, 4):
         raise ValueError(f"topk_idx must have 3 or 4 dimensions, got {topk_idx.dim()}")
-    require_gpu(topk_idx, "topk_idx")
     k_blocks = (max_seqlen_k + block_size - 1) // block_size
-    n64 = (k_blocks + 63) // 64
-    idx = topk_idx.contiguous()
-    out_shape = tuple(idx.shape[:-1]) + (n64,)
-    if (memory_buffer is not None and tuple(memory_buffer.shape) == out_shape and memory_buffer.dtype == torch.int64
-            and memory_buffer.device == idx.device and memory_buffer.is_contiguous()):
-        words = memory_buffer
-    else:
-        words = torch.empty(out_shape, dtype=torch.int64, device=idx.device)
-    with torch.cuda.device(idx.device):
-        _lib.call("infllmv2_topk_to_uint64", stream_ptr(idx.device), idx.data_ptr(), words.data_ptr(),
-                  flat_rows(idx.shape[:-1]), idx.shape[-1], k_blocks, n64)
-    return words, k_blocks
+    return _lib.host.topk_to_uint64(topk_idx, k_blocks, memory_buffer), k_blocks
 
 
 def uint64_to_bool(uint64_array: torch.Tensor, last_dim_size: int) -> torch.Tensor:

@@ -9,7 +9,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from ._util import flat_rows, require_gpu, stream_ptr
+from ._util import require_gpu, stream_ptr
 
 
 def topk_blocks(pooled: torch.Tensor, k: int, *, return_mask: bool = False, by_index: bool = False,
@@ -25,29 +25,8 @@ def topk_blocks(pooled: torch.Tensor, k: int, *, return_mask: bool = False, by_i
     a block whose pooled score is ``-inf`` (no visible key: blocks in a causal query's future), so a query with
     fewer than ``k`` reachable blocks gets ``-1`` padding instead of unreachable blocks."""
     assert pooled.dtype == torch.float16 or pooled.dtype == torch.bfloat16
-    require_gpu(pooled, "pooled")
-    x = pooled if pooled.is_contiguous() else pooled.contiguous()
-    n = x.shape[-1]
-    out = torch.empty(tuple(x.shape[:-1]) + (k,), dtype=torch.int32, device=x.device)
-    rows = flat_rows(x.shape[:-1])
-    if not (return_mask or by_index or drop_unreachable):
-        with torch.cuda.device(x.device):
-            _lib.call("infllmv2_topk_blocks", stream_ptr(x.device), x.data_ptr(), n, out.data_ptr(), rows, n, k)
-        return out
-    n64 = (n + 63) // 64 if n_uint64_per_row is None else int(n_uint64_per_row)
-    mask = torch.empty(tuple(x.shape[:-1]) + (n64,), dtype=torch.int64, device=x.device) if return_mask else None
-    with torch.cuda.device(x.device):
-        _lib.call("infllmv2_topk_select", stream_ptr(x.device), x.data_ptr(), n, int(x.dtype == torch.bfloat16),
-                  out.data_ptr(), None if mask is None else mask.data_ptr(), rows, n, k, n64, int(bool(by_index)),
-                  int(bool(drop_unreachable)))
-    return (out, mask) if return_mask else out
-
-
-def _compressed_rows_bound(batch: int, total_k: int, max_seqlen_k: int, kernel_size: int, stride: int) -> int:
-    """Rows to allocate for compressed keys: their number for one sequence, an upper bound for a packed batch."""
-    if batch == 1:
-        return (max_seqlen_k - kernel_size) // stride + 1 if max_seqlen_k >= kernel_size else 0
-    return total_k // stride + 1
+    idx, mask = _lib.host.topk_blocks(pooled, k, return_mask, by_index, drop_unreachable, n_uint64_per_row)
+    return (idx, mask) if return_mask else idx
 
 
 def compress_keys(k: torch.Tensor, cu_seqlens_k: torch.Tensor, max_seqlen_k: int, kernel_size: int, stride: int,
@@ -61,52 +40,13 @@ def compress_keys(k: torch.Tensor, cu_seqlens_k: torch.Tensor, max_seqlen_k: int
     packed batch, so that no host read is needed) and ``cu_seqlens_cmp`` int32 ``(batch + 1)``.  With ``out`` (a
     buffer returned by an earlier call) and ``first_row`` only rows ``>= first_row`` of each sequence are written.
     """
-    require_gpu(k, "k")
-    if k.dtype not in (torch.float16, torch.bfloat16):
-        raise RuntimeError("FlashAttention only support fp16 and bf16 data type")
-    if k.dim() != 3 or k.stride(-1) != 1:
-        raise RuntimeError("k must have shape (total_k, num_heads_k, head_size) with a contiguous last dimension")
-    if cu_seqlens_k.dtype != torch.int32 or not cu_seqlens_k.is_contiguous():
-        raise RuntimeError("cu_seqlens_k must be a contiguous int32 tensor")
-    batch = cu_seqlens_k.numel() - 1
-    total_k, Hk, d = k.shape
-    rows = _compressed_rows_bound(batch, total_k, max_seqlen_k, kernel_size, stride)
-    if out is None:
-        backing = torch.empty((max(rows, 1), Hk, d), dtype=k.dtype, device=k.device)      # never a null pointer
-        out = backing[:rows]
-    elif out.shape[0] < rows or tuple(out.shape[1:]) != (Hk, d) or not out.is_contiguous() or out.dtype != k.dtype:
-        raise RuntimeError("out must be a contiguous (rows, num_heads_k, head_size) buffer of k's dtype")
-    else:
-        backing = out
-    cu_out = torch.empty(batch + 1, dtype=torch.int32, device=k.device)
-    with torch.cuda.device(k.device):
-        _lib.call_for(k.dtype, "infllmv2_compress_keys", stream_ptr(k.device), k.data_ptr(), backing.data_ptr(), cu_seqlens_k.data_ptr(),
-                  cu_out.data_ptr(), batch, max_seqlen_k, Hk, d, k.stride(0), k.stride(1), kernel_size, stride, first_row)
-    return out, cu_out
+    return _lib.host.compress_keys(k, cu_seqlens_k, max_seqlen_k, kernel_size, stride, out, first_row)
 
 
 def compress_keys_pair(k: torch.Tensor, cu_seqlens_k: torch.Tensor, max_seqlen_k: int, fine, coarse):
     """Two :func:`compress_keys` calls on the same keys in one launch; ``fine`` and ``coarse`` are ``(kernel_size, stride)``.
     Returns ``(k_fine, cu_fine, k_coarse, cu_coarse)``."""
-    require_gpu(k, "k")
-    if k.dtype not in (torch.float16, torch.bfloat16):
-        raise RuntimeError("FlashAttention only support fp16 and bf16 data type")
-    if k.dim() != 3 or k.stride(-1) != 1:
-        raise RuntimeError("k must have shape (total_k, num_heads_k, head_size) with a contiguous last dimension")
-    if cu_seqlens_k.dtype != torch.int32 or not cu_seqlens_k.is_contiguous():
-        raise RuntimeError("cu_seqlens_k must be a contiguous int32 tensor")
-    batch = cu_seqlens_k.numel() - 1
-    total_k, Hk, d = k.shape
-    backing, result = [], []
-    for ks, st in (fine, coarse):
-        rows = _compressed_rows_bound(batch, total_k, max_seqlen_k, ks, st)
-        backing.append(torch.empty((max(rows, 1), Hk, d), dtype=k.dtype, device=k.device))      # never a null pointer
-        result += [backing[-1][:rows], torch.empty(batch + 1, dtype=torch.int32, device=k.device)]
-    with torch.cuda.device(k.device):
-        _lib.call_for(k.dtype, "infllmv2_compress_keys_pair", stream_ptr(k.device), k.data_ptr(), backing[0].data_ptr(),
-                      backing[1].data_ptr(), cu_seqlens_k.data_ptr(), result[1].data_ptr(), result[3].data_ptr(), batch,
-                      max_seqlen_k, Hk, d, k.stride(0), k.stride(1), *fine, *coarse)
-    return tuple(result)
+    return _lib.host.compress_keys_pair(k, cu_seqlens_k, max_seqlen_k, *fine, *coarse)
 
 
 def compress_keys_cache(k_cache: torch.Tensor, new_lens: torch.Tensor, kernel_size: int, stride: int, out: torch.Tensor,
@@ -199,23 +139,19 @@ def select_blocks(q: torch.Tensor, k: torch.Tensor, cu_seqlens_q: torch.Tensor, 
     ``(topk_idx, block_mask)`` and the mask (as wide as ``max_seqlen_k`` needs) can be handed to
     ``infllmv2_attn_varlen_func(block_mask=...)``.
     """
-    from .attention import infllmv2_attn_stage1_pooled, pad_head_dim, HEAD_DIM
+    from .attention import pad_head_dim, HEAD_DIM
+    if softmax_scale is None:
+        softmax_scale = q.shape[-1] ** (-0.5)
     if q.shape[-1] != HEAD_DIM:
-        if softmax_scale is None:
-            softmax_scale = q.shape[-1] ** (-0.5)
         q, k = pad_head_dim(q, k)                              # the mean of zero columns is zero
-    if exact_lse:
-        kf, cu_f = compress_keys(k, cu_seqlens_k, max_seqlen_k, kernel_size, stride)
-        kc, cu_c = kf, cu_f
+    if cache_lens is not None:
+        if max_cache_len is None:
+            max_cache_len = int(cache_lens.max().item()) if cache_lens.numel() > 0 else 0
     else:
-        kf, cu_f, kc, cu_c = compress_keys_pair(k, cu_seqlens_k, max_seqlen_k, (kernel_size, stride), (4 * kernel_size, 4 * stride))
-    max_lk = (max_seqlen_k - kernel_size) // stride + 1 if max_seqlen_k >= kernel_size else 0
-    pooled = infllmv2_attn_stage1_pooled(q, kf, kc, cu_seqlens_q, cu_f, cu_c, max_seqlen_q, max_lk, local_blocks,
-                                         init_blocks, cache_lens=cache_lens, max_cache_len=max_cache_len,
-                                         block_size=block_size, stride=stride, softmax_scale=softmax_scale,
-                                         causal=causal)
-    n64 = ((max_seqlen_k + block_size - 1) // block_size + 63) // 64
-    if n64 * 64 < pooled.shape[-1]:                           # cached tokens widen the pooled rows beyond max_seqlen_k
-        n64 = (pooled.shape[-1] + 63) // 64
-    return topk_blocks(pooled, topk, return_mask=return_mask, by_index=by_index, drop_unreachable=drop_unreachable,
-                       n_uint64_per_row=n64)
+        if cu_seqlens_q.numel() != 2:
+            raise RuntimeError("packed sequences need cache_lens (as max_pooling_1d_varlen does)")
+        max_cache_len = 0
+    idx, mask = _lib.host.select_blocks(q, k, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, topk, local_blocks,
+                                        init_blocks, cache_lens, max_cache_len, softmax_scale, causal, kernel_size, stride,
+                                        block_size, exact_lse, return_mask, by_index, drop_unreachable)
+    return (idx, mask) if return_mask else idx

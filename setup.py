@@ -36,7 +36,7 @@ setup(
     version="0.1.0",
     description="InfLLM-V2 two-stage sparse attention for AMD MI355X (gfx950): hand-written HIP kernels behind a C ABI",
     packages=["infllmv2_cuda_impl_amd", "infllm_v2"],
-    package_data={"infllmv2_cuda_impl_amd": ["libinfllmv2_hip.so", "_C*.so", "csrc/*.cpp", "csrc/*.hip", "csrc/*.h", "csrc/build.py", "include/*.h"]},
+    package_data={"infllmv2_cuda_impl_amd": ["libinfllmv2_hip.so", "_C*.so", "_host*.so", "csrc/*.cpp", "csrc/*.hip", "csrc/*.h", "csrc/build.py", "include/*.h"]},
     include_package_data=True,
     python_requires=">=3.9",
     cmdclass={"build_py": BuildWithHip},

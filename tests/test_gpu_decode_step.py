@@ -1,0 +1,109 @@
+"""The kernels of a decode step at the sizes where they can go wrong: the workgroup-per-row top-k at its row lengths and with
+ties, the index-list form of the decode attention, and the launch that appends a token, extends the compressed keys and
+scores, around the lengths at which windows and 64-key tiles complete."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import infllmv2_oracle as O
+from conftest import bf16_np, words_np
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [257, 511, 512, 513, 1024, 1025, 2047, 2048, 2049, 4097, 8192])
+@pytest.mark.parametrize("k", [1, 16, 64, 65, 300])
+def test_topk_with_a_workgroup_per_row(n, k):
+    from infllmv2_cuda_impl_amd import topk_blocks
+    g = torch.Generator(device="cpu").manual_seed(n * 7 + k)
+    rows = torch.stack([torch.randn(n, generator=g), torch.randint(0, 3, (n,), generator=g).float(), torch.zeros(n),
+                        torch.where(torch.rand(n, generator=g) < 0.995, torch.tensor(float("-inf")), torch.randn(n, generator=g)),
+                        torch.where(torch.rand(n, generator=g) < 0.02, torch.tensor(float("inf")), torch.randn(n, generator=g).abs())])
+    pooled = rows.to(torch.bfloat16)
+    ref = O.topk_blocks(bf16_np(pooled), k)
+    idx, mask = topk_blocks(pooled.cuda(), k, return_mask=True)
+    assert np.array_equal(idx.cpu().numpy(), ref)
+    words = O.topk_to_uint64(ref, n * 64, 64)[0]
+    assert np.array_equal(words_np(mask), words)
+    by_index = topk_blocks(pooled.cuda(), k, by_index=True).cpu().numpy()
+    srt = np.sort(np.where(ref < 0, 1 << 30, ref), axis=-1)
+    assert np.array_equal(by_index, np.where(srt == 1 << 30, -1, srt))
+    kept = topk_blocks(pooled.cuda(), k, drop_unreachable=True).cpu().numpy()
+    vals = bf16_np(pooled)
+    for r in range(len(ref)):
+        want = [c for c in ref[r] if c >= 0 and vals[r, c] > -np.inf]
+        assert kept[r].tolist() == want + [-1] * (k - len(want))
+
+
+@pytest.mark.parametrize("splits", [0, 1, 3, 64])
+@pytest.mark.parametrize("new", [0, 1, 2])
+def test_decode_with_an_index_list_equals_the_mask(splits, new):
+    """Unsorted, repeated and unused (-1) slots; lengths at block and cache edges (the last sequence's cache is full)."""
+    import infllmv2_cuda_impl_amd as ops
+    B, cap, Hk = 5, 4288, 2
+    lens = [4288 - new, 64 - new, 1, 4160, 4288]
+    g = torch.Generator(device="cpu").manual_seed(5)
+    mk = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).cuda()
+    q, kc, vc = mk(B, 1, 32, 128), mk(B, cap, Hk, 128), mk(B, cap, Hk, 128)
+    kn, vn = (mk(B, new, Hk, 128), mk(B, new, Hk, 128)) if new else (None, None)
+    idx = torch.randint(-1, cap // 64 + 2, (B, Hk, 1, 70), generator=g).to(torch.int32)
+    idx[:, :, :, 40:50] = idx[:, :, :, :10]
+    idx[1, 0] = -1                                             # nothing selected
+    idx[:, 1, 0, 3] = ((torch.tensor(lens) + max(new, 1) - 1).clamp(max=cap - 1) // 64).to(torch.int32)    # the newest block
+    words = torch.from_numpy(O.topk_to_uint64(idx.numpy(), cap, 64)[0].view(np.int64)).cuda()
+    L = torch.tensor(lens, dtype=torch.int32).cuda()
+    res = []
+    for opt in ({"topk_idx": idx.cuda()}, {"block_mask": words}):
+        k2, v2 = kc.clone(), vc.clone()
+        out, lse = ops.infllmv2_attn_with_kvcache(q, k2, v2, k=kn, v=vn, cache_seqlens=L, num_splits=splits, return_softmax_lse=True, **opt)
+        res.append((out, lse, k2, v2))
+    # the two forms may cut the row into different numbers of runs
+    assert (res[0][0].float() - res[1][0].float()).abs().max() <= 8e-3 and torch.equal(res[0][2], res[1][2]) and torch.equal(res[0][3], res[1][3])
+    kr, vr = bf16_np(kc).copy(), bf16_np(vc).copy()
+    ro, rl = O.decode_forward(bf16_np(q), kr, vr, np.minimum(np.array(lens), cap - new), words_np(words), 128 ** -0.5,
+                              None if kn is None else bf16_np(kn), None if vn is None else bf16_np(vn))
+    ok = [b for b in range(B) if lens[b] + new <= cap]         # a full cache takes no key: compared between the two forms only
+    err = np.abs(bf16_np(res[0][0]) - ro)[ok]
+    assert err.max() <= 2e-2 and err.mean() <= 1e-3
+    assert np.array_equal(bf16_np(res[0][2])[ok], kr[ok]) and np.array_equal(bf16_np(res[0][3])[ok], vr[ok])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Hk,G", [(2, 16), (1, 8)])
+def test_step_launch_equals_the_separate_operators(dtype, Hk, G):
+    """Append + compressed keys + scores + top-k of one step, per sequence, against compress_keys_cache_pair,
+    infllmv2_attn_stage1_kvcache and topk_blocks; with per-sequence lengths on the device and with one host length."""
+    import infllmv2_cuda_impl_amd as ops
+    from infllmv2_cuda_impl_amd import _lib
+    lens = [30, 31, 32, 47, 126, 127, 128, 191, 64 * 128 + 63, 64 * 64 * 2 + 127, 8703, 5000]
+    cap = 8704
+    g = torch.Generator(device="cuda").manual_seed(11)
+    mk = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dtype)
+    B = len(lens)
+    q, kn, vn = mk(B, 1, Hk * G, 128), mk(B, 1, Hk, 128), mk(B, 1, Hk, 128)
+    k, v = mk(B, cap, Hk, 128), mk(B, cap, Hk, 128)
+    L = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    fine, coarse = mk(B, cap // 16 + 1, Hk, 128), mk(B, cap // 64 + 1, Hk, 128)
+    fl, cl = ops.compress_keys_cache_pair(k, L, (32, 16, fine), (128, 64, coarse))
+    # what the step has to leave behind
+    k2, v2, f2, c2, n2 = k.clone(), v.clone(), fine.clone(), coarse.clone(), L + 1
+    for b, n in enumerate(lens):
+        k2[b, n], v2[b, n] = kn[b, 0], vn[b, 0]
+    fl2, cl2 = ops.compress_keys_cache_pair(k2, n2, (32, 16, f2), (128, 64, c2), old_lens=L, max_new_rows=1)
+    pooled = ops.infllmv2_attn_stage1_kvcache(q, f2, c2, fl2, cl2, L, 2, 1, max_cache_len=cap - 1)
+    _, want = ops.topk_blocks(pooled, 16, return_mask=True, by_index=True)
+    got_n, mask = _lib.host.decode_step(q, kn, vn, k, v, fine, coarse, L, 0, fl, cl, cap, 32, 16, 64, 16, 2, 1, 128 ** -0.5)
+    for a, b in ((got_n, n2), (k, k2), (v, v2), (fine, f2), (coarse, c2), (fl, fl2), (cl, cl2)):
+        assert torch.equal(a, b)
+    assert torch.equal(mask[:, :, 0, :want.shape[-1]], want)
+    # one sequence, its length on the host
+    for b in (1, 5, 10):
+        s = slice(b, b + 1)
+        k[b, lens[b]] = 0
+        n1, m1 = _lib.host.decode_step(q[s], kn[s], vn[s], k[s], v[s], fine[s], coarse[s], None, lens[b], None, None, lens[b] + 1,
+                                       32, 16, 64, 16, 2, 1, 128 ** -0.5)
+        assert int(n1) == lens[b] + 1 and torch.equal(k[s], k2[s]) and torch.equal(fine[s], f2[s]) and torch.equal(coarse[s], c2[s])
+        w = m1.shape[-1]
+        blocks = (lens[b] + 64) // 64
+        bits = lambda m: ops.uint64_to_bool(m.contiguous(), blocks)
+        assert torch.equal(bits(m1[:, :, 0]), bits(want[s]))
