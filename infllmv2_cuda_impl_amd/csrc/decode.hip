@@ -54,7 +54,6 @@ struct DecodeParams {
     const elem_bits* rot_cos;       // (seqlen_ro, rotary_dim / 2)
     const elem_bits* rot_sin;
     int rotary_dim, rotary_interleaved;
-    int slots;                      // block tiles of the split kernel's LDS ring: 1 or 2
     int append_here;                // the split kernel itself writes the one new row per sequence (and sees it whatever the cache holds)
 };
 
@@ -173,36 +172,63 @@ __device__ __forceinline__ void decode_dma16(const void* base, uint32_t lane_off
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(lane_off), "s"(base), "s"(lds) : "memory", "m0");
 }
 
-// One wavefront per (sequence, KV head, split), bound by HBM: 16 KiB of K and of V per block, read once.  Whole rows go
-// to LDS by non-temporal DMA (269 MB of selected blocks: 45 us for the loads alone, against 51 us for the 16-row pieces
-// of 64 bytes that MFMA operands want straight from memory, and no faster with those marked non-temporal: their
-// 128-byte lines are then fetched twice), with as many blocks in flight as there are slots (p.slots: two, or one where a
-// split holds a single block and more workgroups per CU count).
+// Position of the set bit of v with `rank` set bits below it (v holds more than `rank`).
+__device__ __forceinline__ int nth_set_bit(uint64_t v, int rank) {
+    int pos = 0;
+#pragma unroll
+    for (int width = 32; width > 0; width >>= 1) {
+        const int c = __builtin_popcountll((v >> pos) & ((1ull << width) - 1ull));
+        if (rank >= c) { rank -= c; pos += width; }
+    }
+    return pos;
+}
+
+// A workgroup per (sequence, KV head, split), bound by HBM: 16 KiB of K and of V per block, read once.  The split's run of
+// blocks is shared out again among its wavefronts, each with its own tiles, softmax state and output; they meet once, at the
+// end.  Whole rows go to LDS by non-temporal DMA (269 MB of selected blocks: 45 us for the loads alone, against 51 us for the
+// 16-row pieces of 64 bytes that MFMA operands want straight from memory, and no faster with those marked non-temporal: their
+// 128-byte lines are then fetched twice).
+//   kWaves == 1: two block tiles per workgroup, two workgroups per CU.  For launches that fill the chip with them.
+//   kWaves == 4: one tile per wavefront; K of the next block is requested as soon as S is formed, V after the output.  The
+//                same 128 KiB in flight per CU, but four blocks are fetched and used side by side and leave one partial:
+//                for the launches whose runs hold a few blocks, where the time is a chain of round trips, not bandwidth
+//                (with the merge: 1 sequence x 2 heads x 64 blocks 16 -> 9.1 us, 6 sequences 18.4 -> 10.7, 24 sequences
+//                32 -> 23, 64 sequences 51.6 -> 49; 64 x 4 heads, one workgroup each and no merge, 95 -> 89).
 //
-// The set-up is a chain of round trips in front of the first block, which is most of the kernel when a split holds one
-// or two of them, so everything that does not depend on anything is requested together: the sequence's length, the mask
-// words (or the index list, OR-ed into words in LDS: no packing launch), the query and the new row.  The split's blocks
-// (64 at a time) and their pages are then looked up by the lanes in parallel and kept in registers: the walk itself
-// makes no loads but the DMA.
+// The set-up is a chain of round trips in front of the first block, so everything that does not depend on anything is
+// requested together: the sequence's length, the mask words (or the index list, OR-ed into words in LDS: no packing
+// launch), the query and the new row.  The run's blocks (64 at a time) and their pages are then looked up by the lanes in
+// parallel and kept in registers: the walk itself makes no loads but the DMA.
 //
 // append_here: the sequence's one new row is patched into its block's tile (turned by the rotary embedding where asked
-// for), so the row need not be in the cache before the launch: the last workgroup of each (sequence, KV head) writes
-// it there meanwhile, and what a reader of that row gets from memory does not matter.
-template <bool kDirect>
-__global__ __launch_bounds__(64)
+// for), so the row need not be in the cache before the launch: the first workgroup of each (sequence, KV head) writes
+// it there on its way out, and what a reader of that row gets from memory does not matter.
+constexpr int kMergePitch = kHeadDim + 4;                      // floats per head of a wavefront's output in LDS
+
+template <bool kDirect, int kWaves>
+__global__ __launch_bounds__(64 * kWaves)
 void decode_split_kernel(const DecodeParams p) {
+    constexpr int kSlots = kWaves == 1 ? 2 : 1;                // block tiles per wavefront
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
     __shared__ __attribute__((aligned(16))) elem_bits new_row[2 * kHeadDim];        // K, then V
-    __shared__ int list[64];                                   // the split's blocks
-    uint64_t* words = reinterpret_cast<uint64_t*>(smem + p.slots * kSlotBytes);     // the row's mask words, clipped to the sequence
-    const int lane = threadIdx.x;
+    __shared__ int lists[kWaves][64];                          // the wavefronts' blocks
+    uint64_t* words = reinterpret_cast<uint64_t*>(smem + kWaves * kSlots * kSlotBytes);     // the row's mask words, clipped to the sequence
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
     const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+    int* list = lists[wave];
+    const int64_t pair = static_cast<int64_t>(b) * p.num_heads_k + h;
+    const bool listed = p.mask != nullptr || p.topk_idx != nullptr;                 // else: every block
+    uint64_t first_word = 0ull;                                // mask word tid
+    int first_idx = -1;                                        // or list entry tid
+    if (p.mask != nullptr && tid < p.n64) first_word = p.mask[pair * p.n64 + tid];
+    if (p.topk_idx != nullptr && tid < p.k_idx) first_idx = p.topk_idx[pair * p.k_idx + tid];
     const int seqlen = p.cache_seqlens ? p.cache_seqlens[b] : p.capacity - p.seqlen_new;
     const int lp = p.leftpad ? p.leftpad[b] : 0;              // the sequence's key 0 is cache row lp
     // position of the first appended key; a full cache takes no key, and the tables need not reach beyond it
     const int rot_pos = !p.cache_seqlens ? 0 : (seqlen < p.capacity ? seqlen : p.capacity - 1);
-    if (p.append_here) {
+    if (p.append_here && wave == 0) {
         // lanes 0..15: the new K row, lanes 16..31: the new V row, 16 bytes each
         const int chunk = n;
         uint4 val = make_uint4(0, 0, 0, 0);
@@ -212,12 +238,6 @@ void decode_split_kernel(const DecodeParams p) {
         } else if (g == 1) {
             val = *reinterpret_cast<const uint4*>(p.vnew + b * p.vn_batch + h * p.vn_head + chunk * 8);
         }
-        if (split == p.splits) {                               // the workgroup that writes the cache
-            if (seqlen >= p.capacity) return;
-            if (g == 0) *reinterpret_cast<uint4*>(p.kcache + cache_row_offset(p, b, seqlen, p.kc_batch, p.kc_row) + h * p.kc_head + chunk * 8) = val;
-            else if (g == 1) *reinterpret_cast<uint4*>(p.vcache + cache_row_offset(p, b, seqlen, p.vc_batch, p.vc_row) + h * p.vc_head + chunk * 8) = val;
-            return;
-        }
         if (g < 2) *reinterpret_cast<uint4*>(new_row + g * kHeadDim + chunk * 8) = val;    // read by other lanes after the fences below
     }
     int L = seqlen + p.seqlen_new;
@@ -225,7 +245,6 @@ void decode_split_kernel(const DecodeParams p) {
     L -= lp;                                                   // keys of the sequence; mask block j = keys 64 j ..
     const int new_key = (p.append_here && seqlen < p.capacity) ? seqlen - lp : -1;  // its index in the sequence
     const int last_blk = L <= 0 ? -1 : ((L - 1) >> 6);
-    const bool listed = p.mask != nullptr || p.topk_idx != nullptr;                 // else: every block
     int n_words = last_blk < 0 ? 0 : (last_blk >> 6) + 1;
     if (listed && n_words > p.n64) n_words = p.n64;
 
@@ -245,47 +264,62 @@ void decode_split_kernel(const DecodeParams p) {
         }
     }
 
-    // ---- the selected blocks: words in LDS, how many there are, and which run of them is this split's ----
+    // ---- the selected blocks: words in LDS, how many there are, and which run of them is this wavefront's ----
     auto lds_fence = [&]() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     };
-    const uint64_t last_word_bits = (last_blk & 63) == 63 ? ~0ull : ((1ull << ((last_blk & 63) + 1)) - 1ull);
-    int total = 0;
+    auto group_fence = [&]() {
+        if constexpr (kWaves > 1) __syncthreads();
+        else lds_fence();
+    };
+    // bits of words w0 + lane: how many lie in words up to and including this lane's, among the 64 words from w0 on
+    auto scan_words = [&](int w0, uint64_t& bits) -> int {
+        bits = w0 + lane < n_words ? words[w0 + lane] : 0ull;
+        int incl = __builtin_popcountll(bits);
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int o = __shfl_up(incl, off);
+            if (lane >= off) incl += o;
+        }
+        return incl;
+    };
+    int total = 0, incl0 = 0;                                  // incl0, bits0: the first 64 words
+    uint64_t bits0 = 0ull;
     if (!listed) {
         total = last_blk + 1;
-        lds_fence();
+        group_fence();
     } else {
-        const int64_t pair = static_cast<int64_t>(b) * p.num_heads_k + h;
         if (p.mask != nullptr) {
-            for (int w = lane; w < n_words; w += 64) words[w] = p.mask[pair * p.n64 + w];
+            const uint64_t last_word_bits = (last_blk & 63) == 63 ? ~0ull : ((1ull << ((last_blk & 63) + 1)) - 1ull);
+            for (int w = tid; w < n_words; w += 64 * kWaves) {
+                const uint64_t v = w == tid ? first_word : p.mask[pair * p.n64 + w];
+                words[w] = w == (last_blk >> 6) ? v & last_word_bits : v;
+            }
         } else {
-            for (int w = lane; w < n_words; w += 64) words[w] = 0ull;
-            lds_fence();
-            for (int i = lane; i < p.k_idx; i += 64) {
-                const int j = p.topk_idx[pair * p.k_idx + i];
+            for (int w = tid; w < n_words; w += 64 * kWaves) words[w] = 0ull;
+            group_fence();
+            for (int i = tid; i < p.k_idx; i += 64 * kWaves) {
+                const int j = i == tid ? first_idx : p.topk_idx[pair * p.k_idx + i];
                 if (j >= 0 && j <= last_blk && (j >> 6) < n_words)
                     atomicOr(reinterpret_cast<unsigned long long*>(&words[j >> 6]), 1ull << (j & 63));
             }
         }
-        lds_fence();
-        for (int w = lane; w < n_words; w += 64) {
-            uint64_t v = words[w];
-            if (w == (last_blk >> 6)) { v &= last_word_bits; words[w] = v; }
-            total += __builtin_popcountll(v);
+        group_fence();
+        incl0 = scan_words(0, bits0);
+        total = __builtin_amdgcn_readlane(incl0, 63);
+        for (int w0 = 64; w0 < n_words; w0 += 64) {
+            uint64_t bits;
+            total += __builtin_amdgcn_readlane(scan_words(w0, bits), 63);
         }
-        lds_fence();
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) total += __shfl_xor(total, off);
-        total = __builtin_amdgcn_readfirstlane(total);
     }
-    const int per = (total + p.splits - 1) / p.splits;
-    const int begin = split * per;
-    int count = total - begin;
-    if (count > per) count = per;
+    // equal runs: their lengths differ by one at most
+    const int runs = p.splits * kWaves, run = split * kWaves + wave;
+    const int begin = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(total) * run / runs);
+    const int count = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(total) * (run + 1) / runs) - begin;
 
-    // Blocks [base, base + 64) of this split, one per lane, and the cache row (page) they lie in.
+    // Blocks [base, base + 64) of this run, one per lane, and the cache row (page) they lie in.
     const int cache_row = p.block_table ? 0 : (p.cache_batch_idx ? p.cache_batch_idx[b] : b);
     int my_block = 0, my_page = cache_row;
     auto look_up = [&](int base) {
@@ -295,18 +329,18 @@ void decode_split_kernel(const DecodeParams p) {
         } else {
             int passed = 0;                                    // set bits of the words looked at so far
             for (int w0 = 0; passed < hi; w0 += 64) {          // hi <= total: some word holds the last one
-                uint64_t bits = w0 + lane < n_words ? words[w0 + lane] : 0ull;
+                uint64_t bits = bits0;
+                const int incl = w0 == 0 ? incl0 : scan_words(w0, bits);
                 const int c = __builtin_popcountll(bits);
-                int incl = c;                                  // inclusive prefix sum over the lanes
-#pragma unroll
-                for (int off = 1; off < 64; off <<= 1) {
-                    const int o = __shfl_up(incl, off);
-                    if (lane >= off) incl += o;
-                }
                 int ord = passed + incl - c;
-                if (ord + c > lo && ord < hi)
+                if (ord + c > lo && ord < hi) {
+                    if (ord < lo) {                            // the run starts inside this word
+                        bits &= ~0ull << nth_set_bit(bits, lo - ord);
+                        ord = lo;
+                    }
                     for (; bits != 0ull && ord < hi; bits &= bits - 1ull, ++ord)
-                        if (ord >= lo) list[ord - lo] = (w0 + lane) * 64 + __builtin_ctzll(bits);
+                        list[ord - lo] = (w0 + lane) * 64 + __builtin_ctzll(bits);
+                }
                 passed += __builtin_amdgcn_readlane(incl, 63);
             }
             lds_fence();
@@ -322,8 +356,9 @@ void decode_split_kernel(const DecodeParams p) {
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-    // ---- block i of the split into slot i % slots ----
-    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(decode_lds_address(smem));
+    // ---- block i of the run into slot i % kSlots ----
+    unsigned char* tiles = smem + wave * kSlots * kSlotBytes;
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(decode_lds_address(tiles));
     const int k_pitch = static_cast<int>(p.kc_row) * 2, v_pitch = static_cast<int>(p.vc_row) * 2;   // bytes
     uint32_t k_off[4], v_off[4];                               // this lane's piece of rows g, 4 + g, 8 + g, 12 + g
 #pragma unroll
@@ -331,51 +366,56 @@ void decode_split_kernel(const DecodeParams p) {
         k_off[u] = static_cast<uint32_t>((4 * u + g) * k_pitch + (n ^ tile_swizzle(4 * u + g)) * 16);
         v_off[u] = static_cast<uint32_t>((4 * u + g) * v_pitch + (n ^ tile_swizzle(4 * u + g)) * 16);
     }
-    // a block never straddles two pages (page_size is a multiple of 64 and paged caches have no left padding)
-    auto request = [&](int i) {
+    // 16 DMA instructions for K or V of a block, which never straddles two pages (page_size is a multiple of 64 and paged
+    // caches have no left padding)
+    auto request_tile = [&](int i, const elem_bits* cache, int64_t batch_stride, int64_t row_stride, int64_t head_stride, int pitch,
+                            const uint32_t (&off)[4], uint32_t tile) {
         const int jb = __builtin_amdgcn_readlane(my_block, i & 63), page = __builtin_amdgcn_readlane(my_page, i & 63);
         const int key0 = jb * kBlockN;
         const int64_t in_page = p.block_table ? key0 % p.page_size : lp + key0;
-        const elem_bits* kbase = p.kcache + page * p.kc_batch + in_page * p.kc_row + h * p.kc_head;
-        const elem_bits* vbase = p.vcache + page * p.vc_batch + in_page * p.vc_row + h * p.vc_head;
-        const uint32_t slot = lds0 + (p.slots == 2 ? i & 1 : 0) * kSlotBytes;
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // the slot's previous tile has been read
+        const elem_bits* base = cache + page * batch_stride + in_page * row_stride + h * head_stride;
+        uint32_t slot = lds0 + (kSlots == 2 ? i & 1 : 0) * kSlotBytes + tile;
+        // the slot's previous tile has been read; and the sixteen addresses in it are no loop invariants worth a register each
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(slot) : : "memory");
         const int last = L - 1 - key0;
         if (last >= kBlockN - 1) {
 #pragma unroll
-            for (int u = 0; u < 16; ++u) decode_dma16(kbase + (u >> 2) * 16 * p.kc_row, k_off[u & 3], slot + u * 1024);
-#pragma unroll
-            for (int u = 0; u < 16; ++u) decode_dma16(vbase + (u >> 2) * 16 * p.vc_row, v_off[u & 3], slot + kTileBytes + u * 1024);
+            for (int u = 0; u < 16; ++u) decode_dma16(base + (u >> 2) * 16 * row_stride, off[u & 3], slot + u * 1024);
         } else {
             // rows past the end are read from the last row (K is masked below, P is zero there)
 #pragma unroll
             for (int u = 0; u < 16; ++u) {
                 int row = 4 * u + g;
                 row = row < last ? row : last;
-                decode_dma16(kbase, static_cast<uint32_t>(row * k_pitch + (n ^ tile_swizzle(4 * u + g)) * 16), slot + u * 1024);
-                decode_dma16(vbase, static_cast<uint32_t>(row * v_pitch + (n ^ tile_swizzle(4 * u + g)) * 16), slot + kTileBytes + u * 1024);
+                decode_dma16(base, static_cast<uint32_t>(row * pitch + (n ^ tile_swizzle(4 * u + g)) * 16), slot + u * 1024);
             }
         }
     };
+    auto request_k = [&](int i) { request_tile(i, p.kcache, p.kc_batch, p.kc_row, p.kc_head, k_pitch, k_off, 0); };
+    auto request_v = [&](int i) { request_tile(i, p.vcache, p.vc_batch, p.vc_row, p.vc_head, v_pitch, v_off, kTileBytes); };
     // every ordinary load so far has to be back before the waits below count DMA loads only
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
     for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(qf[c]));
     asm volatile("" : "+v"(my_page));
-    if (count > 0) request(0);
-    if (count > 1 && p.slots == 2) request(1);
+    if (count > 0) { request_k(0); request_v(0); }
+    if (kSlots == 2 && count > 1) { request_k(1); request_v(1); }
     for (int i = 0; i < count; ++i) {
-        if (p.slots == 2 && i + 1 < count && (i & 63) != 63) asm volatile("s_waitcnt vmcnt(32)" ::: "memory");   // the block after this one is in flight
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        // in flight, oldest first: K and V of this block, and with two slots K and V of the next one
+        const bool ahead = kSlots == 2 && i + 1 < count && (i & 63) != 63;
+        if (ahead) asm volatile("s_waitcnt vmcnt(48)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
         const int j = __builtin_amdgcn_readlane(my_block, i & 63), key0 = j * kBlockN;
-        unsigned char* ktile = smem + (p.slots == 2 ? i & 1 : 0) * kSlotBytes;
-        if (new_key >= key0 && new_key < key0 + kBlockN) {     // uniform: the block of the row that is being appended
+        unsigned char* ktile = tiles + (kSlots == 2 ? i & 1 : 0) * kSlotBytes;
+        const bool patch = new_key >= key0 && new_key < key0 + kBlockN;            // uniform: the block of the row that is being appended
+        auto patch_row = [&](int which) {                      // 0: K, 1: V
             const int r = new_key - key0;
-            if (g < 2)
-                *reinterpret_cast<uint4*>(ktile + g * kTileBytes + r * 256 + (n ^ tile_swizzle(r)) * 16) =
-                    *reinterpret_cast<const uint4*>(new_row + g * kHeadDim + 8 * n);
+            if (g == 0)
+                *reinterpret_cast<uint4*>(ktile + which * kTileBytes + r * 256 + (n ^ tile_swizzle(r)) * 16) =
+                    *reinterpret_cast<const uint4*>(new_row + which * kHeadDim + 8 * n);
             lds_fence();
-        }
+        };
+        if (patch) patch_row(0);
         floatx4 s[4];
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
@@ -385,6 +425,16 @@ void decode_split_kernel(const DecodeParams p) {
                 const elem8 kf = *reinterpret_cast<const elem8*>(ktile + (16 * kt + n) * 256 + ((4 * c + g) ^ tile_swizzle(n)) * 16);
                 s[kt] = IV2_MFMA(kf, qf[c], s[kt], 0, 0, 0);
             }
+        }
+        bool next_k = false;
+        if (kSlots == 1 && i + 1 < count) {
+            if ((i & 63) == 63) {                              // the looked-up blocks run out
+                look_up(i + 1);
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                asm volatile("" : "+v"(my_page));
+            }
+            request_k(i + 1);
+            next_k = true;
         }
         const int lim = L - 1 - key0;                           // in-block index of the last valid key
         if (lim < kBlockN - 1) {
@@ -424,6 +474,10 @@ void decode_split_kernel(const DecodeParams p) {
                 pf[cc][e] = static_cast<elem_t>(s[2 * cc][e]);
                 pf[cc][4 + e] = static_cast<elem_t>(s[2 * cc + 1][e]);
             }
+        if (ahead) asm volatile("s_waitcnt vmcnt(32)" ::: "memory");
+        else if (next_k) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (patch) patch_row(1);
         // A operand of O^T += V^T P^T: lane (n, g) needs V[32 cc + 4 g + {0..3}, 32 cc + 16 + 4 g + {0..3}][16 dt + n], the
         // keys in the order in which the lane holds P.  One transposing read hands a lane four rows' worth of one
         // column: within 16 lanes, lane i offers the four columns 16 dt + 4 (i % 4) .. of key 4 g + i / 4 (+ 32 cc),
@@ -443,23 +497,72 @@ void decode_split_kernel(const DecodeParams p) {
                 o[dt] = IV2_MFMA(vf, pf[cc], o[dt], 0, 0, 0);
             }
         }
-        const int next = i + p.slots;                          // into the slot that has just been read
-        if ((i & 63) + p.slots >= 64 && i + 1 < count) {       // the looked-up blocks run out: drain, look up, start again
+        if (kSlots == 1) {
+            if (next_k) request_v(i + 1);
+        } else if ((i & 63) + 2 >= 64 && i + 1 < count) {      // the looked-up blocks run out: drain, look up, start again
             if ((i & 63) == 63) {
                 look_up(i + 1);
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 asm volatile("" : "+v"(my_page));
-                request(i + 1);
-                if (p.slots == 2 && i + 2 < count) request(i + 2);
+                request_k(i + 1); request_v(i + 1);
+                if (i + 2 < count) { request_k(i + 2); request_v(i + 2); }
             }
-        } else if (next < count) {
-            request(next);
+        } else if (i + 2 < count) {                            // into the slot that has just been read
+            request_k(i + 2); request_v(i + 2);
         }
     }
 
+    if (p.append_here && split == 0 && wave == 0 && seqlen < p.capacity && g < 2) {
+        const int64_t at = g == 0 ? cache_row_offset(p, b, seqlen, p.kc_batch, p.kc_row) + h * p.kc_head
+                                  : cache_row_offset(p, b, seqlen, p.vc_batch, p.vc_row) + h * p.vc_head;
+        *reinterpret_cast<uint4*>((g == 0 ? p.kcache : p.vcache) + at + 8 * n) = *reinterpret_cast<const uint4*>(new_row + g * kHeadDim + 8 * n);
+    }
     const float l_tot = wave_sum_over_g(l);
+    const int64_t slot = pair * p.splits + split;
+    const float no_keys = kDirect ? INFINITY : -INFINITY;
+    if constexpr (kWaves > 1) {
+        // merge of the wavefronts' (m, l, O): each leaves its own in its tile, then 16 threads per head, 8 columns each
+        __shared__ float merge_m[kWaves][16], merge_l[kWaves][16];
+        float* mine = reinterpret_cast<float*>(tiles) + n * kMergePitch + 4 * g;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) *reinterpret_cast<floatx4*>(mine + 16 * dt) = o[dt];
+        if (g == 0) { merge_m[wave][n] = m; merge_l[wave][n] = l_tot; }
+        __syncthreads();
+        for (int t = tid; t < 256; t += 64 * kWaves) {
+            const int head = t >> 4, col = (t & 15) * 8;
+            float top = -INFINITY;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) top = fmaxf(top, merge_m[w][head]);
+            const float ref = top == -INFINITY ? 0.f : top;
+            float sum = 0.f, acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) {
+                const float f = __builtin_amdgcn_exp2f(merge_m[w][head] - ref);
+                const float* theirs = reinterpret_cast<const float*>(smem + w * kSlots * kSlotBytes) + head * kMergePitch + col;
+                sum += f * merge_l[w][head];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) acc[e] += f * theirs[e];
+            }
+            const float inv = sum > 0.f ? 1.f / sum : 0.f;
+            const float lse = sum > 0.f ? top * 0.69314718055994530942f + logf(sum) : no_keys;
+            if (kDirect) {
+                if (head >= p.group) continue;
+                *reinterpret_cast<uint4*>(p.out + b * p.o_batch + (p.group * h + head) * p.o_head + col) =
+                    make_uint4(pack_elem2(acc[0] * inv, acc[1] * inv), pack_elem2(acc[2] * inv, acc[3] * inv),
+                               pack_elem2(acc[4] * inv, acc[5] * inv), pack_elem2(acc[6] * inv, acc[7] * inv));
+                if (col == 0) p.lse[static_cast<int64_t>(b) * p.num_heads_k * p.group + p.group * h + head] = lse;
+            } else {
+                if (col == 0) p.lse_part[slot * 16 + head] = lse;
+                float* op = p.o_part + (slot * 16 + head) * kHeadDim + col;        // LSE -inf: the combine kernel does not use it
+                *reinterpret_cast<float4*>(op) = make_float4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
+                *reinterpret_cast<float4*>(op + 4) = make_float4(acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv);
+            }
+        }
+        return;
+    }
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    const float lse = l_tot > 0.f ? m * 0.69314718055994530942f + logf(l_tot) : (kDirect ? INFINITY : -INFINITY);
+    const float lse = l_tot > 0.f ? m * 0.69314718055994530942f + logf(l_tot) : no_keys;
     if (kDirect) {
         if (n >= p.group) return;
         elem_bits* op = p.out + b * p.o_batch + (p.group * h + n) * p.o_head + 4 * g;
@@ -472,7 +575,6 @@ void decode_split_kernel(const DecodeParams p) {
         }
         if (g == 0) p.lse[static_cast<int64_t>(b) * p.num_heads_k * p.group + p.group * h + n] = lse;
     } else {
-        const int64_t slot = (static_cast<int64_t>(b) * p.num_heads_k + h) * p.splits + split;
         if (g == 0) p.lse_part[slot * 16 + n] = lse;
         if (count <= 0) return;                                // LSE -inf: the combine kernel does not use the partial
         float* op = p.o_part + (slot * 16 + n) * kHeadDim + 4 * g;
@@ -524,17 +626,19 @@ void decode_combine_kernel(const DecodeParams p) {
 
 using namespace IV2_NS;
 
+// Up to so many workgroups a launch takes the four-wavefront form of the split kernel: one on every CU.
+constexpr int kGroupedWorkgroups = 256;
+
 #ifndef IV2_F16        // element-type independent: defined once
 extern "C" int infllmv2_fwd_kvcache_num_splits(int batch, int num_heads_k, int requested) {
     if (requested > 0) return requested > 64 ? 64 : requested;
-    // Two single-wavefront workgroups fit a CU (two 32 KiB tiles each): as many splits as fill 256 CUs once - one more
-    // and a second, nearly empty round follows (24 sequences x 2 heads, 64 blocks each: 27 us with 10 splits, 35 with
-    // 12).  Beyond 16 splits the merge costs more than the shorter runs gain, unless so few rows are there that most of
-    // the chip would idle (6 sequences: 15.8 us with 16 splits, 18 with 32; 1 sequence: 13.1 with 64, 14.3 with 32).
+    // What fills 256 CUs once, with the four-wavefront workgroups (one per CU) as long as every (sequence, KV head) gets one
+    // of them, with the single-wavefront ones (two per CU) beyond; one more and a second, nearly empty round follows.  More
+    // than 16 partials cost the merge more than the shorter runs gain.
     const int pairs = batch * num_heads_k > 0 ? batch * num_heads_k : 1;
-    const int fit = 512 / pairs;
-    if (fit <= 16) return fit > 1 ? fit : 1;
-    return pairs <= 4 ? 64 : 16;
+    const int fit = kGroupedWorkgroups / pairs;
+    if (fit >= 1) return fit > 16 ? 16 : fit;
+    return 512 / pairs > 1 ? 512 / pairs : 1;
 }
 #endif
 
@@ -625,13 +729,11 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
     p.rotary_dim = rotary_cos ? rotary_dim : 0; p.rotary_interleaved = rotary_interleaved;
     p.topk_idx = topk_idx; p.k_idx = k_idx;
     if (topk_idx != nullptr) p.n64 = ((cache_capacity + kBlockN - 1) / kBlockN + 63) / 64;
-    // mask words of one row, kept in LDS beside the V tile (18 KiB); 16384 words are 67 million tokens
-    // two tiles in flight per workgroup, two workgroups per CU; where a split holds about one block (64 of them: see
-    // infllmv2_fwd_kvcache_num_splits) a second tile would only keep workgroups off the CU
-    p.slots = num_splits >= 32 ? 1 : 2;
+    // mask words of one row, kept in LDS beside the tiles; 8192 words are 33 million tokens, 2048 still fit beside four tiles
     const size_t words = (blockmask || topk_idx) ? static_cast<size_t>(((cache_capacity + kBlockN - 1) / kBlockN + 63) / 64) : 0;
     IV2_CHECK(words <= 8192, "fwd_kvcache: a cache of %d rows needs more mask words than the kernel holds", cache_capacity);
-    const size_t lds = static_cast<size_t>(p.slots) * kSlotBytes + words * sizeof(uint64_t);
+    const bool grouped = static_cast<int64_t>(batch) * num_heads_k * num_splits <= kGroupedWorkgroups && words <= 2048;
+    const size_t lds = (grouped ? 4 : 2) * static_cast<size_t>(kSlotBytes) + words * sizeof(uint64_t);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (k_new != nullptr) {
         IV2_CHECK(reinterpret_cast<uintptr_t>(k_new) % 16 == 0 && reinterpret_cast<uintptr_t>(v_new) % 16 == 0,
@@ -648,21 +750,18 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
             IV2_LAUNCH_CHECK();
         }
     }
-    const void* fn = num_splits == 1 ? reinterpret_cast<const void*>(&decode_split_kernel<true>) : reinterpret_cast<const void*>(&decode_split_kernel<false>);
-    if (lds > 65536 - 2048) {
-        hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        IV2_CHECK(e == hipSuccess, "fwd_kvcache: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
-    }
-    const dim3 grid(num_splits + (p.append_here ? 1 : 0), num_heads_k, batch);
-    if (num_splits == 1) {
-        hipLaunchKernelGGL(decode_split_kernel<true>, grid, dim3(64), lds, st, p);
-        IV2_LAUNCH_CHECK();
-    } else {
+    if (num_splits > 1) {
         float* ws = static_cast<float*>(workspace);
         p.o_part = ws;
         p.lse_part = ws + static_cast<size_t>(batch) * num_heads_k * num_splits * 16 * kHeadDim;
-        hipLaunchKernelGGL(decode_split_kernel<false>, grid, dim3(64), lds, st, p);
-        IV2_LAUNCH_CHECK();
+    }
+    void (*split_kernel)(DecodeParams) = num_splits == 1 ? (grouped ? decode_split_kernel<true, 4> : decode_split_kernel<true, 1>)
+                                                         : (grouped ? decode_split_kernel<false, 4> : decode_split_kernel<false, 1>);
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(split_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+    IV2_CHECK(e == hipSuccess, "fwd_kvcache: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
+    hipLaunchKernelGGL(split_kernel, dim3(num_splits, num_heads_k, batch), dim3(grouped ? 256 : 64), lds, st, p);
+    IV2_LAUNCH_CHECK();
+    if (num_splits > 1) {
         const dim3 cgrid((p.group + kCombineWaves - 1) / kCombineWaves, num_heads_k, batch), cblock(64 * kCombineWaves);
         if (num_splits <= 4) hipLaunchKernelGGL(decode_combine_kernel<4>, cgrid, cblock, 0, st, p);
         else if (num_splits <= 16) hipLaunchKernelGGL(decode_combine_kernel<16>, cgrid, cblock, 0, st, p);

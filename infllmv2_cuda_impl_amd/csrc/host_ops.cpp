@@ -546,9 +546,8 @@ std::tuple<Tensor, Tensor> fwd_kvcache(const Tensor& q, const Tensor& kc, const 
     Tensor out = at::empty_like(q);
     Tensor lse = at::empty({batch, hq, 1}, q.options().dtype(at::kFloat));
     int splits = infllmv2_fwd_kvcache_num_splits(as_int(batch), as_int(hk), as_int(num_splits));
-    // no more splits than there are blocks to share out (a caller's own count stands)
-    if (num_splits <= 0 && idx.has_value())
-        while (splits > 1 && splits / 2 >= idx->size(3)) splits /= 2;
+    // no more splits than leave each of a workgroup's four wavefronts a block (a caller's own count stands)
+    if (num_splits <= 0 && idx.has_value()) splits = as_int(std::min<int64_t>(splits, std::max<int64_t>(1, (idx->size(3) + 3) / 4)));
     Tensor ws = bytes_on(q, infllmv2_fwd_kvcache_workspace_bytes(as_int(batch), as_int(hk), splits));
     const int64_t qs[2] = {q.stride(0), q.stride(2)}, os[2] = {out.stride(0), out.stride(2)};
     const S3 kcs = batch_rows_heads(kc), vcs = batch_rows_heads(vc);

@@ -107,3 +107,28 @@ def test_step_launch_equals_the_separate_operators(dtype, Hk, G):
         blocks = (lens[b] + 64) // 64
         bits = lambda m: ops.uint64_to_bool(m.contiguous(), blocks)
         assert torch.equal(bits(m1[:, :, 0]), bits(want[s]))
+
+
+@pytest.mark.parametrize("held", [64 * 64 * 4 - 1, 64 * 64 * 4 + 65, 64 * 64 * 8 + 1, 40])
+@pytest.mark.parametrize("masked", [False, True])
+def test_decode_runs_longer_than_one_look_up(held, masked):
+    """Workgroups of four wavefronts and of one, runs of up to and over 64 blocks per wavefront, the new row in the last of them."""
+    import infllmv2_cuda_impl_amd as ops
+    g = torch.Generator(device="cuda").manual_seed(held)
+    mk = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    cap, Hk = (held + 64) // 64 * 64, 1
+    q, kc, vc, kn, vn = mk(1, 1, 16, 128), mk(1, cap, Hk, 128), mk(1, cap, Hk, 128), mk(1, 1, Hk, 128), mk(1, 1, Hk, 128)
+    L = torch.tensor([held], dtype=torch.int32, device="cuda")
+    words = torch.randint(-2 ** 62, 2 ** 62, (1, Hk, 1, (cap // 64 + 63) // 64), generator=g, device="cuda") | -(2 ** 63) | 1 if masked else None
+    kr, vr = kc.clone(), vc.clone()
+    kr[:, held], vr[:, held] = kn[:, 0], vn[:, 0]
+    s = (q[0, 0].float() @ kr[0, :held + 1, 0].float().t()) * 128 ** -0.5
+    if masked:
+        j = torch.arange(held + 1, device="cuda") // 64
+        s = s.masked_fill(((words[0, 0, 0][j // 64] >> (j % 64)) & 1) == 0, float("-inf"))
+    ref = torch.softmax(s, -1) @ vr[0, :held + 1, 0].float()
+    for splits in (0, 1, 2, 64):
+        k2, v2 = kc.clone(), vc.clone()
+        out = ops.infllmv2_attn_with_kvcache(q, k2, v2, k=kn, v=vn, cache_seqlens=L, num_splits=splits, block_mask=words)
+        assert torch.equal(k2, kr) and torch.equal(v2, vr)
+        assert (out[0, 0].float() - ref).abs().max() <= 1e-2 * max(1.0, float(ref.abs().max()))
