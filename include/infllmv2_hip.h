@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define INFLLMV2_ABI_VERSION 12
+#define INFLLMV2_ABI_VERSION 13
 
 /* ---- library ------------------------------------------------------------------------------ */
 
@@ -361,6 +361,17 @@ int infllmv2_fwd_kvcache_topk(void* stream, const void* q, void* kcache, void* v
                               int64_t block_table_batch_stride, int page_block_size, const void* rotary_cos,
                               const void* rotary_sin, int rotary_dim, int rotary_interleaved);
 
+/* infllmv2_fwd_kvcache with the selection made by the same launch: the topk largest of the block scores of each row,
+ * scores (batch, Hk, n_scores), dense, of the tensors' element type, as Stage 1 with pooling leaves them (no negative
+ * value but -inf; n_scores <= INFLLMV2_DECODE_MAX_SCORES; batch x Hk x num_splits <= 256).  No new keys. */
+#define INFLLMV2_DECODE_MAX_SCORES 2048
+int infllmv2_fwd_kvcache_scores(void* stream, const void* q, void* kcache, void* vcache, const int32_t* cache_seqlens,
+                                void* out, float* softmax_lse, const void* scores, int n_scores, int topk,
+                                void* workspace, size_t workspace_bytes, int batch, int num_heads, int num_heads_k,
+                                int head_dim, int cache_capacity, const int64_t* q_strides,
+                                const int64_t* kcache_strides, const int64_t* vcache_strides, const int64_t* o_strides,
+                                int num_splits, float softmax_scale);
+
 /* No counterpart in the reference.  infllmv2_fwd_kvcache for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): the same kernels and arguments, without
  * the workspace pair.  The split partials go to a buffer of INFLLMV2_STATIC_SCRATCH_BYTES that is
@@ -462,6 +473,12 @@ int infllmv2_varlen_bwd_f16(void* stream, const void* dout, const void* q, const
                             const int64_t* do_strides, const int64_t* dq_strides, const int64_t* dk_strides,
                             const int64_t* dv_strides, const int64_t* lse_strides, int n_uint64_per_row,
                             float softmax_scale, int is_causal, int deterministic);
+int infllmv2_fwd_kvcache_scores_f16(void* stream, const void* q, void* kcache, void* vcache, const int32_t* cache_seqlens,
+                                    void* out, float* softmax_lse, const void* scores, int n_scores, int topk,
+                                    void* workspace, size_t workspace_bytes, int batch, int num_heads, int num_heads_k,
+                                    int head_dim, int cache_capacity, const int64_t* q_strides,
+                                    const int64_t* kcache_strides, const int64_t* vcache_strides, const int64_t* o_strides,
+                                    int num_splits, float softmax_scale);
 int infllmv2_fwd_kvcache_topk_f16(void* stream, const void* q, void* kcache, void* vcache, const void* k_new,
                                   const void* v_new, const int32_t* cache_seqlens, void* out, float* softmax_lse,
                                   const int32_t* topk_idx, int k_idx, void* workspace, size_t workspace_bytes, int batch,

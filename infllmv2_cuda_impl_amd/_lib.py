@@ -11,7 +11,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libinfllmv2_hip.so")
 
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 _p, _i, _i64, _sz, _f = C.c_void_p, C.c_int, C.c_int64, C.c_size_t, C.c_float
 
@@ -42,13 +42,15 @@ SIGNATURES = {
     "infllmv2_varlen_bwd": [_p] * 14 + [_sz, _i, _i64, _i64, _i, _i, _i, _i, _i] + [_p] * 9 + [_i, _f, _i, _i],
     "infllmv2_fwd_kvcache": [_p] * 11 + [_sz] + [_i] * 7 + [_p] * 6 + [_i, _i, _f, _p, _p, _p, _i64, _i, _p, _p, _i, _i],
     "infllmv2_fwd_kvcache_topk": [_p] * 10 + [_i, _p, _sz] + [_i] * 7 + [_p] * 6 + [_i, _f, _p, _p, _p, _i64, _i, _p, _p, _i, _i],
+    "infllmv2_fwd_kvcache_scores": [_p] * 8 + [_i, _i, _p, _sz] + [_i] * 5 + [_p] * 4 + [_i, _f],
     "infllmv2_fwd_kvcache_static": [_p] * 10 + [_i] * 7 + [_p] * 6 + [_i, _i, _f, _p, _p, _p, _i64, _i, _p, _p, _i, _i],
     "infllmv2_pack_kv": [_p, _p, _p, _p, _p, _sz, _i, _i64, _i, _i, _i, _p, _p],
 }
 # entry points that exist once per element type: the plain name takes bfloat16, name + "_f16" IEEE half
 PER_ELEMENT_TYPE = ["infllmv2_compress_keys", "infllmv2_compress_keys_pair", "infllmv2_compress_keys_cache", "infllmv2_compress_keys_cache_pair", "infllmv2_varlen_fwd_stage1",
                     "infllmv2_varlen_fwd_stage1_pooled", "infllmv2_stage1_decode", "infllmv2_decode_step_scores", "infllmv2_varlen_fwd",
-                    "infllmv2_varlen_bwd", "infllmv2_fwd_kvcache", "infllmv2_fwd_kvcache_topk"]
+                    "infllmv2_varlen_bwd", "infllmv2_fwd_kvcache", "infllmv2_fwd_kvcache_topk",
+                    "infllmv2_fwd_kvcache_scores"]
 for _name in PER_ELEMENT_TYPE:
     SIGNATURES[_name + "_f16"] = SIGNATURES[_name]
 OTHER = {

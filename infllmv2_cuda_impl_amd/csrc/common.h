@@ -115,10 +115,26 @@ __device__ __forceinline__ elem_bits f32_to_elem_hw(float f) {
     return b;
 }
 __device__ __forceinline__ uint32_t pack_elem2(float lo, float hi) {
-    return static_cast<uint32_t>(f32_to_elem(lo)) | (static_cast<uint32_t>(f32_to_elem(hi)) << 16);
+    return static_cast<uint32_t>(f32_to_elem_hw(lo)) | (static_cast<uint32_t>(f32_to_elem_hw(hi)) << 16);
 }
 // the two elements of a 32-bit word
 __device__ __forceinline__ float elem_lo_to_f32(uint32_t w) { return elem_to_f32(static_cast<elem_bits>(w & 0xffffu)); }
 __device__ __forceinline__ float elem_hi_to_f32(uint32_t w) { return elem_to_f32(static_cast<elem_bits>(w >> 16)); }
+
+// Brings every cache line of the kernel's arguments into the scalar cache in one round trip.  The compiler loads arguments
+// where they are first needed, each of these loads with its own wait: with 350 bytes of them that was a quarter of what a
+// short kernel spends before its first request.
+template <int kBytes>
+__device__ __forceinline__ void warm_kernel_arguments() {
+    static_assert(kBytes >= 4 && kBytes <= 7 * 64, "more cache lines than are touched here");
+    constexpr int kLast = kBytes - 4;
+    auto line = [](int i) constexpr { return 64 * i < kLast ? 64 * i : kLast; };
+    uint32_t a, b, c, d, e, f, g;
+    asm volatile("s_load_dword %0, %7, %8\n\ts_load_dword %1, %7, %9\n\ts_load_dword %2, %7, %10\n\ts_load_dword %3, %7, %11\n\t"
+                 "s_load_dword %4, %7, %12\n\ts_load_dword %5, %7, %13\n\ts_load_dword %6, %7, %14\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&s"(a), "=&s"(b), "=&s"(c), "=&s"(d), "=&s"(e), "=&s"(f), "=&s"(g)
+                 : "s"(__builtin_amdgcn_kernarg_segment_ptr()), "n"(line(0)), "n"(line(1)), "n"(line(2)), "n"(line(3)), "n"(line(4)),
+                   "n"(line(5)), "n"(kLast));
+}
 
 }  // namespace IV2_NS

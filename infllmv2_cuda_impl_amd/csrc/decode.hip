@@ -37,6 +37,8 @@ struct DecodeParams {
     const uint64_t* mask;           // (batch, Hk, n64) or null
     const int* topk_idx;            // (batch, Hk, k_idx): the selection as an index list instead (-1: unused slot), or null
     int k_idx;
+    const elem_bits* scores;         // (batch, Hk, n_scores) block scores: the selection is their k_select largest; or null
+    int n_scores, k_select;
     int64_t q_batch, q_head;        // element strides of q (batch, head); head dim dense
     int64_t o_batch, o_head;
     int64_t kc_batch, kc_row, kc_head, vc_batch, vc_row, vc_head;
@@ -172,15 +174,15 @@ __device__ __forceinline__ void decode_dma16(const void* base, uint32_t lane_off
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(lane_off), "s"(base), "s"(lds) : "memory", "m0");
 }
 
-// Position of the set bit of v with `rank` set bits below it (v holds more than `rank`).
-__device__ __forceinline__ int nth_set_bit(uint64_t v, int rank) {
+// v (wavefront-uniform, more than `rank` bits set) without its `rank` lowest set bits
+__device__ __forceinline__ uint64_t drop_set_bits(uint64_t v, int rank) {
     int pos = 0;
 #pragma unroll
     for (int width = 32; width > 0; width >>= 1) {
         const int c = __builtin_popcountll((v >> pos) & ((1ull << width) - 1ull));
         if (rank >= c) { rank -= c; pos += width; }
     }
-    return pos;
+    return v & (~0ull << pos);
 }
 
 // A workgroup per (sequence, KV head, split), bound by HBM: 16 KiB of K and of V per block, read once.  The split's run of
@@ -205,30 +207,142 @@ __device__ __forceinline__ int nth_set_bit(uint64_t v, int rank) {
 // it there on its way out, and what a reader of that row gets from memory does not matter.
 constexpr int kMergePitch = kHeadDim + 4;                      // floats per head of a wavefront's output in LDS
 
-template <bool kDirect, int kWaves>
+__device__ __forceinline__ int scan_lanes(int v) {              // inclusive prefix sum over the lanes, DPP adds only
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);     // row_shr 1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);     // row_bcast 15, 31
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+    return v;
+}
+
+// The k largest of the first `cols` of a row of block scores (the order of topk.hip: larger first, ties by ascending column), by
+// a workgroup of four wavefronts; lane w of each gets mask word w.  Column 256 e + 64 wave + lane is key[e], as signed 16-bit
+// integers: scores of Stage 1 are never negative but for -inf, so that is their order, and -32768 is free for "no column".
+// Bound by the instructions a wavefront issues one after the other (a lone one needs five clocks for each), so it spends few of
+// them per column: one histogram of the keys up to 1023 (eight powers of two) below the largest finite score, in LDS, two
+// scans over the lanes find the k-th key and how many columns equal it.  Halving the 16 bits by counts took three times as
+// long.  Every split of a row repeats this: as a launch of its own the selection took 3.2 us at 12 rows of 313 columns and
+// 6.5 at 128 rows of 2048.
+struct SelectScratch {
+    uint32_t bins[512];                                        // two 16-bit counts each
+    int2 tops[2][4];                                           // per wavefront: its largest key up to the limit, its columns above it
+    uint32_t equal[32];
+    uint64_t words[32];
+};
+constexpr int kNoColumn = -32768;
+
+template <int kItems>
+__device__ __forceinline__ uint64_t select_words(const elem_bits* row, int n, int cols, int k_want, SelectScratch& t, int tid, int wave, int lane) {
+    int key[kItems];
+#pragma unroll
+    for (int e = 0; e < kItems; ++e) {
+        const int col = 256 * e + tid;
+        key[e] = reinterpret_cast<const int16_t*>(row)[col < n ? col : 0];
+    }
+    *reinterpret_cast<uint2*>(&t.bins[2 * tid]) = make_uint2(0, 0);
+    const int k = k_want < cols ? k_want : cols;
+    if (k <= 0) return 0ull;                                   // uniform over the workgroup
+#pragma unroll
+    for (int e = 0; e < kItems; ++e) key[e] = 256 * e + tid < cols ? key[e] : kNoColumn;
+    int limit = kElemPosInf - 1, thr, c_above, c_equal;        // the forced blocks (+inf) stay above the histogram
+    for (int round = 0;; ++round) {
+        int top = kNoColumn, above = 0;
+#pragma unroll
+        for (int e = 0; e < kItems; ++e) {
+            top = max(top, key[e] <= limit ? key[e] : kNoColumn);
+            above += __builtin_popcountll(__builtin_amdgcn_ballot_w64(key[e] > limit));
+        }
+        top = max(top, __builtin_amdgcn_update_dpp(top, top, 0xB1, 0xF, 0xF, false));      // a row's maximum: quad_perm,
+        top = max(top, __builtin_amdgcn_update_dpp(top, top, 0x4E, 0xF, 0xF, false));
+        top = max(top, __builtin_amdgcn_update_dpp(top, top, 0x124, 0xF, 0xF, false));     // row_ror 4, 8
+        top = max(top, __builtin_amdgcn_update_dpp(top, top, 0x128, 0xF, 0xF, false));
+        top = max(max(static_cast<int>(__builtin_amdgcn_readlane(top, 0)), static_cast<int>(__builtin_amdgcn_readlane(top, 16))),
+                  max(static_cast<int>(__builtin_amdgcn_readlane(top, 32)), static_cast<int>(__builtin_amdgcn_readlane(top, 48))));
+        if (lane == 0) t.tops[round & 1][wave] = make_int2(top, above);
+        __syncthreads();
+        const int2 t0 = t.tops[round & 1][0], t1 = t.tops[round & 1][1], t2 = t.tops[round & 1][2], t3 = t.tops[round & 1][3];
+        top = __builtin_amdgcn_readfirstlane(max(max(t0.x, t1.x), max(t2.x, t3.x)));
+        above = __builtin_amdgcn_readfirstlane(t0.y + t1.y + t2.y + t3.y);
+        if (above >= k) { limit = 32767; continue; }           // only at first: no more than forced blocks are wanted
+#pragma unroll
+        for (int e = 0; e < kItems; ++e) {
+            const int bin = min(top - key[e], 1023);
+            if (key[e] <= limit && key[e] != kNoColumn) atomicAdd(&t.bins[bin >> 1], (bin & 1) ? 0x10000u : 1u);
+        }
+        __syncthreads();
+        const uint4 a = *reinterpret_cast<const uint4*>(&t.bins[8 * lane]), b = *reinterpret_cast<const uint4*>(&t.bins[8 * lane + 4]);
+        const uint32_t pairs = a.x + a.y + a.z + a.w + b.x + b.y + b.z + b.w;
+        const int mine = static_cast<int>((pairs & 0xffffu) + (pairs >> 16));
+        const int upto = scan_lanes(mine) + above;
+        const int at = __builtin_ctzll(__builtin_amdgcn_ballot_w64(upto >= k) | 1ull << 63);
+        const int fine = lane < 16 ? static_cast<int>(reinterpret_cast<const uint16_t*>(t.bins)[16 * at + lane]) : 0;
+        const int fine_upto = scan_lanes(fine) + static_cast<int>(__builtin_amdgcn_readlane(upto - mine, at));
+        const int in = __builtin_ctzll(__builtin_amdgcn_ballot_w64(fine_upto >= k) | 1ull << 63) & 15;
+        c_equal = __builtin_amdgcn_readlane(fine, in);
+        c_above = static_cast<int>(__builtin_amdgcn_readlane(fine_upto, in)) - c_equal;
+        thr = top - (16 * at + in);
+        if (16 * at + in < 1023) break;
+        limit = thr;                                           // the last bin holds everything further down: again from there
+        __syncthreads();
+        *reinterpret_cast<uint2*>(&t.bins[2 * tid]) = make_uint2(0, 0);
+    }
+    const int ties = k - c_above;                              // of the columns equal to thr, the first so many
+    int equal_before = 0;                                      // lane w: those in the words before w
+    if (ties < c_equal) {
+#pragma unroll
+        for (int e = 0; e < kItems; ++e) {
+            const int c = __builtin_popcountll(__builtin_amdgcn_ballot_w64(key[e] == thr));
+            if (lane == 0) t.equal[4 * e + wave] = c;
+        }
+        __syncthreads();
+        const int c = lane < 4 * kItems ? static_cast<int>(t.equal[lane]) : 0;
+        equal_before = scan_lanes(c) - c;
+    }
+#pragma unroll
+    for (int e = 0; e < kItems; ++e) {
+        uint64_t take;
+        if (ties < c_equal) {
+            const uint64_t eq = __builtin_amdgcn_ballot_w64(key[e] == thr);
+            const int rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(eq >> 32),
+                                                       __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(eq), __builtin_amdgcn_readlane(equal_before, 4 * e + wave)));
+            take = __builtin_amdgcn_ballot_w64(key[e] > thr || (key[e] == thr && rank < ties));
+        } else {
+            take = __builtin_amdgcn_ballot_w64(key[e] >= thr);
+        }
+        if (lane == 0) t.words[4 * e + wave] = take;
+    }
+    __syncthreads();
+    return lane < 4 * kItems ? t.words[lane] : 0ull;
+}
+
+// kSelect (four wavefronts only): the selection is made here, from block scores
+template <bool kDirect, int kWaves, bool kSelect>
 __global__ __launch_bounds__(64 * kWaves)
 void decode_split_kernel(const DecodeParams p) {
     constexpr int kSlots = kWaves == 1 ? 2 : 1;                // block tiles per wavefront
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    __shared__ __attribute__((aligned(16))) elem_bits new_row[2 * kHeadDim];        // K, then V
-    __shared__ int lists[kWaves][64];                          // the wavefronts' blocks
-    uint64_t* words = reinterpret_cast<uint64_t*>(smem + kWaves * kSlots * kSlotBytes);     // the row's mask words, clipped to the sequence
+    __shared__ __attribute__((aligned(16))) elem_bits new_rows[kWaves][2 * kHeadDim];       // K, then V: a copy per wavefront
+    uint64_t* words = reinterpret_cast<uint64_t*>(smem + kWaves * kSlots * kSlotBytes);     // more than 64 mask words: the row's, clipped to the sequence
+    warm_kernel_arguments<sizeof(DecodeParams)>();
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
     const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-    int* list = lists[wave];
+    elem_bits* new_row = new_rows[wave];
+    unsigned char* tiles = smem + wave * kSlots * kSlotBytes;
     const int64_t pair = static_cast<int64_t>(b) * p.num_heads_k + h;
-    const bool listed = p.mask != nullptr || p.topk_idx != nullptr;                 // else: every block
-    uint64_t first_word = 0ull;                                // mask word tid
-    int first_idx = -1;                                        // or list entry tid
-    if (p.mask != nullptr && tid < p.n64) first_word = p.mask[pair * p.n64 + tid];
-    if (p.topk_idx != nullptr && tid < p.k_idx) first_idx = p.topk_idx[pair * p.k_idx + tid];
+    const bool listed = kSelect || p.mask != nullptr || p.topk_idx != nullptr;      // else: every block
+    uint64_t bits0 = 0ull;                                     // mask word `lane` of the row
+    int first_idx = -1;                                        // or list entry `lane`
+    if (!kSelect && p.mask != nullptr && lane < p.n64) bits0 = p.mask[pair * p.n64 + lane];
+    if (!kSelect && p.topk_idx != nullptr && lane < p.k_idx) first_idx = p.topk_idx[pair * p.k_idx + lane];
     const int seqlen = p.cache_seqlens ? p.cache_seqlens[b] : p.capacity - p.seqlen_new;
     const int lp = p.leftpad ? p.leftpad[b] : 0;              // the sequence's key 0 is cache row lp
     // position of the first appended key; a full cache takes no key, and the tables need not reach beyond it
     const int rot_pos = !p.cache_seqlens ? 0 : (seqlen < p.capacity ? seqlen : p.capacity - 1);
-    if (p.append_here && wave == 0) {
+    if (p.append_here) {
         // lanes 0..15: the new K row, lanes 16..31: the new V row, 16 bytes each
         const int chunk = n;
         uint4 val = make_uint4(0, 0, 0, 0);
@@ -246,7 +360,7 @@ void decode_split_kernel(const DecodeParams p) {
     const int new_key = (p.append_here && seqlen < p.capacity) ? seqlen - lp : -1;  // its index in the sequence
     const int last_blk = L <= 0 ? -1 : ((L - 1) >> 6);
     int n_words = last_blk < 0 ? 0 : (last_blk >> 6) + 1;
-    if (listed && n_words > p.n64) n_words = p.n64;
+    if (listed && !kSelect && n_words > p.n64) n_words = p.n64;
 
     elem8 qf[4];
     {
@@ -270,54 +384,72 @@ void decode_split_kernel(const DecodeParams p) {
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     };
-    auto group_fence = [&]() {
-        if constexpr (kWaves > 1) __syncthreads();
-        else lds_fence();
-    };
-    // bits of words w0 + lane: how many lie in words up to and including this lane's, among the 64 words from w0 on
+    // bits of words w0 + lane, and how many bits lie in words up to and including this lane's, from word w0 on
     auto scan_words = [&](int w0, uint64_t& bits) -> int {
         bits = w0 + lane < n_words ? words[w0 + lane] : 0ull;
-        int incl = __builtin_popcountll(bits);
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int o = __shfl_up(incl, off);
-            if (lane >= off) incl += o;
-        }
-        return incl;
+        return scan_lanes(__builtin_popcountll(bits));
     };
     int total = 0, incl0 = 0;                                  // incl0, bits0: the first 64 words
-    uint64_t bits0 = 0ull;
-    if (!listed) {
-        total = last_blk + 1;
-        group_fence();
-    } else {
-        if (p.mask != nullptr) {
-            const uint64_t last_word_bits = (last_blk & 63) == 63 ? ~0ull : ((1ull << ((last_blk & 63) + 1)) - 1ull);
-            for (int w = tid; w < n_words; w += 64 * kWaves) {
-                const uint64_t v = w == tid ? first_word : p.mask[pair * p.n64 + w];
-                words[w] = w == (last_blk >> 6) ? v & last_word_bits : v;
-            }
-        } else {
-            for (int w = tid; w < n_words; w += 64 * kWaves) words[w] = 0ull;
-            group_fence();
-            for (int i = tid; i < p.k_idx; i += 64 * kWaves) {
-                const int j = i == tid ? first_idx : p.topk_idx[pair * p.k_idx + i];
-                if (j >= 0 && j <= last_blk && (j >> 6) < n_words)
-                    atomicOr(reinterpret_cast<unsigned long long*>(&words[j >> 6]), 1ull << (j & 63));
-            }
-        }
-        group_fence();
-        incl0 = scan_words(0, bits0);
+    if constexpr (kSelect) {
+        // blocks of the sequence only: the columns beyond them, if any, would lose to every one of them or be dropped
+        int cols = last_blk + 1 < p.n_scores ? last_blk + 1 : p.n_scores;
+        cols = __builtin_amdgcn_readfirstlane(cols < 0 ? 0 : cols);
+        __shared__ __attribute__((aligned(16))) SelectScratch scratch_words;
+        const elem_bits* row = p.scores + pair * p.n_scores;
+        if (p.n_scores <= 512) bits0 = select_words<2>(row, p.n_scores, cols, p.k_select, scratch_words, tid, wave, lane);
+        else bits0 = select_words<8>(row, p.n_scores, cols, p.k_select, scratch_words, tid, wave, lane);
+        incl0 = scan_lanes(__builtin_popcountll(bits0));
         total = __builtin_amdgcn_readlane(incl0, 63);
-        for (int w0 = 64; w0 < n_words; w0 += 64) {
-            uint64_t bits;
-            total += __builtin_amdgcn_readlane(scan_words(w0, bits), 63);
+        lds_fence();
+    } else if (!listed) {
+        total = last_blk + 1;
+        lds_fence();
+    } else {
+        const uint64_t last_word_bits = (last_blk & 63) == 63 ? ~0ull : ((1ull << ((last_blk & 63) + 1)) - 1ull);
+        if (p.mask != nullptr && n_words <= 64) {              // straight into registers
+            bits0 = lane < n_words ? (lane == (last_blk >> 6) ? bits0 & last_word_bits : bits0) : 0ull;
+            incl0 = scan_lanes(__builtin_popcountll(bits0));
+            lds_fence();
+        } else {
+            // words in LDS: up to 64 in the wavefront's own tile (no barrier), more in an area shared by the workgroup
+            const bool shared = kWaves > 1 && n_words > 64;
+            if (n_words <= 64) words = reinterpret_cast<uint64_t*>(tiles);
+            const int first = shared ? tid : lane, step = shared ? 64 * kWaves : 64;
+            auto words_fence = [&]() {
+                if (shared) __syncthreads();
+                else lds_fence();
+            };
+            if (p.mask != nullptr) {
+                for (int w = first; w < n_words; w += step) {
+                    const uint64_t v = p.mask[pair * p.n64 + w];
+                    words[w] = w == (last_blk >> 6) ? v & last_word_bits : v;
+                }
+            } else {
+                for (int w = first; w < n_words; w += step) words[w] = 0ull;
+                words_fence();
+                for (int i = first; i < p.k_idx; i += step) {
+                    const int j = i == lane ? first_idx : p.topk_idx[pair * p.k_idx + i];
+                    if (j >= 0 && j <= last_blk && (j >> 6) < n_words)
+                        atomicOr(reinterpret_cast<unsigned long long*>(&words[j >> 6]), 1ull << (j & 63));
+                }
+            }
+            words_fence();
+            incl0 = scan_words(0, bits0);
+            for (int w0 = 64; w0 < n_words; w0 += 64) {
+                uint64_t bits;
+                total += __builtin_amdgcn_readlane(scan_words(w0, bits), 63);
+            }
+            lds_fence();
         }
+        total += __builtin_amdgcn_readlane(incl0, 63);
     }
     // equal runs: their lengths differ by one at most
     const int runs = p.splits * kWaves, run = split * kWaves + wave;
-    const int begin = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(total) * run / runs);
-    const int count = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(total) * (run + 1) / runs) - begin;
+    int each = static_cast<int>(static_cast<float>(total) * __builtin_amdgcn_rcpf(static_cast<float>(runs)));       // total / runs (total < 2^20), off by one at most
+    each = __builtin_amdgcn_readfirstlane(each);
+    each += (each + 1) * runs <= total ? 1 : (each * runs > total ? -1 : 0);
+    const int longer = total - each * runs;                    // so many runs take one block more
+    const int begin = run * each + (run < longer ? run : longer), count = each + (run < longer ? 1 : 0);
 
     // Blocks [base, base + 64) of this run, one per lane, and the cache row (page) they lie in.
     const int cache_row = p.block_table ? 0 : (p.cache_batch_idx ? p.cache_batch_idx[b] : b);
@@ -327,25 +459,26 @@ void decode_split_kernel(const DecodeParams p) {
         if (!listed) {
             my_block = lo + lane;
         } else {
-            int passed = 0;                                    // set bits of the words looked at so far
-            for (int w0 = 0; passed < hi; w0 += 64) {          // hi <= total: some word holds the last one
+            // by scalar instructions, a few per block: runs are short, and every lane's block would need as many
+            int ord = lo, passed = 0;                          // passed: set bits of the words before w0
+            for (int w0 = 0; ord < hi; w0 += 64) {             // hi <= total: some word holds the last one
                 uint64_t bits = bits0;
                 const int incl = w0 == 0 ? incl0 : scan_words(w0, bits);
-                const int c = __builtin_popcountll(bits);
-                int ord = passed + incl - c;
-                if (ord + c > lo && ord < hi) {
-                    if (ord < lo) {                            // the run starts inside this word
-                        bits &= ~0ull << nth_set_bit(bits, lo - ord);
-                        ord = lo;
-                    }
-                    for (; bits != 0ull && ord < hi; bits &= bits - 1ull, ++ord)
-                        list[ord - lo] = (w0 + lane) * 64 + __builtin_ctzll(bits);
+                const int upto = passed + __builtin_amdgcn_readlane(incl, 63);
+                uint64_t left = __builtin_amdgcn_ballot_w64(passed + incl > ord);  // words that still hold bits of the run
+                while (ord < hi && ord < upto) {
+                    const int w = __builtin_ctzll(left);
+                    left &= left - 1ull;
+                    const int w_upto = passed + __builtin_amdgcn_readlane(incl, w);
+                    uint64_t v = (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<uint32_t>(bits >> 32), w))) << 32) |
+                                 static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<uint32_t>(bits), w));
+                    const int skip = ord - (w_upto - static_cast<int>(__builtin_popcountll(v)));
+                    if (skip > 0) v = drop_set_bits(v, skip);  // the run starts inside this word
+                    for (; v != 0ull && ord < hi; v &= v - 1ull, ++ord)
+                        my_block = lane == ord - lo ? (w0 + w) * 64 + __builtin_ctzll(v) : my_block;
                 }
-                passed += __builtin_amdgcn_readlane(incl, 63);
+                passed = upto;
             }
-            lds_fence();
-            my_block = list[lane];
-            lds_fence();
         }
         if (p.block_table && base + lane < count) my_page = p.block_table[b * p.bt_batch + my_block * kBlockN / p.page_size];
     };
@@ -357,7 +490,6 @@ void decode_split_kernel(const DecodeParams p) {
     for (int dt = 0; dt < 8; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     // ---- block i of the run into slot i % kSlots ----
-    unsigned char* tiles = smem + wave * kSlots * kSlotBytes;
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(decode_lds_address(tiles));
     const int k_pitch = static_cast<int>(p.kc_row) * 2, v_pitch = static_cast<int>(p.vc_row) * 2;   // bytes
     uint32_t k_off[4], v_off[4];                               // this lane's piece of rows g, 4 + g, 8 + g, 12 + g
@@ -655,8 +787,8 @@ extern "C" size_t infllmv2_fwd_kvcache_workspace_bytes(int batch, int num_heads_
 
 static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vcache, const void* k_new,
                                     const void* v_new, const int32_t* cache_seqlens, void* out, float* softmax_lse,
-                                    const uint64_t* blockmask, const int32_t* topk_idx, int k_idx, void* workspace,
-                                    size_t workspace_bytes, int batch,
+                                    const uint64_t* blockmask, const int32_t* topk_idx, int k_idx, const void* scores, int n_scores,
+                                    int k_select, void* workspace, size_t workspace_bytes, int batch,
                                     int seqlen_q, int num_heads, int num_heads_k, int head_dim, int cache_capacity,
                                     int seqlen_new, const int64_t* q_strides, const int64_t* kcache_strides,
                                     const int64_t* vcache_strides, const int64_t* knew_strides,
@@ -728,11 +860,15 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
     p.rot_cos = static_cast<const elem_bits*>(rotary_cos); p.rot_sin = static_cast<const elem_bits*>(rotary_sin);
     p.rotary_dim = rotary_cos ? rotary_dim : 0; p.rotary_interleaved = rotary_interleaved;
     p.topk_idx = topk_idx; p.k_idx = k_idx;
+    p.scores = static_cast<const elem_bits*>(scores); p.n_scores = n_scores; p.k_select = k_select;
     if (topk_idx != nullptr) p.n64 = ((cache_capacity + kBlockN - 1) / kBlockN + 63) / 64;
     // mask words of one row, kept in LDS beside the tiles; 8192 words are 33 million tokens, 2048 still fit beside four tiles
     const size_t words = (blockmask || topk_idx) ? static_cast<size_t>(((cache_capacity + kBlockN - 1) / kBlockN + 63) / 64) : 0;
     IV2_CHECK(words <= 8192, "fwd_kvcache: a cache of %d rows needs more mask words than the kernel holds", cache_capacity);
     const bool grouped = static_cast<int64_t>(batch) * num_heads_k * num_splits <= kGroupedWorkgroups && words <= 2048;
+    IV2_CHECK(scores == nullptr || (grouped && n_scores > 0 && n_scores <= INFLLMV2_DECODE_MAX_SCORES && k_select > 0),
+              "fwd_kvcache_scores: 1 to %d block scores per row, topk >= 1 and at most %d (sequence, KV head, split) triples are served",
+              INFLLMV2_DECODE_MAX_SCORES, kGroupedWorkgroups);
     const size_t lds = (grouped ? 4 : 2) * static_cast<size_t>(kSlotBytes) + words * sizeof(uint64_t);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (k_new != nullptr) {
@@ -755,8 +891,10 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
         p.o_part = ws;
         p.lse_part = ws + static_cast<size_t>(batch) * num_heads_k * num_splits * 16 * kHeadDim;
     }
-    void (*split_kernel)(DecodeParams) = num_splits == 1 ? (grouped ? decode_split_kernel<true, 4> : decode_split_kernel<true, 1>)
-                                                         : (grouped ? decode_split_kernel<false, 4> : decode_split_kernel<false, 1>);
+    void (*split_kernel)(DecodeParams);
+    if (scores != nullptr) split_kernel = num_splits == 1 ? decode_split_kernel<true, 4, true> : decode_split_kernel<false, 4, true>;
+    else if (grouped) split_kernel = num_splits == 1 ? decode_split_kernel<true, 4, false> : decode_split_kernel<false, 4, false>;
+    else split_kernel = num_splits == 1 ? decode_split_kernel<true, 1, false> : decode_split_kernel<false, 1, false>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(split_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     IV2_CHECK(e == hipSuccess, "fwd_kvcache: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
     hipLaunchKernelGGL(split_kernel, dim3(num_splits, num_heads_k, batch), dim3(grouped ? 256 : 64), lds, st, p);
@@ -782,7 +920,7 @@ extern "C" int IV2_ENTRY(infllmv2_fwd_kvcache)(void* stream, const void* q, void
                                     const int32_t* cache_leftpad, const int32_t* block_table,
                                     int64_t block_table_batch_stride, int page_block_size, const void* rotary_cos,
                                     const void* rotary_sin, int rotary_dim, int rotary_interleaved) {
-    return fwd_kvcache_impl(stream, q, kcache, vcache, k_new, v_new, cache_seqlens, out, softmax_lse, blockmask, nullptr, 0,
+    return fwd_kvcache_impl(stream, q, kcache, vcache, k_new, v_new, cache_seqlens, out, softmax_lse, blockmask, nullptr, 0, nullptr, 0, 0,
                             workspace, workspace_bytes, batch, seqlen_q, num_heads, num_heads_k, head_dim, cache_capacity, seqlen_new,
                             q_strides, kcache_strides, vcache_strides, knew_strides, vnew_strides, o_strides,
                             n_uint64_per_row, num_splits, softmax_scale, cache_batch_idx, cache_leftpad, block_table,
@@ -802,11 +940,24 @@ extern "C" int IV2_ENTRY(infllmv2_fwd_kvcache_topk)(void* stream, const void* q,
                                          int64_t block_table_batch_stride, int page_block_size, const void* rotary_cos,
                                          const void* rotary_sin, int rotary_dim, int rotary_interleaved) {
     IV2_CHECK(topk_idx != nullptr, "fwd_kvcache_topk: null pointer");
-    return fwd_kvcache_impl(stream, q, kcache, vcache, k_new, v_new, cache_seqlens, out, softmax_lse, nullptr, topk_idx, k_idx,
+    return fwd_kvcache_impl(stream, q, kcache, vcache, k_new, v_new, cache_seqlens, out, softmax_lse, nullptr, topk_idx, k_idx, nullptr, 0, 0,
                             workspace, workspace_bytes, batch, seqlen_q, num_heads, num_heads_k, head_dim, cache_capacity,
                             seqlen_new, q_strides, kcache_strides, vcache_strides, knew_strides, vnew_strides, o_strides, 0,
                             num_splits, softmax_scale, cache_batch_idx, cache_leftpad, block_table, block_table_batch_stride,
                             page_block_size, rotary_cos, rotary_sin, rotary_dim, rotary_interleaved);
+}
+
+extern "C" int IV2_ENTRY(infllmv2_fwd_kvcache_scores)(void* stream, const void* q, void* kcache, void* vcache, const int32_t* cache_seqlens,
+                                         void* out, float* softmax_lse, const void* scores, int n_scores, int topk, void* workspace,
+                                         size_t workspace_bytes, int batch, int num_heads, int num_heads_k, int head_dim,
+                                         int cache_capacity, const int64_t* q_strides, const int64_t* kcache_strides,
+                                         const int64_t* vcache_strides, const int64_t* o_strides, int num_splits, float softmax_scale) {
+    IV2_CHECK(scores != nullptr, "fwd_kvcache_scores: null pointer");
+    const int64_t none[3] = {0, 0, 0};
+    return fwd_kvcache_impl(stream, q, kcache, vcache, nullptr, nullptr, cache_seqlens, out, softmax_lse, nullptr, nullptr, 0, scores,
+                            n_scores, topk, workspace, workspace_bytes, batch, 1, num_heads, num_heads_k, head_dim, cache_capacity, 0,
+                            q_strides, kcache_strides, vcache_strides, none, none, o_strides, 0, num_splits, softmax_scale, nullptr,
+                            nullptr, nullptr, 0, 0, nullptr, nullptr, 0, 0);
 }
 
 #ifndef IV2_F16        // one such entry point in the library: bfloat16 only
@@ -868,7 +1019,7 @@ extern "C" int infllmv2_fwd_kvcache_static(void* stream, const void* q, void* kc
         }
         ws = g_scratch_ptr[dev];
     }
-    return fwd_kvcache_impl(stream, q, kcache, vcache, k_new, v_new, cache_seqlens, out, softmax_lse, blockmask, nullptr, 0, ws,
+    return fwd_kvcache_impl(stream, q, kcache, vcache, k_new, v_new, cache_seqlens, out, softmax_lse, blockmask, nullptr, 0, nullptr, 0, 0, ws,
                             static_cast<size_t>(INFLLMV2_STATIC_SCRATCH_BYTES), batch, seqlen_q, num_heads, num_heads_k,
                             head_dim, cache_capacity, seqlen_new, q_strides, kcache_strides, vcache_strides, knew_strides,
                             vnew_strides, o_strides, n_uint64_per_row, num_splits, softmax_scale, cache_batch_idx,

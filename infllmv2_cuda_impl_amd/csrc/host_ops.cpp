@@ -461,6 +461,11 @@ OptTensor int32_vec(const OptTensor& t, int64_t batch, const char* name) {
     return t->contiguous();
 }
 
+// splits of rows of at most `blocks` blocks: no more than leave each of a workgroup's four wavefronts one
+int decode_splits(int64_t batch, int64_t hk, int64_t blocks) {
+    return as_int(std::min<int64_t>(infllmv2_fwd_kvcache_num_splits(as_int(batch), as_int(hk), 0), std::max<int64_t>(1, (blocks + 3) / 4)));
+}
+
 // topk_idx (batch, Hk, 1, k) int32 or block_mask (batch, Hk, 1, words) int64, or neither (dense).  Returns {out, lse}.
 std::tuple<Tensor, Tensor> fwd_kvcache(const Tensor& q, const Tensor& kc, const Tensor& vc, const OptTensor& kn, const OptTensor& vn,
                                        const OptTensor& seqlens_, double scale, int64_t num_splits, const OptTensor& topk_idx_,
@@ -545,9 +550,8 @@ std::tuple<Tensor, Tensor> fwd_kvcache(const Tensor& q, const Tensor& kc, const 
     DeviceGuard guard(q.device());
     Tensor out = at::empty_like(q);
     Tensor lse = at::empty({batch, hq, 1}, q.options().dtype(at::kFloat));
-    int splits = infllmv2_fwd_kvcache_num_splits(as_int(batch), as_int(hk), as_int(num_splits));
-    // no more splits than leave each of a workgroup's four wavefronts a block (a caller's own count stands)
-    if (num_splits <= 0 && idx.has_value()) splits = as_int(std::min<int64_t>(splits, std::max<int64_t>(1, (idx->size(3) + 3) / 4)));
+    const int splits = num_splits <= 0 && idx.has_value() ? decode_splits(batch, hk, idx->size(3))
+                                                          : infllmv2_fwd_kvcache_num_splits(as_int(batch), as_int(hk), as_int(num_splits));
     Tensor ws = bytes_on(q, infllmv2_fwd_kvcache_workspace_bytes(as_int(batch), as_int(hk), splits));
     const int64_t qs[2] = {q.stride(0), q.stride(2)}, os[2] = {out.stride(0), out.stride(2)};
     const S3 kcs = batch_rows_heads(kc), vcs = batch_rows_heads(vc);
@@ -571,14 +575,14 @@ std::tuple<Tensor, Tensor> fwd_kvcache(const Tensor& q, const Tensor& kc, const 
     return {out, lse};
 }
 
-// One decode step of a layer for a batch of sequences: append the token, extend the compressed keys, and - with
-// topk > 0 - Stage 1, pooling and top-k.  lens: tokens held (device), or none: host_len for every sequence.  max_len
-// bounds the lengths after the step.  Returns {lengths after the step, mask (batch, Hk, 1, words) or none}.
-std::tuple<Tensor, OptTensor> decode_step(const Tensor& q, const Tensor& kn, const Tensor& vn, const Tensor& kc, const Tensor& vc,
-                                          const Tensor& fine, const Tensor& coarse, const OptTensor& lens, int64_t host_len,
-                                          const OptTensor& fine_lens_, const OptTensor& coarse_lens_, int64_t max_len, int64_t kernel_size,
-                                          int64_t stride, int64_t block_size, int64_t topk, int64_t local_blocks, int64_t init_blocks,
-                                          double scale) {
+// The front of a decode step of a layer for a batch of sequences: append the token, extend the compressed keys, and - with
+// scores - Stage 1 and pooling.  lens: tokens held (device), or none: host_len for every sequence.  max_len bounds the
+// lengths after the step.  Returns {lengths after the step, block scores (batch, Hk, blocks) or an undefined tensor}.
+std::tuple<Tensor, Tensor> decode_front(const Tensor& q, const Tensor& kn, const Tensor& vn, const Tensor& kc, const Tensor& vc,
+                                        const Tensor& fine, const Tensor& coarse, const OptTensor& lens, int64_t host_len,
+                                        const OptTensor& fine_lens_, const OptTensor& coarse_lens_, int64_t max_len, int64_t kernel_size,
+                                        int64_t stride, int64_t block_size, bool scores, int64_t local_blocks, int64_t init_blocks,
+                                        double scale) {
     require_gpu(q, "q"); require_gpu(kc, "k_cache");
     require_16bit(q);
     for (const Tensor* t : {&kn, &vn, &kc, &vc, &fine, &coarse}) {
@@ -600,15 +604,14 @@ std::tuple<Tensor, OptTensor> decode_step(const Tensor& q, const Tensor& kn, con
     for (const OptTensor* t : {&lens, &fine_lens_, &coarse_lens_})
         TORCH_CHECK(!t->has_value() || ((*t)->scalar_type() == at::kInt && (*t)->dim() == 1 && (*t)->size(0) == batch && (*t)->is_contiguous() &&
                                         (*t)->device() == q.device()), "lengths must be contiguous int32 tensors of shape (batch_size)");
-    TORCH_CHECK(block_size == kBlock && (topk <= 0 || (stride * 4 == block_size)), "only 64-token blocks over stride-16 compressed keys are fused");
-    DeviceGuard guard(q.device());
+    TORCH_CHECK(block_size == kBlock && (!scores || (stride * 4 == block_size)), "only 64-token blocks over stride-16 compressed keys are fused");
     const auto ints = q.options().dtype(at::kInt);
     Tensor new_lens = at::empty({batch}, ints);
     const Tensor fine_lens = fine_lens_.has_value() ? *fine_lens_ : at::empty({batch}, ints);
     const Tensor coarse_lens = coarse_lens_.has_value() ? *coarse_lens_ : at::empty({batch}, ints);
     const int64_t out_len = (max_len + block_size - 1) / block_size;
     Tensor pooled, ws;
-    if (topk > 0) {
+    if (scores) {
         pooled = at::empty({batch, hk, out_len}, q.options());
         const int64_t max_f = std::min(windows(max_len, kernel_size, stride), fine.size(1));
         const int64_t max_c = std::min(windows(max_len, 4 * kernel_size, 4 * stride), coarse.size(1));
@@ -620,13 +623,56 @@ std::tuple<Tensor, OptTensor> decode_step(const Tensor& q, const Tensor& kn, con
     auto fn = is_half(q) ? infllmv2_decode_step_scores_f16 : infllmv2_decode_step_scores;
     check_rc(fn(stream_of(q), ptr(q), ptr(kn), ptr(vn), ptr(kc), ptr(vc), ptr(fine), ptr(coarse), iptr(lens), as_int(host_len),
                 static_cast<int32_t*>(ptr(new_lens)), static_cast<int32_t*>(ptr(fine_lens)), static_cast<int32_t*>(ptr(coarse_lens)),
-                topk > 0 ? ptr(pooled) : nullptr, topk > 0 ? ptr(ws) : nullptr, topk > 0 ? static_cast<size_t>(ws.numel()) : 0, as_int(batch),
+                scores ? ptr(pooled) : nullptr, scores ? ptr(ws) : nullptr, scores ? static_cast<size_t>(ws.numel()) : 0, as_int(batch),
                 as_int(hq), as_int(hk), as_int(d), as_int(cap), as_int(fine.size(1)), as_int(coarse.size(1)), as_int(max_len), qs, kns, vns,
                 kcs.v, vcs.v, fs.v, cs.v, as_int(kernel_size), as_int(stride), as_int(4 * kernel_size), as_int(4 * stride),
                 static_cast<float>(scale), as_int(out_len), as_int(local_blocks), as_int(init_blocks)), "decode_step_scores");
+    return {new_lens, pooled};
+}
+
+// The front and, with topk > 0, the selection.  Returns {lengths after the step, mask (batch, Hk, 1, words) or none}.
+std::tuple<Tensor, OptTensor> decode_step(const Tensor& q, const Tensor& kn, const Tensor& vn, const Tensor& kc, const Tensor& vc,
+                                          const Tensor& fine, const Tensor& coarse, const OptTensor& lens, int64_t host_len,
+                                          const OptTensor& fine_lens, const OptTensor& coarse_lens, int64_t max_len, int64_t kernel_size,
+                                          int64_t stride, int64_t block_size, int64_t topk, int64_t local_blocks, int64_t init_blocks,
+                                          double scale) {
+    DeviceGuard guard(q.device());
+    auto [new_lens, pooled] = decode_front(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, max_len, kernel_size,
+                                           stride, block_size, topk > 0, local_blocks, init_blocks, scale);
     if (topk <= 0) return {new_lens, std::nullopt};
     auto [idx, mask] = topk_blocks(pooled, topk, true, true, false, std::nullopt);
     return {new_lens, mask->unsqueeze(2)};
+}
+
+// A whole decode step on selected blocks: the front, the selection and the attention.  The selection is made by the
+// attention's own launch where that serves it (a workgroup per CU at most, rows of 2048 block scores at most: see
+// infllmv2_fwd_kvcache_scores), by a top-k launch otherwise.  Returns {out, lengths after the step}.
+std::tuple<Tensor, Tensor> decode_sparse(const Tensor& q, const Tensor& kn, const Tensor& vn, const Tensor& kc, const Tensor& vc,
+                                         const Tensor& fine, const Tensor& coarse, const OptTensor& lens, int64_t host_len,
+                                         const OptTensor& fine_lens, const OptTensor& coarse_lens, int64_t max_len, int64_t kernel_size,
+                                         int64_t stride, int64_t block_size, int64_t topk, int64_t local_blocks, int64_t init_blocks,
+                                         double scale) {
+    TORCH_CHECK(topk > 0, "decode_sparse: topk must be positive");
+    DeviceGuard guard(q.device());
+    auto [new_lens, pooled] = decode_front(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, max_len, kernel_size,
+                                           stride, block_size, true, local_blocks, init_blocks, scale);
+    const int64_t batch = q.size(0), hq = q.size(2), hk = kc.size(2), n = pooled.size(2);
+    const int splits = decode_splits(batch, hk, topk);
+    if (batch * hk * splits > 256 || n > INFLLMV2_DECODE_MAX_SCORES) {
+        auto [idx, mask] = topk_blocks(pooled, topk, true, true, false, std::nullopt);
+        return {std::get<0>(fwd_kvcache(q, kc, vc, std::nullopt, std::nullopt, new_lens, scale, 0, std::nullopt, mask->unsqueeze(2), std::nullopt,
+                                        std::nullopt, std::nullopt, std::nullopt, std::nullopt, false)), new_lens};
+    }
+    Tensor out = at::empty_like(q);
+    const size_t partials = infllmv2_fwd_kvcache_workspace_bytes(as_int(batch), as_int(hk), splits), lse_bytes = sizeof(float) * batch * hq;
+    Tensor ws = bytes_on(q, partials + lse_bytes);
+    const int64_t qs[2] = {q.stride(0), q.stride(2)}, os[2] = {out.stride(0), out.stride(2)};
+    const S3 kcs = batch_rows_heads(kc), vcs = batch_rows_heads(vc);
+    auto fn = is_half(q) ? infllmv2_fwd_kvcache_scores_f16 : infllmv2_fwd_kvcache_scores;
+    check_rc(fn(stream_of(q), ptr(q), ptr(kc), ptr(vc), iptr(new_lens), ptr(out), reinterpret_cast<float*>(static_cast<char*>(ptr(ws)) + partials),
+                ptr(pooled), as_int(n), as_int(topk), ptr(ws), partials, as_int(batch), as_int(hq), as_int(hk), as_int(kHeadDim),
+                as_int(kc.size(1)), qs, kcs.v, vcs.v, os, splits, static_cast<float>(scale)), "fwd_kvcache_scores");
+    return {out, new_lens};
 }
 
 }  // namespace
@@ -647,4 +693,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("varlen_bwd", &varlen_bwd);
     m.def("fwd_kvcache", &fwd_kvcache);
     m.def("decode_step", &decode_step);
+    m.def("decode_sparse", &decode_sparse);
 }

@@ -145,14 +145,17 @@ class InfLLMv2Attention(torch.nn.Module):
                 compress_keys(cache.k[0, :n], cu, n, ks, st, out=buf, first_row=rows(old_length, ks, st))
 
     # ---- decode ----
-    def _step(self, q, k_new, v_new, k, v, k_fine, k_coarse, lens, host_len, fine_lens, coarse_lens, max_len):
-        """Append, compressed keys and (sparse branch) selection of one decode step: see :meth:`decode_batch`.  Returns the
-        lengths after the step (device) and the block mask ``(batch, nheads_k, 1, words)`` or None."""
-        scores = self.selection == "sparse" and max_len > self.dense_len
+    def _step(self, q, k_new, v_new, k, v, k_fine, k_coarse, lens, host_len, fine_lens, coarse_lens, max_len, window_mask):
+        """One decode step: append, compressed keys, selection, attention.  ``window_mask()`` gives the block mask
+        ``(batch, nheads_k, 1, words)`` of the window branch.  Returns the output and the lengths after the step (device)."""
         scale = q.shape[-1] ** (-0.5) if self.softmax_scale is None else self.softmax_scale
-        return _lib.host.decode_step(q, k_new, v_new, k, v, k_fine, k_coarse, lens, host_len, fine_lens, coarse_lens, max_len,
-                                     self.kernel_size, self.stride, self.block_size, self.topk if scores else 0, self.local_blocks,
-                                     self.init_blocks, scale)
+        step = (q, k_new, v_new, k, v, k_fine, k_coarse, lens, host_len, fine_lens, coarse_lens, max_len, self.kernel_size, self.stride,
+                self.block_size)
+        if self.selection == "sparse" and max_len > self.dense_len:
+            return _lib.host.decode_sparse(*step, self.topk, self.local_blocks, self.init_blocks, scale)
+        new, _ = _lib.host.decode_step(*step, 0, self.local_blocks, self.init_blocks, scale)
+        mask = window_mask() if self.selection == "window" and max_len > self.dense_len else None
+        return infllmv2_attn_with_kvcache(q, k, v, cache_seqlens=new, softmax_scale=self.softmax_scale, block_mask=mask), new
 
     def decode(self, q, k_new, v_new, cache: SequenceCache):
         """One token of one sequence: q ``(1, 1, nheads, d)``, k_new/v_new ``(1, 1, nheads_k, d)``.  Appends the token
@@ -163,15 +166,17 @@ class InfLLMv2Attention(torch.nn.Module):
             raise IndexError(f"index {pos} is out of bounds: the K/V cache holds {cache.k.shape[1]} tokens")
         n = pos + 1
         q, k_new, v_new = _dense(q), _dense(k_new), _dense(v_new)
-        lens, mask = self._step(q, k_new, v_new, cache.k, cache.v, cache.k_fine.unsqueeze(0), cache.k_coarse.unsqueeze(0), None, pos,
-                                None, None, n)
-        cache.length = n
-        if self.selection == "window" and n > self.dense_len:
+
+        def window_mask():
             dev = q.device
             _, mask = self._window_blocks(cache.k.shape[2], 1, torch.tensor([0, 1], dtype=torch.int32, device=dev),
                                           torch.tensor([pos], dtype=torch.int32, device=dev), 1, pos, dev)
-            mask = mask.transpose(0, 1).unsqueeze(2).contiguous()
-        return infllmv2_attn_with_kvcache(q, cache.k, cache.v, cache_seqlens=lens, softmax_scale=self.softmax_scale, block_mask=mask)
+            return mask.transpose(0, 1).unsqueeze(2).contiguous()
+
+        out, _ = self._step(q, k_new, v_new, cache.k, cache.v, cache.k_fine.unsqueeze(0), cache.k_coarse.unsqueeze(0), None, pos, None, None,
+                            n, window_mask)
+        cache.length = n
+        return out
 
     # ---- batched decode ----
     def fill_cache(self, cache: BatchCache, k, v, seqlens):
@@ -199,13 +204,14 @@ class InfLLMv2Attention(torch.nn.Module):
         if cache.max_length + 1 > cache.k.shape[1]:
             raise RuntimeError("the K/V cache is full")
         q, k_new, v_new = _dense(q), _dense(k_new), _dense(v_new)
-        new, mask = self._step(q, k_new, v_new, cache.k, cache.v, cache.k_fine, cache.k_coarse, cache.lengths, 0, cache.fine_lens,
-                               cache.coarse_lens, cache.max_length + 1)
-        if self.selection == "window" and cache.max_length + 1 > self.dense_len:
+
+        def window_mask():
             cu_one = torch.arange(batch + 1, dtype=torch.int32, device=q.device)
             _, mask = self._window_blocks(cache.k.shape[2], batch, cu_one, cache.lengths, 1, cache.max_length, q.device)
-            mask = mask.transpose(0, 1).unsqueeze(2).contiguous()                    # (Hk, batch, words) -> (batch, Hk, 1, words)
-        out = infllmv2_attn_with_kvcache(q, cache.k, cache.v, cache_seqlens=new, softmax_scale=self.softmax_scale, block_mask=mask)
+            return mask.transpose(0, 1).unsqueeze(2).contiguous()                    # (Hk, batch, words) -> (batch, Hk, 1, words)
+
+        out, new = self._step(q, k_new, v_new, cache.k, cache.v, cache.k_fine, cache.k_coarse, cache.lengths, 0, cache.fine_lens,
+                              cache.coarse_lens, cache.max_length + 1, window_mask)
         cache.lengths = new
         cache.max_length += 1
         return out

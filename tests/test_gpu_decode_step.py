@@ -132,3 +132,30 @@ def test_decode_runs_longer_than_one_look_up(held, masked):
         out = ops.infllmv2_attn_with_kvcache(q, k2, v2, k=kn, v=vn, cache_seqlens=L, num_splits=splits, block_mask=words)
         assert torch.equal(k2, kr) and torch.equal(v2, vr)
         assert (out[0, 0].float() - ref).abs().max() <= 1e-2 * max(1.0, float(ref.abs().max()))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("topk", [1, 3, 64, 300])
+@pytest.mark.parametrize("tied", [False, True])
+def test_selection_inside_the_attention_equals_topk(dtype, topk, tied):
+    """Whole steps against decode_step (top-k launch, mask) + infllmv2_attn_with_kvcache: rows of 1 to 2048 block scores, lengths
+    at the edges of 64 words and of 256 columns, and all scores equal (a zero query)."""
+    import infllmv2_cuda_impl_amd as ops
+    from infllmv2_cuda_impl_amd import _lib
+    lens = [0, 62, 63, 64 * 64 - 2, 64 * 64 - 1, 64 * 256 - 1, 64 * 256, 64 * 512 + 5, 131070]
+    cap, Hk, B = 131072, 1, len(lens)
+    g = torch.Generator(device="cuda").manual_seed(topk)
+    mk = lambda *s: torch.randn(*s, generator=g, device="cuda", dtype=dtype)
+    q, kn, vn = mk(B, 1, 16, 128) * (0 if tied else 1), mk(B, 1, Hk, 128), mk(B, 1, Hk, 128)
+    k, v = mk(B, cap, Hk, 128), mk(B, cap, Hk, 128)
+    L = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    fine, coarse = mk(B, cap // 16 + 1, Hk, 128), mk(B, cap // 64 + 1, Hk, 128)
+    fl, cl = ops.compress_keys_cache_pair(k, L, (32, 16, fine), (128, 64, coarse))
+    for s, max_len in ((slice(0, B), cap), (slice(0, 1), 1), (slice(3, 4), 64 * 64 - 1), (slice(5, 6), 64 * 256), (slice(6, 7), 64 * 256 + 1)):
+        step = (q[s], kn[s], vn[s], k[s], v[s], fine[s], coarse[s], L[s], 0, fl[s].clone(), cl[s].clone(), max_len, 32, 16, 64, topk, 2, 1,
+                128 ** -0.5)
+        out, n1 = _lib.host.decode_sparse(*step)
+        n2, mask = _lib.host.decode_step(*step[:9], fl[s].clone(), cl[s].clone(), *step[11:])
+        splits = min(_lib.lib.infllmv2_fwd_kvcache_num_splits(mask.shape[0], Hk, 0), (topk + 3) // 4)
+        want = ops.infllmv2_attn_with_kvcache(q[s], k[s], v[s], cache_seqlens=n2, block_mask=mask, num_splits=splits)
+        assert torch.equal(n1, n2) and torch.equal(out, want)
