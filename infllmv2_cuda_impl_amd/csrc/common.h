@@ -126,15 +126,16 @@ __device__ __forceinline__ float elem_hi_to_f32(uint32_t w) { return elem_to_f32
 // short kernel spends before its first request.
 template <int kBytes>
 __device__ __forceinline__ void warm_kernel_arguments() {
-    static_assert(kBytes >= 4 && kBytes <= 7 * 64, "more cache lines than are touched here");
+    static_assert(kBytes >= 4 && kBytes <= 9 * 64, "more cache lines than are touched here");
     constexpr int kLast = kBytes - 4;
     auto line = [](int i) constexpr { return 64 * i < kLast ? 64 * i : kLast; };
-    uint32_t a, b, c, d, e, f, g;
-    asm volatile("s_load_dword %0, %7, %8\n\ts_load_dword %1, %7, %9\n\ts_load_dword %2, %7, %10\n\ts_load_dword %3, %7, %11\n\t"
-                 "s_load_dword %4, %7, %12\n\ts_load_dword %5, %7, %13\n\ts_load_dword %6, %7, %14\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&s"(a), "=&s"(b), "=&s"(c), "=&s"(d), "=&s"(e), "=&s"(f), "=&s"(g)
+    uint32_t a, b, c, d, e, f, g, h, i;
+    asm volatile("s_load_dword %0, %9, %10\n\ts_load_dword %1, %9, %11\n\ts_load_dword %2, %9, %12\n\ts_load_dword %3, %9, %13\n\t"
+                 "s_load_dword %4, %9, %14\n\ts_load_dword %5, %9, %15\n\ts_load_dword %6, %9, %16\n\ts_load_dword %7, %9, %17\n\t"
+                 "s_load_dword %8, %9, %18\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&s"(a), "=&s"(b), "=&s"(c), "=&s"(d), "=&s"(e), "=&s"(f), "=&s"(g), "=&s"(h), "=&s"(i)
                  : "s"(__builtin_amdgcn_kernarg_segment_ptr()), "n"(line(0)), "n"(line(1)), "n"(line(2)), "n"(line(3)), "n"(line(4)),
-                   "n"(line(5)), "n"(kLast));
+                   "n"(line(5)), "n"(line(6)), "n"(line(7)), "n"(kLast));
 }
 
 }  // namespace IV2_NS

@@ -12,9 +12,9 @@
 // Shape of the work: per sequence and KV head the whole compressed-key set is read once (256 bytes per key) for 16
 // query rows, so the launch is bound by memory bandwidth and the stage1.hip kernel (one workgroup per 16 tokens,
 // keys staged for reuse by 16 tokens) is the wrong shape: it would stream every sequence through one workgroup.
-// Here the keys of one (sequence, KV head) are cut into runs of 64-key tiles, the same run length (two tiles unless
+// Here the keys of one (sequence, KV head) are cut into runs of 64-key tiles, the same run length (one or two tiles unless
 // the longest sequence would then need more than 64 runs) for every sequence of the batch, and every run goes to a
-// single-wavefront workgroup that loads its tiles straight into MFMA operand registers: long sequences get many
+// wavefront of its own that loads its tiles straight into MFMA operand registers: long sequences get many
 // workgroups, short ones few, and every workgroup carries the same load.
 // The log-sum-exp needs all coarse keys before any score can be normalised, so there are two launches:
 //   1. stage1_decode_lse_kernel: per run of coarse tiles the running (max, sum) of the 16 heads -> workspace;
@@ -113,6 +113,25 @@ __device__ __forceinline__ void s1d_run_fixed(int tiles, int per, int split, int
     t1 = t0 + per;
     t1 = t1 < tiles ? t1 : tiles;
 }
+__device__ __forceinline__ float s1d_quad_xor1(float x) {
+    return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0xB1, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float s1d_quad_xor2(float x) {
+    return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x4E, 0xF, 0xF, false));
+}
+// maximum and sum over the 16 lanes of a row, by DPP operands of the operations themselves (quad_perm, row_ror)
+__device__ __forceinline__ float s1d_row_max(float x) {
+    x = fmaxf(x, s1d_quad_xor1(x));
+    x = fmaxf(x, s1d_quad_xor2(x));
+    x = fmaxf(x, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x124, 0xF, 0xF, false)));
+    return fmaxf(x, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x128, 0xF, 0xF, false)));
+}
+__device__ __forceinline__ float s1d_row_sum(float x) {
+    x += s1d_quad_xor1(x);
+    x += s1d_quad_xor2(x);
+    x += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x124, 0xF, 0xF, false));
+    return x + __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x128, 0xF, 0xF, false));
+}
 // (max, sum) in log2 units of head 4g + e over the coarse tiles [t0, t1) of one sequence and KV head, merged over the
 // 16 key-column lanes: every lane of row g returns the values of its four heads.  patch(tile registers, tile) runs after
 // a tile is requested.
@@ -170,18 +189,8 @@ __device__ __forceinline__ void s1d_lse_run(const S1DecodeParams& p, const S1Dec
     // merge the 16 key-column lanes of each head
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        float mm = m[e], ll = l[e];
-#pragma unroll
-        for (int off = 1; off < 16; off <<= 1) {
-            const float mo = __shfl_xor(mm, off);
-            const float lo = __shfl_xor(ll, off);
-            const float mn = fmaxf(mm, mo);
-            const float mu = (mn == -INFINITY) ? 0.f : mn;
-            ll = ll * __builtin_amdgcn_exp2f(mm - mu) + lo * __builtin_amdgcn_exp2f(mo - mu);
-            mm = mn;
-        }
-        m_out[e] = mm;
-        l_out[e] = ll;
+        m_out[e] = s1d_row_max(m[e]);
+        l_out[e] = s1d_row_sum(l[e] * __builtin_amdgcn_exp2f(m[e] - (m_out[e] == -INFINITY ? 0.f : m_out[e])));
     }
 }
 
@@ -205,39 +214,24 @@ __device__ __forceinline__ void s1d_load_records(S1DRecords& r, const float* par
         for (int k = 1; k < 4; ++k) fetch(k);
     }
 }
-// log-sum-exp (log2 units) of head 4g + e from those records: each lane folds its own in run order, then the 16 lanes
-// of a row merge among themselves (the merge of (max, sum) pairs is associative and commutative up to rounding, and
-// every lane of a row ends with the same bits because the butterfly combines the same pairs in the same order on both
-// sides).
+// log-sum-exp (log2 units) of head 4g + e from those records: the row's maximum, then the sum of everything relative to it
+// (every lane of a row ends with the same bits).
 __device__ __forceinline__ void s1d_merge_records(const S1DRecords& r, int count, int n, int g, int group, float (&lse2)[4]) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        float mm = -INFINITY, ll = 0.f;
-        auto fold = [&](int k) {
-            const bool have = n + 16 * k < count;              // a record that is not there is the neutral element
-            const float mo = have ? r.m[k][e] : -INFINITY, lo = have ? r.l[k][e] : 0.f;
-            const float mn = fmaxf(mm, mo);
-            const float mu = (mn == -INFINITY) ? 0.f : mn;
-            ll = ll * __builtin_amdgcn_exp2f(mm - mu) + lo * __builtin_amdgcn_exp2f(mo - mu);
-            mm = mn;
-        };
-        fold(0);
+        float mm = n < count ? r.m[0][e] : -INFINITY;          // a record that is not there is the neutral element
         if (count > 16) {                                      // uniform
 #pragma unroll
-            for (int k = 1; k < 4; ++k) fold(k);
+            for (int k = 1; k < 4; ++k) mm = n + 16 * k < count ? fmaxf(mm, r.m[k][e]) : mm;
         }
+        mm = s1d_row_max(mm);
+        const float mu = mm == -INFINITY ? 0.f : mm;
+        float ll = n < count ? r.l[0][e] * __builtin_amdgcn_exp2f(r.m[0][e] - mu) : 0.f;
+        if (count > 16) {
 #pragma unroll
-        for (int off = 1; off < 16; off <<= 1) {
-            const float mo = __shfl_xor(mm, off);
-            const float lo = __shfl_xor(ll, off);
-            const float mn = fmaxf(mm, mo);
-            const float mu = (mn == -INFINITY) ? 0.f : mn;
-            // the same sum on both partners: add the term of the lane with the lower number first
-            const float mine = ll * __builtin_amdgcn_exp2f(mm - mu), theirs = lo * __builtin_amdgcn_exp2f(mo - mu);
-            ll = (n & off) ? theirs + mine : mine + theirs;
-            mm = mn;
+            for (int k = 1; k < 4; ++k) ll += n + 16 * k < count ? r.l[k][e] * __builtin_amdgcn_exp2f(r.m[k][e] - mu) : 0.f;
         }
-        lse2[e] = mm + __builtin_amdgcn_logf(ll);                // v_log_f32 is log2
+        lse2[e] = mm + __builtin_amdgcn_logf(s1d_row_sum(ll));   // v_log_f32 is log2
         if (4 * g + e >= group) lse2[e] = INFINITY;              // a row that only fills the tile adds exp2(x - inf) = 0
     }
 }
@@ -250,10 +244,13 @@ __device__ __forceinline__ void s1d_store_record(const S1DecodeParams& p, int b,
     for (int e = 0; e < 4; ++e) { slot[4 * g + e] = m[e]; slot[16 + 4 * g + e] = l[e]; }
 }
 
-__global__ __launch_bounds__(64)
+// Two wavefronts per workgroup, a run each: see the front kernel below.
+constexpr int kLseWaves = 2;
+__global__ __launch_bounds__(64 * kLseWaves)
 void stage1_decode_lse_kernel(const S1DecodeParams p) {
-    const int lane = threadIdx.x, n = lane & 15, g = lane >> 4;
-    const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+    warm_kernel_arguments<sizeof(S1DecodeParams)>();
+    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    const int split = blockIdx.x * kLseWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = blockIdx.y, b = blockIdx.z;
     const S1DecodeSeq sq = s1d_sequence(p, b, h);
     if (sq.Sq <= 0) return;
     const int s1 = (sq.Lk == sq.Lc) ? 16 : 64;                 // flash_fwd_kernel.h:1236-1240
@@ -307,97 +304,94 @@ __device__ __forceinline__ int s1d_step_rows(int len, int capacity, int kernel_s
     added = rows > first ? first : -1;
     return rows;
 }
-// Elements 2 lane and 2 lane + 1 of the mean of K rows [j stride, j stride + kernel_size) of one head: an fp32 sum in
-// window order divided by kernel_size, rounded once, as compress.hip computes it.  The window's last row is the new
-// token (that is why it is complete now) and comes from the caller.  Rows are requested 64 (32) at a time before they
-// are added up.
-__device__ __forceinline__ uint32_t s1d_window_mean(const S1DecodeStep& t, int b, int h, int j, int kernel_size, int stride, int lane) {
-    const elem_bits* row = t.kcache + b * t.kc_batch + static_cast<int64_t>(j) * stride * t.kc_row + h * t.kc_head + 2 * lane;
-    const uint32_t newest = *reinterpret_cast<const uint32_t*>(t.knew + b * t.kn_batch + h * t.kn_head + 2 * lane);
-    float lo = 0.f, hi = 0.f;
+// One column of the mean of K rows [j stride, j stride + kernel_size) of one head: an fp32 sum in window order divided by
+// kernel_size, rounded once, as compress.hip computes it.  The window's last row is the new token (that is why it is complete
+// now) and comes from the caller.  Rows are requested 64 (32) at a time before they are added up.  A column per lane, over two
+// wavefronts, because a lone wavefront is bound by the instructions it issues: two columns per lane, unpacked, took 640 of them.
+__device__ __forceinline__ elem_bits s1d_window_mean(const S1DecodeStep& t, int b, int h, int j, int kernel_size, int stride, int col) {
+    const elem_bits* row = t.kcache + b * t.kc_batch + static_cast<int64_t>(j) * stride * t.kc_row + h * t.kc_head + col;
+    const elem_bits newest = t.knew[b * t.kn_batch + h * t.kn_head + col];
+    float sum = 0.f;
     int left = kernel_size;
-    auto add = [&](uint32_t v) {
-        lo += elem_lo_to_f32(v);
-        hi += elem_hi_to_f32(v);
-    };
     auto chunk = [&](auto size) {
         constexpr int kRows = decltype(size)::value;
         for (; left >= kRows; left -= kRows) {
-            uint32_t w[kRows];
+            elem_bits w[kRows];
 #pragma unroll
             for (int i = 0; i < kRows; ++i) {
-                w[i] = *reinterpret_cast<const uint32_t*>(row);
+                w[i] = *row;
                 row += t.kc_row;
                 asm volatile("" : "+v"(row));                  // one running address, not one scalar pair per row
             }
             if (left == kRows) w[kRows - 1] = newest;
 #pragma unroll
-            for (int i = 0; i < kRows; ++i) add(w[i]);
+            for (int i = 0; i < kRows; ++i) sum += elem_to_f32(w[i]);
         }
     };
     chunk(std::integral_constant<int, 64>{});
     chunk(std::integral_constant<int, 32>{});
     chunk(std::integral_constant<int, 1>{});
-    const float n = static_cast<float>(kernel_size);
-    return pack_elem2(lo / n, hi / n);
+    return f32_to_elem_hw(sum / static_cast<float>(kernel_size));
 }
 
-__global__ __launch_bounds__(64)
+__global__ __launch_bounds__(64 * kLseWaves)
 void stage1_decode_front_kernel(const S1DecodeParams p, const S1DecodeStep t) {
-    __shared__ __attribute__((aligned(16))) uint32_t newest_key[kHeadDim / 2];      // the coarse key this token completes
-    const int lane = threadIdx.x, n = lane & 15, g = lane >> 4;
-    const int split = static_cast<int>(blockIdx.x) - 1, h = blockIdx.y, b = blockIdx.z;
+    __shared__ __attribute__((aligned(16))) elem_bits newest_key[kHeadDim];         // the coarse key this token completes
+    warm_kernel_arguments<sizeof(S1DecodeParams) + sizeof(S1DecodeStep)>();
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int first = (static_cast<int>(blockIdx.x) - 1) * kLseWaves, h = blockIdx.y, b = blockIdx.z;
     const int len = t.lens ? t.lens[b] : t.host_len;
     int add_f, add_c;
     const int rows_f = s1d_step_rows(len, t.capacity, t.kernel_f, t.stride_f, t.fine_capacity, add_f);
     const int rows_c = s1d_step_rows(len, t.capacity, t.kernel_c, t.stride_c, t.coarse_capacity, add_c);
-    if (split < 0) {                                           // the caches' keeper
-        if (len < t.capacity && g < 2) {
+    if (first < 0) {                                           // the caches' keepers
+        if (wave == 0 && len < t.capacity && g < 2) {
             const elem_bits* src = g == 0 ? t.knew + b * t.kn_batch + h * t.kn_head : t.vnew + b * t.vn_batch + h * t.vn_head;
             elem_bits* dst = g == 0 ? t.kcache + b * t.kc_batch + len * t.kc_row + h * t.kc_head
                                     : t.vcache + b * t.vc_batch + len * t.vc_row + h * t.vc_head;
             *reinterpret_cast<uint4*>(dst + 8 * n) = *reinterpret_cast<const uint4*>(src + 8 * n);
         }
-        if (h == 0 && lane == 0) {
+        if (h == 0 && tid == 0) {
             if (t.new_lens) t.new_lens[b] = len + 1;
             t.fine_lens[b] = rows_f;
             t.coarse_lens[b] = rows_c;
         }
         if (add_f >= 0)
-            reinterpret_cast<uint32_t*>(t.fine + b * p.k_batch_stride + add_f * p.k_row_stride + h * p.k_head_stride)[lane] =
-                s1d_window_mean(t, b, h, add_f, t.kernel_f, t.stride_f, lane);
+            t.fine[b * p.k_batch_stride + add_f * p.k_row_stride + h * p.k_head_stride + tid] =
+                s1d_window_mean(t, b, h, add_f, t.kernel_f, t.stride_f, tid);
         if (add_c >= 0 && !t.with_scores)
-            reinterpret_cast<uint32_t*>(t.coarse + b * p.c_batch_stride + add_c * p.c_row_stride + h * p.c_head_stride)[lane] =
-                s1d_window_mean(t, b, h, add_c, t.kernel_c, t.stride_c, lane);
+            t.coarse[b * p.c_batch_stride + add_c * p.c_row_stride + h * p.c_head_stride + tid] =
+                s1d_window_mean(t, b, h, add_c, t.kernel_c, t.stride_c, tid);
         return;
     }
+    const int tiles = (rows_c + 63) >> 6, split = first + wave;
+    if (first * p.run_c >= tiles && first > 0) return;         // beyond this sequence's runs; run 0 always leaves a record
     int t0, t1;
-    s1d_run_fixed((rows_c + 63) >> 6, p.run_c, split, t0, t1);
-    if (t0 >= t1 && split > 0) return;                         // beyond this sequence's runs; run 0 always leaves a record
+    s1d_run_fixed(tiles, p.run_c, split, t0, t1);
     S1DecodeSeq sq;
     sq.q_row = b; sq.Sq = 1; sq.Lk = rows_f; sq.Lc = rows_c;
     sq.kbase = nullptr;
     sq.cbase = p.c + b * p.c_batch_stride + h * p.c_head_stride;
     elem8 qf[4];
     s1d_load_q(qf, p, sq, h, n, g);
-    const bool adds = add_c >= 0 && add_c >= t0 * 64 && add_c < t1 * 64;            // uniform; add_c is the last key
+    // uniform over the workgroup; add_c is the last key
+    const bool adds = add_c >= 0 && (add_c >> 6) >= first * p.run_c && (add_c >> 6) < (first + kLseWaves) * p.run_c;
     if (adds) {
-        const uint32_t mean = s1d_window_mean(t, b, h, add_c, t.kernel_c, t.stride_c, lane);
-        reinterpret_cast<uint32_t*>(t.coarse + b * p.c_batch_stride + add_c * p.c_row_stride + h * p.c_head_stride)[lane] = mean;
-        newest_key[lane] = mean;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        const elem_bits mean = s1d_window_mean(t, b, h, add_c, t.kernel_c, t.stride_c, tid);
+        t.coarse[b * p.c_batch_stride + add_c * p.c_row_stride + h * p.c_head_stride + tid] = mean;
+        newest_key[tid] = mean;
+        __syncthreads();
     }
+    if (t0 >= t1 && split > 0) return;
     float mm[4], ll[4];
     s1d_lse_run(p, sq, qf, rows_c, t0, t1, n, g, mm, ll, [&](elem8 (&tile)[16], int ti) {
         if (!adds || ti != add_c >> 6) return;
-        const elem_bits* key = reinterpret_cast<const elem_bits*>(newest_key);
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt)
             if (ti * 64 + 16 * kt + n >= add_c) {              // the last key, and the lanes beyond it that repeat it
 #pragma unroll
-                for (int c = 0; c < 4; ++c) tile[kt * 4 + c] = *reinterpret_cast<const elem8*>(key + 32 * c + 8 * g);
+                for (int c = 0; c < 4; ++c) tile[kt * 4 + c] = *reinterpret_cast<const elem8*>(newest_key + 32 * c + 8 * g);
             }
     });
     s1d_store_record(p, b, h, split, mm, ll, n, g);
@@ -413,13 +407,6 @@ __device__ __forceinline__ float s1d_fold_rows32(float x, float y) {
     const u2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
-__device__ __forceinline__ float s1d_quad_xor1(float x) {
-    return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0xB1, 0xF, 0xF, false));
-}
-__device__ __forceinline__ float s1d_quad_xor2(float x) {
-    return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x4E, 0xF, 0xF, false));
-}
-
 // The 16 keys before tile t0 (the last group of tile t0 - 1), whose last key opens the first pooling window of a run
 // that does not start the row; with t0 == 0 the request goes to the row's first keys and is ignored.
 __device__ __forceinline__ void s1d_load_group_before(elem8 (&t4)[4], const S1DecodeSeq& sq, int64_t row_stride, int t0, int n, int g) {
@@ -519,6 +506,7 @@ __device__ __forceinline__ void s1d_fine_extent(const S1DecodeParams& p, const S
 template <bool kPool>
 __global__ __launch_bounds__(64)
 void stage1_decode_score_kernel(const S1DecodeParams p) {
+    warm_kernel_arguments<sizeof(S1DecodeParams)>();
     const int lane = threadIdx.x, n = lane & 15, g = lane >> 4;
     const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
     const S1DecodeSeq sq = s1d_sequence(p, b, h);
@@ -532,8 +520,8 @@ void stage1_decode_score_kernel(const S1DecodeParams p) {
 
     // Everything this run reads is requested before anything waits on memory, in the order in which it is needed:
     // the partial records of the log-sum-exp (merged while the keys are still on their way), the query, two tiles.
-    // A run has one or two tiles (more only when a sequence has over 128 of them); with one, the second request
-    // repeats the first, so that the number of requests in flight is the same on every path.
+    // A run has one or two tiles (more only when a sequence has over 128 of them); a second one is requested wherever runs
+    // may have two (the first again where this run has one), so that the number of requests in flight is known.
     int records = (((vis_c + 63) >> 6) + p.run_c - 1) / p.run_c;                    // the coarse runs of this sequence
     records = records < 1 ? 1 : records;
     S1DRecords rec;
@@ -544,7 +532,7 @@ void stage1_decode_score_kernel(const S1DecodeParams p) {
         s1d_load_q(qf, p, sq, h, n, g);
         if (kPool) s1d_load_group_before(before4, sq, p.k_row_stride, t0, n, g);
         s1d_load_tile(ta, sq.kbase, p.k_row_stride, t0 * 64, sq.Lk, n, g);
-        s1d_load_tile(tb, sq.kbase, p.k_row_stride, (t0 + 1 < t1 ? t0 + 1 : t0) * 64, sq.Lk, n, g);
+        if (p.run_f > 1) s1d_load_tile(tb, sq.kbase, p.k_row_stride, (t0 + 1 < t1 ? t0 + 1 : t0) * 64, sq.Lk, n, g);
         s1d_merge_records(rec, records, n, g, p.group, lse2);
     }
     s1d_score_run<kPool>(p, sq, qf, lse2, before4, ta, tb, vis_f, tiles, t0, t1, owns_tail, b, h, lane);
@@ -556,19 +544,20 @@ using namespace IV2_NS;
 
 namespace {
 
-// Runs of the two-launch form: every run is `run` tiles long whatever its sequence's length, so the single-wavefront
-// workgroups all carry the same load; the longest sequence is cut into at most 64 runs.
+// Every run is `run` tiles long whatever its sequence's length, so the wavefronts all carry the same load; the longest
+// sequence is cut into at most 64 runs.  One tile per run while that makes no more than two wavefronts per SIMD (the time is
+// one wavefront's chain of round trips then), two beyond, both requested before the first is used.
 void s1d_splits(int batch, int num_heads_k, int max_keys, int max_coarse, int& splits_f, int& splits_c, int& run_f, int& run_c) {
-    (void)batch; (void)num_heads_k;
-    auto plan = [&](int tiles, int want_run, int& splits, int& run) {
-        run = want_run;
+    auto plan = [&](int tiles, int& splits, int& run) {
+        run = static_cast<int64_t>(batch) * num_heads_k * tiles <= 2048 ? 1 : 2;
         if ((tiles + run - 1) / run > 64) run = (tiles + 63) / 64;
         splits = (tiles + run - 1) / run;
         if (splits < 1) splits = 1;
     };
-    plan((max_keys + 63) / 64, 2, splits_f, run_f);
-    plan((max_coarse + 63) / 64, 2, splits_c, run_c);
+    plan((max_keys + 63) / 64, splits_f, run_f);
+    plan((max_coarse + 63) / 64, splits_c, run_c);
 }
+unsigned s1d_lse_workgroups(int splits_c) { return static_cast<unsigned>((splits_c + kLseWaves - 1) / kLseWaves); }
 
 }  // namespace
 
@@ -636,7 +625,7 @@ extern "C" int IV2_ENTRY(infllmv2_stage1_decode)(void* stream, const void* q, co
     p.cache_lens = cache_lens; p.cache_len = cache_len; p.pool_len = out_len;
     p.local_blocks = local_blocks; p.init_blocks = init_blocks;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(stage1_decode_lse_kernel, dim3(p.splits_c, num_heads_k, batch), dim3(64), 0, st, p);
+    hipLaunchKernelGGL(stage1_decode_lse_kernel, dim3(s1d_lse_workgroups(p.splits_c), num_heads_k, batch), dim3(64 * kLseWaves), 0, st, p);
     IV2_LAUNCH_CHECK();
     const dim3 grid(p.splits_f, num_heads_k, batch);
     if (pooled) hipLaunchKernelGGL(stage1_decode_score_kernel<true>, grid, dim3(64), 0, st, p);
@@ -713,7 +702,7 @@ extern "C" int IV2_ENTRY(infllmv2_decode_step_scores)(void* stream, const void* 
     t.kernel_f = kernel_size_f; t.stride_f = stride_f; t.kernel_c = kernel_size_c; t.stride_c = stride_c;
     t.with_scores = pooled != nullptr ? 1 : 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(stage1_decode_front_kernel, dim3(1 + p.splits_c, num_heads_k, batch), dim3(64), 0, st, p, t);
+    hipLaunchKernelGGL(stage1_decode_front_kernel, dim3(1 + s1d_lse_workgroups(p.splits_c), num_heads_k, batch), dim3(64 * kLseWaves), 0, st, p, t);
     IV2_LAUNCH_CHECK();
     if (pooled == nullptr || out_len == 0) return 0;
     hipLaunchKernelGGL(stage1_decode_score_kernel<true>, dim3(p.splits_f, num_heads_k, batch), dim3(64), 0, st, p);
