@@ -70,58 +70,58 @@ __device__ __forceinline__ int64_t cache_row_offset(const DecodeParams& p, int b
     return cb * batch_stride + static_cast<int64_t>(row) * row_stride;
 }
 
-// Eight table values from element index i on: one 16-byte load where the interleaved layout needs four of them, too
-// (the tables are only 2-byte aligned, which global loads do not mind; the last four may lie beyond the row, so they are
-// loaded only where they are used).
-__device__ __forceinline__ void rotary_values(float (&v)[8], const elem_bits* table, int i, bool eight) {
-    uint32_t w[4] = {0, 0, 0, 0};
-    if (eight) __builtin_memcpy(w, table + i, 16);
-    else __builtin_memcpy(w, table + i, 8);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        v[2 * e] = elem_lo_to_f32(w[e]);
-        v[2 * e + 1] = elem_hi_to_f32(w[e]);
-    }
+// One 16-byte chunk (8 values, d = 8 chunk ...) of a head vector and what turns it at position pos: requested by
+// rotary_request, used by rotary_turn, so that a caller with several chunks has all of them in flight (one chunk after the
+// other, each waiting for its own, made the set-up of a short split five round trips longer).  Interleaved: pairs (2i, 2i+1)
+// lie inside the chunk; contiguous: the partner of d is d +- rotary_dim / 2, in another chunk of the same head vector.
+// (a, b) -> (a cos - b sin, a sin + b cos) in fp32, one rounding (rotary.h:57-62, 131-133).
+struct RotaryChunk {
+    uint4 own, other;
+    uint2 c[2], s[2];                                          // table values: four (interleaved) or eight
+};
+__device__ __forceinline__ RotaryChunk rotary_request(const DecodeParams& p, const elem_bits* head_vec, int chunk, int pos) {
+    RotaryChunk r;
+    const int half = p.rotary_dim >> 1, d0 = chunk * 8;
+    r.own = *reinterpret_cast<const uint4*>(head_vec + d0);
+    const int d = d0 < p.rotary_dim ? d0 : 0;                  // beyond the turned part: any valid address
+    const int in_half = d < half ? d : d - half;
+    r.other = *reinterpret_cast<const uint4*>(head_vec + (p.rotary_interleaved ? d : (d < half ? d + half : d - half)));
+    // the tables are only 2-byte aligned, which global loads do not mind; interleaved, the second four may lie beyond the row
+    const int64_t at = static_cast<int64_t>(pos) * half + (p.rotary_interleaved ? d >> 1 : in_half);
+    const int second = p.rotary_interleaved ? 0 : 4;
+    __builtin_memcpy(&r.c[0], p.rot_cos + at, 8);
+    __builtin_memcpy(&r.c[1], p.rot_cos + at + second, 8);
+    __builtin_memcpy(&r.s[0], p.rot_sin + at, 8);
+    __builtin_memcpy(&r.s[1], p.rot_sin + at + second, 8);
+    return r;
 }
-
-// One 16-byte chunk (8 values, d = 8 chunk ...) of a head vector turned at position pos.  Interleaved: pairs
-// (2i, 2i+1) lie inside the chunk; contiguous: the partner of d is d +- rotary_dim / 2, in another chunk of the
-// same head vector.  (a, b) -> (a cos - b sin, a sin + b cos) in fp32, one rounding (rotary.h:57-62, 131-133).
-__device__ __forceinline__ uint4 rotary_chunk(const DecodeParams& p, const elem_bits* head_vec, int chunk, int pos) {
-    const uint4 raw = *reinterpret_cast<const uint4*>(head_vec + chunk * 8);
-    const int d0 = chunk * 8, half = p.rotary_dim >> 1;
-    if (d0 >= p.rotary_dim) return raw;
-    const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-    float x[8], y[8], c[8], s[8];
+__device__ __forceinline__ uint4 rotary_turn(const DecodeParams& p, const RotaryChunk& r, int chunk) {
+    const int d0 = chunk * 8;
+    const bool left = d0 < (p.rotary_dim >> 1);
+    const uint32_t w[4] = {r.own.x, r.own.y, r.own.z, r.own.w}, ow[4] = {r.other.x, r.other.y, r.other.z, r.other.w};
+    const uint32_t cw[4] = {r.c[0].x, r.c[0].y, r.c[1].x, r.c[1].y}, sw[4] = {r.s[0].x, r.s[0].y, r.s[1].x, r.s[1].y};
+    uint32_t out[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        x[2 * e] = elem_lo_to_f32(w[e]);
-        x[2 * e + 1] = elem_hi_to_f32(w[e]);
-    }
-    const elem_bits* cs = p.rot_cos + static_cast<int64_t>(pos) * half;
-    const elem_bits* sn = p.rot_sin + static_cast<int64_t>(pos) * half;
-    if (p.rotary_interleaved) {
-        rotary_values(c, cs, d0 >> 1, false);
-        rotary_values(s, sn, d0 >> 1, false);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            y[2 * i] = x[2 * i] * c[i] - x[2 * i + 1] * s[i];
-            y[2 * i + 1] = x[2 * i] * s[i] + x[2 * i + 1] * c[i];
+        const float x0 = elem_lo_to_f32(w[e]), x1 = elem_hi_to_f32(w[e]);
+        float y0, y1;
+        if (p.rotary_interleaved) {                            // uniform: table value e
+            const float c = (e & 1) ? elem_hi_to_f32(cw[e >> 1]) : elem_lo_to_f32(cw[e >> 1]);
+            const float sn = (e & 1) ? elem_hi_to_f32(sw[e >> 1]) : elem_lo_to_f32(sw[e >> 1]);
+            y0 = x0 * c - x1 * sn;
+            y1 = x0 * sn + x1 * c;
+        } else {                                               // table values 2 e and 2 e + 1
+            const float c0 = elem_lo_to_f32(cw[e]), c1 = elem_hi_to_f32(cw[e]), s0 = elem_lo_to_f32(sw[e]), s1 = elem_hi_to_f32(sw[e]);
+            const float o0 = elem_lo_to_f32(ow[e]), o1 = elem_hi_to_f32(ow[e]);
+            y0 = left ? x0 * c0 - o0 * s0 : x0 * c0 + o0 * s0;
+            y1 = left ? x1 * c1 - o1 * s1 : x1 * c1 + o1 * s1;
         }
-    } else {
-        const bool left = d0 < half;
-        const uint4 oraw = *reinterpret_cast<const uint4*>(head_vec + (left ? d0 + half : d0 - half));
-        const uint32_t ow[4] = {oraw.x, oraw.y, oraw.z, oraw.w};
-        const int i0 = left ? d0 : d0 - half;
-        rotary_values(c, cs, i0, true);
-        rotary_values(s, sn, i0, true);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float o = (e & 1) ? elem_hi_to_f32(ow[e >> 1]) : elem_lo_to_f32(ow[e >> 1]);
-            y[e] = left ? x[e] * c[e] - o * s[e] : x[e] * c[e] + o * s[e];
-        }
+        out[e] = d0 < p.rotary_dim ? pack_elem2(y0, y1) : w[e];
     }
-    return make_uint4(pack_elem2(y[0], y[1]), pack_elem2(y[2], y[3]), pack_elem2(y[4], y[5]), pack_elem2(y[6], y[7]));
+    return make_uint4(out[0], out[1], out[2], out[3]);
+}
+__device__ __forceinline__ uint4 rotary_chunk(const DecodeParams& p, const elem_bits* head_vec, int chunk, int pos) {
+    return rotary_turn(p, rotary_request(p, head_vec, chunk, pos), chunk);
 }
 
 // Several new rows per sequence (one is written by the split kernel itself): one thread moves 16 bytes of one new row
@@ -323,14 +323,14 @@ __global__ __launch_bounds__(64 * kWaves)
 void decode_split_kernel(const DecodeParams p) {
     constexpr int kSlots = kWaves == 1 ? 2 : 1;                // block tiles per wavefront
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-    __shared__ __attribute__((aligned(16))) elem_bits new_rows[kWaves][2 * kHeadDim];       // K, then V: a copy per wavefront
+    __shared__ __attribute__((aligned(16))) elem_bits new_row[2 * kHeadDim];        // K, then V
+    __shared__ uint4 turned_q[4][64];
     uint64_t* words = reinterpret_cast<uint64_t*>(smem + kWaves * kSlots * kSlotBytes);     // more than 64 mask words: the row's, clipped to the sequence
     warm_kernel_arguments<sizeof(DecodeParams)>();
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
     const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-    elem_bits* new_row = new_rows[wave];
     unsigned char* tiles = smem + wave * kSlots * kSlotBytes;
     const int64_t pair = static_cast<int64_t>(b) * p.num_heads_k + h;
     const bool listed = kSelect || p.mask != nullptr || p.topk_idx != nullptr;      // else: every block
@@ -342,18 +342,6 @@ void decode_split_kernel(const DecodeParams p) {
     const int lp = p.leftpad ? p.leftpad[b] : 0;              // the sequence's key 0 is cache row lp
     // position of the first appended key; a full cache takes no key, and the tables need not reach beyond it
     const int rot_pos = !p.cache_seqlens ? 0 : (seqlen < p.capacity ? seqlen : p.capacity - 1);
-    if (p.append_here) {
-        // lanes 0..15: the new K row, lanes 16..31: the new V row, 16 bytes each
-        const int chunk = n;
-        uint4 val = make_uint4(0, 0, 0, 0);
-        if (g == 0) {
-            const elem_bits* kvec = p.knew + b * p.kn_batch + h * p.kn_head;
-            val = p.rotary_dim > 0 ? rotary_chunk(p, kvec, chunk, rot_pos) : *reinterpret_cast<const uint4*>(kvec + chunk * 8);
-        } else if (g == 1) {
-            val = *reinterpret_cast<const uint4*>(p.vnew + b * p.vn_batch + h * p.vn_head + chunk * 8);
-        }
-        if (g < 2) *reinterpret_cast<uint4*>(new_row + g * kHeadDim + chunk * 8) = val;    // read by other lanes after the fences below
-    }
     int L = seqlen + p.seqlen_new;
     if (L > p.capacity) L = p.capacity;
     L -= lp;                                                   // keys of the sequence; mask block j = keys 64 j ..
@@ -362,28 +350,47 @@ void decode_split_kernel(const DecodeParams p) {
     int n_words = last_blk < 0 ? 0 : (last_blk >> 6) + 1;
     if (listed && !kSelect && n_words > p.n64) n_words = p.n64;
 
-    elem8 qf[4];
-    {
-        const int qh = p.group * h + (n < p.group ? n : p.group - 1);      // rows beyond the group repeat its last head
-        const elem_bits* qp = p.q + b * p.q_batch + qh * p.q_head;
-        // the query is turned at the position of the first appended key (flash_fwd_kernel.h:899-901)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            if (p.rotary_dim > 0) {
-                const uint4 turned = rotary_chunk(p, qp, 4 * c + g, rot_pos);
-                __builtin_memcpy(&qf[c], &turned, 16);
-            } else {
-                qf[c] = *reinterpret_cast<const elem8*>(qp + 8 * g + 32 * c);
-            }
-        }
-    }
-
-    // ---- the selected blocks: words in LDS, how many there are, and which run of them is this wavefront's ----
     auto lds_fence = [&]() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     };
+    // The query and the new row (lanes 0..15: K, lanes 16..31: V, 16 bytes each).  The query is turned at the position of the
+    // first appended key (flash_fwd_kernel.h:899-901), a quarter by each of four wavefronts: every one turning all of it for
+    // itself pulled 100 KiB of tables and rows through the CU.
+    elem8 qf[4];
+    {
+        const int qh = p.group * h + (n < p.group ? n : p.group - 1);      // rows beyond the group repeat its last head
+        const elem_bits* qp = p.q + b * p.q_batch + qh * p.q_head;
+        if (p.rotary_dim > 0) {
+            constexpr int kOwn = 4 / kWaves;                   // 16-byte chunks of a lane's four that this wavefront turns
+            RotaryChunk r[kOwn];
+#pragma unroll
+            for (int c = 0; c < kOwn; ++c) r[c] = rotary_request(p, qp, 4 * (wave * kOwn + c) + g, rot_pos);
+#pragma unroll
+            for (int c = 0; c < kOwn; ++c) turned_q[wave * kOwn + c][lane] = rotary_turn(p, r[c], 4 * (wave * kOwn + c) + g);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) qf[c] = *reinterpret_cast<const elem8*>(qp + 8 * g + 32 * c);
+        }
+        if (p.append_here && wave == kWaves - 1 && g < 2) {
+            const elem_bits* kvec = p.knew + b * p.kn_batch + h * p.kn_head;
+            uint4 kept;
+            if (g == 1) kept = *reinterpret_cast<const uint4*>(p.vnew + b * p.vn_batch + h * p.vn_head + n * 8);
+            else kept = p.rotary_dim > 0 ? rotary_chunk(p, kvec, n, rot_pos) : *reinterpret_cast<const uint4*>(kvec + n * 8);
+            *reinterpret_cast<uint4*>(new_row + g * kHeadDim + n * 8) = kept;
+        }
+        if (p.append_here || p.rotary_dim > 0) {
+            if constexpr (kWaves > 1) __syncthreads();
+            else lds_fence();
+        }
+        if (p.rotary_dim > 0) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) qf[c] = *reinterpret_cast<const elem8*>(&turned_q[c][lane]);
+        }
+    }
+
+    // ---- the selected blocks: words in LDS, how many there are, and which run of them is this wavefront's ----
     // bits of words w0 + lane, and how many bits lie in words up to and including this lane's, from word w0 on
     auto scan_words = [&](int w0, uint64_t& bits) -> int {
         bits = w0 + lane < n_words ? words[w0 + lane] : 0ull;
