@@ -39,7 +39,7 @@ struct BwdParams {
     float* det_slots;               // (Hk, n_slots, det_slices, 2, 64, 128) fp32
     uint32_t* det_flags;            // (Hk, n_slots, det_slices): 1 where a slot was written
     int det_slices;
-    int dkdv_spread;                // dK/dV work items: 1 = all XCDs share every slice (few slices), 0 = an XCD owns whole slice groups
+    int dkdv_share;                 // dK/dV work items: 1, 2, 4 or 8 XCDs share each group of slices
 };
 
 // dQ, 8 consecutive tokens per workgroup sharing their common blocks through LDS: stage2_bwd_dq.hip
@@ -49,13 +49,15 @@ int launch_bwd_dkdv_wave(hipStream_t st, const BwdParams& p, int batch, int max_
 
 // deterministic mode only: adds the slots of every key block in slice order into dk_acc / dv_acc
 int launch_bwd_dkdv_reduce(hipStream_t st, const BwdParams& p, int batch);
-// Query tokens per dK/dV work item (slices are cut on the packed token axis).  Long inputs use 512-token slices (one
-// flush of the accumulators per 512 tokens); short ones 128, so that a few thousand tokens still make enough work
-// items to fill the device; the deterministic mode, whose workspace grows with the slice count, keeps 512.
+// Query tokens per dK/dV work item (slices are cut on the packed token axis).  Long sequences use 512-token slices (one
+// flush of the accumulators per 512 tokens); short ones 128, so that a few thousand tokens still make enough work items to fill
+// the device and the last of them are short (backward of 10 x 1500 tokens, 16 blocks selected: 844 against 968 us; of 16 x 3000:
+// 2160 / 2240; of 12000: 1640 / 1690; of 32768, 64 blocks: 8280 / 8170); the deterministic mode, whose workspace grows with the
+// slice count, keeps 512.
 constexpr int kDkdvSlice = 512;
 constexpr int kDkdvSliceSmall = 128;
-inline int dkdv_slice_tokens(int64_t total_q, bool deterministic) {
-    return (total_q <= 8192 && !deterministic) ? kDkdvSliceSmall : kDkdvSlice;   // deterministic mode: one slot per slice, so few slices
+inline int dkdv_slice_tokens(int max_seqlen_q, bool deterministic) {
+    return (max_seqlen_q <= 12288 && !deterministic) ? kDkdvSliceSmall : kDkdvSlice;   // deterministic mode: one slot per slice, so few slices
 }
 
 }  // namespace IV2_NS

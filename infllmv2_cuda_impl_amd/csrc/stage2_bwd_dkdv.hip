@@ -104,23 +104,18 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
     // stream the same tokens of q and dout, and because the assignment follows the packed axis (not each
     // sequence's own first group) the groups of a batch of sequences spread evenly over the XCDs.  Within a slice
     // the shared first block comes first, then the diagonal block and outwards, so the long items are dispatched early.
-    // With fewer groups than XCDs (short inputs) that would leave XCDs idle: then all 8 XCDs share every slice, block
-    // rel going to XCD rel % 8, slices latest first.
+    // Where the groups do not divide evenly among the XCDs, 2, 4 or all 8 of them share a group (p.dkdv_share; a group then
+    // goes through as many L2s): sharer `part` takes the blocks rel with rel % share == part.
     const int xcd = blockIdx.x & 7, turn = blockIdx.x >> 3;
     if (Sq <= 0) return;                                       // uniform
     const int last_slice = (q0 + Sq - 1) / kColSlice;
-    int rel, slice;
-    if (p.dkdv_spread) {
-        const int turns_per_slice = (p.k_blocks + 7) >> 3;
-        rel = (turn % turns_per_slice) * 8 + xcd;
-        slice = last_slice - turn / turns_per_slice;
-    } else {
-        rel = turn % p.k_blocks;
-        const int top_group = last_slice / kGroupSlices;
-        const int round = turn / p.k_blocks;                   // an XCD works through one group of slices in consecutive rounds
-        const int grp_idx = top_group - ((top_group - xcd) & 7) - 8 * (round / kGroupSlices);
-        slice = grp_idx < 0 ? -1 : grp_idx * kGroupSlices + (kGroupSlices - 1 - round % kGroupSlices);
-    }
+    const int share = p.dkdv_share, teams = 8 / share;         // powers of two
+    const int blocks_each = (p.k_blocks + share - 1) / share;
+    const int rel = (turn % blocks_each) * share + (xcd & (share - 1));
+    const int round = turn / blocks_each;                      // a team works through one group of slices in consecutive rounds
+    const int top_group = last_slice / kGroupSlices;
+    const int grp_idx = top_group - ((top_group - xcd / share) & (teams - 1)) - teams * (round / kGroupSlices);
+    const int slice = grp_idx < 0 ? -1 : grp_idx * kGroupSlices + (kGroupSlices - 1 - round % kGroupSlices);
     if (rel >= nb || slice > last_slice || slice < q0 / kColSlice) return;      // uniform
     int j;
     if (rel == 0) {
@@ -532,17 +527,21 @@ static int launch_bwd_dkdv_sliced(hipStream_t st, const BwdParams& p_in, int bat
     // a sequence of max_seqlen_q tokens touches at most `groups` consecutive slice groups wherever it starts
     const int group_tokens = kGroupWords * 64;
     const int groups = (max_seqlen_q + group_tokens - 1) / group_tokens + 1;
-    int64_t items;
-    // fewer groups than XCDs in the whole batch: every XCD takes a share of every slice
-    p.dkdv_spread = static_cast<int64_t>(batch) * (groups - 1) < 8 ? 1 : 0;
-    if (p.dkdv_spread) {
-        const int n_slices = (max_seqlen_q + kColSlice - 1) / kColSlice + 1;               // a sequence need not start on a slice boundary
-        items = static_cast<int64_t>(n_slices) * ((p.k_blocks + 7) / 8 * 8);
-    } else {
-        // an XCD takes every 8th group: ceil(groups / 8) rounds of kGroupSlices slices each
-        const int n_slices8 = (groups + 7) / 8 * (8 * kGroupSlices);
-        items = static_cast<int64_t>(n_slices8) * p.k_blocks;
+    // XCDs per group: the number that leaves the fewest of them idle in the last round of groups, weighed with what sharing
+    // costs.  Backward in us with 1 / 2 / 4 / 8 sharers, 64 blocks selected, 2 KV heads: 6000 tokens (3 groups) 2120 / 1400 /
+    // 1160 / 1090, 20000 (10) 5420 / 4720 / 4530 / 5100, 32768 (16) 8400 / 8170 / 8530 / 9450, 71552 (35) 17500 / 16900 / 16950 /
+    // 18900.
+    const int all_groups = static_cast<int>((p.total_q + group_tokens - 1) / group_tokens);
+    const float cost[4] = {1.f, 1.f, 1.02f, 1.12f};
+    float best = 0.f;
+    for (int i = 0; i < 4; ++i) {
+        const int teams = 8 >> i;
+        const float busy = static_cast<float>(all_groups) / ((all_groups + teams - 1) / teams * teams) / cost[i];
+        if (busy > best) { best = busy; p.dkdv_share = 1 << i; }
     }
+    const int teams = 8 / p.dkdv_share;
+    const int64_t rounds = static_cast<int64_t>((groups + teams - 1) / teams) * kGroupSlices;
+    const int64_t items = 8 * rounds * ((p.k_blocks + p.dkdv_share - 1) / p.dkdv_share);
     IV2_CHECK(items <= 0x7fffffffll, "varlen_bwd: too many (slice, block) work items");
     IV2_CHECK(p.q_tok >= 0 && p.q_tok < (1ll << 31) && p.do_tok >= 0 && p.do_tok < (1ll << 31) && p.total_q < (1ll << 31),
               "varlen_bwd: token strides of q and dout must lie in [0, 2^31) elements");
@@ -555,7 +554,7 @@ static int launch_bwd_dkdv_sliced(hipStream_t st, const BwdParams& p_in, int bat
 }
 
 int launch_bwd_dkdv_wave(hipStream_t st, const BwdParams& p, int batch, int max_seqlen_q, bool causal) {
-    if (dkdv_slice_tokens(p.total_q, p.det_slots != nullptr) == kDkdvSliceSmall) return launch_bwd_dkdv_sliced<kDkdvSliceSmall>(st, p, batch, max_seqlen_q, causal);
+    if (dkdv_slice_tokens(max_seqlen_q, p.det_slots != nullptr) == kDkdvSliceSmall) return launch_bwd_dkdv_sliced<kDkdvSliceSmall>(st, p, batch, max_seqlen_q, causal);
     return launch_bwd_dkdv_sliced<kDkdvSlice>(st, p, batch, max_seqlen_q, causal);
 }
 

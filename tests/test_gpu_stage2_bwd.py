@@ -153,3 +153,22 @@ def test_backward_with_duplicate_and_missing_indices(ops):
     check_grad("dv", vg.grad, dv)
 
 
+
+
+@pytest.mark.parametrize("lens", [[700, 1301], [6001], [300, 4000, 77, 3900], [20001], [9000, 15400], [32768], [2048] * 9 + [5]])
+def test_every_pair_reaches_dv_however_the_xcds_share(lens):
+    """Rows of P add up to one, so with dout = 1 the sum of dv over the keys is the number of (token, head) rows: a work item left
+    out, or done twice, by the split of the slices over 1, 2, 4 or 8 sharers shows up whatever the size."""
+    import infllmv2_cuda_impl_amd as ops
+    g = torch.Generator(device="cuda").manual_seed(len(lens))
+    total, mx = sum(lens), max(lens)
+    mk = lambda h: torch.randn(total, h, 128, generator=g, device="cuda").to(torch.bfloat16).requires_grad_(True)
+    q, k, v = mk(16), mk(1), mk(1)
+    cu = torch.tensor([sum(lens[:i]) for i in range(len(lens) + 1)], dtype=torch.int32, device="cuda")
+    layer = ops.InfLLMv2Attention(topk=16, local_blocks=4, init_blocks=1)
+    out = layer(q, k, v, cu, mx)
+    dv, = torch.autograd.grad(out, v, torch.ones_like(out))
+    for i, n in enumerate(lens):
+        got = dv[cu[i]:cu[i + 1], 0].double().sum(0)
+        # one item holds 1/64 of the mass of 128 tokens or more; the bf16 rounding of dv adds up to less than a row or two
+        assert (got - 16 * n).abs().max() <= 2 + 2e-3 * 16 * n ** 0.5 * 4, (i, n, float((got - 16 * n).abs().max()))
