@@ -41,7 +41,7 @@ HIPCC_FLAGS = [
 # the type at run time
 PER_ELEMENT_TYPE = {"compress.hip", "decode.hip", "stage1.hip", "stage1_decode.hip", "stage2_bwd.hip",
                     "stage2_bwd_dkdv.hip", "stage2_bwd_dq.hip", "stage2_fwd.hip",
-                    "stage2_fwd_hybrid.hip"}
+                    "stage2_fwd_hybrid.hip", "stage2_fwd_tile.hip"}
 
 
 def sources():

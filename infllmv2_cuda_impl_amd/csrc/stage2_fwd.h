@@ -28,4 +28,16 @@ struct FwdParams {
 int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q,
                              int max_seqlen_k, bool causal);
 
+// Forward without a mask (stage2_fwd_tile.hip): tiles of 256 query rows, 32 per wavefront.  A token takes 16 rows, 8 in groups of 8.
+inline int tile_row_shift(int group) { return group == 8 ? 3 : 4; }
+inline int tiles_per_sequence(int group, int max_seqlen_q) {
+    const int tokens = 256 >> tile_row_shift(group);
+    return (max_seqlen_q + tokens - 1) / tokens;
+}
+// From about a tile per CU on: with fewer, the hybrid walk's groups of 8 tokens fill the chip better (us, hybrid walk | tiles: 188 tiles
+// 45 | 55, 226 61 | 63, 250 72 | 68, 252 in two sequences 55 | 45, 440 in five 63 | 58).
+constexpr int kMinTiles = 240;
+int launch_stage2_fwd_tile(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q,
+                           int max_seqlen_k, bool causal);
+
 }  // namespace IV2_NS

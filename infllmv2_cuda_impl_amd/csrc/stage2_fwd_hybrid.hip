@@ -25,6 +25,7 @@
 #include "common.h"
 #include "kv_image.h"
 #include "block_walker.h"
+#include "lds_dma.h"
 #include "stage2_fwd.h"
 #include <math.h>
 
@@ -43,22 +44,6 @@ struct HybridExtra {
     int mask_words;                                            // words per LDS mask row: what max_seqlen_k needs, not the maximum
 };
 
-__device__ __forceinline__ uint32_t lds_address_of(const void* ptr) {
-    return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)ptr));
-}
-// One wavefront copies 4 KiB from global memory straight into LDS (no registers): lane l moves bytes
-// [16 l, 16 l + 16) of each 1 KiB quarter (the instruction offset advances source and destination alike).
-// The compiler does not see these loads; callers order them by hand with s_waitcnt vmcnt(n) + barrier.
-__device__ __forceinline__ void dma_copy_4k(const void* src_lane, uint32_t lds_dst) {
-    asm volatile("s_mov_b32 m0, %1\n\t"
-                 "global_load_lds_dwordx4 %0, off\n\t"
-                 "global_load_lds_dwordx4 %0, off offset:1024\n\t"
-                 "global_load_lds_dwordx4 %0, off offset:2048\n\t"
-                 "global_load_lds_dwordx4 %0, off offset:3072\n\t"
-                 :
-                 : "v"(src_lane), "s"(lds_dst)
-                 : "memory", "m0");
-}
 __device__ __forceinline__ uint64_t uniform_u64(uint64_t v) {
     const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
     const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
@@ -372,6 +357,8 @@ int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int 
     const int64_t total = static_cast<int64_t>(num_heads_k) * batch * x.groups_per_seq;
     IV2_CHECK(total <= 0x3fffffff, "varlen_fwd: too many token groups");
     IV2_CHECK((max_seqlen_k + kBlockN - 1) / kBlockN <= kMaxMaskWords * 64, "varlen_fwd: more than %d key blocks per sequence", kMaxMaskWords * 64);
+    if (p.mask == nullptr && static_cast<int64_t>(num_heads_k) * batch * tiles_per_sequence(p.group, max_seqlen_q) >= kMinTiles)
+        return launch_stage2_fwd_tile(st, p, batch, num_heads_k, max_seqlen_q, max_seqlen_k, causal);
     x.total_groups = static_cast<int>(total);
     x.mask_words = ((max_seqlen_k + kBlockN - 1) / kBlockN + 63) / 64;
     if (x.mask_words < 1) x.mask_words = 1;
