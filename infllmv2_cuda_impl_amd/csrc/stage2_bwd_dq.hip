@@ -58,27 +58,36 @@ __device__ __forceinline__ short4q dq_read_tr(const unsigned char* ptr) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4q*)(ptr));
 }
 
-// dS^T of one block as the B operand of dQ^T = K^T dS^T, from the S^T and dP^T accumulators
-// dS^T of one block as the B operand of dQ^T += K^T dS^T.  The dP accumulators were started at -D, so dp holds dP - D.
-// lim: last in-block key index the token may see (>= 63 for a whole block, which is the common case).
-__device__ __forceinline__ void ds_tile(const floatx4 (&s)[4], const floatx4 (&dp)[4], elem8 (&dsf)[2], int lim, int g,
-                                        float scale_log2, float lse2) {
-    if (lim >= kBlockN - 1) {                                  // uniform per wavefront
+// The second half of a block's scores: dP (accumulators started at -D) from V fragments, and beside each of its MFMAs one element of
+// P = exp2(scale S - LSE).  The order is fixed by hand: the compiler puts the exponentials behind the last MFMA, where the wavefront has
+// nothing else to issue (71552 packed tokens, 2 KV heads: 7610 -> 7440 us; with the K^T reads moved in between as well 7700, with the own V
+// requested as soon as its registers are free 8300).  lim: last in-block key index the token may see (>= 63 for a whole block, which is the common case).
+__device__ __forceinline__ void p_and_dp(floatx4 (&s)[4], floatx4 (&dp)[4], const elem8 (&vf)[16], const elem8 (&dof)[4], int lim, int g,
+                                         float scale_log2, float lse2) {
+    if (lim < kBlockN - 1) {                                   // uniform per wavefront
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                dsf[kt >> 1][(kt & 1) * 4 + e] = static_cast<elem_t>(__builtin_amdgcn_exp2f(s[kt][e] * scale_log2 - lse2) * dp[kt][e]);
-    } else {
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float pv = __builtin_amdgcn_exp2f(s[kt][e] * scale_log2 - lse2);
-                if (16 * kt + 4 * g + e > lim) pv = 0.f;
-                dsf[kt >> 1][(kt & 1) * 4 + e] = static_cast<elem_t>(pv * dp[kt][e]);
-            }
+                if (16 * kt + 4 * g + e > lim) s[kt][e] = -INFINITY;
     }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            dp[kt] = IV2_MFMA(vf[kt * 4 + c], dof[c], dp[kt], 0, 0, 0);
+            s[c][kt] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[c][kt], scale_log2, -lse2));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+}
+
+// dS^T = P (dP - D) as the B operand of dQ^T += K^T dS^T
+__device__ __forceinline__ void ds_operand(const floatx4 (&s)[4], const floatx4 (&dp)[4], elem8 (&dsf)[2]) {
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dsf[kt >> 1][(kt & 1) * 4 + e] = static_cast<elem_t>(s[kt][e] * dp[kt][e]);
 }
 
 template <bool kCausal>
@@ -253,13 +262,9 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
                     const uint4 raw = vb[f * 64];
                     __builtin_memcpy(&vreg[f], &raw, 16);
                 }
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-#pragma unroll
-                    for (int kt = 0; kt < 4; ++kt)
-                        dp[kt] = IV2_MFMA(vreg[kt * 4 + c], dof[c], dp[kt], 0, 0, 0);
+                p_and_dp(s, dp, vreg, dof, (j0 == last_blk) ? last_key - j0 * kBlockN : kBlockN - 1, g, p.scale_log2, lse2);
                 elem8 dsf[2];
-                ds_tile(s, dp, dsf, (j0 == last_blk) ? last_key - j0 * kBlockN : kBlockN - 1, g, p.scale_log2, lse2);
+                ds_operand(s, dp, dsf);
                 const unsigned char* ktile = reinterpret_cast<const unsigned char*>(ring + tile * 2048) + tr_lane;
 #pragma unroll
                 for (int cc = 0; cc < 2; ++cc)
@@ -301,13 +306,9 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
                 __builtin_memcpy(&raw, &kreg[f], 16);
                 mine[f * 64] = raw;
             }
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-#pragma unroll
-                for (int kt = 0; kt < 4; ++kt)
-                    dp[kt] = IV2_MFMA(vreg[kt * 4 + c], dof[c], dp[kt], 0, 0, 0);
+            p_and_dp(s, dp, vreg, dof, (jp == last_blk) ? last_key - jp * kBlockN : kBlockN - 1, g, p.scale_log2, lse2);
             elem8 dsf[2];
-            ds_tile(s, dp, dsf, (jp == last_blk) ? last_key - jp * kBlockN : kBlockN - 1, g, p.scale_log2, lse2);
+            ds_operand(s, dp, dsf);
 #pragma unroll
             for (int cc = 0; cc < 2; ++cc) {
                 if (cc == 1) {
