@@ -140,7 +140,14 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     if (i0 >= Sq) return;                                                           // uniform per workgroup
     const int Sk = p.cu_seqlens_k[b + 1] - p.cu_seqlens_k[b];
 
-    const int i = i0 + wave;                                                        // this wavefront's token
+    // A group at the end of a sequence that has four tokens or fewer: 2, 4 or 8 wavefronts share a token's blocks (every so-manyth column
+    // of its mask row each) and merge at the end.  With one wavefront per token such a group took as long as a full one, and where a
+    // launch has few groups per CU the last of them decides (2049 queries behind 17962 keys, 514 groups: 254 -> 236 us).
+    const int in_group = Sq - i0 < kHybTokens ? Sq - i0 : kHybTokens;
+    const int share_log2 = in_group > 4 ? 0 : in_group > 2 ? 1 : in_group > 1 ? 2 : 3;
+    const int slots = kHybTokens >> share_log2;                                     // wavefronts of one share
+    const int part = wave >> (3 - share_log2);
+    const int i = i0 + (wave & (slots - 1));                                        // this wavefront's token
     const bool live = i < Sq;
     int last_key = kCausal ? (i + Sk - Sq) : (Sk - 1);                              // largest allowed key index
     if (last_key > Sk - 1) last_key = Sk - 1;
@@ -160,7 +167,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
         if (nw > x.mask_words) nw = x.mask_words;                                    // a sequence longer than the announced max_seqlen_k
     }
     unsigned long long* own = rows + wave * x.mask_words;                           // this token's row, later minus the common part
-    for (int w = tid; w < nw; w += 512) com[w] = ~0ull;
+    for (int w = tid; w < nw; w += 512) com[w] = share_log2 == 0 ? ~0ull : 0ull;   // shared out: no lock step
     __syncthreads();
     for (int w = lane; w < nw; w += 64) {
         uint64_t v = 0ull;
@@ -175,7 +182,9 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
         if (live && v != ~0ull) atomicAnd(&com[w], static_cast<unsigned long long>(v));
     }
     __syncthreads();
-    for (int w = lane; w < nw; w += 64) own[w] &= ~com[w];
+    const uint64_t columns = (share_log2 == 0 ? ~0ull : share_log2 == 1 ? 0x5555555555555555ull
+                              : share_log2 == 2 ? 0x1111111111111111ull : 0x0101010101010101ull) << part;
+    for (int w = lane; w < nw; w += 64) own[w] &= ~com[w] & columns;
 
     // ---- Q operand ----
     elem8 qf[4];
@@ -327,6 +336,30 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
             c0 = n0;
             c1 = n1;
             half ^= 1;
+        }
+    }
+    if (share_log2 != 0) {                                     // uniform per workgroup
+        // the ring was not used: 34 floats of every lane, lane by lane
+        float* mine = reinterpret_cast<float*>(smem_raw) + wave * (34 * 64) + lane;
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) mine[(4 * dt + e) * 64] = o[dt][e];
+        mine[32 * 64] = m;
+        mine[33 * 64] = l;
+        __syncthreads();
+        if (part != 0 || !live) return;
+        for (int other = 1; other < (1 << share_log2); ++other) {
+            const float* theirs = mine + other * slots * (34 * 64);
+            const float m2 = theirs[32 * 64], m_new = fmaxf(m, m2);
+            const float m_use = (m_new == -INFINITY) ? 0.f : m_new;                 // neither has a key
+            const float a1 = __builtin_amdgcn_exp2f(m - m_use), a2 = __builtin_amdgcn_exp2f(m2 - m_use);
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[dt][e] = o[dt][e] * a1 + theirs[(4 * dt + e) * 64] * a2;
+            l = l * a1 + theirs[33 * 64] * a2;
+            m = m_new;
         }
     }
     if (!live) return;
