@@ -10,11 +10,10 @@
 //
 // Design: decode is HBM-bound (each selected block is 32 KiB of K+V read exactly once, ~2 MiB per
 // sequence and KV head), so the kernel reads the cache in the caller's layout, with no repacking
-// pass.  One single-wavefront workgroup handles one (sequence, KV head, split); a split is a
-// contiguous run of the row's selected blocks (by ordinal, so splits are balanced whatever the
-// mask looks like).  K rows are the MFMA A operand as they lie in memory (contraction over d);
-// V is contracted over keys, so its tile takes one trip through a wavefront-private LDS buffer and
-// is read back transposed.  Partial results are merged by a small combine kernel.
+// pass.  A workgroup of one wavefront, or of four where a launch has at most one workgroup per CU, handles one (sequence, KV
+// head, split); a split is a contiguous run of the row's selected blocks (by ordinal, so splits are balanced whatever the
+// selection looks like).  Whole K and V rows go to an LDS ring by LDS-DMA; K is read from it as the MFMA A operand (contraction
+// over d), V, which is contracted over keys, by transposing reads.  Partial results are merged by a small combine kernel.
 #include "common.h"
 #include "block_walker.h"
 #include "infllmv2_hip.h"
