@@ -203,7 +203,8 @@ __device__ __forceinline__ uint64_t drop_set_bits(uint64_t v, int rank) {
 //
 // append_here: the sequence's one new row is patched into its block's tile (turned by the rotary embedding where asked
 // for), so the row need not be in the cache before the launch: the first workgroup of each (sequence, KV head) writes
-// it there on its way out, and what a reader of that row gets from memory does not matter.
+// it there on its way out.  What a reader of that row gets from memory does not matter, NaN included: the tile's rows
+// behind the end are copies of it, K's are masked by assignment and V's, which are multiplied by P = 0, are patched too.
 constexpr int kMergePitch = kHeadDim + 4;                      // floats per head of a wavefront's output in LDS
 
 __device__ __forceinline__ int scan_lanes(int v) {              // inclusive prefix sum over the lanes, DPP adds only
@@ -520,7 +521,8 @@ void decode_split_kernel(const DecodeParams p) {
 #pragma unroll
             for (int u = 0; u < 16; ++u) decode_dma16(base + (u >> 2) * 16 * row_stride, off[u & 3], slot + u * 1024);
         } else {
-            // rows past the end are read from the last row (K is masked below, P is zero there)
+            // rows past the end are read from the last row (K is masked below, P is zero there); where that is the row being
+            // appended, memory need not hold it yet and the tile is patched
 #pragma unroll
             for (int u = 0; u < 16; ++u) {
                 int row = 4 * u + g;
@@ -546,14 +548,14 @@ void decode_split_kernel(const DecodeParams p) {
         const int j = __builtin_amdgcn_readlane(my_block, i & 63), key0 = j * kBlockN;
         unsigned char* ktile = tiles + (kSlots == 2 ? i & 1 : 0) * kSlotBytes;
         const bool patch = new_key >= key0 && new_key < key0 + kBlockN;            // uniform: the block of the row that is being appended
-        auto patch_row = [&](int which) {                      // 0: K, 1: V
-            const int r = new_key - key0;
-            if (g == 0)
-                *reinterpret_cast<uint4*>(ktile + which * kTileBytes + r * 256 + (n ^ tile_swizzle(r)) * 16) =
-                    *reinterpret_cast<const uint4*>(new_row + which * kHeadDim + 8 * n);
+        // the new row, into the rows of K's tile (0) or V's (1) from its own up to `end`
+        auto patch_rows = [&](int which, int end) {
+            const uint4 kept = *reinterpret_cast<const uint4*>(new_row + which * kHeadDim + 8 * n);
+            for (int r = new_key - key0 + g; r < end; r += 4)
+                *reinterpret_cast<uint4*>(ktile + which * kTileBytes + r * 256 + (n ^ tile_swizzle(r)) * 16) = kept;
             lds_fence();
         };
-        if (patch) patch_row(0);
+        if (patch) patch_rows(0, new_key - key0 + 1);          // the keys behind it are masked
         floatx4 s[4];
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
@@ -615,7 +617,7 @@ void decode_split_kernel(const DecodeParams p) {
         if (ahead) asm volatile("s_waitcnt vmcnt(32)" ::: "memory");
         else if (next_k) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        if (patch) patch_row(1);
+        if (patch) patch_rows(1, kBlockN);                     // P is zero behind it, and 0 x what unwritten memory holds may be NaN
         // A operand of O^T += V^T P^T: lane (n, g) needs V[32 cc + 4 g + {0..3}, 32 cc + 16 + 4 g + {0..3}][16 dt + n], the
         // keys in the order in which the lane holds P.  One transposing read hands a lane four rows' worth of one
         // column: within 16 lanes, lane i offers the four columns 16 dt + 4 (i % 4) .. of key 4 g + i / 4 (+ 32 cc),
