@@ -10,6 +10,7 @@ from __future__ import annotations
 from typing import Optional, Union
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -123,6 +124,13 @@ class Infllmv2AttnVarlenFunc(torch.autograd.Function):
         return (dq, dk, dv) + (None,) * 15
 
 
+def _differentiated(*tensors):
+    """Whether autograd has to see an operator on these tensors: one requires a gradient, or carries a forward-mode
+    tangent (which does not set ``requires_grad``; the operator has no forward-mode derivative, and its node says so)."""
+    return (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)) or any(
+        forward_ad.unpack_dual(t).tangent is not None for t in tensors)
+
+
 def infllmv2_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p=0.0,
                               softmax_scale=None, causal=False, window_size=(-1, -1), softcap=0.0,
                               alibi_slopes=None, deterministic=False, return_attn_probs=False, block_table=None,
@@ -151,8 +159,7 @@ def infllmv2_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
         softmax_scale = head_size_og ** (-0.5)
     if head_size_og != HEAD_DIM and q.dim() == 3 and k.dim() == 3 and v.dim() == 3:
         q, k, v = pad_head_dim(q, k, v)
-    if not return_attn_probs and head_size_og == HEAD_DIM and not (
-            torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)):
+    if not return_attn_probs and head_size_og == HEAD_DIM and not _differentiated(q, k, v):
         # nothing to differentiate: skip the autograd node (it costs as much host time as the launches)
         return _varlen_forward(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p, softmax_scale, causal,
                                window_size, softcap, alibi_slopes, block_table, topk_idx, block_mask)[3]

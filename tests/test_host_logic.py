@@ -57,3 +57,33 @@ def test_native_module_binds_the_reference_names():
     with pytest.raises(RuntimeError, match="does not support softcap"):
         C.fwd_kvcache(z(1, 1, 32, 128), z(1, 64, 2, 128), z(1, 64, 2, 128), None, None, None, None, None, None, None, None,
                       None, None, 0.088, False, -1, -1, 1.0, True, 0, None)
+
+
+def _stub_forward(monkeypatch):
+    """The operator's host call replaced by one that runs without a GPU: what is tested is the route to it."""
+    from types import SimpleNamespace
+    import torch
+    from infllmv2_cuda_impl_amd import _lib
+    monkeypatch.setattr(_lib, "host", SimpleNamespace(varlen_fwd=lambda q, k, *rest: (q * 1.0, torch.zeros(q.shape[1], q.shape[0]), None)))
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+@pytest.mark.parametrize("grad", [False, True])
+def test_tangents_are_not_dropped(monkeypatch, which, grad):
+    """A forward-mode tangent on q, k or v does not set requires_grad; the operator has no forward-mode derivative and says so."""
+    import torch
+    import torch.autograd.forward_ad as fwd
+    from infllmv2_cuda_impl_amd import infllmv2_attn_varlen_func
+    _stub_forward(monkeypatch)
+    qkv = [torch.randn(4, 32, 128), torch.randn(4, 2, 128), torch.randn(4, 2, 128)]
+    cu = torch.tensor([0, 4], dtype=torch.int32)
+    f = lambda *t: infllmv2_attn_varlen_func(*t, cu, cu, 4, 4, causal=True)
+    with torch.set_grad_enabled(grad):
+        assert torch.equal(f(*qkv), qkv[0])
+        with fwd.dual_level():
+            assert torch.equal(f(*qkv), qkv[0])                # no tangent: as outside
+            qkv[which] = fwd.make_dual(qkv[which], torch.ones_like(qkv[which]))
+            with pytest.raises(RuntimeError, match="jvp"):
+                f(*qkv)
+        with pytest.raises(RuntimeError):                      # neither are torch.func's transforms served
+            torch.func.jvp(f, tuple(torch.zeros_like(t) for t in (qkv[0], qkv[1], qkv[2])), tuple(torch.ones_like(t) for t in (qkv[0], qkv[1], qkv[2])))
