@@ -604,12 +604,14 @@ std::tuple<Tensor, Tensor> decode_front(const Tensor& q, const Tensor& kn, const
     for (const OptTensor* t : {&lens, &fine_lens_, &coarse_lens_})
         TORCH_CHECK(!t->has_value() || ((*t)->scalar_type() == at::kInt && (*t)->dim() == 1 && (*t)->size(0) == batch && (*t)->is_contiguous() &&
                                         (*t)->device() == q.device()), "lengths must be contiguous int32 tensors of shape (batch_size)");
-    TORCH_CHECK(block_size == kBlock && (!scores || (stride * 4 == block_size)), "only 64-token blocks over stride-16 compressed keys are fused");
+    // four compressed keys per block, as the pooling of stage1_pooled and stage1_kvcache; without scores nothing looks at the blocks
+    TORCH_CHECK(!scores || (block_size == kBlock && stride > 0 && block_size / stride == 4),
+                "only 64-token blocks over stride-16 compressed keys are fused");
     const auto ints = q.options().dtype(at::kInt);
     Tensor new_lens = at::empty({batch}, ints);
     const Tensor fine_lens = fine_lens_.has_value() ? *fine_lens_ : at::empty({batch}, ints);
     const Tensor coarse_lens = coarse_lens_.has_value() ? *coarse_lens_ : at::empty({batch}, ints);
-    const int64_t out_len = (max_len + block_size - 1) / block_size;
+    const int64_t out_len = scores ? (max_len + block_size - 1) / block_size : 0;
     Tensor pooled, ws;
     if (scores) {
         pooled = at::empty({batch, hk, out_len}, q.options());

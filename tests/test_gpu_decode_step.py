@@ -159,3 +159,36 @@ def test_selection_inside_the_attention_equals_topk(dtype, topk, tied):
         splits = min(_lib.lib.infllmv2_fwd_kvcache_num_splits(mask.shape[0], Hk, 0), (topk + 3) // 4)
         want = ops.infllmv2_attn_with_kvcache(q[s], k[s], v[s], cache_seqlens=n2, block_mask=mask, num_splits=splits)
         assert torch.equal(n1, n2) and torch.equal(out, want)
+
+
+@pytest.mark.parametrize("opt", [{"selection": "dense", "block_size": 128}, {"selection": "dense", "block_size": 32, "stride": 8, "kernel_size": 16},
+                                 {"selection": "sparse", "dense_len": 1 << 20, "block_size": 128}, {"selection": "sparse", "stride": 15}])
+def test_steps_of_layers_with_other_block_sizes_and_strides(opt):
+    """Where nothing is scored the block size is not looked at; where blocks are scored, the strides that put four compressed keys on a
+    block.  Against the operators called one by one."""
+    import infllmv2_cuda_impl_amd as ops
+    layer = ops.InfLLMv2Attention(topk=4, local_blocks=1, **opt)
+    ks, st = layer.kernel_size, layer.stride
+    g = torch.Generator(device="cuda").manual_seed(3)
+    mk = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    n, Hk = 1000, 2
+    one, batch = [c.empty(*a, n + 64, Hk, 128, "cuda", stride=st) for c, a in ((ops.SequenceCache, ()), (ops.BatchCache, (2,)))]
+    k, v = mk(2 * n, Hk, 128), mk(2 * n, Hk, 128)
+    layer.fill_cache(batch, k, v, [n, n])
+    one.k[0, :n], one.v[0, :n], one.length = k[:n], v[:n], n
+    layer._extend_compressed(one, 0)
+    for step in range(3):
+        q, kn, vn = mk(2, 1, 32, 128), mk(2, 1, Hk, 128), mk(2, 1, Hk, 128)
+        out1, out2 = layer.decode(q[:1], kn[:1], vn[:1], one), layer.decode_batch(q, kn, vn, batch)
+        held = batch.lengths - 1
+        assert torch.equal(one.k[0, n + step], kn[0, 0]) and torch.equal(batch.k[:, n + step], kn[:, 0]) and int(held[0]) == n + step
+        idx = None
+        if layer.selection == "sparse" and layer.dense_len == 0:
+            f, c = torch.zeros_like(batch.k_fine), torch.zeros_like(batch.k_coarse)
+            fl, cl = ops.compress_keys_cache_pair(batch.k, batch.lengths, (ks, st, f), (4 * ks, 4 * st, c))
+            assert torch.equal(fl, batch.fine_lens) and torch.equal(cl, batch.coarse_lens)
+            pooled = ops.infllmv2_attn_stage1_kvcache(q, f, c, fl, cl, held, layer.local_blocks, layer.init_blocks, max_cache_len=n + step, stride=st)
+            idx = ops.topk_blocks(pooled, layer.topk).unsqueeze(2)
+        want = ops.infllmv2_attn_with_kvcache(q, batch.k, batch.v, cache_seqlens=batch.lengths, topk_idx=idx)
+        assert (out2.float() - want.float()).abs().max() <= 8e-3          # the runs may be cut differently
+        assert (out1.float() - want[:1].float()).abs().max() <= 8e-3
