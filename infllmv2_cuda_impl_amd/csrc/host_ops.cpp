@@ -607,6 +607,10 @@ std::tuple<Tensor, Tensor> decode_front(const Tensor& q, const Tensor& kn, const
     // four compressed keys per block, as the pooling of stage1_pooled and stage1_kvcache; without scores nothing looks at the blocks
     TORCH_CHECK(!scores || (block_size == kBlock && stride > 0 && block_size / stride == 4),
                 "only 64-token blocks over stride-16 compressed keys are fused");
+    // with the length at hand, as compress_keys checks it: a compressed key that has no row is refused, not dropped
+    for (const auto& [t, kernel, st] : {std::tuple(&fine, kernel_size, stride), std::tuple(&coarse, 4 * kernel_size, 4 * stride)})
+        TORCH_CHECK(lens.has_value() || st <= 0 || windows(host_len + 1, kernel, st) == windows(host_len, kernel, st) ||
+                    t->size(1) >= windows(host_len + 1, kernel, st), "out must be a contiguous (rows, num_heads_k, head_size) buffer of k's dtype");
     const auto ints = q.options().dtype(at::kInt);
     Tensor new_lens = at::empty({batch}, ints);
     const Tensor fine_lens = fine_lens_.has_value() ? *fine_lens_ : at::empty({batch}, ints);

@@ -192,3 +192,20 @@ def test_steps_of_layers_with_other_block_sizes_and_strides(opt):
         want = ops.infllmv2_attn_with_kvcache(q, batch.k, batch.v, cache_seqlens=batch.lengths, topk_idx=idx)
         assert (out2.float() - want.float()).abs().max() <= 8e-3          # the runs may be cut differently
         assert (out1.float() - want[:1].float()).abs().max() <= 8e-3
+
+
+@pytest.mark.parametrize("selection", ["sparse", "dense"])
+@pytest.mark.parametrize("which, rows, last", [("k_fine", 3, 79), ("k_coarse", 1, 191)])
+def test_a_compressed_cache_without_room_is_refused(selection, which, rows, last):
+    """One sequence: the step that completes a window (the fourth of 32/16 with token 80, the second of 128/64 with token 192) finds no
+    row for its mean."""
+    import infllmv2_cuda_impl_amd as ops
+    layer = ops.InfLLMv2Attention(topk=2, local_blocks=0, selection=selection)
+    cache = ops.SequenceCache.empty(256, 1, 128, "cuda")
+    setattr(cache, which, getattr(cache, which)[:rows])
+    mk = lambda h: torch.randn(1, 1, h, 128, device="cuda").to(torch.bfloat16)
+    cache.length = last - 1
+    layer.decode(mk(16), mk(1), mk(1), cache)
+    with pytest.raises(RuntimeError, match="out must be a contiguous"):
+        layer.decode(mk(16), mk(1), mk(1), cache)
+    assert cache.length == last
