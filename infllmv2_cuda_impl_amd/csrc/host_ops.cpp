@@ -642,6 +642,7 @@ std::tuple<Tensor, OptTensor> decode_step(const Tensor& q, const Tensor& kn, con
                                           const OptTensor& fine_lens, const OptTensor& coarse_lens, int64_t max_len, int64_t kernel_size,
                                           int64_t stride, int64_t block_size, int64_t topk, int64_t local_blocks, int64_t init_blocks,
                                           double scale) {
+    require_gpu(q, "q");
     DeviceGuard guard(q.device());
     auto [new_lens, pooled] = decode_front(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, max_len, kernel_size,
                                            stride, block_size, topk > 0, local_blocks, init_blocks, scale);
@@ -659,6 +660,7 @@ std::tuple<Tensor, Tensor> decode_sparse(const Tensor& q, const Tensor& kn, cons
                                          int64_t stride, int64_t block_size, int64_t topk, int64_t local_blocks, int64_t init_blocks,
                                          double scale) {
     TORCH_CHECK(topk > 0, "decode_sparse: topk must be positive");
+    require_gpu(q, "q");
     DeviceGuard guard(q.device());
     auto [new_lens, pooled] = decode_front(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, max_len, kernel_size,
                                            stride, block_size, true, local_blocks, init_blocks, scale);

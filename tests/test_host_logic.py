@@ -87,3 +87,15 @@ def test_tangents_are_not_dropped(monkeypatch, which, grad):
                 f(*qkv)
         with pytest.raises(RuntimeError):                      # neither are torch.func's transforms served
             torch.func.jvp(f, tuple(torch.zeros_like(t) for t in (qkv[0], qkv[1], qkv[2])), tuple(torch.ones_like(t) for t in (qkv[0], qkv[1], qkv[2])))
+
+
+@pytest.mark.parametrize("selection", ["sparse", "dense", "window"])
+def test_decode_on_cpu_tensors_says_that_there_is_no_cpu_path(selection):
+    import torch
+    from infllmv2_cuda_impl_amd import BatchCache, InfLLMv2Attention, SequenceCache
+    layer = InfLLMv2Attention(selection=selection)
+    q, kv = torch.zeros(1, 1, 32, 128, dtype=torch.bfloat16), torch.zeros(1, 1, 2, 128, dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError, match="no CPU path"):
+        layer.decode(q, kv, kv, SequenceCache.empty(128, 2, 128, "cpu"))
+    with pytest.raises(RuntimeError, match="no CPU path"):
+        layer.decode_batch(q, kv, kv, BatchCache.empty(1, 128, 2, 128, "cpu"))
