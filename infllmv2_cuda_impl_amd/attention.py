@@ -98,6 +98,8 @@ class Infllmv2AttnVarlenFunc(torch.autograd.Function):
     def forward(ctx, q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p, softmax_scale,
                 causal, window_size, softcap, alibi_slopes, deterministic, return_softmax, block_table, topk_idx,
                 block_mask=None):
+        if softmax_scale is None:
+            softmax_scale = q.shape[-1] ** (-0.5)
         q, k, v, out, lse, fwd_mask, causal = _varlen_forward(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p,
                                                               softmax_scale, causal, window_size, softcap, alibi_slopes, block_table,
                                                               topk_idx, block_mask)

@@ -99,3 +99,16 @@ def test_decode_on_cpu_tensors_says_that_there_is_no_cpu_path(selection):
         layer.decode(q, kv, kv, SequenceCache.empty(128, 2, 128, "cpu"))
     with pytest.raises(RuntimeError, match="no CPU path"):
         layer.decode_batch(q, kv, kv, BatchCache.empty(1, 128, 2, 128, "cpu"))
+
+
+def test_the_autograd_function_defaults_the_softmax_scale(monkeypatch):
+    """Infllmv2AttnVarlenFunc.apply with no scale: the head size to the power -1/2, as the operator defaults it."""
+    from types import SimpleNamespace
+    import torch
+    from infllmv2_cuda_impl_amd import _lib
+    from infllmv2_cuda_impl_amd.attention import Infllmv2AttnVarlenFunc
+    scales = []
+    monkeypatch.setattr(_lib, "host", SimpleNamespace(varlen_fwd=lambda q, k, v, cq, ck, mq, mk, scale, *rest: (scales.append(scale), (q * 1.0, q, None))[1]))
+    q, kv, cu = torch.zeros(4, 32, 128), torch.zeros(4, 2, 128), torch.tensor([0, 4], dtype=torch.int32)
+    Infllmv2AttnVarlenFunc.apply(q, kv, kv, cu, cu, 4, 4, 0.0, None, True, (-1, -1), 0.0, None, False, False, None, None)
+    assert scales == [128 ** -0.5]
