@@ -363,7 +363,7 @@ int infllmv2_fwd_kvcache_topk(void* stream, const void* q, void* kcache, void* v
 
 /* infllmv2_fwd_kvcache with the selection made by the same launch: the topk largest of the block scores of each row,
  * scores (batch, Hk, n_scores), dense, of the tensors' element type, as Stage 1 with pooling leaves them (no negative
- * value but -inf; n_scores <= INFLLMV2_DECODE_MAX_SCORES; batch x Hk x num_splits <= 256).  No new keys. */
+ * value but -inf, -0 counts as +0; n_scores <= INFLLMV2_DECODE_MAX_SCORES; batch x Hk x num_splits <= 256).  No new keys. */
 #define INFLLMV2_DECODE_MAX_SCORES 2048
 int infllmv2_fwd_kvcache_scores(void* stream, const void* q, void* kcache, void* vcache, const int32_t* cache_seqlens,
                                 void* out, float* softmax_lse, const void* scores, int n_scores, int topk,

@@ -219,7 +219,9 @@ __device__ __forceinline__ int scan_lanes(int v) {              // inclusive pre
 
 // The k largest of the first `cols` of a row of block scores (the order of topk.hip: larger first, ties by ascending column), by
 // a workgroup of four wavefronts; lane w of each gets mask word w.  Column 256 e + 64 wave + lane is key[e], as signed 16-bit
-// integers: scores of Stage 1 are never negative but for -inf, so that is their order, and -32768 is free for "no column".
+// integers: scores of Stage 1 are never negative but for -inf, so that is their order, and -32768, the bits of -0, which counts
+// as +0, is free for "no column".  Whatever bits the row holds, a round finds its k-th column in the histogram or starts
+// the next one 1023 keys further down: with a key on every column there are always k of them to find.
 // Bound by the instructions a wavefront issues one after the other (a lone one needs five clocks for each), so it spends few of
 // them per column: one histogram of the keys up to 1023 (eight powers of two) below the largest finite score, in LDS, two
 // scans over the lanes find the k-th key and how many columns equal it.  Halving the 16 bits by counts took three times as
@@ -245,7 +247,10 @@ __device__ __forceinline__ uint64_t select_words(const elem_bits* row, int n, in
     const int k = k_want < cols ? k_want : cols;
     if (k <= 0) return 0ull;                                   // uniform over the workgroup
 #pragma unroll
-    for (int e = 0; e < kItems; ++e) key[e] = 256 * e + tid < cols ? key[e] : kNoColumn;
+    for (int e = 0; e < kItems; ++e) {
+        key[e] = key[e] == kNoColumn ? 0 : key[e];             // -0
+        key[e] = 256 * e + tid < cols ? key[e] : kNoColumn;
+    }
     int limit = kElemPosInf - 1, thr, c_above, c_equal;        // the forced blocks (+inf) stay above the histogram
     for (int round = 0;; ++round) {
         int top = kNoColumn, above = 0;

@@ -209,3 +209,35 @@ def test_a_compressed_cache_without_room_is_refused(selection, which, rows, last
     with pytest.raises(RuntimeError, match="out must be a contiguous"):
         layer.decode(mk(16), mk(1), mk(1), cache)
     assert cache.length == last
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n", [70, 700])
+@pytest.mark.parametrize("topk", [1, 5, 64, 800])
+def test_selection_inside_the_attention_takes_signed_zeros(dtype, n, topk):
+    """Rows of -0 alone, of both zeros, with -inf and +inf among them: -0 and +0 tie, as in topk_blocks."""
+    import infllmv2_cuda_impl_amd as ops
+    from infllmv2_cuda_impl_amd import _lib
+    g = torch.Generator(device="cpu").manual_seed(n + topk)
+    z = torch.where(torch.rand(4, n, generator=g) < 0.5, -0.0, 0.0)
+    z[0] = -0.0
+    z[2] = torch.where(torch.rand(n, generator=g) < 0.3, torch.tensor(float("-inf")), z[2])
+    z[3] = torch.where(torch.rand(n, generator=g) < 0.1, torch.rand(n, generator=g), z[3])
+    z[3, 0], z[3, n - 1] = float("inf"), float("inf")
+    scores = z.to(dtype).cuda()
+    B, L = 4, 64 * n - 3
+    gc = torch.Generator(device="cuda").manual_seed(1)
+    mk = lambda *s: torch.randn(*s, generator=gc, device="cuda", dtype=dtype)
+    q, kc, vc = mk(B, 1, 16, 128), mk(B, 64 * n, 1, 128), mk(B, 64 * n, 1, 128)
+    lens = torch.full((B,), L, dtype=torch.int32, device="cuda")
+    splits = 4
+    out, lse = torch.empty_like(q), torch.empty((B, 16, 1), dtype=torch.float32, device="cuda")
+    ws = torch.empty(_lib.lib.infllmv2_fwd_kvcache_workspace_bytes(B, 1, splits), dtype=torch.uint8, device="cuda")
+    two, s3 = lambda t: _lib.i64_array([t.stride(0), t.stride(2)]), lambda t: _lib.i64_array(t.stride()[:3])
+    _lib.call_for(dtype, "infllmv2_fwd_kvcache_scores", torch.cuda.current_stream().cuda_stream, q.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+                  lens.data_ptr(), out.data_ptr(), lse.data_ptr(), scores.data_ptr(), n, topk, ws.data_ptr(), ws.numel(), B, 16, 1, 128, 64 * n,
+                  two(q), s3(kc), s3(vc), two(out), splits, 128 ** -0.5)
+    _, mask = ops.topk_blocks(scores, topk, return_mask=True)
+    want, want_lse = ops.infllmv2_attn_with_kvcache(q, kc, vc, cache_seqlens=lens, block_mask=mask.view(B, 1, 1, -1), num_splits=splits,
+                                                    return_softmax_lse=True)
+    assert torch.equal(out, want) and torch.equal(lse, want_lse)
