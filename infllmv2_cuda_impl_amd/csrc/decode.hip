@@ -55,6 +55,7 @@ struct DecodeParams {
     const elem_bits* rot_cos;       // (seqlen_ro, rotary_dim / 2)
     const elem_bits* rot_sin;
     int rotary_dim, rotary_interleaved;
+    int far_rows;                   // cache rows lie too far apart (or backwards) for 32-bit offsets inside a block
     int append_here;                // the split kernel itself writes the one new row per sequence (and sees it whatever the cache holds)
 };
 
@@ -171,6 +172,10 @@ __device__ __forceinline__ uint32_t decode_lds_address(const void* ptr) {
 // The compiler does not see these loads: whoever reads the tile waits for them by hand.
 __device__ __forceinline__ void decode_dma16(const void* base, uint32_t lane_off, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt" : : "v"(lane_off), "s"(base), "s"(lds) : "memory", "m0");
+}
+// the same from an address of each lane's own
+__device__ __forceinline__ void decode_dma16(const void* lane_src, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off nt" : : "v"(lane_src), "s"(lds) : "memory", "m0");
 }
 
 // v (wavefront-uniform, more than `rank` bits set) without its `rank` lowest set bits
@@ -503,16 +508,16 @@ void decode_split_kernel(const DecodeParams p) {
 
     // ---- block i of the run into slot i % kSlots ----
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(decode_lds_address(tiles));
-    const int k_pitch = static_cast<int>(p.kc_row) * 2, v_pitch = static_cast<int>(p.vc_row) * 2;   // bytes
+    const uint32_t k_pitch = static_cast<uint32_t>(p.kc_row) * 2u, v_pitch = static_cast<uint32_t>(p.vc_row) * 2u;   // bytes; not with far_rows
     uint32_t k_off[4], v_off[4];                               // this lane's piece of rows g, 4 + g, 8 + g, 12 + g
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-        k_off[u] = static_cast<uint32_t>((4 * u + g) * k_pitch + (n ^ tile_swizzle(4 * u + g)) * 16);
-        v_off[u] = static_cast<uint32_t>((4 * u + g) * v_pitch + (n ^ tile_swizzle(4 * u + g)) * 16);
+        k_off[u] = (4 * u + g) * k_pitch + (n ^ tile_swizzle(4 * u + g)) * 16;
+        v_off[u] = (4 * u + g) * v_pitch + (n ^ tile_swizzle(4 * u + g)) * 16;
     }
     // 16 DMA instructions for K or V of a block, which never straddles two pages (page_size is a multiple of 64 and paged
     // caches have no left padding)
-    auto request_tile = [&](int i, const elem_bits* cache, int64_t batch_stride, int64_t row_stride, int64_t head_stride, int pitch,
+    auto request_tile = [&](int i, const elem_bits* cache, int64_t batch_stride, int64_t row_stride, int64_t head_stride, uint32_t pitch,
                             const uint32_t (&off)[4], uint32_t tile) {
         const int jb = __builtin_amdgcn_readlane(my_block, i & 63), page = __builtin_amdgcn_readlane(my_page, i & 63);
         const int key0 = jb * kBlockN;
@@ -522,7 +527,13 @@ void decode_split_kernel(const DecodeParams p) {
         // the slot's previous tile has been read; and the sixteen addresses in it are no loop invariants worth a register each
         asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(slot) : : "memory");
         const int last = L - 1 - key0;
-        if (last >= kBlockN - 1) {
+        if (p.far_rows) {
+#pragma unroll 1
+            for (int u = 0; u < 16; ++u) {
+                const int row = 4 * u + g;
+                decode_dma16(base + (row < last ? row : last) * row_stride + (n ^ tile_swizzle(row)) * 8, slot + u * 1024);
+            }
+        } else if (last >= kBlockN - 1) {
 #pragma unroll
             for (int u = 0; u < 16; ++u) decode_dma16(base + (u >> 2) * 16 * row_stride, off[u & 3], slot + u * 1024);
         } else {
@@ -532,7 +543,7 @@ void decode_split_kernel(const DecodeParams p) {
             for (int u = 0; u < 16; ++u) {
                 int row = 4 * u + g;
                 row = row < last ? row : last;
-                decode_dma16(base, static_cast<uint32_t>(row * pitch + (n ^ tile_swizzle(4 * u + g)) * 16), slot + u * 1024);
+                decode_dma16(base, row * pitch + (n ^ tile_swizzle(4 * u + g)) * 16, slot + u * 1024);
             }
         }
     };
@@ -846,10 +857,10 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
     for (int s = 0; s < 3; ++s)
         IV2_CHECK(kcache_strides[s] % 8 == 0 && vcache_strides[s] % 8 == 0, "fwd_kvcache: cache strides must be multiples of 8 elements");
 
-    // a lane's offset inside a block is a 32-bit operand
-    IV2_CHECK(kcache_strides[1] >= 0 && kcache_strides[1] < (1 << 24) && vcache_strides[1] >= 0 && vcache_strides[1] < (1 << 24),
-              "fwd_kvcache: cache row strides must be below 2^24 elements");
     DecodeParams p{};
+    // a lane's offset inside a block is a 32-bit operand wherever it fits: up to 62 rows, or 15 and a piece of one
+    const auto far = [](int64_t row_stride) { return row_stride < 0 || row_stride >= (1 << 24); };
+    p.far_rows = far(kcache_strides[1]) || far(vcache_strides[1]) ? 1 : 0;
     p.q = static_cast<const elem_bits*>(q);
     p.kcache = static_cast<elem_bits*>(kcache);
     p.vcache = static_cast<elem_bits*>(vcache);

@@ -241,3 +241,49 @@ def test_selection_inside_the_attention_takes_signed_zeros(dtype, n, topk):
     want, want_lse = ops.infllmv2_attn_with_kvcache(q, kc, vc, cache_seqlens=lens, block_mask=mask.view(B, 1, 1, -1), num_splits=splits,
                                                     return_softmax_lse=True)
     assert torch.equal(out, want) and torch.equal(lse, want_lse)
+
+
+@pytest.mark.parametrize("batch", [1, 130])                    # workgroups of four wavefronts and, from 257 on, of one
+@pytest.mark.parametrize("both", [False, True])
+@pytest.mark.parametrize("held", [63, 64, 129])
+def test_cache_rows_far_apart(batch, both, held):
+    """Row strides of 2^24 elements, beyond what a 32-bit offset inside a block reaches; K alone, and K and V.  Equal to a dense cache bit
+    for bit.  All sequences of the larger batch read the same cache row."""
+    import infllmv2_cuda_impl_amd as ops
+    cap, Hk, far = 130, 2, 1 << 24
+    g = torch.Generator(device="cuda").manual_seed(held)
+    mk = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    k, v, q = mk(1, cap, Hk, 128), mk(1, cap, Hk, 128), mk(batch, 1, 32, 128)
+    kn, vn = (mk(1, 1, Hk, 128), mk(1, 1, Hk, 128)) if batch == 1 else (None, None)
+    room = torch.empty((cap - 1) * far + 2 * Hk * 128, dtype=torch.bfloat16, device="cuda")      # a row holds K, then V
+    part = lambda at: room[at:].as_strided((1, cap, Hk, 128), (cap * far, far, 128, 1))
+    k_far, v_far = part(0).copy_(k), part(Hk * 128).copy_(v) if both else v.clone()
+    opt = dict(k=kn, v=vn, cache_seqlens=torch.full((batch,), held, dtype=torch.int32, device="cuda"), return_softmax_lse=True,
+               cache_batch_idx=torch.zeros(batch, dtype=torch.int32, device="cuda"), num_splits=1)
+    out, lse = ops.infllmv2_attn_with_kvcache(q, k_far, v_far, **opt)
+    want, want_lse = ops.infllmv2_attn_with_kvcache(q, k, v, **opt)
+    assert torch.equal(out, want) and torch.equal(lse, want_lse) and torch.equal(k_far, k) and torch.equal(v_far, v)
+
+
+@pytest.mark.parametrize("held", [64, 127])
+def test_cache_rows_stored_backwards(held):
+    """Negative row strides, which the C ABI takes: row 0 of the cache is the last one in memory."""
+    from infllmv2_cuda_impl_amd import _lib
+    cap, Hk = 128, 2
+    g = torch.Generator(device="cuda").manual_seed(held)
+    mk = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    k, v, q = mk(1, cap, Hk, 128), mk(1, cap, Hk, 128), mk(1, 1, 32, 128)
+    L = torch.tensor([held], dtype=torch.int32, device="cuda")
+    back_k, back_v = k.flip(1).contiguous(), v.flip(1).contiguous()
+    zero3, row = _lib.i64_array([0, 0, 0]), Hk * 128
+
+    def call(kt, vt, sign):
+        first = 0 if sign > 0 else (cap - 1) * row * 2         # bytes
+        out, lse = torch.empty_like(q), torch.empty((1, 32, 1), dtype=torch.float32, device="cuda")
+        strides = lambda: _lib.i64_array([cap * row, sign * row, 128])
+        _lib.call("infllmv2_fwd_kvcache", torch.cuda.current_stream().cuda_stream, q.data_ptr(), kt.data_ptr() + first, vt.data_ptr() + first, None,
+                  None, L.data_ptr(), out.data_ptr(), lse.data_ptr(), None, None, 0, 1, 1, 32, Hk, 128, cap, 0, _lib.i64_array([32 * 128, 128]),
+                  strides(), strides(), zero3, zero3, _lib.i64_array([32 * 128, 128]), 0, 1, 128 ** -0.5, None, None, None, 0, 0, None, None, 0, 0)
+        return out, lse
+    for a, b in zip(call(k, v, 1), call(back_k, back_v, -1)):
+        assert torch.equal(a, b)
