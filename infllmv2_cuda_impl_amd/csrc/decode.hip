@@ -55,6 +55,7 @@ struct DecodeParams {
     const elem_bits* rot_cos;       // (seqlen_ro, rotary_dim / 2)
     const elem_bits* rot_sin;
     int rotary_dim, rotary_interleaved;
+    int mask_in_place;              // the mask has more words than LDS holds: read where they are
     int far_rows;                   // cache rows lie too far apart (or backwards) for 32-bit offsets inside a block
     int append_here;                // the split kernel itself writes the one new row per sequence (and sees it whatever the cache holds)
 };
@@ -402,8 +403,15 @@ void decode_split_kernel(const DecodeParams p) {
 
     // ---- the selected blocks: words in LDS, how many there are, and which run of them is this wavefront's ----
     // bits of words w0 + lane, and how many bits lie in words up to and including this lane's, from word w0 on
+    const uint64_t last_word_bits = (last_blk & 63) == 63 ? ~0ull : ((1ull << ((last_blk & 63) + 1)) - 1ull);
+    auto mask_word = [&](int w) -> uint64_t {
+        const uint64_t v = p.mask[pair * p.n64 + w];
+        return w == (last_blk >> 6) ? v & last_word_bits : v;
+    };
+    const bool in_place = kWaves == 1 && p.mask_in_place && n_words > 64;           // uniform: more words than LDS holds
     auto scan_words = [&](int w0, uint64_t& bits) -> int {
-        bits = w0 + lane < n_words ? words[w0 + lane] : 0ull;
+        if (in_place) bits = w0 + lane < n_words ? mask_word(w0 + lane) : 0ull;
+        else bits = w0 + lane < n_words ? words[w0 + lane] : 0ull;
         return scan_lanes(__builtin_popcountll(bits));
     };
     int total = 0, incl0 = 0;                                  // incl0, bits0: the first 64 words
@@ -422,7 +430,6 @@ void decode_split_kernel(const DecodeParams p) {
         total = last_blk + 1;
         lds_fence();
     } else {
-        const uint64_t last_word_bits = (last_blk & 63) == 63 ? ~0ull : ((1ull << ((last_blk & 63) + 1)) - 1ull);
         if (p.mask != nullptr && n_words <= 64) {              // straight into registers
             bits0 = lane < n_words ? (lane == (last_blk >> 6) ? bits0 & last_word_bits : bits0) : 0ull;
             incl0 = scan_lanes(__builtin_popcountll(bits0));
@@ -437,10 +444,7 @@ void decode_split_kernel(const DecodeParams p) {
                 else lds_fence();
             };
             if (p.mask != nullptr) {
-                for (int w = first; w < n_words; w += step) {
-                    const uint64_t v = p.mask[pair * p.n64 + w];
-                    words[w] = w == (last_blk >> 6) ? v & last_word_bits : v;
-                }
+                for (int w = in_place ? n_words : first; w < n_words; w += step) words[w] = mask_word(w);
             } else {
                 for (int w = first; w < n_words; w += step) words[w] = 0ull;
                 words_fence();
@@ -462,7 +466,8 @@ void decode_split_kernel(const DecodeParams p) {
     }
     // equal runs: their lengths differ by one at most
     const int runs = p.splits * kWaves, run = split * kWaves + wave;
-    int each = static_cast<int>(static_cast<float>(total) * __builtin_amdgcn_rcpf(static_cast<float>(runs)));       // total / runs (total < 2^20), off by one at most
+    int each = static_cast<int>(static_cast<float>(total) * __builtin_amdgcn_rcpf(static_cast<float>(runs)));       // total / runs, off by one at most
+    if (total >= 1 << 20) each = total / runs;                 // where it might be off by more; integer division is a long chain
     each = __builtin_amdgcn_readfirstlane(each);
     each += (each + 1) * runs <= total ? 1 : (each * runs > total ? -1 : 0);
     const int longer = total - each * runs;                    // so many runs take one block more
@@ -887,9 +892,14 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
     p.scores = static_cast<const elem_bits*>(scores); p.n_scores = n_scores; p.k_select = k_select;
     if (topk_idx != nullptr) p.n64 = ((cache_capacity + kBlockN - 1) / kBlockN + 63) / 64;
     // mask words of one row, kept in LDS beside the tiles; 8192 words are 33 million tokens, 2048 still fit beside four tiles
-    const size_t words = (blockmask || topk_idx) ? static_cast<size_t>(((cache_capacity + kBlockN - 1) / kBlockN + 63) / 64) : 0;
-    IV2_CHECK(words <= 8192, "fwd_kvcache: a cache of %d rows needs more mask words than the kernel holds", cache_capacity);
-    const bool grouped = static_cast<int64_t>(batch) * num_heads_k * num_splits <= kGroupedWorkgroups && words <= 2048;
+    constexpr size_t kMaxWords = 8192;
+    size_t words = (blockmask || topk_idx) ? ((static_cast<size_t>(cache_capacity) + kBlockN - 1) / kBlockN + 63) / 64 : 0;
+    IV2_CHECK(words <= kMaxWords || topk_idx == nullptr, "fwd_kvcache_topk: a cache of %d rows needs more mask words than the kernel holds", cache_capacity);
+    if (words > kMaxWords) {
+        p.mask_in_place = 1;
+        words = 0;
+    }
+    const bool grouped = static_cast<int64_t>(batch) * num_heads_k * num_splits <= kGroupedWorkgroups && words <= 2048 && !p.mask_in_place;
     IV2_CHECK(scores == nullptr || (grouped && n_scores > 0 && n_scores <= INFLLMV2_DECODE_MAX_SCORES && k_select > 0),
               "fwd_kvcache_scores: 1 to %d block scores per row, topk >= 1 and at most %d (sequence, KV head, split) triples are served",
               INFLLMV2_DECODE_MAX_SCORES, kGroupedWorkgroups);

@@ -287,3 +287,31 @@ def test_cache_rows_stored_backwards(held):
         return out, lse
     for a, b in zip(call(k, v, 1), call(back_k, back_v, -1)):
         assert torch.equal(a, b)
+
+
+def test_a_mask_of_more_words_than_lds_holds():
+    """A paged cache of 8193 x 64 blocks (33.6 million rows, a few pages behind all of its table): the first sequence is that long, with
+    blocks selected in the first and the last words; the second has 70 words, the third one.  Equal to the same blocks as short sequences."""
+    import infllmv2_cuda_impl_amd as ops
+    Hk, pages, words = 1, 8, 8193
+    g = torch.Generator(device="cuda").manual_seed(3)
+    mk = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    kc, vc, q = mk(pages, 64, Hk, 128), mk(pages, 64, Hk, 128), mk(3, 1, 16, 128)
+    blocks = words * 64
+    table = (torch.arange(blocks, dtype=torch.int32, device="cuda") % pages).expand(3, -1).contiguous()
+    picked = [[0, 7, 64 * 8192 + 5, blocks - 2, blocks - 1], [3, 4000, 4479], [1, 2]]
+    lens = [blocks * 64 - 17, 4480 * 64, 130]                  # the third's blocks beyond its end do not count
+    mask = torch.zeros(3, Hk, 1, words, dtype=torch.int64)
+    for b, js in enumerate(picked):
+        for j in js + [blocks - 3] * (b > 0):
+            mask[b, 0, 0, j // 64] |= -(2 ** 63) if j % 64 == 63 else 1 << (j % 64)
+    L = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    for splits in (1, 2):
+        out, lse = ops.infllmv2_attn_with_kvcache(q, kc, vc, cache_seqlens=L, block_table=table, block_mask=mask.cuda(), num_splits=splits,
+                                                  return_softmax_lse=True)
+        for b, js in enumerate(picked):
+            js = [j for j in js if j * 64 < lens[b]]
+            rows = lambda t: torch.cat([t[j % pages, :min(64, lens[b] - 64 * j)] for j in js])[:, 0].float()
+            s = q[b, 0].float() @ rows(kc).t().contiguous() * 128 ** -0.5
+            want = torch.softmax(s, -1) @ rows(vc)
+            assert (out[b, 0].float() - want).abs().max() <= 2e-2 and (lse[b, :, 0] - torch.logsumexp(s, -1)).abs().max() <= 2e-3
