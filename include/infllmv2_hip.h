@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define INFLLMV2_ABI_VERSION 13
+#define INFLLMV2_ABI_VERSION 14
 
 /* ---- library ------------------------------------------------------------------------------ */
 
@@ -249,6 +249,11 @@ int infllmv2_decode_step_scores(void* stream, const void* q, const void* k_new, 
 
 /* Scratch needed by infllmv2_varlen_fwd / _bwd for the fragment-major K/V block images. */
 size_t infllmv2_kv_image_bytes(int64_t total_k, int batch, int num_heads_k);
+
+/* Whether infllmv2_varlen_fwd without a blockmask walks these sizes by tiles of 256 query rows (1) or by groups of 8
+ * tokens (0): the same results either way, rounded apart. */
+int infllmv2_varlen_fwd_dense_tiles(int batch, int64_t total_q, int64_t total_k, int num_heads, int num_heads_k,
+                                    int max_seqlen_q, int max_seqlen_k, int is_causal);
 
 /* csrc/entry.cu:14,210 `varlen_fwd` = mha_varlen_fwd (csrc/flash_attn/flash_api.cpp:519-782) on
  * the sparse path (blockmask given) and on the dense path (blockmask null).

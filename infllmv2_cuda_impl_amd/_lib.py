@@ -11,7 +11,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libinfllmv2_hip.so")
 
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 _p, _i, _i64, _sz, _f = C.c_void_p, C.c_int, C.c_int64, C.c_size_t, C.c_float
 
@@ -57,6 +57,7 @@ OTHER = {
     "infllmv2_last_error": (C.c_char_p, []),
     "infllmv2_abi_version": (_i, []),
     "infllmv2_kv_image_bytes": (_sz, [_i64, _i, _i]),
+    "infllmv2_varlen_fwd_dense_tiles": (_i, [_i, _i64, _i64] + [_i] * 5),
     "infllmv2_stage1_decode_workspace_bytes": (_sz, [_i, _i, _i, _i]),
     "infllmv2_fwd_kvcache_workspace_bytes": (_sz, [_i, _i, _i]),
     "infllmv2_fwd_kvcache_num_splits": (_i, [_i, _i, _i]),

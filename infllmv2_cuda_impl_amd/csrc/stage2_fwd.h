@@ -17,7 +17,7 @@ struct FwdParams {
     int64_t o_tok_stride, o_grp_stride, o_kvh_stride;
     int64_t lse_tok_stride, lse_grp_stride, lse_kvh_stride;
     int64_t n_slots;
-    int64_t total_q;
+    int64_t total_q, total_k;
     int n64;
     int group;                      // query heads per KV head, 1..16: MFMA rows >= group repeat head group - 1 and are never stored
     float scale_log2;               // softmax_scale * log2(e)
@@ -34,9 +34,7 @@ inline int tiles_per_sequence(int group, int max_seqlen_q) {
     const int tokens = 256 >> tile_row_shift(group);
     return (max_seqlen_q + tokens - 1) / tokens;
 }
-// From about a tile per CU on: with fewer, the hybrid walk's groups of 8 tokens fill the chip better (us, hybrid walk | tiles: 188 tiles
-// 45 | 55, 226 61 | 63, 250 72 | 68, 252 in two sequences 55 | 45, 440 in five 63 | 58).
-constexpr int kMinTiles = 240;
+bool dense_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal);
 int launch_stage2_fwd_tile(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q,
                            int max_seqlen_k, bool causal);
 

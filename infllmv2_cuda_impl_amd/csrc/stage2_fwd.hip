@@ -185,7 +185,7 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_fwd)(void* stream, const void* q, const
     fp.o_tok_stride = o_strides[0]; fp.o_grp_stride = o_strides[1]; fp.o_kvh_stride = o_strides[2];
     fp.lse_tok_stride = lse_strides[0]; fp.lse_grp_stride = lse_strides[1]; fp.lse_kvh_stride = lse_strides[2];
     fp.n_slots = n_slots;
-    fp.total_q = total_q;
+    fp.total_q = total_q; fp.total_k = total_k;
     fp.group = num_heads / num_heads_k;
     fp.n64 = n_uint64_per_row;
     fp.scale_log2 = softmax_scale * 1.44269504088896340736f;

@@ -390,7 +390,7 @@ int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int 
     const int64_t total = static_cast<int64_t>(num_heads_k) * batch * x.groups_per_seq;
     IV2_CHECK(total <= 0x3fffffff, "varlen_fwd: too many token groups");
     IV2_CHECK((max_seqlen_k + kBlockN - 1) / kBlockN <= kMaxMaskWords * 64, "varlen_fwd: more than %d key blocks per sequence", kMaxMaskWords * 64);
-    if (p.mask == nullptr && static_cast<int64_t>(num_heads_k) * batch * tiles_per_sequence(p.group, max_seqlen_q) >= kMinTiles)
+    if (p.mask == nullptr && dense_tiles_pay(batch, num_heads_k, p.group, p.total_q, p.total_k, max_seqlen_q, max_seqlen_k, causal))
         return launch_stage2_fwd_tile(st, p, batch, num_heads_k, max_seqlen_q, max_seqlen_k, causal);
     x.total_groups = static_cast<int>(total);
     x.mask_words = ((max_seqlen_k + kBlockN - 1) / kBlockN + 63) / 64;

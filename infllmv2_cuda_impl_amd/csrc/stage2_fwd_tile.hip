@@ -22,6 +22,7 @@
 #include "block_walker.h"
 #include "lds_dma.h"
 #include "stage2_fwd.h"
+#include "infllmv2_hip.h"
 #include <math.h>
 
 namespace IV2_NS {
@@ -303,6 +304,42 @@ void stage2_fwd_tile_kernel(const FwdParams p, const TileExtra x) {
     }
 }
 
+// Time of a dense launch whose workgroups take `tokens` tokens each, one workgroup per CU at a time: in microseconds, but for what all
+// launches share.  A workgroup costs `fixed` and `block` per key block; a launch takes as long as its longest walk, or as the
+// work of all of them on 256 CUs with a last round that is `partial` of one more; workgroups behind the end of a sequence, which
+// return at once, 1.7 ns each.  The host knows the longest sequence and the totals: the others are taken to be of equal length.
+static double dense_walk_time(int tokens, double fixed, double block, double partial, int batch, int num_heads_k, int64_t total_q,
+                              int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal) {
+    auto blocks = [&](double q, double k) {                    // of a workgroup of a sequence, on average
+        const double first = causal ? (k > q ? k - q : 0.) : k;
+        return q > tokens ? (first + k) / (2 * kBlockN) + 0.5 : ceil(k / kBlockN);
+    };
+    const int others = batch - 1;
+    const double q = others > 0 && total_q > max_seqlen_q ? static_cast<double>(total_q - max_seqlen_q) / others : 0.;
+    const double k = others > 0 && total_k > max_seqlen_k ? static_cast<double>(total_k - max_seqlen_k) / others : 0.;
+    const double of_longest = ceil(static_cast<double>(max_seqlen_q) / tokens), of_others = others * ceil(q / tokens);
+    const double rounds = num_heads_k * (of_longest + of_others) / 256.;
+    const double each = fixed + block * (of_longest * blocks(max_seqlen_q, max_seqlen_k) + of_others * blocks(q, k)) / (of_longest + of_others);
+    const double chain = fixed + block * ceil(static_cast<double>(max_seqlen_k) / kBlockN);
+    const double all = each * (rounds + (rounds > 1. ? partial : 0.));
+    return (chain > all ? chain : all) + 0.0017 * num_heads_k * batch * of_longest;
+}
+
+// Whether a forward without a mask goes by tiles: a tile walks a block in 1.5 us, the hybrid walk's group of 8 tokens in 1.0, so tiles
+// win where there is more work than the longest chain and lose where that chain, or the rounding up to whole tiles, decides.
+// The constants are a fit to 359 launches of 1 to 300 sequences of 4 to 20000 tokens over up to 16000 keys, 1 to 8 KV heads, groups of 8 and
+// 16 (within 15 to 17 %); the choice costs 0.3 % of the better walk's time on average and over 10 % in one of them.  A number of
+// tiles alone, 240, cost 3.3 % and up to 45 (us, hybrid walk | tiles; * the one taken here):
+//   1 KV head:  3800 tokens 88 * | 101, 5000 143 | 136 *, 16000 1080 | 894 *
+//   2 KV heads: 1000 tokens 27 * | 37, 2000 62 | 61 *, 16000 2132 | 1769 *; with groups of 8 3800 tokens 152 | 105 *
+//   2 KV heads: 1000 and 3 x 16 tokens 30 * | 39; 4000 and 100 x 16 316 | 233 *; 80 x 24 21 * | 31; 2 x 300 over 6300 keys (4 heads) 209 | 163 *
+bool dense_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal) {
+    if (max_seqlen_q <= 0) return false;
+    const double tiles = dense_walk_time(kTileRows >> tile_row_shift(group), 10., 1.5, 0.75, batch, num_heads_k, total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
+    const double groups = dense_walk_time(8, 6., 1., 0.7, batch, num_heads_k, total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
+    return tiles < groups + 1.;
+}
+
 int launch_stage2_fwd_tile(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q, int max_seqlen_k, bool causal) {
     TileExtra x{};
     x.batch = batch;
@@ -324,3 +361,11 @@ int launch_stage2_fwd_tile(hipStream_t st, const FwdParams& p, int batch, int nu
 }
 
 }  // namespace IV2_NS
+
+#ifndef IV2_F16        // element-type independent: defined once
+extern "C" int infllmv2_varlen_fwd_dense_tiles(int batch, int64_t total_q, int64_t total_k, int num_heads, int num_heads_k, int max_seqlen_q,
+                                               int max_seqlen_k, int is_causal) {
+    return num_heads_k > 0 && batch > 0 && IV2_NS::dense_tiles_pay(batch, num_heads_k, num_heads / num_heads_k, total_q, total_k, max_seqlen_q,
+                                                                   max_seqlen_k, is_causal != 0) ? 1 : 0;
+}
+#endif

@@ -18,8 +18,16 @@ CASES = [  # query lengths, key lengths, KV heads, group, mask
     ([2100, 90], [1030, 33], 2, 16, "none"),                  # the first queries see no key
     ([2070, 700], [2070, 700], 4, 8, "none"),
     ([2070, 700], [2070, 700], 4, 4, "none"),
-    ([1920], [1920], 2, 16, "none"),                          # 240 tiles
-    ([1904], [1904], 2, 16, "none"),                          # 238: the walk by groups of eight
+    ([1920], [1920], 2, 16, "none"),
+    ([1904], [1904], 2, 16, "none"),
+    ([1000] + [16] * 30, [1000] + [16] * 30, 4, 16, "none"),  # one long, many short: most workgroups return at once
+    ([2100], [2100], 2, 8, "none"),
+]
+GROUP_CASES = [  # the same without a mask, walked by groups of eight tokens
+    ([1700], [1700], 2, 16, "none"),
+    ([1000] + [16] * 3, [1000] + [16] * 3, 2, 16, "none"),
+    ([24] * 80, [24] * 80, 2, 16, "none"),
+    ([130] * 15, [1130] * 15, 2, 16, "acausal"),
 ]
 
 
@@ -53,7 +61,7 @@ def reference(q, k, v, sq, sk, Hk, group, causal):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("sq, sk, Hk, group, kind", CASES)
+@pytest.mark.parametrize("sq, sk, Hk, group, kind", CASES + GROUP_CASES)
 def test_tile_walk(sq, sk, Hk, group, kind, dtype):
     import infllmv2_cuda_impl_amd as ops
     dev = torch.device("cuda:0")

@@ -112,3 +112,23 @@ def test_the_autograd_function_defaults_the_softmax_scale(monkeypatch):
     q, kv, cu = torch.zeros(4, 32, 128), torch.zeros(4, 2, 128), torch.tensor([0, 4], dtype=torch.int32)
     Infllmv2AttnVarlenFunc.apply(q, kv, kv, cu, cu, 4, 4, 0.0, None, True, (-1, -1), 0.0, None, False, False, None, None)
     assert scales == [128 ** -0.5]
+
+
+def test_which_walk_a_dense_forward_takes():
+    """Sizes at which both walks were timed and differ by more than the timings scatter (query lengths, keys before the first query, KV
+    heads, group, by tiles); a number of tiles taken from the longest sequence, or a number of tiles alone, gets several of them wrong."""
+    from infllmv2_cuda_impl_amd import _lib
+    from test_gpu_tile_walk import CASES, GROUP_CASES
+    f = lambda sq, sk, hk, g, causal=True: bool(_lib.lib.infllmv2_varlen_fwd_dense_tiles(len(sq), sum(sq), sum(sk), hk * g, hk, max(sq), max(sk), int(causal)))
+    for sq, before, hk, g, tiles in (([3800], 0, 1, 16, False), ([5000], 0, 1, 16, True), ([16000], 0, 1, 16, True), ([1000], 0, 2, 16, False),
+                                     ([2200], 0, 2, 16, True), ([1000], 0, 4, 16, True), ([3800], 0, 2, 8, True), ([800], 0, 8, 8, True),
+                                     ([1000] + [16] * 3, 0, 2, 16, False), ([1000] + [16] * 30, 0, 4, 16, True), ([4000] + [16] * 100, 0, 2, 16, True),
+                                     ([24] * 80, 0, 2, 16, False), ([17] * 130, 0, 2, 16, False), ([130] * 15, 2000, 2, 16, False), ([300] * 2, 6000, 4, 16, True),
+                                     ([300] * 2, 6000, 2, 16, False)):
+        assert f(sq, [n + before for n in sq], hk, g) == tiles, (sq[:3], len(sq), before, hk, g)
+    for sizes in ((0, 0, 0), (1, 1, 0), (1, 1, 1), (2 ** 31 - 1, 2 ** 31 - 1, 2 ** 31 - 1)):
+        assert _lib.lib.infllmv2_varlen_fwd_dense_tiles(1, sizes[0], sizes[1], 32, 2, sizes[0], sizes[2], 1) in (0, 1)
+    # the cases of the GPU test take the walk they are there for
+    for cases, tiles in ((CASES, True), (GROUP_CASES, False)):
+        for sq, sk, hk, g, kind in cases:
+            assert kind == "all" or f(sq, sk, hk, g, kind != "acausal") == tiles, (sq[:3], len(sq), hk, g)
