@@ -11,7 +11,7 @@
 // next.  Left to the compiler, which forms clumps of MFMAs and of exponentials, the same work takes 2310 us for 16384 tokens of 2 KV heads
 // instead of 1980 (there the matrix pipe was busy 48 % of the time, LDS reads free of conflicts).
 // Operator with 2 KV heads, us, hybrid walk -> this one: 2000 tokens 72 -> 68, 4096 219 -> 160, 16384 2430 -> 1980 (1.11 PFLOP/s), 50000
-// 20370 -> 17100 (1.2 PFLOP/s), 2500 + 6001 + 4096 665 -> 555, 777 + 5003 + 1291 + 9173 1160 -> 950.
+// 20370 -> 17100 (1.2 PFLOP/s), 2500 + 6001 + 4096 566 -> 472, 777 + 5003 + 1291 + 9173 1160 -> 950.
 //
 // Operands.  S^T = K Q^T: lane (n = lane % 32, h = lane / 32) holds key n of a 32-key chunk, d = 16 ks + 8 h + j: one 16-byte unit of
 // the K image.  The accumulators hold keys 8 i + 4 h + e (register 4 i + e) of row n; a V image unit holds keys 4 g + e and
@@ -70,14 +70,8 @@ void stage2_fwd_tile_kernel(const FwdParams p, const TileExtra x) {
     //      that shares work round robin: each keeps to one head where there are two, four or eight).  Tiles behind the end of a sequence
     //      are then a run of workgroups that return at once.  With the sequences innermost instead (all longest prefixes first) the live
     //      workgroups came at a fixed distance, which the dispatcher maps to the same few shader engines: 1890 us instead of
-    //      TTT us for 777, 5003, 1291 and 9173 tokens. ----
-#if ROT == 1
-    int G = (blockIdx.x & ~7) + ((blockIdx.x + (blockIdx.x >> 3)) & 7);
-#elif ROT == 2
-    int G = (blockIdx.x & ~7) + ((blockIdx.x + (blockIdx.x >> 4)) & 7);
-#else
+    //      950 for 777, 5003, 1291 and 9173 tokens. ----
     int G = blockIdx.x;
-#endif
     if (G >= x.sequences * x.tiles_per_seq) return;                                 // uniform per workgroup
     const int h_kv = G % x.heads_k;
     G /= x.heads_k;
