@@ -2,6 +2,8 @@
 wavefronts and of key blocks, queries fewer and more than the keys, causal and not, as many tiles as the path asks for and fewer; the same
 attention with a mask of everything takes the other walk.  Against fp32 softmax attention; tolerances of the forward tests: 2e-2 on a
 16-bit output of order one, 1e-3 on average, 2e-3 on the log-sum-exp."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -85,3 +87,42 @@ def test_tile_walk(sq, sk, Hk, group, kind, dtype):
         lse = lse.view(Hk, sum(sq), group).transpose(1, 2).reshape(Hk * group, sum(sq))
     both = torch.isinf(ref_lse) == torch.isinf(lse)
     assert both.all() and (torch.nan_to_num(lse - ref_lse, nan=0.0).abs() <= 2e-3).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("group", [16, 8])
+@pytest.mark.parametrize("gain", [1.0, 6.0])
+def test_tile_walk_with_a_reference_exponent_that_moves(dtype, group, gain):
+    """Rows whose largest score arrives late: a key that is a multiple of one query head's vector, in the row's first, a middle and its last
+    block, with a logit far above the rest, so that the block's scores are formed again with sums and outputs that are not zero; with gain 6 the
+    running maxima of all rows move on top of that.  Tokens at the ends of wavefronts and tiles."""
+    import infllmv2_cuda_impl_amd as ops
+    from infllmv2_cuda_impl_amd import _lib
+    S, Hk = 2203, 2
+    assert _lib.lib.infllmv2_varlen_fwd_dense_tiles(1, S, S, Hk * group, Hk, S, S, 1) == 1
+    g = torch.Generator(device="cpu").manual_seed(11)
+    q = (torch.randn(S, Hk * group, 128, generator=g) * gain).to(dtype)
+    k, v = torch.randn(S, Hk, 128, generator=g).to(dtype), torch.randn(S, Hk, 128, generator=g).to(dtype)
+    planted = []
+    for i, t in enumerate((S - 1, 2202 - 70, 2047, 2048, 1601, 1600, 1599, 1057, 700, 335, 97, 64, 63)):
+        for j, key in enumerate((t, 64 * (t // 128) + 11, 5 + i)):                # last, middle and first block of the token
+            h, head = (i + j) % Hk, (5 * i + 3 * j) % group
+            row = q[t, h * group + head].float()
+            k[key, h] = (row / row.norm() * 60.0).to(dtype)
+            planted.append((t, h * group + head, h, key))
+    cu = torch.tensor([0, S], dtype=torch.int32).cuda()
+    q, k, v = q.cuda(), k.cuda(), v.cuda()
+    out, lse, _ = ops.infllmv2_attn_varlen_func(q, k, v, cu, cu, S, S, causal=True, return_attn_probs=True)
+    ref, ref_lse = reference(q, k, v, [S], [S], Hk, group, True)
+    err = (out.float() - ref).abs()
+    # outputs are convex combinations of rows of v whatever the logits: the tolerance of the file.  A logit is a sum of 128 products in fp32,
+    # good to 128 2^-24 of its size: that much more on the log-sum-exp.
+    assert err.max() <= 2e-2 and err.mean() <= 1e-3, (err.max().item(), err.mean().item())
+    assert ((lse - ref_lse).abs() <= 2e-3 + 128 * 2.0 ** -24 * ref_lse.abs()).all()
+    # the planted keys do dominate: most of them are their row's largest logit, by far more than the walk lets pass without a new reference
+    late = 0
+    for t, head, h, key in planted:
+        logits = (k[:t + 1, h].float() @ q[t, head].float()) * 128 ** -0.5
+        before = logits[:key // 64 * 64]
+        late += bool(key >= 64 and logits[key] > before.max() + 5 * math.log(2.0) + 2)
+    assert late >= 10, late
