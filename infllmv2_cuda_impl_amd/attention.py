@@ -194,7 +194,7 @@ def infllmv2_attn_stage1(q, k, v, cu_seqlens_q, cu_seqlens_k, cu_seqlens_v, max_
     if block_table is not None:
         raise RuntimeError("paged KV (block_table) is not supported by this build")
     return _lib.host.stage1_scores(_dense_last_dim(q), _dense_last_dim(k), _dense_last_dim(v), cu_seqlens_q, cu_seqlens_k, cu_seqlens_v,
-                                   max_seqlen_q, max_seqlen_k, softmax_scale, causal, 1)
+                                   max_seqlen_q, max_seqlen_k, softmax_scale, causal)
 
 
 def infllmv2_attn_stage1_pooled(q, k, v, cu_seqlens_q, cu_seqlens_k, cu_seqlens_v, max_seqlen_q, max_seqlen_k,

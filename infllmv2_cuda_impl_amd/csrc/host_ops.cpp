@@ -198,15 +198,14 @@ void check_stage1(const Tensor& q, const Tensor& k, const Tensor& v, const Tenso
 
 // Scores (Hk, total_q, max_seqlen_k).  The reference zero-fills a (Hk, T, round128(max_k)) buffer, slices it and replaces
 // NaNs in a further pass (flash_api.cpp:941, infllmv2_sparse_attention.py:587-589); here the kernel defines every element
-// once and produces no NaN.  row_pad_to > 1 lays the rows out with a padded stride (a view is returned).
+// once and produces no NaN.
 Tensor stage1_scores(const Tensor& q, const Tensor& k_, const Tensor& v_, const Tensor& cu_q, const Tensor& cu_k, const Tensor& cu_v,
-                     int64_t max_q, int64_t max_k, double scale, bool causal, int64_t row_pad_to) {
+                     int64_t max_q, int64_t max_k, double scale, bool causal) {
     check_stage1(q, k_, v_, cu_q, cu_k, cu_v);
     DeviceGuard guard(q.device());
     const int64_t batch = cu_q.numel() - 1, total_q = q.size(0), hq = q.size(1), hk = k_.size(1);
     const Tensor k = readable(k_), v = readable(v_);
-    const int64_t row = (max_k + row_pad_to - 1) / row_pad_to * row_pad_to;
-    Tensor out = at::empty({hk, total_q, row}, q.options());
+    Tensor out = at::empty({hk, total_q, max_k}, q.options());
     if (max_q == 1 && total_q > 0) {
         // decode: one query per sequence, so the parallelism has to come from the keys
         stage1_decode(q, batch, k, v, iptr(cu_q), iptr(cu_k), nullptr, iptr(cu_v), nullptr, max_k, max_rows_bound(v, batch, max_k), scale,
@@ -219,7 +218,7 @@ Tensor stage1_scores(const Tensor& q, const Tensor& k_, const Tensor& v_, const 
                     as_int(hk), as_int(q.size(2)), as_int(max_q), as_int(max_k), qs.v, ks.v, vs.v, out.stride(0), out.stride(1),
                     static_cast<float>(scale), causal ? 1 : 0), "varlen_fwd_stage1");
     }
-    return row == max_k ? out : out.narrow(2, 0, max_k);
+    return out;
 }
 
 // Scores pooled onto key blocks in the same launch: (Hk, total_q, out_len)
@@ -661,16 +660,19 @@ std::tuple<Tensor, Tensor> decode_sparse(const Tensor& q, const Tensor& kn, cons
                                          double scale) {
     TORCH_CHECK(topk > 0, "decode_sparse: topk must be positive");
     require_gpu(q, "q");
+    TORCH_CHECK(q.dim() == 4 && kc.dim() == 4, "q, k_cache, v_cache must have 4 dimensions");
     DeviceGuard guard(q.device());
+    const int64_t batch = q.size(0), hq = q.size(2), hk = kc.size(2);
+    const int splits = decode_splits(batch, hk, topk);
+    if (batch * hk * splits > 256 || max_len > INFLLMV2_DECODE_MAX_SCORES * kBlock) {
+        auto [new_lens, mask] = decode_step(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, max_len, kernel_size, stride,
+                                            block_size, topk, local_blocks, init_blocks, scale);
+        return {std::get<0>(fwd_kvcache(q, kc, vc, std::nullopt, std::nullopt, new_lens, scale, 0, std::nullopt, mask, std::nullopt, std::nullopt,
+                                        std::nullopt, std::nullopt, std::nullopt, false)), new_lens};
+    }
     auto [new_lens, pooled] = decode_front(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, max_len, kernel_size,
                                            stride, block_size, true, local_blocks, init_blocks, scale);
-    const int64_t batch = q.size(0), hq = q.size(2), hk = kc.size(2), n = pooled.size(2);
-    const int splits = decode_splits(batch, hk, topk);
-    if (batch * hk * splits > 256 || n > INFLLMV2_DECODE_MAX_SCORES) {
-        auto [idx, mask] = topk_blocks(pooled, topk, true, true, false, std::nullopt);
-        return {std::get<0>(fwd_kvcache(q, kc, vc, std::nullopt, std::nullopt, new_lens, scale, 0, std::nullopt, mask->unsqueeze(2), std::nullopt,
-                                        std::nullopt, std::nullopt, std::nullopt, std::nullopt, false)), new_lens};
-    }
+    const int64_t n = pooled.size(2);
     Tensor out = at::empty_like(q);
     const size_t partials = infllmv2_fwd_kvcache_workspace_bytes(as_int(batch), as_int(hk), splits), lse_bytes = sizeof(float) * batch * hq;
     Tensor ws = bytes_on(q, partials + lse_bytes);

@@ -315,3 +315,21 @@ def test_a_mask_of_more_words_than_lds_holds():
             s = q[b, 0].float() @ rows(kc).t().contiguous() * 128 ** -0.5
             want = torch.softmax(s, -1) @ rows(vc)
             assert (out[b, 0].float() - want).abs().max() <= 2e-2 and (lse[b, :, 0] - torch.logsumexp(s, -1)).abs().max() <= 2e-3
+
+
+@pytest.mark.parametrize("batch, cap, max_len", [(129, 256, 200), (2, 64 * 2049, 64 * 2048), (2, 64 * 2049, 64 * 2048 + 1)])
+def test_steps_on_both_sides_of_the_selecting_launch(batch, cap, max_len):
+    """More (sequence, KV head) pairs than CUs, and rows of 2048 and of 2049 block scores: a top-k launch and a mask where the attention's
+    launch does not select, through the layer."""
+    import infllmv2_cuda_impl_amd as ops
+    g = torch.Generator(device="cuda").manual_seed(batch)
+    Hk, layer = 2, ops.InfLLMv2Attention(topk=3, local_blocks=1)
+    mk = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)
+    lens = [max_len - 1 - 7 * (b % 9) for b in range(batch)]
+    cache = ops.BatchCache.empty(batch, cap, Hk, 128, "cuda")
+    layer.fill_cache(cache, mk(sum(lens), Hk, 128), mk(sum(lens), Hk, 128), lens)
+    held, q, kn, vn = cache.lengths.clone(), mk(batch, 1, 32, 128), mk(batch, 1, Hk, 128), mk(batch, 1, Hk, 128)
+    out = layer.decode_batch(q, kn, vn, cache)
+    pooled = ops.infllmv2_attn_stage1_kvcache(q, cache.k_fine, cache.k_coarse, cache.fine_lens, cache.coarse_lens, held, 1, 1, max_cache_len=max_len - 1)
+    want = ops.infllmv2_attn_with_kvcache(q, cache.k, cache.v, cache_seqlens=held + 1, topk_idx=ops.topk_blocks(pooled, 3).unsqueeze(2))
+    assert torch.equal(cache.lengths, held + 1) and (out.float() - want.float()).abs().max() <= 8e-3
