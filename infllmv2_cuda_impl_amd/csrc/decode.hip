@@ -997,12 +997,12 @@ extern "C" int IV2_ENTRY(infllmv2_fwd_kvcache_scores)(void* stream, const void* 
 #ifndef IV2_F16        // one such entry point in the library: bfloat16 only
 // ---- decode for callers that cannot allocate ---------------------------------------------------------------------
 //
-// The split partials and the turned query live in a device array that belongs to the library's code object: every GPU
+// The split partials live in a device array that belongs to the library's code object: every GPU
 // the library runs on holds one copy of it, at its own address, from module load to process end.  `scratch` below is
 // only the host-side handle of that array; the device address is looked up once per device with
 // hipGetSymbolAddress and is what the kernels get.  Nothing in the array has to start at zero: every (sequence, KV
-// head, split) workgroup writes its whole partial slot before the combine kernel reads it, and the turned query is
-// written before it is read.  All calls on one GPU share the array, so calls that overlap on one GPU (two streams, two
+// head, split) workgroup writes its log-sum-exp record, and its partial unless it has no block, which the record then says, before
+// the combine kernel reads them.  All calls on one GPU share the array, so calls that overlap on one GPU (two streams, two
 // threads) race; calls on one stream are ordered by the stream.
 static __device__ __align__(256) unsigned char scratch[INFLLMV2_STATIC_SCRATCH_BYTES];
 

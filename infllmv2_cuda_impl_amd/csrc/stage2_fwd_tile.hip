@@ -9,8 +9,8 @@
 // exponentials), which share the issue port: neither may wait for the other.  So the walk is one block ahead with its scores, and the order
 // inside a block is written out: one MFMA of the next block's S, two exponentials of this block's, the LDS reads of the operands that come
 // next.  Left to the compiler, which forms clumps of MFMAs and of exponentials, the same work takes 2310 us for 16384 tokens of 2 KV heads
-// instead of 1980 (there the matrix pipe was busy 48 % of the time, LDS reads free of conflicts).
-// Operator with 2 KV heads, us, hybrid walk -> this one: 2000 tokens 72 -> 68, 4096 219 -> 160, 16384 2430 -> 1980 (1.11 PFLOP/s), 50000
+// instead of 1980.  Counters at 2500 + 6001 + 4096 tokens: matrix pipe busy 48 % of the kernel, vector pipe 37 %, LDS reads free of conflicts.
+// Operator with 2 KV heads, us, hybrid walk -> this one: 2000 tokens 62 -> 61, 3800 156 -> 125, 16384 2430 -> 1980 (1.11 PFLOP/s), 50000
 // 20370 -> 17100 (1.2 PFLOP/s), 2500 + 6001 + 4096 566 -> 472, 777 + 5003 + 1291 + 9173 1160 -> 950.
 //
 // Operands.  S^T = K Q^T: lane (n = lane % 32, h = lane / 32) holds key n of a 32-key chunk, d = 16 ks + 8 h + j: one 16-byte unit of
