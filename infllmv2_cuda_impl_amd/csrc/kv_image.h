@@ -27,6 +27,11 @@ __host__ __device__ inline int64_t image_slots(int64_t total_k, int batch) {
     return total_k / kBlockN + batch + 1;
 }
 
+// bytes of both images of every block
+inline size_t image_bytes(int64_t total_k, int batch, int num_heads_k) {
+    return static_cast<size_t>(image_slots(total_k, batch)) * num_heads_k * kImageElems * sizeof(elem_bits) * 2;
+}
+
 __device__ __forceinline__ int64_t image_slot0(const int* cu_seqlens_k, int b) {
     return cu_seqlens_k[b] / kBlockN + b;
 }

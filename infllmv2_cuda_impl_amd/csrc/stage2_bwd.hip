@@ -97,7 +97,7 @@ struct BwdLayout {
 static BwdLayout bwd_layout(int batch, int64_t total_q, int64_t total_k, int num_heads_k, int max_seqlen_k) {
     BwdLayout L;
     size_t off = 0;
-    L.images = off; off += align256(infllmv2_kv_image_bytes(total_k, batch, num_heads_k));   // K image | V in K-image order
+    L.images = off; off += align256(image_bytes(total_k, batch, num_heads_k));   // K image | V in K-image order
     const int64_t k_blocks = (max_seqlen_k + kBlockN - 1) / kBlockN;
     L.mask = off; off += align256(static_cast<size_t>(num_heads_k) * k_blocks * ((total_q + 63) / 64) * 8);
     L.dsum = off; off += align256(static_cast<size_t>(num_heads_k) * total_q * 16 * 4);

@@ -24,9 +24,10 @@ struct FwdParams {
 };
 
 // Workgroup-hybrid forward (stage2_fwd_hybrid.hip): 8 consecutive tokens per workgroup stage the blocks they all
-// select once in LDS and walk the rest of their rows one wavefront each.
+// select once in LDS and walk the rest of their rows one wavefront each.  in_step: kInStepBytes of scratch that belong to this launch
+// alone (the counters by which workgroups walk long sequences in step), or null.
 int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q,
-                             int max_seqlen_k, bool causal);
+                             int max_seqlen_k, bool causal, void* in_step);
 
 // Forward without a mask (stage2_fwd_tile.hip): tiles of 256 query rows, 32 per wavefront.  A token takes 16 rows, 8 in groups of 8.
 inline int tile_row_shift(int group) { return group == 8 ? 3 : 4; }

@@ -17,6 +17,7 @@
 #include "kv_image.h"
 #include "block_walker.h"
 #include "stage2_fwd.h"
+#include "in_step.h"
 #include "infllmv2_hip.h"
 #include <math.h>
 
@@ -97,7 +98,7 @@ using namespace IV2_NS;
 
 #ifndef IV2_F16        // both element types are 2 bytes wide: defined once
 extern "C" size_t infllmv2_kv_image_bytes(int64_t total_k, int batch, int num_heads_k) {
-    return static_cast<size_t>(image_slots(total_k, batch)) * num_heads_k * kImageElems * sizeof(elem_bits) * 2;
+    return image_bytes(total_k, batch, num_heads_k) + kInStepBytes;           // behind the images: counters of the launch that walks them
 }
 #endif
 
@@ -108,7 +109,7 @@ int launch_pack(hipStream_t st, const void* k, const void* v, const int32_t* cu_
     IV2_CHECK(k && v && cu_seqlens_k && workspace, "pack_kv: null pointer");
     IV2_CHECK(batch > 0 && num_heads_k > 0 && total_k >= 0 && max_seqlen_k >= 0, "pack_kv: bad sizes");
     IV2_CHECK(num_heads_k <= 65535 && batch <= 65535, "pack_kv: batch and num_heads_k must not exceed 65535");
-    IV2_CHECK(workspace_bytes >= infllmv2_kv_image_bytes(total_k, batch, num_heads_k), "pack_kv: workspace too small");
+    IV2_CHECK(workspace_bytes >= image_bytes(total_k, batch, num_heads_k), "pack_kv: workspace too small");
     IV2_CHECK(reinterpret_cast<uintptr_t>(k) % 16 == 0 && reinterpret_cast<uintptr_t>(v) % 16 == 0 &&
               reinterpret_cast<uintptr_t>(workspace) % 16 == 0, "pack_kv: k, v and workspace must be 16-byte aligned");
     IV2_CHECK(k_strides[0] % 8 == 0 && k_strides[1] % 8 == 0 && v_strides[0] % 8 == 0 && v_strides[1] % 8 == 0,
@@ -157,7 +158,7 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_fwd)(void* stream, const void* q, const
     IV2_CHECK(batch > 0 && total_q >= 0 && total_k >= 0 && max_seqlen_q >= 0 && max_seqlen_k >= 0, "varlen_fwd: bad sizes");
     IV2_CHECK(q && out && softmax_lse && cu_seqlens_q && cu_seqlens_k && workspace, "varlen_fwd: null pointer");
     IV2_CHECK(num_heads_k <= 65535 && batch <= 65535, "varlen_fwd: batch and num_heads_k must not exceed 65535");
-    IV2_CHECK(workspace_bytes >= infllmv2_kv_image_bytes(total_k, batch, num_heads_k), "varlen_fwd: workspace too small");
+    IV2_CHECK(workspace_bytes >= image_bytes(total_k, batch, num_heads_k), "varlen_fwd: workspace too small");
     IV2_CHECK(reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 8 == 0 &&
               reinterpret_cast<uintptr_t>(workspace) % 16 == 0, "varlen_fwd: q and workspace must be 16-byte aligned, out 8-byte");
     for (int s = 0; s < 3; ++s) {
@@ -189,5 +190,8 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_fwd)(void* stream, const void* q, const
     fp.group = num_heads / num_heads_k;
     fp.n64 = n_uint64_per_row;
     fp.scale_log2 = softmax_scale * 1.44269504088896340736f;
-    return launch_stage2_fwd_hybrid(st, fp, batch, num_heads_k, max_seqlen_q, max_seqlen_k, is_causal != 0);
+    // Images packed by an earlier call may be read by several launches at once: those leave the workspace as it is.
+    const size_t images = image_bytes(total_k, batch, num_heads_k);
+    void* in_step = kv_prepacked || workspace_bytes < images + kInStepBytes ? nullptr : static_cast<unsigned char*>(workspace) + images;
+    return launch_stage2_fwd_hybrid(st, fp, batch, num_heads_k, max_seqlen_q, max_seqlen_k, is_causal != 0, in_step);
 }

@@ -22,10 +22,12 @@
 // Workgroups are numbered so that each of the 8 XCDs takes whole chunks of consecutive token
 // groups of one KV head (their L2 sees one head's images and neighbouring local windows), and
 // the longest causal prefixes are scheduled first.
+// Long sequences are walked in step with the other workgroups of the XCD (in_step.h).
 #include "common.h"
 #include "kv_image.h"
 #include "block_walker.h"
 #include "lds_dma.h"
+#include "in_step.h"
 #include "stage2_fwd.h"
 #include <math.h>
 
@@ -42,6 +44,7 @@ struct HybridExtra {
     int batch;
     int total_groups;                                          // num_heads_k * batch * groups_per_seq
     int mask_words;                                            // words per LDS mask row: what max_seqlen_k needs, not the maximum
+    unsigned* finished;                                        // the XCDs' counters of in_step.h, or null: no workgroup waits
 };
 
 __device__ __forceinline__ uint64_t uniform_u64(uint64_t v) {
@@ -137,7 +140,11 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     const int q0 = p.cu_seqlens_q[b];
     const int Sq = p.cu_seqlens_q[b + 1] - q0;
     const int i0 = grp * kHybTokens;
-    if (i0 >= Sq) return;                                                           // uniform per workgroup
+    unsigned* finished = x.finished ? x.finished + xcd * kInStepPitch : nullptr;
+    if (i0 >= Sq) {                                                                 // uniform per workgroup
+        if (finished && tid == 0) in_step_finished(finished, kHybTokens);
+        return;
+    }
     const int Sk = p.cu_seqlens_k[b + 1] - p.cu_seqlens_k[b];
 
     // A group at the end of a sequence that has four tokens or fewer: 2, 4 or 8 wavefronts share a token's blocks (every so-manyth column
@@ -184,7 +191,11 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     __syncthreads();
     const uint64_t columns = (share_log2 == 0 ? ~0ull : share_log2 == 1 ? 0x5555555555555555ull
                               : share_log2 == 2 ? 0x1111111111111111ull : 0x0101010101010101ull) << part;
-    for (int w = lane; w < nw; w += 64) own[w] &= ~com[w] & columns;
+    int own_words = 0;                                                              // lanes: words with blocks of this row's own
+    for (int w = lane; w < nw; w += 64) {
+        own[w] &= ~com[w] & columns;
+        own_words += __builtin_popcountll(__builtin_amdgcn_ballot_w64(own[w] != 0ull));
+    }
 
     // ---- Q operand ----
     elem8 qf[4];
@@ -236,6 +247,10 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
         const elem_bits* src = kimg + static_cast<int64_t>(jp) * kImageElems;
 #pragma unroll
         for (int f = 0; f < 16; ++f) kreg[f] = *reinterpret_cast<const elem8*>(src + f * 512);
+    }
+    if (finished) {
+        if (tid == 0 && Sk > kInStepKeys && own_words >= kInStepWords) in_step_wait(finished, sidx, kHybTokens);   // lane 0 took part in every round of the count
+        __syncthreads();
     }
     // All ordinary loads so far (Q, mask words, first K fragments) land before the first LDS-DMA.  From here on the
     // compiler's wait counts know nothing of the DMA loads; they stay correct because loads complete in order (an
@@ -338,6 +353,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
             half ^= 1;
         }
     }
+    if (finished && lane == 0) in_step_finished(finished, 1u);
     if (share_log2 != 0) {                                     // uniform per workgroup
         // the ring was not used: 34 floats of every lane, lane by lane
         float* mine = reinterpret_cast<float*>(smem_raw) + wave * (34 * 64) + lane;
@@ -383,7 +399,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
 }
 
 int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q,
-                             int max_seqlen_k, bool causal) {
+                             int max_seqlen_k, bool causal, void* in_step) {
     HybridExtra x{};
     x.batch = batch;
     x.groups_per_seq = (max_seqlen_q + kHybTokens - 1) / kHybTokens;
@@ -400,6 +416,11 @@ int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int 
     const size_t lds = kRingTiles * kTileBytes + static_cast<size_t>(1 + kHybTokens) * x.mask_words * 8;
     const void* fn = causal ? reinterpret_cast<const void*>(&stage2_fwd_hybrid_kernel<true>)
                             : reinterpret_cast<const void*>(&stage2_fwd_hybrid_kernel<false>);
+    if (in_step != nullptr && p.mask != nullptr && max_seqlen_k > kInStepKeys) {
+        x.finished = static_cast<unsigned*>(in_step);
+        hipLaunchKernelGGL(in_step_clear_kernel, dim3(1), dim3(8 * kInStepPitch), 0, st, x.finished);
+        IV2_LAUNCH_CHECK();
+    }
     hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     IV2_CHECK(e == hipSuccess, "varlen_fwd: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
     if (causal) hipLaunchKernelGGL(stage2_fwd_hybrid_kernel<true>, dim3(static_cast<unsigned>(grid)), dim3(512), lds, st, p, x);
