@@ -86,6 +86,7 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
     constexpr int kSliceWords = kColSlice / 64;                // mask words per slice (a power of two)
     constexpr int kGroupSlices = kGroupWords / kSliceWords;    // slices that pool their light members
     constexpr int kHeavyPairs = kColSlice / 4;                 // a slice with fewer selected tokens is "light"
+    constexpr int kItemTokens = kColSlice;                     // light slices are merged up to about so many selected tokens
     extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));   // which half of the block's keys
@@ -105,14 +106,15 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
     // sequence's own first group) the groups of a batch of sequences spread evenly over the XCDs.  Within a slice
     // the shared first block comes first, then the diagonal block and outwards, so the long items are dispatched early.
     // Where the groups do not divide evenly among the XCDs, 2, 4 or all 8 of them share a group (p.dkdv_share; a group then
-    // goes through as many L2s): sharer `part` takes the blocks rel with rel % share == part.
+    // goes through as many L2s): sharer `part` takes the blocks rel with rel % share == part, with short slices one part
+    // further in every slice, so that the blocks every token selects (the first, the last few) do not stay with the same sharers.
     const int xcd = blockIdx.x & 7, turn = blockIdx.x >> 3;
     if (Sq <= 0) return;                                       // uniform
     const int last_slice = (q0 + Sq - 1) / kColSlice;
     const int share = p.dkdv_share, teams = 8 / share;         // powers of two
     const int blocks_each = (p.k_blocks + share - 1) / share;
-    const int rel = (turn % blocks_each) * share + (xcd & (share - 1));
     const int round = turn / blocks_each;                      // a team works through one group of slices in consecutive rounds
+    const int rel = (turn % blocks_each) * share + ((xcd + (kColSlice < kDkdvSlice ? round : 0)) & (share - 1));
     const int top_group = last_slice / kGroupSlices;
     const int grp_idx = top_group - ((top_group - xcd / share) & (teams - 1)) - teams * (round / kGroupSlices);
     const int slice = grp_idx < 0 ? -1 : grp_idx * kGroupSlices + (kGroupSlices - 1 - round % kGroupSlices);
@@ -138,9 +140,11 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
     if (t_lo >= t_hi) return;                                  // uniform
 
     // ---- light slices are merged ----
-    // A flush costs 32768 fp32 atomics whatever the slice held, so a slice works on its own only if at least
-    // kHeavyPairs of its tokens selected the block; the other slices of the same group hand their tokens
-    // to the first non-empty one among them.  Every workgroup of the group takes the same decision from the
+    // A flush costs 16384 fp32 atomics whatever the slice held, so a slice works on its own only if at least
+    // kHeavyPairs of its tokens selected the block; the other slices of the same group are put together, about
+    // kItemTokens tokens to an item, and the first slice of an item collects.  (All of a group in one item: up to 465 tokens
+    // where a short slice holds 128, and the longest items decided the kernel's time; whole training pass of 12000 tokens, 16
+    // blocks selected: 1535 against 1435 us.)  Every workgroup of the group takes the same decision from the
     // group's 32 mask words (lane l < 32 holds word l; a slice is kSliceWords consecutive lanes).
     unsigned long long* wbuf = reinterpret_cast<unsigned long long*>(ring + kWaveLds);      // [kGroupWords]
     const int group = slice / kGroupSlices, sub = slice % kGroupSlices;
@@ -166,9 +170,22 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
         if ((heavy >> (kSliceWords * sub)) & 1ull) {
             keep = (lane / kSliceWords) == sub;
         } else {
-            const uint64_t light = filled & ~heavy;
-            if (light == 0ull || (__builtin_ctzll(light) / kSliceWords) != sub) return;   // uniform: empty, or another slice collects
-            keep = !((heavy >> lane) & 1ull);
+            uint64_t mates = filled & ~heavy;
+            if (!((mates >> (kSliceWords * sub)) & 1ull)) return;                   // uniform: empty
+            if constexpr ((kGroupSlices - 1) * (kHeavyPairs - 1) > kItemTokens) {
+                // dealt out by how many tokens the light slices before them hold
+                const int own = (mates >> lane) & 1ull ? cnt : 0;                   // every lane of a slice holds the slice's count
+                int upto = own;
+#pragma unroll
+                for (int off = kSliceWords; off < kGroupWords; off <<= 1) {
+                    const int up = __shfl_up(upto, off);
+                    upto += lane >= off ? up : 0;
+                }
+                const int item = (upto - own) / kItemTokens;
+                mates &= __ballot(lane < kGroupWords && item == __builtin_amdgcn_readlane(item, kSliceWords * sub));
+            }
+            if (__builtin_ctzll(mates) / kSliceWords != sub) return;                // uniform: another slice collects
+            keep = (mates >> lane) & 1ull;
         }
         if (lane < kGroupWords) wbuf[lane] = keep ? wv : 0ull;
     }
@@ -538,6 +555,13 @@ static int launch_bwd_dkdv_sliced(hipStream_t st, const BwdParams& p_in, int bat
         const int teams = 8 >> i;
         const float busy = static_cast<float>(all_groups) / ((all_groups + teams - 1) / teams * teams) / cost[i];
         if (busy > best) { best = busy; p.dkdv_share = 1 << i; }
+    }
+    if (kColSlice < kDkdvSlice && (all_groups < 12 || max_seqlen_q > 4096)) {
+        // Short slices: where the groups are few or differ (the first tokens of a sequence select less), sharing pays beyond even
+        // division.  Whole training pass in us with 1 / 2 / 4 / 8 sharers: 6000 tokens (3 groups) 2610 / 1810 / 1560 / 1500, 8000 (4)
+        // 2330 / 2330 / 2190 / 2160, the same with 16 blocks selected - / 980 / 1025 / 1130, 12000 + 9000 (11) 7360 / 6490 / 5960 /
+        // 6000, 3 x 12000 (18) 2180 / 2100 / 2045 / 2390; but 10 x 3000 (15) 2790 / 2790 / 2940 / 2950.
+        p.dkdv_share = all_groups <= 3 ? 8 : 4;
     }
     const int teams = 8 / p.dkdv_share;
     const int64_t rounds = static_cast<int64_t>((groups + teams - 1) / teams) * kGroupSlices;
