@@ -255,6 +255,10 @@ size_t infllmv2_kv_image_bytes(int64_t total_k, int batch, int num_heads_k);
 int infllmv2_varlen_fwd_dense_tiles(int batch, int64_t total_q, int64_t total_k, int num_heads, int num_heads_k,
                                     int max_seqlen_q, int max_seqlen_k, int is_causal);
 
+/* The same for infllmv2_varlen_fwd_selected with a blockmask. */
+int infllmv2_varlen_fwd_masked_tiles(int batch, int64_t total_q, int64_t total_k, int num_heads, int num_heads_k,
+                                     int max_seqlen_q, int max_seqlen_k, int is_causal, int most_selected);
+
 /* csrc/entry.cu:14,210 `varlen_fwd` = mha_varlen_fwd (csrc/flash_attn/flash_api.cpp:519-782) on
  * the sparse path (blockmask given) and on the dense path (blockmask null).
  * bf16, head_dim 128, num_heads == g * num_heads_k with g = 16 (the reference build) or 1, 2, 4, 8; the same holds
@@ -274,6 +278,17 @@ int infllmv2_varlen_fwd(void* stream, const void* q, const void* k, const void* 
                         const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
                         const int64_t* o_strides, const int64_t* lse_strides, int n_uint64_per_row,
                         float softmax_scale, int is_causal);
+
+/* infllmv2_varlen_fwd for a caller that knows how many blocks a row of the mask has set at most (0: not known).  The number decides
+ * which of two walks is the faster; results do not depend on its being right, except for rounding. */
+int infllmv2_varlen_fwd_selected(void* stream, const void* q, const void* k, const void* v, void* out,
+                                 float* softmax_lse, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                                 const uint64_t* blockmask, void* workspace, size_t workspace_bytes,
+                                 int kv_prepacked, int batch, int64_t total_q, int64_t total_k, int num_heads,
+                                 int num_heads_k, int head_dim, int max_seqlen_q, int max_seqlen_k,
+                                 const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+                                 const int64_t* o_strides, const int64_t* lse_strides, int n_uint64_per_row,
+                                 float softmax_scale, int is_causal, int most_selected);
 
 /* First half of infllmv2_varlen_fwd on its own: rewrites k, v (total_k, Hk, 128; strides {row, head})
  * into the block images in `workspace`.  A later infllmv2_varlen_fwd / _bwd call on the same k, v
@@ -468,6 +483,13 @@ int infllmv2_varlen_fwd_f16(void* stream, const void* q, const void* k, const vo
                             const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
                             const int64_t* o_strides, const int64_t* lse_strides, int n_uint64_per_row,
                             float softmax_scale, int is_causal);
+int infllmv2_varlen_fwd_selected_f16(void* stream, const void* q, const void* k, const void* v, void* out,
+                            float* softmax_lse, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                            const uint64_t* blockmask, void* workspace, size_t workspace_bytes, int kv_prepacked,
+                            int batch, int64_t total_q, int64_t total_k, int num_heads, int num_heads_k, int head_dim,
+                            int max_seqlen_q, int max_seqlen_k, const int64_t* q_strides, const int64_t* k_strides,
+                            const int64_t* v_strides, const int64_t* o_strides, const int64_t* lse_strides,
+                            int n_uint64_per_row, float softmax_scale, int is_causal, int most_selected);
 int infllmv2_varlen_bwd_f16(void* stream, const void* dout, const void* q, const void* k, const void* v,
                             const void* out, const float* softmax_lse, void* dq, void* dk, void* dv,
                             const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,

@@ -420,11 +420,13 @@ std::tuple<Tensor, Tensor, OptTensor> varlen_fwd(const Tensor& q, const Tensor& 
     Tensor ws = bytes_on(q, infllmv2_kv_image_bytes(total_k, as_int(batch), as_int(hk)));
     const S3 qs = grouped(q, group), os = grouped(out, group);
     const S2 ks = rows_heads(k), vs = rows_heads(v);
-    auto fn = is_half(q) ? infllmv2_varlen_fwd_f16 : infllmv2_varlen_fwd;
+    auto fn = is_half(q) ? infllmv2_varlen_fwd_selected_f16 : infllmv2_varlen_fwd_selected;
+    // a mask that came with its indices has at most so many blocks to a row
+    const int most_selected = sparse && topk_idx.has_value() && topk_idx->dim() > 0 ? as_int(topk_idx->size(-1)) : 0;
     check_rc(fn(stream_of(q), ptr(q), ptr(k), ptr(v), ptr(out), static_cast<float*>(ptr(lse)), iptr(cu_q), iptr(cu_k),
                 sparse ? static_cast<const uint64_t*>(mask->data_ptr()) : nullptr, ptr(ws), static_cast<size_t>(ws.numel()), 0, as_int(batch),
                 total_q, total_k, as_int(hq), as_int(hk), as_int(d), as_int(max_q), as_int(max_k), qs.v, ks.v, vs.v, os.v, lse_strides,
-                sparse ? as_int(mask->size(-1)) : 0, static_cast<float>(scale), causal ? 1 : 0), "varlen_fwd");
+                sparse ? as_int(mask->size(-1)) : 0, static_cast<float>(scale), causal ? 1 : 0, most_selected), "varlen_fwd");
     return {out, lse, mask};
 }
 

@@ -25,17 +25,20 @@ struct FwdParams {
 
 // Workgroup-hybrid forward (stage2_fwd_hybrid.hip): 8 consecutive tokens per workgroup stage the blocks they all
 // select once in LDS and walk the rest of their rows one wavefront each.  in_step: kInStepBytes of scratch that belong to this launch
-// alone (the counters by which workgroups walk long sequences in step), or null.
+// alone (the counters by which workgroups walk long sequences in step), or null.  most_selected: as in infllmv2_varlen_fwd_selected.  Goes by
+// tiles where that is the faster walk.
 int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q,
-                             int max_seqlen_k, bool causal, void* in_step);
+                             int max_seqlen_k, bool causal, int most_selected, void* in_step);
 
-// Forward without a mask (stage2_fwd_tile.hip): tiles of 256 query rows, 32 per wavefront.  A token takes 16 rows, 8 in groups of 8.
+// Forward by tiles of 256 query rows (stage2_fwd_tile.hip), 64 per wavefront.  A token takes 16 rows, 8 in groups of 8.
 inline int tile_row_shift(int group) { return group == 8 ? 3 : 4; }
 inline int tiles_per_sequence(int group, int max_seqlen_q) {
     const int tokens = 256 >> tile_row_shift(group);
     return (max_seqlen_q + tokens - 1) / tokens;
 }
 bool dense_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal);
+bool masked_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal,
+                      int most_selected);
 int launch_stage2_fwd_tile(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q,
                            int max_seqlen_k, bool causal);
 

@@ -144,14 +144,14 @@ extern "C" int infllmv2_pack_kv(void* stream, const void* k, const void* v, cons
 }
 #endif
 
-extern "C" int IV2_ENTRY(infllmv2_varlen_fwd)(void* stream, const void* q, const void* k, const void* v, void* out,
+extern "C" int IV2_ENTRY(infllmv2_varlen_fwd_selected)(void* stream, const void* q, const void* k, const void* v, void* out,
                                    float* softmax_lse, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
                                    const uint64_t* blockmask, void* workspace, size_t workspace_bytes,
                                    int kv_prepacked, int batch, int64_t total_q, int64_t total_k, int num_heads,
                                    int num_heads_k, int head_dim, int max_seqlen_q, int max_seqlen_k,
                                    const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
                                    const int64_t* o_strides, const int64_t* lse_strides,
-                                   int n_uint64_per_row, float softmax_scale, int is_causal) {
+                                   int n_uint64_per_row, float softmax_scale, int is_causal, int most_selected) {
     IV2_CHECK(head_dim == kHeadDim, "varlen_fwd: this build only supports head_dim 128 (got %d)", head_dim);
     IV2_CHECK(valid_group(num_heads, num_heads_k),
               "varlen_fwd: requires num_heads == g * num_heads_k with g in {1, 2, 4, 8, 16} (got %d and %d)", num_heads, num_heads_k);
@@ -193,5 +193,19 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_fwd)(void* stream, const void* q, const
     // Images packed by an earlier call may be read by several launches at once: those leave the workspace as it is.
     const size_t images = image_bytes(total_k, batch, num_heads_k);
     void* in_step = kv_prepacked || workspace_bytes < images + kInStepBytes ? nullptr : static_cast<unsigned char*>(workspace) + images;
-    return launch_stage2_fwd_hybrid(st, fp, batch, num_heads_k, max_seqlen_q, max_seqlen_k, is_causal != 0, in_step);
+    return launch_stage2_fwd_hybrid(st, fp, batch, num_heads_k, max_seqlen_q, max_seqlen_k, is_causal != 0, most_selected, in_step);
+}
+
+extern "C" int IV2_ENTRY(infllmv2_varlen_fwd)(void* stream, const void* q, const void* k, const void* v, void* out,
+                                   float* softmax_lse, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                                   const uint64_t* blockmask, void* workspace, size_t workspace_bytes,
+                                   int kv_prepacked, int batch, int64_t total_q, int64_t total_k, int num_heads,
+                                   int num_heads_k, int head_dim, int max_seqlen_q, int max_seqlen_k,
+                                   const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+                                   const int64_t* o_strides, const int64_t* lse_strides,
+                                   int n_uint64_per_row, float softmax_scale, int is_causal) {
+    return IV2_ENTRY(infllmv2_varlen_fwd_selected)(stream, q, k, v, out, softmax_lse, cu_seqlens_q, cu_seqlens_k, blockmask, workspace,
+                                                   workspace_bytes, kv_prepacked, batch, total_q, total_k, num_heads, num_heads_k, head_dim,
+                                                   max_seqlen_q, max_seqlen_k, q_strides, k_strides, v_strides, o_strides, lse_strides,
+                                                   n_uint64_per_row, softmax_scale, is_causal, 0);
 }

@@ -399,15 +399,17 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
 }
 
 int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q,
-                             int max_seqlen_k, bool causal, void* in_step) {
+                             int max_seqlen_k, bool causal, int most_selected, void* in_step) {
     HybridExtra x{};
     x.batch = batch;
     x.groups_per_seq = (max_seqlen_q + kHybTokens - 1) / kHybTokens;
     const int64_t total = static_cast<int64_t>(num_heads_k) * batch * x.groups_per_seq;
     IV2_CHECK(total <= 0x3fffffff, "varlen_fwd: too many token groups");
     IV2_CHECK((max_seqlen_k + kBlockN - 1) / kBlockN <= kMaxMaskWords * 64, "varlen_fwd: more than %d key blocks per sequence", kMaxMaskWords * 64);
-    if (p.mask == nullptr && dense_tiles_pay(batch, num_heads_k, p.group, p.total_q, p.total_k, max_seqlen_q, max_seqlen_k, causal))
-        return launch_stage2_fwd_tile(st, p, batch, num_heads_k, max_seqlen_q, max_seqlen_k, causal);
+    const bool tiles = p.mask == nullptr
+        ? dense_tiles_pay(batch, num_heads_k, p.group, p.total_q, p.total_k, max_seqlen_q, max_seqlen_k, causal)
+        : masked_tiles_pay(batch, num_heads_k, p.group, p.total_q, p.total_k, max_seqlen_q, max_seqlen_k, causal, most_selected);
+    if (tiles) return launch_stage2_fwd_tile(st, p, batch, num_heads_k, max_seqlen_q, max_seqlen_k, causal);
     x.total_groups = static_cast<int>(total);
     x.mask_words = ((max_seqlen_k + kBlockN - 1) / kBlockN + 63) / 64;
     if (x.mask_words < 1) x.mask_words = 1;

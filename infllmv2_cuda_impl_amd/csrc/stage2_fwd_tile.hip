@@ -1,17 +1,19 @@
-// Stage-2 forward without a mask (gfx950): dense attention over packed sequences as a flash tile of 256 query rows.
+// Stage-2 forward by flash tiles of 256 query rows (gfx950): without a mask, or with one whose rows select most of what they see.
 //
 // Where every token attends its whole prefix nothing is left to fetch per token, and the hybrid walk (stage2_fwd_hybrid.hip) only
-// keeps its costs: 16 query rows per K / V fragment read from LDS, softmax and MFMAs of a wavefront one after the other.  Here a workgroup of 8
-// wavefronts owns 256 rows (16 tokens of 16 heads, 32 of 8) and a wavefront 32 of them, the N side of v_mfma_f32_32x32x16: a fragment feeds
-// twice the rows in half the instructions.  K and V come from the same block images through the same 4-tile LDS ring.
+// keeps its costs: 16 query rows per K / V fragment read from LDS, softmax and MFMAs of a wavefront one after the other; where the rows differ a
+// little it fetches the rest per token, 32 KiB through the L1 path for 16 rows.  Here a workgroup of 4 wavefronts owns 256 rows (16 tokens of 16
+// heads, 32 of 8) and walks the blocks that any of its tokens selected; a row that did not select one has P = 0 there.  K and V come from
+// the same block images, through an LDS ring of three blocks.
 //
-// What bounds it: per block a SIMD's two wavefronts need 64 MFMAs of 32 clocks and about 250 vector instructions (64 of them
-// exponentials), which share the issue port: neither may wait for the other.  So the walk is one block ahead with its scores, and the order
-// inside a block is written out: one MFMA of the next block's S, two exponentials of this block's, the LDS reads of the operands that come
-// next.  Left to the compiler, which forms clumps of MFMAs and of exponentials, the same work takes 2310 us for 16384 tokens of 2 KV heads
-// instead of 1980.  Counters at 2500 + 6001 + 4096 tokens: matrix pipe busy 48 % of the kernel, vector pipe 37 %, LDS reads free of conflicts.
-// Operator with 2 KV heads, us, hybrid walk -> this one: 2000 tokens 62 -> 61, 3800 156 -> 125, 16384 2430 -> 1980 (1.11 PFLOP/s), 50000
-// 20370 -> 17100 (1.2 PFLOP/s), 2500 + 6001 + 4096 566 -> 472, 777 + 5003 + 1291 + 9173 1160 -> 950.
+// What bounds it: the power the matrix pipe draws.  16384 dense tokens of 2 KV heads take 1825 us (1.2 PFLOP/s) with random inputs and 1460 with zeros,
+// where only the clock differs; a library product of 8192^3 makes 1.38 and 1.79 PFLOP/s.  What a step does beside the MFMAs counts in energy more than in
+// issue slots, and the operand reads from LDS are the largest part: so a wavefront takes 64 rows, in two halves of 32 (the N side of
+// v_mfma_f32_32x32x16), and a fragment feeds both.  That is one wavefront per SIMD with 512 registers (128 of O, 64 each of Q, S, K and V, 32 of P),
+// and the overlap of MFMAs and exponentials is written out: while one half's P V and scores are on the matrix pipe, the other half's exponentials are
+// formed.  Before, eight wavefronts of 32 rows, two to a SIMD, read twice the LDS bytes: 1910 us; four wavefronts of 32 rows in
+// workgroups of two to a CU 1993; this shape with copies and scalar work at the head of a step instead of between its MFMAs 1979.
+// Operator, us, eight wavefronts -> this one: 2500 + 6001 + 4096 tokens 481 -> 455, 777 + 5003 + 1291 + 9173 865 -> 816, 50000 17000 -> 16600.
 //
 // Operands.  S^T = K Q^T: lane (n = lane % 32, h = lane / 32) holds key n of a 32-key chunk, d = 16 ks + 8 h + j: one 16-byte unit of
 // the K image.  The accumulators hold keys 8 i + 4 h + e (register 4 i + e) of row n; a V image unit holds keys 4 g + e and
@@ -27,10 +29,13 @@
 
 namespace IV2_NS {
 
-constexpr int kTileRows = 256;                                 // query rows of a workgroup, 32 per wavefront
-constexpr int kRingTiles = 4;
-constexpr int kTileBytes = 32768;                              // K image | V image of one block
+constexpr int kTileWaves = 4;
+constexpr int kTileRows = 64 * kTileWaves;                     // query rows of a workgroup, 64 per wavefront in two halves
+constexpr int kSlots = 3;                                      // of the ring: K image | V image of a block
+constexpr int kSlotBytes = 2 * kImageElems * 2;
 constexpr float kLazyLimit = 64.f;                             // as in the hybrid walk: a lane's sum of P that the reference exponent has to keep to
+constexpr float kNoReference = -3.4028234e38f;
+constexpr int kMostTokens = 8;                                 // of a wavefront: groups of 8
 
 struct TileExtra {
     int tiles_per_seq;                                         // ceil(max_seqlen_q / tokens of a tile)
@@ -60,11 +65,75 @@ __device__ __forceinline__ float half_sum(float x) {
     return a + b;
 }
 
+// The key blocks of a tile in ascending order: those that any of its tokens selected (all of them without a mask).  Everything here is
+// uniform over the wavefront; the blocks are the same in all wavefronts of a workgroup.
+constexpr int kTokenBits = 20;
+struct TileWalk {
+    const uint64_t* rows;           // mask row of the tile's first token, or null
+    int n64, tokens;                // words of a row; tokens of the tile that exist
+    int mine;                       // first token of this wavefront inside the tile
+    int per_wave;
+    int blocks;                     // blocks at or behind this one are not walked
+    int w;
+    uint64_t bits;                  // of word w: what is left of the union
+    int chosen;                     // lane b: which of this wavefront's tokens selected block b of word w, a bit each
+
+    __device__ __forceinline__ void load() {
+        const int left = blocks - w * 64, lane = __lane_id();
+        if (rows == nullptr) {
+            bits = ~0ull;
+            const int live = tokens - mine < per_wave ? tokens - mine : per_wave;
+            chosen = live > 0 ? (1 << live) - 1 : 0;
+        } else {
+            // lane t holds the word of the tile's token t
+            uint32_t lo = 0u, hi = 0u;
+            if (lane < tokens) {
+                const uint64_t row = rows[static_cast<int64_t>(lane) * n64 + w];
+                lo = static_cast<uint32_t>(row);
+                hi = static_cast<uint32_t>(row >> 32);
+            }
+            chosen = 0;
+#pragma unroll
+            for (int t = 0; t < kMostTokens; ++t) {
+                const int from = mine + t < 64 ? mine + t : 63;
+                const uint32_t a = __builtin_amdgcn_readlane(lo, from), b = __builtin_amdgcn_readlane(hi, from);
+                if (t < per_wave) chosen |= static_cast<int>(((lane < 32 ? a : b) >> (lane & 31)) & 1u) << t;
+            }
+#pragma unroll
+            for (int hop = 16; hop > 0; hop >>= 1) {           // a tile has at most 32 tokens
+                lo |= __shfl_xor(lo, hop);
+                hi |= __shfl_xor(hi, hop);
+            }
+            bits = static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(hi))) << 32 | static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(lo));
+        }
+        if (left < 64) bits &= (1ull << left) - 1ull;
+    }
+    __device__ __forceinline__ void init() {
+        if (rows != nullptr && blocks > n64 * 64) blocks = n64 * 64;
+        w = 0;
+        bits = 0ull;
+        chosen = 0;
+        if (blocks > 0) load();
+    }
+    // the next block and, from kTokenBits up, which of this wavefront's tokens selected it; or -1
+    __device__ __forceinline__ int next() {
+        while (bits == 0ull) {
+            if ((w + 1) * 64 >= blocks) return -1;
+            ++w;
+            load();
+        }
+        const int bit = __builtin_ctzll(bits);
+        bits &= bits - 1ull;
+        return w * 64 + bit | __builtin_amdgcn_readlane(chosen, bit) << kTokenBits;
+    }
+    __device__ __forceinline__ static int index(int block) { return block & ((1 << kTokenBits) - 1); }
+};
+
 template <bool kCausal>
-__global__ __launch_bounds__(512)
+__global__ __launch_bounds__(64 * kTileWaves) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void stage2_fwd_tile_kernel(const FwdParams p, const TileExtra x) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    uint4* ring = reinterpret_cast<uint4*>(smem_raw);                               // [kRingTiles][2048]: K units 0..1023, V units 1024..2047
+    const uint4* ring = reinterpret_cast<const uint4*>(smem_raw);                   // [kSlots][2048]: K units 0..1023, V units 1024..2047
 
     // ---- which tile: sequence by sequence, longest prefixes first, the KV heads of a tile next to each other (on the XCDs of a chip
     //      that shares work round robin: each keeps to one head where there are two, four or eight).  Tiles behind the end of a sequence
@@ -86,216 +155,333 @@ void stage2_fwd_tile_kernel(const FwdParams p, const TileExtra x) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
     const int n = lane & 31, h = lane >> 5;
-    const int per_wave = 32 >> x.row_shift;                                         // tokens of a wavefront
-    const int i_wave = i_first + wave * per_wave;
+    const int per_half = 32 >> x.row_shift;                                         // tokens of half a wavefront
+    const int i_wave = i_first + wave * 2 * per_half;
     auto last_of = [&](int t) {                                                     // last key token t attends
         const int lk = kCausal ? t + Sk - Sq : Sk - 1;
         return lk > Sk - 1 ? Sk - 1 : lk;
     };
-    const int wave_first_key = i_wave + per_wave <= Sq ? last_of(i_wave) : -1;      // of the wavefront's first token; -1: it has rows without a token
+    const int wave_first_key = last_of(i_wave);                                     // of the wavefront's first token
 
-    elem8 qf[8];
-    {
-        const int i = i_wave + (n >> x.row_shift), head = n & ((1 << x.row_shift) - 1);
+    elem8 qf[2][8];
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+        const int i = i_wave + hf * per_half + (n >> x.row_shift), head = n & ((1 << x.row_shift) - 1);
         const int64_t tok = static_cast<int64_t>(q0) + (i < Sq ? i : Sq - 1);
         const elem_bits* qp = p.q + tok * p.q_tok_stride + h_kv * p.q_kvh_stride + (head < p.group ? head : p.group - 1) * p.q_grp_stride + 8 * h;
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) qf[ks] = *reinterpret_cast<const elem8*>(qp + 16 * ks);
+        for (int ks = 0; ks < 8; ++ks) qf[hf][ks] = *reinterpret_cast<const elem8*>(qp + 16 * ks);
+    }
+
+    TileWalk walk;
+    {
+        const int left = Sq - i_first, all = kTileRows >> x.row_shift;
+        walk.tokens = left < all ? left : all;
+        const int lk = last_of(i_first + walk.tokens - 1);                          // of the tile's last token
+        walk.blocks = lk < 0 ? 0 : (lk >> 6) + 1;
+        if (walk.blocks > x.max_blocks) walk.blocks = x.max_blocks;                 // a sequence longer than the announced max_seqlen_k
+        walk.rows = p.mask ? p.mask + (static_cast<int64_t>(h_kv) * p.total_q + q0 + i_first) * p.n64 : nullptr;
+        walk.n64 = p.n64;
+        walk.mine = wave * 2 * per_half;
+        walk.per_wave = 2 * per_half;
+        walk.init();
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                // before the first LDS-DMA (see the hybrid walk)
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+v"(qf[ks]));
+    for (int ks = 0; ks < 8; ++ks) asm volatile("" : "+a"(qf[0][ks]), "+a"(qf[1][ks]));
 
     const int64_t slot0 = static_cast<int64_t>(h_kv) * p.n_slots + image_slot0(p.cu_seqlens_k, b);
-    const elem_bits* src = (wave < 4 ? p.kimg : p.vimg) + slot0 * kImageElems + (wave & 3) * 2048;   // this wavefront's quarter of K or V
-    const uint32_t ring_base = __builtin_amdgcn_readfirstlane(lds_address_of(ring) + wave * 4096);
-    auto issue = [&](int j, int tile) { dma_copy_4k(src + static_cast<int64_t>(j) * kImageElems, 16 * lane, ring_base + tile * kTileBytes); };
-    int blocks = 0;                                                                 // of the tile's last token
-    {
-        const int i_end = i_first + (kTileRows >> x.row_shift) - 1;
-        const int lk = last_of(i_end < Sq ? i_end : Sq - 1);
-        blocks = lk < 0 ? 0 : (lk >> 6) + 1;
-        if (blocks > x.max_blocks) blocks = x.max_blocks;                           // a sequence longer than the announced max_seqlen_k
-    }
+    const elem_bits* kimg = p.kimg + slot0 * kImageElems;
+    const elem_bits* vimg = p.vimg + slot0 * kImageElems;
+    const uint32_t ring_base = __builtin_amdgcn_readfirstlane(lds_address_of(ring) + wave * 4096);      // this wavefront copies a quarter of every image
+    auto issue_part = [&](int block, int slot, int part) {     // 1 KiB of 8
+        const elem_bits* src = (part < 4 ? kimg : vimg) + static_cast<int64_t>(TileWalk::index(block)) * kImageElems + wave * 2048 + (part & 3) * 512;
+        dma_copy_1k(src, 16 * lane, ring_base + slot * kSlotBytes + (part >> 2) * (kSlotBytes / 2) + (part & 3) * 1024);
+    };
+    auto issue = [&](int block, int slot) {
+#pragma unroll
+        for (int part = 0; part < 8; ++part) issue_part(block, slot, part);
+    };
 
     // m: reference exponent as in softmax_step, but finite from the start (a row whose keys are all hidden so far has P = 0 by itself)
-    float m = -3.4028234e38f, l = 0.f;
-    floatx16 o[4];
+    float m[2] = {kNoReference, kNoReference}, l[2] = {0.f, 0.f};
+    floatx16 o[2][4];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[hf][t][r] = 0.f;
 
-    // 16-byte units of this lane inside a tile: K unit (2 cc + n/16, ks/2, n%16 + 16 (2 (ks%2) + h)), V unit (2 t + n/16, cc, n%16 + 16 (2 jj + h))
+    // 16-byte units of this lane inside an image: K unit (2 cc + n/16, ks/2, n%16 + 16 (2 (ks%2) + h)), V unit (2 t + n/16, cc, n%16 + 16 (2 jj + h))
     const int k_unit = (n >> 4) * 256 + (n & 15) + 16 * h;
-    const int v_unit = 1024 + (n >> 4) * 128 + (n & 15) + 16 * h;
-    elem8 kf[16];                                              // K of the next block, kf[2 ks + cc]
-    auto load_k = [&](int tile, int half) {                    // half the depth at a time: 4 of 8 ks
-        const uint4* kb = ring + tile * 2048 + k_unit;
-#pragma unroll
-        for (int ks = 4 * half; ks < 4 * half + 4; ++ks)
-#pragma unroll
-            for (int cc = 0; cc < 2; ++cc) {
-                const uint4 raw = kb[cc * 512 + (ks >> 1) * 64 + (ks & 1) * 32];
-                __builtin_memcpy(&kf[2 * ks + cc], &raw, 16);
-            }
+    const int v_unit = (n >> 4) * 128 + (n & 15) + 16 * h;
+    auto k_at = [](int f) { return (f & 1) * 512 + (f >> 2) * 64 + ((f >> 1) & 1) * 32; };               // fragment f = 2 ks + cc
+    auto v_at = [](int f) { return (f & 3) * 256 + (f >> 3) * 64 + ((f >> 2) & 1) * 32; };               // fragment f = 8 cc + 4 jj + t
+    elem8 kf[16], vf[16];
+    auto read_k = [&](int slot, int f) {
+        const uint4 raw = ring[slot * 2048 + k_unit + k_at(f)];
+        __builtin_memcpy(&kf[f], &raw, 16);
     };
-    auto scores = [&](floatx16 (&s)[2]) {
-#pragma unroll
-        for (int cc = 0; cc < 2; ++cc)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s[cc][r] = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks)
-#pragma unroll
-            for (int cc = 0; cc < 2; ++cc) s[cc] = IV2_MFMA32(kf[2 * ks + cc], qf[ks], s[cc]);
+    auto read_v = [&](int slot, int f) {
+        const uint4 raw = ring[slot * 2048 + 1024 + v_unit + v_at(f)];
+        __builtin_memcpy(&vf[f], &raw, 16);
     };
-    auto hide = [&](floatx16 (&s)[2], int j) {                 // keys behind the row's last one
-        const int i = i_wave + (n >> x.row_shift);
-        const int lim = (i < Sq ? last_of(i) : -1) - j * kBlockN;
+    floatx16 s[2][2];
+    const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    auto hide = [&](int hf, int j) {                           // keys behind the row's last one
+        const int lim = last_of(i_wave + hf * per_half + (n >> x.row_shift)) - j * kBlockN;
 #pragma unroll
         for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
             for (int r = 0; r < 16; ++r)
-                if (32 * cc + 8 * (r >> 2) + 4 * h + (r & 3) > lim) s[cc][r] = -INFINITY;
+                if (32 * cc + 8 * (r >> 2) + 4 * h + (r & 3) > lim) s[hf][cc][r] = -INFINITY;
     };
-    elem8 pf[4];
-    auto exponentials = [&](floatx16 (&s)[2]) -> float {       // s becomes P; returns the lane's sum
-        float part[4] = {0.f, 0.f, 0.f, 0.f};
+    auto largest = [&](int hf) -> float {                      // of the row, log2 units
+        float mx = -INFINITY;
 #pragma unroll
         for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                s[cc][r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[cc][r], p.scale_log2, -m));
-                part[r & 3] += s[cc][r];
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[hf][cc][r]);
+        return half_max(mx) * p.scale_log2;
+    };
+    typedef __attribute__((__vector_size__(4 * sizeof(uint32_t)))) uint32_t words4;
+    typedef __attribute__((__vector_size__(2 * sizeof(elem_t)))) elem_t elem2;
+    auto two_elems = [](float lo, float hi) -> uint32_t {       // one conversion instruction
+        const elem2 v = {static_cast<elem_t>(lo), static_cast<elem_t>(hi)};
+        uint32_t w;
+        __builtin_memcpy(&w, &v, 4);
+        return w;
+    };
+    words4 pf[2][4];                                           // P, two elements to a word
+    auto operand = [](const words4& w) {
+        elem8 v;
+        __builtin_memcpy(&v, &w, 16);
+        return v;
+    };
+    auto exponentials = [&](int hf, float against) -> float {   // P of a block at once; returns the lane's sum
+        float sum = 0.f;
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+            for (int r = 0; r < 16; r += 2) {
+                const float lo = __builtin_amdgcn_exp2f(__builtin_fmaf(s[hf][cc][r], p.scale_log2, -against));
+                const float hi = __builtin_amdgcn_exp2f(__builtin_fmaf(s[hf][cc][r + 1], p.scale_log2, -against));
+                sum += lo;
+                sum += hi;
+                pf[hf][2 * cc + ((r >> 2) & 1)][(r >> 3) * 2 + ((r & 3) >> 1)] = two_elems(lo, hi);
+            }
+        return sum;
+    };
+    auto rescale = [&](int hf, float m_new) {
+        const float alpha = __builtin_amdgcn_exp2f(m[hf] - m_new);
+        l[hf] *= alpha;
+        m[hf] = m_new;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[hf][t] *= alpha;
+    };
+    // Half a step: 32 MFMAs for one half of the rows and, spread between them, the exponentials of a block for the other half, each in three
+    // places (multiply-add, exp2, sum), so that none waits for its predecessor.  They start a group late, when the last scores have left the matrix pipe, and are through
+    // before the last MFMA, so that the branch on their sum costs nothing.  `beside` adds LDS reads, copies and scalar work.  The order is fixed by
+    // hand: the compiler's own clumps both sides.
+    auto half_step = [&](auto&& mfma, auto&& beside, int hf, float against) -> float {
+        float e[32], sum = 0.f;
+        auto upto = [](int group) { return group < 1 ? 0 : (group - 1) * 9 / 8 < 32 ? (group - 1) * 9 / 8 : 32; };
+#pragma unroll
+        for (int g = 0; g < 32; ++g) {
+            mfma(g);
+            beside(g);
+#pragma unroll
+            for (int i = upto(g - 1); i < upto(g); ++i) {
+                sum += e[i];
+                asm volatile("" : "+v"(sum));                  // here, not all at the end
+                if (i & 1) {
+                    uint32_t two = two_elems(e[i - 1], e[i]);
+                    asm volatile("" : "+v"(two));
+                    const int r = i & 15;
+                    pf[hf][2 * (i >> 4) + ((r >> 2) & 1)][(r >> 3) * 2 + ((r & 3) >> 1)] = two;
+                }
             }
 #pragma unroll
-        for (int cc = 0; cc < 2; ++cc)
+            for (int i = upto(g); i < upto(g + 1); ++i) {
+                e[i] = __builtin_amdgcn_exp2f(e[i]);
+                asm volatile("" : "+v"(e[i]));
+            }
 #pragma unroll
-            for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    pf[2 * cc + jj][e] = static_cast<elem_t>(s[cc][4 * jj + e]);
-                    pf[2 * cc + jj][4 + e] = static_cast<elem_t>(s[cc][4 * (jj + 2) + e]);
-                }
-        return (part[0] + part[1]) + (part[2] + part[3]);
+            for (int i = upto(g + 1); i < upto(g + 2); ++i) {
+                e[i] = __builtin_fmaf(s[hf][i >> 4][i & 15], p.scale_log2, -against);
+                asm volatile("" : "+v"(e[i]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        return sum;
     };
+    auto form_s = [&](int hf) { return [&, hf](int f) { s[hf][f & 1] = IV2_MFMA32(kf[f], qf[hf][f >> 1], f < 2 ? zero : s[hf][f & 1]); }; };
+    auto form_o = [&](int hf) { return [&, hf](int f) { o[hf][f & 3] = IV2_MFMA32(vf[f], operand(pf[hf][f >> 2]), o[hf][f & 3]); }; };
+    const int token_bit = kTokenBits + (n >> x.row_shift);     // of this lane's token of the first half, in a block's bits
+    auto selects = [&](int hf, int block) -> bool { return (block >> (token_bit + hf * per_half)) & 1; };
+    auto against = [&](int hf, int block) -> float { return selects(hf, block) ? m[hf] : INFINITY; };     // rows that did not select the block: P = exp2(-inf)
+    auto settle = [&](int hf, int block, float sum) {           // the sum of a block's P, or the block once more
+        if (__ballot(!(sum <= kLazyLimit)) != 0ull) {          // a row without a reference yet, one that grew, or NaN
+            const float mx = largest(hf);
+            const bool selected = selects(hf, block);
+            rescale(hf, selected ? fmaxf(m[hf], mx) : m[hf]);
+            sum = exponentials(hf, selected ? m[hf] : INFINITY);
+        }
+        l[hf] += sum;
+    };
+    auto edge = [&](int block) { return TileWalk::index(block) * kBlockN + kBlockN - 1 > wave_first_key; };   // the last block or two
 
-    // One barrier per block.  Behind the one of block j the tiles of j, j + 1 and j + 2 are in LDS and the fourth is free: V of j and K of
-    // j + 1 and j + 2 are read from LDS, j + 3 is requested.  S of j + 1 is formed between the exponentials of j.
-    for (int j = 0; j < 3 && j < blocks; ++j) issue(j, j);
-    floatx16 sa[2], sb[2];
-    if (blocks > 0) {
+    // The walk: j0 is the current block, j1 the next; j1 and j2 are in the ring or on their way, j3 is requested.  The two halves of the rows take turns: while
+    // the matrix pipe works on one, the exponentials of the other are formed.  At the top of a step P of j0 is there for the first half, its scores
+    // for the second, and V of j0 is in registers.
+    int j0 = walk.next(), j1 = walk.next(), j2 = walk.next();
+    int at1 = 1;                                               // slot of j1
+    int every = ~0;                                            // bits of the tokens that selected all blocks so far
+    if (j0 >= 0) {
+        issue(j0, 0);
+        if (j1 >= 0) issue(j1, 1);
+        if (j2 >= 0) issue(j2, 2);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        load_k(0, 0);
-        load_k(0, 1);
-        scores(sa);
-        load_k(1, 0);                                          // whatever lies there where there is no second block: its scores are not used
+#pragma unroll
+        for (int f = 0; f < 16; ++f) read_k(0, f);
+#pragma unroll
+        for (int f = 0; f < 16; ++f) read_v(0, f);
+#pragma unroll
+        for (int f = 0; f < 16; ++f) form_s(0)(f);
+#pragma unroll
+        for (int f = 0; f < 16; ++f) form_s(1)(f);
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+            // rows that selected the first block take their reference from it
+            if (edge(j0)) hide(hf, TileWalk::index(j0));
+            const float mx = largest(hf);
+            if (selects(hf, j0) && mx > kNoReference && mx < INFINITY) m[hf] = mx;
+        }
+        settle(0, j0, exponentials(0, against(0, j0)));
     }
-    auto step = [&](int j, floatx16 (&sc)[2], floatx16 (&sn)[2]) {
-        const int slot = j & 3;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // this wavefront's part of tile j + 2
+    while (j1 >= 0) {                                          // uniform over the workgroup
+        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");       // this wavefront's part of j1; j2's may be on its way
         __syncthreads();
-        if (j + 3 < blocks) issue(j + 3, (j + 3) & 3);
-        const bool edge = j * kBlockN + kBlockN - 1 > wave_first_key;              // the last block or two
-        if (edge) hide(sc, j);
-        const uint4* vb = ring + slot * 2048 + v_unit;
-        elem8 vf[16];
-        // Region A: S of the next block, MFMA by MFMA, and beside each MFMA two of this block's exponentials and its share of LDS reads
-        // (the rest of K for the coming MFMAs, then V).  The order is fixed by hand: the compiler's own clumps both sides.
-        auto read_k = [&](int f) {
-            const uint4 raw = ring[((slot + 1) & 3) * 2048 + k_unit + (f & 1) * 512 + (f >> 2) * 64 + ((f >> 1) & 1) * 32];
-            __builtin_memcpy(&kf[f], &raw, 16);
-        };
-        auto read_v = [&](int f) {                             // f = 8 cc + 4 jj + t
-            const uint4 raw = vb[(f & 3) * 256 + (f >> 3) * 64 + ((f >> 2) & 1) * 32];
-            __builtin_memcpy(&vf[f], &raw, 16);
-        };
-        float part[2] = {0.f, 0.f};
+        const int slot = at1, freed = at1 == 0 ? 2 : at1 - 1;  // of j1, of j0
+        every &= j0;
+        const int j3 = j2 >= 0 ? walk.next() : -1;
+        settle(1, j0, half_step([&](int g) { if (g < 16) form_o(0)(g); else form_s(0)(g - 16); }, [&](int g) {
+            if (g < 24 && g % 3 != 2) read_k(slot, 2 * (g / 3) + g % 3);
+            if (g >= 24 && g % 2 == 0) issue_part(j3 >= 0 ? j3 : j1, freed, (g - 24) / 2);   // behind the last block the slot takes anything
+        }, 1, against(1, j0)));
+        if (edge(j1)) hide(0, TileWalk::index(j1));
+        settle(0, j1, half_step([&](int g) { if (g < 16) form_o(1)(g); else form_s(1)(g - 16); }, [&](int g) {
+            if (g < 8 && g % 2 == 0) issue_part(j3 >= 0 ? j3 : j1, freed, 4 + g / 2);
+            if (g >= 8 && (g - 8) % 3 != 2) read_v(slot, 2 * ((g - 8) / 3) + (g - 8) % 3);
+        }, 0, against(0, j1)));
+        if (edge(j1)) hide(1, TileWalk::index(j1));
+        at1 = at1 == 2 ? 0 : at1 + 1;
+        j0 = j1; j1 = j2; j2 = j3;
+    }
+    every &= j0;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // nothing is on its way to LDS when the workgroup ends
+    if (j0 >= 0) {                                             // the last block
 #pragma unroll
-        for (int cc = 0; cc < 2; ++cc)
+        for (int f = 0; f < 16; ++f) form_o(0)(f);
+        settle(1, j0, exponentials(1, against(1, j0)));
 #pragma unroll
-            for (int r = 0; r < 16; ++r) sn[cc][r] = 0.f;
-#pragma unroll
-        for (int f = 0; f < 16; ++f) {
-            sn[f & 1] = IV2_MFMA32(kf[f], qf[f >> 1], sn[f & 1]);
-            if (f < 4) {
-                read_k(8 + 2 * f);
-                read_k(9 + 2 * f);
-            } else if (f < 12) {
-                read_v(f - 4);
-            }
-            const int cc = f >> 3, r = 2 * (f & 7);
-            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[cc][r], p.scale_log2, -m));
-            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[cc][r + 1], p.scale_log2, -m));
-            part[0] += p0;
-            part[1] += p1;
-            asm volatile("" : "+v"(part[0]), "+v"(part[1]));   // here, not all at the end
-            pf[2 * cc + ((r >> 2) & 1)][(r >> 3) * 4 + (r & 3)] = static_cast<elem_t>(p0);
-            pf[2 * cc + ((r >> 2) & 1)][(r >> 3) * 4 + (r & 3) + 1] = static_cast<elem_t>(p1);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        float rs = part[0] + part[1];
-        asm volatile("" : "+v"(pf[0]), "+v"(pf[1]), "+v"(pf[2]), "+v"(pf[3]), "+v"(rs));
-        if (__ballot(!(rs <= kLazyLimit)) != 0ull) {           // a row without a reference yet, one that grew, or NaN: the block's scores once more
-            load_k(slot, 0);
-            load_k(slot, 1);
-            scores(sc);
-            if (edge) hide(sc, j);
-            float mx = -INFINITY;
-#pragma unroll
-            for (int cc = 0; cc < 2; ++cc)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[cc][r]);
-            const float m_new = fmaxf(m, half_max(mx) * p.scale_log2);
-            const float alpha = __builtin_amdgcn_exp2f(m - m_new);
-            l *= alpha;
-            m = m_new;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) o[t] *= alpha;
-            rs = exponentials(sc);
-        }
-        l += rs;
-        // Region B: P V, the rest of V ahead of the MFMAs that need it, the first half of the next K behind them.
-#pragma unroll
-        for (int f = 0; f < 16; ++f) {                         // f = 8 cc + 4 jj + t
-            o[f & 3] = IV2_MFMA32(vf[f], pf[f >> 2], o[f & 3]);
-            if (f < 8) {
-                read_v(8 + f);
-            } else {
-                const uint4 raw = ring[((slot + 2) & 3) * 2048 + k_unit + (f & 1) * 512 + ((f - 8) >> 2) * 64 + ((f >> 1) & 1) * 32];
-                __builtin_memcpy(&kf[f - 8], &raw, 16);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    for (int j = 0; j < blocks; j += 2) {                      // uniform over the workgroup
-        step(j, sa, sb);
-        if (j + 1 < blocks) step(j + 1, sb, sa);
+        for (int f = 0; f < 16; ++f) form_o(1)(f);
     }
 
-    const float l_tot = half_sum(l);
-    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    int row = n;
-    asm volatile("" : "+v"(row));                              // computed again: the walk has no registers to spare
-    const int i = i_wave + (row >> x.row_shift), head = row & ((1 << x.row_shift) - 1);
-    if (i >= Sq || head >= p.group) return;
-    const int64_t tok = static_cast<int64_t>(q0) + i;
-    elem_bits* op = p.out + tok * p.o_tok_stride + h_kv * p.o_kvh_stride + head * p.o_grp_stride + 4 * h;
+    // from here on the arguments are read again: what only the end needs would take registers from the walk
+    typedef const __attribute__((address_space(4))) FwdParams* Arguments;
+    Arguments late = reinterpret_cast<Arguments>(reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr()));
+    asm volatile("" : "+s"(late));
+    auto store = [&](const floatx16 (&oo)[4], float mm, float ll, int hf, bool lanes) {
+        const float l_tot = half_sum(ll);
+        const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+        int row = n;
+        asm volatile("" : "+v"(row));                          // computed again: the walk has no registers to spare
+        const int i = i_wave + hf * per_half + (row >> x.row_shift), head = row & ((1 << x.row_shift) - 1);
+        if (i < Sq && head < late->group && lanes) {
+            const int64_t tok = static_cast<int64_t>(q0) + i;
+            elem_bits* op = late->out + tok * late->o_tok_stride + h_kv * late->o_kvh_stride + head * late->o_grp_stride + 4 * h;
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+            for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int i4 = 0; i4 < 4; ++i4) {
-            uint2 wv;
-            wv.x = pack_elem2(o[t][4 * i4] * inv, o[t][4 * i4 + 1] * inv);
-            wv.y = pack_elem2(o[t][4 * i4 + 2] * inv, o[t][4 * i4 + 3] * inv);
-            *reinterpret_cast<uint2*>(op + 32 * t + 8 * i4) = wv;
+                for (int i4 = 0; i4 < 4; ++i4) {
+                    uint2 wv;
+                    wv.x = pack_elem2(oo[t][4 * i4] * inv, oo[t][4 * i4 + 1] * inv);
+                    wv.y = pack_elem2(oo[t][4 * i4 + 2] * inv, oo[t][4 * i4 + 3] * inv);
+                    *reinterpret_cast<uint2*>(op + 32 * t + 8 * i4) = wv;
+                }
+            if (h == 0) {
+                const float lse = l_tot > 0.f ? mm * 0.69314718055994530942f + logf(l_tot) : INFINITY;
+                late->lse[h_kv * late->lse_kvh_stride + tok * late->lse_tok_stride + head * late->lse_grp_stride] = lse;
+            }
         }
-    if (h == 0) {
-        const float lse = l_tot > 0.f ? m * 0.69314718055994530942f + logf(l_tot) : INFINITY;
-        p.lse[h_kv * p.lse_kvh_stride + tok * p.lse_tok_stride + head * p.lse_grp_stride] = lse;
+    };
+    const int full = (1 << 2 * per_half) - 1;
+    if (late->mask != nullptr && (every >> kTokenBits & full) != full) {             // uniform per wavefront: a block was walked for some rows only
+        // An infinity or a NaN in a block passes to rows that did not select it (0 x inf).  Where the result shows one, this wavefront's tokens are
+        // walked once more, one at a time and each over its own blocks alone.
+        float sum = l[0] + l[1];
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sum += __builtin_fabsf(o[hf][t][r]);
+        if (__ballot(!(sum < INFINITY)) != 0ull) {
+            for (int t = 0; t < 2 * per_half && i_wave + t < Sq; ++t) {
+                const int hf = t >= per_half ? 1 : 0, lk = last_of(i_wave + t);
+                {
+                    const int head = n & ((1 << x.row_shift) - 1);                  // every token's rows hold this token's heads: the copies are not stored
+                    const elem_bits* qp = late->q + (static_cast<int64_t>(q0) + i_wave + t) * late->q_tok_stride + h_kv * late->q_kvh_stride +
+                                          (head < late->group ? head : late->group - 1) * late->q_grp_stride + 8 * h;
+#pragma unroll
+                    for (int ks = 0; ks < 8; ++ks) vf[ks] = *reinterpret_cast<const elem8*>(qp + 16 * ks);
+                }
+                BlockWalker own;
+                own.init(late->mask + (static_cast<int64_t>(h_kv) * late->total_q + q0 + i_wave + t) * late->n64, late->n64, lk < 0 ? -1 : lk >> 6);
+                float mm = kNoReference, ll = 0.f;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) o[0][u] = zero;
+                for (int j = own.next(); j >= 0 && j < x.max_blocks; j = own.next()) {
+                    const uint4* ks_src = reinterpret_cast<const uint4*>(kimg + static_cast<int64_t>(j) * kImageElems) + k_unit;
+                    const uint4* vs_src = reinterpret_cast<const uint4*>(vimg + static_cast<int64_t>(j) * kImageElems) + v_unit;
+                    s[0][0] = s[0][1] = zero;
+#pragma unroll
+                    for (int f = 0; f < 16; ++f) {
+                        const uint4 raw = ks_src[k_at(f)];
+                        __builtin_memcpy(&kf[0], &raw, 16);
+                        s[0][f & 1] = IV2_MFMA32(kf[0], vf[f >> 1], s[0][f & 1]);
+                    }
+                    const int lim = lk - j * kBlockN;
+                    float mx = -INFINITY;
+#pragma unroll
+                    for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) {
+                            if (32 * cc + 8 * (r >> 2) + 4 * h + (r & 3) > lim) s[0][cc][r] = -INFINITY;
+                            mx = fmaxf(mx, s[0][cc][r]);
+                        }
+                    const float m_new = fmaxf(mm, half_max(mx) * late->scale_log2), alpha = __builtin_amdgcn_exp2f(mm - m_new);
+                    mm = m_new;
+                    ll = ll * alpha + exponentials(0, mm);
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) o[0][u] *= alpha;
+#pragma unroll
+                    for (int f = 0; f < 16; ++f) {
+                        const uint4 raw = vs_src[v_at(f)];
+                        __builtin_memcpy(&kf[0], &raw, 16);
+                        o[0][f & 3] = IV2_MFMA32(kf[0], operand(pf[0][f >> 2]), o[0][f & 3]);
+                    }
+                }
+                store(o[0], mm, ll, hf, (n >> x.row_shift) == t - hf * per_half);
+            }
+            return;
+        }
     }
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) store(o[hf], m[hf], l[hf], hf, true);
 }
 
 // Time of a dense launch whose workgroups take `tokens` tokens each, one workgroup per CU at a time: in microseconds, but for what all
@@ -334,6 +520,49 @@ bool dense_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int
     return tiles < groups + 1.;
 }
 
+// Time of a launch as in dense_walk_time, where a workgroup whose last token sees b key blocks takes cost(b).
+template <typename Cost>
+static double masked_walk_time(int tokens, Cost cost, double partial, int batch, int num_heads_k, int64_t total_q, int64_t total_k,
+                               int max_seqlen_q, int max_seqlen_k, bool causal) {
+    auto mean = [&](double q, double k) {                      // over the workgroups of a sequence
+        const double first = causal ? (k > q ? k - q : 0.) : k;
+        if (q <= tokens) return cost(ceil(k / kBlockN));
+        double sum = 0.;
+        for (int i = 0; i < 16; ++i) sum += cost((first + (k - first) * (i + 0.5) / 16) / kBlockN + 0.5);
+        return sum / 16;
+    };
+    const int others = batch - 1;
+    const double q = others > 0 && total_q > max_seqlen_q ? static_cast<double>(total_q - max_seqlen_q) / others : 0.;
+    const double k = others > 0 && total_k > max_seqlen_k ? static_cast<double>(total_k - max_seqlen_k) / others : 0.;
+    const double of_longest = ceil(static_cast<double>(max_seqlen_q) / tokens), of_others = others * ceil(q / tokens);
+    const double rounds = num_heads_k * (of_longest + of_others) / 256.;
+    const double each = (of_longest * mean(max_seqlen_q, max_seqlen_k) + (of_others > 0. ? of_others * mean(q, k) : 0.)) / (of_longest + of_others);
+    const double chain = cost(ceil(static_cast<double>(max_seqlen_k) / kBlockN));
+    const double all = each * (rounds + (rounds > 1. ? partial : 0.));
+    return (chain > all ? chain : all) + 0.0017 * num_heads_k * batch * of_longest;
+}
+
+// Whether a forward whose rows select at most `most_selected` blocks goes by tiles.  A tile walks the blocks that any of its tokens selected,
+// nearly all it can see, in 1.4 us each; a group of 8 tokens takes 1.0 us for a block that all of them selected and up to 1.8 for those that its tokens
+// walk on their own.  So tiles win while the rows see up to about two and a half times what they select, and lose where the longest tile's chain decides
+// (one short prompt, one KV head).  The constants are a fit to 139 launches of 1 to 8 sequences of 130 to 25000 tokens, 16 to 64 blocks selected, 1 to 4
+// KV heads, groups of 8 and 16 (within 7 and 9 %); the choice costs 0.1 % of the better walk's time on average, 7 % in the worst, where the groups of 8 tokens alone
+// cost 24 %.  Operator in us, groups of 8 tokens | tiles (* the one taken here), 2 KV heads of 16 unless it says otherwise:
+//   64 blocks selected: 3000 tokens 113 | 89 *, 8000 505 | 454 *, 12000 840 * | 960, 777 + 5003 + 1291 + 9173 883 | 815 *; 4 heads 4 x 4096 1396 | 1010 *
+//   16 blocks selected: 1000 tokens 31 * | 39, 2048 56 * | 62, 1023 + 3001 + 517 + 2200 151 | 145 *; 4 heads of 8 4000 182 | 128 *
+bool masked_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal,
+                      int most_selected) {
+    if (most_selected <= 0 || max_seqlen_q <= 0 || max_seqlen_k <= 0) return false;
+    const double most = most_selected;
+    const double tiles = masked_walk_time(kTileRows >> tile_row_shift(group), [](double b) { return 10. + 1.4 * b; }, 0.5, batch, num_heads_k,
+                                          total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
+    const double groups = masked_walk_time(8, [&](double b) {
+        const double beyond = b > most ? b - most : 0.;
+        return 8. + (b < most ? b : most) + 0.4 * (beyond < most ? beyond : most);
+    }, 0.3, batch, num_heads_k, total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
+    return tiles < groups;
+}
+
 int launch_stage2_fwd_tile(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q, int max_seqlen_k, bool causal) {
     TileExtra x{};
     x.batch = batch;
@@ -345,11 +574,11 @@ int launch_stage2_fwd_tile(hipStream_t st, const FwdParams& p, int batch, int nu
     const int64_t total = static_cast<int64_t>(x.sequences) * x.tiles_per_seq;
     IV2_CHECK(total <= 0x3fffffff, "varlen_fwd: too many token groups");
     const int64_t grid = (total + 7) / 8 * 8;
-    const size_t lds = kRingTiles * kTileBytes;
+    const size_t lds = kSlots * kSlotBytes;
     const auto kernel = causal ? &stage2_fwd_tile_kernel<true> : &stage2_fwd_tile_kernel<false>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     IV2_CHECK(e == hipSuccess, "varlen_fwd: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(512), lds, st, p, x);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(64 * kTileWaves), lds, st, p, x);
     IV2_LAUNCH_CHECK();
     return 0;
 }
@@ -361,5 +590,10 @@ extern "C" int infllmv2_varlen_fwd_dense_tiles(int batch, int64_t total_q, int64
                                                int max_seqlen_k, int is_causal) {
     return num_heads_k > 0 && batch > 0 && IV2_NS::dense_tiles_pay(batch, num_heads_k, num_heads / num_heads_k, total_q, total_k, max_seqlen_q,
                                                                    max_seqlen_k, is_causal != 0) ? 1 : 0;
+}
+extern "C" int infllmv2_varlen_fwd_masked_tiles(int batch, int64_t total_q, int64_t total_k, int num_heads, int num_heads_k, int max_seqlen_q,
+                                                int max_seqlen_k, int is_causal, int most_selected) {
+    return num_heads_k > 0 && batch > 0 && IV2_NS::masked_tiles_pay(batch, num_heads_k, num_heads / num_heads_k, total_q, total_k, max_seqlen_q,
+                                                                    max_seqlen_k, is_causal != 0, most_selected) ? 1 : 0;
 }
 #endif
