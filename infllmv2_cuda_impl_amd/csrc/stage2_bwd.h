@@ -12,8 +12,7 @@ struct BwdParams {
     const elem_bits* out;
     elem_bits* dq;
     const float* lse;
-    float* dsum;                    // (Hk, total_q * 16): D of head 16h+g of token t at [h][16 t + g]
-    float* rowstat;                 // (Hk, total_q, 32): LSE * log2(e) of the 16 heads, then D of the 16 heads
+    float* rowstat;                 // (Hk, total_q, 32): LSE * log2(e) of the 16 heads, then D of the 16 heads; the dQ kernel leaves it for the dK/dV kernel
     const elem_bits* kimg;          // K, K-image order
     const elem_bits* vimg_r;        // V, K-image order
     float* dk_acc;                  // (total_k, Hk, 128) fp32

@@ -14,7 +14,7 @@
 //   * dK/dV: column-parallel (stage2_bwd_dkdv.hip).  Two wavefronts own a 64-key block (32 keys each) and a
 //     slice of 512 query tokens, walk the transposed mask, keep their 32x128 dK^T and dV^T tiles
 //     in accumulation registers and flush once per slice with fp32 atomics.
-// This file holds the preprocessing kernel, the fp32 -> bf16 conversion of dK/dV and the C entry
+// This file holds the fp32 -> bf16 conversion of dK/dV and the C entry
 // point.
 #include "common.h"
 #include "kv_image.h"
@@ -25,40 +25,6 @@
 #include <stdlib.h>
 
 namespace IV2_NS {
-
-// ---------------------------------------------------------------------------------------------
-// preprocessing: D = rowsum(dO * O) (compute_dot_do_o, flash_bwd_preprocess_kernel.h:56-137) and, per token,
-// the 32 row scalars the dK/dV kernel fetches with one 128-byte transfer
-// ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256)
-void bwd_prep_kernel(const BwdParams p) {
-    // one 16-lane group per (token, head-in-group): 16 lanes x 8 elements = 128
-    const int64_t tok = static_cast<int64_t>(blockIdx.x);
-    const int h = blockIdx.y;
-    const int tid = threadIdx.x;
-    const int row = tid >> 4, part = tid & 15;
-    const bool spare = row >= p.group;                         // a row that only fills the 16-row tiles of the other kernels
-    const int rowc = spare ? p.group - 1 : row;
-    const uint4 dv = *reinterpret_cast<const uint4*>(p.dout + tok * p.do_tok + h * p.do_kvh + rowc * p.do_grp + part * 8);
-    const uint4 ov = *reinterpret_cast<const uint4*>(p.out + tok * p.o_tok + h * p.o_kvh + rowc * p.o_grp + part * 8);
-    const uint32_t dw[4] = {dv.x, dv.y, dv.z, dv.w};
-    const uint32_t ow[4] = {ov.x, ov.y, ov.z, ov.w};
-    float acc = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        acc += elem_to_f32(static_cast<elem_bits>(dw[i] & 0xffff)) * elem_to_f32(static_cast<elem_bits>(ow[i] & 0xffff));
-        acc += elem_to_f32(static_cast<elem_bits>(dw[i] >> 16)) * elem_to_f32(static_cast<elem_bits>(ow[i] >> 16));
-    }
-#pragma unroll
-    for (int off = 1; off < 16; off <<= 1) acc += __shfl_xor(acc, off);
-    if (part == 0) {
-        // spare rows get LSE = +inf and D = 0: their P = exp2(x - inf) and dS = P (dP - D) vanish in every kernel
-        p.dsum[static_cast<int64_t>(h) * p.total_q * 16 + tok * 16 + row] = spare ? 0.f : acc;
-        float* rs = p.rowstat + (static_cast<int64_t>(h) * p.total_q + tok) * 32;
-        rs[row] = spare ? INFINITY : p.lse[h * p.lse_kvh + tok * p.lse_tok + row * p.lse_grp] * kLog2e;
-        rs[16 + row] = spare ? 0.f : acc;
-    }
-}
 
 __global__ __launch_bounds__(256)
 void zero_f32_kernel(float4* __restrict__ ptr, int64_t n4) {
@@ -89,7 +55,7 @@ void bwd_convert_dkdv_kernel(const BwdParams p) {
 static size_t align256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
 struct BwdLayout {
-    size_t images, mask, dsum, rowstat, dk_acc, dv_acc, total;
+    size_t images, mask, rowstat, dk_acc, dv_acc, total;
     size_t det_flags, det_slots, det_total;                    // deterministic mode only, after everything else
     int det_slices;
 };
@@ -100,7 +66,6 @@ static BwdLayout bwd_layout(int batch, int64_t total_q, int64_t total_k, int num
     L.images = off; off += align256(image_bytes(total_k, batch, num_heads_k));   // K image | V in K-image order
     const int64_t k_blocks = (max_seqlen_k + kBlockN - 1) / kBlockN;
     L.mask = off; off += align256(static_cast<size_t>(num_heads_k) * k_blocks * ((total_q + 63) / 64) * 8);
-    L.dsum = off; off += align256(static_cast<size_t>(num_heads_k) * total_q * 16 * 4);
     L.rowstat = off; off += align256(static_cast<size_t>(num_heads_k) * total_q * 32 * 4);
     L.dk_acc = off; off += align256(static_cast<size_t>(total_k) * num_heads_k * kHeadDim * 4);
     L.dv_acc = off; off += align256(static_cast<size_t>(total_k) * num_heads_k * kHeadDim * 4);
@@ -171,7 +136,6 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_bwd)(void* stream, const void* dout, co
     p.out = static_cast<const elem_bits*>(out);
     p.dq = static_cast<elem_bits*>(dq);
     p.lse = softmax_lse;
-    p.dsum = reinterpret_cast<float*>(ws + L.dsum);
     p.rowstat = reinterpret_cast<float*>(ws + L.rowstat);
     const int64_t n_slots = image_slots(total_k, batch);
     const int64_t img_elems = n_slots * num_heads_k * kImageElems;
@@ -225,8 +189,6 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_bwd)(void* stream, const void* dout, co
             p.bwd_mask = bwd_mask;
         }
         IV2_CHECK(total_q <= 0x7fffffffll, "varlen_bwd: too many query tokens");
-        hipLaunchKernelGGL(bwd_prep_kernel, dim3(static_cast<unsigned>(total_q), num_heads_k), dim3(256), 0, st, p);
-        IV2_LAUNCH_CHECK();
         rc = launch_bwd_dq_hybrid(st, p, batch, max_seqlen_q, is_causal != 0);
         if (rc != 0) return rc;
         rc = launch_bwd_dkdv_wave(st, p, batch, max_seqlen_q, is_causal != 0);

@@ -13,6 +13,10 @@
 // fragments straight from global memory into registers, the K fragments parked in a private LDS
 // tile for the same transposed read.  The two walks are interleaved, one block of each per turn.
 //
+// The kernel also forms D = rowsum(dO * O) (compute_dot_do_o, flash_bwd_preprocess_kernel.h:56-137): it has dO in registers, and O
+// costs its set-up one more request.  A pass of its own read dO and O once more from HBM: 227 us of 22.7 ms for 71552 packed tokens, 18 of 680 for
+// 6741 in four sequences (whole training passes 22970 -> 22740 and 680 -> 660).  Its row scalars go to the dK/dV kernel.
+//
 // What bounds it: the chain S, dP, dQ of a block in two wavefronts per SIMD that the turn's barrier keeps in step.  At 32768
 // tokens, 64 blocks per row and 2 KV heads (3.65 to 3.9 ms) the matrix pipe is busy 39 % and the return path from L2, as in the
 // forward the busiest unit, 70 %; but with the own blocks' loads taken out the kernel still takes 88 % of its time.
@@ -158,22 +162,22 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
     __syncthreads();
     for (int w = lane; w < nw; w += 64) own[w] &= ~com[w];
 
-    // ---- this token's operands ----
-    elem8 qf[4], dof[4];
+    // ---- this token's operands, and D = rowsum(dO * O) from them ----
+    elem8 qf[4], dof[4], of[4];
+    float lse2;
     {
         const int nq = n < p.group ? n : p.group - 1;          // rows beyond the group repeat its last head; their LSE is +inf
         const elem_bits* qp = p.q + tok * p.q_tok + h * p.q_kvh + nq * p.q_grp + 8 * g;
         const elem_bits* dp = p.dout + tok * p.do_tok + h * p.do_kvh + nq * p.do_grp + 8 * g;
+        const elem_bits* op = p.out + tok * p.o_tok + h * p.o_kvh + nq * p.o_grp + 8 * g;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             qf[c] = *reinterpret_cast<const elem8*>(qp + 32 * c);
             dof[c] = *reinterpret_cast<const elem8*>(dp + 32 * c);
+            of[c] = *reinterpret_cast<const elem8*>(op + 32 * c);
         }
+        lse2 = p.lse[h * p.lse_kvh + tok * p.lse_tok + nq * p.lse_grp] * kLog2e;
     }
-    const float* rs = p.rowstat + (static_cast<int64_t>(h) * p.total_q + tok) * 32;    // [LSE * log2(e) x 16 | D x 16]
-    float lse2 = rs[n];
-    float dsum = rs[16 + n];
-    const floatx4 neg_dsum = {-dsum, -dsum, -dsum, -dsum};     // the dP accumulators start here: dS = P (dP - D) is then one product
     floatx4 dq[8];
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) dq[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -226,10 +230,21 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
     // count the ordinary loads that may be younger than the DMA they wait for.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
-    for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(qf[c]), "+v"(dof[c]));
+    for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(qf[c]), "+v"(dof[c]), "+v"(of[c]));
 #pragma unroll
     for (int f = 0; f < 16; ++f) asm volatile("" : "+v"(kreg[f]));
-    asm volatile("" : "+v"(lse2), "+v"(dsum));
+    asm volatile("" : "+v"(lse2));
+    float dsum = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dsum += static_cast<float>(dof[c][e]) * static_cast<float>(of[c][e]);
+    dsum = wave_sum_over_g(dsum);
+    if (n >= p.group) {                                        // spare rows: P = exp2(x - inf) and dS = P (dP - D) vanish, here and in the dK/dV kernel
+        lse2 = INFINITY;
+        dsum = 0.f;
+    }
+    const floatx4 neg_dsum = {-dsum, -dsum, -dsum, -dsum};     // the dP accumulators start here: dS = P (dP - D) is then one product
     int j0 = next_common();
     if (j0 >= 0) issue(j0, 0);
     int tile = 0;
@@ -345,7 +360,10 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
             jp = jn;
         }
     }
-    if (!live || n >= p.group) return;
+    if (!live) return;
+    // what the dK/dV kernel fetches of a token with one 128-byte transfer: [LSE * log2(e) x 16 | D x 16]
+    if (g < 2) p.rowstat[(static_cast<int64_t>(h) * p.total_q + tok) * 32 + 16 * g + n] = g == 0 ? lse2 : -neg_dsum[0];
+    if (n >= p.group) return;
 
     elem_bits* op = p.dq + tok * p.dq_tok + h * p.dq_kvh + n * p.dq_grp + 4 * g;
 #pragma unroll
