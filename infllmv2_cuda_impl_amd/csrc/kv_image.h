@@ -36,11 +36,25 @@ __device__ __forceinline__ int64_t image_slot0(const int* cu_seqlens_k, int b) {
     return cu_seqlens_k[b] / kBlockN + b;
 }
 
-// Launches the packing pre-pass.  workspace receives [K image | V image] for the forward or, with
-// backward_images, [K image | V in K-image order] (the backward contracts V over d, and reads K^T out of the
-// K image by transposed LDS loads).
+// One block's K image, by a workgroup of 256: rows is the block's first row, `valid` of its keys are inside the sequence.
+__device__ __forceinline__ void write_k_image(const elem_bits* rows, int64_t row_stride, int valid, elem_bits* image, int tid) {
+    uint4 val[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int u = tid + 256 * i, c = (u >> 6) & 3, lane = u & 63;
+        const int key = 16 * (u >> 8) + (lane & 15);
+        val[i] = make_uint4(0, 0, 0, 0);
+        if (key < valid) val[i] = *reinterpret_cast<const uint4*>(rows + key * row_stride + 32 * c + 8 * (lane >> 4));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(image + (tid + 256 * i) * 8) = val[i];
+}
+// What the images ask of k and v.
+int check_pack(const void* k, const void* v, const int32_t* cu_seqlens_k, const void* workspace, size_t workspace_bytes, int batch,
+               int64_t total_k, int num_heads_k, int max_seqlen_k, const int64_t* k_strides, const int64_t* v_strides);
+// Launches the packing pre-pass.  workspace receives [K image | V image].
 int launch_pack(hipStream_t st, const void* k, const void* v, const int32_t* cu_seqlens_k, void* workspace,
                 size_t workspace_bytes, int batch, int64_t total_k, int num_heads_k, int max_seqlen_k,
-                const int64_t* k_strides, const int64_t* v_strides, bool backward_images);
+                const int64_t* k_strides, const int64_t* v_strides);
 
 }  // namespace IV2_NS

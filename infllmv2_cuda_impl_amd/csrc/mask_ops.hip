@@ -6,6 +6,7 @@
 // csrc/blockmask_to_uint64.cuh:10-51 and infllm_v2/infllmv2_sparse_attention.py:344-350 of the
 // reference; the kernels themselves are new.
 #include "common.h"
+#include "mask_tile.h"
 #include "infllmv2_hip.h"
 
 namespace infllmv2 {
@@ -90,31 +91,12 @@ void blockmask_to_uint64_kernel(const uint8_t* __restrict__ in, uint64_t* __rest
 // ---------------------------------------------------------------------------------------------
 // Forward mask (heads, total_q, n64_fwd) -> backward mask (heads, k_blocks, n64_bwd):
 //   bwd[h, kb, w] bit u  =  fwd[h, 64w + u, kb / 64] bit (kb % 64).
-// One wavefront transposes one 64x64 bit tile: lane u holds the forward word of token 64w+u,
-// 64 ballots produce the 64 backward words of the tile, lane b stores word b.
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256)
 void transpose_blockmask_kernel(const uint64_t* __restrict__ fwd, uint64_t* __restrict__ bwd,
                                 int heads, int64_t total_q, int n64_fwd, int k_blocks, int n64_bwd) {
-    const int lane = threadIdx.x & 63;
-    const int64_t tile = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const int64_t tiles_per_head = static_cast<int64_t>(n64_bwd) * n64_fwd;
-    if (tile >= tiles_per_head * heads) return;              // uniform per wavefront
-    const int h = static_cast<int>(tile / tiles_per_head);
-    const int64_t rem = tile - h * tiles_per_head;
-    const int w = static_cast<int>(rem / n64_fwd);           // 64-token group
-    const int c = static_cast<int>(rem - static_cast<int64_t>(w) * n64_fwd);   // forward word column
-    const int64_t tok = static_cast<int64_t>(w) * 64 + lane;
-    uint64_t mine = 0;
-    if (tok < total_q) mine = fwd[(static_cast<int64_t>(h) * total_q + tok) * n64_fwd + c];
-    uint64_t result = 0;
-#pragma unroll
-    for (int b = 0; b < 64; ++b) {
-        const uint64_t col = __builtin_amdgcn_ballot_w64(((mine >> b) & 1ull) != 0);
-        if (lane == b) result = col;
-    }
-    const int kb = c * 64 + lane;
-    if (kb < k_blocks) bwd[(static_cast<int64_t>(h) * k_blocks + kb) * n64_bwd + w] = result;
+    transpose_mask_tile(fwd, bwd, static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6), threadIdx.x & 63, heads, total_q, n64_fwd,
+                        k_blocks, n64_bwd);
 }
 
 }  // namespace infllmv2

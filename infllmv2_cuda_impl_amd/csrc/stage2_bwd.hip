@@ -19,12 +19,63 @@
 #include "common.h"
 #include "kv_image.h"
 #include "block_walker.h"
+#include "mask_tile.h"
 #include "stage2_bwd.h"
 #include "infllmv2_hip.h"
 #include <math.h>
 #include <stdlib.h>
 
 namespace IV2_NS {
+
+// What the two gradient kernels need before they start, in one launch: the images of K and V (both in K-image order: the backward contracts V
+// over d, and reads K^T out of the K image by transposed LDS loads), the transposed mask and zeros in the fp32 accumulators of dK and dV.  The three
+// have nothing to do with one another and are short: as launches of their own they took 5 to 6 us each whatever the size (a training pass of 6741
+// tokens 660 -> 652 us).  Workgroups of the launch: images, then mask tiles (four each), then zeros.
+struct BwdFront {
+    const elem_bits* k;
+    const elem_bits* v;
+    elem_bits* kimg;
+    elem_bits* vimg_r;
+    const int* cu_seqlens_k;
+    int64_t k_row_stride, k_head_stride, v_row_stride, v_head_stride;
+    int64_t n_slots;
+    int max_blocks, batch, heads;
+    const uint64_t* fwd_mask;
+    uint64_t* bwd_mask;
+    int64_t total_q;
+    int n64_fwd, n64_bwd;
+    float4* acc;
+    int64_t acc4;                                              // float4s to clear
+    int64_t images, mask_tiles;
+    int image_groups, mask_groups, zero_groups;                // workgroups of each kind
+};
+constexpr int64_t kMostFrontGroups = 1 << 20;                  // of a kind: a launch has fewer than 2^32 threads
+__global__ __launch_bounds__(256)
+void bwd_front_kernel(const BwdFront f) {
+    int group = blockIdx.x;
+    const int tid = threadIdx.x;
+    if (group < f.image_groups) {
+        for (int64_t i = group; i < f.images; i += f.image_groups) {
+            const int j = static_cast<int>(i % f.max_blocks), b = static_cast<int>(i / f.max_blocks % f.batch), h = static_cast<int>(i / f.max_blocks / f.batch);
+            const int k0 = f.cu_seqlens_k[b], valid = f.cu_seqlens_k[b + 1] - k0 - j * kBlockN;          // keys of this block inside the sequence
+            if (valid <= 0) continue;
+            const int64_t row = k0 + static_cast<int64_t>(j) * kBlockN;
+            const int64_t at = (static_cast<int64_t>(h) * f.n_slots + image_slot0(f.cu_seqlens_k, b) + j) * kImageElems;
+            write_k_image(f.k + row * f.k_row_stride + h * f.k_head_stride, f.k_row_stride, valid, f.kimg + at, tid);
+            write_k_image(f.v + row * f.v_row_stride + h * f.v_head_stride, f.v_row_stride, valid, f.vimg_r + at, tid);
+        }
+        return;
+    }
+    group -= f.image_groups;
+    if (group < f.mask_groups) {
+        for (int64_t tile = static_cast<int64_t>(group) * 4 + (tid >> 6); tile < f.mask_tiles; tile += static_cast<int64_t>(f.mask_groups) * 4)
+            transpose_mask_tile(f.fwd_mask, f.bwd_mask, tile, tid & 63, f.heads, f.total_q, f.n64_fwd, f.max_blocks, f.n64_bwd);
+        return;
+    }
+    group -= f.mask_groups;
+    const int64_t stride = static_cast<int64_t>(f.zero_groups) * 256;
+    for (int64_t i = static_cast<int64_t>(group) * 256 + tid; i < f.acc4; i += stride) f.acc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
 
 __global__ __launch_bounds__(256)
 void zero_f32_kernel(float4* __restrict__ ptr, int64_t n4) {
@@ -170,26 +221,45 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_bwd)(void* stream, const void* dout, co
                            static_cast<int64_t>((L.det_slots - L.det_flags) / 16));
         IV2_LAUNCH_CHECK();
     }
-    // dK/dV accumulators start at zero (fill kernel, no memset node)
+    const bool work = total_q > 0 && max_seqlen_q > 0 && total_k > 0 && max_seqlen_k > 0;
     if (total_k > 0) {
-        const int64_t n4 = static_cast<int64_t>((L.dv_acc - L.dk_acc) / 16) * 2;
         IV2_CHECK((L.dv_acc - L.dk_acc) == align256(static_cast<size_t>(total_k) * num_heads_k * kHeadDim * 4), "varlen_bwd: layout");
-        hipLaunchKernelGGL(zero_f32_kernel, dim3(2048), dim3(256), 0, st, reinterpret_cast<float4*>(p.dk_acc), n4);
+        BwdFront f{};
+        f.acc = reinterpret_cast<float4*>(p.dk_acc);           // dK/dV accumulators start at zero (stores of a kernel, no memset node)
+        f.acc4 = static_cast<int64_t>((L.dv_acc - L.dk_acc) / 16) * 2;
+        f.zero_groups = 1024;
+        if (work) {
+            const int rc = check_pack(k, v, cu_seqlens_k, ws + L.images, L.mask - L.images, batch, total_k, num_heads_k, max_seqlen_k, k_strides, v_strides);
+            if (rc != 0) return rc;
+            f.k = static_cast<const elem_bits*>(k);
+            f.v = static_cast<const elem_bits*>(v);
+            f.kimg = reinterpret_cast<elem_bits*>(ws + L.images);
+            f.vimg_r = f.kimg + img_elems;
+            f.cu_seqlens_k = cu_seqlens_k;
+            f.k_row_stride = k_strides[0]; f.k_head_stride = k_strides[1];
+            f.v_row_stride = v_strides[0]; f.v_head_stride = v_strides[1];
+            f.n_slots = n_slots;
+            f.max_blocks = p.k_blocks; f.batch = batch; f.heads = num_heads_k;
+            f.images = static_cast<int64_t>(p.k_blocks) * batch * num_heads_k;
+            if (fwd_blockmask != nullptr) {
+                IV2_CHECK(static_cast<int64_t>(n_uint64_per_row) * 64 >= p.k_blocks, "varlen_bwd: forward words too few for %d blocks", p.k_blocks);
+                f.mask_tiles = static_cast<int64_t>(num_heads_k) * p.n64_bwd * n_uint64_per_row;
+                f.fwd_mask = fwd_blockmask;
+                f.bwd_mask = reinterpret_cast<uint64_t*>(ws + L.mask);
+                f.total_q = total_q;
+                f.n64_fwd = n_uint64_per_row; f.n64_bwd = p.n64_bwd;
+                p.bwd_mask = f.bwd_mask;
+            }
+            IV2_CHECK(total_q <= 0x7fffffffll, "varlen_bwd: too many query tokens");
+            auto groups = [](int64_t n) { return static_cast<int>(n < kMostFrontGroups ? n : kMostFrontGroups); };
+            f.image_groups = groups(f.images);
+            f.mask_groups = groups((f.mask_tiles + 3) / 4);
+        }
+        hipLaunchKernelGGL(bwd_front_kernel, dim3(static_cast<unsigned>(f.image_groups + f.mask_groups + f.zero_groups)), dim3(256), 0, st, f);
         IV2_LAUNCH_CHECK();
     }
-    if (total_q > 0 && max_seqlen_q > 0 && total_k > 0 && max_seqlen_k > 0) {
-        int rc = launch_pack(st, k, v, cu_seqlens_k, ws + L.images, L.mask - L.images, batch, total_k, num_heads_k,
-                             max_seqlen_k, k_strides, v_strides, true);   // K image | V in K-image order
-        if (rc != 0) return rc;
-        if (fwd_blockmask != nullptr) {
-            uint64_t* bwd_mask = reinterpret_cast<uint64_t*>(ws + L.mask);
-            rc = infllmv2_transpose_blockmask(stream, fwd_blockmask, bwd_mask, num_heads_k, total_q, n_uint64_per_row,
-                                              p.k_blocks, p.n64_bwd);
-            if (rc != 0) return rc;
-            p.bwd_mask = bwd_mask;
-        }
-        IV2_CHECK(total_q <= 0x7fffffffll, "varlen_bwd: too many query tokens");
-        rc = launch_bwd_dq_hybrid(st, p, batch, max_seqlen_q, is_causal != 0);
+    if (work) {
+        int rc = launch_bwd_dq_hybrid(st, p, batch, max_seqlen_q, is_causal != 0);
         if (rc != 0) return rc;
         rc = launch_bwd_dkdv_wave(st, p, batch, max_seqlen_q, is_causal != 0);
         if (rc != 0) return rc;

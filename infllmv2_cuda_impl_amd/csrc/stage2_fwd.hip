@@ -30,8 +30,7 @@ struct PackParams {
     const elem_bits* k;
     const elem_bits* v;
     elem_bits* kimg;                // K in K-image order (operand of a GEMM contracting over d)
-    elem_bits* vimg;                // forward: V in V-image order (A operand of a GEMM contracting over keys), else null
-    elem_bits* vimg_r;              // backward: V in K-image order (dP = dO V^T contracts over d), else null
+    elem_bits* vimg;                // V in V-image order (A operand of a GEMM contracting over keys)
     const int* cu_seqlens_k;
     int64_t k_row_stride, k_head_stride;
     int64_t v_row_stride, v_head_stride;
@@ -53,29 +52,18 @@ void pack_kv_kernel(const PackParams p) {
     const elem_bits* vb = p.v + (k0 + static_cast<int64_t>(j) * kBlockN) * p.v_row_stride + h * p.v_head_stride;
     const int64_t img_off = (static_cast<int64_t>(h) * p.n_slots + slot) * kImageElems;
     const int valid = Sk - j * kBlockN;                       // keys of this block inside the sequence
-    const uint4 zero = make_uint4(0, 0, 0, 0);
-
-    for (int u = tid; u < 1024; u += 256) {
-        const int kt = u >> 8, c = (u >> 6) & 3, lane = u & 63;
-        const int r = lane & 15, g = lane >> 4;
-        const int key = 16 * kt + r;
-        uint4 val = zero;
-        if (key < valid) val = *reinterpret_cast<const uint4*>(kb + key * p.k_row_stride + 32 * c + 8 * g);
-        *reinterpret_cast<uint4*>(p.kimg + img_off + u * 8) = val;
-        if (p.vimg_r != nullptr) {
-            uint4 vv = zero;
-            if (key < valid) vv = *reinterpret_cast<const uint4*>(vb + key * p.v_row_stride + 32 * c + 8 * g);
-            *reinterpret_cast<uint4*>(p.vimg_r + img_off + u * 8) = vv;
-        }
+    uint4 val[4];                                             // requested together with K's rows
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int u = tid + 256 * i, key = u >> 4, d0 = (u & 15) * 8;
+        val[i] = make_uint4(0, 0, 0, 0);
+        if (key < valid) val[i] = *reinterpret_cast<const uint4*>(vb + key * p.v_row_stride + d0);
     }
-    // the image that contracts over the keys: V for the forward
-    if (p.vimg == nullptr) return;                            // uniform per workgroup
-    __syncthreads();
-    for (int u = tid; u < 1024; u += 256) {
-        const int key = u >> 4, d0 = (u & 15) * 8;
-        uint4 val = zero;
-        if (key < valid) val = *reinterpret_cast<const uint4*>(vb + key * p.v_row_stride + d0);
-        *reinterpret_cast<uint4*>(&vt[key][d0]) = val;
+    write_k_image(kb, p.k_row_stride, valid, p.kimg + img_off, tid);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int u = tid + 256 * i;
+        *reinterpret_cast<uint4*>(&vt[u >> 4][(u & 15) * 8]) = val[i];
     }
     __syncthreads();
     for (int u = tid; u < 1024; u += 256) {
@@ -103,9 +91,8 @@ extern "C" size_t infllmv2_kv_image_bytes(int64_t total_k, int batch, int num_he
 #endif
 
 namespace IV2_NS {
-int launch_pack(hipStream_t st, const void* k, const void* v, const int32_t* cu_seqlens_k, void* workspace,
-                size_t workspace_bytes, int batch, int64_t total_k, int num_heads_k, int max_seqlen_k,
-                const int64_t* k_strides, const int64_t* v_strides, bool backward_images) {
+int check_pack(const void* k, const void* v, const int32_t* cu_seqlens_k, const void* workspace, size_t workspace_bytes, int batch,
+               int64_t total_k, int num_heads_k, int max_seqlen_k, const int64_t* k_strides, const int64_t* v_strides) {
     IV2_CHECK(k && v && cu_seqlens_k && workspace, "pack_kv: null pointer");
     IV2_CHECK(batch > 0 && num_heads_k > 0 && total_k >= 0 && max_seqlen_k >= 0, "pack_kv: bad sizes");
     IV2_CHECK(num_heads_k <= 65535 && batch <= 65535, "pack_kv: batch and num_heads_k must not exceed 65535");
@@ -114,6 +101,13 @@ int launch_pack(hipStream_t st, const void* k, const void* v, const int32_t* cu_
               reinterpret_cast<uintptr_t>(workspace) % 16 == 0, "pack_kv: k, v and workspace must be 16-byte aligned");
     IV2_CHECK(k_strides[0] % 8 == 0 && k_strides[1] % 8 == 0 && v_strides[0] % 8 == 0 && v_strides[1] % 8 == 0,
               "pack_kv: k/v row and head strides must be multiples of 8 elements");
+    return 0;
+}
+int launch_pack(hipStream_t st, const void* k, const void* v, const int32_t* cu_seqlens_k, void* workspace,
+                size_t workspace_bytes, int batch, int64_t total_k, int num_heads_k, int max_seqlen_k,
+                const int64_t* k_strides, const int64_t* v_strides) {
+    const int rc = check_pack(k, v, cu_seqlens_k, workspace, workspace_bytes, batch, total_k, num_heads_k, max_seqlen_k, k_strides, v_strides);
+    if (rc != 0) return rc;
     const int64_t n_slots = image_slots(total_k, batch);
     const int max_blocks = (max_seqlen_k + kBlockN - 1) / kBlockN;
     if (max_blocks == 0 || total_k == 0) return 0;
@@ -121,8 +115,7 @@ int launch_pack(hipStream_t st, const void* k, const void* v, const int32_t* cu_
     pp.k = static_cast<const elem_bits*>(k);
     pp.v = static_cast<const elem_bits*>(v);
     pp.kimg = static_cast<elem_bits*>(workspace);
-    elem_bits* second = pp.kimg + n_slots * num_heads_k * kImageElems;
-    if (backward_images) pp.vimg_r = second; else pp.vimg = second;
+    pp.vimg = pp.kimg + n_slots * num_heads_k * kImageElems;
     pp.cu_seqlens_k = cu_seqlens_k;
     pp.k_row_stride = k_strides[0]; pp.k_head_stride = k_strides[1];
     pp.v_row_stride = v_strides[0]; pp.v_head_stride = v_strides[1];
@@ -140,7 +133,7 @@ extern "C" int infllmv2_pack_kv(void* stream, const void* k, const void* v, cons
                                 const int64_t* v_strides) {
     IV2_CHECK(head_dim == kHeadDim, "pack_kv: this build only supports head_dim 128 (got %d)", head_dim);
     return launch_pack(static_cast<hipStream_t>(stream), k, v, cu_seqlens_k, workspace, workspace_bytes, batch,
-                       total_k, num_heads_k, max_seqlen_k, k_strides, v_strides, false);
+                       total_k, num_heads_k, max_seqlen_k, k_strides, v_strides);
 }
 #endif
 
@@ -170,7 +163,7 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_fwd_selected)(void* stream, const void*
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (!kv_prepacked) {
         int rc = launch_pack(st, k, v, cu_seqlens_k, workspace, workspace_bytes, batch, total_k, num_heads_k,
-                             max_seqlen_k, k_strides, v_strides, false);
+                             max_seqlen_k, k_strides, v_strides);
         if (rc != 0) return rc;
     }
     const int64_t n_slots = image_slots(total_k, batch);
