@@ -329,6 +329,23 @@ int infllmv2_varlen_bwd(void* stream, const void* dout, const void* q, const voi
                         const int64_t* dv_strides, const int64_t* lse_strides, int n_uint64_per_row,
                         float softmax_scale, int is_causal, int deterministic);
 
+/* infllmv2_varlen_bwd for a caller that knows how many blocks a row of the mask has set at most (0: not known); without a
+ * mask the number is not looked at.  It decides which of two walks forms dQ; results do not depend on its being right, except for rounding. */
+int infllmv2_varlen_bwd_selected(void* stream, const void* dout, const void* q, const void* k, const void* v,
+                        const void* out, const float* softmax_lse, void* dq, void* dk, void* dv,
+                        const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                        const uint64_t* fwd_blockmask, void* workspace, size_t workspace_bytes, int batch,
+                        int64_t total_q, int64_t total_k, int num_heads, int num_heads_k, int head_dim,
+                        int max_seqlen_q, int max_seqlen_k, const int64_t* q_strides,
+                        const int64_t* k_strides, const int64_t* v_strides, const int64_t* o_strides,
+                        const int64_t* do_strides, const int64_t* dq_strides, const int64_t* dk_strides,
+                        const int64_t* dv_strides, const int64_t* lse_strides, int n_uint64_per_row,
+                        float softmax_scale, int is_causal, int deterministic, int most_selected);
+/* Whether infllmv2_varlen_bwd_selected forms dQ by tiles of 256 query rows (1) or by groups of 8 tokens (0). */
+int infllmv2_varlen_bwd_dq_tiles(int batch, int64_t total_q, int64_t total_k, int num_heads, int num_heads_k,
+                                 int max_seqlen_q, int max_seqlen_k, int is_causal, int most_selected);
+
+
 /* ---- Stage 2: decode against a KV cache -------------------------------------------------------- */
 
 /* The split count infllmv2_fwd_kvcache will use: `requested` if > 0 (capped at 64), else a heuristic
@@ -500,6 +517,16 @@ int infllmv2_varlen_bwd_f16(void* stream, const void* dout, const void* q, const
                             const int64_t* do_strides, const int64_t* dq_strides, const int64_t* dk_strides,
                             const int64_t* dv_strides, const int64_t* lse_strides, int n_uint64_per_row,
                             float softmax_scale, int is_causal, int deterministic);
+int infllmv2_varlen_bwd_selected_f16(void* stream, const void* dout, const void* q, const void* k, const void* v,
+                            const void* out, const float* softmax_lse, void* dq, void* dk, void* dv,
+                            const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                            const uint64_t* fwd_blockmask, void* workspace, size_t workspace_bytes, int batch,
+                            int64_t total_q, int64_t total_k, int num_heads, int num_heads_k, int head_dim,
+                            int max_seqlen_q, int max_seqlen_k, const int64_t* q_strides,
+                            const int64_t* k_strides, const int64_t* v_strides, const int64_t* o_strides,
+                            const int64_t* do_strides, const int64_t* dq_strides, const int64_t* dk_strides,
+                            const int64_t* dv_strides, const int64_t* lse_strides, int n_uint64_per_row,
+                            float softmax_scale, int is_causal, int deterministic, int most_selected);
 int infllmv2_fwd_kvcache_scores_f16(void* stream, const void* q, void* kcache, void* vcache, const int32_t* cache_seqlens,
                                     void* out, float* softmax_lse, const void* scores, int n_scores, int topk,
                                     void* workspace, size_t workspace_bytes, int batch, int num_heads, int num_heads_k,

@@ -42,6 +42,7 @@ SIGNATURES = {
     "infllmv2_varlen_fwd_selected": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _i, _i, _i64, _i64, _i, _i, _i, _i, _i,
                                      _p, _p, _p, _p, _p, _i, _f, _i, _i],
     "infllmv2_varlen_bwd": [_p] * 14 + [_sz, _i, _i64, _i64, _i, _i, _i, _i, _i] + [_p] * 9 + [_i, _f, _i, _i],
+    "infllmv2_varlen_bwd_selected": [_p] * 14 + [_sz, _i, _i64, _i64, _i, _i, _i, _i, _i] + [_p] * 9 + [_i, _f, _i, _i, _i],
     "infllmv2_fwd_kvcache": [_p] * 11 + [_sz] + [_i] * 7 + [_p] * 6 + [_i, _i, _f, _p, _p, _p, _i64, _i, _p, _p, _i, _i],
     "infllmv2_fwd_kvcache_topk": [_p] * 10 + [_i, _p, _sz] + [_i] * 7 + [_p] * 6 + [_i, _f, _p, _p, _p, _i64, _i, _p, _p, _i, _i],
     "infllmv2_fwd_kvcache_scores": [_p] * 8 + [_i, _i, _p, _sz] + [_i] * 5 + [_p] * 4 + [_i, _f],
@@ -52,7 +53,7 @@ SIGNATURES = {
 PER_ELEMENT_TYPE = ["infllmv2_compress_keys", "infllmv2_compress_keys_pair", "infllmv2_compress_keys_cache", "infllmv2_compress_keys_cache_pair", "infllmv2_varlen_fwd_stage1",
                     "infllmv2_varlen_fwd_stage1_pooled", "infllmv2_stage1_decode", "infllmv2_decode_step_scores", "infllmv2_varlen_fwd",
                     "infllmv2_varlen_fwd_selected",
-                    "infllmv2_varlen_bwd", "infllmv2_fwd_kvcache", "infllmv2_fwd_kvcache_topk",
+                    "infllmv2_varlen_bwd", "infllmv2_varlen_bwd_selected", "infllmv2_fwd_kvcache", "infllmv2_fwd_kvcache_topk",
                     "infllmv2_fwd_kvcache_scores"]
 for _name in PER_ELEMENT_TYPE:
     SIGNATURES[_name + "_f16"] = SIGNATURES[_name]
@@ -62,6 +63,7 @@ OTHER = {
     "infllmv2_kv_image_bytes": (_sz, [_i64, _i, _i]),
     "infllmv2_varlen_fwd_dense_tiles": (_i, [_i, _i64, _i64] + [_i] * 5),
     "infllmv2_varlen_fwd_masked_tiles": (_i, [_i, _i64, _i64] + [_i] * 6),
+    "infllmv2_varlen_bwd_dq_tiles": (_i, [_i, _i64, _i64] + [_i] * 6),
     "infllmv2_stage1_decode_workspace_bytes": (_sz, [_i, _i, _i, _i]),
     "infllmv2_fwd_kvcache_workspace_bytes": (_sz, [_i, _i, _i]),
     "infllmv2_fwd_kvcache_num_splits": (_i, [_i, _i, _i]),

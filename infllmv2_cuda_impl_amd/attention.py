@@ -110,6 +110,7 @@ class Infllmv2AttnVarlenFunc(torch.autograd.Function):
         ctx.causal = causal
         ctx.deterministic = deterministic
         ctx.sparse = fwd_mask is not None
+        ctx.most_selected = topk_idx.shape[-1] if topk_idx is not None and topk_idx.dim() else 0    # a mask that came with its indices
         if not return_softmax:
             return out
         # S_dmask is only materialised with dropout, which this build rejects
@@ -122,7 +123,7 @@ class Infllmv2AttnVarlenFunc(torch.autograd.Function):
     def backward(ctx, dout, *args):
         q, k, v, out, lse, cu_seqlens_q, cu_seqlens_k, fwd_mask = ctx.saved_tensors
         dq, dk, dv = _lib.host.varlen_bwd(dout, q, k, v, out, lse, cu_seqlens_q, cu_seqlens_k, ctx.max_seqlen_q, ctx.max_seqlen_k,
-                                          ctx.softmax_scale, ctx.causal, fwd_mask, ctx.sparse, ctx.deterministic)
+                                          ctx.softmax_scale, ctx.causal, fwd_mask, ctx.sparse, ctx.deterministic, ctx.most_selected)
         return (dq, dk, dv) + (None,) * 15
 
 

@@ -430,10 +430,11 @@ std::tuple<Tensor, Tensor, OptTensor> varlen_fwd(const Tensor& q, const Tensor& 
     return {out, lse, mask};
 }
 
-// Returns (dq, dk, dv) with the shapes and dtype of (q, k, v)
+// Returns (dq, dk, dv) with the shapes and dtype of (q, k, v).  most_selected: blocks in a row of the mask at most, 0 where that is not known
 std::tuple<Tensor, Tensor, Tensor> varlen_bwd(const Tensor& dout_, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out,
                                               const Tensor& lse, const Tensor& cu_q, const Tensor& cu_k, int64_t max_q, int64_t max_k,
-                                              double scale, bool causal, const OptTensor& mask, bool lse_expanded, bool deterministic) {
+                                              double scale, bool causal, const OptTensor& mask, bool lse_expanded, bool deterministic,
+                                              int64_t most_selected) {
     const Tensor dout = dout_.stride(-1) == 1 ? dout_ : dout_.contiguous();
     TORCH_CHECK(dout.scalar_type() == q.scalar_type() && dout.sizes() == q.sizes(), "dout must have the shape and dtype of q");
     DeviceGuard guard(q.device());
@@ -444,12 +445,12 @@ std::tuple<Tensor, Tensor, Tensor> varlen_bwd(const Tensor& dout_, const Tensor&
     Tensor ws = bytes_on(q, size_query(as_int(batch), total_q, total_k, as_int(hk), as_int(max_k)));
     const S3 qs = grouped(q, group), os = grouped(out, group), dos = grouped(dout, group), dqs = grouped(dq, group);
     const S2 ks = rows_heads(k), vs = rows_heads(v), dks = rows_heads(dk), dvs = rows_heads(dv);
-    auto fn = is_half(q) ? infllmv2_varlen_bwd_f16 : infllmv2_varlen_bwd;
+    auto fn = is_half(q) ? infllmv2_varlen_bwd_selected_f16 : infllmv2_varlen_bwd_selected;
     check_rc(fn(stream_of(q), ptr(dout), ptr(q), ptr(k), ptr(v), ptr(out), static_cast<float*>(ptr(lse)), ptr(dq), ptr(dk), ptr(dv), iptr(cu_q),
                 iptr(cu_k), static_cast<const uint64_t*>(ptr(mask)), ptr(ws), static_cast<size_t>(ws.numel()), as_int(batch), total_q, total_k,
                 as_int(hq), as_int(hk), as_int(q.size(2)), as_int(max_q), as_int(max_k), qs.v, ks.v, vs.v, os.v, dos.v, dqs.v, dks.v, dvs.v,
-                lse_strides, mask.has_value() ? as_int(mask->size(-1)) : 0, static_cast<float>(scale), causal ? 1 : 0, deterministic ? 1 : 0),
-             "varlen_bwd");
+                lse_strides, mask.has_value() ? as_int(mask->size(-1)) : 0, static_cast<float>(scale), causal ? 1 : 0, deterministic ? 1 : 0,
+                as_int(most_selected)), "varlen_bwd");
     return {dq, dk, dv};
 }
 

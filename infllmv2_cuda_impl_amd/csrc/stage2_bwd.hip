@@ -23,7 +23,6 @@
 #include "stage2_bwd.h"
 #include "infllmv2_hip.h"
 #include <math.h>
-#include <stdlib.h>
 
 namespace IV2_NS {
 
@@ -146,7 +145,7 @@ extern "C" size_t infllmv2_varlen_bwd_deterministic_workspace_bytes(int batch, i
 
 #endif
 
-extern "C" int IV2_ENTRY(infllmv2_varlen_bwd)(void* stream, const void* dout, const void* q, const void* k, const void* v,
+extern "C" int IV2_ENTRY(infllmv2_varlen_bwd_selected)(void* stream, const void* dout, const void* q, const void* k, const void* v,
                                    const void* out, const float* softmax_lse, void* dq, void* dk, void* dv,
                                    const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
                                    const uint64_t* fwd_blockmask, void* workspace, size_t workspace_bytes, int batch,
@@ -155,7 +154,7 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_bwd)(void* stream, const void* dout, co
                                    const int64_t* k_strides, const int64_t* v_strides, const int64_t* o_strides,
                                    const int64_t* do_strides, const int64_t* dq_strides, const int64_t* dk_strides,
                                    const int64_t* dv_strides, const int64_t* lse_strides, int n_uint64_per_row,
-                                   float softmax_scale, int is_causal, int deterministic) {
+                                   float softmax_scale, int is_causal, int deterministic, int most_selected) {
     IV2_CHECK(head_dim == kHeadDim, "varlen_bwd: this build only supports head_dim 128 (got %d)", head_dim);
     IV2_CHECK(valid_group(num_heads, num_heads_k),
               "varlen_bwd: requires num_heads == g * num_heads_k with g in {1, 2, 4, 8, 16} (got %d and %d)", num_heads, num_heads_k);
@@ -259,7 +258,9 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_bwd)(void* stream, const void* dout, co
         IV2_LAUNCH_CHECK();
     }
     if (work) {
-        int rc = launch_bwd_dq_hybrid(st, p, batch, max_seqlen_q, is_causal != 0);
+        const bool tiles = dq_tiles_pay(batch, num_heads_k, p.group, total_q, total_k, max_seqlen_q, max_seqlen_k, is_causal != 0,
+                                        fwd_blockmask == nullptr ? 0x7fffffff : most_selected);
+        int rc = tiles ? launch_bwd_dq_tile(st, p, batch, max_seqlen_q, is_causal != 0) : launch_bwd_dq_hybrid(st, p, batch, max_seqlen_q, is_causal != 0);
         if (rc != 0) return rc;
         rc = launch_bwd_dkdv_wave(st, p, batch, max_seqlen_q, is_causal != 0);
         if (rc != 0) return rc;
@@ -277,4 +278,20 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_bwd)(void* stream, const void* dout, co
         IV2_LAUNCH_CHECK();
     }
     return 0;
+}
+
+extern "C" int IV2_ENTRY(infllmv2_varlen_bwd)(void* stream, const void* dout, const void* q, const void* k, const void* v,
+                                   const void* out, const float* softmax_lse, void* dq, void* dk, void* dv,
+                                   const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                                   const uint64_t* fwd_blockmask, void* workspace, size_t workspace_bytes, int batch,
+                                   int64_t total_q, int64_t total_k, int num_heads, int num_heads_k, int head_dim,
+                                   int max_seqlen_q, int max_seqlen_k, const int64_t* q_strides,
+                                   const int64_t* k_strides, const int64_t* v_strides, const int64_t* o_strides,
+                                   const int64_t* do_strides, const int64_t* dq_strides, const int64_t* dk_strides,
+                                   const int64_t* dv_strides, const int64_t* lse_strides, int n_uint64_per_row,
+                                   float softmax_scale, int is_causal, int deterministic) {
+    return IV2_ENTRY(infllmv2_varlen_bwd_selected)(stream, dout, q, k, v, out, softmax_lse, dq, dk, dv, cu_seqlens_q, cu_seqlens_k, fwd_blockmask, workspace,
+                                                   workspace_bytes, batch, total_q, total_k, num_heads, num_heads_k, head_dim, max_seqlen_q, max_seqlen_k,
+                                                   q_strides, k_strides, v_strides, o_strides, do_strides, dq_strides, dk_strides, dv_strides, lse_strides,
+                                                   n_uint64_per_row, softmax_scale, is_causal, deterministic, 0);
 }

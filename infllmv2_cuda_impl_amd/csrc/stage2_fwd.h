@@ -31,11 +31,6 @@ int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int 
                              int max_seqlen_k, bool causal, int most_selected, void* in_step);
 
 // Forward by tiles of 256 query rows (stage2_fwd_tile.hip), 64 per wavefront.  A token takes 16 rows, 8 in groups of 8.
-inline int tile_row_shift(int group) { return group == 8 ? 3 : 4; }
-inline int tiles_per_sequence(int group, int max_seqlen_q) {
-    const int tokens = 256 >> tile_row_shift(group);
-    return (max_seqlen_q + tokens - 1) / tokens;
-}
 bool dense_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal);
 bool masked_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal,
                       int most_selected);
