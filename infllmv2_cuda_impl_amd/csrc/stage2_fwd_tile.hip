@@ -429,8 +429,8 @@ bool dense_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int
 // nearly all it can see, in 1.4 us each; a group of 8 tokens takes 1.0 us for a block that all of them selected and up to 1.8 for those that its tokens
 // walk on their own.  So tiles win while the rows see up to about two and a half times what they select, and lose where the longest tile's chain decides
 // (one short prompt, one KV head).  The constants are a fit to 139 launches of 1 to 8 sequences of 130 to 25000 tokens, 16 to 64 blocks selected, 1 to 4
-// KV heads, groups of 8 and 16 (within 7 and 9 %); the choice costs 0.1 % of the better walk's time on average, 7 % in the worst, where the groups of 8 tokens alone
-// cost 24 %.  Operator in us, groups of 8 tokens | tiles (* the one taken here), 2 KV heads of 16 unless it says otherwise:
+// KV heads, groups of 8 and 16 (within 7 and 9 %); groups of 8 tokens alone cost 24 % of the better walk's time on average.  Near the line the estimate errs by a few
+// per cent (10612 tokens, 64 blocks selected, 2 heads: a tie by it, tiles 2 % slower): it asks for 8 % more than a tie, which leaves 0.5 % on the table.  Operator in us, groups of 8 tokens | tiles (* the one taken here), 2 KV heads of 16 unless it says otherwise:
 //   64 blocks selected: 3000 tokens 113 | 89 *, 8000 505 | 454 *, 12000 840 * | 960, 777 + 5003 + 1291 + 9173 883 | 815 *; 4 heads 4 x 4096 1396 | 1010 *
 //   16 blocks selected: 1000 tokens 31 * | 39, 2048 56 * | 62, 1023 + 3001 + 517 + 2200 151 | 145 *; 4 heads of 8 4000 182 | 128 *
 bool masked_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal,
@@ -443,7 +443,7 @@ bool masked_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, in
         const double beyond = b > most ? b - most : 0.;
         return 8. + (b < most ? b : most) + 0.4 * (beyond < most ? beyond : most);
     }, 0.3, batch, num_heads_k, total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
-    return tiles < groups;
+    return tiles < 0.92 * groups;
 }
 
 int launch_stage2_fwd_tile(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q, int max_seqlen_k, bool causal) {

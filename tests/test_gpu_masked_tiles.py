@@ -12,7 +12,7 @@ CASES = [  # query lengths, key lengths, KV heads, group, blocks selected, causa
     ([1025], [1025], 8, 16, 16, True),
     ([4500], [4500], 4, 16, 64, True),                        # two mask words
     ([700, 256], [2100, 900], 8, 16, 32, True),               # behind cached keys
-    ([1023], [1500], 8, 16, 16, False),
+    ([1023], [1500], 8, 8, 16, False),
     ([1500, 1], [1500, 1], 8, 4, 16, True),
 ]
 
