@@ -38,6 +38,7 @@ struct BwdParams {
     float* det_slots;               // (Hk, n_slots, det_slices, 2, 64, 128) fp32
     uint32_t* det_flags;            // (Hk, n_slots, det_slices): 1 where a slot was written
     int det_slices;
+    int dkdv_item;                  // tokens of an evenly dealt item at most, no fewer than a slice has
     int dkdv_share;                 // dK/dV work items: 1, 2, 4 or 8 XCDs share each group of slices
 };
 
@@ -48,7 +49,8 @@ bool dq_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_
                   int most_selected);
 int launch_bwd_dq_tile(hipStream_t st, const BwdParams& p, int batch, int max_seqlen_q, bool causal);
 // dK/dV, two wavefronts (32 keys each) per (64-key block, 512-token slice): stage2_bwd_dkdv.hip
-int launch_bwd_dkdv_wave(hipStream_t st, const BwdParams& p, int batch, int max_seqlen_q, bool causal);
+// most_selected: as in infllmv2_varlen_bwd_selected
+int launch_bwd_dkdv_wave(hipStream_t st, const BwdParams& p, int batch, int max_seqlen_q, int max_seqlen_k, bool causal, int most_selected);
 
 // deterministic mode only: adds the slots of every key block in slice order into dk_acc / dv_acc
 int launch_bwd_dkdv_reduce(hipStream_t st, const BwdParams& p, int batch);
@@ -57,6 +59,8 @@ int launch_bwd_dkdv_reduce(hipStream_t st, const BwdParams& p, int batch);
 // the device and the last of them are short (backward of 10 x 1500 tokens, 16 blocks selected: 844 against 968 us; of 16 x 3000:
 // 2160 / 2240; of 12000: 1640 / 1690; of 32768, 64 blocks: 8280 / 8170); the deterministic mode, whose workspace grows with the
 // slice count, keeps 512.
+// That is for inputs of more than kDkdvEvenGroups groups of 2048 tokens and for the deterministic mode: shorter ones deal a group's tokens out evenly.
+constexpr int kDkdvEvenGroups = 14;
 constexpr int kDkdvSlice = 512;
 constexpr int kDkdvSliceSmall = 128;
 inline int dkdv_slice_tokens(int max_seqlen_q, bool deterministic) {

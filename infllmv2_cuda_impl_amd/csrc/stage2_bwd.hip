@@ -262,7 +262,7 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_bwd_selected)(void* stream, const void*
                                         fwd_blockmask == nullptr ? 0x7fffffff : most_selected);
         int rc = tiles ? launch_bwd_dq_tile(st, p, batch, max_seqlen_q, is_causal != 0) : launch_bwd_dq_hybrid(st, p, batch, max_seqlen_q, is_causal != 0);
         if (rc != 0) return rc;
-        rc = launch_bwd_dkdv_wave(st, p, batch, max_seqlen_q, is_causal != 0);
+        rc = launch_bwd_dkdv_wave(st, p, batch, max_seqlen_q, max_seqlen_k, is_causal != 0, most_selected);
         if (rc != 0) return rc;
         if (deterministic) {
             rc = launch_bwd_dkdv_reduce(st, p, batch);

@@ -79,8 +79,22 @@ __device__ __forceinline__ short4v lds_read_tr(const unsigned char* ptr) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v*)(ptr));
 }
 
-// kColSlice: query tokens per work item (512, or 128 for short inputs)
-template <bool kCausal, int kColSlice>
+// the `count` lowest set bits of v (none for a negative count, all for a large one)
+__device__ __forceinline__ uint64_t lowest_set_bits(uint64_t v, int count) {
+    if (count <= 0) return 0ull;
+    int end = 0;                                               // the bits below it hold at most count set ones
+#pragma unroll
+    for (int step = 32; step > 0; step >>= 1) {
+        const int at = end + step;
+        end = __builtin_popcountll(v & ((1ull << at) - 1ull)) <= count ? at : end;
+    }
+    const uint64_t low = v & ((1ull << end) - 1ull);           // end <= 63: bit 63 is still to be looked at
+    return __builtin_popcountll(low) < count ? v : low;
+}
+
+// kColSlice: query tokens per slice.  kEven: the tokens of a group that selected a block are dealt out evenly; else a slice is a work item, light ones
+// are merged.
+template <bool kCausal, int kColSlice, bool kEven>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_dkdv_wave_kernel(const BwdParams p) {
     constexpr int kSliceWords = kColSlice / 64;                // mask words per slice (a power of two)
@@ -139,7 +153,15 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
     }
     if (t_lo >= t_hi) return;                                  // uniform
 
-    // ---- light slices are merged ----
+    // ---- items ----
+    // Dealt out evenly (kEven): as few items as hold at most p.dkdv_item tokens each, all of one size to a token, because the longest items of a short input
+    // decide the kernel's time.  Item i goes to the i-th slice of the group that touches the sequence; there are enough of those, because an
+    // item may hold a slice's worth of tokens.  Merged (below), items are slices, and what walks the same slice at the same time shares its q and dout in L2: that
+    // counts for more where there are many rounds of items anyway.  Whole backward in us, merged | even (* the one taken), 2 KV heads: 2048 tokens, 16 blocks selected
+    // 203 | 169 *, 1023 + 3001 + 517 + 2200, 16 blocks 490 | 429 *, 16000, 64 blocks 3790 | 3590 *, 24000, 32 blocks 3570 | 3400 *, 3 x 8000, 64 blocks 4720 | 4410 *;
+    // 7 x 8000 10690 * | 10640, 20 x 3000 5193 * | 5213, 71552 in four sequences 16500 * | 17100.  (A list of the items, so that no workgroup is empty, cost more than
+    // the empty ones: 2048 tokens 184, 24000 tokens 3490.)
+    //
     // A flush costs 16384 fp32 atomics whatever the slice held, so a slice works on its own only if at least
     // kHeavyPairs of its tokens selected the block; the other slices of the same group are put together, about
     // kItemTokens tokens to an item, and the first slice of an item collects.  (All of a group in one item: up to 465 tokens
@@ -162,32 +184,47 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
             }
         }
         int cnt = __builtin_popcountll(wv);
+        if constexpr (kEven) {
+            int upto = cnt;                                    // tokens in the words up to this one
 #pragma unroll
-        for (int off = 1; off < kSliceWords; off <<= 1) cnt += __shfl_xor(cnt, off);   // tokens of this lane's slice that selected the block
-        const uint64_t heavy = __ballot(cnt >= kHeavyPairs);   // kSliceWords equal bits per slice
-        const uint64_t filled = __ballot(cnt > 0);
-        bool keep;
-        if ((heavy >> (kSliceWords * sub)) & 1ull) {
-            keep = (lane / kSliceWords) == sub;
-        } else {
-            uint64_t mates = filled & ~heavy;
-            if (!((mates >> (kSliceWords * sub)) & 1ull)) return;                   // uniform: empty
-            if constexpr ((kGroupSlices - 1) * (kHeavyPairs - 1) > kItemTokens) {
-                // dealt out by how many tokens the light slices before them hold
-                const int own = (mates >> lane) & 1ull ? cnt : 0;                   // every lane of a slice holds the slice's count
-                int upto = own;
-#pragma unroll
-                for (int off = kSliceWords; off < kGroupWords; off <<= 1) {
-                    const int up = __shfl_up(upto, off);
-                    upto += lane >= off ? up : 0;
-                }
-                const int item = (upto - own) / kItemTokens;
-                mates &= __ballot(lane < kGroupWords && item == __builtin_amdgcn_readlane(item, kSliceWords * sub));
+            for (int off = 1; off < kGroupWords; off <<= 1) {
+                const int up = __shfl_up(upto, off);
+                upto += lane >= off ? up : 0;
             }
-            if (__builtin_ctzll(mates) / kSliceWords != sub) return;                // uniform: another slice collects
-            keep = (mates >> lane) & 1ull;
+            const int total = __builtin_amdgcn_readlane(upto, kGroupWords - 1), items = (total + p.dkdv_item - 1) / p.dkdv_item;
+            const int first_slice = q0 / kColSlice - group * kGroupSlices, item = sub - (first_slice > 0 ? first_slice : 0);
+            if (item >= items) return;                         // uniform
+            const int each = (total + items - 1) / items, from = item * each - (upto - cnt);
+            wv = lowest_set_bits(wv, from + each) & ~lowest_set_bits(wv, from);
+            if (lane < kGroupWords) wbuf[lane] = wv;
+        } else {
+#pragma unroll
+            for (int off = 1; off < kSliceWords; off <<= 1) cnt += __shfl_xor(cnt, off);   // tokens of this lane's slice that selected the block
+            const uint64_t heavy = __ballot(cnt >= kHeavyPairs);   // kSliceWords equal bits per slice
+            const uint64_t filled = __ballot(cnt > 0);
+            bool keep;
+            if ((heavy >> (kSliceWords * sub)) & 1ull) {
+                keep = (lane / kSliceWords) == sub;
+            } else {
+                uint64_t mates = filled & ~heavy;
+                if (!((mates >> (kSliceWords * sub)) & 1ull)) return;                   // uniform: empty
+                if constexpr ((kGroupSlices - 1) * (kHeavyPairs - 1) > kItemTokens) {
+                    // dealt out by how many tokens the light slices before them hold
+                    const int own = (mates >> lane) & 1ull ? cnt : 0;                   // every lane of a slice holds the slice's count
+                    int upto = own;
+#pragma unroll
+                    for (int off = kSliceWords; off < kGroupWords; off <<= 1) {
+                        const int up = __shfl_up(upto, off);
+                        upto += lane >= off ? up : 0;
+                    }
+                    const int item = (upto - own) / kItemTokens;
+                    mates &= __ballot(lane < kGroupWords && item == __builtin_amdgcn_readlane(item, kSliceWords * sub));
+                }
+                if (__builtin_ctzll(mates) / kSliceWords != sub) return;                // uniform: another slice collects
+                keep = (mates >> lane) & 1ull;
+            }
+            if (lane < kGroupWords) wbuf[lane] = keep ? wv : 0ull;
         }
-        if (lane < kGroupWords) wbuf[lane] = keep ? wv : 0ull;
     }
     __syncthreads();
 
@@ -537,9 +574,27 @@ int launch_bwd_dkdv_reduce(hipStream_t st, const BwdParams& p, int batch) {
     return 0;
 }
 
-template <int kColSlice>
-static int launch_bwd_dkdv_sliced(hipStream_t st, const BwdParams& p_in, int batch, int max_seqlen_q, bool causal) {
+// How many pairs of a query token and a key block a mask selects whose rows have at most `most` blocks (not known: 0, taken as all they see).
+static double selected_pairs(int batch, int num_heads_k, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal, int most) {
+    auto of = [&](double q, double k) {                        // of a sequence
+        const double first = causal ? (k > q ? k - q : 0.) : k;
+        double sum = 0.;
+        for (int i = 0; i < 16; ++i) {
+            const double seen = (first + (k - first) * (i + 0.5) / 16) / kBlockN + 0.5;
+            sum += most > 0 && seen > most ? most : seen;
+        }
+        return q * sum / 16;
+    };
+    const int others = batch - 1;
+    const double q = others > 0 && total_q > max_seqlen_q ? static_cast<double>(total_q - max_seqlen_q) / others : 0.;
+    const double k = others > 0 && total_k > max_seqlen_k ? static_cast<double>(total_k - max_seqlen_k) / others : 0.;
+    return num_heads_k * (of(max_seqlen_q, max_seqlen_k) + others * of(q, k));
+}
+
+template <int kColSlice, bool kEven>
+static int launch_bwd_dkdv_sliced(hipStream_t st, const BwdParams& p_in, int batch, int max_seqlen_q, bool causal, int item_tokens) {
     BwdParams p = p_in;
+    p.dkdv_item = item_tokens;
     constexpr int kGroupSlices = kGroupWords * 64 / kColSlice;
     // a sequence of max_seqlen_q tokens touches at most `groups` consecutive slice groups wherever it starts
     const int group_tokens = kGroupWords * 64;
@@ -571,15 +626,30 @@ static int launch_bwd_dkdv_sliced(hipStream_t st, const BwdParams& p_in, int bat
               "varlen_bwd: token strides of q and dout must lie in [0, 2^31) elements");
     const dim3 grid(static_cast<unsigned>(items), batch, p.num_heads_k);
     const size_t lds = kWaveLds + kGroupWords * 8;
-    if (causal) hipLaunchKernelGGL((bwd_dkdv_wave_kernel<true, kColSlice>), grid, dim3(128), lds, st, p);
-    else hipLaunchKernelGGL((bwd_dkdv_wave_kernel<false, kColSlice>), grid, dim3(128), lds, st, p);
+    if (causal) hipLaunchKernelGGL((bwd_dkdv_wave_kernel<true, kColSlice, kEven>), grid, dim3(128), lds, st, p);
+    else hipLaunchKernelGGL((bwd_dkdv_wave_kernel<false, kColSlice, kEven>), grid, dim3(128), lds, st, p);
     IV2_LAUNCH_CHECK();
     return 0;
 }
 
-int launch_bwd_dkdv_wave(hipStream_t st, const BwdParams& p, int batch, int max_seqlen_q, bool causal) {
-    if (dkdv_slice_tokens(max_seqlen_q, p.det_slots != nullptr) == kDkdvSliceSmall) return launch_bwd_dkdv_sliced<kDkdvSliceSmall>(st, p, batch, max_seqlen_q, causal);
-    return launch_bwd_dkdv_sliced<kDkdvSlice>(st, p, batch, max_seqlen_q, causal);
+int launch_bwd_dkdv_wave(hipStream_t st, const BwdParams& p, int batch, int max_seqlen_q, int max_seqlen_k, bool causal, int most_selected) {
+    const int64_t groups = (p.total_q + kGroupWords * 64 - 1) / (kGroupWords * 64);
+    if (p.det_slots == nullptr && groups <= kDkdvEvenGroups) {
+        // How many tokens to an item.  Where all items can run at once the kernel is fastest with about 600 of them, three to a CU at most: a fourth on some CUs adds
+        // 40 us.  So `fit` tokens, 64 at least (a flush costs what 10 tokens do) and 192 at most; past that several rounds of 128, which balance better, and for still
+        // more pairs fewer flushes.  Whole backward in us with 64 / 80 / 96 / 112 / 128 / 160 / 192 / 256 tokens, 2 KV heads, 16 blocks selected unless said: 1000 tokens 107 /
+        // 112 / 118 / 130 / 124 / 140 / 159 / 194, 2048 202 / 169 / 174 / 183 / 190 / 210 / 230 / 273, 3000 265 / 271 / 276 / 269 / 230 / 249 / 270 / 314, 4000 362 / 322 /
+        // 331 / 355 / 365 / 371 / 316 / 356, 1023 + 3001 + 517 + 2200 507 / 468 / 459 / 461 / 429 / 465 / 485 / 505, 12000 1037 / 1016 / 976 / 956 / 937 / 935 / 934 / 969, 6 x
+        // 3000 (32 blocks) 1693 / 1652 / 1638 / 1620 / 1608 / 1588 / 1584 / 1608, 24000 (32 blocks) 3710 / 3597 / 3569 / 3550 / 3477 / 3479 / 3382 / 3476.
+        const double pairs = selected_pairs(batch, p.num_heads_k, p.total_q, p.total_k, max_seqlen_q, max_seqlen_k, causal, most_selected);
+        const double fit = pairs / 600., many = pairs / 6300.;
+        if (fit < 128.) return launch_bwd_dkdv_sliced<64, true>(st, p, batch, max_seqlen_q, causal, fit > 64. ? static_cast<int>(fit) : 64);
+        const int item = fit <= 192. ? static_cast<int>(fit) : many <= 128. ? 128 : many < 256. ? static_cast<int>(many) : 256;
+        return launch_bwd_dkdv_sliced<kDkdvSliceSmall, true>(st, p, batch, max_seqlen_q, causal, item);
+    }
+    if (dkdv_slice_tokens(max_seqlen_q, p.det_slots != nullptr) == kDkdvSliceSmall)
+        return launch_bwd_dkdv_sliced<kDkdvSliceSmall, false>(st, p, batch, max_seqlen_q, causal, 0);
+    return launch_bwd_dkdv_sliced<kDkdvSlice, false>(st, p, batch, max_seqlen_q, causal, 0);
 }
 
 }  // namespace IV2_NS
