@@ -3,16 +3,16 @@
 // Past some length the block images of one KV head exceed an XCD's 4 MiB of L2 many times over, and what a token walks on its own is
 // fetched from the fabric behind it.  Every row is walked in ascending order at the same pace, so workgroups that start
 // together pass a key block at about the same time and share its fetch; started whenever a CU becomes free, they are spread
-// over the whole sequence.  A workgroup therefore sets itself up and then waits until those of its XCD that belong to earlier
-// generations (a generation is what an XCD runs at once: a workgroup on each of its 32 CUs) have finished their walks.
+// over the whole sequence.  A wavefront therefore sets itself up and then waits until the workgroups of its XCD that belong to earlier
+// generations (a generation is what an XCD runs at once: a workgroup on each of its 32 CUs) have finished their walks, by their first wavefronts' word.
 //
 // The wait is a matter of speed only: nothing depends on which workgroups run at once, a workgroup of an earlier generation never
 // waits for a later one, and a wait ends after kInStepPolls looks whatever the counters hold.
 //
 // Which launches: at 30 000 tokens a whole prefill gained 1 % and at 32 768 it gained or lost less (L2 serves 91 % of the requests
 // there and the wait for a generation's slowest workgroup costs 2 %); at 40 000 it gained 7 %, at 49 152 14, at 65 536 22 (10.9 -> 8.5 ms,
-// two KV heads), at 98 304 20, at 131 072 17 (31.3 -> 25.9).  Only workgroups whose rows have blocks of their own in
-// several mask words wait: with window masks everything is shared, and waiting cost 2 %.  Letting up to 8 workgroups of a
+// two KV heads), at 98 304 20, at 131 072 17 (31.3 -> 25.9).  Only wavefronts whose row has blocks of its own in
+// several mask words wait: with window masks everything is shared (60 000 tokens, 6 blocks: 473 us without all this, 478 with the counters and no waits).  Letting up to 8 workgroups of a
 // generation start early gave back a quarter of the gain; more meeting points during the walk, or walking every other
 // generation downwards, gave nothing more.  The dQ kernel walks the same way but is not bound by its fetches: waiting cost it 2 %
 // of its time at 40 000 tokens and gained nothing at 64 000.
@@ -28,19 +28,16 @@ constexpr int kInStepPolls = 256;                              // of about a mic
 constexpr int kInStepPitch = 32;                               // the XCDs' counters lie 128 bytes apart
 constexpr size_t kInStepBytes = 8 * kInStepPitch * sizeof(unsigned);
 
-// counter: of the workgroup's XCD, how many wavefronts have finished their walk; order: the workgroup's number on its XCD
-__device__ __forceinline__ void in_step_finished(unsigned* counter, unsigned wavefronts) {
-    __hip_atomic_fetch_add(counter, wavefronts, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// counter: of the workgroup's XCD, how many workgroups have finished their walk; order: the workgroup's number on its XCD
+__device__ __forceinline__ void in_step_finished(unsigned* counter) {
+    __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void in_step_wait(const unsigned* counter, int order, int wavefronts_per_workgroup) {
-    const unsigned before = static_cast<unsigned>(order / kGeneration) * static_cast<unsigned>(kGeneration * wavefronts_per_workgroup);
+__device__ __forceinline__ void in_step_wait(const unsigned* counter, int order) {
+    const unsigned before = static_cast<unsigned>(order / kGeneration) * static_cast<unsigned>(kGeneration);
     for (int poll = 0; poll < kInStepPolls; ++poll) {
         if (__hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= before) return;
         __builtin_amdgcn_s_sleep(4);
     }
 }
-
-static __global__ __launch_bounds__(8 * kInStepPitch)
-void in_step_clear_kernel(unsigned* counters) { counters[threadIdx.x] = 0u; }
 
 }  // namespace IV2_NS

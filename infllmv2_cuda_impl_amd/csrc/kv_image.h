@@ -52,9 +52,9 @@ __device__ __forceinline__ void write_k_image(const elem_bits* rows, int64_t row
 // What the images ask of k and v.
 int check_pack(const void* k, const void* v, const int32_t* cu_seqlens_k, const void* workspace, size_t workspace_bytes, int batch,
                int64_t total_k, int num_heads_k, int max_seqlen_k, const int64_t* k_strides, const int64_t* v_strides);
-// Launches the packing pre-pass.  workspace receives [K image | V image].
+// Launches the packing pre-pass.  workspace receives [K image | V image].  in_step: counters of in_step.h to clear, or null.
 int launch_pack(hipStream_t st, const void* k, const void* v, const int32_t* cu_seqlens_k, void* workspace,
                 size_t workspace_bytes, int batch, int64_t total_k, int num_heads_k, int max_seqlen_k,
-                const int64_t* k_strides, const int64_t* v_strides);
+                const int64_t* k_strides, const int64_t* v_strides, unsigned* in_step = nullptr);
 
 }  // namespace IV2_NS

@@ -28,7 +28,7 @@ struct FwdParams {
 // alone (the counters by which workgroups walk long sequences in step), or null.  most_selected: as in infllmv2_varlen_fwd_selected.  Goes by
 // tiles where that is the faster walk.
 int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q,
-                             int max_seqlen_k, bool causal, int most_selected, void* in_step);
+                             int max_seqlen_k, bool causal, int most_selected, unsigned* in_step);
 
 // Forward by tiles of 256 query rows (stage2_fwd_tile.hip), 64 per wavefront.  A token takes 16 rows, 8 in groups of 8.
 bool dense_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal);

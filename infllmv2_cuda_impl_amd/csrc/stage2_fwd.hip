@@ -35,7 +35,9 @@ struct PackParams {
     int64_t k_row_stride, k_head_stride;
     int64_t v_row_stride, v_head_stride;
     int64_t n_slots;
+    unsigned* in_step;              // counters of in_step.h to clear for the launch that walks the images, or null (a launch of its own took 10 us)
 };
+static_assert(8 * kInStepPitch == 256, "one counter word per thread of a packing workgroup");
 
 constexpr int kVPad = 8;            // LDS row padding (elements) for the V transposition
 
@@ -43,6 +45,7 @@ __global__ __launch_bounds__(256)
 void pack_kv_kernel(const PackParams p) {
     __shared__ __attribute__((aligned(16))) elem_bits vt[kBlockN][kHeadDim + kVPad];
     const int j = blockIdx.x, b = blockIdx.y, h = blockIdx.z;
+    if (p.in_step != nullptr && j + b + h == 0) p.in_step[threadIdx.x] = 0u;
     const int k0 = p.cu_seqlens_k[b];
     const int Sk = p.cu_seqlens_k[b + 1] - k0;
     if (static_cast<int64_t>(j) * kBlockN >= Sk) return;
@@ -105,7 +108,7 @@ int check_pack(const void* k, const void* v, const int32_t* cu_seqlens_k, const 
 }
 int launch_pack(hipStream_t st, const void* k, const void* v, const int32_t* cu_seqlens_k, void* workspace,
                 size_t workspace_bytes, int batch, int64_t total_k, int num_heads_k, int max_seqlen_k,
-                const int64_t* k_strides, const int64_t* v_strides) {
+                const int64_t* k_strides, const int64_t* v_strides, unsigned* in_step) {
     const int rc = check_pack(k, v, cu_seqlens_k, workspace, workspace_bytes, batch, total_k, num_heads_k, max_seqlen_k, k_strides, v_strides);
     if (rc != 0) return rc;
     const int64_t n_slots = image_slots(total_k, batch);
@@ -120,6 +123,7 @@ int launch_pack(hipStream_t st, const void* k, const void* v, const int32_t* cu_
     pp.k_row_stride = k_strides[0]; pp.k_head_stride = k_strides[1];
     pp.v_row_stride = v_strides[0]; pp.v_head_stride = v_strides[1];
     pp.n_slots = n_slots;
+    pp.in_step = in_step;
     hipLaunchKernelGGL(pack_kv_kernel, dim3(max_blocks, batch, num_heads_k), dim3(256), 0, st, pp);
     IV2_LAUNCH_CHECK();
     return 0;
@@ -161,9 +165,13 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_fwd_selected)(void* stream, const void*
     IV2_CHECK(softmax_scale > 0.f, "varlen_fwd: softmax_scale must be positive");
     if (total_q == 0 || max_seqlen_q == 0) return 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    // Images packed by an earlier call may be read by several launches at once: those leave the workspace as it is.
+    const size_t images = image_bytes(total_k, batch, num_heads_k);
+    unsigned* in_step = kv_prepacked || workspace_bytes < images + kInStepBytes || max_seqlen_k <= kInStepKeys || total_k == 0 || blockmask == nullptr
+                            ? nullptr : reinterpret_cast<unsigned*>(static_cast<unsigned char*>(workspace) + images);
     if (!kv_prepacked) {
         int rc = launch_pack(st, k, v, cu_seqlens_k, workspace, workspace_bytes, batch, total_k, num_heads_k,
-                             max_seqlen_k, k_strides, v_strides);
+                             max_seqlen_k, k_strides, v_strides, in_step);
         if (rc != 0) return rc;
     }
     const int64_t n_slots = image_slots(total_k, batch);
@@ -183,9 +191,6 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_fwd_selected)(void* stream, const void*
     fp.group = num_heads / num_heads_k;
     fp.n64 = n_uint64_per_row;
     fp.scale_log2 = softmax_scale * 1.44269504088896340736f;
-    // Images packed by an earlier call may be read by several launches at once: those leave the workspace as it is.
-    const size_t images = image_bytes(total_k, batch, num_heads_k);
-    void* in_step = kv_prepacked || workspace_bytes < images + kInStepBytes ? nullptr : static_cast<unsigned char*>(workspace) + images;
     return launch_stage2_fwd_hybrid(st, fp, batch, num_heads_k, max_seqlen_q, max_seqlen_k, is_causal != 0, most_selected, in_step);
 }
 

@@ -115,7 +115,9 @@ __device__ __forceinline__ void softmax_step(floatx4 (&s)[4], float& m, float& l
         }
 }
 
-template <bool kCausal>
+// kInStep: with the counters of in_step.h; a variant of its own, because a workgroup has its CU to itself and pays for all set-up (the counting alone took
+// 2.6 % where rows are short: 30000 tokens with a window of 9 blocks 536 -> 550 us)
+template <bool kCausal, bool kInStep>
 __global__ __launch_bounds__(512)
 void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -140,12 +142,14 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     const int q0 = p.cu_seqlens_q[b];
     const int Sq = p.cu_seqlens_q[b + 1] - q0;
     const int i0 = grp * kHybTokens;
-    unsigned* finished = x.finished ? x.finished + xcd * kInStepPitch : nullptr;
+    const int Sk = p.cu_seqlens_k[b + 1] - p.cu_seqlens_k[b];
+    const int64_t slot0 = static_cast<int64_t>(h) * p.n_slots + image_slot0(p.cu_seqlens_k, b);
+    // (All of these are read before the first atomic: behind it the compiler loads them into vector registers, 0.5 us per workgroup.)
+    unsigned* finished = x.finished + xcd * kInStepPitch;
     if (i0 >= Sq) {                                                                 // uniform per workgroup
-        if (finished && tid == 0) in_step_finished(finished, kHybTokens);
+        if (kInStep && tid == 0) in_step_finished(finished);
         return;
     }
-    const int Sk = p.cu_seqlens_k[b + 1] - p.cu_seqlens_k[b];
 
     // A group at the end of a sequence that has four tokens or fewer: 2, 4 or 8 wavefronts share a token's blocks (every so-manyth column
     // of its mask row each) and merge at the end.  With one wavefront per token such a group took as long as a full one, and where a
@@ -191,11 +195,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     __syncthreads();
     const uint64_t columns = (share_log2 == 0 ? ~0ull : share_log2 == 1 ? 0x5555555555555555ull
                               : share_log2 == 2 ? 0x1111111111111111ull : 0x0101010101010101ull) << part;
-    int own_words = 0;                                                              // lanes: words with blocks of this row's own
-    for (int w = lane; w < nw; w += 64) {
-        own[w] &= ~com[w] & columns;
-        own_words += __builtin_popcountll(__builtin_amdgcn_ballot_w64(own[w] != 0ull));
-    }
+    for (int w = lane; w < nw; w += 64) own[w] &= ~com[w] & columns;
 
     // ---- Q operand ----
     elem8 qf[4];
@@ -209,8 +209,6 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     floatx4 o[8];
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-    const int64_t slot0 = static_cast<int64_t>(h) * p.n_slots + image_slot0(p.cu_seqlens_k, b);
 
     // ---- the walk: one turn = two common blocks (lock step, operands from the LDS ring) alternating with two own
     //      blocks (operands from global memory into registers).  The own blocks' loads keep the vector memory path
@@ -248,9 +246,12 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
 #pragma unroll
         for (int f = 0; f < 16; ++f) kreg[f] = *reinterpret_cast<const elem8*>(src + f * 512);
     }
-    if (finished) {
-        if (tid == 0 && Sk > kInStepKeys && own_words >= kInStepWords) in_step_wait(finished, sidx, kHybTokens);   // lane 0 took part in every round of the count
-        __syncthreads();
+    if constexpr (kInStep) {
+        if (Sk > kInStepKeys) {                                // uniform
+            int words = 0;                                     // with blocks of this row's own
+            for (int w = 0; w < nw; w += 64) words += __builtin_popcountll(__builtin_amdgcn_ballot_w64(w + lane < nw && own[w + lane] != 0ull));
+            if (words >= kInStepWords) in_step_wait(finished, sidx);
+        }
     }
     // All ordinary loads so far (Q, mask words, first K fragments) land before the first LDS-DMA.  From here on the
     // compiler's wait counts know nothing of the DMA loads; they stay correct because loads complete in order (an
@@ -353,7 +354,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
             half ^= 1;
         }
     }
-    if (finished && lane == 0) in_step_finished(finished, 1u);
+    if (kInStep && tid == 0) in_step_finished(finished);       // the first wavefront for its workgroup: its row is one of eight neighbours
     if (share_log2 != 0) {                                     // uniform per workgroup
         // the ring was not used: 34 floats of every lane, lane by lane
         float* mine = reinterpret_cast<float*>(smem_raw) + wave * (34 * 64) + lane;
@@ -399,7 +400,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
 }
 
 int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q,
-                             int max_seqlen_k, bool causal, int most_selected, void* in_step) {
+                             int max_seqlen_k, bool causal, int most_selected, unsigned* in_step) {
     HybridExtra x{};
     x.batch = batch;
     x.groups_per_seq = (max_seqlen_q + kHybTokens - 1) / kHybTokens;
@@ -416,17 +417,13 @@ int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int 
     const int64_t per_round = 8 * kHybChunk;
     const int64_t grid = (total + per_round - 1) / per_round * per_round;
     const size_t lds = kRingTiles * kTileBytes + static_cast<size_t>(1 + kHybTokens) * x.mask_words * 8;
-    const void* fn = causal ? reinterpret_cast<const void*>(&stage2_fwd_hybrid_kernel<true>)
-                            : reinterpret_cast<const void*>(&stage2_fwd_hybrid_kernel<false>);
-    if (in_step != nullptr && p.mask != nullptr && max_seqlen_k > kInStepKeys) {
-        x.finished = static_cast<unsigned*>(in_step);
-        hipLaunchKernelGGL(in_step_clear_kernel, dim3(1), dim3(8 * kInStepPitch), 0, st, x.finished);
-        IV2_LAUNCH_CHECK();
-    }
-    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+    const bool wait = in_step != nullptr;
+    auto kernel = causal ? (wait ? stage2_fwd_hybrid_kernel<true, true> : stage2_fwd_hybrid_kernel<true, false>)
+                         : (wait ? stage2_fwd_hybrid_kernel<false, true> : stage2_fwd_hybrid_kernel<false, false>);
+    x.finished = in_step;
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     IV2_CHECK(e == hipSuccess, "varlen_fwd: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
-    if (causal) hipLaunchKernelGGL(stage2_fwd_hybrid_kernel<true>, dim3(static_cast<unsigned>(grid)), dim3(512), lds, st, p, x);
-    else hipLaunchKernelGGL(stage2_fwd_hybrid_kernel<false>, dim3(static_cast<unsigned>(grid)), dim3(512), lds, st, p, x);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(512), lds, st, p, x);
     IV2_LAUNCH_CHECK();
     return 0;
 }
