@@ -121,6 +121,12 @@ int infllmv2_topk_select(void* stream, const void* pooled, int64_t row_stride, i
                          uint64_t* mask_words, int64_t rows, int n, int k, int n_uint64_per_row, int by_index,
                          int drop_neg_inf);
 
+/* The blocks of a window as a selection: of a query at position p of its sequence (cache_lens tokens before its first query, null: none), blocks [0, init_blocks) and
+ * p / block_size - local_blocks to p / block_size, those below n_blocks: what max_pooling_1d_varlen marks +inf.  topk_idx (num_heads, rows,
+ * init_blocks + local_blocks + 1) ascending, then -1; mask_words (num_heads, rows, n_uint64_per_row). */
+int infllmv2_window_blocks(void* stream, int32_t* topk_idx, uint64_t* mask_words, const int* cu_seqlens_q, const int* cache_lens, int batch, int num_heads,
+                           int64_t rows, int n_blocks, int n_uint64_per_row, int block_size, int local_blocks, int init_blocks);
+
 /* ---- Compressed keys (caller-side in the reference) ----------------------------------------- */
 
 /* The Stage-1 inputs are means of K over sliding windows; the reference leaves their construction to its callers,

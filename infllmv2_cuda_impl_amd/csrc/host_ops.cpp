@@ -346,6 +346,24 @@ std::tuple<Tensor, OptTensor> topk_blocks(const Tensor& pooled, int64_t k, bool 
     return {idx, mask};
 }
 
+std::tuple<Tensor, Tensor> window_blocks(int64_t heads, int64_t rows, const Tensor& cu_q_, const OptTensor& positions_, int64_t max_q, int64_t max_position,
+                                         int64_t local_blocks, int64_t init_blocks, int64_t block_size) {
+    require_gpu(cu_q_, "cu_seqlens_q");
+    const Tensor cu_q = cu_q_.contiguous();
+    OptTensor positions;
+    if (positions_.has_value()) positions = positions_->contiguous();
+    TORCH_CHECK(cu_q.scalar_type() == at::kInt && (!positions.has_value() || (positions->scalar_type() == at::kInt && positions->size(0) == cu_q.size(0) - 1)),
+                "window_blocks: int32 sequence starts and positions of as many sequences");
+    const int64_t n = (max_q + max_position + block_size - 1) / block_size, n64 = (n + 63) / 64;
+    DeviceGuard guard(cu_q.device());
+    Tensor idx = at::empty({heads, rows, init_blocks + local_blocks + 1}, cu_q.options());
+    Tensor mask = at::empty({heads, rows, n64}, cu_q.options().dtype(at::kLong));
+    check_rc(infllmv2_window_blocks(stream_of(cu_q), static_cast<int32_t*>(ptr(idx)), static_cast<uint64_t*>(mask.data_ptr()), iptr(cu_q),
+                                    positions.has_value() ? iptr(*positions) : nullptr, as_int(cu_q.size(0) - 1), as_int(heads), rows, as_int(n), as_int(n64), as_int(block_size), as_int(local_blocks),
+                                    as_int(init_blocks)), "window_blocks");
+    return {idx, mask};
+}
+
 Tensor topk_to_uint64(const Tensor& topk_idx, int64_t k_blocks, const OptTensor& buffer) {
     require_gpu(topk_idx, "topk_idx");
     const Tensor idx = topk_idx.contiguous();
@@ -700,6 +718,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("max_pooling_1d", &max_pooling_1d);
     m.def("max_pooling_1d_varlen", &max_pooling_1d_varlen);
     m.def("topk_blocks", &topk_blocks);
+    m.def("window_blocks", &window_blocks);
     m.def("topk_to_uint64", &topk_to_uint64);
     m.def("select_blocks", &select_blocks);
     m.def("varlen_fwd", &varlen_fwd);

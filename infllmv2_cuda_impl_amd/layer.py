@@ -26,8 +26,7 @@ import torch
 
 from . import _lib
 from .attention import HEAD_DIM, infllmv2_attn_varlen_func, infllmv2_attn_with_kvcache, pad_head_dim
-from .pooling import max_pooling_1d_varlen
-from .selection import compress_keys, compress_keys_cache, topk_blocks
+from .selection import compress_keys, compress_keys_cache
 
 
 @dataclass
@@ -91,29 +90,20 @@ class InfLLMv2Attention(torch.nn.Module):
         self.kernel_size, self.stride, self.block_size = kernel_size, stride, block_size
         self.softmax_scale = softmax_scale
 
-    def _window_blocks(self, nheads_k: int, rows: int, cu_seqlens_q, positions, max_seqlen_q: int, max_position: int,
-                       device):
-        """The forced blocks alone as a selection: what the pooling operator marks +inf on a score tensor with no
-        columns, with every other block dropped.  ``rows``: packed query tokens; ``positions`` int32 (batch): tokens before each
-        sequence's first query.  Returns ``(topk_idx, block_mask)`` with ``init_blocks + local_blocks + 1`` index slots."""
-        batch = cu_seqlens_q.numel() - 1
-        empty = torch.empty((nheads_k, rows, 0), dtype=torch.bfloat16, device=device)  # pooled scores: any 16-bit type
-        no_keys = torch.zeros(batch + 1, dtype=torch.int32, device=device)
-        pooled = max_pooling_1d_varlen(empty, cu_seqlens_q, no_keys, positions, max_seqlen_q, 0, self.local_blocks,
-                                       self.init_blocks, block_size=self.block_size, stride=self.stride,
-                                       max_cache_len=max_position)
-        return topk_blocks(pooled, self.init_blocks + self.local_blocks + 1, return_mask=True, by_index=True,
-                           drop_unreachable=True)
+    def _window_blocks(self, nheads_k: int, rows: int, cu_seqlens_q, positions, max_seqlen_q: int, max_position: int):
+        """The forced blocks alone as a selection: what the pooling operator marks +inf, with every other block
+        dropped.  ``rows``: packed query tokens; ``positions`` int32 (batch) or None: tokens before each sequence's
+        first query.  Returns ``(topk_idx, block_mask)`` with ``init_blocks + local_blocks + 1`` index slots."""
+        return _lib.host.window_blocks(nheads_k, rows, cu_seqlens_q, positions, max_seqlen_q, max_position, self.local_blocks,
+                                       self.init_blocks, self.block_size)
 
     # ---- prefill / training ----
     def forward(self, q, k, v, cu_seqlens, max_seqlen: int, cache: SequenceCache | None = None):
         """q ``(total, nheads, d)``, k/v ``(total, nheads_k, d)`` packed; returns ``(total, nheads, d)``.
         With ``cache`` (one sequence only) the keys, values and compressed keys are also stored for decoding."""
         topk_idx = mask = None
-        batch = cu_seqlens.numel() - 1
         if self.selection == "window" and max_seqlen > self.dense_len:
-            topk_idx, mask = self._window_blocks(k.shape[1], q.shape[0], cu_seqlens, torch.zeros(batch, dtype=torch.int32, device=q.device),
-                                                 max_seqlen, 0, q.device)
+            topk_idx, mask = self._window_blocks(k.shape[1], q.shape[0], cu_seqlens, None, max_seqlen, 0)
         elif self.selection == "sparse" and max_seqlen > self.dense_len:
             # the selection launch also writes the packed mask Stage 2 walks; plain prefill: no cached tokens in any sequence
             scale = q.shape[-1] ** (-0.5) if self.softmax_scale is None else self.softmax_scale
@@ -170,7 +160,7 @@ class InfLLMv2Attention(torch.nn.Module):
         def window_mask():
             dev = q.device
             _, mask = self._window_blocks(cache.k.shape[2], 1, torch.tensor([0, 1], dtype=torch.int32, device=dev),
-                                          torch.tensor([pos], dtype=torch.int32, device=dev), 1, pos, dev)
+                                          torch.tensor([pos], dtype=torch.int32, device=dev), 1, pos)
             return mask.transpose(0, 1).unsqueeze(2).contiguous()
 
         out, _ = self._step(q, k_new, v_new, cache.k, cache.v, cache.k_fine.unsqueeze(0), cache.k_coarse.unsqueeze(0), None, pos, None, None,
@@ -207,7 +197,7 @@ class InfLLMv2Attention(torch.nn.Module):
 
         def window_mask():
             cu_one = torch.arange(batch + 1, dtype=torch.int32, device=q.device)
-            _, mask = self._window_blocks(cache.k.shape[2], batch, cu_one, cache.lengths, 1, cache.max_length, q.device)
+            _, mask = self._window_blocks(cache.k.shape[2], batch, cu_one, cache.lengths, 1, cache.max_length)
             return mask.transpose(0, 1).unsqueeze(2).contiguous()                    # (Hk, batch, words) -> (batch, Hk, 1, words)
 
         out, new = self._step(q, k_new, v_new, cache.k, cache.v, cache.k_fine, cache.k_coarse, cache.lengths, 0, cache.fine_lens,
