@@ -285,7 +285,7 @@ int infllmv2_varlen_fwd(void* stream, const void* q, const void* k, const void* 
                         const int64_t* o_strides, const int64_t* lse_strides, int n_uint64_per_row,
                         float softmax_scale, int is_causal);
 
-/* infllmv2_varlen_fwd for a caller that knows how many blocks a row of the mask has set at most (0: not known).  The number decides
+/* infllmv2_varlen_fwd for a caller that knows how many blocks a row of the mask has set at most (0: not known; negative: so many, and neighbouring rows have the same but for a few).  The number decides
  * which of two walks is the faster; results do not depend on its being right, except for rounding. */
 int infllmv2_varlen_fwd_selected(void* stream, const void* q, const void* k, const void* v, void* out,
                                  float* softmax_lse, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
@@ -335,7 +335,7 @@ int infllmv2_varlen_bwd(void* stream, const void* dout, const void* q, const voi
                         const int64_t* dv_strides, const int64_t* lse_strides, int n_uint64_per_row,
                         float softmax_scale, int is_causal, int deterministic);
 
-/* infllmv2_varlen_bwd for a caller that knows how many blocks a row of the mask has set at most (0: not known); without a
+/* infllmv2_varlen_bwd for a caller that knows how many blocks a row of the mask has set at most (0: not known; negative: so many, and neighbouring rows have the same but for a few); without a
  * mask the number is not looked at.  It decides which of two walks forms dQ; results do not depend on its being right, except for rounding. */
 int infllmv2_varlen_bwd_selected(void* stream, const void* dout, const void* q, const void* k, const void* v,
                         const void* out, const float* softmax_lse, void* dq, void* dk, void* dv,

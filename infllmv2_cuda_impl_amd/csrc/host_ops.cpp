@@ -410,7 +410,7 @@ std::tuple<Tensor, OptTensor> select_blocks(const Tensor& q_, const Tensor& k, c
 // Returns {out, lse, packed mask or none}.  lse: (Hk, total_q * group) on the sparse path, (Hq, total_q) on the dense one.
 std::tuple<Tensor, Tensor, OptTensor> varlen_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu_q, const Tensor& cu_k,
                                                  int64_t max_q, int64_t max_k, double scale, bool causal, const OptTensor& topk_idx,
-                                                 const OptTensor& block_mask) {
+                                                 const OptTensor& block_mask, bool alike) {
     check_qkv(q, k, v, cu_q, cu_k, true);
     DeviceGuard guard(q.device());
     const int64_t batch = cu_q.numel() - 1, total_q = q.size(0), hq = q.size(1), d = q.size(2), total_k = k.size(0), hk = k.size(1);
@@ -439,8 +439,8 @@ std::tuple<Tensor, Tensor, OptTensor> varlen_fwd(const Tensor& q, const Tensor& 
     const S3 qs = grouped(q, group), os = grouped(out, group);
     const S2 ks = rows_heads(k), vs = rows_heads(v);
     auto fn = is_half(q) ? infllmv2_varlen_fwd_selected_f16 : infllmv2_varlen_fwd_selected;
-    // a mask that came with its indices has at most so many blocks to a row
-    const int most_selected = sparse && topk_idx.has_value() && topk_idx->dim() > 0 ? as_int(topk_idx->size(-1)) : 0;
+    // a mask that came with its indices has at most so many blocks to a row (negative: neighbouring rows are alike)
+    const int listed = sparse && topk_idx.has_value() && topk_idx->dim() > 0 ? as_int(topk_idx->size(-1)) : 0, most_selected = alike ? -listed : listed;
     check_rc(fn(stream_of(q), ptr(q), ptr(k), ptr(v), ptr(out), static_cast<float*>(ptr(lse)), iptr(cu_q), iptr(cu_k),
                 sparse ? static_cast<const uint64_t*>(mask->data_ptr()) : nullptr, ptr(ws), static_cast<size_t>(ws.numel()), 0, as_int(batch),
                 total_q, total_k, as_int(hq), as_int(hk), as_int(d), as_int(max_q), as_int(max_k), qs.v, ks.v, vs.v, os.v, lse_strides,

@@ -641,7 +641,8 @@ int launch_bwd_dkdv_wave(hipStream_t st, const BwdParams& p, int batch, int max_
         // 112 / 118 / 130 / 124 / 140 / 159 / 194, 2048 202 / 169 / 174 / 183 / 190 / 210 / 230 / 273, 3000 265 / 271 / 276 / 269 / 230 / 249 / 270 / 314, 4000 362 / 322 /
         // 331 / 355 / 365 / 371 / 316 / 356, 1023 + 3001 + 517 + 2200 507 / 468 / 459 / 461 / 429 / 465 / 485 / 505, 12000 1037 / 1016 / 976 / 956 / 937 / 935 / 934 / 969, 6 x
         // 3000 (32 blocks) 1693 / 1652 / 1638 / 1620 / 1608 / 1588 / 1584 / 1608, 24000 (32 blocks) 3710 / 3597 / 3569 / 3550 / 3477 / 3479 / 3382 / 3476.
-        const double pairs = selected_pairs(batch, p.num_heads_k, p.total_q, p.total_k, max_seqlen_q, max_seqlen_k, causal, most_selected);
+        const double pairs = selected_pairs(batch, p.num_heads_k, p.total_q, p.total_k, max_seqlen_q, max_seqlen_k, causal,
+                                            most_selected < 0 ? -most_selected : most_selected);
         const double fit = pairs / 600., many = pairs / 6300.;
         if (fit < 128.) return launch_bwd_dkdv_sliced<64, true>(st, p, batch, max_seqlen_q, causal, fit > 64. ? static_cast<int>(fit) : 64);
         const int item = fit <= 192. ? static_cast<int>(fit) : many <= 128. ? 128 : many < 256. ? static_cast<int>(many) : 256;

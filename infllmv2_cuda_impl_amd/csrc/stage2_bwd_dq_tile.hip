@@ -447,12 +447,14 @@ void bwd_dq_tile_kernel(const BwdParams p, const TileExtra x) {
 //   without a mask: 2048 tokens 231 | 220 *; 4 heads of 8 6000 2095 | 1617 *
 bool dq_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal,
                   int most_selected) {
-    if (most_selected <= 0 || max_seqlen_q <= 0 || max_seqlen_k <= 0) return false;
-    const double most = most_selected;
-    const double tiles = masked_walk_time(kTileRows >> tile_row_shift(group), [](double b) { return 18. + 2.3 * b; }, 0.5, batch, num_heads_k,
+    if (most_selected == 0 || max_seqlen_q <= 0 || max_seqlen_k <= 0) return false;
+    const bool alike = most_selected < 0;
+    const double most = alike ? -static_cast<double>(most_selected) : most_selected;
+    const double walked = alike ? most + 0.25 : 1e9;           // blocks of a tile at most: 16 tokens are a quarter of a block's rows
+    const double tiles = masked_walk_time(kTileRows >> tile_row_shift(group), [&](double b) { return 18. + 2.3 * (b < walked ? b : walked); }, 0.5, batch, num_heads_k,
                                           total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
     const double groups = masked_walk_time(8, [&](double b) {
-        const double beyond = b > most ? b - most : 0.;
+        const double beyond = b > most && !alike ? b - most : 0.;
         return 8. + 1.6 * (b < most ? b : most) + 0.5 * (beyond < most ? beyond : most);
     }, 0.7, batch, num_heads_k, total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
     return tiles < 0.93 * groups;

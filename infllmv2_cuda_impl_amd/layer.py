@@ -25,7 +25,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .attention import HEAD_DIM, infllmv2_attn_varlen_func, infllmv2_attn_with_kvcache, pad_head_dim
+from .attention import HEAD_DIM, attend_varlen, infllmv2_attn_with_kvcache, pad_head_dim
 from .selection import compress_keys, compress_keys_cache
 
 
@@ -111,9 +111,8 @@ class InfLLMv2Attention(torch.nn.Module):
             topk_idx, mask = _lib.host.select_blocks(qs.detach(), ks.detach(), cu_seqlens, cu_seqlens, max_seqlen, max_seqlen, self.topk,
                                                      self.local_blocks, self.init_blocks, None, 0, scale, True, self.kernel_size,
                                                      self.stride, self.block_size, False, True, False, False)
-        out = infllmv2_attn_varlen_func(q, k, v, cu_seqlens, cu_seqlens, max_seqlen, max_seqlen,
-                                        softmax_scale=self.softmax_scale, causal=True, topk_idx=topk_idx,
-                                        block_mask=mask)
+        out = attend_varlen(q, k, v, cu_seqlens, cu_seqlens, max_seqlen, max_seqlen, softmax_scale=self.softmax_scale, causal=True, topk_idx=topk_idx,
+                            block_mask=mask, alike=self.selection == "window")
         if cache is not None:
             if cu_seqlens.numel() != 2:
                 raise RuntimeError("a SequenceCache holds one sequence")

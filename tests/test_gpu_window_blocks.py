@@ -23,3 +23,29 @@ def test_window_blocks(lens, positions, heads, local, init, block):
     pooled = ops.max_pooling_1d_varlen(scores, cu, torch.zeros_like(cu), held, max(lens), 0, local, init, block_size=block, stride=16, max_cache_len=most)
     want_idx, want_mask = ops.topk_blocks(pooled, init + local + 1, return_mask=True, by_index=True, drop_unreachable=True)
     assert torch.equal(idx, want_idx) and torch.equal(mask, want_mask)
+
+
+@pytest.mark.parametrize("lens, Hk, group, local, init", [([40000], 1, 16, 4, 1), ([66000, 33], 1, 8, 2, 0), ([700, 9000, 65], 2, 16, 31, 1), ([5000], 2, 8, 80, 66)])
+def test_windows_by_tiles(lens, Hk, group, local, init):
+    """Told that neighbouring rows are alike, forward and dQ go by tiles, whose walk jumps over the words between the first blocks and the window (more than
+    eight of them in the first two cases): against the walk per token on the same mask."""
+    import infllmv2_cuda_impl_amd as ops
+    from infllmv2_cuda_impl_amd import _lib
+    from infllmv2_cuda_impl_amd.attention import attend_varlen
+    g = torch.Generator(device="cuda").manual_seed(5)
+    total, mx = sum(lens), max(lens)
+    q, k, v = (torch.randn(total, h, 128, generator=g, device="cuda").to(torch.bfloat16).requires_grad_(True) for h in (group * Hk, Hk, Hk))
+    dout = torch.randn(total, group * Hk, 128, generator=g, device="cuda").to(torch.bfloat16)
+    cu = torch.tensor([sum(lens[:i]) for i in range(len(lens) + 1)], dtype=torch.int32, device="cuda")
+    idx, mask = _lib.host.window_blocks(Hk, total, cu, None, mx, 0, local, init, 64)
+    most = -(init + local + 1)
+    assert _lib.lib.infllmv2_varlen_fwd_masked_tiles(len(lens), total, total, group * Hk, Hk, mx, mx, 1, most) == 1
+    got, want = [], []
+    for alike, result in ((True, got), (False, want)):
+        out = attend_varlen(q, k, v, cu, cu, mx, mx, causal=True, topk_idx=idx if alike else None, block_mask=mask, alike=alike)
+        result += [out] + list(torch.autograd.grad(out, (q, k, v), dout))
+    for name, a, b in zip(("out", "dq", "dk", "dv"), got, want):
+        # P, dS and the results are rounded to 8 bits of mantissa on either side, in other orders of summation: 2^-9 each
+        assert (a.float() - b.float()).norm() <= 2.0 ** -7 * b.float().norm(), name
+        rows = (a.float() - b.float()).norm(dim=-1) - 2.0 ** -4 * b.float().norm(dim=-1)
+        assert rows.max() <= 1e-2, (name, rows.max().item())
