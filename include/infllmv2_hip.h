@@ -261,7 +261,7 @@ size_t infllmv2_kv_image_bytes(int64_t total_k, int batch, int num_heads_k);
 int infllmv2_varlen_fwd_dense_tiles(int batch, int64_t total_q, int64_t total_k, int num_heads, int num_heads_k,
                                     int max_seqlen_q, int max_seqlen_k, int is_causal);
 
-/* The same for infllmv2_varlen_fwd_selected with a blockmask. */
+/* The same for infllmv2_varlen_fwd_selected with a blockmask: only most_selected decides, not the sizes. */
 int infllmv2_varlen_fwd_masked_tiles(int batch, int64_t total_q, int64_t total_k, int num_heads, int num_heads_k,
                                      int max_seqlen_q, int max_seqlen_k, int is_causal, int most_selected);
 
@@ -285,8 +285,10 @@ int infllmv2_varlen_fwd(void* stream, const void* q, const void* k, const void* 
                         const int64_t* o_strides, const int64_t* lse_strides, int n_uint64_per_row,
                         float softmax_scale, int is_causal);
 
-/* infllmv2_varlen_fwd for a caller that knows how many blocks a row of the mask has set at most (0: not known; negative: so many, and neighbouring rows have the same but for a few).  The number decides
- * which of two walks is the faster; results do not depend on its being right, except for rounding. */
+/* infllmv2_varlen_fwd for a caller that knows how many blocks a row of the mask has set at most (0: not known; negative: so many, and neighbouring
+ * rows have the same but for a few).  A negative number is walked by tiles, any other by groups of 8 tokens; results do not depend on its being
+ * right, except for rounding.  With a blockmask, a row is the same bit for bit whatever else its launch holds (other sequences, other KV heads, fewer queries
+ * of its sequence), where the sign of the number is the same and the queries begin and end at multiples of 8 tokens or with their sequence. */
 int infllmv2_varlen_fwd_selected(void* stream, const void* q, const void* k, const void* v, void* out,
                                  float* softmax_lse, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
                                  const uint64_t* blockmask, void* workspace, size_t workspace_bytes,
@@ -335,8 +337,9 @@ int infllmv2_varlen_bwd(void* stream, const void* dout, const void* q, const voi
                         const int64_t* dv_strides, const int64_t* lse_strides, int n_uint64_per_row,
                         float softmax_scale, int is_causal, int deterministic);
 
-/* infllmv2_varlen_bwd for a caller that knows how many blocks a row of the mask has set at most (0: not known; negative: so many, and neighbouring rows have the same but for a few); without a
- * mask the number is not looked at.  It decides which of two walks forms dQ; results do not depend on its being right, except for rounding. */
+/* infllmv2_varlen_bwd for a caller that knows how many blocks a row of the mask has set at most (0: not known; negative: so many, and neighbouring
+ * rows have the same but for a few); without a mask the number is not looked at.  It decides which of two walks forms dQ and how dK / dV are dealt
+ * out; results do not depend on its being right, except for rounding.  Rows of dQ are the same bit for bit in every launch as the forward's are. */
 int infllmv2_varlen_bwd_selected(void* stream, const void* dout, const void* q, const void* k, const void* v,
                         const void* out, const float* softmax_lse, void* dq, void* dk, void* dv,
                         const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
@@ -347,7 +350,8 @@ int infllmv2_varlen_bwd_selected(void* stream, const void* dout, const void* q, 
                         const int64_t* do_strides, const int64_t* dq_strides, const int64_t* dk_strides,
                         const int64_t* dv_strides, const int64_t* lse_strides, int n_uint64_per_row,
                         float softmax_scale, int is_causal, int deterministic, int most_selected);
-/* Whether infllmv2_varlen_bwd_selected forms dQ by tiles of 256 query rows (1) or by groups of 8 tokens (0). */
+/* Whether infllmv2_varlen_bwd_selected forms dQ by tiles of 256 query rows (1) or by groups of 8 tokens (0); most_selected 2^31 - 1: without a
+ * mask.  With one, the sizes do not decide. */
 int infllmv2_varlen_bwd_dq_tiles(int batch, int64_t total_q, int64_t total_k, int num_heads, int num_heads_k,
                                  int max_seqlen_q, int max_seqlen_k, int is_causal, int most_selected);
 

@@ -155,7 +155,9 @@ def infllmv2_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
     windows and paged KV are rejected exactly as the reference build rejects them.
     ``block_mask`` (not in the reference's signature) is the packed form of the same selection, int64
     ``(nheads_k, total_q, ceil(ceil(max_seqlen_k / 64) / 64))`` as ``topk_to_uint64`` / ``topk_blocks(return_mask=True)``
-    produce it; when given it is used as is and ``topk_idx`` is ignored.
+    produce it; when given it is used as is and the entries of ``topk_idx`` are ignored.
+    With a selection, a row of the output and of dQ is the same bit for bit whatever else the call holds (other sequences, other KV
+    heads, fewer queries of its sequence, as long as they begin and end at multiples of 8 tokens or with the sequence).
     Head sizes below 128 are served by zero padding (see :func:`pad_head_dim`); ``softmax_scale`` then defaults to
     the caller's head size ``** -0.5``, as in the reference.
     """
@@ -167,7 +169,8 @@ def attend_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_
                   window_size=(-1, -1), softcap=0.0, alibi_slopes=None, deterministic=False, return_attn_probs=False, block_table=None,
                   topk_idx=None, block_mask=None, alike=False):
     """:func:`infllmv2_attn_varlen_func` for callers that know more about the selection: ``alike`` says that neighbouring tokens
-    select the same blocks but for a few (a window).  It decides which walk is taken; results differ by rounding at most."""
+    select the same blocks but for a few (a window).  It decides, together with the width of ``topk_idx``, which walk is taken; results
+    differ by rounding at most."""
     head_size_og = q.shape[-1]
     if softmax_scale is None:
         softmax_scale = head_size_og ** (-0.5)

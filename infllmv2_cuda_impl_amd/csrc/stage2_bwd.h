@@ -44,7 +44,8 @@ struct BwdParams {
 
 // dQ, 8 consecutive tokens per workgroup sharing their common blocks through LDS: stage2_bwd_dq.hip
 int launch_bwd_dq_hybrid(hipStream_t st, const BwdParams& p, int batch, int max_seqlen_q, bool causal);
-// dQ by tiles of 256 query rows, and whether it pays (most_selected: as in infllmv2_varlen_bwd_selected): stage2_bwd_dq_tile.hip
+// dQ by tiles of 256 query rows, and whether it pays (most_selected: as in infllmv2_varlen_bwd_selected, or kNoMask): stage2_bwd_dq_tile.hip
+constexpr int kNoMask = 0x7fffffff;
 bool dq_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal,
                   int most_selected);
 int launch_bwd_dq_tile(hipStream_t st, const BwdParams& p, int batch, int max_seqlen_q, bool causal);

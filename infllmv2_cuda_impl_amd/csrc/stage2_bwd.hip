@@ -259,7 +259,7 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_bwd_selected)(void* stream, const void*
     }
     if (work) {
         const bool tiles = dq_tiles_pay(batch, num_heads_k, p.group, total_q, total_k, max_seqlen_q, max_seqlen_k, is_causal != 0,
-                                        fwd_blockmask == nullptr ? 0x7fffffff : most_selected);
+                                        fwd_blockmask == nullptr ? kNoMask : most_selected < kNoMask ? most_selected : 0);
         int rc = tiles ? launch_bwd_dq_tile(st, p, batch, max_seqlen_q, is_causal != 0) : launch_bwd_dq_hybrid(st, p, batch, max_seqlen_q, is_causal != 0);
         if (rc != 0) return rc;
         rc = launch_bwd_dkdv_wave(st, p, batch, max_seqlen_q, max_seqlen_k, is_causal != 0, most_selected);

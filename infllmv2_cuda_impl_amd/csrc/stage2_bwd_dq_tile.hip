@@ -1,4 +1,4 @@
-// Stage-2 backward, dQ by tiles of 256 query rows (gfx950): without a mask, or with one whose rows select most of what they see.
+// Stage-2 backward, dQ by tiles of 256 query rows (gfx950): without a mask, or for a window, whose neighbouring rows select nearly the same.
 //
 // The mathematics of stage2_bwd_dq.hip on the walk of stage2_fwd_tile.hip: a workgroup of 4 wavefronts owns 256 rows and walks the blocks that any of
 // its tokens selected; a row has P = 0 in a block it did not select.  The hybrid walk reads 48 KiB of LDS per (token, common block) for 16 query rows,
@@ -436,27 +436,22 @@ void bwd_dq_tile_kernel(const BwdParams p, const TileExtra x) {
     store(acc[1], 1, true);
 }
 
-// Whether the backward forms dQ by tiles.  A tile walks the blocks that any of its tokens selected in 2.3 us each, a group of 8 tokens a block in
-// 1.6 us, and up to 2.1 where its tokens walk it on their own.  The constants are a fit to 134 backward passes of 1 to 5 sequences of 130 to 12000
-// tokens, without a mask and with 16 to 64 blocks selected, 1 to 4 KV heads, groups of 8 and 16; groups of 8 tokens alone cost 6.6 % of the better pass
-// on average and up to 33.  Near the line the estimate errs by a few per cent: it asks for 7 % more than a tie, with which none of those passes became slower
-// than by groups and 0.3 % are left on the table.  Whole backward in us, groups of 8 tokens | tiles (* the one taken
-// here), 2 KV heads of 16 unless it says otherwise:
-//   64 blocks selected: 8000 tokens 1615 | 1580 *, 12000 2685 * | 2990, 777 + 5003 + 1291 + 9173 2748 | 2709 *; 4 heads 4 x 4096 5577 | 5152 *
-//   16 blocks selected: 1000 tokens 135 * | 145, 1023 + 3001 + 517 + 2200 463 * | 477;  4 heads of 8, 32 blocks, 3000 596 | 450 *
-//   without a mask: 2048 tokens 231 | 220 *; 4 heads of 8 6000 2095 | 1617 *
+// Whether the backward forms dQ by tiles.
+// Without a mask by an estimate: a tile walks a block in 2.3 us, a group of 8 tokens in 1.6.  The constants are a fit to 134 backward passes of 1 to 5 sequences of 130 to
+// 12000 tokens, 1 to 4 KV heads, groups of 8 and 16.  Near the line the estimate errs by a few per cent: it asks for 7 % more than a tie, with which none of those passes
+// became slower than by groups.  Whole backward in us, groups of 8 tokens | tiles (* the one taken here): 2 KV heads of 16, 2048 tokens 231 * | 220; 4 heads of 8, 6000
+// tokens 2095 | 1617 *.
+// Under a mask, as in the forward, only by what a chunk, a KV head and a batch of the same rows have in common: blocks chosen by score by groups, windows by tiles where
+// tiles are the faster walk in a launch that they fill.  Whole backward in us, groups | tiles, groups of 16 unless said otherwise: 33 blocks: 9000 tokens, 2 KV heads 1049 |
+// 974, 40000, 1 head 2434 | 2262 (2000, 1 head 133 | 154); 6 blocks: 40000 860 | 862, 60000 1303 | 1313 (1000, 2 heads 84 | 93), groups of 8 40000 804 | 680, 1000, 4 heads 105 |
+// 103.
 bool dq_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal,
                   int most_selected) {
-    if (most_selected == 0 || max_seqlen_q <= 0 || max_seqlen_k <= 0) return false;
-    const bool alike = most_selected < 0;
-    const double most = alike ? -static_cast<double>(most_selected) : most_selected;
-    const double walked = alike ? most + 0.25 : 1e9;           // blocks of a tile at most: 16 tokens are a quarter of a block's rows
-    const double tiles = masked_walk_time(kTileRows >> tile_row_shift(group), [&](double b) { return 18. + 2.3 * (b < walked ? b : walked); }, 0.5, batch, num_heads_k,
+    if (most_selected != kNoMask) return most_selected < 0 && (group == 8 || most_selected <= -16);
+    if (max_seqlen_q <= 0 || max_seqlen_k <= 0) return false;
+    const double tiles = masked_walk_time(kTileRows >> tile_row_shift(group), [](double b) { return 18. + 2.3 * b; }, 0.5, batch, num_heads_k,
                                           total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
-    const double groups = masked_walk_time(8, [&](double b) {
-        const double beyond = b > most && !alike ? b - most : 0.;
-        return 8. + 1.6 * (b < most ? b : most) + 0.5 * (beyond < most ? beyond : most);
-    }, 0.7, batch, num_heads_k, total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
+    const double groups = masked_walk_time(8, [](double b) { return 8. + 1.6 * b; }, 0.7, batch, num_heads_k, total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
     return tiles < 0.93 * groups;
 }
 

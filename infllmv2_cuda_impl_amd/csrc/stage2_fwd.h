@@ -26,14 +26,13 @@ struct FwdParams {
 // Workgroup-hybrid forward (stage2_fwd_hybrid.hip): 8 consecutive tokens per workgroup stage the blocks they all
 // select once in LDS and walk the rest of their rows one wavefront each.  in_step: kInStepBytes of scratch that belong to this launch
 // alone (the counters by which workgroups walk long sequences in step), or null.  most_selected: as in infllmv2_varlen_fwd_selected.  Goes by
-// tiles where that is the faster walk.
+// tiles without a mask where that is the faster walk, and for windows.
 int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q,
                              int max_seqlen_k, bool causal, int most_selected, unsigned* in_step);
 
 // Forward by tiles of 256 query rows (stage2_fwd_tile.hip), 64 per wavefront.  A token takes 16 rows, 8 in groups of 8.
 bool dense_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal);
-bool masked_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal,
-                      int most_selected);
+bool masked_by_tiles(int most_selected);
 int launch_stage2_fwd_tile(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q,
                            int max_seqlen_k, bool causal);
 

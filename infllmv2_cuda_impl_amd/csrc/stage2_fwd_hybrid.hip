@@ -409,7 +409,7 @@ int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int 
     IV2_CHECK((max_seqlen_k + kBlockN - 1) / kBlockN <= kMaxMaskWords * 64, "varlen_fwd: more than %d key blocks per sequence", kMaxMaskWords * 64);
     const bool tiles = p.mask == nullptr
         ? dense_tiles_pay(batch, num_heads_k, p.group, p.total_q, p.total_k, max_seqlen_q, max_seqlen_k, causal)
-        : masked_tiles_pay(batch, num_heads_k, p.group, p.total_q, p.total_k, max_seqlen_q, max_seqlen_k, causal, most_selected);
+        : masked_by_tiles(most_selected);
     if (tiles) return launch_stage2_fwd_tile(st, p, batch, num_heads_k, max_seqlen_q, max_seqlen_k, causal);
     x.total_groups = static_cast<int>(total);
     x.mask_words = ((max_seqlen_k + kBlockN - 1) / kBlockN + 63) / 64;

@@ -1,4 +1,4 @@
-// Stage-2 forward by flash tiles of 256 query rows (gfx950): without a mask, or with one whose rows select most of what they see.
+// Stage-2 forward by flash tiles of 256 query rows (gfx950): without a mask, or for a window, whose neighbouring rows select nearly the same.
 //
 // Where every token attends its whole prefix nothing is left to fetch per token, and the hybrid walk (stage2_fwd_hybrid.hip) only
 // keeps its costs: 16 query rows per K / V fragment read from LDS, softmax and MFMAs of a wavefront one after the other; where the rows differ a
@@ -425,30 +425,13 @@ bool dense_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int
     return tiles < groups + 1.;
 }
 
-// Whether a forward whose rows select at most `most_selected` blocks goes by tiles.  A tile walks the blocks that any of its tokens selected,
-// nearly all it can see, in 1.4 us each; a group of 8 tokens takes 1.0 us for a block that all of them selected and up to 1.8 for those that its tokens
-// walk on their own.  So tiles win while the rows see up to about two and a half times what they select, and lose where the longest tile's chain decides
-// (one short prompt, one KV head).  The constants are a fit to 139 launches of 1 to 8 sequences of 130 to 25000 tokens, 16 to 64 blocks selected, 1 to 4
-// KV heads, groups of 8 and 16 (within 7 and 9 %); groups of 8 tokens alone cost 24 % of the better walk's time on average.  Near the line the estimate errs by a few
-// per cent (10612 tokens, 64 blocks selected, 2 heads: a tie by it, tiles 2 % slower): it asks for 8 % more than a tie, which leaves 0.5 % on the table.  Operator in us, groups of 8 tokens | tiles (* the one taken here), 2 KV heads of 16 unless it says otherwise:
-//   64 blocks selected: 3000 tokens 113 | 89 *, 8000 505 | 454 *, 12000 840 * | 960, 777 + 5003 + 1291 + 9173 883 | 815 *; 4 heads 4 x 4096 1396 | 1010 *
-//   16 blocks selected: 1000 tokens 31 * | 39, 2048 56 * | 62, 1023 + 3001 + 517 + 2200 151 | 145 *; 4 heads of 8 4000 182 | 128 *
-bool masked_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal,
-                      int most_selected) {
-    if (most_selected == 0 || max_seqlen_q <= 0 || max_seqlen_k <= 0) return false;
-    // Neighbouring rows alike: a tile walks what one row has and a little, a group of 8 the same in lock step.  Window prefill in us, groups | tiles, 1 KV head: 60000 tokens,
-    // 6 blocks 394 | 343, 110000 769 | 673; 2 KV heads: 2000 tokens, 6 blocks 32.4 | 29.1, 9000, 33 blocks 348 | 272, 40000 in groups of 8 454 | 246.
-    const bool alike = most_selected < 0;
-    const double most = alike ? -static_cast<double>(most_selected) : most_selected;
-    const double walked = alike ? most + 0.25 : 1e9;           // blocks of a tile at most: 16 tokens are a quarter of a block's rows
-    const double tiles = masked_walk_time(kTileRows >> tile_row_shift(group), [&](double b) { return 10. + 1.4 * (b < walked ? b : walked); }, 0.5, batch, num_heads_k,
-                                          total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
-    const double groups = masked_walk_time(8, [&](double b) {
-        const double beyond = b > most && !alike ? b - most : 0.;
-        return 8. + (b < most ? b : most) + 0.4 * (beyond < most ? beyond : most);
-    }, 0.3, batch, num_heads_k, total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
-    return tiles < 0.92 * groups;
-}
+// Whether a forward under a mask goes by tiles.  Masked rows are the same bit for bit whatever else is in their launch (a chunk of the queries, a KV head on
+// its own, other sequences), and the two walks round apart: so the choice may use only what all of those have in common, never the size of the launch.
+// Blocks chosen by score go by groups of 8 tokens, whatever tiles would gain in a launch that they fill.  A window (neighbouring rows alike) goes by tiles: a tile
+// walks what one row has and a little.  Layer prefill in us, groups | tiles, groups of 16 unless said otherwise: 60000 tokens, 1 KV head, 6 blocks 381 | 338; 40000, 33
+// blocks 776 | 649; 40000, 6 blocks, groups of 8 224 | 125; 9000, 2 heads, 33 blocks 322 | 268; 30 x 600, 2 heads, 6 blocks 187 | 165.  Launches that do not fill the chip
+// pay for it: 1000 tokens, 2 heads, 6 blocks 20.9 | 26.2; 2000, 1 head, 33 blocks 43.5 | 57.7.
+bool masked_by_tiles(int most_selected) { return most_selected < 0; }
 
 int launch_stage2_fwd_tile(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q, int max_seqlen_k, bool causal) {
     TileExtra x{};
@@ -478,9 +461,8 @@ extern "C" int infllmv2_varlen_fwd_dense_tiles(int batch, int64_t total_q, int64
     return num_heads_k > 0 && batch > 0 && IV2_NS::dense_tiles_pay(batch, num_heads_k, num_heads / num_heads_k, total_q, total_k, max_seqlen_q,
                                                                    max_seqlen_k, is_causal != 0) ? 1 : 0;
 }
-extern "C" int infllmv2_varlen_fwd_masked_tiles(int batch, int64_t total_q, int64_t total_k, int num_heads, int num_heads_k, int max_seqlen_q,
-                                                int max_seqlen_k, int is_causal, int most_selected) {
-    return num_heads_k > 0 && batch > 0 && IV2_NS::masked_tiles_pay(batch, num_heads_k, num_heads / num_heads_k, total_q, total_k, max_seqlen_q,
-                                                                    max_seqlen_k, is_causal != 0, most_selected) ? 1 : 0;
+extern "C" int infllmv2_varlen_fwd_masked_tiles(int batch, int64_t /*total_q*/, int64_t /*total_k*/, int /*num_heads*/, int num_heads_k, int /*max_seqlen_q*/,
+                                                int /*max_seqlen_k*/, int /*is_causal*/, int most_selected) {
+    return num_heads_k > 0 && batch > 0 && IV2_NS::masked_by_tiles(most_selected) ? 1 : 0;
 }
 #endif

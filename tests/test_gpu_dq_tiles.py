@@ -1,5 +1,6 @@
 """dQ by tiles of 256 query rows, under masks and without: blocks that some tokens of a tile or wavefront selected and others did not, rows that
-selected nothing, masks of two words, ends of tiles, queries behind cached keys and before the first key, groups of 16, 8 and 4.  All gradients (dK and
+selected nothing, masks of two words, ends of tiles, queries behind cached keys and before the first key, groups of 16, 8 and 4.  Under a mask it is the walk
+of callers that say that neighbouring rows are alike, and holds for any mask.  All gradients (dK and
 dV read the row scalars that this kernel leaves) against fp32 attention's; tolerances of the backward tests: 2e-2 and 1e-3 of the largest value."""
 import pytest
 import torch
@@ -47,13 +48,13 @@ def gradients(q, k, v, dout, sq, sk, Hk, group, causal, idx):
 
 def by_tiles(sq, sk, Hk, group, k, causal):
     from infllmv2_cuda_impl_amd import _lib
-    return _lib.lib.infllmv2_varlen_bwd_dq_tiles(len(sq), sum(sq), sum(sk), Hk * group, Hk, max(sq), max(sk), int(causal), k or 2 ** 31 - 1)
+    return _lib.lib.infllmv2_varlen_bwd_dq_tiles(len(sq), sum(sq), sum(sk), Hk * group, Hk, max(sq), max(sk), int(causal), -k or 2 ** 31 - 1)
 
 
 def backward(q, k, v, dout, cu_q, cu_k, sq, sk, causal, idx):
-    import infllmv2_cuda_impl_amd as ops
+    from infllmv2_cuda_impl_amd.attention import attend_varlen
     leaves = [t.detach().clone().requires_grad_(True) for t in (q, k, v)]
-    out = ops.infllmv2_attn_varlen_func(*leaves, cu_q, cu_k, max(sq), max(sk), causal=causal, topk_idx=idx)
+    out = attend_varlen(*leaves, cu_q, cu_k, max(sq), max(sk), causal=causal, topk_idx=idx, alike=idx is not None)
     return torch.autograd.grad(out, leaves, dout)
 
 
@@ -97,8 +98,11 @@ def test_infinities_stay_with_the_rows_that_selected_them(group, dtype):
 
 def test_which_backward_passes_form_dq_by_tiles():
     f = lambda lens, Hk, group, k: by_tiles(lens, lens, Hk, group, k, True)
-    assert f([8000], 2, 16, 64) and f([777, 5003, 1291, 9173], 2, 16, 64) and f([3000], 4, 8, 32) and f([6000], 4, 8, 0)
-    assert not f([1000], 2, 16, 16) and not f([12000], 2, 16, 64) and not f([1023, 3001, 517, 2200], 2, 16, 16)
+    assert f([6000], 4, 8, 0) and f([16384], 2, 16, 0) and not f([300], 2, 16, 0)            # without a mask
+    for lens, Hk in (([1000], 2), ([8000], 2), ([777, 5003, 1291, 9173], 2), ([3000], 4)):
+        assert f(lens, Hk, 16, 33) and f(lens, Hk, 8, 6) and not f(lens, Hk, 16, 6)        # windows, whatever the sizes
+        for k in (16, 64):                                     # blocks chosen by score
+            assert not f(lens, Hk, 16, -k) and not f(lens, Hk, 8, -k)
     from infllmv2_cuda_impl_amd import _lib
     assert _lib.lib.infllmv2_varlen_bwd_dq_tiles(1, 3000, 3000, 32, 4, 3000, 3000, 1, 0) == 0     # how many blocks a row selects is not known
     for n in (0, 1, 2 ** 31 - 1):

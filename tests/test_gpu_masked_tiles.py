@@ -1,5 +1,6 @@
 """Stage-2 forward by tiles of 256 query rows under a mask: blocks that some tokens of a tile or wavefront selected and others did not, rows that
-selected nothing, masks of two words, ends of tiles, queries behind cached keys, groups of 16, 8 and 4.  Against fp32 softmax attention over the selected
+selected nothing, masks of two words, ends of tiles, queries behind cached keys, groups of 16, 8 and 4.  It is the walk of callers that say that neighbouring
+rows are alike, and holds for any mask.  Against fp32 softmax attention over the selected
 blocks; tolerances of the forward tests: 2e-2 on a 16-bit output of order one, 1e-3 on average, 2e-3 on the log-sum-exp."""
 import numpy as np
 import pytest
@@ -67,7 +68,12 @@ def inputs(sq, sk, Hk, group, dtype, gen):
 
 def by_tiles(sq, sk, Hk, group, k, causal):
     from infllmv2_cuda_impl_amd import _lib
-    return _lib.lib.infllmv2_varlen_fwd_masked_tiles(len(sq), sum(sq), sum(sk), Hk * group, Hk, max(sq), max(sk), int(causal), k)
+    return _lib.lib.infllmv2_varlen_fwd_masked_tiles(len(sq), sum(sq), sum(sk), Hk * group, Hk, max(sq), max(sk), int(causal), -k)
+
+
+def attend(*args, **more):
+    from infllmv2_cuda_impl_amd.attention import attend_varlen
+    return attend_varlen(*args, causal=more.pop("causal", True), alike=True, **more)
 
 
 def check(out, lse, ref, ref_lse, Hk, group):
@@ -81,13 +87,11 @@ def check(out, lse, ref, ref_lse, Hk, group):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("sq, sk, Hk, group, k, causal", CASES)
 def test_masked_tiles(sq, sk, Hk, group, k, causal, dtype):
-    import infllmv2_cuda_impl_amd as ops
     assert by_tiles(sq, sk, Hk, group, k, causal) == 1
     gen = torch.Generator(device="cpu").manual_seed(3)
     q, kk, v, cu_q, cu_k = inputs(sq, sk, Hk, group, dtype, gen)
     idx = selection(sq, sk, Hk, k, causal, gen)
-    out, lse, _ = ops.infllmv2_attn_varlen_func(q, kk, v, cu_q, cu_k, max(sq), max(sk), causal=causal, topk_idx=idx.cuda(),
-                                                return_attn_probs=True)
+    out, lse, _ = attend(q, kk, v, cu_q, cu_k, max(sq), max(sk), causal=causal, topk_idx=idx.cuda(), return_attn_probs=True)
     check(out, lse, *reference(q, kk, v, sq, sk, Hk, group, causal, idx), Hk, group)
 
 
@@ -95,7 +99,6 @@ def test_masked_tiles(sq, sk, Hk, group, k, causal, dtype):
 @pytest.mark.parametrize("group", [16, 8])
 def test_infinities_stay_with_the_rows_that_selected_them(group, dtype):
     """Blocks that hold infinities and NaN, each selected by one token of a tile: every other row is what it is without them."""
-    import infllmv2_cuda_impl_amd as ops
     S, Hk, k = 1100, 8, 16
     assert by_tiles([S], [S], Hk, group, k, True) == 1
     gen = torch.Generator(device="cpu").manual_seed(4)
@@ -105,9 +108,9 @@ def test_infinities_stay_with_the_rows_that_selected_them(group, dtype):
     for block, token in bad.items():
         idx = torch.where(idx == block, -1, idx)
         idx[:, token, 1] = block
-    clean = ops.infllmv2_attn_varlen_func(q, kk, v, cu, cu, S, S, causal=True, topk_idx=idx.cuda())
+    clean = attend(q, kk, v, cu, cu, S, S, topk_idx=idx.cuda())
     kk[3 * 64 + 5, :, 7], v[7 * 64 + 40, :, 100], v[9 * 64, :, 3] = float("nan"), float("inf"), float("-inf")
-    out = ops.infllmv2_attn_varlen_func(q, kk, v, cu, cu, S, S, causal=True, topk_idx=idx.cuda())
+    out = attend(q, kk, v, cu, cu, S, S, topk_idx=idx.cuda())
     touched = torch.zeros(S, dtype=torch.bool, device=out.device)
     touched[list(bad.values())] = True
     touched[[t for t in range(S) if t // 64 in bad]] = True   # a block's own tokens select it whatever the indices above say
@@ -119,8 +122,9 @@ def test_infinities_stay_with_the_rows_that_selected_them(group, dtype):
 
 def test_which_masked_launches_go_by_tiles():
     f = lambda lens, Hk, group, k: by_tiles(lens, lens, Hk, group, k, True)
-    assert f([3000], 2, 16, 64) and f([8000], 2, 16, 64) and f([777, 5003, 1291, 9173], 2, 16, 64) and f([4000], 4, 8, 16)
-    assert not f([1000], 2, 16, 16) and not f([2048], 2, 16, 16) and not f([16000], 2, 16, 64) and not f([131072], 2, 16, 64)
-    assert not f([3000], 2, 16, 0)                             # how many blocks a row selects is not known
+    for lens, Hk, group in (([1000], 2, 16), ([3000], 2, 16), ([777, 5003, 1291, 9173], 2, 16), ([4000], 4, 8), ([131072], 2, 16)):
+        assert f(lens, Hk, group, 16) == 1                     # a window, whatever the sizes
+        for k in (0, 16, 64, 2 ** 31 - 1):                     # blocks chosen by score, or how many is not known
+            assert f(lens, Hk, group, -k) == 0
     for n in (0, 1, 2 ** 31 - 1):
         assert f([n], 2, 16, 2 ** 31 - 1) in (0, 1)
