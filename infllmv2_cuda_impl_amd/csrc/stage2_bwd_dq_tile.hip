@@ -108,7 +108,8 @@ void bwd_dq_tile_kernel(const BwdParams p, const TileExtra x) {
         }
     }
 
-    TileWalk walk;
+    typedef TileWalk<kCausal> Walk;
+    Walk walk;
     {
         const int left = Sq - i_first, all = kTileRows >> x.row_shift;
         walk.tokens = left < all ? left : all;
@@ -119,6 +120,7 @@ void bwd_dq_tile_kernel(const BwdParams p, const TileExtra x) {
         walk.n64 = p.n64_fwd;
         walk.mine = wave * 2 * per_half;
         walk.per_wave = 2 * per_half;
+        walk.last_key = last_of(i_first);
         walk.init();
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                // before the first LDS-DMA (see the hybrid walk)
@@ -133,7 +135,7 @@ void bwd_dq_tile_kernel(const BwdParams p, const TileExtra x) {
     // the unit that lands in this lane's place of a kilobyte
     const uint32_t dma_lane = static_cast<uint32_t>(((lane >> 4) * 16 + (((lane & 15) - 4 * (lane >> 4)) & 15)) * 16);
     auto issue_part = [&](int block, int slot, int part) {     // 1 KiB of 8
-        const elem_bits* src = (part < 4 ? kimg : vimg) + static_cast<int64_t>(TileWalk::index(block)) * kImageElems + wave * 2048 + (part & 3) * 512;
+        const elem_bits* src = (part < 4 ? kimg : vimg) + static_cast<int64_t>(Walk::index(block)) * kImageElems + wave * 2048 + (part & 3) * 512;
         dq_dma_1k(src, dma_lane, ring_base + slot * kSlotBytes + (part >> 2) * (kSlotBytes / 2) + (part & 3) * 1024);
     };
     auto issue = [&](int block, int slot) {
@@ -170,13 +172,13 @@ void bwd_dq_tile_kernel(const BwdParams p, const TileExtra x) {
     auto hide = [&](int cc, int block) {                       // keys behind the rows' last ones
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
-            const int lim = last_of(i_wave + hf * per_half + (n >> x.row_shift)) - TileWalk::index(block) * kBlockN;
+            const int lim = last_of(i_wave + hf * per_half + (n >> x.row_shift)) - Walk::index(block) * kBlockN;
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 if (32 * cc + 8 * (r >> 2) + 4 * h + (r & 3) > lim) s[hf][cc][r] = -INFINITY;
         }
     };
-    auto edge = [&](int block) { return TileWalk::index(block) * kBlockN + kBlockN - 1 > wave_first_key; };   // the last block or two
+    auto edge = [&](int block) { return Walk::index(block) * kBlockN + kBlockN - 1 > wave_first_key; };   // the last block or two
 
     // ---- operands: 48 a step, each read three uses ahead ----
     elem8 fr[4];
@@ -362,7 +364,7 @@ void bwd_dq_tile_kernel(const BwdParams p, const TileExtra x) {
         }
     }
     const int full = (1 << 2 * per_half) - 1;
-    if (late->fwd_mask != nullptr && (every >> kTokenBits & full) != full) {         // uniform per wavefront: a block was walked for some rows only
+    if ((every >> kTokenBits & full) != full) {                            // uniform per wavefront: a block was walked for some rows only
         // An infinity or a NaN in a block passes to rows that did not select it (0 x inf).  Where the result shows one, this wavefront's tokens are
         // walked once more, one at a time and each over its own blocks alone.
         float sum = 0.f;
@@ -383,7 +385,8 @@ void bwd_dq_tile_kernel(const BwdParams p, const TileExtra x) {
                 const int from = (n & ((1 << x.row_shift) - 1)) + ((t - hf * per_half) << x.row_shift);
                 const float lse_t = __shfl(hf ? lse2[1] : lse2[0], from), d_t = __shfl(hf ? dsum[1] : dsum[0], from);
                 BlockWalker own;
-                own.init(late->fwd_mask + (static_cast<int64_t>(h_kv) * late->total_q + tok) * late->n64_fwd, late->n64_fwd, lk < 0 ? -1 : lk >> 6);
+                own.init(late->fwd_mask ? late->fwd_mask + (static_cast<int64_t>(h_kv) * late->total_q + tok) * late->n64_fwd : nullptr, late->n64_fwd,
+                         lk < 0 ? -1 : lk >> 6);
                 floatx16 a[4] = {zero, zero, zero, zero};
                 for (int j = own.next(); j >= 0 && j < x.max_blocks; j = own.next()) {
                     const elem_bits* kb = kimg + static_cast<int64_t>(j) * kImageElems;

@@ -78,7 +78,8 @@ void stage2_fwd_tile_kernel(const FwdParams p, const TileExtra x) {
         for (int ks = 0; ks < 8; ++ks) qf[hf][ks] = *reinterpret_cast<const elem8*>(qp + 16 * ks);
     }
 
-    TileWalk walk;
+    typedef TileWalk<kCausal> Walk;
+    Walk walk;
     {
         const int left = Sq - i_first, all = kTileRows >> x.row_shift;
         walk.tokens = left < all ? left : all;
@@ -89,6 +90,7 @@ void stage2_fwd_tile_kernel(const FwdParams p, const TileExtra x) {
         walk.n64 = p.n64;
         walk.mine = wave * 2 * per_half;
         walk.per_wave = 2 * per_half;
+        walk.last_key = last_of(i_first);
         walk.init();
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                                // before the first LDS-DMA (see the hybrid walk)
@@ -100,7 +102,7 @@ void stage2_fwd_tile_kernel(const FwdParams p, const TileExtra x) {
     const elem_bits* vimg = p.vimg + slot0 * kImageElems;
     const uint32_t ring_base = __builtin_amdgcn_readfirstlane(lds_address_of(ring) + wave * 4096);      // this wavefront copies a quarter of every image
     auto issue_part = [&](int block, int slot, int part) {     // 1 KiB of 8
-        const elem_bits* src = (part < 4 ? kimg : vimg) + static_cast<int64_t>(TileWalk::index(block)) * kImageElems + wave * 2048 + (part & 3) * 512;
+        const elem_bits* src = (part < 4 ? kimg : vimg) + static_cast<int64_t>(Walk::index(block)) * kImageElems + wave * 2048 + (part & 3) * 512;
         dma_copy_1k(src, 16 * lane, ring_base + slot * kSlotBytes + (part >> 2) * (kSlotBytes / 2) + (part & 3) * 1024);
     };
     auto issue = [&](int block, int slot) {
@@ -235,7 +237,7 @@ void stage2_fwd_tile_kernel(const FwdParams p, const TileExtra x) {
         }
         l[hf] += sum;
     };
-    auto edge = [&](int block) { return TileWalk::index(block) * kBlockN + kBlockN - 1 > wave_first_key; };   // the last block or two
+    auto edge = [&](int block) { return Walk::index(block) * kBlockN + kBlockN - 1 > wave_first_key; };   // the last block or two
 
     // The walk: j0 is the current block, j1 the next; j1 and j2 are in the ring or on their way, j3 is requested.  The two halves of the rows take turns: while
     // the matrix pipe works on one, the exponentials of the other are formed.  At the top of a step P of j0 is there for the first half, its scores
@@ -260,7 +262,7 @@ void stage2_fwd_tile_kernel(const FwdParams p, const TileExtra x) {
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
             // rows that selected the first block take their reference from it
-            if (edge(j0)) hide(hf, TileWalk::index(j0));
+            if (edge(j0)) hide(hf, Walk::index(j0));
             const float mx = largest(hf);
             if (selects(hf, j0) && mx > kNoReference && mx < INFINITY) m[hf] = mx;
         }
@@ -276,12 +278,12 @@ void stage2_fwd_tile_kernel(const FwdParams p, const TileExtra x) {
             if (g < 24 && g % 3 != 2) read_k(slot, 2 * (g / 3) + g % 3);
             if (g >= 24 && g % 2 == 0) issue_part(j3 >= 0 ? j3 : j1, freed, (g - 24) / 2);   // behind the last block the slot takes anything
         }, 1, against(1, j0)));
-        if (edge(j1)) hide(0, TileWalk::index(j1));
+        if (edge(j1)) hide(0, Walk::index(j1));
         settle(0, j1, half_step([&](int g) { if (g < 16) form_o(1)(g); else form_s(1)(g - 16); }, [&](int g) {
             if (g < 8 && g % 2 == 0) issue_part(j3 >= 0 ? j3 : j1, freed, 4 + g / 2);
             if (g >= 8 && (g - 8) % 3 != 2) read_v(slot, 2 * ((g - 8) / 3) + (g - 8) % 3);
         }, 0, against(0, j1)));
-        if (edge(j1)) hide(1, TileWalk::index(j1));
+        if (edge(j1)) hide(1, Walk::index(j1));
         at1 = at1 == 2 ? 0 : at1 + 1;
         j0 = j1; j1 = j2; j2 = j3;
     }
@@ -324,7 +326,7 @@ void stage2_fwd_tile_kernel(const FwdParams p, const TileExtra x) {
         }
     };
     const int full = (1 << 2 * per_half) - 1;
-    if (late->mask != nullptr && (every >> kTokenBits & full) != full) {             // uniform per wavefront: a block was walked for some rows only
+    if ((every >> kTokenBits & full) != full) {             // uniform per wavefront: a block was walked for some rows only
         // An infinity or a NaN in a block passes to rows that did not select it (0 x inf).  Where the result shows one, this wavefront's tokens are
         // walked once more, one at a time and each over its own blocks alone.
         float sum = l[0] + l[1];
@@ -345,7 +347,8 @@ void stage2_fwd_tile_kernel(const FwdParams p, const TileExtra x) {
                     for (int ks = 0; ks < 8; ++ks) vf[ks] = *reinterpret_cast<const elem8*>(qp + 16 * ks);
                 }
                 BlockWalker own;
-                own.init(late->mask + (static_cast<int64_t>(h_kv) * late->total_q + q0 + i_wave + t) * late->n64, late->n64, lk < 0 ? -1 : lk >> 6);
+                own.init(late->mask ? late->mask + (static_cast<int64_t>(h_kv) * late->total_q + q0 + i_wave + t) * late->n64 : nullptr, late->n64,
+                         lk < 0 ? -1 : lk >> 6);
                 float mm = kNoReference, ll = 0.f;
 #pragma unroll
                 for (int u = 0; u < 4; ++u) o[0][u] = zero;

@@ -46,30 +46,38 @@ __device__ __forceinline__ float half_sum(float x) {
     return a + b;
 }
 
-// The key blocks of a tile in ascending order: those that any of its tokens selected (all of them without a mask).  Everything here is
-// uniform over the wavefront; the blocks are the same in all wavefronts of a workgroup.
+// The key blocks of a tile in ascending order: those that any of its tokens selected (all of them without a mask) and that do not begin behind that token's
+// last key.  A tile that straddles the beginning of a block walks it for the tokens behind; those before it must not count as having selected it, whatever their
+// mask says, or what the block holds would reach them as 0 x inf.  Everything here is uniform over the wavefront; the blocks are the same in all
+// wavefronts of a workgroup.
 constexpr int kTokenBits = 20;
+__device__ __forceinline__ uint64_t lowest_bits(int n) { return n >= 64 ? ~0ull : n <= 0 ? 0ull : (1ull << n) - 1ull; }
+template <bool kCausal>
 struct TileWalk {
     const uint64_t* rows;           // mask row of the tile's first token, or null
     int n64, tokens;                // words of a row; tokens of the tile that exist
     int mine;                       // first token of this wavefront inside the tile
     int per_wave;
+    int last_key;                   // of the tile's first token (negative: it has none); causal: the next ones see a key more each
     int blocks;                     // blocks at or behind this one are not walked
     int w;
     uint64_t bits;                  // of word w: what is left of the union
     int chosen;                     // lane b: which of this wavefront's tokens selected block b of word w, a bit each
 
+    __device__ __forceinline__ int seen(int t) const { return ((last_key + (kCausal ? t : 0)) >> 6) + 1; }     // blocks of the tile's token t
     __device__ __forceinline__ void load() {
         const int left = blocks - w * 64, lane = __lane_id();
         if (rows == nullptr) {
             bits = ~0ull;
             const int live = tokens - mine < per_wave ? tokens - mine : per_wave;
             chosen = live > 0 ? (1 << live) - 1 : 0;
+            const int blind = (w * 64 + lane) * kBlockN - last_key - (kCausal ? mine : 0);       // this wavefront's tokens that end before the block
+            if (blind > 0) chosen &= kCausal && blind < kMostTokens ? ~0 << blind : 0;
         } else {
             // lane t holds the word of the tile's token t
             uint32_t lo = 0u, hi = 0u;
             if (lane < tokens) {
-                const uint64_t row = rows[static_cast<int64_t>(lane) * n64 + w];
+                const uint64_t row = rows[static_cast<int64_t>(lane) * n64 + w] & lowest_bits(seen(lane) - w * 64);
                 lo = static_cast<uint32_t>(row);
                 hi = static_cast<uint32_t>(row >> 32);
             }
@@ -87,7 +95,7 @@ struct TileWalk {
             }
             bits = static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(hi))) << 32 | static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(lo));
         }
-        if (left < 64) bits &= (1ull << left) - 1ull;
+        bits &= lowest_bits(left);
     }
     __device__ __forceinline__ void init() {
         if (rows != nullptr && blocks > n64 * 64) blocks = n64 * 64;
