@@ -20,6 +20,7 @@
 #include "common.h"
 #include "kv_image.h"
 #include "block_walker.h"
+#include "lds_dma.h"
 #include "tile_walk.h"
 #include "stage2_bwd.h"
 #include "infllmv2_hip.h"
@@ -45,9 +46,6 @@ __device__ __forceinline__ void mfma_both(floatx16& acc0, floatx16& acc1, const 
     __builtin_memcpy(&ai, &a, 16);
     asm volatile("s_nop 1\n\t" IV2_MFMA32_ASM " %0, %2, %3, %0\n\t" IV2_MFMA32_ASM " %1, %2, %4, %1"
                  : "+a"(acc0), "+a"(acc1) : "v"(ai), "v"(b0), "v"(b1));
-}
-__device__ __forceinline__ void dq_dma_1k(const void* base, uint32_t lane_bytes, uint32_t lds_dst) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_bytes), "s"(base), "s"(lds_dst) : "memory", "m0");
 }
 
 template <bool kCausal>
@@ -130,13 +128,12 @@ void bwd_dq_tile_kernel(const BwdParams p, const TileExtra x) {
     const int64_t slot0 = static_cast<int64_t>(h_kv) * p.n_slots + image_slot0(p.cu_seqlens_k, b);
     const elem_bits* kimg = p.kimg + slot0 * kImageElems;
     const elem_bits* vimg = p.vimg_r + slot0 * kImageElems;
-    const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)smem_raw));
-    const uint32_t ring_base = __builtin_amdgcn_readfirstlane(lds0 + wave * 4096);  // this wavefront copies a quarter of every image
+    const uint32_t ring_base = __builtin_amdgcn_readfirstlane(lds_address_of(smem_raw) + wave * 4096);  // this wavefront copies a quarter of every image
     // the unit that lands in this lane's place of a kilobyte
     const uint32_t dma_lane = static_cast<uint32_t>(((lane >> 4) * 16 + (((lane & 15) - 4 * (lane >> 4)) & 15)) * 16);
     auto issue_part = [&](int block, int slot, int part) {     // 1 KiB of 8
         const elem_bits* src = (part < 4 ? kimg : vimg) + static_cast<int64_t>(Walk::index(block)) * kImageElems + wave * 2048 + (part & 3) * 512;
-        dq_dma_1k(src, dma_lane, ring_base + slot * kSlotBytes + (part >> 2) * (kSlotBytes / 2) + (part & 3) * 1024);
+        dma_copy_1k(src, dma_lane, ring_base + slot * kSlotBytes + (part >> 2) * (kSlotBytes / 2) + (part & 3) * 1024);
     };
     auto issue = [&](int block, int slot) {
 #pragma unroll
@@ -452,9 +449,9 @@ bool dq_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_
                   int most_selected) {
     if (most_selected != kNoMask) return most_selected < 0 && (group == 8 || most_selected <= -16);
     if (max_seqlen_q <= 0 || max_seqlen_k <= 0) return false;
-    const double tiles = masked_walk_time(kTileRows >> tile_row_shift(group), [](double b) { return 18. + 2.3 * b; }, 0.5, batch, num_heads_k,
-                                          total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
-    const double groups = masked_walk_time(8, [](double b) { return 8. + 1.6 * b; }, 0.7, batch, num_heads_k, total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
+    const double tiles = walk_time(kTileRows >> tile_row_shift(group), [](double b) { return 18. + 2.3 * b; }, 0.5, batch, num_heads_k, total_q, total_k, max_seqlen_q,
+                                   max_seqlen_k, causal);
+    const double groups = walk_time(8, [](double b) { return 8. + 1.6 * b; }, 0.7, batch, num_heads_k, total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
     return tiles < 0.93 * groups;
 }
 

@@ -326,7 +326,7 @@ void stage2_fwd_tile_kernel(const FwdParams p, const TileExtra x) {
         }
     };
     const int full = (1 << 2 * per_half) - 1;
-    if ((every >> kTokenBits & full) != full) {             // uniform per wavefront: a block was walked for some rows only
+    if ((every >> kTokenBits & full) != full) {                            // uniform per wavefront: a block was walked for some rows only
         // An infinity or a NaN in a block passes to rows that did not select it (0 x inf).  Where the result shows one, this wavefront's tokens are
         // walked once more, one at a time and each over its own blocks alone.
         float sum = l[0] + l[1];
@@ -392,27 +392,6 @@ void stage2_fwd_tile_kernel(const FwdParams p, const TileExtra x) {
     for (int hf = 0; hf < 2; ++hf) store(o[hf], m[hf], l[hf], hf, true);
 }
 
-// Time of a dense launch whose workgroups take `tokens` tokens each, one workgroup per CU at a time: in microseconds, but for what all
-// launches share.  A workgroup costs `fixed` and `block` per key block; a launch takes as long as its longest walk, or as the
-// work of all of them on 256 CUs with a last round that is `partial` of one more; workgroups behind the end of a sequence, which
-// return at once, 1.7 ns each.  The host knows the longest sequence and the totals: the others are taken to be of equal length.
-static double dense_walk_time(int tokens, double fixed, double block, double partial, int batch, int num_heads_k, int64_t total_q,
-                              int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal) {
-    auto blocks = [&](double q, double k) {                    // of a workgroup of a sequence, on average
-        const double first = causal ? (k > q ? k - q : 0.) : k;
-        return q > tokens ? (first + k) / (2 * kBlockN) + 0.5 : ceil(k / kBlockN);
-    };
-    const int others = batch - 1;
-    const double q = others > 0 && total_q > max_seqlen_q ? static_cast<double>(total_q - max_seqlen_q) / others : 0.;
-    const double k = others > 0 && total_k > max_seqlen_k ? static_cast<double>(total_k - max_seqlen_k) / others : 0.;
-    const double of_longest = ceil(static_cast<double>(max_seqlen_q) / tokens), of_others = others * ceil(q / tokens);
-    const double rounds = num_heads_k * (of_longest + of_others) / 256.;
-    const double each = fixed + block * (of_longest * blocks(max_seqlen_q, max_seqlen_k) + of_others * blocks(q, k)) / (of_longest + of_others);
-    const double chain = fixed + block * ceil(static_cast<double>(max_seqlen_k) / kBlockN);
-    const double all = each * (rounds + (rounds > 1. ? partial : 0.));
-    return (chain > all ? chain : all) + 0.0017 * num_heads_k * batch * of_longest;
-}
-
 // Whether a forward without a mask goes by tiles: a tile walks a block in 1.5 us, the hybrid walk's group of 8 tokens in 1.0, so tiles
 // win where there is more work than the longest chain and lose where that chain, or the rounding up to whole tiles, decides.
 // The constants are a fit to 359 launches of 1 to 300 sequences of 4 to 20000 tokens over up to 16000 keys, 1 to 8 KV heads, groups of 8 and
@@ -423,8 +402,9 @@ static double dense_walk_time(int tokens, double fixed, double block, double par
 //   2 KV heads: 1000 and 3 x 16 tokens 30 * | 39; 4000 and 100 x 16 316 | 233 *; 80 x 24 21 * | 31; 2 x 300 over 6300 keys (4 heads) 209 | 163 *
 bool dense_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal) {
     if (max_seqlen_q <= 0) return false;
-    const double tiles = dense_walk_time(kTileRows >> tile_row_shift(group), 10., 1.5, 0.75, batch, num_heads_k, total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
-    const double groups = dense_walk_time(8, 6., 1., 0.7, batch, num_heads_k, total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
+    const double tiles = walk_time(kTileRows >> tile_row_shift(group), [](double b) { return 10. + 1.5 * b; }, 0.75, batch, num_heads_k, total_q, total_k, max_seqlen_q,
+                                   max_seqlen_k, causal);
+    const double groups = walk_time(8, [](double b) { return 6. + b; }, 0.7, batch, num_heads_k, total_q, total_k, max_seqlen_q, max_seqlen_k, causal);
     return tiles < groups + 1.;
 }
 

@@ -143,8 +143,8 @@ struct TileWalk {
 // that is `partial` of one more; workgroups behind the end of a sequence, which return at once, 1.7 ns each.  The host knows the longest sequence
 // and the totals: the others are taken to be of equal length.
 template <typename Cost>
-static double masked_walk_time(int tokens, Cost cost, double partial, int batch, int num_heads_k, int64_t total_q, int64_t total_k,
-                               int max_seqlen_q, int max_seqlen_k, bool causal) {
+static double walk_time(int tokens, Cost cost, double partial, int batch, int num_heads_k, int64_t total_q, int64_t total_k, int max_seqlen_q,
+                        int max_seqlen_k, bool causal) {
     auto mean = [&](double q, double k) {                      // over the workgroups of a sequence
         const double first = causal ? (k > q ? k - q : 0.) : k;
         if (q <= tokens) return cost(ceil(k / kBlockN));
