@@ -25,7 +25,10 @@ def test_window_blocks(lens, positions, heads, local, init, block):
     assert torch.equal(idx, want_idx) and torch.equal(mask, want_mask)
 
 
-@pytest.mark.parametrize("lens, Hk, group, local, init", [([40000], 1, 16, 4, 1), ([66000, 33], 1, 8, 2, 0), ([700, 9000, 65], 2, 16, 31, 1), ([5000], 2, 8, 80, 66)])
+WINDOWS = [([40000], 1, 16, 4, 1), ([66000, 33], 1, 8, 2, 0), ([700, 9000, 65], 2, 16, 31, 1), ([5000], 2, 8, 80, 66)]   # lengths, KV heads, group, local, init
+
+
+@pytest.mark.parametrize("lens, Hk, group, local, init", WINDOWS)
 def test_windows_by_tiles(lens, Hk, group, local, init):
     """Told that neighbouring rows are alike, forward and dQ go by tiles, whose walk jumps over the words between the first blocks and the window (more than
     eight of them in the first two cases): against the walk per token on the same mask."""
@@ -49,3 +52,37 @@ def test_windows_by_tiles(lens, Hk, group, local, init):
         assert (a.float() - b.float()).norm() <= 2.0 ** -7 * b.float().norm(), name
         rows = (a.float() - b.float()).norm(dim=-1) - 2.0 ** -4 * b.float().norm(dim=-1)
         assert rows.max() <= 1e-2, (name, rows.max().item())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens, Hk, group, local, init", WINDOWS)
+def test_layer_window_against_fp32_attention(lens, Hk, group, local, init, dtype):
+    """Output and dQ of the layer's window branch on sampled tokens (the edges of sequences, of the first blocks, of mask words, of tiles and some at random) against
+    fp32 softmax attention over exactly the window's keys; tolerances of the forward and backward tests: 2e-2 and 1e-3 of values of order one."""
+    import infllmv2_cuda_impl_amd as ops
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    total, mx = sum(lens), max(lens)
+    rand = lambda h: torch.randn(total, h, 128, generator=gen, device="cuda").to(dtype)
+    q, k, v, dout = rand(group * Hk).requires_grad_(True), rand(Hk), rand(Hk), rand(group * Hk)
+    cu = torch.tensor([sum(lens[:i]) for i in range(len(lens) + 1)], dtype=torch.int32, device="cuda")
+    out = ops.InfLLMv2Attention(local_blocks=local, init_blocks=init, selection="window")(q, k, v, cu, mx)
+    dq, = torch.autograd.grad(out, q, dout)
+    start, worst = 0, []
+    for n in lens:
+        near = [0, 1, 15, 16, 31, 63, 64, 65, 64 * (local + 1) - 1, 64 * (local + 1), 64 * (local + init + 1), 64 * (local + init + 1) + 15, 4095, 4096, n - 17, n - 2, n - 1]
+        tokens = sorted({t for t in near if 0 <= t < n} | set(torch.randint(0, n, (24,), generator=torch.Generator().manual_seed(n)).tolist()))
+        for t in tokens:
+            at = torch.arange(t + 1, device="cuda")
+            at = at[(at // 64 < init) | (at // 64 >= t // 64 - local)]
+            kk, vv = k[start + at].float().transpose(0, 1).contiguous(), v[start + at].float().transpose(0, 1).contiguous()        # (Hk, keys, 128)
+            qq, do = (x[start + t].detach().float().view(Hk, group, 128) for x in (q, dout))
+            p = torch.softmax(qq @ kk.transpose(1, 2).contiguous() * 128 ** -0.5, 2)
+            ref = p @ vv
+            dp = do @ vv.transpose(1, 2).contiguous()
+            ref_dq = (p * (dp - (p * dp).sum(2, keepdim=True)) * 128 ** -0.5) @ kk
+            worst.append(torch.stack([x for a, b in ((out, ref), (dq, ref_dq)) for e in [(a[start + t].detach().float().view(Hk, group, 128) - b).abs()]
+                                      for x in (e.max(), e.mean())]))
+        start += n
+    worst = torch.stack(worst)
+    assert worst[:, 0].max() <= 2e-2 and worst[:, 1].mean() <= 1e-3, worst.max(0).values.tolist()
+    assert worst[:, 2].max() <= 2e-2 and worst[:, 3].mean() <= 1e-3, worst.max(0).values.tolist()
