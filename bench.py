@@ -36,7 +36,7 @@ FLOPS_PER_BLOCK = 4 * 16 * 64 * 128
 # the Stage-2 forward kernel's HBM traffic cannot be read from inside this process (rocprofv3 --pmc counters); it is
 # taken from the tracked summary below, which names the sources it was measured on by their hash
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "stage2_fwd_config2_hbm_traffic.md")
-FWD_KERNEL_SOURCES = ["stage2_fwd_hybrid.hip", "stage2_fwd.hip", "stage2_fwd.h", "kv_image.h", "block_walker.h", "common.h"]
+FWD_KERNEL_SOURCES = ["stage2_fwd_hybrid.hip", "stage2_fwd.hip", "stage2_fwd.h", "kv_image.h", "block_walker.h", "lds_dma.h", "in_step.h", "common.h"]
 
 
 def fwd_kernel_source_hash() -> str:

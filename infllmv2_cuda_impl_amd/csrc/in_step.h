@@ -9,6 +9,11 @@
 // The wait is a matter of speed only: nothing depends on which workgroups run at once, a workgroup of an earlier generation never
 // waits for a later one, and a wait ends after kInStepPolls looks whatever the counters hold.
 //
+// With the device shared a generation is more than an XCD runs at once, and CUs that become free wait for its second half.  What sharing fetches gives is still
+// more than that costs; forward in ms, in step | not, 2 KV heads, 64 blocks selected, as many as keep both streams busy: 65 536 tokens alone 6.9 | 9.5, two such forwards on two
+// streams (time of both) 19.5 | 25.0, beside products of 8192^3 14.8 | 16.7, beside copies of 0.5 GiB 14.1 | 15.5, beside products of 64 rows 10.7 | 10.7; 131 072: 19.2 | 24.7,
+// 50.2 | 57.6, 38.2 | 41.1, 32.9 | 37.0, 21.5 | 25.6; 40 000: 3.6 | 3.8, 9.4 | 12.4, 7.5 | 7.7, 6.5 | 6.8, 5.4 | 5.4.
+//
 // Which launches: at 30 000 tokens a whole prefill gained 1 % and at 32 768 it gained or lost less (L2 serves 91 % of the requests
 // there and the wait for a generation's slowest workgroup costs 2 %); at 40 000 it gained 7 %, at 49 152 14, at 65 536 22 (10.9 -> 8.5 ms,
 // two KV heads), at 98 304 20, at 131 072 17 (31.3 -> 25.9).  Only wavefronts whose row has blocks of its own in
