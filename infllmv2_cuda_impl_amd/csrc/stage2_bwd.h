@@ -49,7 +49,7 @@ constexpr int kNoMask = 0x7fffffff;
 bool dq_tiles_pay(int batch, int num_heads_k, int group, int64_t total_q, int64_t total_k, int max_seqlen_q, int max_seqlen_k, bool causal,
                   int most_selected);
 int launch_bwd_dq_tile(hipStream_t st, const BwdParams& p, int batch, int max_seqlen_q, bool causal);
-// dK/dV, two wavefronts (32 keys each) per (64-key block, 512-token slice): stage2_bwd_dkdv.hip
+// dK/dV, two wavefronts (32 keys each) per work item of a 64-key block: stage2_bwd_dkdv.hip
 // most_selected: as in infllmv2_varlen_bwd_selected
 int launch_bwd_dkdv_wave(hipStream_t st, const BwdParams& p, int batch, int max_seqlen_q, int max_seqlen_k, bool causal, int most_selected);
 

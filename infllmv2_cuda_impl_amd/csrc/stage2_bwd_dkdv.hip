@@ -1,5 +1,5 @@
-// Stage-2 backward, dK / dV (gfx950): two wavefronts per (64-key block, slice of 512 or 128 query tokens), each owning
-// 32 of the keys.
+// Stage-2 backward, dK / dV (gfx950): two wavefronts per work item, each owning 32 keys of a 64-key block.  An item is a block and some query tokens that
+// selected it: those of a slice of 512 or 128 (merged with its neighbours' where they are few), or for short inputs an even share of those of 2048 tokens.
 //
 // Mathematics as in compute_dq_dk_dv_1colblock (csrc/flash_attn/src/flash_bwd_kernel.h:498-794):
 // P = exp(scale S - LSE), dV += P^T dO, dS = P (dP - D), dK += scale dS^T Q, the 16 grouped heads
@@ -613,9 +613,10 @@ static int launch_bwd_dkdv_sliced(hipStream_t st, const BwdParams& p_in, int bat
     }
     if (kColSlice < kDkdvSlice && (all_groups < 12 || max_seqlen_q > 4096)) {
         // Short slices: where the groups are few or differ (the first tokens of a sequence select less), sharing pays beyond even
-        // division.  Whole training pass in us with 1 / 2 / 4 / 8 sharers: 6000 tokens (3 groups) 2610 / 1810 / 1560 / 1500, 8000 (4)
-        // 2330 / 2330 / 2190 / 2160, the same with 16 blocks selected - / 980 / 1025 / 1130, 12000 + 9000 (11) 7360 / 6490 / 5960 /
-        // 6000, 3 x 12000 (18) 2180 / 2100 / 2045 / 2390; but 10 x 3000 (15) 2790 / 2790 / 2940 / 2950.
+        // division.  Items dealt out evenly, whole backward in us with 1 / 2 / 4 / 8 sharers: 2048 tokens, 16 blocks selected (1 group) 503 / 301 / 217 / 161,
+        // 3000 (2) 504 / 333 / 269 / 227, 1023 + 3001 + 517 + 2200 (4) 692 / 501 / 419 / 431, 12000 (6) 1053 / 1020 / 915 / 949; 64 blocks selected: 6000 tokens (3) 2163 /
+        // 1389 / 1103 / 1032, 8000 (4) 2583 / 1716 / 1574 / 1543, 12000 + 9000 (11) 5833 / 4682 / 4663 / 4557, 28000 (14) 7717 / 7168 / 6985 / 7134; 6 x 3000, 32 blocks (9)
+        // 1936 / 1703 / 1656 / 1680.  Slices as items, whole training pass: 3 x 12000 (18) 2180 / 2100 / 2045 / 2390; but 10 x 3000 (15) 2790 / 2790 / 2940 / 2950.
         p.dkdv_share = all_groups <= 3 ? 8 : 4;
     }
     const int teams = 8 / p.dkdv_share;

@@ -15,7 +15,7 @@
 //
 // The kernel also forms D = rowsum(dO * O) (compute_dot_do_o, flash_bwd_preprocess_kernel.h:56-137): it has dO in registers, and O
 // costs its set-up one more request.  A pass of its own read dO and O once more from HBM: 227 us of 22.7 ms for 71552 packed tokens, 18 of 680 for
-// 6741 in four sequences (whole training passes 22970 -> 22740 and 680 -> 660).  Its row scalars go to the dK/dV kernel.
+// 6741 in four sequences (whole training pass of the latter 680 -> 660; of the former inside the spread of its runs).  Its row scalars go to the dK/dV kernel.
 //
 // What bounds it: the chain S, dP, dQ of a block in two wavefronts per SIMD that the turn's barrier keeps in step.  At 32768
 // tokens, 64 blocks per row and 2 KV heads (3.65 to 3.9 ms) the matrix pipe is busy 39 % and the return path from L2, as in the

@@ -7,7 +7,7 @@
 // the same block images, through an LDS ring of three blocks.
 //
 // What bounds it: the power the matrix pipe draws.  16384 dense tokens of 2 KV heads take 1825 us (1.2 PFLOP/s) with random inputs and 1460 with zeros,
-// where only the clock differs; a library product of 8192^3 makes 1.38 and 1.79 PFLOP/s.  What a step does beside the MFMAs counts in energy more than in
+// where only the clock differs; a library product of 8192^3 in bf16 makes 1.40 and 1.80 PFLOP/s with both operands in rows, 1.62 and 2.25 with the right one transposed.  What a step does beside the MFMAs counts in energy more than in
 // issue slots, and the operand reads from LDS are the largest part: so a wavefront takes 64 rows, in two halves of 32 (the N side of
 // v_mfma_f32_32x32x16), and a fragment feeds both.  That is one wavefront per SIMD with 512 registers (128 of O, 64 each of Q, S, K and V, 32 of P),
 // and the overlap of MFMAs and exponentials is written out: while one half's P V and scores are on the matrix pipe, the other half's exponentials are
