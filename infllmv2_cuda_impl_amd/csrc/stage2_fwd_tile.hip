@@ -6,13 +6,13 @@
 // heads, 32 of 8) and walks the blocks that any of its tokens selected; a row that did not select one has P = 0 there.  K and V come from
 // the same block images, through an LDS ring of three blocks.
 //
-// What bounds it: the power the matrix pipe draws.  16384 dense tokens of 2 KV heads take 1825 us (1.2 PFLOP/s) with random inputs and 1460 with zeros,
-// where only the clock differs; a library product of 8192^3 in bf16 makes 1.40 and 1.80 PFLOP/s with both operands in rows, 1.62 and 2.25 with the right one transposed.  What a step does beside the MFMAs counts in energy more than in
-// issue slots, and the operand reads from LDS are the largest part: so a wavefront takes 64 rows, in two halves of 32 (the N side of
-// v_mfma_f32_32x32x16), and a fragment feeds both.  That is one wavefront per SIMD with 512 registers (128 of O, 64 each of Q, S, K and V, 32 of P),
-// and the overlap of MFMAs and exponentials is written out: while one half's P V and scores are on the matrix pipe, the other half's exponentials are
-// formed.  Before, eight wavefronts of 32 rows, two to a SIMD, read twice the LDS bytes: 1910 us; four wavefronts of 32 rows in
-// workgroups of two to a CU 1993; this shape with copies and scalar work at the head of a step instead of between its MFMAs 1979.
+// What bounds it: the power the matrix pipe draws.  16384 dense tokens of 2 KV heads take 1825 us (1.2 PFLOP/s) with random inputs and 1460 with zeros, where
+// only the clock differs; a library product of 8192^3 in bf16 makes 1.40 and 1.80 PFLOP/s with both operands in rows, 1.62 and 2.25 with the right one
+// transposed.  What a step does beside the MFMAs counts in energy more than in issue slots, and the operand reads from LDS are the largest part: so a
+// wavefront takes 64 rows, in two halves of 32 (the N side of v_mfma_f32_32x32x16), and a fragment feeds both.  That is one wavefront per SIMD with 512
+// registers (128 of O, 64 each of Q, S, K and V, 32 of P), and the overlap of MFMAs and exponentials is written out: while one half's P V and scores are on
+// the matrix pipe, the other half's exponentials are formed.  Before, eight wavefronts of 32 rows, two to a SIMD, read twice the LDS bytes: 1910 us; four
+// wavefronts of 32 rows in workgroups of two to a CU 1993; this shape with copies and scalar work at the head of a step instead of between its MFMAs 1979.
 // Operator, us, eight wavefronts -> this one: 2500 + 6001 + 4096 tokens 481 -> 455, 777 + 5003 + 1291 + 9173 865 -> 816, 50000 17000 -> 16600.
 //
 // Operands.  S^T = K Q^T: lane (n = lane % 32, h = lane / 32) holds key n of a 32-key chunk, d = 16 ks + 8 h + j: one 16-byte unit of
