@@ -9,12 +9,22 @@
 // The wait is a matter of speed only: nothing depends on which workgroups run at once, a workgroup of an earlier generation never
 // waits for a later one, and a wait ends after kInStepPolls looks whatever the counters hold.
 //
-// With the device shared a generation is more than an XCD runs at once, and CUs that become free wait for its second half.  What sharing fetches gives is still
-// more than that costs; forward in ms, in step | not, 2 KV heads, 64 blocks selected, as many as keep both streams busy: 65 536 tokens alone 6.9 | 9.5, two such forwards on two
-// streams (time of both) 19.5 | 25.0, beside products of 8192^3 14.8 | 16.7, beside copies of 0.5 GiB 14.1 | 15.5, beside products of 64 rows 10.7 | 10.7; 131 072: 19.2 | 24.7,
-// 50.2 | 57.6, 38.2 | 41.1, 32.9 | 37.0, 21.5 | 25.6; 40 000: 3.6 | 3.8, 9.4 | 12.4, 7.5 | 7.7, 6.5 | 6.8, 5.4 | 5.4.
+// Started together is not enough: a row's own blocks lie where they lie, and after as many of them two rows are up to a fifth of the sequence apart (131 072
+// tokens, 31 blocks of a row's own: standard deviation 9 % in the middle, 180 blocks of 32 KiB), while L2 holds 128 blocks.  So the walk is paced too: the blocks that a group of 8
+// tokens has in common, walked in lock step, are its clock.  Behind each of them come kPacedSteps steps for a block of a wavefront's own, and a wavefront takes its next block in a
+// step only if the block lies before a front that crosses the group's keys evenly in the steps there are - or if it has a block left for every
+// step left, so that no row ends later for it, wherever its blocks lie.  With two steps to a common block a row has twice as many as blocks of its own, is rarely
+// held up, and passes a block when the others do.  The rule looks at the group's rows alone: the order in which a row's blocks are added up,
+// and with it the result's bits, are the same in every launch.  131 072 tokens, 64 blocks: L2 serves 80 % of the requests instead of 57, 60 GB come from behind it instead of 125,
+// forward 19.4 -> 14.1 ms, whole prefill 26.0 -> 20.9; 65 536: 8.8 -> 7.95; 40 000: 4.5 -> 4.4.  One step to a common block 24.9, 8.6, 4.5, three 20.9, 8.0, 4.4.
+// Groups that end behind block 384: 20.8, 7.9, 4.4; 768: 21.2, 8.2, 4.6.  Below 32 768 keys, waiting and paced or not: within 1 % either way.
 //
-// Which launches: at 30 000 tokens a whole prefill gained 1 % and at 32 768 it gained or lost less (L2 serves 91 % of the requests
+// With the device shared a generation is more than an XCD runs at once, and CUs that become free wait for its second half.  What sharing fetches gives is still
+// more than that costs; forward in ms, in step and paced | in step | neither, 2 KV heads, 64 blocks selected (the first, a window of 32, the rest anywhere), as many as keep both
+// streams busy: 131 072 tokens alone 13.2 | 18.4 | 24.9, two such forwards on two streams (time of one) 40.7 | 49.7 | 60.5, beside products of 8192^3 45.7 | 51.3 | 53.4, beside
+// copies of 0.5 GiB 29.9 | 31.6 | 35.9, beside products of 64 rows 24.0 | 26.8 | 29.7; 40 000: 3.3 | 3.4 | 3.6, 8.1 | 8.9 | 11.8, 10.4 | 10.7 | 11.4, 7.4 | 7.4 | 7.2, 4.9 | 5.1 | 5.6.
+//
+// Which launches (measured before there was a pace): at 30 000 tokens a whole prefill gained 1 % and at 32 768 it gained or lost less (L2 serves 91 % of the requests
 // there and the wait for a generation's slowest workgroup costs 2 %); at 40 000 it gained 7 %, at 49 152 14, at 65 536 22 (10.9 -> 8.5 ms,
 // two KV heads), at 98 304 20, at 131 072 17 (31.3 -> 25.9).  Only wavefronts whose row has blocks of its own in
 // several mask words wait: with window masks everything is shared (60 000 tokens, 6 blocks: 473 us without all this, 478 with the counters and no waits).  Letting up to 8 workgroups of a
@@ -29,6 +39,8 @@ namespace IV2_NS {
 constexpr int kGeneration = 32;
 constexpr int kInStepKeys = 32768;                             // sequences with more keys than this
 constexpr int kInStepWords = 4;                                // and rows with blocks of their own in at least so many mask words
+constexpr int kPacedBlocks = kInStepKeys / kBlockN;            // groups that reach beyond so many blocks are paced, in every launch that can hold such a group
+constexpr int kPacedSteps = 2;
 constexpr int kInStepPolls = 256;                              // of about a microsecond each
 constexpr int kInStepPitch = 32;                               // the XCDs' counters lie 128 bytes apart
 constexpr size_t kInStepBytes = 8 * kInStepPitch * sizeof(unsigned);

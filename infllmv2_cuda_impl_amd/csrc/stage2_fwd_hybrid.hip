@@ -22,7 +22,7 @@
 // Workgroups are numbered so that each of the 8 XCDs takes whole chunks of consecutive token
 // groups of one KV head (their L2 sees one head's images and neighbouring local windows), and
 // the longest causal prefixes are scheduled first.
-// Long sequences are walked in step with the other workgroups of the XCD (in_step.h).
+// Long sequences are walked in step with the other workgroups of the XCD, at a given pace (in_step.h).
 #include "common.h"
 #include "kv_image.h"
 #include "block_walker.h"
@@ -115,9 +115,9 @@ __device__ __forceinline__ void softmax_step(floatx4 (&s)[4], float& m, float& l
         }
 }
 
-// kInStep: with the counters of in_step.h; a variant of its own, because a workgroup has its CU to itself and pays for all set-up (the counting alone took
-// 2.6 % where rows are short: 30000 tokens with a window of 9 blocks 536 -> 550 us)
-template <bool kCausal, bool kInStep>
+// kLong: sequences long enough for in_step.h, its counters and its pacing; a variant of its own, because a workgroup has its CU to itself and pays for all
+// set-up (the counting alone took 2.6 % where rows are short: 30000 tokens with a window of 9 blocks 536 -> 550 us)
+template <bool kCausal, bool kLong>
 __global__ __launch_bounds__(512)
 void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -147,7 +147,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     // (All of these are read before the first atomic: behind it the compiler loads them into vector registers, 0.5 us per workgroup.)
     unsigned* finished = x.finished + xcd * kInStepPitch;
     if (i0 >= Sq) {                                                                 // uniform per workgroup
-        if (kInStep && tid == 0) in_step_finished(finished);
+        if (kLong && tid == 0 && x.finished) in_step_finished(finished);
         return;
     }
 
@@ -246,8 +246,27 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
 #pragma unroll
         for (int f = 0; f < 16; ++f) kreg[f] = *reinterpret_cast<const elem8*>(src + f * 512);
     }
-    if constexpr (kInStep) {
-        if (Sk > kInStepKeys) {                                // uniform
+    // Pacing (in_step.h): steps for own blocks per common block, the steps and own blocks that are left, and the block the walk may reach by now
+    // in 1/256.  With these values there is none: own_left and steps_left count down together.
+    int steps = 1, steps_left = 0, own_left = 0, front = 0, front_step = 0;
+    if constexpr (kLong) {
+        int last = i0 + kHybTokens - 1 < Sq ? i0 + kHybTokens - 1 : Sq - 1;    // the group's last key block
+        last = (kCausal && last + Sk - Sq < Sk - 1 ? last + Sk - Sq : Sk - 1) >> 6;
+        if (last >= kPacedBlocks) {                            // uniform
+            int count = 0;                                     // blocks in common << 16 | this row's own
+            for (int w = lane; w < nw; w += 64) count += (__builtin_popcountll(com[w]) << 16) + __builtin_popcountll(own[w]);
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) count += __shfl_xor(count, d);
+            count = __builtin_amdgcn_readfirstlane(count);
+            if (count >> 16) {
+                steps = kPacedSteps;
+                steps_left = (count >> 16) * kPacedSteps;
+                own_left = count & 0xffff;
+                front_step = ((last + 1) << 8) / steps_left;
+                front = front_step;
+            }
+        }
+        if (Sk > kInStepKeys && x.finished) {                  // uniform
             int words = 0;                                     // with blocks of this row's own
             for (int w = 0; w < nw; w += 64) words += __builtin_popcountll(__builtin_amdgcn_ballot_w64(w + lane < nw && own[w + lane] != 0ull));
             if (words >= kInStepWords) in_step_wait(finished, sidx);
@@ -269,7 +288,8 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     if (c0 >= 0) issue(c0, 0);
     if (c1 >= 0) issue(c1, 1);
     int half = 0;
-    bool k_ahead = false;                                      // the coming own block's 16 K-fragment loads were issued already
+    bool k_ready = jp >= 0;                                    // the coming own block's K fragments are in registers or on their way
+    bool k_ahead = false;                                      // ... and were requested after the last DMA
     auto common_part = [&](int j0, int tile) {
         // all 16 fragments of a tile are fetched before the MFMAs that use them (vreg is free between own
         // blocks), and the MFMAs run over independent accumulators first
@@ -302,35 +322,46 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
                 o[dt] = IV2_MFMA(vreg[dt * 2 + cc], pf[cc], o[dt], 0, 0, 0);
     };
     auto own_part = [&]() {
-        {
+        if (!kLong || k_ready) {
             const elem_bits* src = vimg + static_cast<int64_t>(jp) * kImageElems;
 #pragma unroll
             for (int f = 0; f < 16; ++f) vreg[f] = *reinterpret_cast<const elem8*>(src + f * 512);
+            floatx4 s[4];
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) s[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt)
+                    s[kt] = IV2_MFMA(kreg[kt * 4 + c], qf[c], s[kt], 0, 0, 0);
+            elem8 pf[2];
+            softmax_step(s, m, l, o, pf, (jp == last_blk) ? last_key - jp * kBlockN : kBlockN, g, p.scale_log2);
+#pragma unroll
+            for (int cc = 0; cc < 2; ++cc)
+#pragma unroll
+                for (int dt = 0; dt < 8; ++dt)
+                    o[dt] = IV2_MFMA(vreg[dt * 2 + cc], pf[cc], o[dt], 0, 0, 0);
+            jp = next_own();
+            k_ready = k_ahead = false;
+            if constexpr (kLong) --own_left;
         }
-        floatx4 s[4];
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) s[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int kt = 0; kt < 4; ++kt)
-                s[kt] = IV2_MFMA(kreg[kt * 4 + c], qf[c], s[kt], 0, 0, 0);
-        elem8 pf[2];
-        softmax_step(s, m, l, o, pf, (jp == last_blk) ? last_key - jp * kBlockN : kBlockN, g, p.scale_log2);
-#pragma unroll
-        for (int cc = 0; cc < 2; ++cc)
-#pragma unroll
-            for (int dt = 0; dt < 8; ++dt)
-                o[dt] = IV2_MFMA(vreg[dt * 2 + cc], pf[cc], o[dt], 0, 0, 0);
-        const int jn = next_own();
-        k_ahead = false;
-        if (jn >= 0) {                                         // K fragments of the next own block
-            const elem_bits* src = kimg + static_cast<int64_t>(jn) * kImageElems;
+        if constexpr (kLong) {
+            if (steps_left > 0) front += front_step;           // (no overflow: a walk may go on for long after its last step)
+            --steps_left;
+        }
+        if (jp >= 0 && (!kLong || jp < (front >> 8) || own_left >= steps_left)) {   // K fragments of the next own block
+            const elem_bits* src = kimg + static_cast<int64_t>(jp) * kImageElems;
 #pragma unroll
             for (int f = 0; f < 16; ++f) kreg[f] = *reinterpret_cast<const elem8*>(src + f * 512);
-            k_ahead = true;
+            k_ready = k_ahead = true;
         }
-        jp = jn;
+    };
+    auto own_parts = [&]() {
+        own_part();
+        if constexpr (kLong) {
+#pragma unroll 1
+            for (int r = 1; r < steps && jp >= 0; ++r) own_part();
+        }
     };
     while (c0 >= 0 || jp >= 0) {
         int n0 = -1, n1 = -1;
@@ -345,16 +376,16 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
             if (n1 >= 0) issue(n1, 3 - 2 * half);
             if (live) common_part(c0, 2 * half);
         }
-        if (jp >= 0) own_part();                               // per wavefront
+        if (jp >= 0) own_parts();                              // per wavefront
         if (c1 >= 0 && live) common_part(c1, 2 * half + 1);
-        if (jp >= 0 && c1 >= 0) own_part();
+        if (jp >= 0 && c1 >= 0) own_parts();
         if (c0 >= 0) {
             c0 = n0;
             c1 = n1;
             half ^= 1;
         }
     }
-    if (kInStep && tid == 0) in_step_finished(finished);       // the first wavefront for its workgroup: its row is one of eight neighbours
+    if (kLong && tid == 0 && x.finished) in_step_finished(finished);       // the first wavefront for its workgroup: its row is one of eight neighbours
     if (share_log2 != 0) {                                     // uniform per workgroup
         // the ring was not used: 34 floats of every lane, lane by lane
         float* mine = reinterpret_cast<float*>(smem_raw) + wave * (34 * 64) + lane;
@@ -417,9 +448,9 @@ int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int 
     const int64_t per_round = 8 * kHybChunk;
     const int64_t grid = (total + per_round - 1) / per_round * per_round;
     const size_t lds = kRingTiles * kTileBytes + static_cast<size_t>(1 + kHybTokens) * x.mask_words * 8;
-    const bool wait = in_step != nullptr;
-    auto kernel = causal ? (wait ? stage2_fwd_hybrid_kernel<true, true> : stage2_fwd_hybrid_kernel<true, false>)
-                         : (wait ? stage2_fwd_hybrid_kernel<false, true> : stage2_fwd_hybrid_kernel<false, false>);
+    const bool far = max_seqlen_k > kInStepKeys;
+    auto kernel = causal ? (far ? stage2_fwd_hybrid_kernel<true, true> : stage2_fwd_hybrid_kernel<true, false>)
+                         : (far ? stage2_fwd_hybrid_kernel<false, true> : stage2_fwd_hybrid_kernel<false, false>);
     x.finished = in_step;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     IV2_CHECK(e == hipSuccess, "varlen_fwd: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
