@@ -11,7 +11,7 @@
 //
 // Started together is not enough: a row's own blocks lie where they lie, and after as many of them two rows are up to a fifth of the sequence apart (131 072
 // tokens, 31 blocks of a row's own: standard deviation 9 % in the middle, 180 blocks of 32 KiB), while L2 holds 128 blocks.  So the walk is paced too: the blocks that a group of 8
-// tokens has in common, walked in lock step, are its clock.  Behind each of them come kPacedSteps steps for a block of a wavefront's own, and a wavefront takes its next block in a
+// tokens walks together, in lock step, are its clock.  Behind each of them come kPacedSteps steps for a block of a wavefront's own, and a wavefront takes its next block in a
 // step only if the block lies before a front that crosses the group's keys evenly in the steps there are - or if it has a block left for every
 // step left, so that no row ends later for it, wherever its blocks lie.  With two steps to a common block a row has twice as many as blocks of its own, is rarely
 // held up, and passes a block when the others do.  The rule looks at the group's rows alone: the order in which a row's blocks are added up,

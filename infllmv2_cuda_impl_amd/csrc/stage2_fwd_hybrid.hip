@@ -5,11 +5,16 @@
 // A workgroup of 8 wavefronts owns 8 consecutive tokens of one sequence and KV head and splits
 // each token's mask row in two:
 //
-//   * the blocks that ALL 8 rows select (for InfLLM-V2 masks: the initial block and the local
-//     window, which neighbouring tokens share) are walked in lock step: every such block is
+//   * the blocks that five or more of the 8 rows select (for InfLLM-V2 masks: the initial block, the local
+//     window, and what neighbouring tokens share beyond) are walked in lock step: every such block is
 //     copied once, by LDS-DMA, from its fragment-major image into a 4-tile LDS ring (two blocks in
-//     use, the next two in flight: one workgroup barrier per two blocks), and each wavefront
+//     use, the next two in flight: one workgroup barrier per two blocks), and each wavefront whose row selects it
 //     reads its MFMA operands with conflict-free ds_read_b128;
+//     Five: a block of the ring costs the vector memory path one fetch and the LDS pipe, twice as wide, one for every row that selects it, a block outside
+//     it the former one for every such row.  From all eight down to six | five | four | three, whole passes in us: one prompt of 2048 tokens with 16 blocks
+//     80.3 -> 79.3 | 77.2 | 77.4 | 80.0; four ragged prompts 1032 -> 1037 | 1023 | 1001 | 1013; training on four short samples 617 -> 614 | 612 | 612 | 617;
+//     2049 queries behind 17962 keys 321.5 -> 322.3 | 322.8 | 328.9 | 330.7; 32768 tokens the same | the same | 1 % more | 9 % more: where rows share
+//     little, wavefronts wait for the few that want a ring block.
 //   * the remaining blocks of a row are walked by its wavefront alone, operands straight from
 //     global memory into registers, as in stage2_fwd_kernel;
 //   * the two walks are interleaved, common, own, common, own per turn: the first is bound by
@@ -167,7 +172,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     const int64_t tok = static_cast<int64_t>(q0) + (live ? i : i0);
     const uint64_t* mrow = p.mask ? p.mask + (static_cast<int64_t>(h) * p.total_q + tok) * p.n64 : nullptr;
 
-    // ---- the row words every live token of the group has in common, and what is left of each row ----
+    // ---- the row words, and which blocks the group walks together ----
     int nw;                                                                          // words that can hold an allowed block of any token
     {
         const int i_last = (i0 + kHybTokens - 1 < Sq) ? i0 + kHybTokens - 1 : Sq - 1;
@@ -177,9 +182,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
         if (mrow && nw > p.n64) nw = p.n64;
         if (nw > x.mask_words) nw = x.mask_words;                                    // a sequence longer than the announced max_seqlen_k
     }
-    unsigned long long* own = rows + wave * x.mask_words;                           // this token's row, later minus the common part
-    for (int w = tid; w < nw; w += 512) com[w] = share_log2 == 0 ? ~0ull : 0ull;   // shared out: no lock step
-    __syncthreads();
+    unsigned long long* own = rows + wave * x.mask_words;                           // this token's row
     for (int w = lane; w < nw; w += 64) {
         uint64_t v = 0ull;
         if (last_blk >= 0 && w <= (last_blk >> 6)) {
@@ -190,12 +193,30 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
             }
         }
         own[w] = v;
-        if (live && v != ~0ull) atomicAnd(&com[w], static_cast<unsigned long long>(v));
+    }
+    __syncthreads();
+    for (int w = tid; w < nw; w += 512) {
+        uint64_t shared = 0ull;
+        if (share_log2 == 0) {
+            // how many of the eight rows select a block, a binary digit to a word: ones, twos (two of each), fours, eights
+            uint64_t r[kHybTokens];
+#pragma unroll
+            for (int t = 0; t < kHybTokens; ++t) r[t] = t < in_group ? rows[t * x.mask_words + w] : ~0ull;
+            auto sum3 = [](uint64_t a, uint64_t b, uint64_t c, uint64_t& carry) { carry = (a & b) | (c & (a | b)); return a ^ b ^ c; };
+            uint64_t t0, t1, t2, t3, f0, f1;
+            const uint64_t s0 = sum3(r[0], r[1], r[2], t0), s1 = sum3(r[3], r[4], r[5], t1), s2 = sum3(r[6], r[7], s0, t2);
+            const uint64_t ones = s1 ^ s2;
+            t3 = s1 & s2;
+            const uint64_t u = sum3(t0, t1, t2, f0), twos = u ^ t3;
+            f1 = u & t3;
+            const uint64_t fours = f0 ^ f1, eights = f0 & f1;
+            shared = in_group < kHybTokens ? eights : eights | (fours & (twos | ones));     // all of them, or five of eight
+        }
+        com[w] = shared;
     }
     __syncthreads();
     const uint64_t columns = (share_log2 == 0 ? ~0ull : share_log2 == 1 ? 0x5555555555555555ull
                               : share_log2 == 2 ? 0x1111111111111111ull : 0x0101010101010101ull) << part;
-    for (int w = lane; w < nw; w += 64) own[w] &= ~com[w] & columns;
 
     // ---- Q operand ----
     elem8 qf[4];
@@ -218,20 +239,22 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     const uint32_t ring_base = __builtin_amdgcn_readfirstlane(lds_address_of(ring) + wave * 4096);
     auto issue = [&](int jj, int tile) { dma_copy_4k(src_lane + static_cast<int64_t>(jj) * 1024, ring_base + tile * kTileBytes); };
     int cw = -1, ow = -1;
-    uint64_t cbits = 0ull, obits = 0ull;
-    auto next_common = [&]() -> int {
+    uint64_t cbits = 0ull, crow = 0ull, obits = 0ull;
+    auto next_common = [&](bool& mine) -> int {
         while (cbits == 0ull) {
             if (++cw >= nw) return -1;
             cbits = uniform_u64(com[cw]);
+            crow = uniform_u64(own[cw]);
         }
         const int bit = __builtin_ctzll(cbits);
+        mine = (crow >> bit) & 1ull;
         cbits &= cbits - 1ull;
         return cw * 64 + bit;
     };
     auto next_own = [&]() -> int {
         while (obits == 0ull) {
             if (++ow >= nw) return -1;
-            obits = uniform_u64(own[ow]);
+            obits = uniform_u64(own[ow] & ~com[ow] & columns);
         }
         const int bit = __builtin_ctzll(obits);
         obits &= obits - 1ull;
@@ -253,8 +276,8 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
         int last = i0 + kHybTokens - 1 < Sq ? i0 + kHybTokens - 1 : Sq - 1;    // the group's last key block
         last = (kCausal && last + Sk - Sq < Sk - 1 ? last + Sk - Sq : Sk - 1) >> 6;
         if (last >= kPacedBlocks) {                            // uniform
-            int count = 0;                                     // blocks in common << 16 | this row's own
-            for (int w = lane; w < nw; w += 64) count += (__builtin_popcountll(com[w]) << 16) + __builtin_popcountll(own[w]);
+            int count = 0;                                     // blocks walked together << 16 | this row's own
+            for (int w = lane; w < nw; w += 64) count += (__builtin_popcountll(com[w]) << 16) + __builtin_popcountll(own[w] & ~com[w]);
 #pragma unroll
             for (int d = 1; d < 64; d <<= 1) count += __shfl_xor(count, d);
             count = __builtin_amdgcn_readfirstlane(count);
@@ -268,7 +291,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
         }
         if (Sk > kInStepKeys && x.finished) {                  // uniform
             int words = 0;                                     // with blocks of this row's own
-            for (int w = 0; w < nw; w += 64) words += __builtin_popcountll(__builtin_amdgcn_ballot_w64(w + lane < nw && own[w + lane] != 0ull));
+            for (int w = 0; w < nw; w += 64) words += __builtin_popcountll(__builtin_amdgcn_ballot_w64(w + lane < nw && (own[w + lane] & ~com[w + lane]) != 0ull));
             if (words >= kInStepWords) in_step_wait(finished, sidx);
         }
     }
@@ -283,8 +306,9 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     for (int f = 0; f < 16; ++f) asm volatile("" : "+v"(kreg[f]));
     // The common blocks go through the ring in pairs: tiles {0, 1} and {2, 3} alternate, the pair after the current
     // one is in flight, and one workgroup barrier serves two blocks.
-    int c0 = next_common();
-    int c1 = c0 >= 0 ? next_common() : -1;
+    bool mine0 = false, mine1 = false;                         // whether this row selects them
+    int c0 = next_common(mine0);
+    int c1 = c0 >= 0 ? next_common(mine1) : -1;
     if (c0 >= 0) issue(c0, 0);
     if (c1 >= 0) issue(c1, 1);
     int half = 0;
@@ -365,23 +389,26 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     };
     while (c0 >= 0 || jp >= 0) {
         int n0 = -1, n1 = -1;
+        bool next_mine0 = false, next_mine1 = false;
         if (c0 >= 0) {                                         // uniform over the workgroup
             // younger than this wavefront's DMA loads of the pair: the 16 K loads of the coming own block
             if (k_ahead) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
             else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();                                   // the pair is in LDS for everyone; the other two tiles are free
-            n0 = c1 >= 0 ? next_common() : -1;
-            n1 = n0 >= 0 ? next_common() : -1;
+            n0 = c1 >= 0 ? next_common(next_mine0) : -1;
+            n1 = n0 >= 0 ? next_common(next_mine1) : -1;
             if (n0 >= 0) issue(n0, 2 - 2 * half);
             if (n1 >= 0) issue(n1, 3 - 2 * half);
-            if (live) common_part(c0, 2 * half);
+            if (mine0) common_part(c0, 2 * half);
         }
         if (jp >= 0) own_parts();                              // per wavefront
-        if (c1 >= 0 && live) common_part(c1, 2 * half + 1);
+        if (c1 >= 0 && mine1) common_part(c1, 2 * half + 1);
         if (jp >= 0 && c1 >= 0) own_parts();
         if (c0 >= 0) {
             c0 = n0;
             c1 = n1;
+            mine0 = next_mine0;
+            mine1 = next_mine1;
             half ^= 1;
         }
     }
