@@ -18,6 +18,12 @@
 // wavefronts x 2 consecutive tokens; each 64-key tile of compressed keys is staged once in LDS
 // (LDS-DMA, straight into MFMA-operand order, read back with conflict-free ds_read_b128) and reused
 // by all 16 tokens, and inside a wavefront one operand read feeds two MFMAs.
+//
+// Bound by vector instructions (the vector pipe was 80 % busy, the matrix pipe 42 %) and by power: what is saved in instructions is half lost to a lower
+// clock.  Tiles without a test, offsets in scalar registers, DPP maxima spelled out and results stored a tile later took them from 163 to 126 per 64
+// fine keys and two tokens; pooled, two KV heads, us: 131 072 tokens 5800 -> 5580, 32 768 428 -> 415, 9173 62 -> 60; 2049 queries against 20 011 keys 60.3 -> 58.5.
+// With 32-row MFMAs and plain sums in pass 1: 5470, 407, 59, 54, but sums in another order round some scores to the neighbouring 16-bit value, and
+// single rows then attend another block.
 #include "common.h"
 #include "block_walker.h"
 #include "infllmv2_hip.h"
@@ -68,6 +74,7 @@ __device__ __forceinline__ int stage1_visible(int i, int s, int L, int Sq, bool 
 // A (64 keys x 128 d) tile goes from global memory to LDS by LDS-DMA, in MFMA-operand order: 16-byte unit
 // u = (kt*4 + c)*64 + 16*g + n holds K[16*kt + n][32*c + 8*g ..].  Wavefront w of the workgroup moves the 64-unit groups
 // grp = w, w + 8 (key tile grp / 4, chunk grp % 4 of its 16 keys): lane l's unit lands at lds_base + 16 l, which is exactly operand order, so the operand reads are linear and free of bank conflicts.
+// A lane's offset inside a tile is the same in every whole tile (first_off) and the tile's own goes into the scalar base: no vector instruction.
 // Keys beyond the last one are read from the last row (finite values that every consumer masks).
 // The compiler's wait counts do not see these loads: the code waits for them by hand before the barrier that
 // publishes the tile.
@@ -78,8 +85,18 @@ __device__ __forceinline__ void s1_dma16(const void* base, uint32_t lane_off, ui
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
                  : : "v"(lane_off), "s"(base), "s"(lds_base) : "memory", "m0");
 }
-__device__ __forceinline__ void issue_tile(const elem_bits* base, int row_stride, int key0, int L, uint32_t lds_tile,
+__device__ __forceinline__ uint32_t s1_first_off(int row_stride, int wave, int n, int g) {
+    return static_cast<uint32_t>((16 * (wave >> 2) + n) * row_stride + 32 * (wave & 3) + 8 * g) * 2u;
+}
+__device__ __forceinline__ void issue_tile(const elem_bits* base, int row_stride, uint32_t first_off, int key0, int L, uint32_t lds_tile,
                                            int wave, int n, int g) {
+    static_assert(kWavesS1 == 8, "first_off: two groups of a wavefront are 32 keys apart");
+    if (key0 + 64 <= L) {                                      // uniform
+        const elem_bits* tile_base = base + static_cast<int64_t>(key0) * row_stride;
+        s1_dma16(tile_base, first_off, lds_tile + wave * 1024);
+        s1_dma16(tile_base + 32 * static_cast<int64_t>(row_stride), first_off, lds_tile + (wave + 8) * 1024);
+        return;
+    }
 #pragma unroll
     for (int it = 0; it < 16 / kWavesS1; ++it) {
         const int grp = it * kWavesS1 + wave;                  // (kt, c) = (grp / 4, grp % 4)
@@ -121,11 +138,24 @@ __device__ __forceinline__ float row16_sum(float x) {
     x += dpp_row_ror<2>(x);
     return x + dpp_row_ror<1>(x);
 }
-__device__ __forceinline__ float dpp_quad_xor1(float x) {
-    return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0xB1, 0xF, 0xF, false));    // quad_perm:[1,0,3,2]
-}
-__device__ __forceinline__ float dpp_quad_xor2(float x) {
-    return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x4E, 0xF, 0xF, false));    // quad_perm:[2,3,0,1]
+// Of every quad's first lane: the maximum of the quad and of the lane before it, for two registers at a time; lane 0's lane before is prev's lane 63.
+// Spelled out because the compiler makes three instructions (a move, a canonicalisation, a maximum) of what one can do.  A
+// lane read by DPP must have been written three instructions before; the registers are each other's distance.
+__device__ __forceinline__ void pool_quads(float a, float b, float prev_a, float prev_b, float& best_a, float& best_b) {
+    float x, y;
+    asm volatile("s_nop 1\n\t"
+                 "v_max_f32_dpp %0, %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+                 "v_max_f32_dpp %1, %3, %3 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+                 "s_nop 0\n\t"
+                 "v_max_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                 "v_max_f32_dpp %1, %1, %1 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+                 "v_max_f32_dpp %0, %2, %0 wave_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_max_f32_dpp %1, %3, %1 wave_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_max_f32_dpp %0, %4, %0 wave_ror:1 row_mask:0x1 bank_mask:0x1\n\t"
+                 "v_max_f32_dpp %1, %5, %1 wave_ror:1 row_mask:0x1 bank_mask:0x1"
+                 : "=&v"(x), "=&v"(y) : "v"(a), "v"(b), "v"(prev_a), "v"(prev_b));
+    best_a = x;
+    best_b = y;
 }
 
 // kPool: instead of the score rows, write their 1-D max-pooling onto 64-token key blocks (window of 5 compressed
@@ -192,19 +222,19 @@ void stage1_kernel(const Stage1Params p) {
     const uint32_t lds_tiles = __builtin_amdgcn_readfirstlane(s1_lds_addr(tile));
     const int wave_u = wave;
     const int c_stride = static_cast<int>(p.c_row_stride), k_stride = static_cast<int>(p.k_row_stride);
+    const uint32_t c_off = s1_first_off(c_stride, wave, n, g), k_off = s1_first_off(k_stride, wave, n, g);
     // every ordinary load so far (q) lands before the first LDS-DMA goes out
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
     for (int t = 0; t < kTokPerWave; ++t)
 #pragma unroll
         for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(qf[t][c]));
-    if (tiles_c > 0) issue_tile(cbase, c_stride, 0, Lc, lds_tiles, wave_u, n, g);
+    if (tiles_c > 0) issue_tile(cbase, c_stride, c_off, 0, Lc, lds_tiles, wave_u, n, g);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    for (int ti = 0; ti < tiles_c; ++ti) {
-        if (ti + 1 < tiles_c) issue_tile(cbase, c_stride, (ti + 1) * 64, Lc, lds_tiles + ((ti + 1) & 1) * 16384, wave_u, n, g);
+    auto coarse_tile = [&](int ti, floatx4 (&s)[kTokPerWave][4]) {
+        if (ti + 1 < tiles_c) issue_tile(cbase, c_stride, c_off, (ti + 1) * 64, Lc, lds_tiles + ((ti + 1) & 1) * 16384, wave_u, n, g);
         const uint4* cur = tile[ti & 1];
-        floatx4 s[kTokPerWave][4];
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
 #pragma unroll
@@ -219,46 +249,54 @@ void stage1_kernel(const Stage1Params p) {
                     s[t][kt] = IV2_MFMA(qf[t][c], kf, s[t][kt], 0, 0, 0);
             }
         }
-        // only the tile that holds a token's last visible key needs the per-key test
-        const bool cut = (ti + 1) * 64 > min_vis_c;            // uniform per wavefront
-        if (!cut) {
-            // every key of the tile is visible to both tokens: the maximum is finite, no key test, and the scale
-            // rides in the multiply-add that feeds exp2
-#pragma unroll
-            for (int t = 0; t < kTokPerWave; ++t) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float mx = fmaxf(fmaxf(s[t][0][e], s[t][1][e]), fmaxf(s[t][2][e], s[t][3][e]));
-                    const float m_new = fmaxf(m[t][e], mx * p.scale_log2);
-                    float acc = l[t][e] * __builtin_amdgcn_exp2f(m[t][e] - m_new);
-#pragma unroll
-                    for (int kt = 0; kt < 4; ++kt) acc += __builtin_amdgcn_exp2f(s[t][kt][e] * p.scale_log2 - m_new);
-                    l[t][e] = acc;
-                    m[t][e] = m_new;
-                }
-            }
-        } else {
-#pragma unroll
-            for (int t = 0; t < kTokPerWave; ++t) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float v[4];
-#pragma unroll
-                    for (int kt = 0; kt < 4; ++kt)
-                        v[kt] = (ti * 64 + kt * 16 + n < vis_c[t]) ? s[t][kt][e] * p.scale_log2 : -INFINITY;
-                    const float mx = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
-                    const float m_new = fmaxf(m[t][e], mx);
-                    const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-                    float acc = l[t][e] * __builtin_amdgcn_exp2f(m[t][e] - m_use);
-#pragma unroll
-                    for (int kt = 0; kt < 4; ++kt) acc += __builtin_amdgcn_exp2f(v[kt] - m_use);
-                    l[t][e] = acc;
-                    m[t][e] = m_new;
-                }
-            }
-        }
+    };
+    auto coarse_done = [&]() {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // this wavefront's share of the next tile has landed
         __syncthreads();
+    };
+    // Two loops, as many rounds in all for every wavefront of the workgroup.  In the first every key of the tile is visible to both
+    // tokens: the maximum is finite, no key test, and the scale rides in the multiply-add that feeds exp2.
+    const int whole_c = min_vis_c >> 6 < tiles_c ? min_vis_c >> 6 : tiles_c;
+    for (int ti = 0; ti < whole_c; ++ti) {
+        floatx4 s[kTokPerWave][4];
+        coarse_tile(ti, s);
+#pragma unroll
+        for (int t = 0; t < kTokPerWave; ++t) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float mx = fmaxf(fmaxf(s[t][0][e], s[t][1][e]), fmaxf(s[t][2][e], s[t][3][e]));
+                const float m_new = fmaxf(m[t][e], mx * p.scale_log2);
+                float acc = l[t][e] * __builtin_amdgcn_exp2f(m[t][e] - m_new);
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt) acc += __builtin_amdgcn_exp2f(s[t][kt][e] * p.scale_log2 - m_new);
+                l[t][e] = acc;
+                m[t][e] = m_new;
+            }
+        }
+        coarse_done();
+    }
+    for (int ti = whole_c; ti < tiles_c; ++ti) {               // the tiles that hold a token's last visible key
+        floatx4 s[kTokPerWave][4];
+        coarse_tile(ti, s);
+#pragma unroll
+        for (int t = 0; t < kTokPerWave; ++t) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float v[4];
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt)
+                    v[kt] = (ti * 64 + kt * 16 + n < vis_c[t]) ? s[t][kt][e] * p.scale_log2 : -INFINITY;
+                const float mx = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
+                const float m_new = fmaxf(m[t][e], mx);
+                const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+                float acc = l[t][e] * __builtin_amdgcn_exp2f(m[t][e] - m_use);
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt) acc += __builtin_amdgcn_exp2f(v[kt] - m_use);
+                l[t][e] = acc;
+                m[t][e] = m_new;
+            }
+        }
+        coarse_done();
     }
     // merge the 16 key-column lanes of each head: lse2 = m + log2(l) in log2 units
     float lse2[kTokPerWave][4];
@@ -275,21 +313,35 @@ void stage1_kernel(const Stage1Params p) {
         }
 
     // ---------------- pass 2: scores over the fine keys ----------------
-    if (tiles_f > 0) issue_tile(kbase, k_stride, 0, Lk, lds_tiles, wave_u, n, g);
+    if (tiles_f > 0) issue_tile(kbase, k_stride, k_off, 0, Lk, lds_tiles, wave_u, n, g);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+    static_assert(kTokPerWave == 2, "pool_quads takes two tokens");
     elem_bits* out_rows[kTokPerWave];
     int bq[kTokPerWave];                                       // pooled output: the key block the token itself sits in
-    float carry[kTokPerWave];                                  // pooled output: score of the last key of the previous tile
+    float prev[kTokPerWave];                                   // pooled output: scores of the previous tile, for its last key
+    int plain_first = 0, plain_end;                            // tiles that need no test, below
     {
         const int cache_len = kPool ? (p.cache_lens ? p.cache_lens[b] : p.cache_len) : 0;
+        int seen = 0x7fffffff, before_local = 0x7fffffff;
 #pragma unroll
         for (int t = 0; t < kTokPerWave; ++t) {
             const int64_t row = static_cast<int64_t>(q0) + tok0 + t;
             out_rows[t] = kPool ? p.score + (static_cast<int64_t>(h) * p.score_head_stride + row * p.pool_len)
                                 : p.score + h * p.score_head_stride + row * p.score_row_stride;
             bq[t] = (tok0 + t + cache_len) / kBlockN;
-            carry[t] = 0.f;
+            prev[t] = 0.f;
+            seen = vis_f[t] < seen ? vis_f[t] : seen;          // 0: no such token
+            before_local = bq[t] - p.local_blocks < before_local ? bq[t] - p.local_blocks : before_local;
+        }
+        // most tiles lie inside the visible keys and the output row, and pooled wholly before the tokens' local windows and after the
+        // initial blocks: no key of theirs is hidden, no block forced or empty
+        if (seen > p.score_cols) seen = p.score_cols;
+        plain_end = seen >> 6;
+        if (kPool) {
+            before_local = before_local < p.pool_len ? before_local : p.pool_len;
+            plain_end = before_local < 0 ? 0 : (before_local >> 4) < plain_end ? before_local >> 4 : plain_end;
+            plain_first = (p.init_blocks + 15) >> 4;
         }
     }
     // value of a pooled entry that no visible key reaches
@@ -300,8 +352,20 @@ void stage1_kernel(const Stage1Params p) {
         return forced ? kElemPosInf : (empty ? kElemNegInf : f32_to_elem_hw(reached));
     };
 
+    // A plain tile's results are stored when the next tile begins: the wait at a tile's end counts stores too, and one just
+    // issued would add its round trip to every tile.
+    float held[kTokPerWave] = {0.f, 0.f};
+    bool pending = false;
+    auto store_held = [&](int ti) {
+        const uint32_t at = static_cast<uint32_t>(kPool ? ti * 16 + (lane >> 2) : ti * 64 + lane);
+        if (!kPool || (lane & 3) == 0) {
+#pragma unroll
+            for (int t = 0; t < kTokPerWave; ++t) out_rows[t][at] = f32_to_elem_hw(held[t]);
+        }
+    };
     for (int ti = 0; ti < tiles_f; ++ti) {
-        if (ti + 1 < tiles_f) issue_tile(kbase, k_stride, (ti + 1) * 64, Lk, lds_tiles + ((ti + 1) & 1) * 16384, wave_u, n, g);
+        if (pending) store_held(ti - 1);                       // uniform per wavefront
+        if (ti + 1 < tiles_f) issue_tile(kbase, k_stride, k_off, (ti + 1) * 64, Lk, lds_tiles + ((ti + 1) & 1) * 16384, wave_u, n, g);
         const uint4* cur = tile[ti & 1];
         float part[kTokPerWave][4];                            // [t][kt]: this lane's four heads summed, key 16 kt + n
 #pragma unroll
@@ -326,41 +390,38 @@ void stage1_kernel(const Stage1Params p) {
                 part[t][kt] = sum;
             }
         }
-        const int col = ti * 64 + lane;                        // lane = 16*g + n  <->  key 16*g + n of this tile
+        // sum over the four 16-lane rows (the head groups) and hand row kt the total of key tile kt, in three
+        // exchanges: (row0 + row1 | row2 + row3) of tiles 0/1 and of tiles 2/3, then the two halves.  lane = 16*g + n  <->  key 16*g + n of this tile
+        float mine[kTokPerWave];
 #pragma unroll
-        for (int t = 0; t < kTokPerWave; ++t) {
-            // sum over the four 16-lane rows (the head groups) and hand row kt the total of key tile kt, in three
-            // exchanges: (row0 + row1 | row2 + row3) of tiles 0/1 and of tiles 2/3, then the two halves
-            float mine = fold_rows32(fold_rows16(part[t][0], part[t][1]), fold_rows16(part[t][2], part[t][3]));
-            if ((ti + 1) * 64 > vis_f[t]) mine = (col < vis_f[t]) ? mine : 0.f;   // keys the token may not see score 0 (last tiles only)
-            if (!kPool) {
-                if (live[t] && col < p.score_cols) out_rows[t][col] = f32_to_elem_hw(mine);
-            } else {
-                // block kb = col / 4 pools keys 4 kb - 1 .. 4 kb + 3: its quad and the last key of the quad before
-                // the score of the key before: the lane below (one DPP shift over the whole wavefront; lane 0 takes the
-                // last key of the tile before), no trip through the LDS crossbar
-                float left = __uint_as_float(__builtin_amdgcn_update_dpp(__float_as_uint(carry[t]), __float_as_uint(mine),
-                                                                         0x138 /* wave_shr:1 */, 0xF, 0xF, false));
-                carry[t] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(mine), 63));
-                float best = fmaxf(mine, dpp_quad_xor1(mine));
-                best = fmaxf(best, dpp_quad_xor2(best));
-                best = fmaxf(best, left);
-                const int kb = col >> 2;
-                // most tiles lie wholly before the token's local window and after the initial blocks, inside the visible
-                // keys and the pooled row: no block of theirs is forced or empty (wavefront-uniform test)
-                const int kb0 = ti * 16;
-                const bool plain = live[t] && (ti + 1) * 64 <= vis_f[t] && kb0 >= p.init_blocks && kb0 + 15 < bq[t] - p.local_blocks &&
-                                   kb0 + 15 < p.pool_len;
-                if (plain) {
-                    if ((lane & 3) == 0) out_rows[t][kb] = f32_to_elem_hw(best);
-                } else if (live[t] && (lane & 3) == 0 && kb < p.pool_len) {
-                    out_rows[t][kb] = pool_rest(kb, bq[t], best);
-                }
+        for (int t = 0; t < kTokPerWave; ++t)
+            mine[t] = fold_rows32(fold_rows16(part[t][0], part[t][1]), fold_rows16(part[t][2], part[t][3]));
+        pending = ti >= plain_first && ti < plain_end;
+        const int col = ti * 64 + lane;
+        if (!pending) {
+#pragma unroll
+            for (int t = 0; t < kTokPerWave; ++t) mine[t] = col < vis_f[t] ? mine[t] : 0.f;     // keys the token may not see score 0
+        }
+        if (!kPool) {
+#pragma unroll
+            for (int t = 0; t < kTokPerWave; ++t) {
+                held[t] = mine[t];
+                if (!pending && live[t] && col < p.score_cols) out_rows[t][col] = f32_to_elem_hw(mine[t]);
+            }
+        } else {
+            // block kb = col / 4 pools keys 4 kb - 1 .. 4 kb + 3: its quad and the last key of the quad before
+            pool_quads(mine[0], mine[1], prev[0], prev[1], held[0], held[1]);
+            const int kb = col >> 2;
+#pragma unroll
+            for (int t = 0; t < kTokPerWave; ++t) {
+                prev[t] = mine[t];
+                if (!pending && live[t] && (lane & 3) == 0 && kb < p.pool_len) out_rows[t][kb] = pool_rest(kb, bq[t], held[t]);
             }
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
     }
+    if (pending) store_held(tiles_f - 1);
     // columns no tile covered
 #pragma unroll
     for (int t = 0; t < kTokPerWave; ++t) {
@@ -369,8 +430,9 @@ void stage1_kernel(const Stage1Params p) {
             for (int col = tiles_f * 64 + lane; col < p.score_cols; col += 64) out_rows[t][col] = 0;
         } else {
             // the first of them still sees the last key of the last tile
+            const float last_score = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(prev[t]), 63));
             for (int kb = tiles_f * 16 + lane; kb < p.pool_len; kb += 64)
-                out_rows[t][kb] = pool_rest(kb, bq[t], kb == tiles_f * 16 ? carry[t] : 0.f);
+                out_rows[t][kb] = pool_rest(kb, bq[t], kb == tiles_f * 16 ? last_score : 0.f);
         }
     }
 }
