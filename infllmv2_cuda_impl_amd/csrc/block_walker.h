@@ -42,6 +42,20 @@ struct BlockWalker {
     }
 };
 
+// A word of the mask rows of a group of up to eight tokens, `pitch` words apart: the blocks that the group walks together, which is those that five or
+// more of eight rows select, or all rows of a smaller group.  The row-parallel kernels say what that measured.
+__device__ __forceinline__ uint64_t walked_together(const unsigned long long* words, int pitch, int tokens) {
+    // how many of the rows select a block, a binary digit to a word
+    uint64_t r[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) r[t] = t < tokens ? words[t * pitch] : ~0ull;
+    auto sum3 = [](uint64_t a, uint64_t b, uint64_t c, uint64_t& carry) { carry = (a & b) | (c & (a | b)); return a ^ b ^ c; };
+    uint64_t t0, t1, t2, f0;
+    const uint64_t s0 = sum3(r[0], r[1], r[2], t0), s1 = sum3(r[3], r[4], r[5], t1), s2 = sum3(r[6], r[7], s0, t2);
+    const uint64_t ones = s1 ^ s2, t3 = s1 & s2, u = sum3(t0, t1, t2, f0), twos = u ^ t3, f1 = u & t3, fours = f0 ^ f1, eights = f0 & f1;
+    return tokens < 8 ? eights : eights | (fours & (twos | ones));
+}
+
 // Cross-row exchanges with gfx950's v_permlane16_swap / v_permlane32_swap (VALU speed; a ds_bpermute takes a trip
 // through the LDS crossbar): swapping a register with itself hands every lane its own row's value and the partner
 // row's value.

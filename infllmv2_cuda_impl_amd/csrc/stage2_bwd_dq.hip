@@ -6,7 +6,7 @@
 // dQ stays in registers for a token's whole row and is written once as bf16: no fp32 dQ scratch,
 // no atomics, no conversion pass, bit-reproducible.
 //
-// Schedule as in stage2_fwd_hybrid.hip: 8 wavefronts = 8 consecutive tokens; the blocks all 8
+// Schedule as in stage2_fwd_hybrid.hip: 8 wavefronts = 8 consecutive tokens; the blocks five or more of the 8
 // mask rows select go once through a 2-tile LDS ring ([K image | V in K-image order], 32 KiB),
 // and there the K^T operand of dQ^T = K^T dS^T is a transposed read (ds_read_b64_tr_b16) of
 // the same K tile; the remaining blocks of each row are walked by its wavefront alone, K and V
@@ -16,6 +16,9 @@
 // The kernel also forms D = rowsum(dO * O) (compute_dot_do_o, flash_bwd_preprocess_kernel.h:56-137): it has dO in registers, and O
 // costs its set-up one more request.  A pass of its own read dO and O once more from HBM: 227 us of 22.7 ms for 71552 packed tokens, 18 of 680 for
 // 6741 in four sequences (whole training pass of the latter 680 -> 660; of the former inside the spread of its runs).  Its row scalars go to the dK/dV kernel.
+//
+// Five, as in the forward.  Kernel alone in us, from all eight rows down to six | five | four: 8000 tokens, 32 blocks 477 -> 468 | 462 | 464; 4000 in
+// groups of 8 heads 386 -> 372 | 368 | 372; four short samples 215 -> 212 | 213 | 216; 71 552 packed tokens 7720 -> 7670 | 7640 | 7700.
 //
 // What bounds it: the chain S, dP, dQ of a block in two wavefronts per SIMD that the turn's barrier keeps in step.  At 32768
 // tokens, 64 blocks per row and 2 KV heads (3.65 to 3.9 ms) the matrix pipe is busy 39 % and the return path from L2, as in the
@@ -134,7 +137,7 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
     const int64_t tok = static_cast<int64_t>(q0) + (live ? i : i0);
     const uint64_t* mrow = p.fwd_mask ? p.fwd_mask + (static_cast<int64_t>(h) * p.total_q + tok) * p.n64_fwd : nullptr;
 
-    // ---- the row words every live token of the group has in common, and what is left of each row ----
+    // ---- the row words, and which blocks the group walks together ----
     int nw;
     {
         const int i_last = (i0 + kDqTokens - 1 < Sq) ? i0 + kDqTokens - 1 : Sq - 1;
@@ -145,8 +148,6 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
         if (nw > x.mask_words) nw = x.mask_words;                                    // a sequence longer than the announced max_seqlen_k
     }
     unsigned long long* own = rows + wave * x.mask_words;
-    for (int w = tid; w < nw; w += 512) com[w] = ~0ull;
-    __syncthreads();
     for (int w = lane; w < nw; w += 64) {
         uint64_t v = 0ull;
         if (last_blk >= 0 && w <= (last_blk >> 6)) {
@@ -157,10 +158,10 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
             }
         }
         own[w] = v;
-        if (live && v != ~0ull) atomicAnd(&com[w], static_cast<unsigned long long>(v));
     }
     __syncthreads();
-    for (int w = lane; w < nw; w += 64) own[w] &= ~com[w];
+    for (int w = tid; w < nw; w += 512) com[w] = walked_together(rows + w, x.mask_words, Sq - i0);
+    __syncthreads();
 
     // ---- this token's operands, and D = rowsum(dO * O) from them ----
     elem8 qf[4], dof[4], of[4];
@@ -196,20 +197,23 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
     const uint32_t ring_base = __builtin_amdgcn_readfirstlane(lds_address_dq(ring) + wave * 4096);
     auto issue = [&](int jj, int tile) { dq_dma_copy_4k(src_lane + static_cast<int64_t>(jj) * 1024, ring_base + tile * kDqTileBytes); };
     int cw = -1, ow = -1;
-    uint64_t cbits = 0ull, obits = 0ull;
-    auto next_common = [&]() -> int {
+    uint64_t cbits = 0ull, crow = 0ull, obits = 0ull;
+    auto next_common = [&](bool& mine_too) -> int {             // mine_too: whether this row selects it
+
         while (cbits == 0ull) {
             if (++cw >= nw) return -1;
             cbits = dq_uniform_u64(com[cw]);
+            crow = dq_uniform_u64(own[cw]);
         }
         const int bit = __builtin_ctzll(cbits);
+        mine_too = (crow >> bit) & 1ull;
         cbits &= cbits - 1ull;
         return cw * 64 + bit;
     };
     auto next_own = [&]() -> int {
         while (obits == 0ull) {
             if (++ow >= nw) return -1;
-            obits = dq_uniform_u64(own[ow]);
+            obits = dq_uniform_u64(own[ow] & ~com[ow]);
         }
         const int bit = __builtin_ctzll(obits);
         obits &= obits - 1ull;
@@ -245,7 +249,8 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
         dsum = 0.f;
     }
     const floatx4 neg_dsum = {-dsum, -dsum, -dsum, -dsum};     // the dP accumulators start here: dS = P (dP - D) is then one product
-    int j0 = next_common();
+    bool mine0 = false;
+    int j0 = next_common(mine0);
     if (j0 >= 0) issue(j0, 0);
     int tile = 0;
     bool k_ahead = false;                                      // the coming own block's 16 K-fragment loads were issued last turn
@@ -254,9 +259,10 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
             // younger than this wavefront's 4 DMA loads of block j0: last turn's 16 K loads
             if (k_ahead) asm volatile("s_waitcnt vmcnt(16)" ::: "memory"); else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();                                   // block j0 is in LDS for everyone; the other tile is free
-            const int j1 = next_common();
+            bool mine1 = false;
+            const int j1 = next_common(mine1);
             if (j1 >= 0) issue(j1, tile ^ 1);
-            if (live) {
+            if (mine0) {
                 const uint4* kb = ring + tile * 2048 + lane;
                 const uint4* vb = kb + 1024;
                 floatx4 s[4], dp[4];
@@ -299,6 +305,7 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
                     }
             }
             j0 = j1;
+            mine0 = mine1;
             tile ^= 1;
         }
         k_ahead = false;

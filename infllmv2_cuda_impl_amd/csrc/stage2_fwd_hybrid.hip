@@ -195,25 +195,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
         own[w] = v;
     }
     __syncthreads();
-    for (int w = tid; w < nw; w += 512) {
-        uint64_t shared = 0ull;
-        if (share_log2 == 0) {
-            // how many of the eight rows select a block, a binary digit to a word: ones, twos (two of each), fours, eights
-            uint64_t r[kHybTokens];
-#pragma unroll
-            for (int t = 0; t < kHybTokens; ++t) r[t] = t < in_group ? rows[t * x.mask_words + w] : ~0ull;
-            auto sum3 = [](uint64_t a, uint64_t b, uint64_t c, uint64_t& carry) { carry = (a & b) | (c & (a | b)); return a ^ b ^ c; };
-            uint64_t t0, t1, t2, t3, f0, f1;
-            const uint64_t s0 = sum3(r[0], r[1], r[2], t0), s1 = sum3(r[3], r[4], r[5], t1), s2 = sum3(r[6], r[7], s0, t2);
-            const uint64_t ones = s1 ^ s2;
-            t3 = s1 & s2;
-            const uint64_t u = sum3(t0, t1, t2, f0), twos = u ^ t3;
-            f1 = u & t3;
-            const uint64_t fours = f0 ^ f1, eights = f0 & f1;
-            shared = in_group < kHybTokens ? eights : eights | (fours & (twos | ones));     // all of them, or five of eight
-        }
-        com[w] = shared;
-    }
+    for (int w = tid; w < nw; w += 512) com[w] = share_log2 == 0 ? walked_together(rows + w, x.mask_words, in_group) : 0ull;   // shared out: no lock step
     __syncthreads();
     const uint64_t columns = (share_log2 == 0 ? ~0ull : share_log2 == 1 ? 0x5555555555555555ull
                               : share_log2 == 2 ? 0x1111111111111111ull : 0x0101010101010101ull) << part;

@@ -1,7 +1,6 @@
 """Stage-2 forward of rows far enough in their sequence to be walked at a pace (behind key block 512): the pace changes the order of a row's blocks, so
 rows are checked against fp32 attention, and bit for bit across launches that hold them differently (alone, as a chunk of fewer queries, one KV head,
 packed behind another sequence, images packed earlier, causal or not where that is the same), with rows on both sides of the line in one launch."""
-import numpy as np
 import pytest
 import torch
 
