@@ -749,10 +749,19 @@ void decode_split_kernel(const DecodeParams p) {
 // for the weights, split l.  kMax >= splits: the loads are unrolled (beyond the last split the last one is read again),
 // so every partial is requested before the first is used.  A wavefront per head keeps the merge of 64 splits at one
 // round trip; one workgroup per KV head pulled 16 times as much through one CU.
+// What it spends is latency: its arguments in one cache line, reductions over the lanes by DPP (12 exchanges through LDS took 0.55 us of its 2.4).
 constexpr int kCombineWaves = 4;
+struct CombineParams {
+    const float* o_part;
+    const float* lse_part;
+    elem_bits* out;
+    float* lse;
+    int64_t o_batch, o_head;
+    int num_heads_k, splits, group;
+};
 template <int kMax>
 __global__ __launch_bounds__(64 * kCombineWaves)
-void decode_combine_kernel(const DecodeParams p) {
+void decode_combine_kernel(const CombineParams p) {
     const int lane = threadIdx.x & 63;
     const int head = blockIdx.x * kCombineWaves + (threadIdx.x >> 6);
     const int h = blockIdx.y, b = blockIdx.z;
@@ -763,13 +772,26 @@ void decode_combine_kernel(const DecodeParams p) {
 #pragma unroll
     for (int s = 0; s < kMax; ++s)
         part[s] = *reinterpret_cast<const float2*>(p.o_part + ((slot0 + (s < p.splits ? s : p.splits - 1)) * 16 + head) * kHeadDim + 2 * lane);
-    float mx = lse;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+    // exchanges by 1, 2, 4 and 8 lanes (4 and 8 as mirrors: by then every quad, every eight lanes agree), and between rows where splits reach beyond one
+    auto over_splits = [&](float x, auto both) {
+        x = both(x, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0xB1, 0xF, 0xF, false)));
+        x = both(x, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x4E, 0xF, 0xF, false)));
+        x = both(x, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x141, 0xF, 0xF, false)));
+        x = both(x, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x140, 0xF, 0xF, false)));
+        if constexpr (kMax > 16) {
+            float mine, other;
+            row_pair_xor16(x, mine, other);
+            x = both(mine, other);
+            row_pair_xor32(x, mine, other);
+            x = both(mine, other);
+        } else {
+            x = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x)));
+        }
+        return x;
+    };
+    const float mx = over_splits(lse, [](float x, float y) { return fmaxf(x, y); });
     const float w = lse == -INFINITY ? 0.f : expf(lse - mx);   // a split without blocks has no partial
-    float wsum = w;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) wsum += __shfl_xor(wsum, off);
+    const float wsum = over_splits(w, [](float x, float y) { return x + y; });
     float acc0 = 0.f, acc1 = 0.f;
 #pragma unroll
     for (int s = 0; s < kMax; ++s) {
@@ -934,10 +956,11 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
     hipLaunchKernelGGL(split_kernel, dim3(num_splits, num_heads_k, batch), dim3(grouped ? 256 : 64), lds, st, p);
     IV2_LAUNCH_CHECK();
     if (num_splits > 1) {
+        const CombineParams c{p.o_part, p.lse_part, p.out, p.lse, p.o_batch, p.o_head, num_heads_k, num_splits, p.group};
         const dim3 cgrid((p.group + kCombineWaves - 1) / kCombineWaves, num_heads_k, batch), cblock(64 * kCombineWaves);
-        if (num_splits <= 4) hipLaunchKernelGGL(decode_combine_kernel<4>, cgrid, cblock, 0, st, p);
-        else if (num_splits <= 16) hipLaunchKernelGGL(decode_combine_kernel<16>, cgrid, cblock, 0, st, p);
-        else hipLaunchKernelGGL(decode_combine_kernel<64>, cgrid, cblock, 0, st, p);
+        if (num_splits <= 4) hipLaunchKernelGGL(decode_combine_kernel<4>, cgrid, cblock, 0, st, c);
+        else if (num_splits <= 16) hipLaunchKernelGGL(decode_combine_kernel<16>, cgrid, cblock, 0, st, c);
+        else hipLaunchKernelGGL(decode_combine_kernel<64>, cgrid, cblock, 0, st, c);
         IV2_LAUNCH_CHECK();
     }
     return 0;
