@@ -595,14 +595,11 @@ std::tuple<Tensor, Tensor> fwd_kvcache(const Tensor& q, const Tensor& kc, const 
     return {out, lse};
 }
 
-// The front of a decode step of a layer for a batch of sequences: append the token, extend the compressed keys, and - with
-// scores - Stage 1 and pooling.  lens: tokens held (device), or none: host_len for every sequence.  max_len bounds the
-// lengths after the step.  Returns {lengths after the step, block scores (batch, Hk, blocks) or an undefined tensor}.
-std::tuple<Tensor, Tensor> decode_front(const Tensor& q, const Tensor& kn, const Tensor& vn, const Tensor& kc, const Tensor& vc,
-                                        const Tensor& fine, const Tensor& coarse, const OptTensor& lens, int64_t host_len,
-                                        const OptTensor& fine_lens_, const OptTensor& coarse_lens_, int64_t max_len, int64_t kernel_size,
-                                        int64_t stride, int64_t block_size, bool scores, int64_t local_blocks, int64_t init_blocks,
-                                        double scale) {
+// What a decode step asks of its tensors.
+void check_step(const Tensor& q, const Tensor& kn, const Tensor& vn, const Tensor& kc, const Tensor& vc,
+                const Tensor& fine, const Tensor& coarse, const OptTensor& lens, int64_t host_len,
+                const OptTensor& fine_lens_, const OptTensor& coarse_lens_, int64_t kernel_size,
+                int64_t stride, int64_t block_size, bool scores) {
     require_gpu(q, "q"); require_gpu(kc, "k_cache");
     require_16bit(q);
     for (const Tensor* t : {&kn, &vn, &kc, &vc, &fine, &coarse}) {
@@ -611,9 +608,9 @@ std::tuple<Tensor, Tensor> decode_front(const Tensor& q, const Tensor& kn, const
         TORCH_CHECK(t->dim() == 4 && t->stride(-1) == 1, "Input tensor must have contiguous last dimension");
     }
     TORCH_CHECK(q.dim() == 4 && q.size(1) == 1 && q.stride(-1) == 1, "q must have shape (batch_size, 1, num_heads, head_size)");
-    const int64_t batch = q.size(0), hq = q.size(2), d = q.size(3), hk = kc.size(2), cap = kc.size(1);
+    const int64_t batch = q.size(0), hq = q.size(2), d = q.size(3), hk = kc.size(2);
     TORCH_CHECK(d == kHeadDim, "this build only supports head dimension 128");
-    const int64_t group = group_size(hq, hk);
+    group_size(hq, hk);
     TORCH_CHECK(kc.size(0) == batch && kc.size(3) == d && vc.sizes() == kc.sizes(),
                 "k_cache and v_cache must have shape (batch_size, seqlen_cache, num_heads_k, head_size)");
     TORCH_CHECK(kn.size(0) == batch && kn.size(1) == 1 && kn.size(2) == hk && kn.size(3) == d && vn.sizes() == kn.sizes(),
@@ -623,7 +620,7 @@ std::tuple<Tensor, Tensor> decode_front(const Tensor& q, const Tensor& kn, const
                     "compressed-key caches must have shape (batch_size, rows, num_heads_k, head_size)");
     for (const OptTensor* t : {&lens, &fine_lens_, &coarse_lens_})
         TORCH_CHECK(!t->has_value() || ((*t)->scalar_type() == at::kInt && (*t)->dim() == 1 && (*t)->size(0) == batch && (*t)->is_contiguous() &&
-                                        (*t)->device() == q.device()), "lengths must be contiguous int32 tensors of shape (batch_size)");
+                (*t)->device() == q.device()), "lengths must be contiguous int32 tensors of shape (batch_size)");
     // four compressed keys per block, as the pooling of stage1_pooled and stage1_kvcache; without scores nothing looks at the blocks
     TORCH_CHECK(!scores || (block_size == kBlock && stride > 0 && block_size / stride == 4),
                 "only 64-token blocks over stride-16 compressed keys are fused");
@@ -631,6 +628,18 @@ std::tuple<Tensor, Tensor> decode_front(const Tensor& q, const Tensor& kn, const
     for (const auto& [t, kernel, st] : {std::tuple(&fine, kernel_size, stride), std::tuple(&coarse, 4 * kernel_size, 4 * stride)})
         TORCH_CHECK(lens.has_value() || st <= 0 || windows(host_len + 1, kernel, st) == windows(host_len, kernel, st) ||
                     t->size(1) >= windows(host_len + 1, kernel, st), "out must be a contiguous (rows, num_heads_k, head_size) buffer of k's dtype");
+}
+
+// The front of a decode step of a layer for a batch of sequences: append the token, extend the compressed keys, and - with
+// scores - Stage 1 and pooling.  lens: tokens held (device), or none: host_len for every sequence.  max_len bounds the
+// lengths after the step.  Returns {lengths after the step, block scores (batch, Hk, blocks) or an undefined tensor}.
+std::tuple<Tensor, Tensor> decode_front(const Tensor& q, const Tensor& kn, const Tensor& vn, const Tensor& kc, const Tensor& vc,
+                                        const Tensor& fine, const Tensor& coarse, const OptTensor& lens, int64_t host_len,
+                                        const OptTensor& fine_lens_, const OptTensor& coarse_lens_, int64_t max_len, int64_t kernel_size,
+                                        int64_t stride, int64_t block_size, bool scores, int64_t local_blocks, int64_t init_blocks,
+                                        double scale) {
+    check_step(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens_, coarse_lens_, kernel_size, stride, block_size, scores);
+    const int64_t batch = q.size(0), hq = q.size(2), d = q.size(3), hk = kc.size(2), cap = kc.size(1), group = hq / hk;
     const auto ints = q.options().dtype(at::kInt);
     Tensor new_lens = at::empty({batch}, ints);
     const Tensor fine_lens = fine_lens_.has_value() ? *fine_lens_ : at::empty({batch}, ints);
@@ -673,7 +682,8 @@ std::tuple<Tensor, OptTensor> decode_step(const Tensor& q, const Tensor& kn, con
 
 // A whole decode step on selected blocks: the front, the selection and the attention.  The selection is made by the
 // attention's own launch where that serves it (a workgroup per CU at most, rows of 2048 block scores at most: see
-// infllmv2_fwd_kvcache_scores), by a top-k launch otherwise.  Returns {out, lengths after the step}.
+// infllmv2_fwd_kvcache_scores), by a top-k launch otherwise.  Returns {out, lengths after the step}; a step of one sequence whose length the
+// host gives has no lengths to return.
 std::tuple<Tensor, Tensor> decode_sparse(const Tensor& q, const Tensor& kn, const Tensor& vn, const Tensor& kc, const Tensor& vc,
                                          const Tensor& fine, const Tensor& coarse, const OptTensor& lens, int64_t host_len,
                                          const OptTensor& fine_lens, const OptTensor& coarse_lens, int64_t max_len, int64_t kernel_size,
@@ -691,18 +701,39 @@ std::tuple<Tensor, Tensor> decode_sparse(const Tensor& q, const Tensor& kn, cons
         return {std::get<0>(fwd_kvcache(q, kc, vc, std::nullopt, std::nullopt, new_lens, scale, 0, std::nullopt, mask, std::nullopt, std::nullopt,
                                         std::nullopt, std::nullopt, std::nullopt, false)), new_lens};
     }
-    auto [new_lens, pooled] = decode_front(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, max_len, kernel_size,
-                                           stride, block_size, true, local_blocks, init_blocks, scale);
-    const int64_t n = pooled.size(2);
-    Tensor out = at::empty_like(q);
-    const size_t partials = infllmv2_fwd_kvcache_workspace_bytes(as_int(batch), as_int(hk), splits), lse_bytes = sizeof(float) * batch * hq;
-    Tensor ws = bytes_on(q, partials + lse_bytes);
-    const int64_t qs[2] = {q.stride(0), q.stride(2)}, os[2] = {out.stride(0), out.stride(2)};
-    const S3 kcs = batch_rows_heads(kc), vcs = batch_rows_heads(vc);
-    auto fn = is_half(q) ? infllmv2_fwd_kvcache_scores_f16 : infllmv2_fwd_kvcache_scores;
-    check_rc(fn(stream_of(q), ptr(q), ptr(kc), ptr(vc), iptr(new_lens), ptr(out), reinterpret_cast<float*>(static_cast<char*>(ptr(ws)) + partials),
-                ptr(pooled), as_int(n), as_int(topk), ptr(ws), partials, as_int(batch), as_int(hq), as_int(hk), as_int(kHeadDim),
-                as_int(kc.size(1)), qs, kcs.v, vcs.v, os, splits, static_cast<float>(scale)), "fwd_kvcache_scores");
+    check_step(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, kernel_size, stride, block_size, true);
+    // What lives inside the step shares one allocation, and lengths that the host has get no tensor of their own: a step that the device finishes in 19 to 20 us was
+    // bound by the host that issues it (one sequence, seven allocations 22.6 us to issue, two 19.6; six sequences 19.2 and 17.3).
+    Tensor new_lens, out = at::empty_like(q);
+    if (lens.has_value()) new_lens = at::empty({batch}, q.options().dtype(at::kInt));
+    const int64_t blocks = (max_len + block_size - 1) / block_size;
+    const int64_t max_f = std::min(windows(max_len, kernel_size, stride), fine.size(1)), max_c = std::min(windows(max_len, 4 * kernel_size, 4 * stride), coarse.size(1));
+    size_t at_byte = 0;
+    auto take = [&](size_t bytes) { const size_t start = at_byte; at_byte += (bytes + 255) / 256 * 256; return start; };
+    const size_t record_bytes = infllmv2_stage1_decode_workspace_bytes(as_int(batch), as_int(hk), as_int(max_f), as_int(max_c));
+    const size_t partial_bytes = infllmv2_fwd_kvcache_workspace_bytes(as_int(batch), as_int(hk), splits);
+    const size_t scores = take(2 * static_cast<size_t>(batch * hk * blocks)), records = take(std::max<size_t>(record_bytes, 16)), partials = take(partial_bytes);
+    const size_t lse = take(sizeof(float) * static_cast<size_t>(batch * hq)), own_lens = take(3 * sizeof(int32_t) * static_cast<size_t>(batch));
+    Tensor ws = bytes_on(q, at_byte);
+    char* base = static_cast<char*>(ptr(ws));
+    int32_t* own = reinterpret_cast<int32_t*>(base + own_lens);
+    int32_t* new_ptr = lens.has_value() ? static_cast<int32_t*>(ptr(new_lens)) : own;
+    int32_t* fine_ptr = fine_lens.has_value() ? static_cast<int32_t*>(ptr(*fine_lens)) : own + batch;
+    int32_t* coarse_ptr = coarse_lens.has_value() ? static_cast<int32_t*>(ptr(*coarse_lens)) : own + 2 * batch;
+    const int64_t group = hq / hk, qs[3] = {q.stride(0), q.stride(2), group * q.stride(2)}, os[2] = {out.stride(0), out.stride(2)};
+    const int64_t kns[2] = {kn.stride(0), kn.stride(2)}, vns[2] = {vn.stride(0), vn.stride(2)};
+    const S3 kcs = batch_rows_heads(kc), vcs = batch_rows_heads(vc), fs = batch_rows_heads(fine), cs = batch_rows_heads(coarse);
+    void* stream = stream_of(q);
+    auto front = is_half(q) ? infllmv2_decode_step_scores_f16 : infllmv2_decode_step_scores;
+    check_rc(front(stream, ptr(q), ptr(kn), ptr(vn), ptr(kc), ptr(vc), ptr(fine), ptr(coarse), iptr(lens), as_int(host_len), new_ptr, fine_ptr, coarse_ptr,
+                   base + scores, base + records, record_bytes, as_int(batch), as_int(hq), as_int(hk), as_int(kHeadDim), as_int(kc.size(1)),
+                   as_int(fine.size(1)), as_int(coarse.size(1)), as_int(max_len), qs, kns, vns, kcs.v, vcs.v, fs.v, cs.v, as_int(kernel_size),
+                   as_int(stride), as_int(4 * kernel_size), as_int(4 * stride), static_cast<float>(scale), as_int(blocks), as_int(local_blocks),
+                   as_int(init_blocks)), "decode_step_scores");
+    auto attend = is_half(q) ? infllmv2_fwd_kvcache_scores_f16 : infllmv2_fwd_kvcache_scores;
+    check_rc(attend(stream, ptr(q), ptr(kc), ptr(vc), new_ptr, ptr(out), reinterpret_cast<float*>(base + lse), base + scores, as_int(blocks), as_int(topk),
+                    base + partials, partial_bytes, as_int(batch), as_int(hq), as_int(hk), as_int(kHeadDim), as_int(kc.size(1)), qs, kcs.v, vcs.v, os,
+                    splits, static_cast<float>(scale)), "fwd_kvcache_scores");
     return {out, new_lens};
 }
 
