@@ -35,6 +35,7 @@ constexpr int kCompressRowsPerWg = 8;
 constexpr int kCompressThreads = 256;
 constexpr int kCompressUnits = 16;           // units of one output row a workgroup works on: 128 elements
 constexpr int kCompressMaxLds = 49152;       // the K rows a workgroup stages: 192 rows of 256 bytes
+constexpr int kCompressPieces = kCompressMaxLds / 16 / kCompressThreads;      // of 16 bytes, per thread
 
 // A workgroup takes rows_per_wg consecutive output rows of one KV head (128 elements of it).  Their windows are one
 // stretch of (rows - 1) * stride + kernel_size K rows: it goes into LDS with every load in flight at once, and then
@@ -72,11 +73,16 @@ __device__ __forceinline__ void compress_rows_of_head(const CompressParams& p, i
     for (int base = 0; base < span; base += step) {
         const int staged = span - base < step ? span - base : step;
         if (base > 0) __syncthreads();
-#pragma unroll 4
-        for (int it = tid; it < staged * kCompressUnits; it += kCompressThreads) {
-            const int i = it / kCompressUnits, u = it % kCompressUnits;
-            if (u < nu) stage[it] = *reinterpret_cast<const uint4*>(src + (base + i) * p.k_row_stride + u * 8);
+        uint4 piece[kCompressPieces];                          // all of them requested before the first is waited for
+#pragma unroll
+        for (int t = 0; t < kCompressPieces; ++t) {
+            const int it = tid + t * kCompressThreads, i = it / kCompressUnits, u = it % kCompressUnits;
+            piece[t] = make_uint4(0, 0, 0, 0);
+            if (i < staged && u < nu) piece[t] = *reinterpret_cast<const uint4*>(src + (base + i) * p.k_row_stride + u * 8);
         }
+#pragma unroll
+        for (int t = 0; t < kCompressPieces; ++t)
+            if ((tid + t * kCompressThreads) / kCompressUnits < staged) stage[tid + t * kCompressThreads] = piece[t];
         __syncthreads();
         const uint32_t* words = reinterpret_cast<const uint32_t*>(stage) + lane;
 #pragma unroll
