@@ -471,12 +471,13 @@ void decode_split_kernel(const DecodeParams p) {
     each = __builtin_amdgcn_readfirstlane(each);
     each += (each + 1) * runs <= total ? 1 : (each * runs > total ? -1 : 0);
     // So many runs take one block more, dealt out to the splits in turn: a CU's wavefronts share its bandwidth, and all of a split's four runs longer by one
-    // were a workgroup that took a quarter longer (24 sequences x 2 heads, 64 blocks over 5 splits: whole paged step 45.0 -> 43.6 us).
+    // were a workgroup that took a quarter longer (24 sequences x 2 heads, 64 blocks over 5 splits: whole paged step 45.0 -> 43.6 us).  Where
+    // there are fewer blocks than runs the first runs take them: a row of a few blocks is then the same whatever the number of splits.
     const int longer = total - each * runs;
     const int every = kWaves == 1 ? 0 : (longer >= p.splits ? 1 : 0) + (longer >= 2 * p.splits ? 1 : 0) + (longer >= 3 * p.splits ? 1 : 0);    // of each split's
     const int over = longer - every * p.splits, mine_longer = every + (split < over ? 1 : 0);
-    const int begin = run * each + split * every + (split < over ? split : over) + (wave < mine_longer ? wave : mine_longer);
-    const int count = each + (wave < mine_longer ? 1 : 0);
+    const int begin = each == 0 ? (run < longer ? run : longer) : run * each + split * every + (split < over ? split : over) + (wave < mine_longer ? wave : mine_longer);
+    const int count = each + ((each == 0 ? run < longer : wave < mine_longer) ? 1 : 0);
 
     // Blocks [base, base + 64) of this run, one per lane, and the cache row (page) they lie in.
     const int cache_row = p.block_table ? 0 : (p.cache_batch_idx ? p.cache_batch_idx[b] : b);
