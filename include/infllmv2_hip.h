@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define INFLLMV2_ABI_VERSION 14
+#define INFLLMV2_ABI_VERSION 15
 
 /* ---- library ------------------------------------------------------------------------------ */
 
@@ -120,6 +120,10 @@ int infllmv2_topk_blocks(void* stream, const void* pooled, int64_t row_stride, i
 int infllmv2_topk_select(void* stream, const void* pooled, int64_t row_stride, int dtype, int32_t* topk_idx,
                          uint64_t* mask_words, int64_t rows, int n, int k, int n_uint64_per_row, int by_index,
                          int drop_neg_inf);
+
+/* The mask words of infllmv2_topk_select alone, for callers that do not read the list. */
+int infllmv2_topk_mask(void* stream, const void* pooled, int64_t row_stride, int dtype, uint64_t* mask_words, int64_t rows,
+                       int n, int k, int n_uint64_per_row, int drop_neg_inf);
 
 /* The blocks of a window as a selection: of a query at position p of its sequence (cache_lens tokens before its first query, null: none), blocks [0, init_blocks) and
  * p / block_size - local_blocks to p / block_size, those below n_blocks: what max_pooling_1d_varlen marks +inf.  topk_idx (num_heads, rows,

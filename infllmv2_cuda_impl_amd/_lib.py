@@ -11,7 +11,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libinfllmv2_hip.so")
 
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 _p, _i, _i64, _sz, _f = C.c_void_p, C.c_int, C.c_int64, C.c_size_t, C.c_float
 
@@ -30,6 +30,7 @@ SIGNATURES = {
     "infllmv2_topk_blocks": [_p, _p, _i64, _p, _i64, _i, _i],
     "infllmv2_window_blocks": [_p, _p, _p, _p, _p, _i, _i, _i64, _i, _i, _i, _i, _i],
     "infllmv2_topk_select": [_p, _p, _i64, _i, _p, _p, _i64, _i, _i, _i, _i, _i],
+    "infllmv2_topk_mask": [_p, _p, _i64, _i, _p, _i64, _i, _i, _i, _i],
     "infllmv2_compress_keys": [_p, _p, _p, _p, _p, _i, _i, _i, _i, _i64, _i64, _i, _i, _i],
     "infllmv2_compress_keys_pair": [_p] * 7 + [_i] * 4 + [_i64, _i64] + [_i] * 4,
     "infllmv2_compress_keys_cache": [_p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _p, _p, _i, _i, _i, _i],

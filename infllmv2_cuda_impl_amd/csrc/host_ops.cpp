@@ -346,6 +346,22 @@ std::tuple<Tensor, OptTensor> topk_blocks(const Tensor& pooled, int64_t k, bool 
     return {idx, mask};
 }
 
+// The mask of the same selection, where nobody reads the list.
+Tensor topk_mask(const Tensor& pooled, int64_t k, std::optional<int64_t> words) {
+    require_gpu(pooled, "pooled");
+    const Tensor x = pooled.contiguous();
+    const int64_t n = x.size(-1), n64 = words.has_value() ? *words : (n + 63) / 64;
+    c10::SmallVector<int64_t, 5> shape(x.sizes().begin(), x.sizes().end());
+    int64_t rows = 1;
+    for (size_t i = 0; i + 1 < shape.size(); ++i) rows *= shape[i];
+    shape.back() = n64;
+    DeviceGuard guard(x.device());
+    Tensor mask = at::empty(shape, x.options().dtype(at::kLong));
+    check_rc(infllmv2_topk_mask(stream_of(x), ptr(x), n, is_half(x) ? 0 : 1, static_cast<uint64_t*>(ptr(mask)), rows, as_int(n), as_int(k), as_int(n64), 0),
+             "topk_mask");
+    return mask;
+}
+
 std::tuple<Tensor, Tensor> window_blocks(int64_t heads, int64_t rows, const Tensor& cu_q_, const OptTensor& positions_, int64_t max_q, int64_t max_position,
                                          int64_t local_blocks, int64_t init_blocks, int64_t block_size) {
     require_gpu(cu_q_, "cu_seqlens_q");
@@ -386,10 +402,11 @@ Tensor topk_to_uint64(const Tensor& topk_idx, int64_t k_blocks, const OptTensor&
 }
 
 // the selection front end: compressed keys, fused Stage 1 and pooling, top-k with the mask words
-std::tuple<Tensor, OptTensor> select_blocks(const Tensor& q_, const Tensor& k, const Tensor& cu_q, const Tensor& cu_k, int64_t max_q,
-                                            int64_t max_k, int64_t topk, int64_t local_blocks, int64_t init_blocks, const OptTensor& cache_lens,
-                                            int64_t max_cache_len, double scale, bool causal, int64_t kernel_size, int64_t stride,
-                                            int64_t block_size, bool exact_lse, bool return_mask, bool by_index, bool drop_unreachable) {
+// Block scores (Hk, total_q, blocks) of packed queries, and how many mask words a row of the selection takes.
+std::tuple<Tensor, int64_t> block_scores(const Tensor& q_, const Tensor& k, const Tensor& cu_q, const Tensor& cu_k, int64_t max_q,
+                                         int64_t max_k, int64_t local_blocks, int64_t init_blocks, const OptTensor& cache_lens,
+                                         int64_t max_cache_len, double scale, bool causal, int64_t kernel_size, int64_t stride,
+                                         int64_t block_size, bool exact_lse) {
     const Tensor q = q_.stride(-1) == 1 ? q_ : q_.contiguous();
     Tensor kf, cu_f, kc, cu_c;
     if (exact_lse) {
@@ -403,7 +420,24 @@ std::tuple<Tensor, OptTensor> select_blocks(const Tensor& q_, const Tensor& k, c
                                         0, local_blocks, init_blocks, block_size, stride);
     int64_t n64 = ((max_k + block_size - 1) / block_size + 63) / 64;
     if (n64 * 64 < out_len) n64 = (out_len + 63) / 64;                 // cached tokens widen the pooled rows beyond max_seqlen_k
+    return {pooled, n64};
+}
+
+std::tuple<Tensor, OptTensor> select_blocks(const Tensor& q, const Tensor& k, const Tensor& cu_q, const Tensor& cu_k, int64_t max_q,
+                                            int64_t max_k, int64_t topk, int64_t local_blocks, int64_t init_blocks, const OptTensor& cache_lens,
+                                            int64_t max_cache_len, double scale, bool causal, int64_t kernel_size, int64_t stride,
+                                            int64_t block_size, bool exact_lse, bool return_mask, bool by_index, bool drop_unreachable) {
+    const auto [pooled, n64] = block_scores(q, k, cu_q, cu_k, max_q, max_k, local_blocks, init_blocks, cache_lens, max_cache_len, scale, causal,
+                                            kernel_size, stride, block_size, exact_lse);
     return topk_blocks(pooled, topk, return_mask, by_index, drop_unreachable, n64);
+}
+
+// The selection of plain prefill for a caller that goes on with the mask: {an empty list whose width says how many blocks a row has at most, mask}.
+std::tuple<Tensor, Tensor> select_mask(const Tensor& q, const Tensor& k, const Tensor& cu, int64_t max_len, int64_t topk, int64_t local_blocks,
+                                       int64_t init_blocks, double scale, int64_t kernel_size, int64_t stride, int64_t block_size) {
+    const auto [pooled, n64] = block_scores(q, k, cu, cu, max_len, max_len, local_blocks, init_blocks, std::nullopt, 0, scale, true, kernel_size,
+                                            stride, block_size, false);
+    return {at::empty({k.size(1), 0, topk}, q.options().dtype(at::kInt)), topk_mask(pooled, topk, n64)};
 }
 
 // ---- Stage 2 (mha_varlen_fwd, flash_api.cpp:519-782; mha_varlen_bwd, :1278-1547) ---------------------------------------
@@ -676,8 +710,7 @@ std::tuple<Tensor, OptTensor> decode_step(const Tensor& q, const Tensor& kn, con
     auto [new_lens, pooled] = decode_front(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, max_len, kernel_size,
                                            stride, block_size, topk > 0, local_blocks, init_blocks, scale);
     if (topk <= 0) return {new_lens, std::nullopt};
-    auto [idx, mask] = topk_blocks(pooled, topk, true, true, false, std::nullopt);
-    return {new_lens, mask->unsqueeze(2)};
+    return {new_lens, topk_mask(pooled, topk, std::nullopt).unsqueeze(2)};
 }
 
 // A whole decode step on selected blocks: the front, the selection and the attention.  The selection is made by the
@@ -752,6 +785,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("window_blocks", &window_blocks);
     m.def("topk_to_uint64", &topk_to_uint64);
     m.def("select_blocks", &select_blocks);
+    m.def("select_mask", &select_mask);
     m.def("varlen_fwd", &varlen_fwd);
     m.def("varlen_bwd", &varlen_bwd);
     m.def("fwd_kvcache", &fwd_kvcache);

@@ -41,7 +41,7 @@ constexpr uint32_t kKeyNegInfFp16 = 0x10000u - 0xfc00u;
 struct TopkParams {
     const uint16_t* x;
     int64_t row_stride;
-    int32_t* out_idx;
+    int32_t* out_idx;                // null: only the mask words are wanted
     uint16_t* out_val;               // optional: the selected values, in output order
     uint64_t* out_mask;              // optional: (rows, n64) mask words of the selection
     int out_stride, n64;
@@ -123,8 +123,12 @@ __device__ __forceinline__ uint32_t bitonic_sort_desc(uint32_t x) {      // 64 k
     return bitonic_merge<kSize, kSize / 2>(x);
 }
 
+// What becomes of the selected columns besides their mask words: a list in value order, one in column order, or nothing (a third of the
+// instructions are the list's: 65 536 rows of 512 columns 57 -> 40 us, 262 144 of 2048 618 -> 446).
+enum TopkList { kByValue, kByColumn, kNoList };
+
 // kFull: the row has exactly 64 * kItems columns (no lane ever holds "no element")
-template <int kItems, bool kByIndex, bool kMask, bool kFull>
+template <int kItems, TopkList kList, bool kMask, bool kFull>
 __global__ __launch_bounds__(kTopkWaves * 64)
 void topk_rows_kernel(const TopkParams p) {
     extern __shared__ uint32_t lds_keys[];                    // kTopkWaves * (k + 64): survivors, then one dummy slot per lane
@@ -227,12 +231,14 @@ void topk_rows_kernel(const TopkParams p) {
         uint32_t words0_lo = 0, words0_hi = 0, words1_lo = 0, words1_hi = 0;   // lane e holds mask word e (e + 64)
         const uint32_t inv_lane = 0xffffu - static_cast<uint32_t>(lane);
         auto emit = [&](int e, bool take, uint64_t take_mask) {
-            const int slot = lanes_below(take_mask, base);
-            uint32_t val;
-            if constexpr (kByIndex) val = static_cast<uint32_t>(e * 64 + lane);
-            else val = (key[e] << 16) | (inv_lane - static_cast<uint32_t>(e * 64));
-            sel[take ? slot : dummy] = val;
-            base += __builtin_popcountll(take_mask);
+            if constexpr (kList != kNoList) {
+                const int slot = lanes_below(take_mask, base);
+                uint32_t val;
+                if constexpr (kList == kByColumn) val = static_cast<uint32_t>(e * 64 + lane);
+                else val = (key[e] << 16) | (inv_lane - static_cast<uint32_t>(e * 64));
+                sel[take ? slot : dummy] = val;
+                base += __builtin_popcountll(take_mask);
+            }
             if constexpr (kMask) {                             // the ballot is the mask word
                 if (e < 64) write_lane64(words0_lo, words0_hi, take_mask, e & 63);
                 else write_lane64(words1_lo, words1_hi, take_mask, e & 63);
@@ -262,6 +268,7 @@ void topk_rows_kernel(const TopkParams p) {
             const uint64_t words1 = (static_cast<uint64_t>(words1_hi) << 32) | words1_lo;
             for (int w = lane; w < p.n64; w += 64) mask_row[w] = w < 64 ? words0 : (w < 128 ? words1 : 0ull);
         }
+        if constexpr (kList == kNoList) continue;
         const int taken = base;                                // <= k_sel
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_wave_barrier();
@@ -270,7 +277,7 @@ void topk_rows_kernel(const TopkParams p) {
         int32_t* dst = p.out_idx + row * p.out_stride;
         uint16_t* dst_val = p.out_val ? p.out_val + row * p.out_stride : nullptr;
         const uint16_t* src = p.x + row * p.row_stride;
-        if constexpr (kByIndex) {
+        if constexpr (kList == kByColumn) {
             for (int i = lane; i < taken; i += 64) {
                 const uint32_t col = sel[i];
                 dst[i] = static_cast<int32_t>(col);
@@ -392,7 +399,7 @@ void topk_wide_kernel(const TopkParams p) {
         const bool take = key[e] > thr || (!no_equal && key[e] == thr && equal + lanes_below(eq_mask, 0) < ties);
         const uint64_t take_mask = __builtin_amdgcn_ballot_w64(take);
         if (mask_row && lane == 0 && word < p.n64) mask_row[word] = take_mask;
-        if (take) {
+        if (take && p.out_idx != nullptr) {
             const int col = word * 64 + lane;
             const int slot = lanes_below(take_mask, above + (equal < ties ? equal : ties));
             sel[slot] = p.by_index ? static_cast<uint32_t>(col) : (key[e] << 16) | (0xffffu - static_cast<uint32_t>(col));
@@ -400,6 +407,7 @@ void topk_wide_kernel(const TopkParams p) {
     }
     if (mask_row)
         for (int w = kItems * kTopkRowWaves + tid; w < p.n64; w += kTopkRowWaves * 64) mask_row[w] = 0ull;
+    if (p.out_idx == nullptr) return;                          // uniform
     __syncthreads();
     int32_t* dst = p.out_idx + row * p.out_stride;
     uint16_t* dst_val = p.out_val ? p.out_val + row * p.out_stride : nullptr;
@@ -447,16 +455,18 @@ static int launch_topk(void* stream, const TopkParams& p) {
     const size_t lds = sizeof(uint32_t) * kTopkWaves * (p.k + 64);
     const dim3 grid(static_cast<unsigned>(blocks)), block(kTopkWaves * 64);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const int variant = (p.by_index ? 4 : 0) | (p.out_mask ? 2 : 0) | (p.n == kItems * 64 ? 1 : 0);
+    const int variant = (p.out_idx == nullptr ? 8 : p.by_index ? 4 : 0) | (p.out_mask ? 2 : 0) | (p.n == kItems * 64 ? 1 : 0);
     switch (variant) {
-        case 0: hipLaunchKernelGGL((topk_rows_kernel<kItems, false, false, false>), grid, block, lds, st, p); break;
-        case 1: hipLaunchKernelGGL((topk_rows_kernel<kItems, false, false, true>), grid, block, lds, st, p); break;
-        case 2: hipLaunchKernelGGL((topk_rows_kernel<kItems, false, true, false>), grid, block, lds, st, p); break;
-        case 3: hipLaunchKernelGGL((topk_rows_kernel<kItems, false, true, true>), grid, block, lds, st, p); break;
-        case 4: hipLaunchKernelGGL((topk_rows_kernel<kItems, true, false, false>), grid, block, lds, st, p); break;
-        case 5: hipLaunchKernelGGL((topk_rows_kernel<kItems, true, false, true>), grid, block, lds, st, p); break;
-        case 6: hipLaunchKernelGGL((topk_rows_kernel<kItems, true, true, false>), grid, block, lds, st, p); break;
-        default: hipLaunchKernelGGL((topk_rows_kernel<kItems, true, true, true>), grid, block, lds, st, p); break;
+        case 0: hipLaunchKernelGGL((topk_rows_kernel<kItems, kByValue, false, false>), grid, block, lds, st, p); break;
+        case 1: hipLaunchKernelGGL((topk_rows_kernel<kItems, kByValue, false, true>), grid, block, lds, st, p); break;
+        case 2: hipLaunchKernelGGL((topk_rows_kernel<kItems, kByValue, true, false>), grid, block, lds, st, p); break;
+        case 3: hipLaunchKernelGGL((topk_rows_kernel<kItems, kByValue, true, true>), grid, block, lds, st, p); break;
+        case 4: hipLaunchKernelGGL((topk_rows_kernel<kItems, kByColumn, false, false>), grid, block, lds, st, p); break;
+        case 5: hipLaunchKernelGGL((topk_rows_kernel<kItems, kByColumn, false, true>), grid, block, lds, st, p); break;
+        case 6: hipLaunchKernelGGL((topk_rows_kernel<kItems, kByColumn, true, false>), grid, block, lds, st, p); break;
+        case 7: hipLaunchKernelGGL((topk_rows_kernel<kItems, kByColumn, true, true>), grid, block, lds, st, p); break;
+        case 10: hipLaunchKernelGGL((topk_rows_kernel<kItems, kNoList, true, false>), grid, block, 0, st, p); break;
+        default: hipLaunchKernelGGL((topk_rows_kernel<kItems, kNoList, true, true>), grid, block, 0, st, p); break;
     }
     IV2_LAUNCH_CHECK();
     return 0;
@@ -516,6 +526,14 @@ extern "C" int infllmv2_topk_select(void* stream, const void* pooled, int64_t ro
     IV2_CHECK(topk_idx != nullptr, "topk_select: topk_idx must be given");
     return topk_dispatch(stream, static_cast<const uint16_t*>(pooled), row_stride, topk_idx, nullptr, mask_words,
                          n_uint64_per_row, k, rows, n, k, by_index ? 1 : 0, drop_neg_inf ? 1 : 0, dtype);
+}
+
+extern "C" int infllmv2_topk_mask(void* stream, const void* pooled, int64_t row_stride, int dtype, uint64_t* mask_words,
+                                  int64_t rows, int n, int k, int n_uint64_per_row, int drop_neg_inf) {
+    IV2_CHECK(dtype == 0 || dtype == 1, "topk_mask: dtype must be 0 (fp16) or 1 (bf16)");
+    IV2_CHECK(mask_words != nullptr, "topk_mask: mask_words must be given");
+    return topk_dispatch(stream, static_cast<const uint16_t*>(pooled), row_stride, nullptr, nullptr, mask_words, n_uint64_per_row, k, rows, n, k, 1,
+                         drop_neg_inf ? 1 : 0, dtype);
 }
 
 extern "C" int infllmv2_topk(void* stream, int num_tokens, int dim, int top, int dtype, const void* x,

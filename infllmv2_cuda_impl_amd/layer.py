@@ -105,12 +105,11 @@ class InfLLMv2Attention(torch.nn.Module):
         if self.selection == "window" and max_seqlen > self.dense_len:
             topk_idx, mask = self._window_blocks(k.shape[1], q.shape[0], cu_seqlens, None, max_seqlen, 0)
         elif self.selection == "sparse" and max_seqlen > self.dense_len:
-            # the selection launch also writes the packed mask Stage 2 walks; plain prefill: no cached tokens in any sequence
+            # the selection launch writes the packed mask Stage 2 walks, and no list
             scale = q.shape[-1] ** (-0.5) if self.softmax_scale is None else self.softmax_scale
             qs, ks = (q, k) if q.shape[-1] == HEAD_DIM else pad_head_dim(q, k)
-            topk_idx, mask = _lib.host.select_blocks(qs.detach(), ks.detach(), cu_seqlens, cu_seqlens, max_seqlen, max_seqlen, self.topk,
-                                                     self.local_blocks, self.init_blocks, None, 0, scale, True, self.kernel_size,
-                                                     self.stride, self.block_size, False, True, False, False)
+            topk_idx, mask = _lib.host.select_mask(qs.detach(), ks.detach(), cu_seqlens, max_seqlen, self.topk, self.local_blocks, self.init_blocks, scale,
+                                                   self.kernel_size, self.stride, self.block_size)
         out = attend_varlen(q, k, v, cu_seqlens, cu_seqlens, max_seqlen, max_seqlen, softmax_scale=self.softmax_scale, causal=True, topk_idx=topk_idx,
                             block_mask=mask, alike=self.selection == "window")
         if cache is not None:
