@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define INFLLMV2_ABI_VERSION 15
+#define INFLLMV2_ABI_VERSION 16
 
 /* ---- library ------------------------------------------------------------------------------ */
 
@@ -150,6 +150,13 @@ int infllmv2_compress_keys_pair(void* stream, const void* k, void* out_a, void* 
                                 int32_t* cu_seqlens_out_a, int32_t* cu_seqlens_out_b, int batch, int max_seqlen_k,
                                 int num_heads_k, int head_dim, int64_t k_row_stride, int64_t k_head_stride,
                                 int kernel_size_a, int stride_a, int kernel_size_b, int stride_b);
+
+/* infllmv2_compress_keys_pair and infllmv2_pack_kv (below) in one launch: what prefill needs of k and v before its first scores.
+ * k_strides, v_strides {row, head}; head_dim 128; workspace: infllmv2_kv_image_bytes() bytes, 16-byte aligned. */
+int infllmv2_compress_keys_and_pack(void* stream, const void* k, const void* v, void* out_a, void* out_b, const int32_t* cu_seqlens_k,
+                                    int32_t* cu_seqlens_out_a, int32_t* cu_seqlens_out_b, void* workspace, size_t workspace_bytes,
+                                    int batch, int64_t total_k, int max_seqlen_k, int num_heads_k, int head_dim, const int64_t* k_strides,
+                                    const int64_t* v_strides, int kernel_size_a, int stride_a, int kernel_size_b, int stride_b);
 
 /* The same means for per-sequence key caches, as a batched decode loop keeps them: kcache (batch, capacity, Hk, d)
  * holds new_lens[b] keys of sequence b, out_cache (batch, rows capacity, Hk, d) its compressed keys; strides
@@ -460,6 +467,11 @@ int infllmv2_compress_keys_pair_f16(void* stream, const void* k, void* out_a, vo
                                     int32_t* cu_seqlens_out_a, int32_t* cu_seqlens_out_b, int batch, int max_seqlen_k,
                                     int num_heads_k, int head_dim, int64_t k_row_stride, int64_t k_head_stride,
                                     int kernel_size_a, int stride_a, int kernel_size_b, int stride_b);
+int infllmv2_compress_keys_and_pack_f16(void* stream, const void* k, const void* v, void* out_a, void* out_b, const int32_t* cu_seqlens_k,
+                                        int32_t* cu_seqlens_out_a, int32_t* cu_seqlens_out_b, void* workspace, size_t workspace_bytes,
+                                        int batch, int64_t total_k, int max_seqlen_k, int num_heads_k, int head_dim,
+                                        const int64_t* k_strides, const int64_t* v_strides, int kernel_size_a, int stride_a,
+                                        int kernel_size_b, int stride_b);
 int infllmv2_compress_keys_cache_f16(void* stream, const void* kcache, void* out_cache, const int32_t* old_lens,
                                      const int32_t* new_lens, int32_t* out_lens, int batch, int max_new_rows,
                                      int num_heads_k, int head_dim, const int64_t* kcache_strides,

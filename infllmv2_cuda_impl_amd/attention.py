@@ -77,7 +77,7 @@ def pad_head_dim(*tensors):
 
 
 def _varlen_forward(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p, softmax_scale, causal, window_size,
-                    softcap, alibi_slopes, block_table, topk_idx, block_mask, alike):
+                    softcap, alibi_slopes, block_table, topk_idx, block_mask, alike, images=None):
     """The forward without autograd.  Returns (q, k, v as used, out, lse, packed mask or None, causal flag of the launch)."""
     causal = _reject_unsupported(dropout_p, window_size, softcap, alibi_slopes, causal, max_seqlen_k)
     if block_table is not None:
@@ -87,7 +87,7 @@ def _varlen_forward(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqle
     q, k, v = _dense_last_dim(q), _dense_last_dim(k), _dense_last_dim(v)
     # with block_mask - the packed selection itself (topk_blocks(return_mask=True)) - there is nothing to pack
     out, lse, mask = _lib.host.varlen_fwd(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, softmax_scale, causal,
-                                          topk_idx, block_mask, alike)
+                                          topk_idx, block_mask, alike, images)
     return q, k, v, out, lse, mask, causal
 
 
@@ -97,12 +97,12 @@ class Infllmv2AttnVarlenFunc(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p, softmax_scale,
                 causal, window_size, softcap, alibi_slopes, deterministic, return_softmax, block_table, topk_idx,
-                block_mask=None, alike=False):
+                block_mask=None, alike=False, images=None):
         if softmax_scale is None:
             softmax_scale = q.shape[-1] ** (-0.5)
         q, k, v, out, lse, fwd_mask, causal = _varlen_forward(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p,
                                                               softmax_scale, causal, window_size, softcap, alibi_slopes, block_table,
-                                                              topk_idx, block_mask, alike)
+                                                              topk_idx, block_mask, alike, images)
         ctx.save_for_backward(q, k, v, out, lse, cu_seqlens_q, cu_seqlens_k, fwd_mask)
         ctx.max_seqlen_q = max_seqlen_q
         ctx.max_seqlen_k = max_seqlen_k
@@ -126,7 +126,7 @@ class Infllmv2AttnVarlenFunc(torch.autograd.Function):
         q, k, v, out, lse, cu_seqlens_q, cu_seqlens_k, fwd_mask = ctx.saved_tensors
         dq, dk, dv = _lib.host.varlen_bwd(dout, q, k, v, out, lse, cu_seqlens_q, cu_seqlens_k, ctx.max_seqlen_q, ctx.max_seqlen_k,
                                           ctx.softmax_scale, ctx.causal, fwd_mask, ctx.sparse, ctx.deterministic, ctx.most_selected)
-        return (dq, dk, dv) + (None,) * 16
+        return (dq, dk, dv) + (None,) * 17
 
 
 def _differentiated(*tensors):
@@ -167,10 +167,11 @@ def infllmv2_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q,
 
 def attend_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p=0.0, softmax_scale=None, causal=False,
                   window_size=(-1, -1), softcap=0.0, alibi_slopes=None, deterministic=False, return_attn_probs=False, block_table=None,
-                  topk_idx=None, block_mask=None, alike=False):
+                  topk_idx=None, block_mask=None, alike=False, images=None):
     """:func:`infllmv2_attn_varlen_func` for callers that know more about the selection: ``alike`` says that neighbouring tokens
     select the same blocks but for a few (a window).  It decides, together with the width of ``topk_idx``, which walk is taken; results
-    differ by rounding at most."""
+    differ by rounding at most.  ``images``: the block images of these k and v that the selection made in its first launch
+    (``select_mask``); without them the call makes them."""
     head_size_og = q.shape[-1]
     if softmax_scale is None:
         softmax_scale = head_size_og ** (-0.5)
@@ -179,10 +180,10 @@ def attend_varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_
     if not return_attn_probs and head_size_og == HEAD_DIM and not _differentiated(q, k, v):
         # nothing to differentiate: skip the autograd node (it costs as much host time as the launches)
         return _varlen_forward(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p, softmax_scale, causal,
-                               window_size, softcap, alibi_slopes, block_table, topk_idx, block_mask, alike)[3]
+                               window_size, softcap, alibi_slopes, block_table, topk_idx, block_mask, alike, images)[3]
     res = Infllmv2AttnVarlenFunc.apply(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, dropout_p,
                                        softmax_scale, causal, window_size, softcap, alibi_slopes, deterministic,
-                                       return_attn_probs, block_table, topk_idx, block_mask, alike)
+                                       return_attn_probs, block_table, topk_idx, block_mask, alike, images)
     if head_size_og == HEAD_DIM:
         return res
     if isinstance(res, tuple):

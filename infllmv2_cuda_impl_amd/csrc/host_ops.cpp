@@ -159,6 +159,42 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> compress_keys_pair(const Tensor& k, c
     return {a.size(0) == rows_a ? a : a.narrow(0, 0, rows_a), cu_a, b.size(0) == rows_b ? b : b.narrow(0, 0, rows_b), cu_b};
 }
 
+// Whether the block images of (k, v) are made where k is compressed, for attention that follows the scores of q: k and v are as the attention takes them,
+// without a copy, no sequence is so long that it is walked in step (with counters that the packing clears for the one launch behind it), and the images
+// are still in the 256 MB behind the L2s when the scores have read q.  Packed just before the walk, they are there in any case: with 64 blocks
+// selected and 2 KV heads of 16 query heads, packing early gains 3 us of a whole prefill at 512 and 2048 tokens, 7 at 12 288 and 16 384 (128 MiB of q) and
+// nothing at 20 480 to 28 672, and at 32 768 the walk is 1 to 3 % slower for it (2.81 -> 2.87 ms).
+constexpr int64_t kPackEarlyBytes = 128ll << 20, kPackEarlyKeys = 32768;
+bool pack_early(const Tensor& q, const Tensor& k, const Tensor& v, int64_t max_seqlen_k) {
+    if (q.numel() * q.element_size() > kPackEarlyBytes || max_seqlen_k > kPackEarlyKeys) return false;
+    const auto fits = [](const Tensor& t) {
+        return t.stride(2) == 1 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0;
+    };
+    return k.dim() == 3 && k.size(2) == kHeadDim && v.dim() == 3 && v.sizes() == k.sizes() && v.scalar_type() == k.scalar_type() &&
+           v.device() == k.device() && fits(k) && fits(v);
+}
+Tensor image_workspace(const Tensor& k, int64_t batch) { return bytes_on(k, infllmv2_kv_image_bytes(k.size(0), as_int(batch), as_int(k.size(1)))); }
+
+// compress_keys_pair that also gives the block images of (k, v)
+std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> compress_keys_and_pack(const Tensor& k, const Tensor& v, const Tensor& cu, int64_t max_seqlen_k,
+                                                                          int64_t ks_a, int64_t st_a, int64_t ks_b, int64_t st_b) {
+    check_compress(k, cu);
+    TORCH_CHECK(st_a > 0 && st_b > 0, "compress_keys_pair: kernel_size and stride must be positive");
+    const int64_t batch = cu.numel() - 1;
+    const int64_t rows_a = compressed_rows_bound(batch, k.size(0), max_seqlen_k, ks_a, st_a);
+    const int64_t rows_b = compressed_rows_bound(batch, k.size(0), max_seqlen_k, ks_b, st_b);
+    DeviceGuard guard(k.device());
+    Tensor a = compressed_buffer(k, rows_a), b = compressed_buffer(k, rows_b);
+    Tensor cu_a = at::empty({batch + 1}, cu.options()), cu_b = at::empty({batch + 1}, cu.options());
+    Tensor images = image_workspace(k, batch);
+    const S2 ks = rows_heads(k), vs = rows_heads(v);
+    auto fn = is_half(k) ? infllmv2_compress_keys_and_pack_f16 : infllmv2_compress_keys_and_pack;
+    check_rc(fn(stream_of(k), ptr(k), ptr(v), ptr(a), ptr(b), iptr(cu), static_cast<int32_t*>(ptr(cu_a)), static_cast<int32_t*>(ptr(cu_b)),
+                ptr(images), static_cast<size_t>(images.numel()), as_int(batch), k.size(0), as_int(max_seqlen_k), as_int(k.size(1)),
+                as_int(k.size(2)), ks.v, vs.v, as_int(ks_a), as_int(st_a), as_int(ks_b), as_int(st_b)), "compress_keys_and_pack");
+    return {a.size(0) == rows_a ? a : a.narrow(0, 0, rows_a), cu_a, b.size(0) == rows_b ? b : b.narrow(0, 0, rows_b), cu_b, images};
+}
+
 // ---- Stage 1 (mha_varlen_fwd_stage1, flash_api.cpp:784-1049) ---------------------------------------------------------
 // a key set with no rows (sequences shorter than one window) still needs a valid pointer; no row of it is read
 Tensor readable(const Tensor& t) { return t.size(0) > 0 ? t : at::zeros({1, t.size(1), t.size(2)}, t.options()); }
@@ -402,16 +438,21 @@ Tensor topk_to_uint64(const Tensor& topk_idx, int64_t k_blocks, const OptTensor&
 }
 
 // the selection front end: compressed keys, fused Stage 1 and pooling, top-k with the mask words
-// Block scores (Hk, total_q, blocks) of packed queries, and how many mask words a row of the selection takes.
+// Block scores (Hk, total_q, blocks) of packed queries, and how many mask words a row of the selection takes.  images: where the block
+// images of (k, v) go, which are then made in the same launch as the compressed keys where pack_early says so.
 std::tuple<Tensor, int64_t> block_scores(const Tensor& q_, const Tensor& k, const Tensor& cu_q, const Tensor& cu_k, int64_t max_q,
                                          int64_t max_k, int64_t local_blocks, int64_t init_blocks, const OptTensor& cache_lens,
                                          int64_t max_cache_len, double scale, bool causal, int64_t kernel_size, int64_t stride,
-                                         int64_t block_size, bool exact_lse) {
+                                         int64_t block_size, bool exact_lse, const Tensor* v = nullptr, OptTensor* images = nullptr) {
     const Tensor q = q_.stride(-1) == 1 ? q_ : q_.contiguous();
     Tensor kf, cu_f, kc, cu_c;
     if (exact_lse) {
         std::tie(kf, cu_f) = compress_keys(k, cu_k, max_k, kernel_size, stride, std::nullopt, 0);
         kc = kf; cu_c = cu_f;
+    } else if (images != nullptr && pack_early(q, k, *v, max_k)) {
+        Tensor packed;
+        std::tie(kf, cu_f, kc, cu_c, packed) = compress_keys_and_pack(k, *v, cu_k, max_k, kernel_size, stride, 4 * kernel_size, 4 * stride);
+        *images = packed;
     } else {
         std::tie(kf, cu_f, kc, cu_c) = compress_keys_pair(k, cu_k, max_k, kernel_size, stride, 4 * kernel_size, 4 * stride);
     }
@@ -432,19 +473,23 @@ std::tuple<Tensor, OptTensor> select_blocks(const Tensor& q, const Tensor& k, co
     return topk_blocks(pooled, topk, return_mask, by_index, drop_unreachable, n64);
 }
 
-// The selection of plain prefill for a caller that goes on with the mask: {an empty list whose width says how many blocks a row has at most, mask}.
-std::tuple<Tensor, Tensor> select_mask(const Tensor& q, const Tensor& k, const Tensor& cu, int64_t max_len, int64_t topk, int64_t local_blocks,
-                                       int64_t init_blocks, double scale, int64_t kernel_size, int64_t stride, int64_t block_size) {
+// The selection of plain prefill for a caller that goes on with the mask and attends to the same k and v: {an empty list whose width says how many
+// blocks a row has at most, mask, the block images of (k, v) for varlen_fwd or none}.
+std::tuple<Tensor, Tensor, OptTensor> select_mask(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu, int64_t max_len, int64_t topk,
+                                                  int64_t local_blocks, int64_t init_blocks, double scale, int64_t kernel_size, int64_t stride,
+                                                  int64_t block_size) {
+    OptTensor images;
     const auto [pooled, n64] = block_scores(q, k, cu, cu, max_len, max_len, local_blocks, init_blocks, std::nullopt, 0, scale, true, kernel_size,
-                                            stride, block_size, false);
-    return {at::empty({k.size(1), 0, topk}, q.options().dtype(at::kInt)), topk_mask(pooled, topk, n64)};
+                                            stride, block_size, false, &v, &images);
+    return {at::empty({k.size(1), 0, topk}, q.options().dtype(at::kInt)), topk_mask(pooled, topk, n64), images};
 }
 
 // ---- Stage 2 (mha_varlen_fwd, flash_api.cpp:519-782; mha_varlen_bwd, :1278-1547) ---------------------------------------
-// Returns {out, lse, packed mask or none}.  lse: (Hk, total_q * group) on the sparse path, (Hq, total_q) on the dense one.
+// images: of (k, v), as select_mask gives them.  Returns {out, lse, packed mask or none}.  lse: (Hk, total_q * group) on the sparse path,
+// (Hq, total_q) on the dense one.
 std::tuple<Tensor, Tensor, OptTensor> varlen_fwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& cu_q, const Tensor& cu_k,
                                                  int64_t max_q, int64_t max_k, double scale, bool causal, const OptTensor& topk_idx,
-                                                 const OptTensor& block_mask, bool alike) {
+                                                 const OptTensor& block_mask, bool alike, const OptTensor& images) {
     check_qkv(q, k, v, cu_q, cu_k, true);
     DeviceGuard guard(q.device());
     const int64_t batch = cu_q.numel() - 1, total_q = q.size(0), hq = q.size(1), d = q.size(2), total_k = k.size(0), hk = k.size(1);
@@ -469,16 +514,19 @@ std::tuple<Tensor, Tensor, OptTensor> varlen_fwd(const Tensor& q, const Tensor& 
     Tensor lse = sparse ? at::empty({hk, total_q * group}, q.options().dtype(at::kFloat))             // flash_api.cpp:665
                         : at::empty({hq, total_q}, q.options().dtype(at::kFloat));
     const int64_t lse_strides[3] = {sparse ? group : 1, sparse ? 1 : total_q, group * total_q};
-    Tensor ws = bytes_on(q, infllmv2_kv_image_bytes(total_k, as_int(batch), as_int(hk)));
+    TORCH_CHECK(!images.has_value() || (images->device() == k.device() && images->is_contiguous() && images->scalar_type() == at::kByte &&
+                                        images->numel() >= static_cast<int64_t>(infllmv2_kv_image_bytes(total_k, as_int(batch), as_int(hk)))),
+                "images must hold the block images of k and v");
+    Tensor ws = images.has_value() ? *images : image_workspace(k, batch);
     const S3 qs = grouped(q, group), os = grouped(out, group);
     const S2 ks = rows_heads(k), vs = rows_heads(v);
     auto fn = is_half(q) ? infllmv2_varlen_fwd_selected_f16 : infllmv2_varlen_fwd_selected;
     // a mask that came with its indices has at most so many blocks to a row (negative: neighbouring rows are alike)
     const int listed = sparse && topk_idx.has_value() && topk_idx->dim() > 0 ? as_int(topk_idx->size(-1)) : 0, most_selected = alike ? -listed : listed;
     check_rc(fn(stream_of(q), ptr(q), ptr(k), ptr(v), ptr(out), static_cast<float*>(ptr(lse)), iptr(cu_q), iptr(cu_k),
-                sparse ? static_cast<const uint64_t*>(mask->data_ptr()) : nullptr, ptr(ws), static_cast<size_t>(ws.numel()), 0, as_int(batch),
-                total_q, total_k, as_int(hq), as_int(hk), as_int(d), as_int(max_q), as_int(max_k), qs.v, ks.v, vs.v, os.v, lse_strides,
-                sparse ? as_int(mask->size(-1)) : 0, static_cast<float>(scale), causal ? 1 : 0, most_selected), "varlen_fwd");
+                sparse ? static_cast<const uint64_t*>(mask->data_ptr()) : nullptr, ptr(ws), static_cast<size_t>(ws.numel()),
+                images.has_value() ? 1 : 0, as_int(batch), total_q, total_k, as_int(hq), as_int(hk), as_int(d), as_int(max_q), as_int(max_k), qs.v,
+                ks.v, vs.v, os.v, lse_strides, sparse ? as_int(mask->size(-1)) : 0, static_cast<float>(scale), causal ? 1 : 0, most_selected), "varlen_fwd");
     return {out, lse, mask};
 }
 

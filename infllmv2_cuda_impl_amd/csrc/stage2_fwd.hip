@@ -26,61 +26,10 @@ namespace IV2_NS {
 // ---------------------------------------------------------------------------------------------
 // K/V -> block images
 // ---------------------------------------------------------------------------------------------
-struct PackParams {
-    const elem_bits* k;
-    const elem_bits* v;
-    elem_bits* kimg;                // K in K-image order (operand of a GEMM contracting over d)
-    elem_bits* vimg;                // V in V-image order (A operand of a GEMM contracting over keys)
-    const int* cu_seqlens_k;
-    int64_t k_row_stride, k_head_stride;
-    int64_t v_row_stride, v_head_stride;
-    int64_t n_slots;
-    unsigned* in_step;              // counters of in_step.h to clear for the launch that walks the images, or null (a launch of its own took 10 us)
-};
-static_assert(8 * kInStepPitch == 256, "one counter word per thread of a packing workgroup");
-
-constexpr int kVPad = 8;            // LDS row padding (elements) for the V transposition
-
 __global__ __launch_bounds__(256)
 void pack_kv_kernel(const PackParams p) {
-    __shared__ __attribute__((aligned(16))) elem_bits vt[kBlockN][kHeadDim + kVPad];
-    const int j = blockIdx.x, b = blockIdx.y, h = blockIdx.z;
-    if (p.in_step != nullptr && j + b + h == 0) p.in_step[threadIdx.x] = 0u;
-    const int k0 = p.cu_seqlens_k[b];
-    const int Sk = p.cu_seqlens_k[b + 1] - k0;
-    if (static_cast<int64_t>(j) * kBlockN >= Sk) return;
-    const int64_t slot = image_slot0(p.cu_seqlens_k, b) + j;
-    const int tid = threadIdx.x;
-    const elem_bits* kb = p.k + (k0 + static_cast<int64_t>(j) * kBlockN) * p.k_row_stride + h * p.k_head_stride;
-    const elem_bits* vb = p.v + (k0 + static_cast<int64_t>(j) * kBlockN) * p.v_row_stride + h * p.v_head_stride;
-    const int64_t img_off = (static_cast<int64_t>(h) * p.n_slots + slot) * kImageElems;
-    const int valid = Sk - j * kBlockN;                       // keys of this block inside the sequence
-    uint4 val[4];                                             // requested together with K's rows
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int u = tid + 256 * i, key = u >> 4, d0 = (u & 15) * 8;
-        val[i] = make_uint4(0, 0, 0, 0);
-        if (key < valid) val[i] = *reinterpret_cast<const uint4*>(vb + key * p.v_row_stride + d0);
-    }
-    write_k_image(kb, p.k_row_stride, valid, p.kimg + img_off, tid);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int u = tid + 256 * i;
-        *reinterpret_cast<uint4*>(&vt[u >> 4][(u & 15) * 8]) = val[i];
-    }
-    __syncthreads();
-    for (int u = tid; u < 1024; u += 256) {
-        const int dt = u >> 7, cc = (u >> 6) & 1, lane = u & 63;
-        const int r = lane & 15, g = lane >> 4;
-        const int d = 16 * dt + r;
-        uint32_t w[4];
-#pragma unroll
-        for (int jj = 0; jj < 8; jj += 2) {
-            const int key_a = 32 * cc + (jj < 4 ? 4 * g + jj : 16 + 4 * g + jj - 4);
-            w[jj >> 1] = static_cast<uint32_t>(vt[key_a][d]) | (static_cast<uint32_t>(vt[key_a + 1][d]) << 16);
-        }
-        *reinterpret_cast<uint4*>(p.vimg + img_off + u * 8) = make_uint4(w[0], w[1], w[2], w[3]);
-    }
+    __shared__ __attribute__((aligned(16))) elem_bits rows[kPackElems];
+    pack_block(p, blockIdx.x, blockIdx.y, blockIdx.z, rows);
 }
 
 }  // namespace IV2_NS
@@ -111,19 +60,9 @@ int launch_pack(hipStream_t st, const void* k, const void* v, const int32_t* cu_
                 const int64_t* k_strides, const int64_t* v_strides, unsigned* in_step) {
     const int rc = check_pack(k, v, cu_seqlens_k, workspace, workspace_bytes, batch, total_k, num_heads_k, max_seqlen_k, k_strides, v_strides);
     if (rc != 0) return rc;
-    const int64_t n_slots = image_slots(total_k, batch);
     const int max_blocks = (max_seqlen_k + kBlockN - 1) / kBlockN;
     if (max_blocks == 0 || total_k == 0) return 0;
-    PackParams pp{};
-    pp.k = static_cast<const elem_bits*>(k);
-    pp.v = static_cast<const elem_bits*>(v);
-    pp.kimg = static_cast<elem_bits*>(workspace);
-    pp.vimg = pp.kimg + n_slots * num_heads_k * kImageElems;
-    pp.cu_seqlens_k = cu_seqlens_k;
-    pp.k_row_stride = k_strides[0]; pp.k_head_stride = k_strides[1];
-    pp.v_row_stride = v_strides[0]; pp.v_head_stride = v_strides[1];
-    pp.n_slots = n_slots;
-    pp.in_step = in_step;
+    const PackParams pp = pack_params(k, v, cu_seqlens_k, workspace, batch, total_k, num_heads_k, k_strides, v_strides, in_step);
     hipLaunchKernelGGL(pack_kv_kernel, dim3(max_blocks, batch, num_heads_k), dim3(256), 0, st, pp);
     IV2_LAUNCH_CHECK();
     return 0;

@@ -101,17 +101,17 @@ class InfLLMv2Attention(torch.nn.Module):
     def forward(self, q, k, v, cu_seqlens, max_seqlen: int, cache: SequenceCache | None = None):
         """q ``(total, nheads, d)``, k/v ``(total, nheads_k, d)`` packed; returns ``(total, nheads, d)``.
         With ``cache`` (one sequence only) the keys, values and compressed keys are also stored for decoding."""
-        topk_idx = mask = None
+        topk_idx = mask = images = None
         if self.selection == "window" and max_seqlen > self.dense_len:
             topk_idx, mask = self._window_blocks(k.shape[1], q.shape[0], cu_seqlens, None, max_seqlen, 0)
         elif self.selection == "sparse" and max_seqlen > self.dense_len:
-            # the selection launch writes the packed mask Stage 2 walks, and no list
+            # the selection writes the packed mask Stage 2 walks, no list, and the block images of k and v
             scale = q.shape[-1] ** (-0.5) if self.softmax_scale is None else self.softmax_scale
             qs, ks = (q, k) if q.shape[-1] == HEAD_DIM else pad_head_dim(q, k)
-            topk_idx, mask = _lib.host.select_mask(qs.detach(), ks.detach(), cu_seqlens, max_seqlen, self.topk, self.local_blocks, self.init_blocks, scale,
-                                                   self.kernel_size, self.stride, self.block_size)
+            topk_idx, mask, images = _lib.host.select_mask(qs.detach(), ks.detach(), v.detach(), cu_seqlens, max_seqlen, self.topk, self.local_blocks,
+                                                           self.init_blocks, scale, self.kernel_size, self.stride, self.block_size)
         out = attend_varlen(q, k, v, cu_seqlens, cu_seqlens, max_seqlen, max_seqlen, softmax_scale=self.softmax_scale, causal=True, topk_idx=topk_idx,
-                            block_mask=mask, alike=self.selection == "window")
+                            block_mask=mask, alike=self.selection == "window", images=images)
         if cache is not None:
             if cu_seqlens.numel() != 2:
                 raise RuntimeError("a SequenceCache holds one sequence")
