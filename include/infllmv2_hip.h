@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define INFLLMV2_ABI_VERSION 16
+#define INFLLMV2_ABI_VERSION 17
 
 /* ---- library ------------------------------------------------------------------------------ */
 
@@ -317,6 +317,11 @@ int infllmv2_pack_kv(void* stream, const void* k, const void* v, const int32_t* 
                      void* workspace, size_t workspace_bytes, int batch, int64_t total_k,
                      int num_heads_k, int head_dim, int max_seqlen_k, const int64_t* k_strides,
                      const int64_t* v_strides);
+
+/* infllmv2_pack_kv and infllmv2_topk_to_uint64 (topk_idx (rows, topk) -> mask (rows, n_uint64_per_row)) in one launch. */
+int infllmv2_pack_kv_and_topk(void* stream, const void* k, const void* v, const int32_t* cu_seqlens_k, void* workspace, size_t workspace_bytes,
+                              int batch, int64_t total_k, int num_heads_k, int head_dim, int max_seqlen_k, const int64_t* k_strides,
+                              const int64_t* v_strides, const int32_t* topk_idx, uint64_t* mask, int64_t rows, int topk, int n_uint64_per_row);
 
 /* Scratch for infllmv2_varlen_bwd: the K/V block images, the transposed mask, D = rowsum(dO*O),
  * transposed per-token images of q and dout, fp32 dK/dV accumulators. */

@@ -11,7 +11,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libinfllmv2_hip.so")
 
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 _p, _i, _i64, _sz, _f = C.c_void_p, C.c_int, C.c_int64, C.c_size_t, C.c_float
 
@@ -51,6 +51,7 @@ SIGNATURES = {
     "infllmv2_fwd_kvcache_scores": [_p] * 8 + [_i, _i, _p, _sz] + [_i] * 5 + [_p] * 4 + [_i, _f],
     "infllmv2_fwd_kvcache_static": [_p] * 10 + [_i] * 7 + [_p] * 6 + [_i, _i, _f, _p, _p, _p, _i64, _i, _p, _p, _i, _i],
     "infllmv2_pack_kv": [_p, _p, _p, _p, _p, _sz, _i, _i64, _i, _i, _i, _p, _p],
+    "infllmv2_pack_kv_and_topk": [_p, _p, _p, _p, _p, _sz, _i, _i64, _i, _i, _i, _p, _p, _p, _p, _i64, _i, _i],
 }
 # entry points that exist once per element type: the plain name takes bfloat16, name + "_f16" IEEE half
 PER_ELEMENT_TYPE = ["infllmv2_compress_keys", "infllmv2_compress_keys_pair", "infllmv2_compress_keys_and_pack", "infllmv2_compress_keys_cache", "infllmv2_compress_keys_cache_pair", "infllmv2_varlen_fwd_stage1",

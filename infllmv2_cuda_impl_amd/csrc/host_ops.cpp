@@ -164,9 +164,9 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> compress_keys_pair(const Tensor& k, c
 // are still in the 256 MB behind the L2s when the scores have read q.  Packed just before the walk, they are there in any case: with 64 blocks
 // selected and 2 KV heads of 16 query heads, packing early gains 3 us of a whole prefill at 512 and 2048 tokens, 7 at 12 288 and 16 384 (128 MiB of q) and
 // nothing at 20 480 to 28 672, and at 32 768 the walk is 1 to 3 % slower for it (2.81 -> 2.87 ms).
-constexpr int64_t kPackEarlyBytes = 128ll << 20, kPackEarlyKeys = 32768;
+constexpr int64_t kPackEarlyBytes = 128ll << 20, kInStepKeys = 32768;
 bool pack_early(const Tensor& q, const Tensor& k, const Tensor& v, int64_t max_seqlen_k) {
-    if (q.numel() * q.element_size() > kPackEarlyBytes || max_seqlen_k > kPackEarlyKeys) return false;
+    if (q.numel() * q.element_size() > kPackEarlyBytes || max_seqlen_k > kInStepKeys) return false;
     const auto fits = [](const Tensor& t) {
         return t.stride(2) == 1 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0;
     };
@@ -494,7 +494,7 @@ std::tuple<Tensor, Tensor, OptTensor> varlen_fwd(const Tensor& q, const Tensor& 
     DeviceGuard guard(q.device());
     const int64_t batch = cu_q.numel() - 1, total_q = q.size(0), hq = q.size(1), d = q.size(2), total_k = k.size(0), hk = k.size(1);
     const int64_t group = hq / hk;
-    OptTensor mask;
+    OptTensor mask, packed = images;                           // packed: the block images of (k, v), where there are any before the walk's launch
     if (block_mask.has_value()) {
         // rows may be wider than max_seqlen_k needs (select_blocks widens them for cached tokens): the kernels take
         // the width as a row stride and never look at a block beyond the sequence
@@ -507,7 +507,22 @@ std::tuple<Tensor, Tensor, OptTensor> varlen_fwd(const Tensor& q, const Tensor& 
     } else if (topk_idx.has_value()) {
         TORCH_CHECK(topk_idx->dim() == 3 && topk_idx->size(0) == hk && topk_idx->size(1) == total_q,
                     "topk_idx must have shape (num_heads_k, total_q, k)");
-        mask = topk_to_uint64(*topk_idx, (max_k + kBlock - 1) / kBlock, std::nullopt);
+        const int64_t k_blocks = (max_k + kBlock - 1) / kBlock, n64 = (k_blocks + 63) / 64;
+        if (max_k <= kInStepKeys && total_q > 0 && max_q > 0 && !images.has_value()) {
+            // The mask words are made by the launch that packs k and v (2049 queries behind 17 962 keys, from the compressed keys on, 325.2 -> 323.4 us, 512 behind each of three
+            // prompts 219.6 -> 217.2, 2000 tokens 85.4 -> 83.9).  Not for sequences that are
+            // walked in step: the packing clears the counters of the one launch behind it, and is then part of that call.
+            require_gpu(*topk_idx, "topk_idx");
+            const Tensor idx = topk_idx->contiguous();
+            mask = at::empty({hk, total_q, n64}, idx.options().dtype(at::kLong));
+            packed = image_workspace(k, batch);
+            const S2 ks = rows_heads(k), vs = rows_heads(v);
+            check_rc(infllmv2_pack_kv_and_topk(stream_of(q), ptr(k), ptr(v), iptr(cu_k), ptr(*packed), static_cast<size_t>(packed->numel()), as_int(batch),
+                                               total_k, as_int(hk), as_int(d), as_int(max_k), ks.v, vs.v, iptr(idx), static_cast<uint64_t*>(mask->data_ptr()),
+                                               hk * total_q, as_int(idx.size(2)), as_int(n64)), "pack_kv_and_topk");
+        } else {
+            mask = topk_to_uint64(*topk_idx, k_blocks, std::nullopt);
+        }
     }
     Tensor out = at::empty_like(q);
     const bool sparse = mask.has_value();
@@ -517,7 +532,7 @@ std::tuple<Tensor, Tensor, OptTensor> varlen_fwd(const Tensor& q, const Tensor& 
     TORCH_CHECK(!images.has_value() || (images->device() == k.device() && images->is_contiguous() && images->scalar_type() == at::kByte &&
                                         images->numel() >= static_cast<int64_t>(infllmv2_kv_image_bytes(total_k, as_int(batch), as_int(hk)))),
                 "images must hold the block images of k and v");
-    Tensor ws = images.has_value() ? *images : image_workspace(k, batch);
+    Tensor ws = packed.has_value() ? *packed : image_workspace(k, batch);
     const S3 qs = grouped(q, group), os = grouped(out, group);
     const S2 ks = rows_heads(k), vs = rows_heads(v);
     auto fn = is_half(q) ? infllmv2_varlen_fwd_selected_f16 : infllmv2_varlen_fwd_selected;
@@ -525,7 +540,7 @@ std::tuple<Tensor, Tensor, OptTensor> varlen_fwd(const Tensor& q, const Tensor& 
     const int listed = sparse && topk_idx.has_value() && topk_idx->dim() > 0 ? as_int(topk_idx->size(-1)) : 0, most_selected = alike ? -listed : listed;
     check_rc(fn(stream_of(q), ptr(q), ptr(k), ptr(v), ptr(out), static_cast<float*>(ptr(lse)), iptr(cu_q), iptr(cu_k),
                 sparse ? static_cast<const uint64_t*>(mask->data_ptr()) : nullptr, ptr(ws), static_cast<size_t>(ws.numel()),
-                images.has_value() ? 1 : 0, as_int(batch), total_q, total_k, as_int(hq), as_int(hk), as_int(d), as_int(max_q), as_int(max_k), qs.v,
+                packed.has_value() ? 1 : 0, as_int(batch), total_q, total_k, as_int(hq), as_int(hk), as_int(d), as_int(max_q), as_int(max_k), qs.v,
                 ks.v, vs.v, os.v, lse_strides, sparse ? as_int(mask->size(-1)) : 0, static_cast<float>(scale), causal ? 1 : 0, most_selected), "varlen_fwd");
     return {out, lse, mask};
 }

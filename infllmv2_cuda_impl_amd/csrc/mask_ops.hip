@@ -11,35 +11,14 @@
 
 namespace infllmv2 {
 
-// ---------------------------------------------------------------------------------------------
-// topk_idx (rows, k) int32  ->  words (rows, n64) uint64.
-// One wavefront per row.  Each lane ORs its indices into an LDS copy of the row's words
-// (ds_or_b64), then the first n64 lanes store the row: every input index is read exactly once
-// and every output word is written exactly once.
-// ---------------------------------------------------------------------------------------------
+// topk_idx (rows, k) int32 -> words (rows, n64) uint64: see topk_row_words.
 template <int kWavesPerBlock>
 __global__ __launch_bounds__(kWavesPerBlock * 64)
 void topk_to_uint64_kernel(const int32_t* __restrict__ idx, uint64_t* __restrict__ out,
                            int64_t rows, int k, int n64) {
     extern __shared__ unsigned long long lds_words[];          // kWavesPerBlock * n64
-    const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    const int64_t row = static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + wave;
-    unsigned long long* words = lds_words + wave * n64;
-    for (int w = lane; w < n64; w += 64) words[w] = 0ull;
-    __syncthreads();
-    if (row < rows) {
-        const int32_t* src = idx + row * k;
-        const int limit = n64 * 64;
-        for (int i = lane; i < k; i += 64) {
-            const int v = src[i];
-            if (v >= 0 && v < limit) atomicOr(&words[v >> 6], 1ull << (v & 63));
-        }
-    }
-    __syncthreads();
-    if (row < rows) {
-        for (int w = lane; w < n64; w += 64) out[row * n64 + w] = words[w];
-    }
+    topk_row_words(idx, out, static_cast<int64_t>(blockIdx.x) * kWavesPerBlock + wave, rows, k, n64, lds_words + wave * n64, threadIdx.x & 63);
 }
 
 // ---------------------------------------------------------------------------------------------

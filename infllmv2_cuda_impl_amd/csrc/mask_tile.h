@@ -1,7 +1,28 @@
-// Transposition of the block mask, a 64 x 64 bit tile at a time.
+// Block masks: their words from an index list, and their transposition, a 64 x 64 bit tile at a time.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+// Row `row` of topk_idx (rows, k) int32 as words (rows, n64) uint64, by one wavefront of a workgroup whose wavefronts all come here.  Each lane ORs
+// its indices into an LDS copy of the row's words (ds_or_b64), then the first n64 lanes store the row: every input index is read exactly once
+// and every output word is written exactly once.
+static __device__ __forceinline__ void topk_row_words(const int32_t* __restrict__ idx, uint64_t* __restrict__ out, int64_t row, int64_t rows, int k, int n64,
+                                                      unsigned long long* words, int lane) {
+    for (int w = lane; w < n64; w += 64) words[w] = 0ull;
+    __syncthreads();
+    if (row < rows) {
+        const int32_t* src = idx + row * k;
+        const int limit = n64 * 64;
+        for (int i = lane; i < k; i += 64) {
+            const int v = src[i];
+            if (v >= 0 && v < limit) atomicOr(&words[v >> 6], 1ull << (v & 63));
+        }
+    }
+    __syncthreads();
+    if (row < rows) {
+        for (int w = lane; w < n64; w += 64) out[row * n64 + w] = words[w];
+    }
+}
 
 // bwd[h, kb, w] bit u = fwd[h, 64 w + u, kb / 64] bit (kb % 64).  One wavefront takes one tile: lane u holds the forward word of token
 // 64 w + u, 64 ballots produce the 64 backward words of the tile, lane b stores word b.

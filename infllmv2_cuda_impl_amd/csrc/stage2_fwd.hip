@@ -18,6 +18,7 @@
 #include "block_walker.h"
 #include "stage2_fwd.h"
 #include "in_step.h"
+#include "mask_tile.h"
 #include "infllmv2_hip.h"
 #include <math.h>
 
@@ -31,6 +32,24 @@ void pack_kv_kernel(const PackParams p) {
     __shared__ __attribute__((aligned(16))) elem_bits rows[kPackElems];
     pack_block(p, blockIdx.x, blockIdx.y, blockIdx.z, rows);
 }
+
+#ifndef IV2_F16
+// The images, and the mask words of an index list, in one launch: for each sequence and KV head the first `blocks` workgroups pack, the others take four
+// rows of the list each.  Both are bound by latency.
+constexpr int kMaskRowsPerWg = 4;
+
+__global__ __launch_bounds__(256)
+void pack_kv_and_topk_kernel(const PackParams p, int blocks, const int32_t* __restrict__ idx, uint64_t* __restrict__ mask, int64_t rows, int k, int n64) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    if (static_cast<int>(blockIdx.x) < blocks) {
+        pack_block(p, blockIdx.x, blockIdx.y, blockIdx.z, reinterpret_cast<elem_bits*>(lds));
+        return;
+    }
+    const int64_t wg = (static_cast<int64_t>(blockIdx.z) * gridDim.y + blockIdx.y) * (gridDim.x - blocks) + (blockIdx.x - blocks);
+    const int wave = threadIdx.x >> 6;
+    topk_row_words(idx, mask, wg * kMaskRowsPerWg + wave, rows, k, n64, reinterpret_cast<unsigned long long*>(lds) + wave * n64, threadIdx.x & 63);
+}
+#endif
 
 }  // namespace IV2_NS
 
@@ -77,6 +96,27 @@ extern "C" int infllmv2_pack_kv(void* stream, const void* k, const void* v, cons
     IV2_CHECK(head_dim == kHeadDim, "pack_kv: this build only supports head_dim 128 (got %d)", head_dim);
     return launch_pack(static_cast<hipStream_t>(stream), k, v, cu_seqlens_k, workspace, workspace_bytes, batch,
                        total_k, num_heads_k, max_seqlen_k, k_strides, v_strides);
+}
+
+extern "C" int infllmv2_pack_kv_and_topk(void* stream, const void* k, const void* v, const int32_t* cu_seqlens_k, void* workspace, size_t workspace_bytes,
+                                         int batch, int64_t total_k, int num_heads_k, int head_dim, int max_seqlen_k, const int64_t* k_strides,
+                                         const int64_t* v_strides, const int32_t* topk_idx, uint64_t* mask, int64_t rows, int topk, int n_uint64_per_row) {
+    IV2_CHECK(head_dim == kHeadDim, "pack_kv: this build only supports head_dim 128 (got %d)", head_dim);
+    IV2_CHECK(rows >= 0 && topk >= 0 && n_uint64_per_row >= 0 && n_uint64_per_row <= 1024, "pack_kv_and_topk: bad sizes");
+    IV2_CHECK(rows == 0 || n_uint64_per_row == 0 || (mask && (topk_idx || topk == 0)), "pack_kv_and_topk: null pointer");
+    if (int rc = check_pack(k, v, cu_seqlens_k, workspace, workspace_bytes, batch, total_k, num_heads_k, max_seqlen_k, k_strides, v_strides)) return rc;
+    const int blocks = total_k == 0 ? 0 : (max_seqlen_k + kBlockN - 1) / kBlockN;
+    const int64_t pairs = static_cast<int64_t>(batch) * num_heads_k;
+    const int64_t mask_wgs = n_uint64_per_row == 0 ? 0 : ((rows + kMaskRowsPerWg - 1) / kMaskRowsPerWg + pairs - 1) / pairs;
+    if (blocks + mask_wgs == 0) return 0;
+    IV2_CHECK(blocks + mask_wgs <= 0x7fffffffll, "pack_kv_and_topk: too many rows");
+    const PackParams pp = pack_params(k, v, cu_seqlens_k, workspace, batch, total_k, num_heads_k, k_strides, v_strides, nullptr);
+    size_t lds = sizeof(uint64_t) * kMaskRowsPerWg * n_uint64_per_row;
+    if (lds < kPackElems * sizeof(elem_bits)) lds = kPackElems * sizeof(elem_bits);
+    hipLaunchKernelGGL(pack_kv_and_topk_kernel, dim3(static_cast<unsigned>(blocks + mask_wgs), batch, num_heads_k), dim3(256), lds,
+                       static_cast<hipStream_t>(stream), pp, blocks, topk_idx, mask, rows, topk, n_uint64_per_row);
+    IV2_LAUNCH_CHECK();
+    return 0;
 }
 #endif
 
