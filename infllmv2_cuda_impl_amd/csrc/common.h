@@ -138,4 +138,15 @@ __device__ __forceinline__ void warm_kernel_arguments() {
                    "n"(line(5)), "n"(line(6)), "n"(line(7)), "n"(kLast));
 }
 
+// inclusive prefix sum over the lanes, DPP adds only (two 16-bit halves may be summed at once)
+__device__ __forceinline__ int scan_lanes(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);     // row_shr 1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);     // row_bcast 15, 31
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+    return v;
+}
+
 }  // namespace IV2_NS

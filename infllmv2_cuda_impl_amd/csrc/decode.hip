@@ -213,16 +213,6 @@ __device__ __forceinline__ uint64_t drop_set_bits(uint64_t v, int rank) {
 // behind the end are copies of it, K's are masked by assignment and V's, which are multiplied by P = 0, are patched too.
 constexpr int kMergePitch = kHeadDim + 4;                      // floats per head of a wavefront's output in LDS
 
-__device__ __forceinline__ int scan_lanes(int v) {              // inclusive prefix sum over the lanes, DPP adds only
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);     // row_shr 1, 2, 4, 8
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);     // row_bcast 15, 31
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
-    return v;
-}
-
 // The k largest of the first `cols` of a row of block scores (the order of topk.hip: larger first, ties by ascending column), by
 // a workgroup of four wavefronts; lane w of each gets mask word w.  Column 256 e + 64 wave + lane is key[e], as signed 16-bit
 // integers: scores of Stage 1 are never negative but for -inf, so that is their order, and -32768, the bits of -0, which counts

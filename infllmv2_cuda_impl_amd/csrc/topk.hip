@@ -1,4 +1,4 @@
-// Deterministic top-k over rows of 16-bit scores (gfx950), one wavefront per row (one workgroup where there are few
+// Deterministic top-k over rows of 16-bit scores (gfx950), one wavefront per row (one workgroup for few or long
 // rows), with the uint64 block mask of
 // the selection emitted by the same wavefront.
 //
@@ -228,7 +228,7 @@ void topk_rows_kernel(const TopkParams p) {
         if (k_sel == 0) { thr = 0x10000u; all_ge = true; }     // nothing to take
 
         int base = 0;
-        uint32_t words0_lo = 0, words0_hi = 0, words1_lo = 0, words1_hi = 0;   // lane e holds mask word e (e + 64)
+        uint32_t words_lo = 0, words_hi = 0;                   // lane e holds mask word e
         const uint32_t inv_lane = 0xffffu - static_cast<uint32_t>(lane);
         auto emit = [&](int e, bool take, uint64_t take_mask) {
             if constexpr (kList != kNoList) {
@@ -239,10 +239,7 @@ void topk_rows_kernel(const TopkParams p) {
                 sel[take ? slot : dummy] = val;
                 base += __builtin_popcountll(take_mask);
             }
-            if constexpr (kMask) {                             // the ballot is the mask word
-                if (e < 64) write_lane64(words0_lo, words0_hi, take_mask, e & 63);
-                else write_lane64(words1_lo, words1_hi, take_mask, e & 63);
-            }
+            if constexpr (kMask) write_lane64(words_lo, words_hi, take_mask, e);                 // the ballot is the mask word
         };
         if (all_ge) {
 #pragma unroll
@@ -264,9 +261,8 @@ void topk_rows_kernel(const TopkParams p) {
         }
         if constexpr (kMask) {
             uint64_t* mask_row = p.out_mask + row * p.n64;
-            const uint64_t words0 = (static_cast<uint64_t>(words0_hi) << 32) | words0_lo;
-            const uint64_t words1 = (static_cast<uint64_t>(words1_hi) << 32) | words1_lo;
-            for (int w = lane; w < p.n64; w += 64) mask_row[w] = w < 64 ? words0 : (w < 128 ? words1 : 0ull);
+            const uint64_t words = (static_cast<uint64_t>(words_hi) << 32) | words_lo;
+            for (int w = lane; w < p.n64; w += 64) mask_row[w] = w < 64 ? words : 0ull;
         }
         if constexpr (kList == kNoList) continue;
         const int taken = base;                                // <= k_sel
@@ -313,17 +309,43 @@ void topk_rows_kernel(const TopkParams p) {
     }
 }
 
-// The same selection with a whole workgroup per row, for the few rows of a decode step: there a wavefront per row leaves
-// the chip idle and the kernel takes as long as one wavefront needs for one row (13 us at 2048 columns and 128 rows, 6.6 here; 8.0 and 5.9 at 1024).  Column
-// 512 e + 64 wave + lane sits in register e, so a wavefront's ballot is mask word 8 e + wave.  Two bits of the
-// threshold per round: three counts per wavefront, added up in LDS (a slot of its own per round: one barrier).
+// over eight lanes that hold something each (the other lanes hold the same eight): quad_perm, row_ror 4
+__device__ __forceinline__ int eight_max(int v) {
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x124, 0xF, 0xF, false));
+    return __builtin_amdgcn_readfirstlane(v);
+}
+__device__ __forceinline__ int eight_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(v, v, 0x124, 0xF, 0xF, false);
+    return __builtin_amdgcn_readfirstlane(v);
+}
+__device__ __forceinline__ int wave_max(int v) {
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false));      // a row's maximum
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false));
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x124, 0xF, 0xF, false));
+    v = max(v, __builtin_amdgcn_update_dpp(v, v, 0x128, 0xF, 0xF, false));
+    return max(max(static_cast<int>(__builtin_amdgcn_readlane(v, 0)), static_cast<int>(__builtin_amdgcn_readlane(v, 16))),
+               max(static_cast<int>(__builtin_amdgcn_readlane(v, 32)), static_cast<int>(__builtin_amdgcn_readlane(v, 48))));
+}
+
+// The same selection with a whole workgroup per row, for few or long rows: with a wavefront per row few rows leave the chip idle and the kernel takes as long
+// as one wavefront needs for one row, and a long row is more than its registers hold.  Column
+// 512 e + 64 wave + lane sits in register e, so a wavefront's ballot is mask word 8 e + wave.  Bound by a chain of barriers and trips to LDS, so it has few:
+// one histogram of the keys up to 1022 (eight powers of two of bfloat16) below the largest finite score, and two scans over the lanes, find the k-th
+// key.  Whatever bits the row holds, a round finds it or starts the next one 1023 keys further down.  (Two bits of the key per round by counts, a barrier
+// each: 48 rows of 626 columns 5.7 -> 4.2 us, 128 of 2048 6.5 -> 4.3, 64 of 4000 8.5 -> 5.2, 16 of 8000 14.4 -> 7.4; a whole paged decode step of 24 sequences
+// 44.0 -> 42.6.  What lies below the histogram counted in a bin of its own, one address for all of them: 64 of 4000 8.5.)
 constexpr int kTopkRowWaves = 8;
 
 template <int kItems>
 __global__ __launch_bounds__(kTopkRowWaves * 64)
 void topk_wide_kernel(const TopkParams p) {
     extern __shared__ uint32_t sel[];                          // k survivors
-    __shared__ int counts[8][4];                               // per round: columns at or above each candidate
+    __shared__ __attribute__((aligned(16))) uint32_t bins[512];                                      // two 16-bit counts each
+    __shared__ int2 tops[2][kTopkRowWaves];                    // per wavefront: its largest key up to the limit, its columns above it
     __shared__ uint32_t word_counts[kItems * kTopkRowWaves];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -331,39 +353,54 @@ void topk_wide_kernel(const TopkParams p) {
     const int n = p.n, k = p.k;
     const int k_sel = k < n ? k : n;
     const uint16_t* src = p.x + row * p.row_stride;
-    uint32_t key[kItems];
+    int key[kItems];                                           // -1: no column
 #pragma unroll
     for (int e = 0; e < kItems; ++e) {
         const int col = e * kTopkRowWaves * 64 + tid;
         key[e] = col < n ? src[col] : 0;
     }
-    if (tid < 32) counts[tid >> 2][tid & 3] = 0;
+    bins[tid] = 0u;
 #pragma unroll
-    for (int e = 0; e < kItems; ++e) key[e] = e * kTopkRowWaves * 64 + tid < n ? sortable16(key[e]) : 0u;
-    __syncthreads();
-    auto count_ge = [&](uint32_t cand) -> int {
-        int cnt = 0;
+    for (int e = 0; e < kItems; ++e) key[e] = e * kTopkRowWaves * 64 + tid < n ? static_cast<int>(sortable16(key[e])) : -1;
+    int thr = 0, limit = 0xffff - p.neg_inf_key;               // +inf, the forced blocks, stays above the histogram
+    for (int round = 0; k_sel > 0; ++round) {
+        int top = -1, above = 0;
 #pragma unroll
-        for (int e = 0; e < kItems; ++e) cnt += __builtin_popcountll(__builtin_amdgcn_ballot_w64(key[e] >= cand));
-        return cnt;
-    };
-    // thr = largest candidate with count(key >= thr) >= k_sel (0 always satisfies it: every register counts)
-    uint32_t thr = 0;
-    for (int round = 0; round < 8; ++round) {
-        const uint32_t unit = 1u << (14 - 2 * round);
-        const int c1 = count_ge(thr + unit), c2 = count_ge(thr + 2 * unit), c3 = count_ge(thr + 3 * unit);
-        if (lane == 0) {
-            atomicAdd(&counts[round][0], c1);
-            atomicAdd(&counts[round][1], c2);
-            atomicAdd(&counts[round][2], c3);
+        for (int e = 0; e < kItems; ++e) {
+            top = max(top, key[e] <= limit ? key[e] : -1);
+            above += __builtin_popcountll(__builtin_amdgcn_ballot_w64(key[e] > limit));
+        }
+        top = wave_max(top);
+        if (lane == 0) tops[round & 1][wave] = make_int2(top, above);
+        __syncthreads();
+        const int2 t = tops[round & 1][lane & (kTopkRowWaves - 1)];
+        top = eight_max(t.x);
+        above = eight_sum(t.y);
+        if (above >= k_sel) { limit = 0xffff; continue; }      // only at first: no more than forced blocks are wanted
+        const int lowest = max(top - 1022, 0);                 // of the histogram; what lies further down would all add to one bin
+#pragma unroll
+        for (int e = 0; e < kItems; ++e) {
+            const int bin = top - key[e];
+            if (key[e] <= limit && key[e] >= lowest) atomicAdd(&bins[bin >> 1], (bin & 1) ? 0x10000u : 1u);
         }
         __syncthreads();
-        const int s1 = counts[round][0], s2 = counts[round][1], s3 = counts[round][2];
-        thr += (s3 >= k_sel ? 3u : (s2 >= k_sel ? 2u : (s1 >= k_sel ? 1u : 0u))) * unit;
+        const uint4 a = *reinterpret_cast<const uint4*>(&bins[8 * lane]), b = *reinterpret_cast<const uint4*>(&bins[8 * lane + 4]);
+        const uint32_t pairs = a.x + a.y + a.z + a.w + b.x + b.y + b.z + b.w;
+        const int mine = static_cast<int>((pairs & 0xffffu) + (pairs >> 16));
+        const int upto = scan_lanes(mine) + above;
+        const int at = __builtin_ctzll(__builtin_amdgcn_ballot_w64(upto >= k_sel) | 1ull << 63);
+        const int fine = lane < 16 ? static_cast<int>(reinterpret_cast<const uint16_t*>(bins)[16 * at + lane]) : 0;
+        const int fine_upto = scan_lanes(fine) + static_cast<int>(__builtin_amdgcn_readlane(upto - mine, at));
+        const int in = __builtin_ctzll(__builtin_amdgcn_ballot_w64(fine_upto >= k_sel) | 1ull << 63) & 15;
+        thr = top - (16 * at + in);
+        if (16 * at + in < 1023) break;
+        limit = thr;                                           // further down than the histogram goes: again from there
+        __syncthreads();
+        bins[tid] = 0u;
     }
-    if (p.drop_neg_inf && thr <= p.neg_inf_key) thr = p.neg_inf_key;                 // scores above -inf only: none of those equal to thr
-    const bool no_equal = p.drop_neg_inf && thr == p.neg_inf_key;
-    if (k_sel == 0) thr = 0xffffffffu;
+    if (p.drop_neg_inf && thr <= static_cast<int>(p.neg_inf_key)) thr = p.neg_inf_key;                 // scores above -inf only: none of those equal to thr
+    const bool no_equal = p.drop_neg_inf && thr == static_cast<int>(p.neg_inf_key);
+    if (k_sel == 0) thr = 0x10000;
     // per mask word: how many columns lie above the threshold (low half) and how many equal it (high half)
 #pragma unroll
     for (int e = 0; e < kItems; ++e) {
@@ -377,13 +414,7 @@ void topk_wide_kernel(const TopkParams p) {
     uint32_t upto[kScans], all = 0;
 #pragma unroll
     for (int c = 0; c < kScans; ++c) {
-        uint32_t v = c * 64 + lane < kWords ? word_counts[c * 64 + lane] : 0u;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t o = __shfl_up(v, off);
-            v += lane >= off ? o : 0u;
-        }
-        upto[c] = v + all;
+        upto[c] = static_cast<uint32_t>(scan_lanes(c * 64 + lane < kWords ? static_cast<int>(word_counts[c * 64 + lane]) : 0)) + all;
         all = __builtin_amdgcn_readlane(upto[c], 63);
     }
     const int total_above = static_cast<int>(all & 0xffffu), total_equal = static_cast<int>(all >> 16);
@@ -402,7 +433,7 @@ void topk_wide_kernel(const TopkParams p) {
         if (take && p.out_idx != nullptr) {
             const int col = word * 64 + lane;
             const int slot = lanes_below(take_mask, above + (equal < ties ? equal : ties));
-            sel[slot] = p.by_index ? static_cast<uint32_t>(col) : (key[e] << 16) | (0xffffu - static_cast<uint32_t>(col));
+            sel[slot] = p.by_index ? static_cast<uint32_t>(col) : (static_cast<uint32_t>(key[e]) << 16) | (0xffffu - static_cast<uint32_t>(col));
         }
     }
     if (mask_row)
@@ -472,7 +503,13 @@ static int launch_topk(void* stream, const TopkParams& p) {
     return 0;
 }
 
-constexpr int kTopkWideRows = 512;
+// Up to how many rows of n columns a workgroup per row is the faster one.  us by wavefronts | by workgroups, a list of 64 wanted: 400 columns, 768 rows 5.1 | 4.6,
+// 1024 5.1 | 4.7, 2048 5.9 | 7.7 (of 512, a wavefront's registers full, 4.7 | 4.4, 4.7 | 4.8, 5.5 | 7.7); 900, 1024 rows 7.4 | 5.4, 2048 8.6 | 8.9; 1500, 2048 rows 14.7 | 10.9,
+// 4096 25.4 | 19.9, 8192 40.7 | 36.9 (of 2048 13.1 | 11.0, 18.9 | 20.2, 33.1 | 37.9); 3000, 16 384 rows 249 | 104, 65 536 763 | 406 (of 4096 136 | 106, 429 | 421, mask words
+// alone 93 | 95, 283 | 376); 8192, 2048 rows 80 | 28, 65 536 1500 | 768.  Up to 256 columns both take what a launch takes (4.3).
+static int64_t wide_rows(int n) {
+    return n <= 256 ? 0 : n <= 512 ? 768 : n <= 1024 ? 1024 : n <= 2048 ? 2048 : n <= 4096 ? 16384 : 0x7fffffff;
+}
 
 static int topk_dispatch(void* stream, const uint16_t* x, int64_t row_stride, int32_t* idx, uint16_t* val,
                          uint64_t* mask, int n64, int out_stride, int64_t rows, int n, int k, int by_index,
@@ -488,9 +525,9 @@ static int topk_dispatch(void* stream, const uint16_t* x, int64_t row_stride, in
     p.x = x; p.row_stride = row_stride; p.out_idx = idx; p.out_val = val; p.out_mask = mask;
     p.out_stride = out_stride; p.n64 = n64; p.rows = rows; p.n = n; p.k = k;
     p.by_index = by_index; p.drop_neg_inf = drop_neg_inf; p.neg_inf_key = dtype == 0 ? kKeyNegInfFp16 : kKeyNegInfBf16;
-    // few rows (two workgroups per CU at most): a workgroup per row.  Up to 512 columns one wavefront holds the row in
-    // eight registers and is done before a workgroup has met at its barriers (4.4 against 5.5 us at 512 columns).
-    if (rows <= kTopkWideRows && n > 512) {
+    IV2_CHECK(n <= 4096 || rows <= 0x7fffffff, "topk: too many rows");
+    if (rows <= wide_rows(n)) {
+        if (n <= 512) return launch_topk_wide<1>(stream, p);
         if (n <= 1024) return launch_topk_wide<2>(stream, p);
         if (n <= 2048) return launch_topk_wide<4>(stream, p);
         if (n <= 4096) return launch_topk_wide<8>(stream, p);
@@ -505,8 +542,7 @@ static int topk_dispatch(void* stream, const uint16_t* x, int64_t row_stride, in
     if (n <= 512) return launch_topk<8>(stream, p);
     if (n <= 1024) return launch_topk<16>(stream, p);
     if (n <= 2048) return launch_topk<32>(stream, p);
-    if (n <= 4096) return launch_topk<64>(stream, p);
-    return launch_topk<128>(stream, p);
+    return launch_topk<64>(stream, p);
 }
 
 }  // namespace infllmv2

@@ -1,0 +1,67 @@
+"""Top-k with a workgroup per row against a sort of unique keys (larger score first, equal scores by ascending column), on both sides of every number of
+columns and rows at which the kernel or its registers change: rows of arbitrary bits, so that the search goes through many histograms, infinities more and
+fewer than are wanted, rows of one value, and scores as Stage 1 makes them."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def rows_of(kind, rows, n, gen):
+    if kind == "bits":                                           # NaN included: its bits order it
+        return torch.randint(-32768, 32768, (rows, n), generator=gen, device="cuda", dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    x = torch.rand(rows, n, generator=gen, device="cuda") ** 6
+    if kind == "inf":
+        x[torch.rand(rows, n, generator=gen, device="cuda") < 0.3] = float("-inf")
+        x[:, ::5] = float("inf")
+    if kind == "flat":
+        x[:] = 0.25
+        x[::2, 1::3] = -0.0
+        x[::4, 2::7] = 0.0
+    return x.to(torch.bfloat16)
+
+
+def check(x, k):
+    from infllmv2_cuda_impl_amd import _lib
+    rows, n = x.shape
+    bits = x.view(torch.int16).to(torch.int64) & 0xffff
+    key = torch.where(bits < 0x8000, bits + 0x8000, 0x10000 - bits)                                        # -0 and +0 alike
+    order = torch.topk(key * 16384 + (16383 - torch.arange(n, device="cuda")), min(k, n), dim=1).values
+    want = torch.full((rows, max(k, 1)), -1, dtype=torch.int64, device="cuda")
+    want[:, :min(k, n)] = 16383 - (order & 16383)
+    n64, stream = (n + 63) // 64 + 1, torch.cuda.current_stream().cuda_stream
+    idx = torch.empty(rows, max(k, 1), dtype=torch.int32, device="cuda")
+    words = torch.empty(rows, n64, dtype=torch.int64, device="cuda")
+    for by_index in (0, 1):
+        _lib.call("infllmv2_topk_select", stream, x.data_ptr(), n, 1, idx.data_ptr(), words.data_ptr(), rows, n, k, n64, by_index, 0)
+        got = idx[:, :k].to(torch.int64)
+        ref = want[:, :k]
+        if by_index:
+            ref = torch.where(ref < 0, 1 << 20, ref).sort(1).values
+            ref = torch.where(ref == 1 << 20, -1, ref)
+        assert torch.equal(got, ref), (rows, n, k, by_index)
+        taken = torch.zeros(rows, n64 * 64 + 1, dtype=torch.bool, device="cuda").scatter_(1, torch.where(want[:, :k] < 0, n64 * 64, want[:, :k]), True)
+        shown = (words[:, :, None] >> torch.arange(64, device="cuda") & 1).bool().view(rows, -1)
+        assert torch.equal(shown, taken[:, :-1]), (rows, n, k)
+    if k > 0:
+        stride = 1 << (k - 1).bit_length()                       # of this entry point's rows
+        val, idx = torch.empty(rows, stride, dtype=torch.bfloat16, device="cuda"), torch.empty(rows, stride, dtype=torch.int32, device="cuda")
+        _lib.call("infllmv2_topk", stream, rows, n, k, 1, x.data_ptr(), val.data_ptr(), idx.data_ptr())
+        assert torch.equal(idx[:, :k].to(torch.int64), want[:, :k])
+        got = x.gather(1, want[:, :min(k, n)])
+        assert torch.equal(val[:, :min(k, n)].view(torch.int16), got.view(torch.int16))
+
+
+@pytest.mark.parametrize("kind", ["bits", "inf", "flat", "scores"])
+@pytest.mark.parametrize("n", [256, 257, 511, 512, 513, 1024, 1025, 2048, 2049, 4096, 4097, 8192])
+def test_few_rows(n, kind):
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    for k in (0, 1, 16, 64, 65, 300):
+        check(rows_of(kind, 5, n, gen), k)
+
+
+@pytest.mark.parametrize("rows, n", [(768, 400), (769, 400), (1024, 700), (1025, 700), (2048, 1100), (2049, 1100), (16384, 2100), (16385, 2100)])
+def test_both_sides_of_the_rule(rows, n):
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    for kind in ("scores", "inf"):
+        check(rows_of(kind, rows, n, gen), 32)
