@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define INFLLMV2_ABI_VERSION 17
+#define INFLLMV2_ABI_VERSION 18
 
 /* ---- library ------------------------------------------------------------------------------ */
 
@@ -214,6 +214,16 @@ int infllmv2_varlen_fwd_stage1_pooled(void* stream, const void* q, const void* k
                                       const int64_t* k_strides, const int64_t* v_strides, int out_len,
                                       float softmax_scale, int is_causal, int kernel_size, int stride, int padding,
                                       int block_size, int local_blocks, int init_blocks);
+
+/* That (causal, no tokens before the queries) and infllmv2_topk_mask of its result, drop_neg_inf 0, in one launch: mask (Hk, total_q, n_uint64_per_row),
+ * rows of at most INFLLMV2_STAGE1_SELECT_BLOCKS blocks. */
+#define INFLLMV2_STAGE1_SELECT_BLOCKS 512
+int infllmv2_varlen_fwd_stage1_selected(void* stream, const void* q, const void* k, const void* v, uint64_t* mask,
+                                        const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, const int32_t* cu_seqlens_v, int batch,
+                                        int64_t total_q, int num_heads, int num_heads_k, int head_dim, int max_seqlen_q, int max_seqlen_k,
+                                        const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides, int out_len,
+                                        float softmax_scale, int kernel_size, int stride, int padding, int block_size, int local_blocks,
+                                        int init_blocks, int topk, int n_uint64_per_row);
 
 /* Stage 1 for decode: one query token per sequence, a batch of sequences, each against its own compressed keys.  The
  * reference serves this case with the same `varlen_fwd_stage1` launch (infllm_v2/infllmv2_sparse_attention.py:483-606
@@ -504,6 +514,12 @@ int infllmv2_varlen_fwd_stage1_pooled_f16(void* stream, const void* q, const voi
                                           const int64_t* k_strides, const int64_t* v_strides, int out_len,
                                           float softmax_scale, int is_causal, int kernel_size, int stride, int padding,
                                           int block_size, int local_blocks, int init_blocks);
+int infllmv2_varlen_fwd_stage1_selected_f16(void* stream, const void* q, const void* k, const void* v, uint64_t* mask,
+                                        const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, const int32_t* cu_seqlens_v, int batch,
+                                        int64_t total_q, int num_heads, int num_heads_k, int head_dim, int max_seqlen_q, int max_seqlen_k,
+                                        const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides, int out_len,
+                                        float softmax_scale, int kernel_size, int stride, int padding, int block_size, int local_blocks,
+                                        int init_blocks, int topk, int n_uint64_per_row);
 int infllmv2_decode_step_scores_f16(void* stream, const void* q, const void* k_new, const void* v_new, void* kcache,
                                 void* vcache, void* fine_cache, void* coarse_cache, const int32_t* lens, int host_len,
                                 int32_t* new_lens, int32_t* fine_lens, int32_t* coarse_lens, void* pooled,

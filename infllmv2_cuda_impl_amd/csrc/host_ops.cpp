@@ -285,6 +285,25 @@ Tensor stage1_pooled(const Tensor& q, const Tensor& k_, const Tensor& v_, const 
     return out;
 }
 
+// The mask words of the topk best blocks of that, causal and without cached tokens, in the same launch.
+Tensor stage1_selected(const Tensor& q, const Tensor& k_, const Tensor& v_, const Tensor& cu_q, const Tensor& cu_k, const Tensor& cu_v, int64_t max_q,
+                       int64_t max_k, double scale, int64_t out_len, int64_t local_blocks, int64_t init_blocks, int64_t block_size, int64_t stride,
+                       int64_t topk, int64_t n64) {
+    check_stage1(q, k_, v_, cu_q, cu_k, cu_v);
+    const int64_t batch = cu_q.numel() - 1, total_q = q.size(0), hq = q.size(1), hk = k_.size(1);
+    DeviceGuard guard(q.device());
+    const Tensor k = readable(k_), v = readable(v_);
+    Tensor mask = at::empty({hk, total_q, n64}, q.options().dtype(at::kLong));
+    const S3 qs = grouped(q, hq / hk);
+    const S2 ks = rows_heads(k), vs = rows_heads(v);
+    const int per = as_int(block_size / stride);
+    auto fn = is_half(q) ? infllmv2_varlen_fwd_stage1_selected_f16 : infllmv2_varlen_fwd_stage1_selected;
+    check_rc(fn(stream_of(q), ptr(q), ptr(k), ptr(v), static_cast<uint64_t*>(mask.data_ptr()), iptr(cu_q), iptr(cu_k), iptr(cu_v), as_int(batch), total_q,
+                as_int(hq), as_int(hk), as_int(q.size(2)), as_int(max_q), as_int(max_k), qs.v, ks.v, vs.v, as_int(out_len), static_cast<float>(scale),
+                per + 1, per, 1, as_int(block_size), as_int(local_blocks), as_int(init_blocks), as_int(topk), as_int(n64)), "varlen_fwd_stage1_pooled");
+    return mask;
+}
+
 Tensor stage1_kvcache(const Tensor& q, const Tensor& fine, const Tensor& coarse, const Tensor& fine_lens, const Tensor& coarse_lens,
                       const Tensor& cache_seqlens, int64_t local_blocks, int64_t init_blocks, std::optional<int64_t> max_cache_len,
                       int64_t block_size, int64_t stride, double scale, bool causal, bool pooled) {
@@ -439,11 +458,13 @@ Tensor topk_to_uint64(const Tensor& topk_idx, int64_t k_blocks, const OptTensor&
 
 // the selection front end: compressed keys, fused Stage 1 and pooling, top-k with the mask words
 // Block scores (Hk, total_q, blocks) of packed queries, and how many mask words a row of the selection takes.  images: where the block
-// images of (k, v) go, which are then made in the same launch as the compressed keys where pack_early says so.
+// images of (k, v) go, which are then made in the same launch as the compressed keys where pack_early says so.  mask: where the mask words of the topk best go, if
+// the rows are short enough for the launch that makes the scores to choose among them; there are no scores then.
 std::tuple<Tensor, int64_t> block_scores(const Tensor& q_, const Tensor& k, const Tensor& cu_q, const Tensor& cu_k, int64_t max_q,
                                          int64_t max_k, int64_t local_blocks, int64_t init_blocks, const OptTensor& cache_lens,
                                          int64_t max_cache_len, double scale, bool causal, int64_t kernel_size, int64_t stride,
-                                         int64_t block_size, bool exact_lse, const Tensor* v = nullptr, OptTensor* images = nullptr) {
+                                         int64_t block_size, bool exact_lse, const Tensor* v = nullptr, OptTensor* images = nullptr,
+                                         int64_t topk = 0, Tensor* mask = nullptr) {
     const Tensor q = q_.stride(-1) == 1 ? q_ : q_.contiguous();
     Tensor kf, cu_f, kc, cu_c;
     if (exact_lse) {
@@ -457,10 +478,15 @@ std::tuple<Tensor, int64_t> block_scores(const Tensor& q_, const Tensor& k, cons
         std::tie(kf, cu_f, kc, cu_c) = compress_keys_pair(k, cu_k, max_k, kernel_size, stride, 4 * kernel_size, 4 * stride);
     }
     const int64_t out_len = (max_q + max_cache_len + block_size - 1) / block_size;
-    const Tensor pooled = stage1_pooled(q, kf, kc, cu_q, cu_f, cu_c, max_q, windows(max_k, kernel_size, stride), scale, causal, out_len, cache_lens,
-                                        0, local_blocks, init_blocks, block_size, stride);
     int64_t n64 = ((max_k + block_size - 1) / block_size + 63) / 64;
     if (n64 * 64 < out_len) n64 = (out_len + 63) / 64;                 // cached tokens widen the pooled rows beyond max_seqlen_k
+    if (mask != nullptr && out_len > 0 && out_len <= INFLLMV2_STAGE1_SELECT_BLOCKS && max_q > 1) {
+        *mask = stage1_selected(q, kf, kc, cu_q, cu_f, cu_c, max_q, windows(max_k, kernel_size, stride), scale, out_len, local_blocks, init_blocks, block_size,
+                                stride, topk, n64);
+        return {Tensor(), n64};
+    }
+    const Tensor pooled = stage1_pooled(q, kf, kc, cu_q, cu_f, cu_c, max_q, windows(max_k, kernel_size, stride), scale, causal, out_len, cache_lens,
+                                        0, local_blocks, init_blocks, block_size, stride);
     return {pooled, n64};
 }
 
@@ -479,9 +505,11 @@ std::tuple<Tensor, Tensor, OptTensor> select_mask(const Tensor& q, const Tensor&
                                                   int64_t local_blocks, int64_t init_blocks, double scale, int64_t kernel_size, int64_t stride,
                                                   int64_t block_size) {
     OptTensor images;
+    Tensor mask;
     const auto [pooled, n64] = block_scores(q, k, cu, cu, max_len, max_len, local_blocks, init_blocks, std::nullopt, 0, scale, true, kernel_size,
-                                            stride, block_size, false, &v, &images);
-    return {at::empty({k.size(1), 0, topk}, q.options().dtype(at::kInt)), topk_mask(pooled, topk, n64), images};
+                                            stride, block_size, false, &v, &images, topk, &mask);
+    if (!mask.defined()) mask = topk_mask(pooled, topk, n64);
+    return {at::empty({k.size(1), 0, topk}, q.options().dtype(at::kInt)), mask, images};
 }
 
 // ---- Stage 2 (mha_varlen_fwd, flash_api.cpp:519-782; mha_varlen_bwd, :1278-1547) ---------------------------------------

@@ -51,6 +51,10 @@ struct Stage1Params {
     int cache_len;
     int pool_len;                    // key blocks per output row
     int local_blocks, init_blocks;
+    // selection only
+    uint64_t* mask;                  // (Hk, total_q, mask_words)
+    int64_t total_q;
+    int mask_words, topk;
 };
 
 // 8 wavefronts x 2 tokens: 112 registers, so four wavefronts share a SIMD and the exp-heavy VALU work of one hides
@@ -161,10 +165,16 @@ __device__ __forceinline__ void pool_quads(float a, float b, float prev_a, float
 // kPool: instead of the score rows, write their 1-D max-pooling onto 64-token key blocks (window of 5 compressed
 // keys, stride 4, padding 1, forced blocks +inf, empty windows -inf: the rule of csrc/max_pooling_1d.cuh:12-160
 // applied to the scores this kernel would have written, which never reach memory).
-template <bool kCausal, bool kPool>
+// kItems > 0: nor do these; of a row of at most 64 kItems blocks the topk best (larger score first, ties by ascending block: topk.hip) are chosen here, and their
+// mask words written.  A wavefront has its tokens' rows in LDS by the end, 64 kItems scores each, and finds the last key that is in bit by bit.
+// Bound by the counts, 16 kItems of them to a token, in scalar instructions beside the other wavefronts' exponentials; scores and selection in us, two launches | one, 2 KV heads:
+// 2048 tokens 15.9 | 11.9, 4096 27.3 | 21.2, 8192 56.2 | 48.5, 16 384 133 | 125, 20 480 201 | 196, 32 768 443 | 443, 49 152 931 | 944: rows of 512 blocks and no more.  Whole prefill of
+// 1000 tokens, 16 blocks selected, 42.0 -> 40.7, of 2048 74.4 -> 70.0, training on 1023 + 3001 + 517 + 2200 606 -> 596.
+template <bool kCausal, bool kPool, int kItems = 0>
 __global__ __launch_bounds__(64 * kWavesS1) __attribute__((amdgpu_waves_per_eu(kWavesPerSimdS1, kWavesPerSimdS1)))
 void stage1_kernel(const Stage1Params p) {
     __shared__ uint4 tile[2][1024];                            // two 16 KiB operand-ordered key tiles
+    __shared__ elem_bits pooled[kItems > 0 ? kTokPerBlock : 1][kItems > 0 ? 64 * kItems : 1];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);     // wavefront-uniform: what depends on it alone stays in scalar registers
@@ -356,11 +366,15 @@ void stage1_kernel(const Stage1Params p) {
     // issued would add its round trip to every tile.
     float held[kTokPerWave] = {0.f, 0.f};
     bool pending = false;
+    auto store = [&](int t, uint32_t at, elem_bits value) {
+        if constexpr (kItems > 0) pooled[wave * kTokPerWave + t][at] = value;
+        else out_rows[t][at] = value;
+    };
     auto store_held = [&](int ti) {
         const uint32_t at = static_cast<uint32_t>(kPool ? ti * 16 + (lane >> 2) : ti * 64 + lane);
         if (!kPool || (lane & 3) == 0) {
 #pragma unroll
-            for (int t = 0; t < kTokPerWave; ++t) out_rows[t][at] = f32_to_elem_hw(held[t]);
+            for (int t = 0; t < kTokPerWave; ++t) store(t, at, f32_to_elem_hw(held[t]));
         }
     };
     for (int ti = 0; ti < tiles_f; ++ti) {
@@ -415,7 +429,7 @@ void stage1_kernel(const Stage1Params p) {
 #pragma unroll
             for (int t = 0; t < kTokPerWave; ++t) {
                 prev[t] = mine[t];
-                if (!pending && live[t] && (lane & 3) == 0 && kb < p.pool_len) out_rows[t][kb] = pool_rest(kb, bq[t], held[t]);
+                if (!pending && live[t] && (lane & 3) == 0 && kb < p.pool_len) store(t, kb, pool_rest(kb, bq[t], held[t]));
             }
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -432,7 +446,53 @@ void stage1_kernel(const Stage1Params p) {
             // the first of them still sees the last key of the last tile
             const float last_score = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(prev[t]), 63));
             for (int kb = tiles_f * 16 + lane; kb < p.pool_len; kb += 64)
-                out_rows[t][kb] = pool_rest(kb, bq[t], kb == tiles_f * 16 ? last_score : 0.f);
+                store(t, kb, pool_rest(kb, bq[t], kb == tiles_f * 16 ? last_score : 0.f));
+        }
+    }
+    if constexpr (kItems > 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        uint32_t key[kTokPerWave][kItems];                     // 0: no column
+        const int take_at_most = p.topk < p.pool_len ? p.topk : p.pool_len;
+#pragma unroll
+        for (int t = 0; t < kTokPerWave; ++t)
+#pragma unroll
+            for (int e = 0; e < kItems; ++e) {
+                const int kb = 64 * e + lane;
+                key[t][e] = kb < p.pool_len ? sortable16(pooled[wave * kTokPerWave + t][kb]) : 0u;
+            }
+        auto count = [&](int t, auto&& in) {
+            int c = 0;
+#pragma unroll
+            for (int e = 0; e < kItems; ++e) c += __builtin_popcountll(__builtin_amdgcn_ballot_w64(in(key[t][e])));
+            return c;
+        };
+        uint32_t thr[kTokPerWave];                             // the largest key that so many keys reach
+#pragma unroll
+        for (int t = 0; t < kTokPerWave; ++t) thr[t] = 0;
+#pragma unroll
+        for (int bit = 15; bit >= 0; --bit)
+#pragma unroll
+            for (int t = 0; t < kTokPerWave; ++t) {
+                const uint32_t next = thr[t] | (1u << bit);
+                thr[t] = count(t, [&](uint32_t x) { return x >= next; }) >= take_at_most ? next : thr[t];
+            }
+#pragma unroll
+        for (int t = 0; t < kTokPerWave; ++t) {
+            if (!live[t]) continue;
+            int ties = take_at_most - count(t, [&](uint32_t x) { return x > thr[t]; });          // of the keys equal to it
+            uint64_t words = 0ull;                             // lane w: word w
+#pragma unroll
+            for (int e = 0; e < kItems; ++e) {
+                const uint64_t equal = __builtin_amdgcn_ballot_w64(key[t][e] == thr[t]);
+                const int rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(equal >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(equal), 0));
+                const uint64_t taken = __builtin_amdgcn_ballot_w64(key[t][e] > thr[t] || (key[t][e] == thr[t] && rank < ties));
+                words = lane == e ? taken : words;
+                ties -= __builtin_popcountll(equal);
+            }
+            uint64_t* row = p.mask + (static_cast<int64_t>(h) * p.total_q + q0 + tok0 + t) * p.mask_words;
+            for (int w = lane; w < p.mask_words; w += 64) row[w] = w < kItems ? words : 0ull;
         }
     }
 }
@@ -446,6 +506,8 @@ namespace {
 struct Stage1Pool {                  // pooled-output mode of the launch below
     const int32_t* cache_lens;
     int cache_len, pool_len, local_blocks, init_blocks;
+    uint64_t* mask = nullptr;        // not null: the selection instead
+    int mask_words = 0, topk = 0;
 };
 
 int launch_stage1(const char* who, void* stream, const void* q, const void* k, const void* v, void* out,
@@ -458,7 +520,7 @@ int launch_stage1(const char* who, void* stream, const void* q, const void* k, c
     IV2_CHECK(valid_group(num_heads, num_heads_k),
               "%s: requires num_heads == g * num_heads_k with g in {1, 2, 4, 8, 16} (got %d and %d)", who, num_heads, num_heads_k);
     IV2_CHECK(batch > 0 && total_q >= 0 && max_seqlen_q >= 0 && max_seqlen_k >= 0, "%s: bad sizes", who);
-    IV2_CHECK(q && k && v && out && cu_seqlens_q && cu_seqlens_k && cu_seqlens_v, "%s: null pointer", who);
+    IV2_CHECK(q && k && v && (out || (pool && pool->mask)) && cu_seqlens_q && cu_seqlens_k && cu_seqlens_v, "%s: null pointer", who);
     IV2_CHECK(num_heads_k <= 65535 && batch <= 65535, "%s: batch and num_heads_k must not exceed 65535", who);
     IV2_CHECK(reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(k) % 16 == 0 &&
               reinterpret_cast<uintptr_t>(v) % 16 == 0, "%s: q, k, v must be 16-byte aligned", who);
@@ -488,10 +550,14 @@ int launch_stage1(const char* who, void* stream, const void* q, const void* k, c
     if (pool) {
         p.cache_lens = pool->cache_lens; p.cache_len = pool->cache_len; p.pool_len = pool->pool_len;
         p.local_blocks = pool->local_blocks; p.init_blocks = pool->init_blocks;
+        p.mask = pool->mask; p.total_q = total_q; p.mask_words = pool->mask_words; p.topk = pool->topk;
     }
     const dim3 grid((max_seqlen_q + kTokPerBlock - 1) / kTokPerBlock, batch, num_heads_k);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (pool) {
+    if (p.mask) {
+        auto kernel = p.pool_len <= 64 ? stage1_kernel<true, true, 1> : p.pool_len <= 128 ? stage1_kernel<true, true, 2> : p.pool_len <= 256 ? stage1_kernel<true, true, 4> : stage1_kernel<true, true, 8>;
+        hipLaunchKernelGGL(kernel, grid, dim3(64 * kWavesS1), 0, st, p);
+    } else if (pool) {
         if (is_causal) hipLaunchKernelGGL((stage1_kernel<true, true>), grid, dim3(64 * kWavesS1), 0, st, p);
         else hipLaunchKernelGGL((stage1_kernel<false, true>), grid, dim3(64 * kWavesS1), 0, st, p);
     } else {
@@ -536,4 +602,26 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_fwd_stage1_pooled)(void* stream, const 
                          batch, total_q, num_heads, num_heads_k, head_dim, max_seqlen_q, max_seqlen_k, q_strides,
                          k_strides, v_strides, total_q * static_cast<int64_t>(out_len), out_len, softmax_scale,
                          is_causal, &pool);
+}
+
+extern "C" int IV2_ENTRY(infllmv2_varlen_fwd_stage1_selected)(void* stream, const void* q, const void* k, const void* v, uint64_t* mask,
+                                                   const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+                                                   const int32_t* cu_seqlens_v, int batch, int64_t total_q, int num_heads,
+                                                   int num_heads_k, int head_dim, int max_seqlen_q, int max_seqlen_k,
+                                                   const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+                                                   int out_len, float softmax_scale, int kernel_size, int stride, int padding,
+                                                   int block_size, int local_blocks, int init_blocks, int topk, int n_uint64_per_row) {
+    IV2_CHECK(kernel_size == 5 && stride == 4 && padding == 1 && block_size == kBlockN,
+              "varlen_fwd_stage1_pooled: only the 5/4/1 window on 64-token blocks is fused (got %d/%d/%d on %d); "
+              "use varlen_fwd_stage1 and max_pooling_1d", kernel_size, stride, padding, block_size);
+    IV2_CHECK(out_len > 0 && out_len <= INFLLMV2_STAGE1_SELECT_BLOCKS, "varlen_fwd_stage1_selected: 1 to %d blocks (got %d)",
+              INFLLMV2_STAGE1_SELECT_BLOCKS, out_len);
+    IV2_CHECK(topk >= 0, "topk: negative size");
+    IV2_CHECK(topk <= 2048, "topk: k %d exceeds 2048", topk);
+    IV2_CHECK(mask != nullptr && n_uint64_per_row > 0 && static_cast<int64_t>(n_uint64_per_row) * 64 >= out_len,
+              "topk: %d mask words per row cannot hold %d columns", n_uint64_per_row, out_len);
+    const Stage1Pool pool{nullptr, 0, out_len, local_blocks, init_blocks, mask, n_uint64_per_row, topk};
+    return launch_stage1("varlen_fwd_stage1_pooled", stream, q, k, v, nullptr, cu_seqlens_q, cu_seqlens_k, cu_seqlens_v,
+                         batch, total_q, num_heads, num_heads_k, head_dim, max_seqlen_q, max_seqlen_k, q_strides,
+                         k_strides, v_strides, 0, 0, softmax_scale, 1, &pool);
 }

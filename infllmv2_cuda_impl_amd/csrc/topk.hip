@@ -30,11 +30,6 @@
 
 namespace infllmv2 {
 
-// order-preserving map of IEEE half / bfloat16 bits onto 1..0xffff: larger float <=> larger key; -0 and +0 share
-// 0x8000; key 0 is free and marks "no element" (it loses every comparison and, lying in columns >= n, every tie)
-__device__ __forceinline__ uint32_t sortable16(uint32_t b) {
-    return b < 0x8000u ? b + 0x8000u : 0x10000u - b;
-}
 constexpr uint32_t kKeyNegInfBf16 = 0x10000u - 0xff80u;
 constexpr uint32_t kKeyNegInfFp16 = 0x10000u - 0xfc00u;
 
