@@ -27,9 +27,9 @@
 // Which launches (measured before there was a pace): at 30 000 tokens a whole prefill gained 1 % and at 32 768 it gained or lost less (L2 serves 91 % of the requests
 // there and the wait for a generation's slowest workgroup costs 2 %); at 40 000 it gained 7 %, at 49 152 14, at 65 536 22 (10.9 -> 8.5 ms,
 // two KV heads), at 98 304 20, at 131 072 17 (31.3 -> 25.9).  Only wavefronts whose row has blocks of its own in
-// several mask words wait: with window masks everything is shared (60 000 tokens, 6 blocks: 473 us without all this, 478 with the counters and no waits).  Letting up to 8 workgroups of a
-// generation start early gave back a quarter of the gain; more meeting points during the walk, or walking every other
-// generation downwards, gave nothing more.  The dQ kernel walks the same way but is not bound by its fetches: waiting cost it 2 %
+// several mask words wait: with window masks everything is shared (60 000 tokens, 6 blocks: 473 us without all this, 478 with the counters and no waits).  Letting up to 2 | 4 | 8 workgroups of a
+// generation start early: 131 072 tokens 14.05 -> 14.85 | 15.7 | 17.8 ms.  Meeting again 1 | 3 | 7 times during the walk: 13.95 | 14.7 | 16.8, 65 536 tokens 6.05 -> 6.2 | 6.6 | 7.4.  Walking
+// every other generation downwards gave nothing (before there was a pace).  The dQ kernel walks the same way but is not bound by its fetches: waiting cost it 2 %
 // of its time at 40 000 tokens and gained nothing at 64 000.
 #pragma once
 #include "common.h"
