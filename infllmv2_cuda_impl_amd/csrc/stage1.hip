@@ -45,6 +45,7 @@ struct Stage1Params {
     int score_cols;                  // columns to define in every row (max_seqlen_k)
     float scale_log2;
     int causal;
+    int splits;                      // workgroups that share a block of tokens, each with a run of its fine tiles
     int group;                       // query heads per KV head, 1..16: MFMA rows >= group repeat head group - 1 and add nothing
     // pooled output only
     const int* cache_lens;           // per sequence, or null: cache_len for all
@@ -170,7 +171,8 @@ __device__ __forceinline__ void pool_quads(float a, float b, float prev_a, float
 // Bound by the counts, 16 kItems of them to a token, in scalar instructions beside the other wavefronts' exponentials; scores and selection in us, two launches | one, 2 KV heads:
 // 2048 tokens 15.9 | 11.9, 4096 27.3 | 21.2, 8192 56.2 | 48.5, 16 384 133 | 125, 20 480 201 | 196, 32 768 443 | 443, 49 152 931 | 944: rows of 512 blocks and no more.  Whole prefill of
 // 1000 tokens, 16 blocks selected, 42.0 -> 40.7, of 2048 74.4 -> 70.0, training on 1023 + 3001 + 517 + 2200 606 -> 596.
-template <bool kCausal, bool kPool, int kItems = 0>
+// kShared: workgroups share a block of tokens (launch_stage1); a variant of its own, because the others paid 0.5 us for the possibility.
+template <bool kCausal, bool kPool, int kItems = 0, bool kShared = false>
 __global__ __launch_bounds__(64 * kWavesS1) __attribute__((amdgpu_waves_per_eu(kWavesPerSimdS1, kWavesPerSimdS1)))
 void stage1_kernel(const Stage1Params p) {
     __shared__ uint4 tile[2][1024];                            // two 16 KiB operand-ordered key tiles
@@ -183,7 +185,9 @@ void stage1_kernel(const Stage1Params p) {
     const int q0 = p.cu_seqlens_q[b];
     const int Sq = p.cu_seqlens_q[b + 1] - q0;
     // late tokens see the most keys: they go first, so the long workgroups do not form the tail of the launch
-    const int tok_block0 = (static_cast<int>(gridDim.x) - 1 - static_cast<int>(blockIdx.x)) * kTokPerBlock;
+    const int splits = kShared ? p.splits : 1;
+    const int from_end = blockIdx.x / splits, split = blockIdx.x - from_end * splits;
+    const int tok_block0 = (static_cast<int>(gridDim.x) / splits - 1 - from_end) * kTokPerBlock;
     if (tok_block0 >= Sq) return;                              // uniform per workgroup
     const int k0 = p.cu_seqlens_k[b], Lk = p.cu_seqlens_k[b + 1] - k0;
     const int c0 = p.cu_seqlens_c[b], Lc = p.cu_seqlens_c[b + 1] - c0;
@@ -209,6 +213,11 @@ void stage1_kernel(const Stage1Params p) {
     const int wg_vis_f = wg_vis_c == 0 ? 0 : stage1_visible(i_last, 16, Lk, Sq, kCausal);
     const int tiles_c = (wg_vis_c + 63) >> 6;
     const int tiles_f = (wg_vis_f + 63) >> 6;
+    // this workgroup's fine tiles; pooled, the scores of the tile before them are made too, for its last key
+    const int each = (tiles_f + splits - 1) / splits;
+    const int first_f = split * each, end_f = first_f + each < tiles_f ? first_f + each : tiles_f;
+    if (kShared && split > 0 && first_f >= tiles_f) return;    // uniform per workgroup
+    const int begin_f = kShared && kPool && first_f > 0 ? first_f - 1 : first_f;
 
     const elem_bits* cbase = p.c + static_cast<int64_t>(c0) * p.c_row_stride + h * p.c_head_stride;
     const elem_bits* kbase = p.k + static_cast<int64_t>(k0) * p.k_row_stride + h * p.k_head_stride;
@@ -326,7 +335,7 @@ void stage1_kernel(const Stage1Params p) {
         }
 
     // ---------------- pass 2: scores over the fine keys ----------------
-    if (tiles_f > 0) issue_tile(kbase, k_stride, k_off, 0, Lk, lds_tiles, wave_u, n, g);
+    if (begin_f < end_f) issue_tile(kbase, k_stride, k_off, begin_f * 64, Lk, lds_tiles + (begin_f & 1) * 16384, wave_u, n, g);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     static_assert(kTokPerWave == 2, "pool_quads takes two tokens");
@@ -380,9 +389,9 @@ void stage1_kernel(const Stage1Params p) {
             for (int t = 0; t < kTokPerWave; ++t) store(t, at, f32_to_elem_hw(held[t]));
         }
     };
-    for (int ti = 0; ti < tiles_f; ++ti) {
+    for (int ti = begin_f; ti < end_f; ++ti) {
         if (pending) store_held(ti - 1);                       // uniform per wavefront
-        if (ti + 1 < tiles_f) issue_tile(kbase, k_stride, k_off, (ti + 1) * 64, Lk, lds_tiles + ((ti + 1) & 1) * 16384, wave_u, n, g);
+        if (ti + 1 < end_f) issue_tile(kbase, k_stride, k_off, (ti + 1) * 64, Lk, lds_tiles + ((ti + 1) & 1) * 16384, wave_u, n, g);
         const uint4* cur = tile[ti & 1];
         float part[kTokPerWave][4];                            // [t][kt]: this lane's four heads summed, key 16 kt + n
 #pragma unroll
@@ -413,7 +422,8 @@ void stage1_kernel(const Stage1Params p) {
 #pragma unroll
         for (int t = 0; t < kTokPerWave; ++t)
             mine[t] = fold_rows32(fold_rows16(part[t][0], part[t][1]), fold_rows16(part[t][2], part[t][3]));
-        pending = ti >= plain_first && ti < plain_end;
+        const bool mine_too = !kShared || !kPool || ti >= first_f;                   // not the tile before
+        pending = ti >= plain_first && ti < plain_end && mine_too;
         const int col = ti * 64 + lane;
         if (!pending) {
 #pragma unroll
@@ -432,13 +442,14 @@ void stage1_kernel(const Stage1Params p) {
 #pragma unroll
             for (int t = 0; t < kTokPerWave; ++t) {
                 prev[t] = mine[t];
-                if (!pending && live[t] && (lane & 3) == 0 && kb < p.pool_len) store(t, kb, pool_rest(kb, bq[t], held[t]));
+                if (!pending && mine_too && live[t] && (lane & 3) == 0 && kb < p.pool_len) store(t, kb, pool_rest(kb, bq[t], held[t]));
             }
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
     }
-    if (pending) store_held(tiles_f - 1);
+    if (pending) store_held(end_f - 1);
+    if (kShared && end_f < tiles_f) return;                // uniform per workgroup; the rest is the last one's
     // columns no tile covered
 #pragma unroll
     for (int t = 0; t < kTokPerWave; ++t) {
@@ -555,17 +566,25 @@ int launch_stage1(const char* who, void* stream, const void* q, const void* k, c
         p.local_blocks = pool->local_blocks; p.init_blocks = pool->init_blocks;
         p.mask = pool->mask; p.total_q = total_q; p.mask_words = pool->mask_words; p.topk = pool->topk;
     }
-    const dim3 grid((max_seqlen_q + kTokPerBlock - 1) / kTokPerBlock, batch, num_heads_k);
+    // Few workgroups leave CUs idle while each walks all tiles, so they share the fine ones (every one walks the coarse tiles, a quarter as many): as many sharers as
+    // give each CU a workgroup, with four tiles each at least.  Kernel alone, us, 2 KV heads, 20 011 keys: 16 queries 34.8 -> 19.3, 256 35.4 -> 20.1, 512 34.8 -> 21.2, 700 35.2 ->
+    // 25.6, 1024 35.5 -> 27.2; 60 000 keys, one KV head, 300 queries 90.4 -> 36.1; a whole chunk of 512 queries behind 19 499 keys 154.7 -> 139.9.  Two workgroups to a
+    // CU: 700 queries 31.0, 1500 36.1 -> 39.5; two tiles each at least: 256 queries 26.7.
+    const int64_t wgs = static_cast<int64_t>((max_seqlen_q + kTokPerBlock - 1) / kTokPerBlock) * batch * num_heads_k;
+    const int64_t fill = wgs > 0 ? 256 / wgs : 1, most = max_seqlen_k / 256;
+    p.splits = p.mask != nullptr || fill < 2 || most < 2 ? 1 : static_cast<int>(fill < most ? fill : most);
+    const dim3 grid((max_seqlen_q + kTokPerBlock - 1) / kTokPerBlock * p.splits, batch, num_heads_k);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (p.mask) {
         auto kernel = p.pool_len <= 64 ? stage1_kernel<true, true, 1> : p.pool_len <= 128 ? stage1_kernel<true, true, 2> : p.pool_len <= 256 ? stage1_kernel<true, true, 4> : stage1_kernel<true, true, 8>;
         hipLaunchKernelGGL(kernel, grid, dim3(64 * kWavesS1), 0, st, p);
-    } else if (pool) {
-        if (is_causal) hipLaunchKernelGGL((stage1_kernel<true, true>), grid, dim3(64 * kWavesS1), 0, st, p);
-        else hipLaunchKernelGGL((stage1_kernel<false, true>), grid, dim3(64 * kWavesS1), 0, st, p);
     } else {
-        if (is_causal) hipLaunchKernelGGL((stage1_kernel<true, false>), grid, dim3(64 * kWavesS1), 0, st, p);
-        else hipLaunchKernelGGL((stage1_kernel<false, false>), grid, dim3(64 * kWavesS1), 0, st, p);
+        const bool shared = p.splits > 1;
+        auto kernel = pool ? (is_causal ? (shared ? stage1_kernel<true, true, 0, true> : stage1_kernel<true, true>)
+                                        : (shared ? stage1_kernel<false, true, 0, true> : stage1_kernel<false, true>))
+                           : (is_causal ? (shared ? stage1_kernel<true, false, 0, true> : stage1_kernel<true, false>)
+                                        : (shared ? stage1_kernel<false, false, 0, true> : stage1_kernel<false, false>));
+        hipLaunchKernelGGL(kernel, grid, dim3(64 * kWavesS1), 0, st, p);
     }
     IV2_LAUNCH_CHECK();
     return 0;
