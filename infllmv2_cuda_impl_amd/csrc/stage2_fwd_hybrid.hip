@@ -35,6 +35,7 @@
 #include "in_step.h"
 #include "stage2_fwd.h"
 #include <math.h>
+#include <type_traits>
 
 namespace IV2_NS {
 
@@ -69,7 +70,8 @@ __device__ __forceinline__ uint64_t uniform_u64(uint64_t v) {
 // m: its relative rounding error does not depend on the offset, and fp32 l and O have room for 2^kLazyBits many times over.
 constexpr float kLazyLimit = 64.f;                             // 2^6
 
-__device__ __forceinline__ void softmax_step(floatx4 (&s)[4], float& m, float& l, floatx4 (&o)[8], elem8 (&pf)[2],
+template <int kDTiles>
+__device__ __forceinline__ void softmax_step(floatx4 (&s)[4], float& m, float& l, floatx4 (&o)[kDTiles], elem8 (&pf)[2],
                                              int lim, int g, float scale_log2) {
     if (lim < kBlockN - 1) {
 #pragma unroll
@@ -108,7 +110,7 @@ __device__ __forceinline__ void softmax_step(floatx4 (&s)[4], float& m, float& l
         l *= alpha;
         m = m_new;
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt) o[dt] *= alpha;
+        for (int dt = 0; dt < kDTiles; ++dt) o[dt] *= alpha;
     }
     l += rs;
 #pragma unroll
@@ -122,9 +124,15 @@ __device__ __forceinline__ void softmax_step(floatx4 (&s)[4], float& m, float& l
 
 // kLong: sequences long enough for in_step.h, its counters and its pacing; a variant of its own, because a workgroup has its CU to itself and pays for all
 // set-up (the counting alone took 2.6 % where rows are short: 30000 tokens with a window of 9 blocks 536 -> 550 us)
-template <bool kCausal, bool kLong>
+// kParts: so many workgroups share a group, each with its columns of V and O; each computes all of S and P.  A group by itself is a serial chain of
+// turns, 0.98 us for a block of the ring and 1.6 for an own one.  Of a turn, the fetch of V's fragments, the product with them and the rescale are divided, and
+// the CUs that take the other parts are idle where groups are few.  The arithmetic of an element of O and of LSE is the same, step by step, for
+// any kParts: a row keeps its bits.
+template <bool kCausal, bool kLong, int kParts>
 __global__ __launch_bounds__(512)
 void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
+    constexpr int kDTiles = 8 / kParts;                        // of 16 columns each
+    const int d_tile0 = kParts == 1 ? 0 : blockIdx.y * kDTiles;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     uint4* ring = reinterpret_cast<uint4*>(smem_raw);                               // [kRingTiles][2048]: K units 0..1023, V units 1024..2047
     unsigned long long* com = reinterpret_cast<unsigned long long*>(smem_raw + kRingTiles * kTileBytes);   // [mask_words]
@@ -132,7 +140,8 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
 
     // ---- which tokens: XCD-chunked, heaviest first ----
     const int bid = blockIdx.x;
-    const int xcd = bid & 7, sidx = bid >> 3;
+    // (few groups are few chunks: two parts to an XCD fill its CUs, the next two go to another)
+    const int xcd = kParts == 4 ? (bid - 4 * (static_cast<int>(blockIdx.y) >> 1)) & 7 : bid & 7, sidx = bid >> 3;
     int G = ((sidx / kHybChunk) * 8 + xcd) * kHybChunk + (sidx % kHybChunk);
     if (G >= x.total_groups) return;                                                // uniform per workgroup
     G = x.total_groups - 1 - G;
@@ -209,9 +218,9 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
         for (int c = 0; c < 4; ++c) qf[c] = *reinterpret_cast<const elem8*>(qp + 32 * c);
     }
     float m = -INFINITY, l = 0.f;
-    floatx4 o[8];
+    floatx4 o[kDTiles];
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int dt = 0; dt < kDTiles; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     // ---- the walk: one turn = two common blocks (lock step, operands from the LDS ring) alternating with two own
     //      blocks (operands from global memory into registers).  The own blocks' loads keep the vector memory path
@@ -243,7 +252,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
         return ow * 64 + bit;
     };
     const elem_bits* kimg = p.kimg + slot0 * kImageElems + lane * 8;
-    const elem_bits* vimg = p.vimg + slot0 * kImageElems + lane * 8;
+    const elem_bits* vimg = p.vimg + slot0 * kImageElems + lane * 8 + d_tile0 * 1024;
     elem8 kreg[16], vreg[16];
     int jp = live ? next_own() : -1;                           // own block of this turn; its K fragments are loaded a turn ahead
     if (jp >= 0) {
@@ -300,7 +309,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
         // all 16 fragments of a tile are fetched before the MFMAs that use them (vreg is free between own
         // blocks), and the MFMAs run over independent accumulators first
         const uint4* kb = ring + tile * 2048 + lane;
-        const uint4* vb = kb + 1024;
+        const uint4* vb = kb + 1024 + d_tile0 * 128;
 #pragma unroll
         for (int f = 0; f < 16; ++f) {
             const uint4 raw = kb[f * 64];
@@ -315,7 +324,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
             for (int kt = 0; kt < 4; ++kt)
                 s[kt] = IV2_MFMA(vreg[kt * 4 + c], qf[c], s[kt], 0, 0, 0);
 #pragma unroll
-        for (int f = 0; f < 16; ++f) {
+        for (int f = 0; f < 2 * kDTiles; ++f) {
             const uint4 raw = vb[f * 64];
             __builtin_memcpy(&vreg[f], &raw, 16);
         }
@@ -324,14 +333,14 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
 #pragma unroll
         for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
-            for (int dt = 0; dt < 8; ++dt)
+            for (int dt = 0; dt < kDTiles; ++dt)
                 o[dt] = IV2_MFMA(vreg[dt * 2 + cc], pf[cc], o[dt], 0, 0, 0);
     };
     auto own_part = [&]() {
         if (!kLong || k_ready) {
             const elem_bits* src = vimg + static_cast<int64_t>(jp) * kImageElems;
 #pragma unroll
-            for (int f = 0; f < 16; ++f) vreg[f] = *reinterpret_cast<const elem8*>(src + f * 512);
+            for (int f = 0; f < 2 * kDTiles; ++f) vreg[f] = *reinterpret_cast<const elem8*>(src + f * 512);
             floatx4 s[4];
 #pragma unroll
             for (int kt = 0; kt < 4; ++kt) s[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -345,7 +354,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
 #pragma unroll
             for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
-                for (int dt = 0; dt < 8; ++dt)
+                for (int dt = 0; dt < kDTiles; ++dt)
                     o[dt] = IV2_MFMA(vreg[dt * 2 + cc], pf[cc], o[dt], 0, 0, 0);
             jp = next_own();
             k_ready = k_ahead = false;
@@ -396,26 +405,27 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     }
     if (kLong && tid == 0 && x.finished) in_step_finished(finished);       // the first wavefront for its workgroup: its row is one of eight neighbours
     if (share_log2 != 0) {                                     // uniform per workgroup
-        // the ring was not used: 34 floats of every lane, lane by lane
-        float* mine = reinterpret_cast<float*>(smem_raw) + wave * (34 * 64) + lane;
+        // the ring was not used: O, m and l of every lane, lane by lane
+        constexpr int kFloats = 4 * kDTiles + 2;
+        float* mine = reinterpret_cast<float*>(smem_raw) + wave * (kFloats * 64) + lane;
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt)
+        for (int dt = 0; dt < kDTiles; ++dt)
 #pragma unroll
             for (int e = 0; e < 4; ++e) mine[(4 * dt + e) * 64] = o[dt][e];
-        mine[32 * 64] = m;
-        mine[33 * 64] = l;
+        mine[4 * kDTiles * 64] = m;
+        mine[(4 * kDTiles + 1) * 64] = l;
         __syncthreads();
         if (part != 0 || !live) return;
         for (int other = 1; other < (1 << share_log2); ++other) {
-            const float* theirs = mine + other * slots * (34 * 64);
-            const float m2 = theirs[32 * 64], m_new = fmaxf(m, m2);
+            const float* theirs = mine + other * slots * (kFloats * 64);
+            const float m2 = theirs[4 * kDTiles * 64], m_new = fmaxf(m, m2);
             const float m_use = (m_new == -INFINITY) ? 0.f : m_new;                 // neither has a key
             const float a1 = __builtin_amdgcn_exp2f(m - m_use), a2 = __builtin_amdgcn_exp2f(m2 - m_use);
 #pragma unroll
-            for (int dt = 0; dt < 8; ++dt)
+            for (int dt = 0; dt < kDTiles; ++dt)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) o[dt][e] = o[dt][e] * a1 + theirs[(4 * dt + e) * 64] * a2;
-            l = l * a1 + theirs[33 * 64] * a2;
+            l = l * a1 + theirs[(4 * kDTiles + 1) * 64] * a2;
             m = m_new;
         }
     }
@@ -425,15 +435,15 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     const float l_tot = wave_sum_over_g(l);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     if (n >= p.group) return;                                  // rows that only fill the MFMA tile
-    elem_bits* op = p.out + tok * p.o_tok_stride + h * p.o_kvh_stride + n * p.o_grp_stride + 4 * g;
+    elem_bits* op = p.out + tok * p.o_tok_stride + h * p.o_kvh_stride + n * p.o_grp_stride + 4 * g + 16 * d_tile0;
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) {
+    for (int dt = 0; dt < kDTiles; ++dt) {
         uint2 wv;
         wv.x = pack_elem2(o[dt][0] * inv, o[dt][1] * inv);
         wv.y = pack_elem2(o[dt][2] * inv, o[dt][3] * inv);
         *reinterpret_cast<uint2*>(op + 16 * dt) = wv;
     }
-    if (g == 0) {
+    if (g == 0 && d_tile0 == 0) {
         const float lse = l_tot > 0.f ? m * 0.69314718055994530942f + logf(l_tot) : INFINITY;
         p.lse[h * p.lse_kvh_stride + tok * p.lse_tok_stride + n * p.lse_grp_stride] = lse;
     }
@@ -458,12 +468,25 @@ int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int 
     const int64_t grid = (total + per_round - 1) / per_round * per_round;
     const size_t lds = kRingTiles * kTileBytes + static_cast<size_t>(1 + kHybTokens) * x.mask_words * 8;
     const bool far = max_seqlen_k > kInStepKeys;
-    auto kernel = causal ? (far ? stage2_fwd_hybrid_kernel<true, true> : stage2_fwd_hybrid_kernel<true, false>)
-                         : (far ? stage2_fwd_hybrid_kernel<false, true> : stage2_fwd_hybrid_kernel<false, false>);
-    x.finished = in_step;
+    // As many parts as give every workgroup a CU of its own (256).  Up to 64 groups, kernel in us, one part -> four: 16 tokens behind 20011 with 2 KV heads and 96
+    // blocks 92.6 -> 70.3, 256 of them 88.0 -> 67.3, 256 tokens of 3000 52.0 -> 42.4; up to 128, one -> two: 512 behind 20011 88.0 -> 76.0, 300 behind 60000
+    // with one KV head 105 -> 81, 1024 of them 104 -> 87.  Sequences of their own too: 4 tokens each of 32
+    // with 8192 keys 148 -> 97, one each of 60 with 4096 58 -> 48.  More parts than CUs run in two rounds: four parts of 16 tokens on the CUs of one XCD took 138.
+    // So few groups run all at once and need no pace: they neither count nor wait (in_step.h).
+    // A part may end before another has read Q: outputs written over Q are left to one part.
+    auto spread = [&](int64_t tok, int64_t grp, int64_t kvh) { return (p.total_q - 1) * tok + (p.group - 1) * grp + (num_heads_k - 1) * kvh + kHeadDim; };
+    const bool apart = p.out >= p.q + spread(p.q_tok_stride, p.q_grp_stride, p.q_kvh_stride) || p.q >= p.out + spread(p.o_tok_stride, p.o_grp_stride, p.o_kvh_stride);
+    const int parts = !apart || total * 2 > 256 ? 1 : total * 4 > 256 ? 2 : 4;
+    x.finished = parts > 1 ? nullptr : in_step;
+    auto pick = [&](auto two) {
+        constexpr int kParts = decltype(two)::value;
+        return causal ? (far ? stage2_fwd_hybrid_kernel<true, true, kParts> : stage2_fwd_hybrid_kernel<true, false, kParts>)
+                      : (far ? stage2_fwd_hybrid_kernel<false, true, kParts> : stage2_fwd_hybrid_kernel<false, false, kParts>);
+    };
+    auto kernel = parts == 4 ? pick(std::integral_constant<int, 4>{}) : parts == 2 ? pick(std::integral_constant<int, 2>{}) : pick(std::integral_constant<int, 1>{});
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     IV2_CHECK(e == hipSuccess, "varlen_fwd: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(512), lds, st, p, x);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid), parts), dim3(512), lds, st, p, x);
     IV2_LAUNCH_CHECK();
     return 0;
 }
