@@ -70,8 +70,7 @@ __device__ __forceinline__ uint64_t uniform_u64(uint64_t v) {
 // m: its relative rounding error does not depend on the offset, and fp32 l and O have room for 2^kLazyBits many times over.
 constexpr float kLazyLimit = 64.f;                             // 2^6
 
-template <int kDTiles>
-__device__ __forceinline__ void softmax_step(floatx4 (&s)[4], float& m, float& l, floatx4 (&o)[kDTiles], elem8 (&pf)[2],
+__device__ __forceinline__ void softmax_step(floatx4 (&s)[4], float& m, float& l, floatx4 (&o)[8], elem8 (&pf)[2],
                                              int lim, int g, float scale_log2) {
     if (lim < kBlockN - 1) {
 #pragma unroll
@@ -110,7 +109,7 @@ __device__ __forceinline__ void softmax_step(floatx4 (&s)[4], float& m, float& l
         l *= alpha;
         m = m_new;
 #pragma unroll
-        for (int dt = 0; dt < kDTiles; ++dt) o[dt] *= alpha;
+        for (int dt = 0; dt < 8; ++dt) o[dt] *= alpha;
     }
     l += rs;
 #pragma unroll
@@ -124,15 +123,11 @@ __device__ __forceinline__ void softmax_step(floatx4 (&s)[4], float& m, float& l
 
 // kLong: sequences long enough for in_step.h, its counters and its pacing; a variant of its own, because a workgroup has its CU to itself and pays for all
 // set-up (the counting alone took 2.6 % where rows are short: 30000 tokens with a window of 9 blocks 536 -> 550 us)
-// kParts: so many workgroups share a group, each with its columns of V and O; each computes all of S and P.  A group by itself is a serial chain of
-// turns, 0.98 us for a block of the ring and 1.6 for an own one.  Of a turn, the fetch of V's fragments, the product with them and the rescale are divided, and
-// the CUs that take the other parts are idle where groups are few.  The arithmetic of an element of O and of LSE is the same, step by step, for
-// any kParts: a row keeps its bits.
+// kParts: so many workgroups share a group, each with some of its tokens.  All of them choose the blocks walked together from the group's eight rows and bring them
+// through their rings; a wavefront of another part's token only helps with that.  A row is added up in the same order for any kParts.
 template <bool kCausal, bool kLong, int kParts>
 __global__ __launch_bounds__(512)
 void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
-    constexpr int kDTiles = 8 / kParts;                        // of 16 columns each
-    const int d_tile0 = kParts == 1 ? 0 : blockIdx.y * kDTiles;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     uint4* ring = reinterpret_cast<uint4*>(smem_raw);                               // [kRingTiles][2048]: K units 0..1023, V units 1024..2047
     unsigned long long* com = reinterpret_cast<unsigned long long*>(smem_raw + kRingTiles * kTileBytes);   // [mask_words]
@@ -141,7 +136,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     // ---- which tokens: XCD-chunked, heaviest first ----
     const int bid = blockIdx.x;
     // (few groups are few chunks: two parts to an XCD fill its CUs, the next two go to another)
-    const int xcd = kParts == 4 ? (bid - 4 * (static_cast<int>(blockIdx.y) >> 1)) & 7 : bid & 7, sidx = bid >> 3;
+    const int xcd = (kParts <= 2 ? bid : bid - 16 / kParts * (static_cast<int>(blockIdx.y) >> 1)) & 7, sidx = bid >> 3;
     int G = ((sidx / kHybChunk) * 8 + xcd) * kHybChunk + (sidx % kHybChunk);
     if (G >= x.total_groups) return;                                                // uniform per workgroup
     G = x.total_groups - 1 - G;
@@ -174,6 +169,9 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     const int part = wave >> (3 - share_log2);
     const int i = i0 + (wave & (slots - 1));                                        // this wavefront's token
     const bool live = i < Sq;
+    const int slots_of_part = slots > kParts ? slots / kParts : 1;
+    const bool walks = live && (kParts == 1 || (wave & (slots - 1)) / slots_of_part == static_cast<int>(blockIdx.y));
+    if (kParts > 1 && static_cast<int>(blockIdx.y) * slots_of_part >= in_group) return;    // uniform: none of the part's tokens is there
     int last_key = kCausal ? (i + Sk - Sq) : (Sk - 1);                              // largest allowed key index
     if (last_key > Sk - 1) last_key = Sk - 1;
     if (!live) last_key = -1;
@@ -218,9 +216,9 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
         for (int c = 0; c < 4; ++c) qf[c] = *reinterpret_cast<const elem8*>(qp + 32 * c);
     }
     float m = -INFINITY, l = 0.f;
-    floatx4 o[kDTiles];
+    floatx4 o[8];
 #pragma unroll
-    for (int dt = 0; dt < kDTiles; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int dt = 0; dt < 8; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     // ---- the walk: one turn = two common blocks (lock step, operands from the LDS ring) alternating with two own
     //      blocks (operands from global memory into registers).  The own blocks' loads keep the vector memory path
@@ -238,7 +236,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
             crow = uniform_u64(own[cw]);
         }
         const int bit = __builtin_ctzll(cbits);
-        mine = (crow >> bit) & 1ull;
+        mine = (kParts == 1 || walks) && ((crow >> bit) & 1ull);
         cbits &= cbits - 1ull;
         return cw * 64 + bit;
     };
@@ -252,9 +250,9 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
         return ow * 64 + bit;
     };
     const elem_bits* kimg = p.kimg + slot0 * kImageElems + lane * 8;
-    const elem_bits* vimg = p.vimg + slot0 * kImageElems + lane * 8 + d_tile0 * 1024;
+    const elem_bits* vimg = p.vimg + slot0 * kImageElems + lane * 8;
     elem8 kreg[16], vreg[16];
-    int jp = live ? next_own() : -1;                           // own block of this turn; its K fragments are loaded a turn ahead
+    int jp = walks ? next_own() : -1;                           // own block of this turn; its K fragments are loaded a turn ahead
     if (jp >= 0) {
         const elem_bits* src = kimg + static_cast<int64_t>(jp) * kImageElems;
 #pragma unroll
@@ -309,7 +307,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
         // all 16 fragments of a tile are fetched before the MFMAs that use them (vreg is free between own
         // blocks), and the MFMAs run over independent accumulators first
         const uint4* kb = ring + tile * 2048 + lane;
-        const uint4* vb = kb + 1024 + d_tile0 * 128;
+        const uint4* vb = kb + 1024;
 #pragma unroll
         for (int f = 0; f < 16; ++f) {
             const uint4 raw = kb[f * 64];
@@ -324,7 +322,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
             for (int kt = 0; kt < 4; ++kt)
                 s[kt] = IV2_MFMA(vreg[kt * 4 + c], qf[c], s[kt], 0, 0, 0);
 #pragma unroll
-        for (int f = 0; f < 2 * kDTiles; ++f) {
+        for (int f = 0; f < 16; ++f) {
             const uint4 raw = vb[f * 64];
             __builtin_memcpy(&vreg[f], &raw, 16);
         }
@@ -333,14 +331,14 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
 #pragma unroll
         for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
-            for (int dt = 0; dt < kDTiles; ++dt)
+            for (int dt = 0; dt < 8; ++dt)
                 o[dt] = IV2_MFMA(vreg[dt * 2 + cc], pf[cc], o[dt], 0, 0, 0);
     };
     auto own_part = [&]() {
         if (!kLong || k_ready) {
             const elem_bits* src = vimg + static_cast<int64_t>(jp) * kImageElems;
 #pragma unroll
-            for (int f = 0; f < 2 * kDTiles; ++f) vreg[f] = *reinterpret_cast<const elem8*>(src + f * 512);
+            for (int f = 0; f < 16; ++f) vreg[f] = *reinterpret_cast<const elem8*>(src + f * 512);
             floatx4 s[4];
 #pragma unroll
             for (int kt = 0; kt < 4; ++kt) s[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -354,7 +352,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
 #pragma unroll
             for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
-                for (int dt = 0; dt < kDTiles; ++dt)
+                for (int dt = 0; dt < 8; ++dt)
                     o[dt] = IV2_MFMA(vreg[dt * 2 + cc], pf[cc], o[dt], 0, 0, 0);
             jp = next_own();
             k_ready = k_ahead = false;
@@ -405,45 +403,44 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     }
     if (kLong && tid == 0 && x.finished) in_step_finished(finished);       // the first wavefront for its workgroup: its row is one of eight neighbours
     if (share_log2 != 0) {                                     // uniform per workgroup
-        // the ring was not used: O, m and l of every lane, lane by lane
-        constexpr int kFloats = 4 * kDTiles + 2;
-        float* mine = reinterpret_cast<float*>(smem_raw) + wave * (kFloats * 64) + lane;
+        // the ring was not used: 34 floats of every lane, lane by lane
+        float* mine = reinterpret_cast<float*>(smem_raw) + wave * (34 * 64) + lane;
 #pragma unroll
-        for (int dt = 0; dt < kDTiles; ++dt)
+        for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
             for (int e = 0; e < 4; ++e) mine[(4 * dt + e) * 64] = o[dt][e];
-        mine[4 * kDTiles * 64] = m;
-        mine[(4 * kDTiles + 1) * 64] = l;
+        mine[32 * 64] = m;
+        mine[33 * 64] = l;
         __syncthreads();
-        if (part != 0 || !live) return;
+        if (part != 0 || !walks) return;
         for (int other = 1; other < (1 << share_log2); ++other) {
-            const float* theirs = mine + other * slots * (kFloats * 64);
-            const float m2 = theirs[4 * kDTiles * 64], m_new = fmaxf(m, m2);
+            const float* theirs = mine + other * slots * (34 * 64);
+            const float m2 = theirs[32 * 64], m_new = fmaxf(m, m2);
             const float m_use = (m_new == -INFINITY) ? 0.f : m_new;                 // neither has a key
             const float a1 = __builtin_amdgcn_exp2f(m - m_use), a2 = __builtin_amdgcn_exp2f(m2 - m_use);
 #pragma unroll
-            for (int dt = 0; dt < kDTiles; ++dt)
+            for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) o[dt][e] = o[dt][e] * a1 + theirs[(4 * dt + e) * 64] * a2;
-            l = l * a1 + theirs[(4 * kDTiles + 1) * 64] * a2;
+            l = l * a1 + theirs[33 * 64] * a2;
             m = m_new;
         }
     }
-    if (!live) return;
+    if (!walks) return;
 
     // ---- epilogue ----
     const float l_tot = wave_sum_over_g(l);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     if (n >= p.group) return;                                  // rows that only fill the MFMA tile
-    elem_bits* op = p.out + tok * p.o_tok_stride + h * p.o_kvh_stride + n * p.o_grp_stride + 4 * g + 16 * d_tile0;
+    elem_bits* op = p.out + tok * p.o_tok_stride + h * p.o_kvh_stride + n * p.o_grp_stride + 4 * g;
 #pragma unroll
-    for (int dt = 0; dt < kDTiles; ++dt) {
+    for (int dt = 0; dt < 8; ++dt) {
         uint2 wv;
         wv.x = pack_elem2(o[dt][0] * inv, o[dt][1] * inv);
         wv.y = pack_elem2(o[dt][2] * inv, o[dt][3] * inv);
         *reinterpret_cast<uint2*>(op + 16 * dt) = wv;
     }
-    if (g == 0 && d_tile0 == 0) {
+    if (g == 0) {
         const float lse = l_tot > 0.f ? m * 0.69314718055994530942f + logf(l_tot) : INFINITY;
         p.lse[h * p.lse_kvh_stride + tok * p.lse_tok_stride + n * p.lse_grp_stride] = lse;
     }
@@ -468,22 +465,21 @@ int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int 
     const int64_t grid = (total + per_round - 1) / per_round * per_round;
     const size_t lds = kRingTiles * kTileBytes + static_cast<size_t>(1 + kHybTokens) * x.mask_words * 8;
     const bool far = max_seqlen_k > kInStepKeys;
-    // As many parts as give every workgroup a CU of its own (256).  Up to 64 groups, kernel in us, one part -> four: 16 tokens behind 20011 with 2 KV heads and 96
-    // blocks 92.6 -> 70.3, 256 of them 88.0 -> 67.3, 256 tokens of 3000 52.0 -> 42.4; up to 128, one -> two: 512 behind 20011 88.0 -> 76.0, 300 behind 60000
-    // with one KV head 105 -> 81, 1024 of them 104 -> 87.  Sequences of their own too: 4 tokens each of 32
-    // with 8192 keys 148 -> 97, one each of 60 with 4096 58 -> 48.  More parts than CUs run in two rounds: four parts of 16 tokens on the CUs of one XCD took 138.
+    // As many parts as give every workgroup a CU of its own (256).  A group's turn is bound by what its eight rows fetch through one CU's vector memory path (256 KiB for
+    // a block of their own each, 1.6 us) and read from its LDS; its parts have a CU each for that, at the price of a ring each.  Kernel in us, one part ->
+    // two: 512 tokens behind 20011 with 2 KV heads and 96 blocks 88 -> 60, 300 behind 60000 with one head 105 -> 67, 1024 of them 104 -> 78; four: 256
+    // tokens behind 20011 88 -> 51 (two 60), 256 of 3000 52 -> 41; eight: 64 behind 20011 95 -> 50 (four 54), 8 each of 8 sequences with 9000 keys
+    // 101 -> 55 (four 64).  Parts by columns of V, which repeat the products with K: 70 for the four and the eight, 76 for the two.  More workgroups than CUs run in two rounds
+    // and gain nothing: 700 tokens behind 20011, 176 groups, take 102 whole.
     // So few groups run all at once and need no pace: they neither count nor wait (in_step.h).
-    // A part may end before another has read Q: outputs written over Q are left to one part.
-    auto spread = [&](int64_t tok, int64_t grp, int64_t kvh) { return (p.total_q - 1) * tok + (p.group - 1) * grp + (num_heads_k - 1) * kvh + kHeadDim; };
-    const bool apart = p.out >= p.q + spread(p.q_tok_stride, p.q_grp_stride, p.q_kvh_stride) || p.q >= p.out + spread(p.o_tok_stride, p.o_grp_stride, p.o_kvh_stride);
-    const int parts = !apart || total * 2 > 256 ? 1 : total * 4 > 256 ? 2 : 4;
+    const int parts = total * 2 > 256 ? 1 : total * 4 > 256 ? 2 : total * 8 > 256 ? 4 : 8;
     x.finished = parts > 1 ? nullptr : in_step;
-    auto pick = [&](auto two) {
-        constexpr int kParts = decltype(two)::value;
+    auto pick = [&](auto n) {
+        constexpr int kParts = decltype(n)::value;
         return causal ? (far ? stage2_fwd_hybrid_kernel<true, true, kParts> : stage2_fwd_hybrid_kernel<true, false, kParts>)
                       : (far ? stage2_fwd_hybrid_kernel<false, true, kParts> : stage2_fwd_hybrid_kernel<false, false, kParts>);
     };
-    auto kernel = parts == 4 ? pick(std::integral_constant<int, 4>{}) : parts == 2 ? pick(std::integral_constant<int, 2>{}) : pick(std::integral_constant<int, 1>{});
+    auto kernel = parts == 8 ? pick(std::integral_constant<int, 8>{}) : parts == 4 ? pick(std::integral_constant<int, 4>{}) : parts == 2 ? pick(std::integral_constant<int, 2>{}) : pick(std::integral_constant<int, 1>{});
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     IV2_CHECK(e == hipSuccess, "varlen_fwd: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid), parts), dim3(512), lds, st, p, x);
