@@ -465,11 +465,22 @@ void topk_wide_kernel(const TopkParams p) {
     }
 }
 
+// A dispatch holds fewer than 2^32 work-items in a dimension: 8 388 607 workgroups.
+constexpr int64_t kTopkWideChunk = 1 << 22;
+
 template <int kItems>
 static int launch_topk_wide(void* stream, const TopkParams& p) {
-    hipLaunchKernelGGL(topk_wide_kernel<kItems>, dim3(static_cast<unsigned>(p.rows)), dim3(kTopkRowWaves * 64),
-                       sizeof(uint32_t) * (p.k > 0 ? p.k : 1), static_cast<hipStream_t>(stream), p);
-    IV2_LAUNCH_CHECK();
+    for (int64_t first = 0; first < p.rows; first += kTopkWideChunk) {
+        TopkParams c = p;
+        c.x += first * p.row_stride;
+        if (c.out_idx) c.out_idx += first * p.out_stride;
+        if (c.out_val) c.out_val += first * p.out_stride;
+        if (c.out_mask) c.out_mask += first * p.n64;
+        c.rows = p.rows - first < kTopkWideChunk ? p.rows - first : kTopkWideChunk;
+        hipLaunchKernelGGL(topk_wide_kernel<kItems>, dim3(static_cast<unsigned>(c.rows)), dim3(kTopkRowWaves * 64),
+                           sizeof(uint32_t) * (p.k > 0 ? p.k : 1), static_cast<hipStream_t>(stream), c);
+        IV2_LAUNCH_CHECK();
+    }
     return 0;
 }
 
@@ -503,7 +514,7 @@ static int launch_topk(void* stream, const TopkParams& p) {
 // 4096 25.4 | 19.9, 8192 40.7 | 36.9 (of 2048 13.1 | 11.0, 18.9 | 20.2, 33.1 | 37.9); 3000, 16 384 rows 249 | 104, 65 536 763 | 406 (of 4096 136 | 106, 429 | 421, mask words
 // alone 93 | 95, 283 | 376); 8192, 2048 rows 80 | 28, 65 536 1500 | 768.  Up to 256 columns both take what a launch takes (4.3).
 static int64_t wide_rows(int n) {
-    return n <= 256 ? 0 : n <= 512 ? 768 : n <= 1024 ? 1024 : n <= 2048 ? 2048 : n <= 4096 ? 16384 : 0x7fffffff;
+    return n <= 256 ? 0 : n <= 512 ? 768 : n <= 1024 ? 1024 : n <= 2048 ? 2048 : n <= 4096 ? 16384 : INT64_MAX;
 }
 
 static int topk_dispatch(void* stream, const uint16_t* x, int64_t row_stride, int32_t* idx, uint16_t* val,
@@ -520,7 +531,6 @@ static int topk_dispatch(void* stream, const uint16_t* x, int64_t row_stride, in
     p.x = x; p.row_stride = row_stride; p.out_idx = idx; p.out_val = val; p.out_mask = mask;
     p.out_stride = out_stride; p.n64 = n64; p.rows = rows; p.n = n; p.k = k;
     p.by_index = by_index; p.drop_neg_inf = drop_neg_inf; p.neg_inf_key = dtype == 0 ? kKeyNegInfFp16 : kKeyNegInfBf16;
-    IV2_CHECK(n <= 4096 || rows <= 0x7fffffff, "topk: too many rows");
     if (rows <= wide_rows(n)) {
         if (n <= 512) return launch_topk_wide<1>(stream, p);
         if (n <= 1024) return launch_topk_wide<2>(stream, p);

@@ -65,3 +65,15 @@ def test_both_sides_of_the_rule(rows, n):
     gen = torch.Generator(device="cuda").manual_seed(rows)
     for kind in ("scores", "inf"):
         check(rows_of(kind, rows, n, gen), 32)
+
+
+def test_more_long_rows_than_a_dispatch_holds():
+    """Rows of more than 4096 columns take a workgroup of 512 threads each, and a dispatch fewer than 2^32 threads: 8 388 608 rows and some more, all of them
+    the same one (row stride 0), so that the scores take little memory."""
+    from infllmv2_cuda_impl_amd import _lib
+    n, rows = 4097, (1 << 23) + 5
+    x = torch.rand(1, n, generator=torch.Generator(device="cuda").manual_seed(3), device="cuda").to(torch.bfloat16)
+    idx = torch.full((rows, 1), -7, dtype=torch.int32, device="cuda")
+    _lib.call("infllmv2_topk_select", torch.cuda.current_stream().cuda_stream, x.data_ptr(), 0, 1, idx.data_ptr(), None, rows, n, 1, 0, 0, 0)
+    best = int((x[0] == x[0].max()).nonzero()[0])
+    assert (idx == best).all()
