@@ -363,7 +363,7 @@ void stage1_kernel(const Stage1Params p) {
         if (kPool) {
             before_local = before_local < p.pool_len ? before_local : p.pool_len;
             plain_end = before_local < 0 ? 0 : (before_local >> 4) < plain_end ? before_local >> 4 : plain_end;
-            plain_first = (p.init_blocks + 15) >> 4;
+            plain_first = (p.init_blocks >> 4) + ((p.init_blocks & 15) != 0 ? 1 : 0);      // (rounded up without a sum that could overflow)
         }
     }
     // value of a pooled entry that no visible key reaches

@@ -106,3 +106,14 @@ def test_other_windows_are_rejected(ops):
             256, int(cu_f[-1]))
     with pytest.raises(RuntimeError, match="only the 5/4/1 window"):
         ops.infllmv2_attn_stage1_pooled(*args, 1, 1, block_size=128, causal=True)
+
+
+@pytest.mark.parametrize("init", [2 ** 31 - 1, 2 ** 31 - 16, 130])
+def test_more_initial_blocks_than_a_row_has(ops, init):
+    """Every block that is there is an initial one, whatever the number: the first key tiles of long rows are the ones that skip the test for it."""
+    S = 4160
+    q, cu, kf, cu_f, kc, cu_c = inputs(5, [S])
+    args = (q.to("cuda:0"), to_dev(kf, torch.bfloat16), to_dev(kc, torch.bfloat16), to_dev(cu), to_dev(cu_f), to_dev(cu_c),
+            S, int(cu_f[-1]))
+    fused = ops.infllmv2_attn_stage1_pooled(*args, 1, init, causal=True)
+    assert torch.isposinf(fused).all()
