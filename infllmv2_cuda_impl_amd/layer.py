@@ -105,6 +105,8 @@ class InfLLMv2Attention(torch.nn.Module):
         if self.selection == "window" and max_seqlen > self.dense_len:
             topk_idx, mask = self._window_blocks(k.shape[1], q.shape[0], cu_seqlens, None, max_seqlen, 0)
         elif self.selection == "sparse" and max_seqlen > self.dense_len:
+            if self.topk < 1:
+                raise RuntimeError("topk: the sparse selection takes at least one block per row")
             # the selection writes the packed mask Stage 2 walks, no list, and the block images of k and v
             scale = q.shape[-1] ** (-0.5) if self.softmax_scale is None else self.softmax_scale
             qs, ks = (q, k) if q.shape[-1] == HEAD_DIM else pad_head_dim(q, k)

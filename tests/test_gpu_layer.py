@@ -129,3 +129,11 @@ def test_window_and_dense_branches(ops):
                               v1[t][None, None].expand(2, 1, 2, 128).contiguous(), bcache)
         e = (ob[0, 0].float() - full[t].float()).abs()
         assert float(e.max()) <= 2e-2 and float(e.mean()) <= 1e-3, t
+
+
+def test_prefill_refuses_to_select_nothing():
+    import infllmv2_cuda_impl_amd as ops
+    r = lambda heads: torch.zeros(300, heads, 128, dtype=torch.bfloat16, device="cuda")
+    cu = torch.tensor([0, 300], dtype=torch.int32, device="cuda")
+    with pytest.raises(RuntimeError, match="topk"):
+        ops.InfLLMv2Attention(topk=0, local_blocks=1, init_blocks=1)(r(32), r(2), r(2), cu, 300)
