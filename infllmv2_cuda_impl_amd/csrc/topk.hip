@@ -46,6 +46,7 @@ struct TopkParams {
     int drop_neg_inf;                // 1: columns whose score is -inf are never selected (-1 instead)
     int rows_per_wave;
     uint32_t neg_inf_key;
+    int first_shift;                 // keys per bin of a workgroup's first histogram, log2
 };
 
 constexpr int kTopkWaves = 4;
@@ -329,18 +330,21 @@ __device__ __forceinline__ int wave_max(int v) {
 // The same selection with a whole workgroup per row, for few or long rows: with a wavefront per row few rows leave the chip idle and the kernel takes as long
 // as one wavefront needs for one row, and a long row is more than its registers hold.  Column
 // 512 e + 64 wave + lane sits in register e, so a wavefront's ballot is mask word 8 e + wave.  Bound by a chain of barriers and trips to LDS, so it has few:
-// one histogram of the keys up to 1022 (eight powers of two of bfloat16) below the largest finite score, and two scans over the lanes, find the k-th
-// key.  Whatever bits the row holds, a round finds it or starts the next one 1023 keys further down.  (Two bits of the key per round by counts, a barrier
-// each: 48 rows of 626 columns 5.7 -> 4.2 us, 128 of 2048 6.5 -> 4.3, 64 of 4000 8.5 -> 5.2, 16 of 8000 14.4 -> 7.4; a whole paged decode step of 24 sequences
-// 44.0 -> 42.6.  What lies below the histogram counted in a bin of its own, one address for all of them: 64 of 4000 8.5.)
-constexpr int kTopkRowWaves = 8;
+// one histogram of 1023 bins below the largest finite score and two scans over the lanes find the bin of the k-th key.  The bins reach down eight powers of two: a
+// key each in bfloat16, eight keys in IEEE half.  What lies further down goes into a second histogram whose bins of 64 keys reach the smallest key there is, and a bin of
+// several keys is opened once: three barriers or five, whatever bits the row holds.
+// us, by counts of two bits of the key per barrier | by histograms of 1023 single keys, each from where the last ended | now: bfloat16 scores within a few powers of two, 16 rows
+// of 626 columns 5.7 | 3.3 | 3.3, 512 of 2048 8.3 | 5.4 | 5.2, 128 of 8000 14.5 | 7.4 | 7.5; in IEEE half 512 of 626 6.6 | 7.9 | 4.3; half over thirty powers of two, 512 of 2048
+// 8.3 | 14.2 | 6.4; fewer columns above -inf than wanted, 128 of 2048 6.6 | 7.6 | 4.7, 1024 of 8000 42 | 46 | 21; one value in all columns, 1024 of 4096 21 | 20 | 9.1.
+constexpr int kTopkRowWaves = 8, kTopkBins = 1023;
 
 template <int kItems>
 __global__ __launch_bounds__(kTopkRowWaves * 64)
 void topk_wide_kernel(const TopkParams p) {
     extern __shared__ uint32_t sel[];                          // k survivors
-    __shared__ __attribute__((aligned(16))) uint32_t bins[512];                                      // two 16-bit counts each
-    __shared__ int2 tops[2][kTopkRowWaves];                    // per wavefront: its largest key up to the limit, its columns above it
+    __shared__ __attribute__((aligned(16))) uint32_t bins[2][512];                                   // two 16-bit counts each
+    __shared__ uint32_t fine_bins[32];                         // of the bin that is opened
+    __shared__ int2 tops[kTopkRowWaves];                       // per wavefront: its largest key up to the limit, its columns above it
     __shared__ uint32_t word_counts[kItems * kTopkRowWaves];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -354,11 +358,13 @@ void topk_wide_kernel(const TopkParams p) {
         const int col = e * kTopkRowWaves * 64 + tid;
         key[e] = col < n ? src[col] : 0;
     }
-    bins[tid] = 0u;
+    bins[0][tid] = bins[1][tid] = 0u;
+    if (tid < 32) fine_bins[tid] = 0u;
 #pragma unroll
     for (int e = 0; e < kItems; ++e) key[e] = e * kTopkRowWaves * 64 + tid < n ? static_cast<int>(sortable16(key[e])) : -1;
-    int thr = 0, limit = 0xffff - p.neg_inf_key;               // +inf, the forced blocks, stays above the histogram
-    for (int round = 0; k_sel > 0; ++round) {
+    int thr = 0;                                               // the k-th key
+    if (k_sel > 0) {
+        const int limit = 0xffff - p.neg_inf_key;              // +inf, the forced blocks, stays above the first histogram
         int top = -1, above = 0;
 #pragma unroll
         for (int e = 0; e < kItems; ++e) {
@@ -366,32 +372,73 @@ void topk_wide_kernel(const TopkParams p) {
             above += __builtin_popcountll(__builtin_amdgcn_ballot_w64(key[e] > limit));
         }
         top = wave_max(top);
-        if (lane == 0) tops[round & 1][wave] = make_int2(top, above);
+        if (lane == 0) tops[wave] = make_int2(top, above);
         __syncthreads();
-        const int2 t = tops[round & 1][lane & (kTopkRowWaves - 1)];
+        const int2 t = tops[lane & (kTopkRowWaves - 1)];
         top = eight_max(t.x);
         above = eight_sum(t.y);
-        if (above >= k_sel) { limit = 0xffff; continue; }      // only at first: no more than forced blocks are wanted
-        const int lowest = max(top - 1022, 0);                 // of the histogram; what lies further down would all add to one bin
+        if (above >= k_sel) { top = 0xffff; above = 0; }       // no more than forced blocks are wanted
+        auto add = [&](uint32_t* counts, int bin, int n) { atomicAdd(&counts[bin >> 1], static_cast<uint32_t>(n) << (16 * (bin & 1))); };
+        // A key's bin, negative: none.  Many of a wavefront's keys may be in one (zeros, -inf), and an atomic takes a turn for each of them: those in lane 0's are added at once.
+        auto add_together = [&](uint32_t* counts, int bin) {
+            const int its = __builtin_amdgcn_readfirstlane(bin);
+            const int alike = __builtin_popcountll(__builtin_amdgcn_ballot_w64(bin == its));
+            if (bin >= 0 && (bin != its || lane == 0)) add(counts, bin, bin != its ? 1 : alike);
+        };
+        int bin = 0;                                           // of the k-th key, of 2^shift keys
+        auto find = [&](const uint32_t* counts) {
+            __syncthreads();
+            const uint4 a = *reinterpret_cast<const uint4*>(&counts[8 * lane]), b = *reinterpret_cast<const uint4*>(&counts[8 * lane + 4]);
+            const uint32_t pairs = a.x + a.y + a.z + a.w + b.x + b.y + b.z + b.w;
+            const int mine = static_cast<int>((pairs & 0xffffu) + (pairs >> 16));
+            const int upto = scan_lanes(mine) + above;
+            const uint64_t enough = __builtin_amdgcn_ballot_w64(upto >= k_sel);
+            if (enough == 0ull) {                              // uniform over the workgroup
+                above = __builtin_amdgcn_readlane(upto, 63);
+                return false;
+            }
+            const int at = __builtin_ctzll(enough);
+            const int here = lane < 16 ? static_cast<int>(reinterpret_cast<const uint16_t*>(counts)[16 * at + lane]) : 0;
+            const int here_upto = scan_lanes(here) + static_cast<int>(__builtin_amdgcn_readlane(upto - mine, at));
+            const int in = __builtin_ctzll(__builtin_amdgcn_ballot_w64(here_upto >= k_sel));
+            above = __builtin_amdgcn_readlane(here_upto - here, in);
+            bin = 16 * at + in;
+            return true;
+        };
+        int shift = p.first_shift;
+        {
+            const int span = min(kTopkBins << shift, top);     // a key is at least 1
+            int tops_here = 0;                                 // counted apart: in a row of equal scores they are all
 #pragma unroll
-        for (int e = 0; e < kItems; ++e) {
-            const int bin = top - key[e];
-            if (key[e] <= limit && key[e] >= lowest) atomicAdd(&bins[bin >> 1], (bin & 1) ? 0x10000u : 1u);
+            for (int e = 0; e < kItems; ++e) {
+                const int down = top - key[e];
+                tops_here += __builtin_popcountll(__builtin_amdgcn_ballot_w64(down == 0));
+                if (static_cast<uint32_t>(down - 1) < static_cast<uint32_t>(span - 1)) add(bins[0], down >> shift, 1);
+            }
+            if (lane == 0 && tops_here > 0) add(bins[0], 0, tops_here);
         }
-        __syncthreads();
-        const uint4 a = *reinterpret_cast<const uint4*>(&bins[8 * lane]), b = *reinterpret_cast<const uint4*>(&bins[8 * lane + 4]);
-        const uint32_t pairs = a.x + a.y + a.z + a.w + b.x + b.y + b.z + b.w;
-        const int mine = static_cast<int>((pairs & 0xffffu) + (pairs >> 16));
-        const int upto = scan_lanes(mine) + above;
-        const int at = __builtin_ctzll(__builtin_amdgcn_ballot_w64(upto >= k_sel) | 1ull << 63);
-        const int fine = lane < 16 ? static_cast<int>(reinterpret_cast<const uint16_t*>(bins)[16 * at + lane]) : 0;
-        const int fine_upto = scan_lanes(fine) + static_cast<int>(__builtin_amdgcn_readlane(upto - mine, at));
-        const int in = __builtin_ctzll(__builtin_amdgcn_ballot_w64(fine_upto >= k_sel) | 1ull << 63) & 15;
-        thr = top - (16 * at + in);
-        if (16 * at + in < 1023) break;
-        limit = thr;                                           // further down than the histogram goes: again from there
-        __syncthreads();
-        bins[tid] = 0u;
+        if (!find(bins[0])) {
+            top -= kTopkBins << shift;
+            shift = 6;
+#pragma unroll
+            for (int e = 0; e < kItems; ++e) {
+                const int down = top - key[e];
+                add_together(bins[1], static_cast<uint32_t>(down) < static_cast<uint32_t>(top) ? down >> shift : -1);
+            }
+            find(bins[1]);
+        }
+        thr = top - (bin << shift);
+        if (shift > 0) {                                       // uniform over the workgroup
+            const int span = min(1 << shift, thr);
+#pragma unroll
+            for (int e = 0; e < kItems; ++e) {
+                const int down = thr - key[e];
+                add_together(fine_bins, static_cast<uint32_t>(down) < static_cast<uint32_t>(span) ? down : -1);
+            }
+            __syncthreads();
+            const int upto = scan_lanes(reinterpret_cast<const uint16_t*>(fine_bins)[lane]) + above;
+            thr -= __builtin_ctzll(__builtin_amdgcn_ballot_w64(upto >= k_sel));
+        }
     }
     if (p.drop_neg_inf && thr <= static_cast<int>(p.neg_inf_key)) thr = p.neg_inf_key;                 // scores above -inf only: none of those equal to thr
     const bool no_equal = p.drop_neg_inf && thr == static_cast<int>(p.neg_inf_key);
@@ -531,6 +578,7 @@ static int topk_dispatch(void* stream, const uint16_t* x, int64_t row_stride, in
     p.x = x; p.row_stride = row_stride; p.out_idx = idx; p.out_val = val; p.out_mask = mask;
     p.out_stride = out_stride; p.n64 = n64; p.rows = rows; p.n = n; p.k = k;
     p.by_index = by_index; p.drop_neg_inf = drop_neg_inf; p.neg_inf_key = dtype == 0 ? kKeyNegInfFp16 : kKeyNegInfBf16;
+    p.first_shift = dtype == 0 ? 3 : 0;                        // eight powers of two, whatever the type
     if (rows <= wide_rows(n)) {
         if (n <= 512) return launch_topk_wide<1>(stream, p);
         if (n <= 1024) return launch_topk_wide<2>(stream, p);
