@@ -556,12 +556,22 @@ static int launch_topk(void* stream, const TopkParams& p) {
     return 0;
 }
 
-// Up to how many rows of n columns a workgroup per row is the faster one.  us by wavefronts | by workgroups, a list of 64 wanted: 400 columns, 768 rows 5.1 | 4.6,
-// 1024 5.1 | 4.7, 2048 5.9 | 7.7 (of 512, a wavefront's registers full, 4.7 | 4.4, 4.7 | 4.8, 5.5 | 7.7); 900, 1024 rows 7.4 | 5.4, 2048 8.6 | 8.9; 1500, 2048 rows 14.7 | 10.9,
-// 4096 25.4 | 19.9, 8192 40.7 | 36.9 (of 2048 13.1 | 11.0, 18.9 | 20.2, 33.1 | 37.9); 3000, 16 384 rows 249 | 104, 65 536 763 | 406 (of 4096 136 | 106, 429 | 421, mask words
-// alone 93 | 95, 283 | 376); 8192, 2048 rows 80 | 28, 65 536 1500 | 768.  Up to 256 columns both take what a launch takes (4.3).
-static int64_t wide_rows(int n) {
-    return n <= 256 ? 0 : n <= 512 ? 768 : n <= 1024 ? 1024 : n <= 2048 ? 2048 : n <= 4096 ? 16384 : INT64_MAX;
+// Up to how many rows of n columns a workgroup per row is the faster one.  us by wavefronts | by workgroups, a list of 64 wanted in ascending columns; bfloat16 scores within a
+// few powers of two, and IEEE half spread over thirty, the dearest rows for a workgroup:
+//   400 columns, 512 rows 4.6 | 3.6, 4.5 | 4.2; 768 rows 4.6 | 4.4, 4.7 | 4.9            512: 512 rows 4.4 | 3.6, 4.4 | 4.3
+//   700, 1024 rows 7.1 | 5.3, 7.2 | 6.5; 1536 8.1 | 7.0, 8.0 | 8.8                       1024: 768 rows 6.7 | 4.7, 6.7 | 5.9; 1024 rows 6.7 | 5.3, 6.6 | 6.9
+//   1500, 2048 rows 13.8 | 10.8, 13.7 | 13.9; 4096 24.8 | 19.3, 22.9 | 24.9              2048: 1536 rows 12.9 | 9.0, 12.3 | 12.0; 2048 rows 12.8 | 11.1, 12.5 | 14.7
+//   3000, 16 384 rows 255 | 104, 304 | 130; 131 072 1466 | 825, 2085 | 1009              4096: 16 384 rows 139 | 106, 163 | 134; 65 536 434 | 428, and 440 | 510 where half is -inf
+// A row that fills a wavefront's registers (the right-hand ones) costs it less, and mask words alone cost it less too: 3000 columns, 16 384 rows 133 | 93, 157 | 120; 65 536
+// 395 | 364, and 398 | 463 where most is -inf; 4096 columns, 4096 rows 37 | 26, 35 | 35; 8192 rows 59 | 50, 54 | 65.  Up to 256 columns both take what a launch takes.
+static int64_t wide_rows(int n, bool list) {
+    const bool full = n == 512 || n == 1024 || n == 2048 || n == 4096;
+    if (n <= 256) return 0;
+    if (n <= 512) return 512;
+    if (n <= 1024) return full ? 768 : 1024;
+    if (n <= 2048) return full ? 1536 : 2048;
+    if (n <= 4096) return full ? (list ? 16384 : 4096) : (list ? INT64_MAX : 16384);
+    return INT64_MAX;                                          // more than a wavefront's registers hold
 }
 
 static int topk_dispatch(void* stream, const uint16_t* x, int64_t row_stride, int32_t* idx, uint16_t* val,
@@ -579,7 +589,7 @@ static int topk_dispatch(void* stream, const uint16_t* x, int64_t row_stride, in
     p.out_stride = out_stride; p.n64 = n64; p.rows = rows; p.n = n; p.k = k;
     p.by_index = by_index; p.drop_neg_inf = drop_neg_inf; p.neg_inf_key = dtype == 0 ? kKeyNegInfFp16 : kKeyNegInfBf16;
     p.first_shift = dtype == 0 ? 3 : 0;                        // eight powers of two, whatever the type
-    if (rows <= wide_rows(n)) {
+    if (rows <= wide_rows(n, idx != nullptr)) {
         if (n <= 512) return launch_topk_wide<1>(stream, p);
         if (n <= 1024) return launch_topk_wide<2>(stream, p);
         if (n <= 2048) return launch_topk_wide<4>(stream, p);

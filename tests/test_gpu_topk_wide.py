@@ -67,11 +67,25 @@ def test_few_rows(n, kind):
         check(rows_of(kind, 5, n, gen), k)
 
 
-@pytest.mark.parametrize("rows, n", [(768, 400), (769, 400), (1024, 700), (1025, 700), (2048, 1100), (2049, 1100), (16384, 2100), (16385, 2100)])
+@pytest.mark.parametrize("rows, n", [(768, 400), (769, 400), (1024, 700), (1025, 700), (2048, 1100), (2049, 1100), (16384, 2100), (16385, 2100),
+                                     (512, 400), (513, 400), (768, 1024), (769, 1024), (1536, 2048), (1537, 2048), (16384, 4096), (16385, 4096)])
 def test_both_sides_of_the_rule(rows, n):
     gen = torch.Generator(device="cuda").manual_seed(rows)
     for kind in ("scores", "inf"):
         check(rows_of(kind, rows, n, gen), 32)
+
+
+@pytest.mark.parametrize("rows, n", [(16384, 2100), (16385, 2100), (4096, 4096), (4097, 4096)])
+def test_both_sides_of_the_rule_for_words_alone(rows, n):
+    """The words without a list against those with it, which another kernel makes on one side."""
+    from infllmv2_cuda_impl_amd import _lib
+    x = rows_of("spread", rows, n, torch.Generator(device="cuda").manual_seed(rows), torch.float16)
+    n64, stream = (n + 63) // 64, torch.cuda.current_stream().cuda_stream
+    idx = torch.empty(rows, 48, dtype=torch.int32, device="cuda")
+    want, got = torch.empty(2, rows, n64, dtype=torch.int64, device="cuda").unbind(0)
+    _lib.call("infllmv2_topk_select", stream, x.data_ptr(), n, 0, idx.data_ptr(), want.data_ptr(), rows, n, 48, n64, 1, 0)
+    _lib.call("infllmv2_topk_mask", stream, x.data_ptr(), n, 0, got.data_ptr(), rows, n, 48, n64, 0)
+    assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("drop", [0, 1])
