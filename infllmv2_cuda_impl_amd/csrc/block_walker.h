@@ -43,17 +43,27 @@ struct BlockWalker {
 };
 
 // A word of the mask rows of a group of up to eight tokens, `pitch` words apart: the blocks that the group walks together, which is those that five or
-// more of eight rows select, or all rows of a smaller group.  The row-parallel kernels say what that measured.
+// more of eight rows select, or all rows of a smaller group.  The row-parallel kernels say what that measured.  Rows that are all alike, as under a window or without a
+// mask, have nothing from it and are found first: the count is 50 vector instructions of one wavefront for which the others wait.  Forward in us, blocks of all eight
+// rows | counted | counted where rows differ: 30 000 tokens, 2 KV heads, groups of 8, 34 blocks 1110 | 1126 | 1109; 2000, 33 blocks 60.7 | 61.5 | 60.7; 30 x 600,
+// 7 blocks 197.4 | 196.5 | 194.3; without a mask 3800, one KV head 83.9 | 85.2 | 84.1.
 __device__ __forceinline__ uint64_t walked_together(const unsigned long long* words, int pitch, int tokens) {
+    if (tokens < 8) {
+        uint64_t all = words[0];
+        for (int t = 1; t < tokens; ++t) all &= words[t * pitch];
+        return all;
+    }
     // how many of the rows select a block, a binary digit to a word
     uint64_t r[8];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) r[t] = t < tokens ? words[t * pitch] : ~0ull;
+    for (int t = 0; t < 8; ++t) r[t] = words[t * pitch];
+    const uint64_t all = r[0] & r[1] & r[2] & r[3] & r[4] & r[5] & r[6] & r[7], any = r[0] | r[1] | r[2] | r[3] | r[4] | r[5] | r[6] | r[7];
+    if (__builtin_amdgcn_ballot_w64(all != any) == 0ull) return all;
     auto sum3 = [](uint64_t a, uint64_t b, uint64_t c, uint64_t& carry) { carry = (a & b) | (c & (a | b)); return a ^ b ^ c; };
     uint64_t t0, t1, t2, f0;
     const uint64_t s0 = sum3(r[0], r[1], r[2], t0), s1 = sum3(r[3], r[4], r[5], t1), s2 = sum3(r[6], r[7], s0, t2);
     const uint64_t ones = s1 ^ s2, t3 = s1 & s2, u = sum3(t0, t1, t2, f0), twos = u ^ t3, f1 = u & t3, fours = f0 ^ f1, eights = f0 & f1;
-    return tokens < 8 ? eights : eights | (fours & (twos | ones));
+    return eights | (fours & (twos | ones));
 }
 
 // Cross-row exchanges with gfx950's v_permlane16_swap / v_permlane32_swap (VALU speed; a ds_bpermute takes a trip
