@@ -42,6 +42,22 @@ struct BlockWalker {
     }
 };
 
+// The word after `at` (at first -1) that is not zero, for a walk over words in LDS, or `words`; `filled` (at first 0) is the walk's.  For long rows: words without
+// blocks are passed over 64 at a time.  One by one, a trip to LDS each, they took 0.03 us a word of a group's set-up (window of 6 blocks in 60 000 tokens, 15 words: 422 -> 410 us).
+template <typename Word>
+__device__ __forceinline__ int next_filled_word(int at, int words, uint64_t& filled, Word word) {
+    int from = at & ~63;
+    while (filled == 0ull) {
+        from += 64;
+        if (from >= words) return words;
+        const int w = from + static_cast<int>(__lane_id());
+        filled = __builtin_amdgcn_ballot_w64(w < words && word(w) != 0ull);
+    }
+    const int w = from + __builtin_ctzll(filled);
+    filled &= filled - 1ull;
+    return w;
+}
+
 // A word of the mask rows of a group of up to eight tokens, `pitch` words apart: the blocks that the group walks together, which is those that five or
 // more of eight rows select, or all rows of a smaller group.  The row-parallel kernels say what that measured.  Rows that are all alike, as under a window or without a
 // mask, have nothing from it and are found first: the count is 50 vector instructions of one wavefront for which the others wait.  Forward in us, blocks of all eight

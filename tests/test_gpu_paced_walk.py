@@ -12,6 +12,8 @@ CASES = [  # keys, queries, group, window blocks, blocks anywhere, blocks near t
     (70011, 64, 8, 31, 0, 70),                                 # all own blocks behind where the front is for most of the walk: more than there are steps
     (48000, 24, 16, 0, 20, 0),                                 # only the first block in common
     (48000, 24, 16, -1, 20, 0),                                # nothing in common: no clock
+    (300011, 20, 16, 2, 0, 40),                                # 74 mask words, most of them empty
+    (300011, 20, 16, -1, 30, 0),
 ]
 
 
