@@ -300,7 +300,7 @@ Tensor stage1_selected(const Tensor& q, const Tensor& k_, const Tensor& v_, cons
     auto fn = is_half(q) ? infllmv2_varlen_fwd_stage1_selected_f16 : infllmv2_varlen_fwd_stage1_selected;
     check_rc(fn(stream_of(q), ptr(q), ptr(k), ptr(v), static_cast<uint64_t*>(mask.data_ptr()), iptr(cu_q), iptr(cu_k), iptr(cu_v), as_int(batch), total_q,
                 as_int(hq), as_int(hk), as_int(q.size(2)), as_int(max_q), as_int(max_k), qs.v, ks.v, vs.v, as_int(out_len), static_cast<float>(scale),
-                per + 1, per, 1, as_int(block_size), as_int(local_blocks), as_int(init_blocks), as_int(topk), as_int(n64)), "varlen_fwd_stage1_pooled");
+                per + 1, per, 1, as_int(block_size), as_int(local_blocks), as_int(init_blocks), as_int(topk), as_int(n64)), "varlen_fwd_stage1_selected");
     return mask;
 }
 

@@ -634,16 +634,17 @@ extern "C" int IV2_ENTRY(infllmv2_varlen_fwd_stage1_selected)(void* stream, cons
                                                    int out_len, float softmax_scale, int kernel_size, int stride, int padding,
                                                    int block_size, int local_blocks, int init_blocks, int topk, int n_uint64_per_row) {
     IV2_CHECK(kernel_size == 5 && stride == 4 && padding == 1 && block_size == kBlockN,
-              "varlen_fwd_stage1_pooled: only the 5/4/1 window on 64-token blocks is fused (got %d/%d/%d on %d); "
-              "use varlen_fwd_stage1 and max_pooling_1d", kernel_size, stride, padding, block_size);
+              "varlen_fwd_stage1_selected: only the 5/4/1 window on 64-token blocks is fused (got %d/%d/%d on %d); "
+              "use varlen_fwd_stage1, max_pooling_1d and topk_mask", kernel_size, stride, padding, block_size);
     IV2_CHECK(out_len > 0 && out_len <= INFLLMV2_STAGE1_SELECT_BLOCKS, "varlen_fwd_stage1_selected: 1 to %d blocks (got %d)",
               INFLLMV2_STAGE1_SELECT_BLOCKS, out_len);
     IV2_CHECK(topk >= 0, "topk: negative size");
     IV2_CHECK(topk <= 2048, "topk: k %d exceeds 2048", topk);
-    IV2_CHECK(mask != nullptr && n_uint64_per_row > 0 && static_cast<int64_t>(n_uint64_per_row) * 64 >= out_len,
+    IV2_CHECK(mask != nullptr, "varlen_fwd_stage1_selected: null pointer");
+    IV2_CHECK(n_uint64_per_row > 0 && static_cast<int64_t>(n_uint64_per_row) * 64 >= out_len,
               "topk: %d mask words per row cannot hold %d columns", n_uint64_per_row, out_len);
     const Stage1Pool pool{nullptr, 0, out_len, local_blocks, init_blocks, mask, n_uint64_per_row, topk};
-    return launch_stage1("varlen_fwd_stage1_pooled", stream, q, k, v, nullptr, cu_seqlens_q, cu_seqlens_k, cu_seqlens_v,
+    return launch_stage1("varlen_fwd_stage1_selected", stream, q, k, v, nullptr, cu_seqlens_q, cu_seqlens_k, cu_seqlens_v,
                          batch, total_q, num_heads, num_heads_k, head_dim, max_seqlen_q, max_seqlen_k, q_strides,
                          k_strides, v_strides, 0, 0, softmax_scale, 1, &pool);
 }

@@ -137,3 +137,17 @@ def test_ctypes_signatures_have_the_headers_parameter_counts():
         assert got == want, (name, "".join(got), "".join(want))
         checked += 1
     assert checked >= 10
+
+
+def test_selecting_stage1_names_itself_in_its_errors():
+    from infllmv2_cuda_impl_amd import _lib
+    lib, i64, fake = _lib.lib, _lib.i64_array, 0x1000
+
+    def call(mask=fake, heads=32, kernel=5, out_len=2, topk=4, words=1):
+        return lib.infllmv2_varlen_fwd_stage1_selected(None, fake, fake, fake, mask, fake, fake, fake, 1, 128, heads, 2, 128, 128, 7, i64([4096, 128, 2048]),
+                                                       i64([256, 128]), i64([256, 128]), out_len, 0.088, kernel, 4, 1, 64, 1, 1, topk, words)
+    for wrong, text in ((dict(kernel=9), "only the 5/4/1 window"), (dict(out_len=513), "1 to 512 blocks"), (dict(mask=None), "null pointer"),
+                        (dict(heads=24), "g * num_heads_k")):
+        assert call(**wrong) != 0 and text in _err(lib) and _err(lib).startswith("varlen_fwd_stage1_selected"), (wrong, _err(lib))
+    assert call(topk=2049) != 0 and "exceeds 2048" in _err(lib)
+    assert call(out_len=65) != 0 and "cannot hold" in _err(lib)
