@@ -296,7 +296,10 @@ int infllmv2_varlen_fwd_masked_tiles(int batch, int64_t total_q, int64_t total_k
  *   the reference's (Hk, T*16) layout (flash_api.cpp:665) is {16, 1, T*16}.
  * blockmask (Hk, total_q, n_uint64_per_row): block indices local to each sequence, rows by packed
  *   token index (flash_blockmask.h:20-31).
- * workspace: infllmv2_kv_image_bytes() bytes, 16-byte aligned; filled here unless kv_prepacked. */
+ * workspace: infllmv2_kv_image_bytes() bytes, 16-byte aligned; filled here unless kv_prepacked.
+ * Where max_seqlen_k exceeds INFLLMV2_IN_STEP_KEYS and there is a blockmask, the call that fills the workspace also has its workgroups start together, so that they
+ * find each other's blocks in L2; with kv_prepacked it cannot (several launches may read the images at once): results are the same, long sequences take longer. */
+#define INFLLMV2_IN_STEP_KEYS 32768
 int infllmv2_varlen_fwd(void* stream, const void* q, const void* k, const void* v, void* out,
                         float* softmax_lse, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
                         const uint64_t* blockmask, void* workspace, size_t workspace_bytes,

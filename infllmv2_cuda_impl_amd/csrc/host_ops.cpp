@@ -164,9 +164,9 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> compress_keys_pair(const Tensor& k, c
 // are still in the 256 MB behind the L2s when the scores have read q.  Packed just before the walk, they are there in any case: with 64 blocks
 // selected and 2 KV heads of 16 query heads, packing early gains 3 us of a whole prefill at 512 and 2048 tokens, 7 at 12 288 and 16 384 (128 MiB of q) and
 // nothing at 20 480 to 28 672, and at 32 768 the walk is 1 to 3 % slower for it (2.81 -> 2.87 ms).
-constexpr int64_t kPackEarlyBytes = 128ll << 20, kInStepKeys = 32768;
+constexpr int64_t kPackEarlyBytes = 128ll << 20;
 bool pack_early(const Tensor& q, const Tensor& k, const Tensor& v, int64_t max_seqlen_k) {
-    if (q.numel() * q.element_size() > kPackEarlyBytes || max_seqlen_k > kInStepKeys) return false;
+    if (q.numel() * q.element_size() > kPackEarlyBytes || max_seqlen_k > INFLLMV2_IN_STEP_KEYS) return false;
     const auto fits = [](const Tensor& t) {
         return t.stride(2) == 1 && t.stride(0) % 8 == 0 && t.stride(1) % 8 == 0 && reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0;
     };
@@ -536,7 +536,7 @@ std::tuple<Tensor, Tensor, OptTensor> varlen_fwd(const Tensor& q, const Tensor& 
         TORCH_CHECK(topk_idx->dim() == 3 && topk_idx->size(0) == hk && topk_idx->size(1) == total_q,
                     "topk_idx must have shape (num_heads_k, total_q, k)");
         const int64_t k_blocks = (max_k + kBlock - 1) / kBlock, n64 = (k_blocks + 63) / 64;
-        if (max_k <= kInStepKeys && total_q > 0 && max_q > 0 && !images.has_value()) {
+        if (max_k <= INFLLMV2_IN_STEP_KEYS && total_q > 0 && max_q > 0 && !images.has_value()) {
             // The mask words are made by the launch that packs k and v (2049 queries behind 17 962 keys, from the compressed keys on, 325.2 -> 323.4 us, 512 behind each of three
             // prompts 219.6 -> 217.2, 2000 tokens 85.4 -> 83.9).  Not for sequences that are
             // walked in step: the packing clears the counters of the one launch behind it, and is then part of that call.

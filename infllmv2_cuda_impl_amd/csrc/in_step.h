@@ -33,11 +33,12 @@
 // of its time at 40 000 tokens and gained nothing at 64 000.
 #pragma once
 #include "common.h"
+#include "infllmv2_hip.h"
 
 namespace IV2_NS {
 
 constexpr int kGeneration = 32;
-constexpr int kInStepKeys = 32768;                             // sequences with more keys than this
+constexpr int kInStepKeys = INFLLMV2_IN_STEP_KEYS;             // sequences with more keys than this: 32 768
 constexpr int kInStepWords = 4;                                // and rows with blocks of their own in at least so many mask words
 constexpr int kPacedBlocks = kInStepKeys / kBlockN;            // groups that reach beyond so many blocks are paced, in every launch that can hold such a group
 constexpr int kPacedSteps = 2;
