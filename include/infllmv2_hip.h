@@ -151,7 +151,8 @@ int infllmv2_compress_keys_pair(void* stream, const void* k, void* out_a, void* 
                                 int num_heads_k, int head_dim, int64_t k_row_stride, int64_t k_head_stride,
                                 int kernel_size_a, int stride_a, int kernel_size_b, int stride_b);
 
-/* infllmv2_compress_keys_pair and infllmv2_pack_kv (below) in one launch: what prefill needs of k and v before its first scores.
+/* infllmv2_compress_keys_pair and infllmv2_pack_kv (below) in one launch: what prefill needs of k and v before its first scores, for sequences of up to
+ * INFLLMV2_IN_STEP_KEYS keys (longer ones are better packed by the forward itself).
  * k_strides, v_strides {row, head}; head_dim 128; workspace: infllmv2_kv_image_bytes() bytes, 16-byte aligned. */
 int infllmv2_compress_keys_and_pack(void* stream, const void* k, const void* v, void* out_a, void* out_b, const int32_t* cu_seqlens_k,
                                     int32_t* cu_seqlens_out_a, int32_t* cu_seqlens_out_b, void* workspace, size_t workspace_bytes,

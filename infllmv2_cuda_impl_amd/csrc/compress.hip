@@ -74,7 +74,9 @@ __device__ __forceinline__ void compress_rows_of_head(const CompressParams& p, i
     for (int base = 0; base < span; base += step) {
         const int staged = span - base < step ? span - base : step;
         if (base > 0) __syncthreads();
-        uint4 piece[kCompressPieces];                          // all of them requested before the first is waited for
+        // All of them are requested before the first is waited for.  A set on its own, us, four at a time before: 32 keys every 16 of 2048 tokens 4.11 -> 4.03, of 131 072
+        // 15.8 -> 15.2; 128 every 64 4.80 -> 4.88, 21.3 -> 19.7; both in one launch, 2048 tokens, 0.35 less.
+        uint4 piece[kCompressPieces];
 #pragma unroll
         for (int t = 0; t < kCompressPieces; ++t) {
             const int it = tid + t * kCompressThreads, i = it / kCompressUnits, u = it % kCompressUnits;

@@ -18,6 +18,11 @@
 // and with it the result's bits, are the same in every launch.  131 072 tokens, 64 blocks: L2 serves 80 % of the requests instead of 57, 60 GB come from behind it instead of 125,
 // forward 19.4 -> 14.1 ms, whole prefill 26.0 -> 20.9; 65 536: 8.8 -> 7.95; 40 000: 4.5 -> 4.4.  One step to a common block 24.9, 8.6, 4.5, three 20.9, 8.0, 4.4.
 // Groups that end behind block 384: 20.8, 7.9, 4.4; 768: 21.2, 8.2, 4.6.  Below 32 768 keys, waiting and paced or not: within 1 % either way.
+// That is with a row's own blocks anywhere.  Forward in ms, in step | paced too (and five of eight rows in the ring), a window of 32 blocks and 32 blocks that lie, 131 072 tokens with
+// one KV head; 65 536 with two: anywhere 9.5 | 6.7; 6.5 | 5.8.  In four runs of eight 13.0 | 10.3; 9.5 | 7.4.  In one run 15.1 | 15.2; 11.3 | 11.2.  Half of them anywhere, half the same
+// for 64 tokens 7.0 | 5.8; 5.8 | 5.3.  Within one block of the same for 8 tokens 6.13 | 6.08; 5.58 | 5.61, for 64 5.58 | 5.71; 5.36 | 5.40, for 512 5.55 | 5.60; 5.29 | 5.33.  In the first
+// tenth 5.29 | 5.23; 4.72 | 4.60, in the 64 blocks before the window 5.18 | 5.17; 5.04 | 5.04, between 80 and 95 % of the way 5.27 | 5.40; 4.62 | 4.68: where L2 has the blocks
+// anyway the pace costs up to 2 %, where it has not it gives up to 30.
 //
 // With the device shared a generation is more than an XCD runs at once, and CUs that become free wait for its second half.  What sharing fetches gives is still
 // more than that costs; forward in ms, in step and paced | in step | neither, 2 KV heads, 64 blocks selected (the first, a window of 32, the rest anywhere), as many as keep both

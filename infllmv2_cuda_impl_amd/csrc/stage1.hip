@@ -20,8 +20,9 @@
 // by all 16 tokens, and inside a wavefront one operand read feeds two MFMAs.
 //
 // Bound by vector instructions (the vector pipe was 80 % busy, the matrix pipe 42 %) and by power: what is saved in instructions is half lost to a lower
-// clock.  Tiles without a test, offsets in scalar registers, DPP maxima spelled out and results stored a tile later took them from 163 to 126 per 64
-// fine keys and two tokens; pooled, two KV heads, us: 131 072 tokens 5800 -> 5580, 32 768 428 -> 415, 9173 62 -> 60; 2049 queries against 20 011 keys 60.3 -> 58.5.
+// clock.  Tiles without a test, offsets in scalar registers, DPP maxima spelled out and results stored a tile later took them from 202 to 184 per 64
+// fine keys, 16 coarse ones and two tokens (counted, beside 40 MFMAs); pooled, two KV heads, us: 131 072 tokens 5800 -> 5580, 32 768 428 -> 415, 9173 62 -> 60; 2049 queries against 20 011
+// keys 60.3 -> 58.5.  Launches of one or two tiles pay 0.1 to 0.25 us for the set-up (500 tokens, scores 7.9 -> 8.0, pooled 8.2 -> 8.45).
 // With 32-row MFMAs and plain sums in pass 1: 5470, 407, 59, 54, but sums in another order round some scores to the neighbouring 16-bit value, and
 // single rows then attend another block.
 #include "common.h"

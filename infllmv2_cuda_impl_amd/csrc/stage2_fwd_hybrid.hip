@@ -475,7 +475,8 @@ int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int 
     // tokens behind 20011 88 -> 51 (two 60), 256 of 3000 52 -> 41; eight: 64 behind 20011 95 -> 50 (four 54), 8 each of 8 sequences with 9000 keys
     // 101 -> 55 (four 64).  Parts by columns of V, which repeat the products with K: 70 for the four and the eight, 76 for the two.  More workgroups than CUs run in two rounds
     // and gain nothing: 700 tokens behind 20011, 176 groups, take 102 whole.
-    // So few groups run all at once and need no pace: they neither count nor wait (in_step.h).
+    // So few groups run all at once: they neither count nor wait (in_step.h).  They keep the pace: it gives the order in which a row's blocks are added up, which must not
+    // depend on the number of parts.
     const int parts = total * 2 > 256 ? 1 : total * 4 > 256 ? 2 : total * 8 > 256 ? 4 : 8;
     x.finished = parts > 1 ? nullptr : in_step;
     auto pick = [&](auto n) {
