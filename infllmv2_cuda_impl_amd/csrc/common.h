@@ -68,6 +68,9 @@ inline bool valid_group(int num_heads, int num_heads_k) {
         }                                                                         \
     } while (0)
 
+// A dispatch holds fewer than 2^32 work-items in a dimension, and the runtime reports no error for more: it starts too few workgroups.
+constexpr int64_t max_workgroups(int threads) { return 0xffffffffll / threads; }
+
 __device__ __forceinline__ float bf16_to_f32(bf16_bits b) {
     return __uint_as_float(static_cast<uint32_t>(b) << 16);
 }

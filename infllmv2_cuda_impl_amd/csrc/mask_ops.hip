@@ -89,12 +89,14 @@ extern "C" int infllmv2_topk_to_uint64(void* stream, const int32_t* topk_idx, ui
     (void)k_blocks;
     if (rows == 0 || n_uint64_per_row == 0) return 0;
     constexpr int kWaves = 4;
-    const int64_t blocks = (rows + kWaves - 1) / kWaves;
-    IV2_CHECK(blocks <= 0x7fffffffll, "topk_to_uint64: too many rows");
     const size_t lds = sizeof(uint64_t) * kWaves * n_uint64_per_row;
-    hipLaunchKernelGGL(topk_to_uint64_kernel<kWaves>, dim3(static_cast<unsigned>(blocks)), dim3(kWaves * 64), lds,
-                       static_cast<hipStream_t>(stream), topk_idx, result, rows, k, n_uint64_per_row);
-    IV2_LAUNCH_CHECK();
+    const int64_t part = max_workgroups(kWaves * 64) * kWaves;
+    for (int64_t first = 0; first < rows; first += part) {
+        const int64_t here = rows - first < part ? rows - first : part;
+        hipLaunchKernelGGL(topk_to_uint64_kernel<kWaves>, dim3(static_cast<unsigned>((here + kWaves - 1) / kWaves)), dim3(kWaves * 64), lds,
+                           static_cast<hipStream_t>(stream), topk_idx + first * k, result + first * n_uint64_per_row, here, k, n_uint64_per_row);
+        IV2_LAUNCH_CHECK();
+    }
     return 0;
 }
 
@@ -105,14 +107,14 @@ extern "C" int infllmv2_uint64_to_bool(void* stream, const uint64_t* input, uint
               "uint64_to_bool: %d words cannot hold %d bits", n_uint64_per_row, last_dim_size);
     if (rows == 0 || last_dim_size == 0) return 0;
     const int groups = (last_dim_size + 7) / 8;
-    const int64_t total = rows * groups;
-    const int64_t blocks = (total + 255) / 256;
-    IV2_CHECK(blocks <= 0x7fffffffll, "uint64_to_bool: too many elements");
     const bool aligned = (last_dim_size % 8 == 0) && (reinterpret_cast<uintptr_t>(result) % 8 == 0);
-    hipLaunchKernelGGL(uint64_to_bool_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), input, result, rows, last_dim_size,
-                       n_uint64_per_row, groups, aligned);
-    IV2_LAUNCH_CHECK();
+    const int64_t part = max_workgroups(256) * 256 / groups;
+    for (int64_t first = 0; first < rows; first += part) {
+        const int64_t here = rows - first < part ? rows - first : part;
+        hipLaunchKernelGGL(uint64_to_bool_kernel, dim3(static_cast<unsigned>((here * groups + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream),
+                           input + first * n_uint64_per_row, result + first * last_dim_size, here, last_dim_size, n_uint64_per_row, groups, aligned);
+        IV2_LAUNCH_CHECK();
+    }
     return 0;
 }
 
@@ -121,13 +123,15 @@ extern "C" int infllmv2_blockmask_to_uint64(void* stream, const uint8_t* blockma
     IV2_CHECK(rows >= 0 && last_dim_size >= 0, "blockmask_to_uint64: negative size");
     IV2_CHECK(n_uint64_per_row == (last_dim_size + 63) / 64,
               "blockmask_to_uint64: n_uint64_per_row %d does not match last dim %d", n_uint64_per_row, last_dim_size);
-    const int64_t words = rows * n_uint64_per_row;
-    if (words == 0) return 0;
-    const int64_t blocks = (words + 3) / 4;
-    IV2_CHECK(blocks <= 0x7fffffffll, "blockmask_to_uint64: too many elements");
-    hipLaunchKernelGGL(blockmask_to_uint64_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
-                       static_cast<hipStream_t>(stream), blockmask, result, rows, last_dim_size, n_uint64_per_row);
-    IV2_LAUNCH_CHECK();
+    if (rows == 0 || n_uint64_per_row == 0) return 0;
+    const int64_t part = max_workgroups(256) * 4 / n_uint64_per_row;
+    for (int64_t first = 0; first < rows; first += part) {
+        const int64_t here = rows - first < part ? rows - first : part;
+        hipLaunchKernelGGL(blockmask_to_uint64_kernel, dim3(static_cast<unsigned>((here * n_uint64_per_row + 3) / 4)), dim3(256), 0,
+                           static_cast<hipStream_t>(stream), blockmask + first * last_dim_size, result + first * n_uint64_per_row, here, last_dim_size,
+                           n_uint64_per_row);
+        IV2_LAUNCH_CHECK();
+    }
     return 0;
 }
 
@@ -139,7 +143,7 @@ extern "C" int infllmv2_transpose_blockmask(void* stream, const uint64_t* fwd_ma
     const int64_t tiles = static_cast<int64_t>(heads) * n64_bwd * n64_fwd;
     if (tiles == 0 || k_blocks == 0) return 0;
     const int64_t blocks = (tiles + 3) / 4;
-    IV2_CHECK(blocks <= 0x7fffffffll, "transpose_blockmask: too many tiles");
+    IV2_CHECK(blocks <= max_workgroups(256), "transpose_blockmask: too many tiles");
     hipLaunchKernelGGL(transpose_blockmask_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
                        static_cast<hipStream_t>(stream), fwd_mask, bwd_mask, heads, total_q, n64_fwd, k_blocks, n64_bwd);
     IV2_LAUNCH_CHECK();

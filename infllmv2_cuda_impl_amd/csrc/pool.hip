@@ -221,7 +221,7 @@ static int launch_pool(void* stream, PoolParams& p) {
         constexpr int kWaves = 4;
         const int rows_per_wave = total_rows >= 64 * 1024 ? 4 : 1;
         const int64_t blocks = (total_rows + kWaves * rows_per_wave - 1) / (kWaves * rows_per_wave);
-        IV2_CHECK(blocks <= 0x7fffffffll, "max_pooling_1d: too many rows");
+        IV2_CHECK(blocks <= max_workgroups(kWaves * 64), "max_pooling_1d: too many rows");
         hipLaunchKernelGGL(max_pooling_1d_rows_kernel<kWaves>, dim3(static_cast<unsigned>(blocks)), dim3(kWaves * 64),
                            kWaves * slice_bytes, st, p, units, rows_per_wave);
         IV2_LAUNCH_CHECK();

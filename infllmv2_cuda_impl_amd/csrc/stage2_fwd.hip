@@ -109,7 +109,7 @@ extern "C" int infllmv2_pack_kv_and_topk(void* stream, const void* k, const void
     const int64_t pairs = static_cast<int64_t>(batch) * num_heads_k;
     const int64_t mask_wgs = n_uint64_per_row == 0 ? 0 : ((rows + kMaskRowsPerWg - 1) / kMaskRowsPerWg + pairs - 1) / pairs;
     if (blocks + mask_wgs == 0) return 0;
-    IV2_CHECK(blocks + mask_wgs <= 0x7fffffffll, "pack_kv_and_topk: too many rows");
+    IV2_CHECK(blocks + mask_wgs <= max_workgroups(256), "pack_kv_and_topk: too many rows");
     const PackParams pp = pack_params(k, v, cu_seqlens_k, workspace, batch, total_k, num_heads_k, k_strides, v_strides, nullptr);
     size_t lds = sizeof(uint64_t) * kMaskRowsPerWg * n_uint64_per_row;
     if (lds < kPackElems * sizeof(elem_bits)) lds = kPackElems * sizeof(elem_bits);

@@ -512,8 +512,8 @@ void topk_wide_kernel(const TopkParams p) {
     }
 }
 
-// A dispatch holds fewer than 2^32 work-items in a dimension: 8 388 607 workgroups.
-constexpr int64_t kTopkWideChunk = 1 << 22;
+constexpr int64_t kTopkWideChunk = 1 << 22;                    // workgroups of a launch
+static_assert(kTopkWideChunk <= max_workgroups(kTopkRowWaves * 64), "more than a dispatch holds");
 
 template <int kItems>
 static int launch_topk_wide(void* stream, const TopkParams& p) {
@@ -535,7 +535,7 @@ template <int kItems>
 static int launch_topk(void* stream, const TopkParams& p) {
     const int64_t waves = (p.rows + p.rows_per_wave - 1) / p.rows_per_wave;
     const int64_t blocks = (waves + kTopkWaves - 1) / kTopkWaves;
-    IV2_CHECK(blocks <= 0x7fffffffll, "topk: too many rows");
+    IV2_CHECK(blocks <= max_workgroups(kTopkWaves * 64), "topk: too many rows");
     const size_t lds = sizeof(uint32_t) * kTopkWaves * (p.k + 64);
     const dim3 grid(static_cast<unsigned>(blocks)), block(kTopkWaves * 64);
     hipStream_t st = static_cast<hipStream_t>(stream);

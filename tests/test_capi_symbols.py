@@ -151,3 +151,12 @@ def test_selecting_stage1_names_itself_in_its_errors():
         assert call(**wrong) != 0 and text in _err(lib) and _err(lib).startswith("varlen_fwd_stage1_selected"), (wrong, _err(lib))
     assert call(topk=2049) != 0 and "exceeds 2048" in _err(lib)
     assert call(out_len=65) != 0 and "cannot hold" in _err(lib)
+
+
+def test_more_rows_than_a_dispatch_holds_are_refused():
+    """Fewer than 2^32 work-items in a dimension; the runtime would start too few workgroups for more, without an error."""
+    from infllmv2_cuda_impl_amd import _lib
+    lib, i64, fake = _lib.lib, _lib.i64_array, 0x1000
+    assert lib.infllmv2_topk_mask(None, fake, 32, 1, fake, 1 << 31, 32, 4, 1, 0) != 0 and "too many rows" in _err(lib)
+    assert lib.infllmv2_pack_kv_and_topk(None, fake, fake, fake, fake, 1 << 40, 1, 64, 1, 128, 64, i64([128, 128]), i64([128, 128]), fake, fake, 1 << 27, 4,
+                                         1) != 0 and "too many rows" in _err(lib)
