@@ -622,7 +622,7 @@ static int launch_bwd_dkdv_sliced(hipStream_t st, const BwdParams& p_in, int bat
     const int teams = 8 / p.dkdv_share;
     const int64_t rounds = static_cast<int64_t>((groups + teams - 1) / teams) * kGroupSlices;
     const int64_t items = 8 * rounds * ((p.k_blocks + p.dkdv_share - 1) / p.dkdv_share);
-    IV2_CHECK(items <= 0x7fffffffll, "varlen_bwd: too many (slice, block) work items");
+    IV2_CHECK(items <= max_workgroups(128), "varlen_bwd: too many (slice, block) work items");
     IV2_CHECK(p.q_tok >= 0 && p.q_tok < (1ll << 31) && p.do_tok >= 0 && p.do_tok < (1ll << 31) && p.total_q < (1ll << 31),
               "varlen_bwd: token strides of q and dout must lie in [0, 2^31) elements");
     const dim3 grid(static_cast<unsigned>(items), batch, p.num_heads_k);

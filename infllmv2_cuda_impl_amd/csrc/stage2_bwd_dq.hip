@@ -386,9 +386,22 @@ int launch_bwd_dq_hybrid(hipStream_t st, const BwdParams& p, int batch, int max_
     DqExtra x{};
     x.batch = batch;
     x.groups_per_seq = (max_seqlen_q + kDqTokens - 1) / kDqTokens;
-    const int64_t total = static_cast<int64_t>(p.num_heads_k) * batch * x.groups_per_seq;
-    IV2_CHECK(total <= 0x3fffffff, "varlen_bwd: too many token groups");
+    const int64_t of_sequence = static_cast<int64_t>(p.num_heads_k) * x.groups_per_seq, total = of_sequence * batch;
     IV2_CHECK(p.k_blocks <= kDqMaskWords * 64, "varlen_bwd: more than %d key blocks per sequence", kDqMaskWords * 64);
+    const int64_t most = max_workgroups(512) - 8 * kDqChunk;
+    if (total > most) {                                        // some sequences at a time, as in the forward
+        const int fit = static_cast<int>(most / of_sequence);
+        IV2_CHECK(fit > 0, "varlen_bwd: too many token groups");
+        for (int b = 0; b < batch; b += fit) {
+            BwdParams some = p;
+            some.cu_seqlens_q += b;
+            some.cu_seqlens_k += b;
+            some.kimg += static_cast<int64_t>(b) * kImageElems;
+            some.vimg_r += static_cast<int64_t>(b) * kImageElems;
+            if (int rc = launch_bwd_dq_hybrid(st, some, batch - b < fit ? batch - b : fit, max_seqlen_q, causal)) return rc;
+        }
+        return 0;
+    }
     x.total_groups = static_cast<int>(total);
     x.mask_words = (p.k_blocks + 63) / 64 > 0 ? (p.k_blocks + 63) / 64 : 1;
     const int64_t per_round = 8 * kDqChunk;

@@ -464,7 +464,7 @@ int launch_bwd_dq_tile(hipStream_t st, const BwdParams& p, int batch, int max_se
     x.tiles_per_seq = tiles_per_sequence(p.group, max_seqlen_q);
     x.max_blocks = p.k_blocks;
     const int64_t total = static_cast<int64_t>(x.sequences) * x.tiles_per_seq;
-    IV2_CHECK(total <= 0x3fffffff, "varlen_bwd: too many token groups");
+    IV2_CHECK(total <= max_workgroups(64 * kTileWaves) - 8, "varlen_bwd: too many token groups");
     IV2_CHECK(p.k_blocks <= 16384, "varlen_bwd: more than %d key blocks per sequence", 16384);      // what the hybrid walk's mask rows hold: accepted by either or by none
     const int64_t grid = (total + 7) / 8 * 8;
     const size_t lds = kDqSlots * kSlotBytes;

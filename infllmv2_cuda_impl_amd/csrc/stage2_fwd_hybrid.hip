@@ -450,18 +450,25 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     }
 }
 
-int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q,
-                             int max_seqlen_k, bool causal, int most_selected, unsigned* in_step) {
+static int launch_groups(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q, int max_seqlen_k, bool causal, unsigned* in_step) {
     HybridExtra x{};
     x.batch = batch;
     x.groups_per_seq = (max_seqlen_q + kHybTokens - 1) / kHybTokens;
-    const int64_t total = static_cast<int64_t>(num_heads_k) * batch * x.groups_per_seq;
-    IV2_CHECK(total <= 0x3fffffff, "varlen_fwd: too many token groups");
-    IV2_CHECK((max_seqlen_k + kBlockN - 1) / kBlockN <= kMaxMaskWords * 64, "varlen_fwd: more than %d key blocks per sequence", kMaxMaskWords * 64);
-    const bool tiles = p.mask == nullptr
-        ? dense_tiles_pay(batch, num_heads_k, p.group, p.total_q, p.total_k, max_seqlen_q, max_seqlen_k, causal)
-        : masked_by_tiles(most_selected);
-    if (tiles) return launch_stage2_fwd_tile(st, p, batch, num_heads_k, max_seqlen_q, max_seqlen_k, causal);
+    const int64_t of_sequence = static_cast<int64_t>(num_heads_k) * x.groups_per_seq, total = of_sequence * batch;
+    const int64_t most = max_workgroups(512) - 8 * kHybChunk;
+    if (total > most) {                                        // more than a dispatch holds (thousands of sequences beside a long one): some sequences at a time
+        const int fit = static_cast<int>(most / of_sequence);
+        IV2_CHECK(fit > 0, "varlen_fwd: too many token groups");
+        for (int b = 0; b < batch; b += fit) {
+            FwdParams some = p;
+            some.cu_seqlens_q += b;
+            some.cu_seqlens_k += b;
+            some.kimg += static_cast<int64_t>(b) * kImageElems;               // a sequence's first image: image_slot0
+            some.vimg += static_cast<int64_t>(b) * kImageElems;
+            if (int rc = launch_groups(st, some, batch - b < fit ? batch - b : fit, num_heads_k, max_seqlen_q, max_seqlen_k, causal, in_step)) return rc;
+        }
+        return 0;
+    }
     x.total_groups = static_cast<int>(total);
     x.mask_words = ((max_seqlen_k + kBlockN - 1) / kBlockN + 63) / 64;
     if (x.mask_words < 1) x.mask_words = 1;
@@ -490,6 +497,16 @@ int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int 
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid), parts), dim3(512), lds, st, p, x);
     IV2_LAUNCH_CHECK();
     return 0;
+}
+
+int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q,
+                             int max_seqlen_k, bool causal, int most_selected, unsigned* in_step) {
+    IV2_CHECK((max_seqlen_k + kBlockN - 1) / kBlockN <= kMaxMaskWords * 64, "varlen_fwd: more than %d key blocks per sequence", kMaxMaskWords * 64);
+    const bool tiles = p.mask == nullptr
+        ? dense_tiles_pay(batch, num_heads_k, p.group, p.total_q, p.total_k, max_seqlen_q, max_seqlen_k, causal)
+        : masked_by_tiles(most_selected);
+    return tiles ? launch_stage2_fwd_tile(st, p, batch, num_heads_k, max_seqlen_q, max_seqlen_k, causal)
+                 : launch_groups(st, p, batch, num_heads_k, max_seqlen_q, max_seqlen_k, causal, in_step);
 }
 
 }  // namespace IV2_NS

@@ -425,7 +425,7 @@ int launch_stage2_fwd_tile(hipStream_t st, const FwdParams& p, int batch, int nu
     x.tiles_per_seq = tiles_per_sequence(p.group, max_seqlen_q);
     x.max_blocks = (max_seqlen_k + kBlockN - 1) / kBlockN;
     const int64_t total = static_cast<int64_t>(x.sequences) * x.tiles_per_seq;
-    IV2_CHECK(total <= 0x3fffffff, "varlen_fwd: too many token groups");
+    IV2_CHECK(total <= max_workgroups(64 * kTileWaves) - 8, "varlen_fwd: too many token groups");
     const int64_t grid = (total + 7) / 8 * 8;
     const size_t lds = kSlots * kSlotBytes;
     const auto kernel = causal ? &stage2_fwd_tile_kernel<true> : &stage2_fwd_tile_kernel<false>;

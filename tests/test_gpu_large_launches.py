@@ -6,6 +6,28 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
+def test_thousands_of_sequences_beside_a_long_one():
+    """20 000 sequences and a longest of 8192 tokens are 41 million groups of 8 tokens; nearly all of them are empty."""
+    from infllmv2_cuda_impl_amd.attention import attend_varlen
+    B, Hk = 20000, 2
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    lens = torch.randint(0, 12, (B,), generator=gen, device="cuda")
+    cu = torch.cat([lens.new_zeros(1), lens.cumsum(0)]).to(torch.int32)
+    T = int(cu[-1])
+    q, k, v, dout = (torch.randn(T, Hk, 128, generator=gen, device="cuda").to(torch.bfloat16) for _ in range(4))
+    idx = torch.zeros(Hk, T, 4, dtype=torch.int32, device="cuda")
+    mask = torch.ones(Hk, T, 1, dtype=torch.int64, device="cuda")
+
+    def run(longest):
+        leaves = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        out = attend_varlen(*leaves, cu, cu, longest, 64, causal=True, topk_idx=idx, block_mask=mask)
+        return (out,) + torch.autograd.grad(out, leaves, dout)
+    want, got = run(11), run(8192)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])                                    # output and dQ
+    for a, b in zip(got[2:], want[2:]):                          # dK, dV: sums of at most 11 tokens in fp32 in any order, rounded once
+        assert (a.float() - b.float()).abs().max() <= 2.0 ** -7 * b.float().abs().max()
+
+
 def test_mask_words_of_many_rows():
     from infllmv2_cuda_impl_amd import _lib
     rows, stream = (1 << 26) + 5, torch.cuda.current_stream().cuda_stream
