@@ -253,7 +253,7 @@ int infllmv2_stage1_decode(void* stream, const void* q, const void* k, const voi
                            int out_len, int kernel_size, int stride, int padding, int block_size, int local_blocks,
                            int init_blocks);
 
-/* Everything of a batched decode step in front of its top-k, in two launches (no counterpart in the reference, whose
+/* Everything of a batched decode step in front of its top-k, in one or two launches (no counterpart in the reference, whose
  * callers do it in Python): the new token's K/V rows (k_new, v_new: strides {batch, head}) are written to the caches
  * (batch, capacity, Hk, 128; strides {batch, row, head}) at row lens[b] (host_len for every sequence when lens is null);
  * where the token completes a window its compressed key is appended to fine_cache / coarse_cache (fine_rows, coarse_rows

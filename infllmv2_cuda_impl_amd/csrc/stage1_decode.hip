@@ -22,6 +22,7 @@
 //      fine tiles and writes either the score row or its pooling onto key blocks.  A pooled block needs the last
 //      key of the tile before the run: that one 16-key group is scored again by the run that needs it (same MFMA,
 //      same operands, same bits).
+// Few and short sequences take one launch instead, in which every workgroup forms the log-sum-exp for itself (stage1_decode_whole_kernel): the same bits.
 // Keys can be packed (cu_seqlens) or lie in per-sequence caches (batch stride + lengths).
 #include "common.h"
 #include "infllmv2_hip.h"
@@ -132,45 +133,51 @@ __device__ __forceinline__ float s1d_row_sum(float x) {
     x += __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x124, 0xF, 0xF, false));
     return x + __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(x), 0x128, 0xF, 0xF, false));
 }
-// (max, sum) in log2 units of head 4g + e over the coarse tiles [t0, t1) of one sequence and KV head, merged over the
-// 16 key-column lanes: every lane of row g returns the values of its four heads.  patch(tile registers, tile) runs after
-// a tile is requested.
+// Running (max, sum) in log2 units of head 4g + e over the keys == n (mod 16) of the coarse tiles seen so far: tile ti's are added.
+__device__ __forceinline__ void s1d_lse_tile(const S1DecodeParams& p, const elem8 (&qf)[4], const elem8 (&t)[16], int ti, int vis_c, int n,
+                                             float (&m)[4], float (&l)[4]) {
+    floatx4 s[4];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+        s[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) s[kt] = IV2_MFMA(qf[c], t[kt * 4 + c], s[kt], 0, 0, 0);
+    }
+    const bool cut = (ti + 1) * 64 > vis_c;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float v[4];
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) v[kt] = s[kt][e] * p.scale_log2;
+        if (cut) {
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) v[kt] = (ti * 64 + kt * 16 + n < vis_c) ? v[kt] : -INFINITY;
+        }
+        const float mx = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
+        const float m_new = fmaxf(m[e], mx);
+        const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+        float acc = l[e] * __builtin_amdgcn_exp2f(m[e] - m_use);
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) acc += __builtin_amdgcn_exp2f(v[kt] - m_use);
+        l[e] = acc;
+        m[e] = m_new;
+    }
+}
+// ... merged over the 16 key-column lanes: every lane of row g gets the values of its four heads
+__device__ __forceinline__ void s1d_lse_close(const float (&m)[4], const float (&l)[4], float (&m_out)[4], float (&l_out)[4]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        m_out[e] = s1d_row_max(m[e]);
+        l_out[e] = s1d_row_sum(l[e] * __builtin_amdgcn_exp2f(m[e] - (m_out[e] == -INFINITY ? 0.f : m_out[e])));
+    }
+}
+// Both over the coarse tiles [t0, t1) of one sequence and KV head.  patch(tile registers, tile) runs after a tile is requested.
 template <typename Patch>
 __device__ __forceinline__ void s1d_lse_run(const S1DecodeParams& p, const S1DecodeSeq& sq, const elem8 (&qf)[4], int vis_c,
                                             int t0, int t1, int n, int g, float (&m_out)[4], float (&l_out)[4], Patch patch) {
-    float m[4], l[4];                                          // head 4g + e over the keys == n (mod 16) of the run
+    float m[4], l[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) { m[e] = -INFINITY; l[e] = 0.f; }
-
-    auto consume = [&](const elem8 (&t)[16], int ti) {
-        floatx4 s[4];
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt) {
-            s[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int c = 0; c < 4; ++c) s[kt] = IV2_MFMA(qf[c], t[kt * 4 + c], s[kt], 0, 0, 0);
-        }
-        const bool cut = (ti + 1) * 64 > vis_c;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            float v[4];
-#pragma unroll
-            for (int kt = 0; kt < 4; ++kt) v[kt] = s[kt][e] * p.scale_log2;
-            if (cut) {
-#pragma unroll
-                for (int kt = 0; kt < 4; ++kt) v[kt] = (ti * 64 + kt * 16 + n < vis_c) ? v[kt] : -INFINITY;
-            }
-            const float mx = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
-            const float m_new = fmaxf(m[e], mx);
-            const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-            float acc = l[e] * __builtin_amdgcn_exp2f(m[e] - m_use);
-#pragma unroll
-            for (int kt = 0; kt < 4; ++kt) acc += __builtin_amdgcn_exp2f(v[kt] - m_use);
-            l[e] = acc;
-            m[e] = m_new;
-        }
-    };
-
     elem8 ta[16], tb[16];
     auto load = [&](elem8 (&t)[16], int ti) {
         s1d_load_tile(t, sq.cbase, p.c_row_stride, ti * 64, sq.Lc, n, g);
@@ -179,19 +186,14 @@ __device__ __forceinline__ void s1d_lse_run(const S1DecodeParams& p, const S1Dec
     if (t0 < t1) load(ta, t0);
     if (t0 + 1 < t1) load(tb, t0 + 1);
     for (int ti = t0; ti < t1; ti += 2) {
-        consume(ta, ti);
+        s1d_lse_tile(p, qf, ta, ti, vis_c, n, m, l);
         if (ti + 2 < t1) load(ta, ti + 2);
         if (ti + 1 < t1) {
-            consume(tb, ti + 1);
+            s1d_lse_tile(p, qf, tb, ti + 1, vis_c, n, m, l);
             if (ti + 3 < t1) load(tb, ti + 3);
         }
     }
-    // merge the 16 key-column lanes of each head
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        m_out[e] = s1d_row_max(m[e]);
-        l_out[e] = s1d_row_sum(l[e] * __builtin_amdgcn_exp2f(m[e] - (m_out[e] == -INFINITY ? 0.f : m_out[e])));
-    }
+    s1d_lse_close(m, l, m_out, l_out);
 }
 
 // The partial records {max x 16, sum x 16} of one (sequence, head) as a lane needs them: lane (n, g) takes the records
@@ -334,6 +336,30 @@ __device__ __forceinline__ elem_bits s1d_window_mean(const S1DecodeStep& t, int 
     return f32_to_elem_hw(sum / static_cast<float>(kernel_size));
 }
 
+// What a step leaves behind for one sequence and KV head, by a workgroup of its own: the new token's rows, the lengths, the compressed keys it completes
+// (the coarse one only where nobody else forms it).
+__device__ __forceinline__ void s1d_keep_caches(const S1DecodeParams& p, const S1DecodeStep& t, int b, int h, int len, int rows_f, int rows_c, int add_f,
+                                                int add_c, int tid) {
+    const int g = tid >> 4, n = tid & 15;
+    if (tid < 32 && len < t.capacity) {
+        const elem_bits* src = g == 0 ? t.knew + b * t.kn_batch + h * t.kn_head : t.vnew + b * t.vn_batch + h * t.vn_head;
+        elem_bits* dst = g == 0 ? t.kcache + b * t.kc_batch + len * t.kc_row + h * t.kc_head
+                                : t.vcache + b * t.vc_batch + len * t.vc_row + h * t.vc_head;
+        *reinterpret_cast<uint4*>(dst + 8 * n) = *reinterpret_cast<const uint4*>(src + 8 * n);
+    }
+    if (h == 0 && tid == 0) {
+        if (t.new_lens) t.new_lens[b] = len + 1;
+        t.fine_lens[b] = rows_f;
+        t.coarse_lens[b] = rows_c;
+    }
+    if (add_f >= 0 && tid < kHeadDim)
+        t.fine[b * p.k_batch_stride + add_f * p.k_row_stride + h * p.k_head_stride + tid] =
+            s1d_window_mean(t, b, h, add_f, t.kernel_f, t.stride_f, tid);
+    if (add_c >= 0 && !t.with_scores && tid < kHeadDim)
+        t.coarse[b * p.c_batch_stride + add_c * p.c_row_stride + h * p.c_head_stride + tid] =
+            s1d_window_mean(t, b, h, add_c, t.kernel_c, t.stride_c, tid);
+}
+
 __global__ __launch_bounds__(64 * kLseWaves)
 void stage1_decode_front_kernel(const S1DecodeParams p, const S1DecodeStep t) {
     __shared__ __attribute__((aligned(16))) elem_bits newest_key[kHeadDim];         // the coarse key this token completes
@@ -346,23 +372,7 @@ void stage1_decode_front_kernel(const S1DecodeParams p, const S1DecodeStep t) {
     const int rows_f = s1d_step_rows(len, t.capacity, t.kernel_f, t.stride_f, t.fine_capacity, add_f);
     const int rows_c = s1d_step_rows(len, t.capacity, t.kernel_c, t.stride_c, t.coarse_capacity, add_c);
     if (first < 0) {                                           // the caches' keepers
-        if (wave == 0 && len < t.capacity && g < 2) {
-            const elem_bits* src = g == 0 ? t.knew + b * t.kn_batch + h * t.kn_head : t.vnew + b * t.vn_batch + h * t.vn_head;
-            elem_bits* dst = g == 0 ? t.kcache + b * t.kc_batch + len * t.kc_row + h * t.kc_head
-                                    : t.vcache + b * t.vc_batch + len * t.vc_row + h * t.vc_head;
-            *reinterpret_cast<uint4*>(dst + 8 * n) = *reinterpret_cast<const uint4*>(src + 8 * n);
-        }
-        if (h == 0 && tid == 0) {
-            if (t.new_lens) t.new_lens[b] = len + 1;
-            t.fine_lens[b] = rows_f;
-            t.coarse_lens[b] = rows_c;
-        }
-        if (add_f >= 0)
-            t.fine[b * p.k_batch_stride + add_f * p.k_row_stride + h * p.k_head_stride + tid] =
-                s1d_window_mean(t, b, h, add_f, t.kernel_f, t.stride_f, tid);
-        if (add_c >= 0 && !t.with_scores)
-            t.coarse[b * p.c_batch_stride + add_c * p.c_row_stride + h * p.c_head_stride + tid] =
-                s1d_window_mean(t, b, h, add_c, t.kernel_c, t.stride_c, tid);
+        s1d_keep_caches(p, t, b, h, len, rows_f, rows_c, add_f, add_c, tid);
         return;
     }
     const int tiles = (rows_c + 63) >> 6, split = first + wave;
@@ -538,6 +548,226 @@ void stage1_decode_score_kernel(const S1DecodeParams p) {
     s1d_score_run<kPool>(p, sq, qf, lse2, before4, ta, tb, vis_f, tiles, t0, t1, owns_tail, b, h, lane);
 }
 
+
+// One tile's results: lane l brings the score of key l (pooled: and the last key before the tile), the row's last tile also fills the columns behind it.
+template <bool kPool>
+__device__ __forceinline__ void s1d_store_tile(const S1DecodeParams& p, const S1DecodeSeq& sq, float mine, float carry, int vis_f, int tiles, int ti, bool live,
+                                               bool owns_tail, int b, int h, int lane) {
+    elem_bits* out = p.out + static_cast<int64_t>(h) * p.out_head_stride + static_cast<int64_t>(sq.q_row) * p.out_row_stride;
+    if constexpr (!kPool) {
+        if (owns_tail)
+            for (int col = tiles * 64 + lane; col < p.cols; col += 64) out[col] = 0;
+    } else {
+        const int bq = (p.cache_lens ? p.cache_lens[b] : p.cache_len) / kBlockN;
+        const int Lk_cols = sq.Lk < p.cols ? sq.Lk : p.cols;
+        auto pool_rest = [&](int kb, float reached) -> elem_bits {
+            const bool forced = (kb < p.init_blocks) || (bq >= kb && bq <= kb + p.local_blocks);
+            const int first = kb * 4 - 1;
+            const bool empty = (first < 0 ? 0 : first) >= Lk_cols;
+            return forced ? kElemPosInf : (empty ? kElemNegInf : f32_to_elem_hw(reached));
+        };
+        float left = __shfl_up(mine, 1);
+        if (lane == 0) left = carry;
+        float best = fmaxf(mine, s1d_quad_xor1(mine));
+        best = fmaxf(best, s1d_quad_xor2(best));
+        best = fmaxf(best, left);
+        const int kb = ti * 16 + (lane >> 2);
+        if (live && (lane & 3) == 0 && kb < p.pool_len) out[kb] = pool_rest(kb, best);
+        if (owns_tail) {
+            const float last = live ? __shfl(mine, 63) : 0.f;
+            for (int k = tiles * 16 + lane; k < p.pool_len; k += 64) out[k] = pool_rest(k, k == tiles * 16 ? last : 0.f);
+        }
+    }
+}
+
+// Both halves in one launch, for few and short sequences: a workgroup per fine tile, of four wavefronts, forms the log-sum-exp of its sequence and KV head for
+// itself.  The coarse tiles go round the wavefronts, their records through LDS; then a wavefront scores 16 keys of the fine tile, and the last one
+// also the key before it that opens the tile's first pooling window.  The time is a chain of round trips: arguments and lengths 0.8 us, the keys 1.4 to 2.7
+// (112 KiB through one CU with four coarse tiles), records, merge and scores 1.5; which launches: s1d_whole.
+// kStep: and the rest of the front of a decode step (above).  The keys this very token completes are not read from the caches, which a workgroup of this launch
+// is writing: a workgroup that needs one forms it itself.
+constexpr int kWholeWaves = 4;
+constexpr int kWholeWindow = 128;                              // rows of a coarse window at most
+constexpr int kWholeRecords = 8;                               // coarse tiles at most (s1d_whole takes fewer)
+struct S1DecodeNoStep {};
+
+template <bool kPool, typename Step>
+__global__ __launch_bounds__(64 * kWholeWaves)
+void stage1_decode_whole_kernel(const S1DecodeParams p, const Step t) {
+    constexpr bool kStep = !std::is_same<Step, S1DecodeNoStep>::value;
+    __shared__ __attribute__((aligned(16))) float records[kWholeRecords * 32];
+    __shared__ float score[64];                                // of the tile's keys
+    __shared__ __attribute__((aligned(16))) elem_bits window[kStep ? kWholeWindow * kHeadDim : 8];
+    __shared__ __attribute__((aligned(16))) elem_bits newest[kStep ? 2 * kHeadDim : 8];                 // the coarse key this token completes, and the fine one
+    warm_kernel_arguments<sizeof(S1DecodeParams) + (kStep ? sizeof(Step) : 0)>();
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ti = static_cast<int>(blockIdx.x) - (kStep ? 1 : 0), h = blockIdx.y, b = blockIdx.z;
+    int add_f = -1, add_c = -1;
+    S1DecodeSeq sq;
+    if constexpr (kStep) {
+        const int len = t.lens ? t.lens[b] : t.host_len;
+        sq.q_row = b; sq.Sq = 1;
+        sq.Lk = s1d_step_rows(len, t.capacity, t.kernel_f, t.stride_f, t.fine_capacity, add_f);
+        sq.Lc = s1d_step_rows(len, t.capacity, t.kernel_c, t.stride_c, t.coarse_capacity, add_c);
+        sq.kbase = p.k + b * p.k_batch_stride + h * p.k_head_stride;
+        sq.cbase = p.c + b * p.c_batch_stride + h * p.c_head_stride;
+        if (ti < 0) {                                          // the caches' keepers
+            s1d_keep_caches(p, t, b, h, len, sq.Lk, sq.Lc, add_f, add_c, tid);
+            return;
+        }
+    } else {
+        sq = s1d_sequence(p, b, h);
+        if (sq.Sq <= 0) return;
+    }
+    int vis_c, vis_f, tiles;
+    s1d_fine_extent<kPool>(p, sq, vis_c, vis_f, tiles);
+    if (ti >= tiles && ti > 0) return;                         // uniform over the workgroup
+    const bool live = ti < tiles, owns_tail = ti + 1 >= tiles; // not live: the row's first workgroup, which fills a row without scores
+    const int tiles_c = vis_c > 64 * kWholeRecords ? kWholeRecords : (vis_c + 63) >> 6;     // lengths beyond what the launch was announced stay inside
+
+    // what is read, requested in the order in which it is needed
+    elem8 qf[4], ca[16], cb[16], mine[4], before[4];
+    s1d_load_q(qf, p, sq, h, n, g);
+    if (wave < tiles_c) s1d_load_tile(ca, sq.cbase, p.c_row_stride, wave * 64, sq.Lc, n, g);
+    if (wave + kWholeWaves < tiles_c) s1d_load_tile(cb, sq.cbase, p.c_row_stride, (wave + kWholeWaves) * 64, sq.Lc, n, g);
+    if (live) {
+        int row = ti * 64 + 16 * wave + n;
+        row = row < sq.Lk ? row : sq.Lk - 1;
+        const elem_bits* src = sq.kbase + row * p.k_row_stride + 8 * g;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) mine[c] = *reinterpret_cast<const elem8*>(src + 32 * c);
+        if (kPool) s1d_load_group_before(before, sq, p.k_row_stride, ti, n, g);     // every wavefront: a condition on it costs a wait for the loads
+    }
+    if constexpr (kStep) {
+        const bool adds_f = live && add_f >> 6 == ti;          // uniform over the workgroup
+        if (add_c >= 0) {
+            // the window's rows to LDS, all of them requested at once; its last row is the new token's
+            const elem_bits* rows = t.kcache + b * t.kc_batch + static_cast<int64_t>(add_c) * t.stride_c * t.kc_row + h * t.kc_head + (tid & 15) * 8;
+            const elem_bits* last = t.knew + b * t.kn_batch + h * t.kn_head + (tid & 15) * 8;
+            uint4 w[kWholeWindow / (4 * kWholeWaves)];
+#pragma unroll
+            for (int i = 0; i < kWholeWindow / (4 * kWholeWaves); ++i) {
+                const int row = 4 * kWholeWaves * i + (tid >> 4);
+                w[i] = *reinterpret_cast<const uint4*>(row < t.kernel_c - 1 ? rows + row * t.kc_row : last);
+            }
+#pragma unroll
+            for (int i = 0; i < kWholeWindow / (4 * kWholeWaves); ++i)
+                *reinterpret_cast<uint4*>(&window[(4 * kWholeWaves * i + (tid >> 4)) * kHeadDim + (tid & 15) * 8]) = w[i];
+        }
+        if (adds_f && wave >= 2) newest[kHeadDim + (tid & 127)] = s1d_window_mean(t, b, h, add_f, t.kernel_f, t.stride_f, tid & 127);
+        if (add_c >= 0) {
+            __syncthreads();
+            if (wave < 2) {
+                // in window order; the next rows are on their way while these are added up
+                constexpr int kRows = 32;
+                float sum = 0.f;
+                elem_bits even[kRows], odd[kRows];
+                auto fetch = [&](elem_bits (&rows)[kRows], int from) {
+#pragma unroll
+                    for (int r = 0; r < kRows; ++r) rows[r] = window[(from + r) * kHeadDim + tid];
+                };
+                auto add = [&](const elem_bits (&rows)[kRows], int from) {
+                    if (from + kRows <= t.kernel_c) {
+#pragma unroll
+                        for (int r = 0; r < kRows; ++r) sum += elem_to_f32(rows[r]);
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < kRows; ++r) sum += from + r < t.kernel_c ? elem_to_f32(rows[r]) : 0.f;
+                    }
+                };
+                fetch(even, 0);
+#pragma unroll
+                for (int from = 0; from < kWholeWindow; from += 2 * kRows) {
+                    fetch(odd, from + kRows);
+                    add(even, from);
+                    if (from + 2 * kRows < kWholeWindow) fetch(even, from + 2 * kRows);
+                    add(odd, from + kRows);
+                }
+                const elem_bits mean = f32_to_elem_hw(sum / static_cast<float>(t.kernel_c));
+                newest[tid] = mean;
+                if (ti == 0) t.coarse[b * p.c_batch_stride + add_c * p.c_row_stride + h * p.c_head_stride + tid] = mean;
+            }
+        }
+        if (adds_f || add_c >= 0) __syncthreads();
+        if (adds_f && ti * 64 + 16 * wave + n >= add_f) {      // the newest key, and the lanes beyond it that repeat it
+#pragma unroll
+            for (int c = 0; c < 4; ++c) mine[c] = *reinterpret_cast<const elem8*>(newest + kHeadDim + 32 * c + 8 * g);
+        }
+    }
+    auto patch = [&](elem8 (&tile)[16], int r) {
+        if (!kStep || add_c < 0 || r != add_c >> 6) return;    // uniform
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+            if (r * 64 + 16 * kt + n >= add_c) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) tile[kt * 4 + c] = *reinterpret_cast<const elem8*>(newest + 32 * c + 8 * g);
+            }
+    };
+    auto record = [&](elem8 (&tile)[16], int r) {
+        patch(tile, r);
+        float m[4], l[4], mm[4], ll[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { m[e] = -INFINITY; l[e] = 0.f; }
+        s1d_lse_tile(p, qf, tile, r, vis_c, n, m, l);
+        s1d_lse_close(m, l, mm, ll);
+        if (n == 0) {
+            *reinterpret_cast<floatx4*>(records + r * 32 + 4 * g) = floatx4{mm[0], mm[1], mm[2], mm[3]};
+            *reinterpret_cast<floatx4*>(records + r * 32 + 16 + 4 * g) = floatx4{ll[0], ll[1], ll[2], ll[3]};
+        }
+    };
+    for (int r = wave; r < tiles_c; r += 2 * kWholeWaves) {
+        record(ca, r);
+        if (r + 2 * kWholeWaves < tiles_c) s1d_load_tile(ca, sq.cbase, p.c_row_stride, (r + 2 * kWholeWaves) * 64, sq.Lc, n, g);
+        if (r + kWholeWaves < tiles_c) {
+            record(cb, r + kWholeWaves);
+            if (r + 3 * kWholeWaves < tiles_c) s1d_load_tile(cb, sq.cbase, p.c_row_stride, (r + 3 * kWholeWaves) * 64, sq.Lc, n, g);
+        }
+    }
+    // S of the 16 keys, before the wait for the other records
+    auto products = [&](const elem8 (&t4)[4]) {
+        floatx4 s = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < 4; ++c) s = IV2_MFMA(qf[c], t4[c], s, 0, 0, 0);
+        return s;
+    };
+    floatx4 s_mine = {0.f, 0.f, 0.f, 0.f}, s_before = {0.f, 0.f, 0.f, 0.f};
+    if (live) {
+        s_mine = products(mine);
+        if (kPool && wave == kWholeWaves - 1 && ti > 0) s_before = products(before);
+    }
+    __syncthreads();
+    float carry = 0.f;                                         // score of the last key before the tile (the last wavefront's)
+    if (live) {
+        S1DRecords rec;
+        float lse2[4];
+        s1d_load_records(rec, records, tiles_c, n, g);
+        s1d_merge_records(rec, tiles_c, n, g, p.group, lse2);
+        auto score_of = [&](const floatx4& s) {                // of key n of the 16, in every row
+            float sum = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum += __builtin_amdgcn_exp2f(s[e] * p.scale_log2 - lse2[e]);
+            const float rows = s1d_fold_rows16(sum, sum);
+            return s1d_fold_rows32(rows, rows);
+        };
+        const float got = score_of(s_mine);
+        const int key = ti * 64 + 16 * wave + n;
+        if (!kPool) {
+            if (g == 0 && key < p.cols) p.out[static_cast<int64_t>(h) * p.out_head_stride + static_cast<int64_t>(sq.q_row) * p.out_row_stride + key] =
+                f32_to_elem_hw(key < vis_f ? got : 0.f);
+        } else {
+            if (g == 0) score[16 * wave + n] = key < vis_f ? got : 0.f;
+            if (wave == kWholeWaves - 1 && ti > 0) {
+                const float prev = ti * 64 - 16 + n < vis_f ? score_of(s_before) : 0.f;
+                carry = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(prev), 15));
+            }
+        }
+    }
+    if constexpr (kPool) __syncthreads();
+    if (wave != kWholeWaves - 1) return;
+    s1d_store_tile<kPool>(p, sq, live ? score[lane] : 0.f, carry, vis_f, tiles, ti, live, owns_tail, b, h, lane);
+}
+
 }  // namespace IV2_NS
 
 using namespace IV2_NS;
@@ -556,6 +786,18 @@ void s1d_splits(int batch, int num_heads_k, int max_keys, int max_coarse, int& s
     };
     plan((max_keys + 63) / 64, splits_f, run_f);
     plan((max_coarse + 63) / 64, splits_c, run_c);
+}
+// One launch (stage1_decode_whole_kernel) instead of two: up to five coarse tiles, i.e. 20 543 tokens, and a workgroup per CU.  Every workgroup loads all coarse
+// tiles, 16 KiB each, through its CU's vector memory path and forms their records; that costs 0.4 us a tile, and the launch it saves is worth 1.5 us of the device
+// and 2.5 us of the host that issues it.  A decode step in us, two launches | one: one sequence of 1000 tokens 17.5 | 14.8, 4000 17.6 | 15.1, 8000 17.9 | 15.9, 16 000
+// 18.0 | 16.9, 20 000 18.0 | 18.1, 24 000 18.1 | 18.6, 32 000 18.0 | 19.4; two of up to 8000 17.5 | 15.6, six of up to 20 000 19.2 | 18.1, eight of up to 8000 19.7 | 17.9,
+// 16 of them (256 workgroups) 24.2 | 23.0; 32 (512) 34.4 | 37.4, 24 of up to 16 000 34.0 | 41.8; eight paged ones of up to 8000, called operator by operator, 25.5 | 22.8.
+constexpr int kWholeCoarseTiles = 5;
+static_assert(kWholeCoarseTiles <= kWholeRecords, "a record per coarse tile");
+constexpr int kWholeWorkgroups = 256;
+bool s1d_whole(const S1DecodeParams& p, int batch, int num_heads_k) {
+    return p.run_c == 1 && p.run_f == 1 && p.splits_c <= kWholeCoarseTiles &&
+           static_cast<int64_t>(batch) * num_heads_k * p.splits_f <= kWholeWorkgroups;
 }
 unsigned s1d_lse_workgroups(int splits_c) { return static_cast<unsigned>((splits_c + kLseWaves - 1) / kLseWaves); }
 
@@ -625,6 +867,12 @@ extern "C" int IV2_ENTRY(infllmv2_stage1_decode)(void* stream, const void* q, co
     p.cache_lens = cache_lens; p.cache_len = cache_len; p.pool_len = out_len;
     p.local_blocks = local_blocks; p.init_blocks = init_blocks;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (s1d_whole(p, batch, num_heads_k)) {
+        auto kernel = pooled ? stage1_decode_whole_kernel<true, S1DecodeNoStep> : stage1_decode_whole_kernel<false, S1DecodeNoStep>;
+        hipLaunchKernelGGL(kernel, dim3(p.splits_f, num_heads_k, batch), dim3(64 * kWholeWaves), 0, st, p, S1DecodeNoStep{});
+        IV2_LAUNCH_CHECK();
+        return 0;
+    }
     hipLaunchKernelGGL(stage1_decode_lse_kernel, dim3(s1d_lse_workgroups(p.splits_c), num_heads_k, batch), dim3(64 * kLseWaves), 0, st, p);
     IV2_LAUNCH_CHECK();
     const dim3 grid(p.splits_f, num_heads_k, batch);
@@ -702,6 +950,12 @@ extern "C" int IV2_ENTRY(infllmv2_decode_step_scores)(void* stream, const void* 
     t.kernel_f = kernel_size_f; t.stride_f = stride_f; t.kernel_c = kernel_size_c; t.stride_c = stride_c;
     t.with_scores = pooled != nullptr ? 1 : 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (pooled != nullptr && out_len > 0 && kernel_size_c <= kWholeWindow && s1d_whole(p, batch, num_heads_k)) {
+        hipLaunchKernelGGL((stage1_decode_whole_kernel<true, S1DecodeStep>), dim3(1 + p.splits_f, num_heads_k, batch),
+                           dim3(64 * kWholeWaves), 0, st, p, t);
+        IV2_LAUNCH_CHECK();
+        return 0;
+    }
     hipLaunchKernelGGL(stage1_decode_front_kernel, dim3(1 + s1d_lse_workgroups(p.splits_c), num_heads_k, batch), dim3(64 * kLseWaves), 0, st, p, t);
     IV2_LAUNCH_CHECK();
     if (pooled == nullptr || out_len == 0) return 0;
