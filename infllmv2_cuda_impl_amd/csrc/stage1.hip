@@ -29,6 +29,7 @@
 #include "block_walker.h"
 #include "infllmv2_hip.h"
 #include <math.h>
+#include <type_traits>
 
 namespace IV2_NS {
 
@@ -60,7 +61,7 @@ struct Stage1Params {
 };
 
 // 8 wavefronts x 2 tokens: 112 registers, so four wavefronts share a SIMD and the exp-heavy VALU work of one hides
-// behind the MFMAs of another (4 x 4 at two wavefronts per SIMD measures 6 % slower, 8 x 1 15 % slower)
+// behind the MFMAs of another (4 x 4 at two wavefronts per SIMD measures 6 % slower, 8 x 1 15 % slower where the launch fills the chip; where it does not: launch_stage1)
 constexpr int kTokPerWave = 2;
 constexpr int kWavesS1 = 8;
 constexpr int kWavesPerSimdS1 = 4;
@@ -173,11 +174,13 @@ __device__ __forceinline__ void pool_quads(float a, float b, float prev_a, float
 // 2048 tokens 15.9 | 11.9, 4096 27.3 | 21.2, 8192 56.2 | 48.5, 16 384 133 | 125, 20 480 201 | 196, 32 768 443 | 443, 49 152 931 | 944: rows of 512 blocks and no more.  Whole prefill of
 // 1000 tokens, 16 blocks selected, 42.0 -> 40.7, of 2048 74.4 -> 70.0, training on 1023 + 3001 + 517 + 2200 606 -> 596.
 // kShared: workgroups share a block of tokens (launch_stage1); a variant of its own, because the others paid 0.5 us for the possibility.
-template <bool kCausal, bool kPool, int kItems = 0, bool kShared = false>
+// kTok: tokens of a wavefront, 2 or, in launches of few workgroups (launch_stage1), 1.  A token's row is the same bits either way.
+template <bool kCausal, bool kPool, int kItems = 0, bool kShared = false, int kTok = kTokPerWave>
 __global__ __launch_bounds__(64 * kWavesS1) __attribute__((amdgpu_waves_per_eu(kWavesPerSimdS1, kWavesPerSimdS1)))
 void stage1_kernel(const Stage1Params p) {
+    constexpr int kTokens = kTok * kWavesS1;                   // of the workgroup
     __shared__ uint4 tile[2][1024];                            // two 16 KiB operand-ordered key tiles
-    __shared__ elem_bits pooled[kItems > 0 ? kTokPerBlock : 1][kItems > 0 ? 64 * kItems : 1];
+    __shared__ elem_bits pooled[kItems > 0 ? kTokens : 1][kItems > 0 ? 64 * kItems : 1];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);     // wavefront-uniform: what depends on it alone stays in scalar registers
@@ -188,18 +191,18 @@ void stage1_kernel(const Stage1Params p) {
     // late tokens see the most keys: they go first, so the long workgroups do not form the tail of the launch
     const int splits = kShared ? p.splits : 1;
     const int from_end = blockIdx.x / splits, split = blockIdx.x - from_end * splits;
-    const int tok_block0 = (static_cast<int>(gridDim.x) / splits - 1 - from_end) * kTokPerBlock;
+    const int tok_block0 = (static_cast<int>(gridDim.x) / splits - 1 - from_end) * kTokens;
     if (tok_block0 >= Sq) return;                              // uniform per workgroup
     const int k0 = p.cu_seqlens_k[b], Lk = p.cu_seqlens_k[b + 1] - k0;
     const int c0 = p.cu_seqlens_c[b], Lc = p.cu_seqlens_c[b + 1] - c0;
     const int s1 = (Lk == Lc) ? 16 : 64;                       // flash_fwd_kernel.h:1236-1240
 
-    const int tok0 = tok_block0 + wave * kTokPerWave;          // first token of this wavefront
-    int vis_f[kTokPerWave], vis_c[kTokPerWave];
-    bool live[kTokPerWave];
+    const int tok0 = tok_block0 + wave * kTok;                 // first token of this wavefront
+    int vis_f[kTok], vis_c[kTok];
+    bool live[kTok];
     int min_vis_c = 0x7fffffff;
 #pragma unroll
-    for (int t = 0; t < kTokPerWave; ++t) {
+    for (int t = 0; t < kTok; ++t) {
         const int i = tok0 + t;
         live[t] = i < Sq;
         vis_f[t] = live[t] ? stage1_visible(i, 16, Lk, Sq, kCausal) : 0;
@@ -209,7 +212,7 @@ void stage1_kernel(const Stage1Params p) {
         min_vis_c = vis_c[t] < min_vis_c ? vis_c[t] : min_vis_c;
     }
     // tile counts are taken over the whole workgroup (its last live token sees the most keys)
-    const int i_last = (tok_block0 + kTokPerBlock - 1 < Sq ? tok_block0 + kTokPerBlock - 1 : Sq - 1);
+    const int i_last = (tok_block0 + kTokens - 1 < Sq ? tok_block0 + kTokens - 1 : Sq - 1);
     const int wg_vis_c = stage1_visible(i_last, s1, Lc, Sq, kCausal);
     const int wg_vis_f = wg_vis_c == 0 ? 0 : stage1_visible(i_last, 16, Lk, Sq, kCausal);
     const int tiles_c = (wg_vis_c + 63) >> 6;
@@ -231,9 +234,9 @@ void stage1_kernel(const Stage1Params p) {
     // (Waiting for Q before the tile was requested: kernel alone 20.8 us instead of 20.0 at 4096 tokens, 48.6 instead of 47.2 at 8192.  Of 11 us at 2048 tokens
     // this wait is 3: all of Q, 16.8 MB, at once.)
     // Q as the A operand, requested behind the first tile: r = lane % 16 is the head, g the k-group
-    elem8 qf[kTokPerWave][4];
+    elem8 qf[kTok][4];
 #pragma unroll
-    for (int t = 0; t < kTokPerWave; ++t) {
+    for (int t = 0; t < kTok; ++t) {
         const int i = live[t] ? tok0 + t : Sq - 1;
         const elem_bits* qp = p.q + (static_cast<int64_t>(q0) + i) * p.q_tok_stride + h * p.q_kvh_stride + (n < p.group ? n : p.group - 1) * p.q_grp_stride + 8 * g;
 #pragma unroll
@@ -243,37 +246,39 @@ void stage1_kernel(const Stage1Params p) {
     // both have landed from here on: the compiler's wait counts know nothing of the DMA loads
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
-    for (int t = 0; t < kTokPerWave; ++t)
+    for (int t = 0; t < kTok; ++t)
 #pragma unroll
         for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(qf[t][c]));
     __syncthreads();
 
     // ---------------- pass 1: per-head log-sum-exp over the coarse keys ----------------
-    float m[kTokPerWave][4], l[kTokPerWave][4];                // lane-local over keys == n (mod 16); head 4g+e
+    float m[kTok][4], l[kTok][4];                              // lane-local over keys == n (mod 16); head 4g+e
 #pragma unroll
-    for (int t = 0; t < kTokPerWave; ++t)
+    for (int t = 0; t < kTok; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) { m[t][e] = -INFINITY; l[t][e] = 0.f; }
 
-    auto coarse_tile = [&](int ti, floatx4 (&s)[kTokPerWave][4]) {
+    auto next_coarse = [&](int ti) {
         if (ti + 1 < tiles_c) issue_tile(cbase, c_stride, c_off, (ti + 1) * 64, Lc, lds_tiles + ((ti + 1) & 1) * 16384, wave_u, n, g);
+    };
+    auto coarse_tile = [&](int ti, floatx4 (&s)[kTok][4]) {
         const uint4* cur = tile[ti & 1];
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
 #pragma unroll
-            for (int t = 0; t < kTokPerWave; ++t) s[t][kt] = floatx4{0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < kTok; ++t) s[t][kt] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 const uint4 raw = cur[(kt * 4 + c) * 64 + lane];
                 elem8 kf;
                 __builtin_memcpy(&kf, &raw, 16);
 #pragma unroll
-                for (int t = 0; t < kTokPerWave; ++t)
+                for (int t = 0; t < kTok; ++t)
                     s[t][kt] = IV2_MFMA(qf[t][c], kf, s[t][kt], 0, 0, 0);
             }
         }
     };
-    auto coarse_done = [&]() {
+    auto tile_done = [&]() {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // this wavefront's share of the next tile has landed
         __syncthreads();
     };
@@ -281,10 +286,11 @@ void stage1_kernel(const Stage1Params p) {
     // tokens: the maximum is finite, no key test, and the scale rides in the multiply-add that feeds exp2.
     const int whole_c = min_vis_c >> 6 < tiles_c ? min_vis_c >> 6 : tiles_c;
     for (int ti = 0; ti < whole_c; ++ti) {
-        floatx4 s[kTokPerWave][4];
+        next_coarse(ti);
+        floatx4 s[kTok][4];
         coarse_tile(ti, s);
 #pragma unroll
-        for (int t = 0; t < kTokPerWave; ++t) {
+        for (int t = 0; t < kTok; ++t) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float mx = fmaxf(fmaxf(s[t][0][e], s[t][1][e]), fmaxf(s[t][2][e], s[t][3][e]));
@@ -296,13 +302,18 @@ void stage1_kernel(const Stage1Params p) {
                 m[t][e] = m_new;
             }
         }
-        coarse_done();
+        tile_done();
     }
     for (int ti = whole_c; ti < tiles_c; ++ti) {               // the tiles that hold a token's last visible key
-        floatx4 s[kTokPerWave][4];
+        next_coarse(ti);
+        if (!live[0]) {                                        // uniform: a wavefront without a token only brings its share of the tiles
+            tile_done();
+            continue;
+        }
+        floatx4 s[kTok][4];
         coarse_tile(ti, s);
 #pragma unroll
-        for (int t = 0; t < kTokPerWave; ++t) {
+        for (int t = 0; t < kTok; ++t) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 float v[4];
@@ -319,12 +330,12 @@ void stage1_kernel(const Stage1Params p) {
                 m[t][e] = m_new;
             }
         }
-        coarse_done();
+        tile_done();
     }
     // merge the 16 key-column lanes of each head: lse2 = m + log2(l) in log2 units
-    float lse2[kTokPerWave][4];
+    float lse2[kTok][4];
 #pragma unroll
-    for (int t = 0; t < kTokPerWave; ++t)
+    for (int t = 0; t < kTok; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             // the row's maximum first, then every lane's sum rescaled to it once, then the sum of those
@@ -339,16 +350,16 @@ void stage1_kernel(const Stage1Params p) {
     if (begin_f < end_f) issue_tile(kbase, k_stride, k_off, begin_f * 64, Lk, lds_tiles + (begin_f & 1) * 16384, wave_u, n, g);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    static_assert(kTokPerWave == 2, "pool_quads takes two tokens");
-    elem_bits* out_rows[kTokPerWave];
-    int bq[kTokPerWave];                                       // pooled output: the key block the token itself sits in
-    float prev[kTokPerWave];                                   // pooled output: scores of the previous tile, for its last key
+    static_assert(kTok == 1 || kTok == 2, "pool_quads takes two tokens");
+    elem_bits* out_rows[kTok];
+    int bq[kTok];                                              // pooled output: the key block the token itself sits in
+    float prev[kTok];                                          // pooled output: scores of the previous tile, for its last key
     int plain_first = 0, plain_end;                            // tiles that need no test, below
     {
         const int cache_len = kPool ? (p.cache_lens ? p.cache_lens[b] : p.cache_len) : 0;
         int seen = 0x7fffffff, before_local = 0x7fffffff;
 #pragma unroll
-        for (int t = 0; t < kTokPerWave; ++t) {
+        for (int t = 0; t < kTok; ++t) {
             const int64_t row = static_cast<int64_t>(q0) + tok0 + t;
             out_rows[t] = kPool ? p.score + (static_cast<int64_t>(h) * p.score_head_stride + row * p.pool_len)
                                 : p.score + h * p.score_head_stride + row * p.score_row_stride;
@@ -377,40 +388,44 @@ void stage1_kernel(const Stage1Params p) {
 
     // A plain tile's results are stored when the next tile begins: the wait at a tile's end counts stores too, and one just
     // issued would add its round trip to every tile.
-    float held[kTokPerWave] = {0.f, 0.f};
+    float held[kTok] = {};
     bool pending = false;
     auto store = [&](int t, uint32_t at, elem_bits value) {
-        if constexpr (kItems > 0) pooled[wave * kTokPerWave + t][at] = value;
+        if constexpr (kItems > 0) pooled[wave * kTok + t][at] = value;
         else out_rows[t][at] = value;
     };
     auto store_held = [&](int ti) {
         const uint32_t at = static_cast<uint32_t>(kPool ? ti * 16 + (lane >> 2) : ti * 64 + lane);
         if (!kPool || (lane & 3) == 0) {
 #pragma unroll
-            for (int t = 0; t < kTokPerWave; ++t) store(t, at, f32_to_elem_hw(held[t]));
+            for (int t = 0; t < kTok; ++t) store(t, at, f32_to_elem_hw(held[t]));
         }
     };
     for (int ti = begin_f; ti < end_f; ++ti) {
         if (pending) store_held(ti - 1);                       // uniform per wavefront
         if (ti + 1 < end_f) issue_tile(kbase, k_stride, k_off, (ti + 1) * 64, Lk, lds_tiles + ((ti + 1) & 1) * 16384, wave_u, n, g);
+        if (!live[0]) {
+            tile_done();
+            continue;
+        }
         const uint4* cur = tile[ti & 1];
-        float part[kTokPerWave][4];                            // [t][kt]: this lane's four heads summed, key 16 kt + n
+        float part[kTok][4];                                   // [t][kt]: this lane's four heads summed, key 16 kt + n
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
-            floatx4 s[kTokPerWave];
+            floatx4 s[kTok];
 #pragma unroll
-            for (int t = 0; t < kTokPerWave; ++t) s[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < kTok; ++t) s[t] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 const uint4 raw = cur[(kt * 4 + c) * 64 + lane];
                 elem8 kf;
                 __builtin_memcpy(&kf, &raw, 16);
 #pragma unroll
-                for (int t = 0; t < kTokPerWave; ++t)
+                for (int t = 0; t < kTok; ++t)
                     s[t] = IV2_MFMA(qf[t][c], kf, s[t], 0, 0, 0);
             }
 #pragma unroll
-            for (int t = 0; t < kTokPerWave; ++t) {
+            for (int t = 0; t < kTok; ++t) {
                 float sum = 0.f;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) sum += __builtin_amdgcn_exp2f(s[t][e] * p.scale_log2 - lse2[t][e]);
@@ -419,41 +434,45 @@ void stage1_kernel(const Stage1Params p) {
         }
         // sum over the four 16-lane rows (the head groups) and hand row kt the total of key tile kt, in three
         // exchanges: (row0 + row1 | row2 + row3) of tiles 0/1 and of tiles 2/3, then the two halves.  lane = 16*g + n  <->  key 16*g + n of this tile
-        float mine[kTokPerWave];
+        float mine[kTok];
 #pragma unroll
-        for (int t = 0; t < kTokPerWave; ++t)
+        for (int t = 0; t < kTok; ++t)
             mine[t] = fold_rows32(fold_rows16(part[t][0], part[t][1]), fold_rows16(part[t][2], part[t][3]));
         const bool mine_too = !kShared || !kPool || ti >= first_f;                   // not the tile before
         pending = ti >= plain_first && ti < plain_end && mine_too;
         const int col = ti * 64 + lane;
         if (!pending) {
 #pragma unroll
-            for (int t = 0; t < kTokPerWave; ++t) mine[t] = col < vis_f[t] ? mine[t] : 0.f;     // keys the token may not see score 0
+            for (int t = 0; t < kTok; ++t) mine[t] = col < vis_f[t] ? mine[t] : 0.f;     // keys the token may not see score 0
         }
         if (!kPool) {
 #pragma unroll
-            for (int t = 0; t < kTokPerWave; ++t) {
+            for (int t = 0; t < kTok; ++t) {
                 held[t] = mine[t];
                 if (!pending && live[t] && col < p.score_cols) out_rows[t][col] = f32_to_elem_hw(mine[t]);
             }
         } else {
             // block kb = col / 4 pools keys 4 kb - 1 .. 4 kb + 3: its quad and the last key of the quad before
-            pool_quads(mine[0], mine[1], prev[0], prev[1], held[0], held[1]);
+            if constexpr (kTok == 2) {
+                pool_quads(mine[0], mine[1], prev[0], prev[1], held[0], held[1]);
+            } else {
+                float same;
+                pool_quads(mine[0], mine[0], prev[0], prev[0], held[0], same);
+            }
             const int kb = col >> 2;
 #pragma unroll
-            for (int t = 0; t < kTokPerWave; ++t) {
+            for (int t = 0; t < kTok; ++t) {
                 prev[t] = mine[t];
                 if (!pending && mine_too && live[t] && (lane & 3) == 0 && kb < p.pool_len) store(t, kb, pool_rest(kb, bq[t], held[t]));
             }
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
+        tile_done();
     }
     if (pending) store_held(end_f - 1);
     if (kShared && end_f < tiles_f) return;                // uniform per workgroup; the rest is the last one's
     // columns no tile covered
 #pragma unroll
-    for (int t = 0; t < kTokPerWave; ++t) {
+    for (int t = 0; t < kTok; ++t) {
         if (!live[t]) continue;
         if (!kPool) {
             for (int col = tiles_f * 64 + lane; col < p.score_cols; col += 64) out_rows[t][col] = 0;
@@ -468,14 +487,14 @@ void stage1_kernel(const Stage1Params p) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        uint32_t key[kTokPerWave][kItems];                     // 0: no column
+        uint32_t key[kTok][kItems];                     // 0: no column
         const int take_at_most = p.topk < p.pool_len ? p.topk : p.pool_len;
 #pragma unroll
-        for (int t = 0; t < kTokPerWave; ++t)
+        for (int t = 0; t < kTok; ++t)
 #pragma unroll
             for (int e = 0; e < kItems; ++e) {
                 const int kb = 64 * e + lane;
-                key[t][e] = kb < p.pool_len ? sortable16(pooled[wave * kTokPerWave + t][kb]) : 0u;
+                key[t][e] = kb < p.pool_len ? sortable16(pooled[wave * kTok + t][kb]) : 0u;
             }
         auto count = [&](int t, auto&& in) {
             int c = 0;
@@ -483,18 +502,18 @@ void stage1_kernel(const Stage1Params p) {
             for (int e = 0; e < kItems; ++e) c += __builtin_popcountll(__builtin_amdgcn_ballot_w64(in(key[t][e])));
             return c;
         };
-        uint32_t thr[kTokPerWave];                             // the largest key that so many keys reach
+        uint32_t thr[kTok];                             // the largest key that so many keys reach
 #pragma unroll
-        for (int t = 0; t < kTokPerWave; ++t) thr[t] = 0;
+        for (int t = 0; t < kTok; ++t) thr[t] = 0;
 #pragma unroll
         for (int bit = 15; bit >= 0; --bit)
 #pragma unroll
-            for (int t = 0; t < kTokPerWave; ++t) {
+            for (int t = 0; t < kTok; ++t) {
                 const uint32_t next = thr[t] | (1u << bit);
                 thr[t] = count(t, [&](uint32_t x) { return x >= next; }) >= take_at_most ? next : thr[t];
             }
 #pragma unroll
-        for (int t = 0; t < kTokPerWave; ++t) {
+        for (int t = 0; t < kTok; ++t) {
             if (!live[t]) continue;
             int ties = take_at_most - count(t, [&](uint32_t x) { return x > thr[t]; });          // of the keys equal to it
             uint64_t words = 0ull;                             // lane w: word w
@@ -574,19 +593,27 @@ int launch_stage1(const char* who, void* stream, const void* q, const void* k, c
     const int64_t wgs = static_cast<int64_t>((max_seqlen_q + kTokPerBlock - 1) / kTokPerBlock) * batch * num_heads_k;
     const int64_t fill = wgs > 0 ? 256 / wgs : 1, most = max_seqlen_k / 256;
     p.splits = p.mask != nullptr || fill < 2 || most < 2 ? 1 : static_cast<int>(fill < most ? fill : most);
-    const dim3 grid((max_seqlen_q + kTokPerBlock - 1) / kTokPerBlock * p.splits, batch, num_heads_k);
+    // One token to a wavefront, twice the workgroups, up to 384 of the others: fewer than one and a half to a CU that holds two.  The time is then that of the CU with the most, half a
+    // workgroup finer, and of the chain of one tile (one wavefront's products and exponentials behind the other's on a SIMD), which is shorter.  Scores alone, us, two tokens | one, 2 KV heads, 20 011 keys:
+    // 17 queries 18.8 | 12.5, 256 19.3 | 13.3, 512 20.1 | 20.6, 1100 35.1 | 32.9, 2049 54.0 | 49.7, 3000 (376 workgroups) 56.1 | 51.1; 3500 (438) 57.2 | 62.8, 4096 60.3 | 64.1; 60 000
+    // keys, one head, 2049 89.6 | 73.5; selecting prefill of 1000 tokens 15.2 | 12.4, 2048 17.1 | 15.8, 3000 22.4 | 21.5.
+    constexpr int64_t kOneTokenWorkgroups = 384;
+    const bool one = wgs <= kOneTokenWorkgroups;
+    const int tokens = one ? kWavesS1 : kTokPerBlock;
+    const dim3 grid((max_seqlen_q + tokens - 1) / tokens * p.splits, batch, num_heads_k);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (p.mask) {
-        auto kernel = p.pool_len <= 64 ? stage1_kernel<true, true, 1> : p.pool_len <= 128 ? stage1_kernel<true, true, 2> : p.pool_len <= 256 ? stage1_kernel<true, true, 4> : stage1_kernel<true, true, 8>;
-        hipLaunchKernelGGL(kernel, grid, dim3(64 * kWavesS1), 0, st, p);
-    } else {
+    auto pick = [&](auto tok) {
+        constexpr int kTok = decltype(tok)::value;
+        if (p.mask) return p.pool_len <= 64 ? stage1_kernel<true, true, 1, false, kTok> : p.pool_len <= 128 ? stage1_kernel<true, true, 2, false, kTok>
+                         : p.pool_len <= 256 ? stage1_kernel<true, true, 4, false, kTok> : stage1_kernel<true, true, 8, false, kTok>;
         const bool shared = p.splits > 1;
-        auto kernel = pool ? (is_causal ? (shared ? stage1_kernel<true, true, 0, true> : stage1_kernel<true, true>)
-                                        : (shared ? stage1_kernel<false, true, 0, true> : stage1_kernel<false, true>))
-                           : (is_causal ? (shared ? stage1_kernel<true, false, 0, true> : stage1_kernel<true, false>)
-                                        : (shared ? stage1_kernel<false, false, 0, true> : stage1_kernel<false, false>));
-        hipLaunchKernelGGL(kernel, grid, dim3(64 * kWavesS1), 0, st, p);
-    }
+        return pool ? (is_causal ? (shared ? stage1_kernel<true, true, 0, true, kTok> : stage1_kernel<true, true, 0, false, kTok>)
+                                 : (shared ? stage1_kernel<false, true, 0, true, kTok> : stage1_kernel<false, true, 0, false, kTok>))
+                    : (is_causal ? (shared ? stage1_kernel<true, false, 0, true, kTok> : stage1_kernel<true, false, 0, false, kTok>)
+                                 : (shared ? stage1_kernel<false, false, 0, true, kTok> : stage1_kernel<false, false, 0, false, kTok>));
+    };
+    auto kernel = one ? pick(std::integral_constant<int, 1>{}) : pick(std::integral_constant<int, kTokPerWave>{});
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * kWavesS1), 0, st, p);
     IV2_LAUNCH_CHECK();
     return 0;
 }
