@@ -49,6 +49,7 @@ struct HybridExtra {
     int groups_per_seq;                                        // ceil(max_seqlen_q / kHybTokens)
     int batch;
     int total_groups;                                          // num_heads_k * batch * groups_per_seq
+    int late;                                                  // short groups that go last: num_heads_k * batch, or 0
     int mask_words;                                            // words per LDS mask row: what max_seqlen_k needs, not the maximum
     unsigned* finished;                                        // the XCDs' counters of in_step.h, or null: no workgroup waits
 };
@@ -133,15 +134,22 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     unsigned long long* com = reinterpret_cast<unsigned long long*>(smem_raw + kRingTiles * kTileBytes);   // [mask_words]
     unsigned long long* rows = com + x.mask_words;                                  // [kHybTokens][mask_words]
 
-    // ---- which tokens: XCD-chunked, heaviest first ----
+    // ---- which tokens: XCD-chunked, heaviest first (x.late: but the last group of every sequence at the end) ----
     const int bid = blockIdx.x;
     // (few groups are few chunks: two parts to an XCD fill its CUs, the next two go to another)
     const int xcd = (kParts <= 2 ? bid : bid - 16 / kParts * (static_cast<int>(blockIdx.y) >> 1)) & 7, sidx = bid >> 3;
     int G = ((sidx / kHybChunk) * 8 + xcd) * kHybChunk + (sidx % kHybChunk);
     if (G >= x.total_groups) return;                                                // uniform per workgroup
-    G = x.total_groups - 1 - G;
-    const int grp = G % x.groups_per_seq;
-    const int hb = G / x.groups_per_seq;
+    int grp, hb;
+    if (kParts == 1 && G >= x.total_groups - x.late) {
+        grp = x.groups_per_seq - 1;
+        hb = G - (x.total_groups - x.late);
+    } else {
+        G = x.total_groups - x.late - 1 - G;
+        const int each = x.groups_per_seq - (x.late != 0 ? 1 : 0);
+        grp = G % each;
+        hb = G / each;
+    }
     const int b = hb % x.batch, h = hb / x.batch;
 
     const int tid = threadIdx.x;
@@ -450,7 +458,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     }
 }
 
-static int launch_groups(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q, int max_seqlen_k, bool causal, unsigned* in_step) {
+static int launch_groups(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q, int max_seqlen_k, bool causal, int most_selected, unsigned* in_step) {
     HybridExtra x{};
     x.batch = batch;
     x.groups_per_seq = (max_seqlen_q + kHybTokens - 1) / kHybTokens;
@@ -465,7 +473,7 @@ static int launch_groups(hipStream_t st, const FwdParams& p, int batch, int num_
             some.cu_seqlens_k += b;
             some.kimg += static_cast<int64_t>(b) * kImageElems;               // a sequence's first image: image_slot0
             some.vimg += static_cast<int64_t>(b) * kImageElems;
-            if (int rc = launch_groups(st, some, batch - b < fit ? batch - b : fit, num_heads_k, max_seqlen_q, max_seqlen_k, causal, in_step)) return rc;
+            if (int rc = launch_groups(st, some, batch - b < fit ? batch - b : fit, num_heads_k, max_seqlen_q, max_seqlen_k, causal, most_selected, in_step)) return rc;
         }
         return 0;
     }
@@ -486,6 +494,14 @@ static int launch_groups(hipStream_t st, const FwdParams& p, int batch, int num_
     // depend on the number of parts.
     const int parts = total * 2 > 256 ? 1 : total * 4 > 256 ? 2 : total * 8 > 256 ? 4 : 8;
     x.finished = parts > 1 ? nullptr : in_step;
+    // Heaviest first is also longest prefix first, which puts the one short group of a chunk of queries in front.  Where the chunk's groups are alike, with at least twice as many
+    // blocks behind the first of them as a row selects, it holds up a CU that then has as many whole groups to walk as the others, and goes last instead.  Forward with the images in us, first | last, 2 KV heads, 2049
+    // queries, 64 blocks: behind 8192 keys 215 | 208, 17 962 234 | 212 (2048 of them 197), 40 960 312 | 238; 32 blocks behind 4096 114 | 114, 12 288 133 | 121; 16 behind 2048 68.6 | 69.0, 10 240 81.2 | 78.0;
+    // 4097 queries, 64 blocks, behind 15 914 432 | 391.  Where the groups do not fill whole rounds, 1412 to 3500 queries, the same within 0.6 %.  With fewer blocks behind them last is slower: 64 blocks
+    // behind 4096 175 | 187, behind none 332 | 359 (6145 queries).
+    const int over = max_seqlen_q % kHybTokens;
+    const int64_t held = static_cast<int64_t>(max_seqlen_k) - max_seqlen_q, selected = most_selected < 0 ? -static_cast<int64_t>(most_selected) : most_selected;
+    if (parts == 1 && over > 0 && over <= 4 && x.groups_per_seq > 1 && selected > 0 && held >= 2 * kBlockN * selected) x.late = num_heads_k * batch;
     auto pick = [&](auto n) {
         constexpr int kParts = decltype(n)::value;
         return causal ? (far ? stage2_fwd_hybrid_kernel<true, true, kParts> : stage2_fwd_hybrid_kernel<true, false, kParts>)
@@ -506,7 +522,7 @@ int launch_stage2_fwd_hybrid(hipStream_t st, const FwdParams& p, int batch, int 
         ? dense_tiles_pay(batch, num_heads_k, p.group, p.total_q, p.total_k, max_seqlen_q, max_seqlen_k, causal)
         : masked_by_tiles(most_selected);
     return tiles ? launch_stage2_fwd_tile(st, p, batch, num_heads_k, max_seqlen_q, max_seqlen_k, causal)
-                 : launch_groups(st, p, batch, num_heads_k, max_seqlen_q, max_seqlen_k, causal, in_step);
+                 : launch_groups(st, p, batch, num_heads_k, max_seqlen_q, max_seqlen_k, causal, most_selected, in_step);
 }
 
 }  // namespace IV2_NS
