@@ -273,6 +273,18 @@ int infllmv2_decode_step_scores(void* stream, const void* q, const void* k_new, 
                                 int stride_f, int kernel_size_c, int stride_c, float softmax_scale, int out_len,
                                 int local_blocks, int init_blocks);
 
+/* A whole decode step that selects every block (of max_len tokens at most): what infllmv2_decode_step_scores keeps (same arguments, no
+ * scores), and infllmv2_fwd_kvcache without a mask on the caches with the new row (q, out: strides {batch, head}; workspace:
+ * infllmv2_fwd_kvcache_workspace_bytes), in two launches, with one split in one.  batch x num_heads_k x num_splits must not exceed 256. */
+int infllmv2_decode_step_all(void* stream, const void* q, const void* k_new, const void* v_new, void* kcache, void* vcache,
+                             void* fine_cache, void* coarse_cache, const int32_t* lens, int host_len, int32_t* new_lens,
+                             int32_t* fine_lens, int32_t* coarse_lens, void* out, float* softmax_lse, void* workspace,
+                             size_t workspace_bytes, int batch, int num_heads, int num_heads_k, int head_dim, int capacity,
+                             int fine_rows, int coarse_rows, int max_len, const int64_t* q_strides, const int64_t* knew_strides,
+                             const int64_t* vnew_strides, const int64_t* kcache_strides, const int64_t* vcache_strides,
+                             const int64_t* fine_strides, const int64_t* coarse_strides, const int64_t* o_strides, int kernel_size_f,
+                             int stride_f, int kernel_size_c, int stride_c, int num_splits, float softmax_scale);
+
 /* ---- Stage 2: block-sparse attention -------------------------------------------------------- */
 
 /* Scratch needed by infllmv2_varlen_fwd / _bwd for the fragment-major K/V block images. */
@@ -534,6 +546,14 @@ int infllmv2_decode_step_scores_f16(void* stream, const void* q, const void* k_n
                                 const int64_t* fine_strides, const int64_t* coarse_strides, int kernel_size_f,
                                 int stride_f, int kernel_size_c, int stride_c, float softmax_scale, int out_len,
                                 int local_blocks, int init_blocks);
+int infllmv2_decode_step_all_f16(void* stream, const void* q, const void* k_new, const void* v_new, void* kcache, void* vcache,
+                             void* fine_cache, void* coarse_cache, const int32_t* lens, int host_len, int32_t* new_lens,
+                             int32_t* fine_lens, int32_t* coarse_lens, void* out, float* softmax_lse, void* workspace,
+                             size_t workspace_bytes, int batch, int num_heads, int num_heads_k, int head_dim, int capacity,
+                             int fine_rows, int coarse_rows, int max_len, const int64_t* q_strides, const int64_t* knew_strides,
+                             const int64_t* vnew_strides, const int64_t* kcache_strides, const int64_t* vcache_strides,
+                             const int64_t* fine_strides, const int64_t* coarse_strides, const int64_t* o_strides, int kernel_size_f,
+                             int stride_f, int kernel_size_c, int stride_c, int num_splits, float softmax_scale);
 int infllmv2_stage1_decode_f16(void* stream, const void* q, const void* k, const void* v, void* out,
                                const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, const int32_t* k_lens,
                                const int32_t* cu_seqlens_v, const int32_t* v_lens, void* workspace,

@@ -40,6 +40,7 @@ SIGNATURES = {
     "infllmv2_varlen_fwd_stage1_pooled": [_p] * 9 + [_i, _i, _i64, _i, _i, _i, _i, _i, _p, _p, _p, _i, _f] + [_i] * 7,
     "infllmv2_varlen_fwd_stage1_selected": [_p] * 8 + [_i, _i64, _i, _i, _i, _i, _i, _p, _p, _p, _i, _f] + [_i] * 8,
     "infllmv2_stage1_decode": [_p] * 11 + [_sz] + [_i] * 6 + [_p] * 3 + [_i64, _i64, _f, _i, _i, _p] + [_i] * 8,
+    "infllmv2_decode_step_all": [_p] * 9 + [_i] + [_p] * 6 + [_sz] + [_i] * 8 + [_p] * 8 + [_i] * 5 + [_f],
     "infllmv2_decode_step_scores": [_p] * 9 + [_i] + [_p] * 5 + [_sz] + [_i] * 8 + [_p] * 7 + [_i] * 4 + [_f, _i, _i, _i],
     "infllmv2_varlen_fwd": [_p, _p, _p, _p, _p, _p, _p, _p, _p, _p, _sz, _i, _i, _i64, _i64, _i, _i, _i, _i, _i,
                             _p, _p, _p, _p, _p, _i, _f, _i],
@@ -56,7 +57,7 @@ SIGNATURES = {
 }
 # entry points that exist once per element type: the plain name takes bfloat16, name + "_f16" IEEE half
 PER_ELEMENT_TYPE = ["infllmv2_compress_keys", "infllmv2_compress_keys_pair", "infllmv2_compress_keys_and_pack", "infllmv2_compress_keys_cache", "infllmv2_compress_keys_cache_pair", "infllmv2_varlen_fwd_stage1",
-                    "infllmv2_varlen_fwd_stage1_pooled", "infllmv2_varlen_fwd_stage1_selected", "infllmv2_stage1_decode", "infllmv2_decode_step_scores", "infllmv2_varlen_fwd",
+                    "infllmv2_varlen_fwd_stage1_pooled", "infllmv2_varlen_fwd_stage1_selected", "infllmv2_stage1_decode", "infllmv2_decode_step_scores", "infllmv2_decode_step_all", "infllmv2_varlen_fwd",
                     "infllmv2_varlen_fwd_selected",
                     "infllmv2_varlen_bwd", "infllmv2_varlen_bwd_selected", "infllmv2_fwd_kvcache", "infllmv2_fwd_kvcache_topk",
                     "infllmv2_fwd_kvcache_scores"]

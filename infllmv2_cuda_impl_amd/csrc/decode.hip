@@ -16,6 +16,7 @@
 // over d), V, which is contracted over keys, by transposing reads.  Partial results are merged by a small combine kernel.
 #include "common.h"
 #include "block_walker.h"
+#include "decode_step.h"
 #include "infllmv2_hip.h"
 #include <math.h>
 #include <mutex>
@@ -32,12 +33,13 @@ struct DecodeParams {
     float* lse;                     // (batch, Hq)
     float* o_part;                  // (batch, Hk, splits, 16, 128) fp32, normalised per split
     float* lse_part;                // (batch, Hk, splits, 16)
-    const int* cache_seqlens;       // null: every sequence fills the whole cache
+    const int* cache_seqlens;       // null: every sequence holds `held` tokens
+    int held;
     const uint64_t* mask;           // (batch, Hk, n64) or null
     const int* topk_idx;            // (batch, Hk, k_idx): the selection as an index list instead (-1: unused slot), or null
     int k_idx;
     const elem_bits* scores;         // (batch, Hk, n_scores) block scores: the selection is their k_select largest; or null
-    int n_scores, k_select;
+    int n_scores, k_select;         // (a whole step: blocks of a row at most)
     int64_t q_batch, q_head;        // element strides of q (batch, head); head dim dense
     int64_t o_batch, o_head;
     int64_t kc_batch, kc_row, kc_head, vc_batch, vc_row, vc_head;
@@ -319,9 +321,21 @@ __device__ __forceinline__ uint64_t select_words(const elem_bits* row, int n, in
 }
 
 // kSelect (four wavefronts only): the selection is made here, from block scores
-template <bool kDirect, int kWaves, bool kSelect>
+// Keep (four wavefronts only): a whole step that selects every block, so that nothing has to come before the attention.  One workgroup more per (sequence, KV
+// head), or the last split's where that would be a second round, keeps the lengths and the compressed keys, which no other looks at; the new row is appended as
+// above.  Steps of the layer in us, launches for the front, the scores, the attention and the merge | for the front, the attention and the merge | this and the
+// merge, 2 KV heads, 64 blocks selected: one sequence of 4000 tokens 19.0 | 15.2 | 10.6 (all the host's), 16 of up to 4000 23.2 | 15.9 | 13.7, 32 of 2000 26.4 | 18.6 |
+// 16.7 (with workgroups for the keepers alone 21.7), 64 of 1500 29.9 | 22.4 | 21.0 (27.4).
+struct NoKeep {};
+struct KeepStep {
+    S1DecodeStep step;
+    S1DecodeStrides strides;
+};
+template <bool kDirect, int kWaves, bool kSelect, typename Keep = NoKeep>
 __global__ __launch_bounds__(64 * kWaves)
-void decode_split_kernel(const DecodeParams p) {
+void decode_split_kernel(const DecodeParams p, const Keep keep) {
+    constexpr bool kKeep = std::is_same<Keep, KeepStep>::value;
+    static_assert(kWaves == 4 || !(kSelect || kKeep), "by four wavefronts");
     constexpr int kSlots = kWaves == 1 ? 2 : 1;                // block tiles per wavefront
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
     __shared__ __attribute__((aligned(16))) elem_bits new_row[2 * kHeadDim];        // K, then V
@@ -332,6 +346,20 @@ void decode_split_kernel(const DecodeParams p) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
     const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+    auto keep_caches = [&]() {
+        if constexpr (kKeep) {
+            const S1DecodeStep& t = keep.step;
+            const int len = t.lens ? t.lens[b] : t.host_len;
+            int add_f, add_c;
+            const int rows_f = s1d_step_rows(len, t.capacity, t.kernel_f, t.stride_f, t.fine_capacity, add_f);
+            const int rows_c = s1d_step_rows(len, t.capacity, t.kernel_c, t.stride_c, t.coarse_capacity, add_c);
+            s1d_keep_caches(keep.strides, t, b, h, len, rows_f, rows_c, add_f, add_c, tid, false, true, kHeadDim);
+        }
+    };
+    if (kKeep && split == p.splits) {                          // uniform over the workgroup
+        keep_caches();
+        return;
+    }
     unsigned char* tiles = smem + wave * kSlots * kSlotBytes;
     const int64_t pair = static_cast<int64_t>(b) * p.num_heads_k + h;
     const bool listed = kSelect || p.mask != nullptr || p.topk_idx != nullptr;      // else: every block
@@ -339,7 +367,7 @@ void decode_split_kernel(const DecodeParams p) {
     int first_idx = -1;                                        // or list entry `lane`
     if (!kSelect && p.mask != nullptr && lane < p.n64) bits0 = p.mask[pair * p.n64 + lane];
     if (!kSelect && p.topk_idx != nullptr && lane < p.k_idx) first_idx = p.topk_idx[pair * p.k_idx + lane];
-    const int seqlen = p.cache_seqlens ? p.cache_seqlens[b] : p.capacity - p.seqlen_new;
+    const int seqlen = p.cache_seqlens ? p.cache_seqlens[b] : p.held;
     const int lp = p.leftpad ? p.leftpad[b] : 0;              // the sequence's key 0 is cache row lp
     // position of the first appended key; a full cache takes no key, and the tables need not reach beyond it
     const int rot_pos = !p.cache_seqlens ? 0 : (seqlen < p.capacity ? seqlen : p.capacity - 1);
@@ -418,6 +446,7 @@ void decode_split_kernel(const DecodeParams p) {
         lds_fence();
     } else if (!listed) {
         total = last_blk + 1;
+        if (kKeep && total > p.n_scores) total = p.n_scores;   // a longer sequence than was announced
         lds_fence();
     } else {
         if (p.mask != nullptr && n_words <= 64) {              // straight into registers
@@ -716,6 +745,7 @@ void decode_split_kernel(const DecodeParams p) {
                 *reinterpret_cast<float4*>(op + 4) = make_float4(acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv);
             }
         }
+        if (kKeep && static_cast<int>(gridDim.x) == p.splits && split == p.splits - 1) keep_caches();      // no workgroup of their own
         return;
     }
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
@@ -843,7 +873,7 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
                                     int num_splits, float softmax_scale, const int32_t* cache_batch_idx,
                                     const int32_t* cache_leftpad, const int32_t* block_table,
                                     int64_t block_table_batch_stride, int page_block_size, const void* rotary_cos,
-                                    const void* rotary_sin, int rotary_dim, int rotary_interleaved) {
+                                    const void* rotary_sin, int rotary_dim, int rotary_interleaved, const KeepStep* keep = nullptr) {
     IV2_CHECK(head_dim == kHeadDim, "fwd_kvcache: this build only supports head_dim 128 (got %d)", head_dim);
     IV2_CHECK(seqlen_q == 1, "fwd_kvcache: this build only supports one query token per sequence (got %d)", seqlen_q);
     IV2_CHECK(valid_group(num_heads, num_heads_k),
@@ -900,6 +930,7 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
     p.batch = batch; p.num_heads_k = num_heads_k; p.capacity = cache_capacity;
     p.group = num_heads / num_heads_k;
     p.seqlen_new = k_new ? seqlen_new : 0;
+    p.held = keep ? keep->step.host_len : cache_capacity - p.seqlen_new;
     p.n64 = n_uint64_per_row; p.splits = num_splits;
     p.scale_log2 = softmax_scale * 1.44269504088896340736f;
     p.cache_batch_idx = cache_batch_idx; p.leftpad = cache_leftpad;
@@ -917,7 +948,9 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
         p.mask_in_place = 1;
         words = 0;
     }
-    const bool grouped = static_cast<int64_t>(batch) * num_heads_k * num_splits <= kGroupedWorkgroups && words <= 2048 && !p.mask_in_place;
+    const int64_t pairs = static_cast<int64_t>(batch) * num_heads_k;
+    const bool grouped = pairs * num_splits <= kGroupedWorkgroups && words <= 2048 && !p.mask_in_place;
+    IV2_CHECK(keep == nullptr || grouped, "decode_step_all: at most %d (sequence, KV head, split) triples are served", kGroupedWorkgroups);
     IV2_CHECK(scores == nullptr || (grouped && n_scores > 0 && n_scores <= INFLLMV2_DECODE_MAX_SCORES && k_select > 0),
               "fwd_kvcache_scores: 1 to %d block scores per row, topk >= 1 and at most %d (sequence, KV head, split) triples are served",
               INFLLMV2_DECODE_MAX_SCORES, kGroupedWorkgroups);
@@ -931,7 +964,7 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
         p.kn_batch = knew_strides[0]; p.kn_row = knew_strides[1]; p.kn_head = knew_strides[2];
         p.vn_batch = vnew_strides[0]; p.vn_row = vnew_strides[1]; p.vn_head = vnew_strides[2];
         // one new row at a known place: the split kernel takes care of it (one launch less, and no wait for it)
-        p.append_here = seqlen_new == 1 && cache_seqlens != nullptr ? 1 : 0;
+        p.append_here = seqlen_new == 1 && (cache_seqlens != nullptr || keep != nullptr) ? 1 : 0;
         if (!p.append_here) {
             const int64_t total = static_cast<int64_t>(batch) * seqlen_new * num_heads_k * 16;
             hipLaunchKernelGGL(decode_append_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, st, p);
@@ -943,14 +976,19 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
         p.o_part = ws;
         p.lse_part = ws + static_cast<size_t>(batch) * num_heads_k * num_splits * 16 * kHeadDim;
     }
-    void (*split_kernel)(DecodeParams);
-    if (scores != nullptr) split_kernel = num_splits == 1 ? decode_split_kernel<true, 4, true> : decode_split_kernel<false, 4, true>;
-    else if (grouped) split_kernel = num_splits == 1 ? decode_split_kernel<true, 4, false> : decode_split_kernel<false, 4, false>;
-    else split_kernel = num_splits == 1 ? decode_split_kernel<true, 1, false> : decode_split_kernel<false, 1, false>;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(split_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-    IV2_CHECK(e == hipSuccess, "fwd_kvcache: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
-    hipLaunchKernelGGL(split_kernel, dim3(num_splits, num_heads_k, batch), dim3(grouped ? 256 : 64), lds, st, p);
-    IV2_LAUNCH_CHECK();
+    auto launch = [&](auto kernel, auto with, int workgroups) -> int {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+        IV2_CHECK(e == hipSuccess, "fwd_kvcache: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
+        hipLaunchKernelGGL(kernel, dim3(workgroups, num_heads_k, batch), dim3(grouped ? 256 : 64), lds, st, p, with);
+        IV2_LAUNCH_CHECK();
+        return 0;
+    };
+    int rc;
+    if (keep != nullptr) rc = launch(num_splits == 1 ? decode_split_kernel<true, 4, false, KeepStep> : decode_split_kernel<false, 4, false, KeepStep>, *keep, num_splits + (pairs * (num_splits + 1) <= kGroupedWorkgroups ? 1 : 0));
+    else if (scores != nullptr) rc = launch(num_splits == 1 ? decode_split_kernel<true, 4, true> : decode_split_kernel<false, 4, true>, NoKeep{}, num_splits);
+    else if (grouped) rc = launch(num_splits == 1 ? decode_split_kernel<true, 4, false> : decode_split_kernel<false, 4, false>, NoKeep{}, num_splits);
+    else rc = launch(num_splits == 1 ? decode_split_kernel<true, 1, false> : decode_split_kernel<false, 1, false>, NoKeep{}, num_splits);
+    if (rc != 0) return rc;
     if (num_splits > 1) {
         const CombineParams c{p.o_part, p.lse_part, p.out, p.lse, p.o_batch, p.o_head, num_heads_k, num_splits, p.group};
         const dim3 cgrid((p.group + kCombineWaves - 1) / kCombineWaves, num_heads_k, batch), cblock(64 * kCombineWaves);
@@ -1011,6 +1049,43 @@ extern "C" int IV2_ENTRY(infllmv2_fwd_kvcache_scores)(void* stream, const void* 
                             n_scores, topk, workspace, workspace_bytes, batch, 1, num_heads, num_heads_k, head_dim, cache_capacity, 0,
                             q_strides, kcache_strides, vcache_strides, none, none, o_strides, 0, num_splits, softmax_scale, nullptr,
                             nullptr, nullptr, 0, 0, nullptr, nullptr, 0, 0);
+}
+
+extern "C" int IV2_ENTRY(infllmv2_decode_step_all)(void* stream, const void* q, const void* k_new, const void* v_new, void* kcache, void* vcache,
+                                      void* fine_cache, void* coarse_cache, const int32_t* lens, int host_len, int32_t* new_lens,
+                                      int32_t* fine_lens, int32_t* coarse_lens, void* out, float* softmax_lse, void* workspace, size_t workspace_bytes,
+                                      int batch, int num_heads, int num_heads_k, int head_dim, int capacity, int fine_rows, int coarse_rows, int max_len,
+                                      const int64_t* q_strides, const int64_t* knew_strides, const int64_t* vnew_strides, const int64_t* kcache_strides,
+                                      const int64_t* vcache_strides, const int64_t* fine_strides, const int64_t* coarse_strides, const int64_t* o_strides,
+                                      int kernel_size_f, int stride_f, int kernel_size_c, int stride_c, int num_splits, float softmax_scale) {
+    const char* who = "decode_step_all";
+    IV2_CHECK(k_new && v_new && fine_cache && coarse_cache && fine_lens && coarse_lens, "%s: null pointer", who);
+    IV2_CHECK(fine_rows > 0 && coarse_rows > 0 && max_len > 0 && host_len >= 0, "%s: bad sizes", who);
+    IV2_CHECK(kernel_size_f > 0 && stride_f > 0 && kernel_size_c > 0 && stride_c > 0, "%s: kernel_size and stride must be positive", who);
+    IV2_CHECK(reinterpret_cast<uintptr_t>(fine_cache) % 16 == 0 && reinterpret_cast<uintptr_t>(coarse_cache) % 16 == 0, "%s: tensors must be 16-byte aligned", who);
+    for (int s = 0; s < 3; ++s)
+        IV2_CHECK(fine_strides[s] % 8 == 0 && coarse_strides[s] % 8 == 0, "%s: strides must be multiples of 8 elements", who);
+    KeepStep keep{};
+    S1DecodeStep& t = keep.step;
+    t.knew = static_cast<const elem_bits*>(k_new);
+    t.vnew = static_cast<const elem_bits*>(v_new);
+    t.kcache = static_cast<elem_bits*>(kcache);
+    t.vcache = static_cast<elem_bits*>(vcache);
+    t.fine = static_cast<elem_bits*>(fine_cache);
+    t.coarse = static_cast<elem_bits*>(coarse_cache);
+    t.kn_batch = knew_strides[0]; t.kn_head = knew_strides[1]; t.vn_batch = vnew_strides[0]; t.vn_head = vnew_strides[1];
+    t.kc_batch = kcache_strides[0]; t.kc_row = kcache_strides[1]; t.kc_head = kcache_strides[2];
+    t.vc_batch = vcache_strides[0]; t.vc_row = vcache_strides[1]; t.vc_head = vcache_strides[2];
+    t.lens = lens; t.host_len = host_len;
+    t.new_lens = new_lens; t.fine_lens = fine_lens; t.coarse_lens = coarse_lens;
+    t.capacity = capacity; t.fine_capacity = fine_rows; t.coarse_capacity = coarse_rows;
+    t.kernel_f = kernel_size_f; t.stride_f = stride_f; t.kernel_c = kernel_size_c; t.stride_c = stride_c;
+    keep.strides = {fine_strides[0], fine_strides[1], fine_strides[2], coarse_strides[0], coarse_strides[1], coarse_strides[2]};
+    const int64_t kn[3] = {knew_strides[0], 0, knew_strides[1]}, vn[3] = {vnew_strides[0], 0, vnew_strides[1]};     // of the one row
+    return fwd_kvcache_impl(stream, q, kcache, vcache, k_new, v_new, lens, out, softmax_lse, nullptr, nullptr, 0, nullptr,
+                            (max_len + kBlockN - 1) / kBlockN, 0, workspace, workspace_bytes, batch, 1, num_heads, num_heads_k, head_dim, capacity, 1, q_strides,
+                            kcache_strides, vcache_strides, kn, vn, o_strides, 0, num_splits, softmax_scale, nullptr, nullptr, nullptr, 0, 0, nullptr, nullptr,
+                            0, 0, &keep);
 }
 
 #ifndef IV2_F16        // one such entry point in the library: bfloat16 only

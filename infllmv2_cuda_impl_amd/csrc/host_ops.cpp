@@ -819,7 +819,16 @@ std::tuple<Tensor, Tensor> decode_sparse(const Tensor& q, const Tensor& kn, cons
     DeviceGuard guard(q.device());
     const int64_t batch = q.size(0), hq = q.size(2), hk = kc.size(2);
     const int splits = decode_splits(batch, hk, topk);
+    const int64_t blocks = (max_len + block_size - 1) / block_size;
+    const bool all = blocks <= topk;                           // nothing to select: no scores
     if (batch * hk * splits > 256 || max_len > INFLLMV2_DECODE_MAX_SCORES * kBlock) {
+        if (all && topk <= INFLLMV2_DECODE_MAX_SCORES) {
+            check_step(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, kernel_size, stride, block_size, true);
+            const Tensor new_lens = std::get<0>(decode_front(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, max_len, kernel_size,
+                                                             stride, block_size, false, local_blocks, init_blocks, scale));
+            return {std::get<0>(fwd_kvcache(q, kc, vc, std::nullopt, std::nullopt, new_lens, scale, 0, std::nullopt, std::nullopt, std::nullopt, std::nullopt,
+                                            std::nullopt, std::nullopt, std::nullopt, false)), new_lens};
+        }
         auto [new_lens, mask] = decode_step(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, max_len, kernel_size, stride,
                                             block_size, topk, local_blocks, init_blocks, scale);
         return {std::get<0>(fwd_kvcache(q, kc, vc, std::nullopt, std::nullopt, new_lens, scale, 0, std::nullopt, mask, std::nullopt, std::nullopt,
@@ -830,7 +839,6 @@ std::tuple<Tensor, Tensor> decode_sparse(const Tensor& q, const Tensor& kn, cons
     // bound by the host that issues it (one sequence, seven allocations 22.6 us to issue, two 19.6; six sequences 19.2 and 17.3).
     Tensor new_lens, out = at::empty_like(q);
     if (lens.has_value()) new_lens = at::empty({batch}, q.options().dtype(at::kInt));
-    const int64_t blocks = (max_len + block_size - 1) / block_size;
     const int64_t max_f = std::min(windows(max_len, kernel_size, stride), fine.size(1)), max_c = std::min(windows(max_len, 4 * kernel_size, 4 * stride), coarse.size(1));
     size_t at_byte = 0;
     auto take = [&](size_t bytes) { const size_t start = at_byte; at_byte += (bytes + 255) / 256 * 256; return start; };
@@ -848,6 +856,14 @@ std::tuple<Tensor, Tensor> decode_sparse(const Tensor& q, const Tensor& kn, cons
     const int64_t kns[2] = {kn.stride(0), kn.stride(2)}, vns[2] = {vn.stride(0), vn.stride(2)};
     const S3 kcs = batch_rows_heads(kc), vcs = batch_rows_heads(vc), fs = batch_rows_heads(fine), cs = batch_rows_heads(coarse);
     void* stream = stream_of(q);
+    if (all) {
+        auto step = is_half(q) ? infllmv2_decode_step_all_f16 : infllmv2_decode_step_all;
+        check_rc(step(stream, ptr(q), ptr(kn), ptr(vn), ptr(kc), ptr(vc), ptr(fine), ptr(coarse), iptr(lens), as_int(host_len), new_ptr, fine_ptr, coarse_ptr, ptr(out),
+                      reinterpret_cast<float*>(base + lse), base + partials, partial_bytes, as_int(batch), as_int(hq), as_int(hk), as_int(kHeadDim),
+                      as_int(kc.size(1)), as_int(fine.size(1)), as_int(coarse.size(1)), as_int(max_len), qs, kns, vns, kcs.v, vcs.v, fs.v, cs.v, os,
+                      as_int(kernel_size), as_int(stride), as_int(4 * kernel_size), as_int(4 * stride), splits, static_cast<float>(scale)), "decode_step_all");
+        return {out, new_lens};
+    }
     auto front = is_half(q) ? infllmv2_decode_step_scores_f16 : infllmv2_decode_step_scores;
     check_rc(front(stream, ptr(q), ptr(kn), ptr(vn), ptr(kc), ptr(vc), ptr(fine), ptr(coarse), iptr(lens), as_int(host_len), new_ptr, fine_ptr, coarse_ptr,
                    base + scores, base + records, record_bytes, as_int(batch), as_int(hq), as_int(hk), as_int(kHeadDim), as_int(kc.size(1)),
