@@ -127,6 +127,13 @@ __device__ __forceinline__ float fold_rows32(float x, float y) {
     const u2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
+// the lower halves of x and y, and the upper halves
+__device__ __forceinline__ void halves(float x, float y, float& lower, float& upper) {
+    typedef unsigned u2 __attribute__((ext_vector_type(2)));
+    const u2 r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    lower = __uint_as_float(r[0]);
+    upper = __uint_as_float(r[1]);
+}
 // value of lane (n + k) % 16 of the same 16-lane row (DPP row_ror:k)
 template <int kRot>
 __device__ __forceinline__ float dpp_row_ror(float x) {
@@ -174,11 +181,12 @@ __device__ __forceinline__ void pool_quads(float a, float b, float prev_a, float
 // 2048 tokens 15.9 | 11.9, 4096 27.3 | 21.2, 8192 56.2 | 48.5, 16 384 133 | 125, 20 480 201 | 196, 32 768 443 | 443, 49 152 931 | 944: rows of 512 blocks and no more.  Whole prefill of
 // 1000 tokens, 16 blocks selected, 42.0 -> 40.7, of 2048 74.4 -> 70.0, training on 1023 + 3001 + 517 + 2200 606 -> 596.
 // kShared: workgroups share a block of tokens (launch_stage1); a variant of its own, because the others paid 0.5 us for the possibility.
-// kTok: tokens of a wavefront, 2 or, in launches of few workgroups (launch_stage1), 1.  A token's row is the same bits either way.
-template <bool kCausal, bool kPool, int kItems = 0, bool kShared = false, int kTok = kTokPerWave>
+// kTok: tiles of 16 rows of a wavefront, a token each: 2 or, in launches of few workgroups (launch_stage1), 1.  kPack == 2: two tokens to a tile, heads 0 to 7 of
+// its rows 0 to 7 and 8 to 15.  The head sums then end where the two halves of the rows would have been added.  A token's row is the same bits in every form.
+template <bool kCausal, bool kPool, int kItems = 0, bool kShared = false, int kTok = kTokPerWave, int kPack = 1>
 __global__ __launch_bounds__(64 * kWavesS1) __attribute__((amdgpu_waves_per_eu(kWavesPerSimdS1, kWavesPerSimdS1)))
 void stage1_kernel(const Stage1Params p) {
-    constexpr int kTokens = kTok * kWavesS1;                   // of the workgroup
+    constexpr int kMine = kTok * kPack, kTokens = kMine * kWavesS1;                 // tokens of a wavefront and of the workgroup
     __shared__ uint4 tile[2][1024];                            // two 16 KiB operand-ordered key tiles
     __shared__ elem_bits pooled[kItems > 0 ? kTokens : 1][kItems > 0 ? 64 * kItems : 1];
     const int tid = threadIdx.x;
@@ -197,19 +205,17 @@ void stage1_kernel(const Stage1Params p) {
     const int c0 = p.cu_seqlens_c[b], Lc = p.cu_seqlens_c[b + 1] - c0;
     const int s1 = (Lk == Lc) ? 16 : 64;                       // flash_fwd_kernel.h:1236-1240
 
-    const int tok0 = tok_block0 + wave * kTok;                 // first token of this wavefront
-    int vis_f[kTok], vis_c[kTok];
-    bool live[kTok];
-    int min_vis_c = 0x7fffffff;
+    const int tok0 = tok_block0 + wave * kMine;                // first token of this wavefront
+    int vis_f[kMine], vis_c[kMine];
+    bool live[kMine];
 #pragma unroll
-    for (int t = 0; t < kTok; ++t) {
+    for (int t = 0; t < kMine; ++t) {
         const int i = tok0 + t;
         live[t] = i < Sq;
         vis_f[t] = live[t] ? stage1_visible(i, 16, Lk, Sq, kCausal) : 0;
         vis_c[t] = live[t] ? stage1_visible(i, s1, Lc, Sq, kCausal) : 0;
         if (vis_c[t] == 0) vis_f[t] = 0;                       // early exit of flash_fwd_kernel.h:1271-1276
         if (kPool && vis_f[t] > p.score_cols) vis_f[t] = p.score_cols;               // the score row the pooling would have read ends there
-        min_vis_c = vis_c[t] < min_vis_c ? vis_c[t] : min_vis_c;
     }
     // tile counts are taken over the whole workgroup (its last live token sees the most keys)
     const int i_last = (tok_block0 + kTokens - 1 < Sq ? tok_block0 + kTokens - 1 : Sq - 1);
@@ -225,7 +231,7 @@ void stage1_kernel(const Stage1Params p) {
         if (wg_vis_f / kKeysPerBlock < p.topk && i_last / kBlockN < p.topk) {                        // uniform per workgroup
             const int taken = p.topk < p.pool_len ? p.topk : p.pool_len;
 #pragma unroll
-            for (int t = 0; t < kTok; ++t) {
+            for (int t = 0; t < kMine; ++t) {
                 if (!live[t]) continue;
                 uint64_t* row = p.mask + (static_cast<int64_t>(h) * p.total_q + q0 + tok0 + t) * p.mask_words;
                 for (int w = lane; w < p.mask_words; w += 64) row[w] = 64 * w + 64 <= taken ? ~0ull : 64 * w < taken ? (1ull << (taken - 64 * w)) - 1ull : 0ull;
@@ -253,8 +259,8 @@ void stage1_kernel(const Stage1Params p) {
     elem8 qf[kTok][4];
 #pragma unroll
     for (int t = 0; t < kTok; ++t) {
-        const int i = live[t] ? tok0 + t : Sq - 1;
-        const elem_bits* qp = p.q + (static_cast<int64_t>(q0) + i) * p.q_tok_stride + h * p.q_kvh_stride + (n < p.group ? n : p.group - 1) * p.q_grp_stride + 8 * g;
+        const int r = kPack == 2 ? n & 7 : n, want = tok0 + t * kPack + (kPack == 2 ? n >> 3 : 0), i = want < Sq ? want : Sq - 1;
+        const elem_bits* qp = p.q + (static_cast<int64_t>(q0) + i) * p.q_tok_stride + h * p.q_kvh_stride + (r < p.group ? r : p.group - 1) * p.q_grp_stride + 8 * g;
 #pragma unroll
         for (int c = 0; c < 4; ++c) qf[t][c] = *reinterpret_cast<const elem8*>(qp + 32 * c);
     }
@@ -274,6 +280,9 @@ void stage1_kernel(const Stage1Params p) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) { m[t][e] = -INFINITY; l[t][e] = 0.f; }
 
+    int vis_here[kTok];                                        // of the token whose heads this lane holds
+#pragma unroll
+    for (int t = 0; t < kTok; ++t) vis_here[t] = vis_c[t * kPack] + (g >= 2 ? vis_c[t * kPack + kPack - 1] - vis_c[t * kPack] : 0);      // (a choice of two elements put the array in LDS)
     auto next_coarse = [&](int ti) {
         if (ti + 1 < tiles_c) issue_tile(cbase, c_stride, c_off, (ti + 1) * 64, Lc, lds_tiles + ((ti + 1) & 1) * 16384, wave_u, n, g);
     };
@@ -298,9 +307,11 @@ void stage1_kernel(const Stage1Params p) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // this wavefront's share of the next tile has landed
         __syncthreads();
     };
-    // Two loops, as many rounds in all for every wavefront of the workgroup.  In the first every key of the tile is visible to both
-    // tokens: the maximum is finite, no key test, and the scale rides in the multiply-add that feeds exp2.
-    const int whole_c = min_vis_c >> 6 < tiles_c ? min_vis_c >> 6 : tiles_c;
+    // Two loops, as many rounds in all for every wavefront of the workgroup.  In the first every key of the tile is visible to all of its
+    // tokens: the maximum is finite, no key test, and the scale rides in the multiply-add that feeds exp2, which rounds otherwise: which tiles these are is
+    // decided by the first of four tokens, however many of them a wavefront has, so that a row does not depend on that.
+    const int seen_c = live[0] ? stage1_visible(tok0 & ~3, s1, Lc, Sq, kCausal) : 0;
+    const int whole_c = seen_c >> 6 < tiles_c ? seen_c >> 6 : tiles_c;
     for (int ti = 0; ti < whole_c; ++ti) {
         next_coarse(ti);
         floatx4 s[kTok][4];
@@ -322,7 +333,7 @@ void stage1_kernel(const Stage1Params p) {
     }
     for (int ti = whole_c; ti < tiles_c; ++ti) {               // the tiles that hold a token's last visible key
         next_coarse(ti);
-        if (kTok == 1 && !live[0]) {                                        // uniform: a wavefront without a token only brings its share of the tiles
+        if (kTok == 1 && !live[0]) {                           // uniform: a wavefront without a token only brings its share of the tiles
             tile_done();
             continue;
         }
@@ -335,7 +346,7 @@ void stage1_kernel(const Stage1Params p) {
                 float v[4];
 #pragma unroll
                 for (int kt = 0; kt < 4; ++kt)
-                    v[kt] = (ti * 64 + kt * 16 + n < vis_c[t]) ? s[t][kt][e] * p.scale_log2 : -INFINITY;
+                    v[kt] = (ti * 64 + kt * 16 + n < vis_here[t]) ? s[t][kt][e] * p.scale_log2 : -INFINITY;
                 const float mx = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
                 const float m_new = fmaxf(m[t][e], mx);
                 const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
@@ -359,23 +370,23 @@ void stage1_kernel(const Stage1Params p) {
             const float mu = (mm == -INFINITY) ? 0.f : mm;
             const float ll = row16_sum(l[t][e] * __builtin_amdgcn_exp2f(m[t][e] - mu));
             lse2[t][e] = mm + __builtin_amdgcn_logf(ll);        // v_log_f32 is log2
-            if (4 * g + e >= p.group) lse2[t][e] = INFINITY;    // a row that only fills the tile: exp2(x - inf) = 0 in the head sum
+            if ((kPack == 2 ? 4 * (g & 1) : 4 * g) + e >= p.group) lse2[t][e] = INFINITY;    // a row that only fills the tile: exp2(x - inf) = 0 in the head sum
         }
 
     // ---------------- pass 2: scores over the fine keys ----------------
     if (begin_f < end_f) issue_tile(kbase, k_stride, k_off, begin_f * 64, Lk, lds_tiles + (begin_f & 1) * 16384, wave_u, n, g);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    static_assert(kTok == 1 || kTok == 2, "pool_quads takes two tokens");
-    elem_bits* out_rows[kTok];
-    int bq[kTok];                                              // pooled output: the key block the token itself sits in
-    float prev[kTok];                                          // pooled output: scores of the previous tile, for its last key
+    static_assert(kMine == 1 || kMine % 2 == 0, "pool_quads takes two tokens");
+    elem_bits* out_rows[kMine];
+    int bq[kMine];                                             // pooled output: the key block the token itself sits in
+    float prev[kMine];                                         // pooled output: scores of the previous tile, for its last key
     int plain_first = 0, plain_end;                            // tiles that need no test, below
     {
         const int cache_len = kPool ? (p.cache_lens ? p.cache_lens[b] : p.cache_len) : 0;
         int seen = 0x7fffffff, before_local = 0x7fffffff;
 #pragma unroll
-        for (int t = 0; t < kTok; ++t) {
+        for (int t = 0; t < kMine; ++t) {
             const int64_t row = static_cast<int64_t>(q0) + tok0 + t;
             out_rows[t] = kPool ? p.score + (static_cast<int64_t>(h) * p.score_head_stride + row * p.pool_len)
                                 : p.score + h * p.score_head_stride + row * p.score_row_stride;
@@ -404,17 +415,17 @@ void stage1_kernel(const Stage1Params p) {
 
     // A plain tile's results are stored when the next tile begins: the wait at a tile's end counts stores too, and one just
     // issued would add its round trip to every tile.
-    float held[kTok] = {};
+    float held[kMine] = {};
     bool pending = false;
     auto store = [&](int t, uint32_t at, elem_bits value) {
-        if constexpr (kItems > 0) pooled[wave * kTok + t][at] = value;
+        if constexpr (kItems > 0) pooled[wave * kMine + t][at] = value;
         else out_rows[t][at] = value;
     };
     auto store_held = [&](int ti) {
         const uint32_t at = static_cast<uint32_t>(kPool ? ti * 16 + (lane >> 2) : ti * 64 + lane);
         if (!kPool || (lane & 3) == 0) {
 #pragma unroll
-            for (int t = 0; t < kTok; ++t) store(t, at, f32_to_elem_hw(held[t]));
+            for (int t = 0; t < kMine; ++t) store(t, at, f32_to_elem_hw(held[t]));
         }
     };
     for (int ti = begin_f; ti < end_f; ++ti) {
@@ -450,34 +461,38 @@ void stage1_kernel(const Stage1Params p) {
         }
         // sum over the four 16-lane rows (the head groups) and hand row kt the total of key tile kt, in three
         // exchanges: (row0 + row1 | row2 + row3) of tiles 0/1 and of tiles 2/3, then the two halves.  lane = 16*g + n  <->  key 16*g + n of this tile
-        float mine[kTok];
+        float mine[kMine];
 #pragma unroll
-        for (int t = 0; t < kTok; ++t)
-            mine[t] = fold_rows32(fold_rows16(part[t][0], part[t][1]), fold_rows16(part[t][2], part[t][3]));
+        for (int t = 0; t < kTok; ++t) {
+            const float even = fold_rows16(part[t][0], part[t][1]), odd = fold_rows16(part[t][2], part[t][3]);
+            if constexpr (kPack == 1) mine[t] = fold_rows32(even, odd);
+            else halves(even, odd, mine[2 * t], mine[2 * t + 1]);
+        }
         const bool mine_too = !kShared || !kPool || ti >= first_f;                   // not the tile before
         pending = ti >= plain_first && ti < plain_end && mine_too;
         const int col = ti * 64 + lane;
         if (!pending) {
 #pragma unroll
-            for (int t = 0; t < kTok; ++t) mine[t] = col < vis_f[t] ? mine[t] : 0.f;     // keys the token may not see score 0
+            for (int t = 0; t < kMine; ++t) mine[t] = col < vis_f[t] ? mine[t] : 0.f;     // keys the token may not see score 0
         }
         if (!kPool) {
 #pragma unroll
-            for (int t = 0; t < kTok; ++t) {
+            for (int t = 0; t < kMine; ++t) {
                 held[t] = mine[t];
                 if (!pending && live[t] && col < p.score_cols) out_rows[t][col] = f32_to_elem_hw(mine[t]);
             }
         } else {
             // block kb = col / 4 pools keys 4 kb - 1 .. 4 kb + 3: its quad and the last key of the quad before
-            if constexpr (kTok == 2) {
-                pool_quads(mine[0], mine[1], prev[0], prev[1], held[0], held[1]);
-            } else {
+            if constexpr (kMine == 1) {
                 float same;
                 pool_quads(mine[0], mine[0], prev[0], prev[0], held[0], same);
+            } else {
+#pragma unroll
+                for (int t = 0; t < kMine; t += 2) pool_quads(mine[t], mine[t + 1], prev[t], prev[t + 1], held[t], held[t + 1]);
             }
             const int kb = col >> 2;
 #pragma unroll
-            for (int t = 0; t < kTok; ++t) {
+            for (int t = 0; t < kMine; ++t) {
                 prev[t] = mine[t];
                 if (!pending && mine_too && live[t] && (lane & 3) == 0 && kb < p.pool_len) store(t, kb, pool_rest(kb, bq[t], held[t]));
             }
@@ -488,7 +503,7 @@ void stage1_kernel(const Stage1Params p) {
     if (kShared && end_f < tiles_f) return;                // uniform per workgroup; the rest is the last one's
     // columns no tile covered
 #pragma unroll
-    for (int t = 0; t < kTok; ++t) {
+    for (int t = 0; t < kMine; ++t) {
         if (!live[t]) continue;
         if (!kPool) {
             for (int col = tiles_f * 64 + lane; col < p.score_cols; col += 64) out_rows[t][col] = 0;
@@ -503,14 +518,14 @@ void stage1_kernel(const Stage1Params p) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        uint32_t key[kTok][kItems];                     // 0: no column
+        uint32_t key[kMine][kItems];                           // 0: no column
         const int take_at_most = p.topk < p.pool_len ? p.topk : p.pool_len;
 #pragma unroll
-        for (int t = 0; t < kTok; ++t)
+        for (int t = 0; t < kMine; ++t)
 #pragma unroll
             for (int e = 0; e < kItems; ++e) {
                 const int kb = 64 * e + lane;
-                key[t][e] = kb < p.pool_len ? sortable16(pooled[wave * kTok + t][kb]) : 0u;
+                key[t][e] = kb < p.pool_len ? sortable16(pooled[wave * kMine + t][kb]) : 0u;
             }
         auto count = [&](int t, auto&& in) {
             int c = 0;
@@ -518,18 +533,18 @@ void stage1_kernel(const Stage1Params p) {
             for (int e = 0; e < kItems; ++e) c += __builtin_popcountll(__builtin_amdgcn_ballot_w64(in(key[t][e])));
             return c;
         };
-        uint32_t thr[kTok];                             // the largest key that so many keys reach
+        uint32_t thr[kMine];                                   // the largest key that so many keys reach
 #pragma unroll
-        for (int t = 0; t < kTok; ++t) thr[t] = 0;
+        for (int t = 0; t < kMine; ++t) thr[t] = 0;
 #pragma unroll
         for (int bit = 15; bit >= 0; --bit)
 #pragma unroll
-            for (int t = 0; t < kTok; ++t) {
+            for (int t = 0; t < kMine; ++t) {
                 const uint32_t next = thr[t] | (1u << bit);
                 thr[t] = count(t, [&](uint32_t x) { return x >= next; }) >= take_at_most ? next : thr[t];
             }
 #pragma unroll
-        for (int t = 0; t < kTok; ++t) {
+        for (int t = 0; t < kMine; ++t) {
             if (!live[t]) continue;
             int ties = take_at_most - count(t, [&](uint32_t x) { return x > thr[t]; });          // of the keys equal to it
             uint64_t words = 0ull;                             // lane w: word w
@@ -606,29 +621,37 @@ int launch_stage1(const char* who, void* stream, const void* q, const void* k, c
     // give each CU a workgroup, with four tiles each at least.  Kernel alone, us, 2 KV heads, 20 011 keys: 16 queries 34.8 -> 19.3, 256 35.4 -> 20.1, 512 34.8 -> 21.2, 700 35.2 ->
     // 25.6, 1024 35.5 -> 27.2; 60 000 keys, one KV head, 300 queries 90.4 -> 36.1; a whole chunk of 512 queries behind 19 499 keys 154.7 -> 139.9.  Two workgroups to a
     // CU: 700 queries 31.0, 1500 36.1 -> 39.5; two tiles each at least: 256 queries 26.7.
-    const int64_t wgs = static_cast<int64_t>((max_seqlen_q + kTokPerBlock - 1) / kTokPerBlock) * batch * num_heads_k;
+    // Groups of 8 heads and fewer: two tokens share the 16 rows of a product, of which half were spare.  us, groups of 8, 2 KV heads, one | two tokens: scores of 256 queries against 20 011
+    // keys 13.6 | 13.6, 2049 51.1 | 36.5, 8000 92 | 63; selecting prefill of 2048 tokens 15.7 | 15.0, 32 768 391 | 257; scores of 65 536, one KV head, with the top-k launch 733 | 453.
+    const int pack = p.group <= 8 ? 2 : 1;
+    const int64_t wgs = static_cast<int64_t>((max_seqlen_q + kTokPerBlock * pack - 1) / (kTokPerBlock * pack)) * batch * num_heads_k;
     const int64_t fill = wgs > 0 ? 256 / wgs : 1, most = max_seqlen_k / 256;
     p.splits = p.mask != nullptr || fill < 2 || most < 2 ? 1 : static_cast<int>(fill < most ? fill : most);
-    // One token to a wavefront, twice the workgroups, up to 384 of the others: fewer than one and a half to a CU that holds two.  The time is then that of the CU with the most, half a
+    // One token to a wavefront (two, where two share the rows), twice the workgroups, up to 384 of the others: fewer than one and a half to a CU that holds two.  The time is then that of the CU with the most, half a
     // workgroup finer, and of the chain of one tile (one wavefront's products and exponentials behind the other's on a SIMD), which is shorter.  Scores alone, us, two tokens | one, 2 KV heads, 20 011 keys:
     // 17 queries 18.8 | 12.5, 256 19.3 | 13.3, 512 20.1 | 20.6, 1100 35.1 | 32.9, 2049 54.0 | 49.7, 3000 (376 workgroups) 56.1 | 51.1; 3500 (438) 57.2 | 62.8, 4096 60.3 | 64.1; 60 000
     // keys, one head, 2049 89.6 | 73.5; selecting prefill of 1000 tokens 15.2 | 12.4, 2048 17.1 | 15.8, 3000 22.4 | 21.5.
+    // Workgroups whose rows take every block return at once and do not count (selecting prefill of 5000 tokens, 64 blocks, 22.9 | 19.8, of 8192 with one KV head 26.2 | 23.8).
     constexpr int64_t kOneTokenWorkgroups = 384;
-    const bool one = wgs <= kOneTokenWorkgroups;
-    const int tokens = one ? kWavesS1 : kTokPerBlock;
+    const int64_t scored = p.mask ? static_cast<int64_t>(max_seqlen_q) - static_cast<int64_t>(kBlockN) * p.topk : max_seqlen_q;
+    const bool one = (scored + kTokPerBlock * pack - 1) / (kTokPerBlock * pack) * batch * num_heads_k <= kOneTokenWorkgroups;
+    const int tokens = (one ? kWavesS1 : kTokPerBlock) * pack;
     const dim3 grid((max_seqlen_q + tokens - 1) / tokens * p.splits, batch, num_heads_k);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    auto pick = [&](auto tok) {
-        constexpr int kTok = decltype(tok)::value;
-        if (p.mask) return p.pool_len <= 64 ? stage1_kernel<true, true, 1, false, kTok> : p.pool_len <= 128 ? stage1_kernel<true, true, 2, false, kTok>
-                         : p.pool_len <= 256 ? stage1_kernel<true, true, 4, false, kTok> : stage1_kernel<true, true, 8, false, kTok>;
+    auto pick = [&](auto tok, auto packed) {
+        constexpr int kTok = decltype(tok)::value, kPack = decltype(packed)::value;
+        if (p.mask) return p.pool_len <= 64 ? stage1_kernel<true, true, 1, false, kTok, kPack> : p.pool_len <= 128 ? stage1_kernel<true, true, 2, false, kTok, kPack>
+                         : p.pool_len <= 256 ? stage1_kernel<true, true, 4, false, kTok, kPack> : stage1_kernel<true, true, 8, false, kTok, kPack>;
         const bool shared = p.splits > 1;
-        return pool ? (is_causal ? (shared ? stage1_kernel<true, true, 0, true, kTok> : stage1_kernel<true, true, 0, false, kTok>)
-                                 : (shared ? stage1_kernel<false, true, 0, true, kTok> : stage1_kernel<false, true, 0, false, kTok>))
-                    : (is_causal ? (shared ? stage1_kernel<true, false, 0, true, kTok> : stage1_kernel<true, false, 0, false, kTok>)
-                                 : (shared ? stage1_kernel<false, false, 0, true, kTok> : stage1_kernel<false, false, 0, false, kTok>));
+        return pool ? (is_causal ? (shared ? stage1_kernel<true, true, 0, true, kTok, kPack> : stage1_kernel<true, true, 0, false, kTok, kPack>)
+                                 : (shared ? stage1_kernel<false, true, 0, true, kTok, kPack> : stage1_kernel<false, true, 0, false, kTok, kPack>))
+                    : (is_causal ? (shared ? stage1_kernel<true, false, 0, true, kTok, kPack> : stage1_kernel<true, false, 0, false, kTok, kPack>)
+                                 : (shared ? stage1_kernel<false, false, 0, true, kTok, kPack> : stage1_kernel<false, false, 0, false, kTok, kPack>));
     };
-    auto kernel = one ? pick(std::integral_constant<int, 1>{}) : pick(std::integral_constant<int, kTokPerWave>{});
+    constexpr std::integral_constant<int, 1> k1{};
+    constexpr std::integral_constant<int, 2> k2{};
+    static_assert(kTokPerWave == 2, "k2");
+    auto kernel = one ? (pack == 2 ? pick(k1, k2) : pick(k1, k1)) : (pack == 2 ? pick(k2, k2) : pick(k2, k1));
     hipLaunchKernelGGL(kernel, grid, dim3(64 * kWavesS1), 0, st, p);
     IV2_LAUNCH_CHECK();
     return 0;

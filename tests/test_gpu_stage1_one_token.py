@@ -1,6 +1,6 @@
-"""Stage 1 in launches of few workgroups, whose wavefronts take one token each: scores, pooled scores and mask words are, bit for bit, those of the same
-sequences among so many copies that the launch takes two tokens to a wavefront.  Lengths around the 8 and 16 tokens of a workgroup, the 64 keys of a
-tile and the row lengths of the selection."""
+"""Stage 1 in launches of few workgroups, whose wavefronts take one token each (two in groups of 8 heads and fewer): scores, pooled scores and mask words are,
+bit for bit, those of the same sequences among so many copies that the launch takes twice as many tokens to a wavefront.  Lengths around the 8, 16 and
+32 tokens of a workgroup, the 64 keys of a tile and the row lengths of the selection."""
 import numpy as np
 import pytest
 import torch
@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dtype, hk, group, lens", [
     (torch.bfloat16, 1, 16, [2]), (torch.bfloat16, 2, 16, [15, 16, 17]), (torch.float16, 1, 16, [1, 0, 9, 1040]), (torch.bfloat16, 1, 4, [1087]),
-    (torch.bfloat16, 2, 16, [2049]), (torch.float16, 1, 8, [130, 4096]), (torch.bfloat16, 1, 16, [4097]), (torch.bfloat16, 1, 16, [5999])])
+    (torch.bfloat16, 2, 16, [2049]), (torch.float16, 1, 8, [130, 4096]), (torch.bfloat16, 1, 16, [4097]), (torch.bfloat16, 1, 16, [5999]),
+    (torch.bfloat16, 2, 8, [2, 31, 33]), (torch.float16, 1, 2, [8333]), (torch.bfloat16, 1, 1, [4163, 7])])
 def test_as_among_many(dtype, hk, group, lens):
     import infllmv2_cuda_impl_amd as ops
     from infllmv2_cuda_impl_amd import _lib
@@ -18,7 +19,8 @@ def test_as_among_many(dtype, hk, group, lens):
     r = lambda heads: torch.randn(sum(lens), heads, 128, generator=gen, device="cuda").to(dtype)
     q, k, v = r(hk * group), r(hk), r(hk)
     longest = max(lens)
-    copies = 385 // (-(-longest // 16) * len(lens) * hk) + 1           # more than 384 workgroups of two tokens to a wavefront
+    tokens = 16 if group == 16 else 32
+    copies = 385 // (-(-longest // tokens) * len(lens) * hk) + 1       # more than 384 workgroups of the larger kind
     cu = lambda n: torch.tensor(np.cumsum([0] + lens * n), dtype=torch.int32, device="cuda")
 
     def run(n):
