@@ -34,7 +34,6 @@ struct DecodeParams {
     float* o_part;                  // (batch, Hk, splits, 16, 128) fp32, normalised per split
     float* lse_part;                // (batch, Hk, splits, 16)
     const int* cache_seqlens;       // null: every sequence holds `held` tokens
-    int held;
     const uint64_t* mask;           // (batch, Hk, n64) or null
     const int* topk_idx;            // (batch, Hk, k_idx): the selection as an index list instead (-1: unused slot), or null
     int k_idx;
@@ -59,6 +58,7 @@ struct DecodeParams {
     int rotary_dim, rotary_interleaved;
     int mask_in_place;              // the mask has more words than LDS holds: read where they are
     int far_rows;                   // cache rows lie too far apart (or backwards) for 32-bit offsets inside a block
+    int held;
     int append_here;                // the split kernel itself writes the one new row per sequence (and sees it whatever the cache holds)
 };
 
@@ -331,9 +331,8 @@ struct KeepStep {
     S1DecodeStep step;
     S1DecodeStrides strides;
 };
-template <bool kDirect, int kWaves, bool kSelect, typename Keep = NoKeep>
-__global__ __launch_bounds__(64 * kWaves)
-void decode_split_kernel(const DecodeParams p, const Keep keep) {
+template <bool kDirect, int kWaves, bool kSelect, typename Keep>
+__device__ __forceinline__ void decode_split(const DecodeParams& p, const Keep& keep) {
     constexpr bool kKeep = std::is_same<Keep, KeepStep>::value;
     static_assert(kWaves == 4 || !(kSelect || kKeep), "by four wavefronts");
     constexpr int kSlots = kWaves == 1 ? 2 : 1;                // block tiles per wavefront
@@ -771,6 +770,17 @@ void decode_split_kernel(const DecodeParams p, const Keep keep) {
     }
 }
 
+template <bool kDirect, int kWaves, bool kSelect>
+__global__ __launch_bounds__(64 * kWaves)
+void decode_split_kernel(const DecodeParams p) {
+    decode_split<kDirect, kWaves, kSelect>(p, NoKeep{});
+}
+template <bool kDirect>
+__global__ __launch_bounds__(256)
+void decode_step_kernel(const DecodeParams p, const KeepStep keep) {
+    decode_split<kDirect, 4, false>(p, keep);
+}
+
 // Merge of the per-split partials: one wavefront per (sequence, query head), lane l holds columns 2 l and 2 l + 1 and,
 // for the weights, split l.  kMax >= splits: the loads are unrolled (beyond the last split the last one is read again),
 // so every partial is requested before the first is used.  A wavefront per head keeps the merge of 64 splits at one
@@ -976,18 +986,19 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
         p.o_part = ws;
         p.lse_part = ws + static_cast<size_t>(batch) * num_heads_k * num_splits * 16 * kHeadDim;
     }
-    auto launch = [&](auto kernel, auto with, int workgroups) -> int {
+    auto launch = [&](auto kernel, int workgroups, const auto&... with) -> int {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
         IV2_CHECK(e == hipSuccess, "fwd_kvcache: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
-        hipLaunchKernelGGL(kernel, dim3(workgroups, num_heads_k, batch), dim3(grouped ? 256 : 64), lds, st, p, with);
+        hipLaunchKernelGGL(kernel, dim3(workgroups, num_heads_k, batch), dim3(grouped ? 256 : 64), lds, st, p, with...);
         IV2_LAUNCH_CHECK();
         return 0;
     };
     int rc;
-    if (keep != nullptr) rc = launch(num_splits == 1 ? decode_split_kernel<true, 4, false, KeepStep> : decode_split_kernel<false, 4, false, KeepStep>, *keep, num_splits + (pairs * (num_splits + 1) <= kGroupedWorkgroups ? 1 : 0));
-    else if (scores != nullptr) rc = launch(num_splits == 1 ? decode_split_kernel<true, 4, true> : decode_split_kernel<false, 4, true>, NoKeep{}, num_splits);
-    else if (grouped) rc = launch(num_splits == 1 ? decode_split_kernel<true, 4, false> : decode_split_kernel<false, 4, false>, NoKeep{}, num_splits);
-    else rc = launch(num_splits == 1 ? decode_split_kernel<true, 1, false> : decode_split_kernel<false, 1, false>, NoKeep{}, num_splits);
+    if (keep != nullptr) rc = launch(num_splits == 1 ? decode_step_kernel<true> : decode_step_kernel<false>,
+                                     num_splits + (pairs * (num_splits + 1) <= kGroupedWorkgroups ? 1 : 0), *keep);
+    else if (scores != nullptr) rc = launch(num_splits == 1 ? decode_split_kernel<true, 4, true> : decode_split_kernel<false, 4, true>, num_splits);
+    else if (grouped) rc = launch(num_splits == 1 ? decode_split_kernel<true, 4, false> : decode_split_kernel<false, 4, false>, num_splits);
+    else rc = launch(num_splits == 1 ? decode_split_kernel<true, 1, false> : decode_split_kernel<false, 1, false>, num_splits);
     if (rc != 0) return rc;
     if (num_splits > 1) {
         const CombineParams c{p.o_part, p.lse_part, p.out, p.lse, p.o_batch, p.o_head, num_heads_k, num_splits, p.group};
