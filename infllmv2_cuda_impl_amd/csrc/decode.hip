@@ -33,7 +33,7 @@ struct DecodeParams {
     float* lse;                     // (batch, Hq)
     float* o_part;                  // (batch, Hk, splits, 16, 128) fp32, normalised per split
     float* lse_part;                // (batch, Hk, splits, 16)
-    const int* cache_seqlens;       // null: every sequence holds `held` tokens
+    const int* cache_seqlens;       // null: every sequence fills the whole cache
     const uint64_t* mask;           // (batch, Hk, n64) or null
     const int* topk_idx;            // (batch, Hk, k_idx): the selection as an index list instead (-1: unused slot), or null
     int k_idx;
@@ -58,7 +58,6 @@ struct DecodeParams {
     int rotary_dim, rotary_interleaved;
     int mask_in_place;              // the mask has more words than LDS holds: read where they are
     int far_rows;                   // cache rows lie too far apart (or backwards) for 32-bit offsets inside a block
-    int held;
     int append_here;                // the split kernel itself writes the one new row per sequence (and sees it whatever the cache holds)
 };
 
@@ -326,14 +325,15 @@ __device__ __forceinline__ uint64_t select_words(const elem_bits* row, int n, in
 // above.  Steps of the layer in us, launches for the front, the scores, the attention and the merge | for the front, the attention and the merge | this and the
 // merge, 2 KV heads, 64 blocks selected: one sequence of 4000 tokens 19.0 | 15.2 | 10.6 (all the host's), 16 of up to 4000 23.2 | 15.9 | 13.7, 32 of 2000 26.4 | 18.6 |
 // 16.7 (with workgroups for the keepers alone 21.7), 64 of 1500 29.9 | 22.4 | 21.0 (27.4).
-struct NoKeep {};
 struct KeepStep {
     S1DecodeStep step;
     S1DecodeStrides strides;
 };
-template <bool kDirect, int kWaves, bool kSelect, typename Keep>
-__device__ __forceinline__ void decode_split(const DecodeParams& p, const Keep& keep) {
-    constexpr bool kKeep = std::is_same<Keep, KeepStep>::value;
+__device__ __forceinline__ const KeepStep& step_of(const KeepStep& keep) { return keep; }
+template <bool kDirect, int kWaves, bool kSelect, typename... Keep>
+__global__ __launch_bounds__(64 * kWaves)
+void decode_split_kernel(const DecodeParams p, const Keep... keep) {
+    constexpr bool kKeep = sizeof...(Keep) == 1;
     static_assert(kWaves == 4 || !(kSelect || kKeep), "by four wavefronts");
     constexpr int kSlots = kWaves == 1 ? 2 : 1;                // block tiles per wavefront
     extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
@@ -347,12 +347,13 @@ __device__ __forceinline__ void decode_split(const DecodeParams& p, const Keep& 
     const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
     auto keep_caches = [&]() {
         if constexpr (kKeep) {
-            const S1DecodeStep& t = keep.step;
+            const KeepStep& with = step_of(keep...);
+            const S1DecodeStep& t = with.step;
             const int len = t.lens ? t.lens[b] : t.host_len;
             int add_f, add_c;
             const int rows_f = s1d_step_rows(len, t.capacity, t.kernel_f, t.stride_f, t.fine_capacity, add_f);
             const int rows_c = s1d_step_rows(len, t.capacity, t.kernel_c, t.stride_c, t.coarse_capacity, add_c);
-            s1d_keep_caches(keep.strides, t, b, h, len, rows_f, rows_c, add_f, add_c, tid, false, true, kHeadDim);
+            s1d_keep_caches(with.strides, t, b, h, len, rows_f, rows_c, add_f, add_c, tid, false, true, kHeadDim);
         }
     };
     if (kKeep && split == p.splits) {                          // uniform over the workgroup
@@ -366,7 +367,10 @@ __device__ __forceinline__ void decode_split(const DecodeParams& p, const Keep& 
     int first_idx = -1;                                        // or list entry `lane`
     if (!kSelect && p.mask != nullptr && lane < p.n64) bits0 = p.mask[pair * p.n64 + lane];
     if (!kSelect && p.topk_idx != nullptr && lane < p.k_idx) first_idx = p.topk_idx[pair * p.k_idx + lane];
-    const int seqlen = p.cache_seqlens ? p.cache_seqlens[b] : p.held;
+    int without = 0;                                           // the length of a sequence where no lengths are given
+    if constexpr (kKeep) without = step_of(keep...).step.host_len;
+    else without = p.capacity - p.seqlen_new;
+    const int seqlen = p.cache_seqlens ? p.cache_seqlens[b] : without;
     const int lp = p.leftpad ? p.leftpad[b] : 0;              // the sequence's key 0 is cache row lp
     // position of the first appended key; a full cache takes no key, and the tables need not reach beyond it
     const int rot_pos = !p.cache_seqlens ? 0 : (seqlen < p.capacity ? seqlen : p.capacity - 1);
@@ -445,7 +449,7 @@ __device__ __forceinline__ void decode_split(const DecodeParams& p, const Keep& 
         lds_fence();
     } else if (!listed) {
         total = last_blk + 1;
-        if (kKeep && total > p.n_scores) total = p.n_scores;   // a longer sequence than was announced
+        if constexpr (kKeep) total = total < p.n_scores ? total : p.n_scores;      // a longer sequence than was announced
         lds_fence();
     } else {
         if (p.mask != nullptr && n_words <= 64) {              // straight into registers
@@ -770,17 +774,6 @@ __device__ __forceinline__ void decode_split(const DecodeParams& p, const Keep& 
     }
 }
 
-template <bool kDirect, int kWaves, bool kSelect>
-__global__ __launch_bounds__(64 * kWaves)
-void decode_split_kernel(const DecodeParams p) {
-    decode_split<kDirect, kWaves, kSelect>(p, NoKeep{});
-}
-template <bool kDirect>
-__global__ __launch_bounds__(256)
-void decode_step_kernel(const DecodeParams p, const KeepStep keep) {
-    decode_split<kDirect, 4, false>(p, keep);
-}
-
 // Merge of the per-split partials: one wavefront per (sequence, query head), lane l holds columns 2 l and 2 l + 1 and,
 // for the weights, split l.  kMax >= splits: the loads are unrolled (beyond the last split the last one is read again),
 // so every partial is requested before the first is used.  A wavefront per head keeps the merge of 64 splits at one
@@ -940,7 +933,6 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
     p.batch = batch; p.num_heads_k = num_heads_k; p.capacity = cache_capacity;
     p.group = num_heads / num_heads_k;
     p.seqlen_new = k_new ? seqlen_new : 0;
-    p.held = keep ? keep->step.host_len : cache_capacity - p.seqlen_new;
     p.n64 = n_uint64_per_row; p.splits = num_splits;
     p.scale_log2 = softmax_scale * 1.44269504088896340736f;
     p.cache_batch_idx = cache_batch_idx; p.leftpad = cache_leftpad;
@@ -994,7 +986,7 @@ static int fwd_kvcache_impl(void* stream, const void* q, void* kcache, void* vca
         return 0;
     };
     int rc;
-    if (keep != nullptr) rc = launch(num_splits == 1 ? decode_step_kernel<true> : decode_step_kernel<false>,
+    if (keep != nullptr) rc = launch(num_splits == 1 ? decode_split_kernel<true, 4, false, KeepStep> : decode_split_kernel<false, 4, false, KeepStep>,
                                      num_splits + (pairs * (num_splits + 1) <= kGroupedWorkgroups ? 1 : 0), *keep);
     else if (scores != nullptr) rc = launch(num_splits == 1 ? decode_split_kernel<true, 4, true> : decode_split_kernel<false, 4, true>, num_splits);
     else if (grouped) rc = launch(num_splits == 1 ? decode_split_kernel<true, 4, false> : decode_split_kernel<false, 4, false>, num_splits);
