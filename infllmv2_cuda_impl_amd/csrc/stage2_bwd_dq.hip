@@ -40,8 +40,7 @@ constexpr int kDqLdsTiles = 2 * kDqTileBytes + 8 * 8192;       // 2-tile ring + 
 typedef short short4q __attribute__((ext_vector_type(4)));
 
 struct DqExtra {
-    int groups_per_seq;
-    int batch;
+    GroupOrder order;
     int total_groups;
     int mask_words;                                            // words per LDS mask row: what the longest key sequence needs
 };
@@ -113,10 +112,8 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
     const int xcd = bid & 7, sidx = bid >> 3;
     int G = ((sidx / kDqChunk) * 8 + xcd) * kDqChunk + (sidx % kDqChunk);
     if (G >= x.total_groups) return;                                                // uniform per workgroup
-    G = x.total_groups - 1 - G;
-    const int grp = G % x.groups_per_seq;
-    const int hb = G / x.groups_per_seq;
-    const int b = hb % x.batch, h = hb / x.batch;
+    int grp, h, b;
+    if (!group_at(x.order, x.total_groups - 1 - G, grp, h, b)) return;              // uniform per workgroup
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -384,9 +381,8 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
 
 int launch_bwd_dq_hybrid(hipStream_t st, const BwdParams& p, int batch, int max_seqlen_q, bool causal) {
     DqExtra x{};
-    x.batch = batch;
-    x.groups_per_seq = (max_seqlen_q + kDqTokens - 1) / kDqTokens;
-    const int64_t of_sequence = static_cast<int64_t>(p.num_heads_k) * x.groups_per_seq, total = of_sequence * batch;
+    x.order = group_order(batch, p.num_heads_k, (max_seqlen_q + kDqTokens - 1) / kDqTokens);
+    const int64_t of_sequence = x.order.per_seq, total = x.order.places();
     IV2_CHECK(p.k_blocks <= kDqMaskWords * 64, "varlen_bwd: more than %d key blocks per sequence", kDqMaskWords * 64);
     const int64_t most = max_workgroups(512) - 8 * kDqChunk;
     if (total > most) {                                        // some sequences at a time, as in the forward

@@ -26,7 +26,7 @@
 //
 // Workgroups are numbered so that each of the 8 XCDs takes whole chunks of consecutive token
 // groups of one KV head (their L2 sees one head's images and neighbouring local windows), and
-// the longest causal prefixes are scheduled first.
+// the longest causal prefixes are scheduled first (GroupOrder in block_walker.h).
 // Long sequences are walked in step with the other workgroups of the XCD, at a given pace (in_step.h).
 #include "common.h"
 #include "kv_image.h"
@@ -47,8 +47,8 @@ constexpr int kMaxMaskWords = 256;                             // LDS copies of 
 
 struct HybridExtra {
     int groups_per_seq;                                        // ceil(max_seqlen_q / kHybTokens)
-    int batch;
-    int total_groups;                                          // num_heads_k * batch * groups_per_seq
+    GroupOrder order;                                          // of all groups, or of all but the late ones
+    int total_groups;                                          // places
     int late;                                                  // short groups that go last: num_heads_k * batch, or 0
     int mask_words;                                            // words per LDS mask row: what max_seqlen_k needs, not the maximum
     unsigned* finished;                                        // the XCDs' counters of in_step.h, or null: no workgroup waits
@@ -140,17 +140,16 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     const int xcd = (kParts <= 2 ? bid : bid - 16 / kParts * (static_cast<int>(blockIdx.y) >> 1)) & 7, sidx = bid >> 3;
     int G = ((sidx / kHybChunk) * 8 + xcd) * kHybChunk + (sidx % kHybChunk);
     if (G >= x.total_groups) return;                                                // uniform per workgroup
-    int grp, hb;
+    int grp, h, b;
+    bool there = true;
     if (kParts == 1 && G >= x.total_groups - x.late) {
         grp = x.groups_per_seq - 1;
-        hb = G - (x.total_groups - x.late);
+        const int hb = G - (x.total_groups - x.late);
+        b = hb % x.order.batch;
+        h = hb / x.order.batch;
     } else {
-        G = x.total_groups - x.late - 1 - G;
-        const int each = x.groups_per_seq - (x.late != 0 ? 1 : 0);
-        grp = G % each;
-        hb = G / each;
+        there = group_at(x.order, x.total_groups - x.late - 1 - G, grp, h, b);
     }
-    const int b = hb % x.batch, h = hb / x.batch;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -163,7 +162,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     const int64_t slot0 = static_cast<int64_t>(h) * p.n_slots + image_slot0(p.cu_seqlens_k, b);
     // (All of these are read before the first atomic: behind it the compiler loads them into vector registers, 0.5 us per workgroup.)
     unsigned* finished = x.finished + xcd * kInStepPitch;
-    if (i0 >= Sq) {                                                                 // uniform per workgroup
+    if (i0 >= Sq || !there) {                                                            // uniform per workgroup
         if (kLong && tid == 0 && x.finished) in_step_finished(finished);
         return;
     }
@@ -460,9 +459,10 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
 
 static int launch_groups(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q, int max_seqlen_k, bool causal, int most_selected, unsigned* in_step) {
     HybridExtra x{};
-    x.batch = batch;
     x.groups_per_seq = (max_seqlen_q + kHybTokens - 1) / kHybTokens;
-    const int64_t of_sequence = static_cast<int64_t>(num_heads_k) * x.groups_per_seq, total = of_sequence * batch;
+    x.order = group_order(batch, num_heads_k, x.groups_per_seq);
+    const int64_t of_sequence = x.order.per_seq, groups = static_cast<int64_t>(num_heads_k) * x.groups_per_seq * batch;
+    int64_t total = x.order.places();
     const int64_t most = max_workgroups(512) - 8 * kHybChunk;
     if (total > most) {                                        // more than a dispatch holds (thousands of sequences beside a long one): some sequences at a time
         const int fit = static_cast<int>(most / of_sequence);
@@ -477,11 +477,8 @@ static int launch_groups(hipStream_t st, const FwdParams& p, int batch, int num_
         }
         return 0;
     }
-    x.total_groups = static_cast<int>(total);
     x.mask_words = ((max_seqlen_k + kBlockN - 1) / kBlockN + 63) / 64;
     if (x.mask_words < 1) x.mask_words = 1;
-    const int64_t per_round = 8 * kHybChunk;
-    const int64_t grid = (total + per_round - 1) / per_round * per_round;
     const size_t lds = kRingTiles * kTileBytes + static_cast<size_t>(1 + kHybTokens) * x.mask_words * 8;
     const bool far = max_seqlen_k > kInStepKeys;
     // As many parts as give every workgroup a CU of its own (256).  A group's turn is bound by what its eight rows fetch through one CU's vector memory path (256 KiB for
@@ -492,7 +489,7 @@ static int launch_groups(hipStream_t st, const FwdParams& p, int batch, int num_
     // and gain nothing: 700 tokens behind 20011, 176 groups, take 102 whole.
     // So few groups run all at once: they neither count nor wait (in_step.h).  They keep the pace: it gives the order in which a row's blocks are added up, which must not
     // depend on the number of parts.
-    const int parts = total * 2 > 256 ? 1 : total * 4 > 256 ? 2 : total * 8 > 256 ? 4 : 8;
+    const int parts = groups * 2 > 256 ? 1 : groups * 4 > 256 ? 2 : groups * 8 > 256 ? 4 : 8;
     x.finished = parts > 1 ? nullptr : in_step;
     // Heaviest first is also longest prefix first, which puts the one short group of a chunk of queries in front.  Where the chunk's groups are alike, with at least twice as many
     // blocks behind the first of them as a row selects, it holds up a CU that then has as many whole groups to walk as the others, and goes last instead.  Forward with the images in us, first | last, 2 KV heads, 2049
@@ -501,7 +498,14 @@ static int launch_groups(hipStream_t st, const FwdParams& p, int batch, int num_
     // behind 4096 175 | 187, behind none 332 | 359 (6145 queries).
     const int over = max_seqlen_q % kHybTokens;
     const int64_t held = static_cast<int64_t>(max_seqlen_k) - max_seqlen_q, selected = most_selected < 0 ? -static_cast<int64_t>(most_selected) : most_selected;
-    if (parts == 1 && over > 0 && over <= 4 && x.groups_per_seq > 1 && selected > 0 && held >= 2 * kBlockN * selected) x.late = num_heads_k * batch;
+    if (parts == 1 && over > 0 && over <= 4 && x.groups_per_seq > 1 && selected > 0 && held >= 2 * kBlockN * selected) {
+        x.late = num_heads_k * batch;
+        x.order = group_order(batch, num_heads_k, x.groups_per_seq - 1);
+        total = x.order.places() + x.late;
+    }
+    x.total_groups = static_cast<int>(total);
+    const int64_t per_round = 8 * kHybChunk;
+    const int64_t grid = (total + per_round - 1) / per_round * per_round;
     auto pick = [&](auto n) {
         constexpr int kParts = decltype(n)::value;
         return causal ? (far ? stage2_fwd_hybrid_kernel<true, true, kParts> : stage2_fwd_hybrid_kernel<true, false, kParts>)
