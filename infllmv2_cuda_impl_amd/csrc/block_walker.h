@@ -82,6 +82,20 @@ __device__ __forceinline__ uint64_t walked_together(const unsigned long long* wo
     return eights | (fours & (twos | ones));
 }
 
+// How many of the ring's blocks that a row selects have one of its own walked beside them (beside those it does not select there always is one).  A row that has its
+// own blocks beside every ring block until they run out waits, from then on, at ring blocks that are not its own; with so many fewer beside the others it has one for each
+// of those.  That is its blocks less the ring's: negative, none, with few blocks to choose from.  Rows with more than kOwnBeside over take one every time: their own blocks outnumber the ring's that are not theirs, and
+// balanced all the same four packed sequences (71 552 tokens) took 5740 | 7450 us instead of 5625 | 7320, forward and dQ.  Whole passes, every time | balanced: 2048 tokens with 16 blocks
+// 65.0 -> 63.5 us, four ragged prompts 931 -> 922, training on four short samples 588 -> 585; 32 768 tokens and chunks as before.  Two beside a ring block that is not the
+// row's, too, as long as there are enough: 64.1, 942, 584, and 32 768 tokens 3164 -> 3212.  A rule on the group's rows alone, which gives the order in which they are added up.
+constexpr int kOwnBeside = 8;
+__device__ __forceinline__ int own_beside(const unsigned long long* row, const unsigned long long* together, int words, int lane) {
+    int over = 0;
+    for (int w = lane; w < words; w += 64) over += __builtin_popcountll(row[w]) - __builtin_popcountll(together[w]);
+    over = __builtin_amdgcn_readlane(scan_lanes(over), 63);
+    return over > kOwnBeside ? 1 << 30 : over;
+}
+
 // The order of the token groups of a launch of the row-parallel kernels, which take it from the end: one (head, sequence) after the other, its longest prefixes first; or, in
 // launches of up to 4096 groups (16 to a CU), one sequence after the other and in it 16 groups of a head, the same ones of the next head, and so on, so that the longest
 // prefixes of all heads come first and the shortest last.  Head by head the second head's longest groups were begun half-way.  Forward with the images in us, head by head | by turns: 1000 tokens,

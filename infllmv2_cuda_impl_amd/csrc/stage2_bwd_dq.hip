@@ -160,6 +160,8 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
     for (int w = tid; w < nw; w += 512) com[w] = walked_together(rows + w, x.mask_words, Sq - i0);
     __syncthreads();
 
+    int beside = own_beside(own, com, nw, lane);
+
     // ---- this token's operands, and D = rowsum(dO * O) from them ----
     elem8 qf[4], dof[4], of[4];
     float lse2;
@@ -251,14 +253,74 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
     if (j0 >= 0) issue(j0, 0);
     int tile = 0;
     bool k_ahead = false;                                      // the coming own block's 16 K-fragment loads were issued last turn
-    while (j0 >= 0 || jp >= 0) {
-        if (j0 >= 0) {                                         // uniform over the workgroup
+    auto own_part = [&]() {
+        {
+            const elem_bits* vsrc = p.vimg_r + img0 + static_cast<int64_t>(jp) * kImageElems;
+#pragma unroll
+            for (int f = 0; f < 16; ++f) vreg[f] = *reinterpret_cast<const elem8*>(vsrc + f * 512);
+        }
+        floatx4 s[4], dp[4];
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            s[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
+            dp[kt] = neg_dsum;
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt)
+                s[kt] = IV2_MFMA(kreg[kt * 4 + c], qf[c], s[kt], 0, 0, 0);
+#pragma unroll
+        for (int f = 0; f < 8; ++f) {                      // keys 0..31 of K -> private tile
+            uint4 raw;
+            __builtin_memcpy(&raw, &kreg[f], 16);
+            mine[f * 64] = raw;
+        }
+        p_and_dp(s, dp, vreg, dof, (jp == last_blk) ? last_key - jp * kBlockN : kBlockN - 1, g, p.scale_log2, lse2);
+        elem8 dsf[2];
+        ds_operand(s, dp, dsf);
+#pragma unroll
+        for (int cc = 0; cc < 2; ++cc) {
+            if (cc == 1) {
+#pragma unroll
+                for (int f = 0; f < 8; ++f) {              // keys 32..63 (LDS executes a wavefront's accesses in order)
+                    uint4 raw;
+                    __builtin_memcpy(&raw, &kreg[8 + f], 16);
+                    mine[f * 64] = raw;
+                }
+            }
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) {
+                const unsigned char* at = mine_tr + (dt >> 1) * 1024 + (dt & 1) * 512;
+                const short4q lo = dq_read_tr(at), hi = dq_read_tr(at + 4096);
+                elem8 kt_f;
+                __builtin_memcpy(&kt_f, &lo, 8);
+                __builtin_memcpy(reinterpret_cast<unsigned char*>(&kt_f) + 8, &hi, 8);
+                dq[dt] = IV2_MFMA(kt_f, dsf[cc], dq[dt], 0, 0, 0);
+            }
+        }
+        // the K fragments of the next own block go out last: they are the only ordinary loads in flight when the
+        // next turn waits for its DMA
+        const int jn = next_own();
+        k_ahead = jn >= 0;
+        if (jn >= 0) {
+            const elem_bits* ksrc = p.kimg + img0 + static_cast<int64_t>(jn) * kImageElems;
+#pragma unroll
+            for (int f = 0; f < 16; ++f) kreg[f] = *reinterpret_cast<const elem8*>(ksrc + f * 512);
+        }
+        jp = jn;
+    };
+    while (j0 >= 0) {                                          // uniform over the workgroup
+        {
             // younger than this wavefront's 4 DMA loads of block j0: last turn's 16 K loads
             if (k_ahead) asm volatile("s_waitcnt vmcnt(16)" ::: "memory"); else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();                                   // block j0 is in LDS for everyone; the other tile is free
             bool mine1 = false;
             const int j1 = next_common(mine1);
             if (j1 >= 0) issue(j1, tile ^ 1);
+            k_ahead = false;
+            int blocks = mine0 ? 0 : 1;                        // of its own beside this one
+            if (mine0 && beside > 0) { blocks = 1; --beside; }
             if (mine0) {
                 const uint4* kb = ring + tile * 2048 + lane;
                 const uint4* vb = kb + 1024;
@@ -304,66 +366,10 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
             j0 = j1;
             mine0 = mine1;
             tile ^= 1;
-        }
-        k_ahead = false;
-        if (jp >= 0) {                                         // per wavefront
-            {
-                const elem_bits* vsrc = p.vimg_r + img0 + static_cast<int64_t>(jp) * kImageElems;
-#pragma unroll
-                for (int f = 0; f < 16; ++f) vreg[f] = *reinterpret_cast<const elem8*>(vsrc + f * 512);
-            }
-            floatx4 s[4], dp[4];
-#pragma unroll
-            for (int kt = 0; kt < 4; ++kt) {
-                s[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
-                dp[kt] = neg_dsum;
-            }
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-#pragma unroll
-                for (int kt = 0; kt < 4; ++kt)
-                    s[kt] = IV2_MFMA(kreg[kt * 4 + c], qf[c], s[kt], 0, 0, 0);
-#pragma unroll
-            for (int f = 0; f < 8; ++f) {                      // keys 0..31 of K -> private tile
-                uint4 raw;
-                __builtin_memcpy(&raw, &kreg[f], 16);
-                mine[f * 64] = raw;
-            }
-            p_and_dp(s, dp, vreg, dof, (jp == last_blk) ? last_key - jp * kBlockN : kBlockN - 1, g, p.scale_log2, lse2);
-            elem8 dsf[2];
-            ds_operand(s, dp, dsf);
-#pragma unroll
-            for (int cc = 0; cc < 2; ++cc) {
-                if (cc == 1) {
-#pragma unroll
-                    for (int f = 0; f < 8; ++f) {              // keys 32..63 (LDS executes a wavefront's accesses in order)
-                        uint4 raw;
-                        __builtin_memcpy(&raw, &kreg[8 + f], 16);
-                        mine[f * 64] = raw;
-                    }
-                }
-#pragma unroll
-                for (int dt = 0; dt < 8; ++dt) {
-                    const unsigned char* at = mine_tr + (dt >> 1) * 1024 + (dt & 1) * 512;
-                    const short4q lo = dq_read_tr(at), hi = dq_read_tr(at + 4096);
-                    elem8 kt_f;
-                    __builtin_memcpy(&kt_f, &lo, 8);
-                    __builtin_memcpy(reinterpret_cast<unsigned char*>(&kt_f) + 8, &hi, 8);
-                    dq[dt] = IV2_MFMA(kt_f, dsf[cc], dq[dt], 0, 0, 0);
-                }
-            }
-            // the K fragments of the next own block go out last: they are the only ordinary loads in flight when the
-            // next turn waits for its DMA
-            const int jn = next_own();
-            if (jn >= 0) {
-                const elem_bits* ksrc = p.kimg + img0 + static_cast<int64_t>(jn) * kImageElems;
-#pragma unroll
-                for (int f = 0; f < 16; ++f) kreg[f] = *reinterpret_cast<const elem8*>(ksrc + f * 512);
-                k_ahead = true;
-            }
-            jp = jn;
+            if (blocks > 0 && jp >= 0) own_part();
         }
     }
+    while (jp >= 0) own_part();
     if (!live) return;
     // what the dK/dV kernel fetches of a token with one 128-byte transfer: [LSE * log2(e) x 16 | D x 16]
     if (g < 2) p.rowstat[(static_cast<int64_t>(h) * p.total_q + tok) * 32 + 16 * g + n] = g == 0 ? lse2 : -neg_dsum[0];

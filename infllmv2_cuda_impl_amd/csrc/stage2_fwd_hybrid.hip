@@ -18,7 +18,8 @@
 //   * the remaining blocks of a row are walked by its wavefront alone, operands straight from
 //     global memory into registers, as in stage2_fwd_kernel;
 //   * the two walks are interleaved, common, own, common, own per turn: the first is bound by
-//     the matrix pipeline and the VALU, the second by the vector memory path.
+//     the matrix pipeline and the VALU, the second by the vector memory path.  A row with few blocks more than the ring
+//     walks them beside ring blocks that are not its own (kOwnBeside in block_walker.h).
 //
 // A per-token kernel is bound by what the vector memory path can deliver (32 KiB of operands per
 // 512 MFMA cycles); the shared walk takes the common half of the work off that path.  Online
@@ -211,6 +212,7 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     __syncthreads();
     for (int w = tid; w < nw; w += 512) com[w] = share_log2 == 0 ? walked_together(rows + w, x.mask_words, in_group) : 0ull;   // shared out: no lock step
     __syncthreads();
+    int beside = own_beside(own, com, nw, lane);
     const uint64_t columns = (share_log2 == 0 ? ~0ull : share_log2 == 1 ? 0x5555555555555555ull
                               : share_log2 == 2 ? 0x1111111111111111ull : 0x0101010101010101ull) << part;
 
@@ -380,38 +382,37 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
             k_ready = k_ahead = true;
         }
     };
-    auto own_parts = [&]() {
-        own_part();
+    // a ring block, and what of its own a row walks beside it
+    auto slot = [&](int c, bool mine, int tile) {
+        if (mine) common_part(c, tile);
+        int blocks = mine ? 0 : 1;
+        if (mine && beside > 0) { blocks = 1; --beside; }
+        if (kLong && steps == kPacedSteps) blocks = kPacedSteps;
         if constexpr (kLong) {
 #pragma unroll 1
-            for (int r = 1; r < steps && jp >= 0; ++r) own_part();
-        }
+            for (; blocks > 0 && jp >= 0; --blocks) own_part();
+        } else if (blocks > 0 && jp >= 0) own_part();
     };
-    while (c0 >= 0 || jp >= 0) {
-        int n0 = -1, n1 = -1;
+    while (c0 >= 0) {                                          // uniform over the workgroup
+        // younger than this wavefront's DMA loads of the pair: the 16 K loads of the coming own block
+        if (k_ahead) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();                                       // the pair is in LDS for everyone; the other two tiles are free
         bool next_mine0 = false, next_mine1 = false;
-        if (c0 >= 0) {                                         // uniform over the workgroup
-            // younger than this wavefront's DMA loads of the pair: the 16 K loads of the coming own block
-            if (k_ahead) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();                                   // the pair is in LDS for everyone; the other two tiles are free
-            n0 = c1 >= 0 ? next_common(next_mine0) : -1;
-            n1 = n0 >= 0 ? next_common(next_mine1) : -1;
-            if (n0 >= 0) issue(n0, 2 - 2 * half);
-            if (n1 >= 0) issue(n1, 3 - 2 * half);
-            if (mine0) common_part(c0, 2 * half);
-        }
-        if (jp >= 0) own_parts();                              // per wavefront
-        if (c1 >= 0 && mine1) common_part(c1, 2 * half + 1);
-        if (jp >= 0 && c1 >= 0) own_parts();
-        if (c0 >= 0) {
-            c0 = n0;
-            c1 = n1;
-            mine0 = next_mine0;
-            mine1 = next_mine1;
-            half ^= 1;
-        }
+        const int n0 = c1 >= 0 ? next_common(next_mine0) : -1;
+        const int n1 = n0 >= 0 ? next_common(next_mine1) : -1;
+        if (n0 >= 0) issue(n0, 2 - 2 * half);
+        if (n1 >= 0) issue(n1, 3 - 2 * half);
+        k_ahead = false;
+        slot(c0, mine0, 2 * half);
+        if (c1 >= 0) slot(c1, mine1, 2 * half + 1);
+        c0 = n0;
+        c1 = n1;
+        mine0 = next_mine0;
+        mine1 = next_mine1;
+        half ^= 1;
     }
+    while (jp >= 0) own_part();
     if (kLong && tid == 0 && x.finished) in_step_finished(finished);       // the first wavefront for its workgroup: its row is one of eight neighbours
     if (share_log2 != 0) {                                     // uniform per workgroup
         // the ring was not used: 34 floats of every lane, lane by lane
