@@ -320,8 +320,9 @@ void stage1_kernel(const Stage1Params p) {
         for (int t = 0; t < kTok; ++t) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float mx = fmaxf(fmaxf(s[t][0][e], s[t][1][e]), fmaxf(s[t][2][e], s[t][3][e]));
-                const float m_new = fmaxf(m[t][e], mx * p.scale_log2);
+                // (fmaxf quiets its operands first, an instruction each: 131 072 tokens 5380 -> 5300 us)
+                const float mx = __builtin_elementwise_maximum(__builtin_elementwise_maximum(s[t][0][e], s[t][1][e]), __builtin_elementwise_maximum(s[t][2][e], s[t][3][e]));
+                const float m_new = __builtin_elementwise_maximum(m[t][e], mx * p.scale_log2);
                 float acc = l[t][e] * __builtin_amdgcn_exp2f(m[t][e] - m_new);
 #pragma unroll
                 for (int kt = 0; kt < 4; ++kt) acc += __builtin_amdgcn_exp2f(s[t][kt][e] * p.scale_log2 - m_new);
