@@ -348,6 +348,10 @@ int infllmv2_pack_kv(void* stream, const void* k, const void* v, const int32_t* 
 int infllmv2_pack_kv_and_topk(void* stream, const void* k, const void* v, const int32_t* cu_seqlens_k, void* workspace, size_t workspace_bytes,
                               int batch, int64_t total_k, int num_heads_k, int head_dim, int max_seqlen_k, const int64_t* k_strides,
                               const int64_t* v_strides, const int32_t* topk_idx, uint64_t* mask, int64_t rows, int topk, int n_uint64_per_row);
+/* ... and mask words of rows that all have the first blocks_set blocks. */
+int infllmv2_pack_kv_and_first(void* stream, const void* k, const void* v, const int32_t* cu_seqlens_k, void* workspace, size_t workspace_bytes,
+                               int batch, int64_t total_k, int num_heads_k, int head_dim, int max_seqlen_k, const int64_t* k_strides,
+                               const int64_t* v_strides, uint64_t* mask, int64_t rows, int blocks_set, int n_uint64_per_row);
 
 /* Scratch for infllmv2_varlen_bwd: the K/V block images, the transposed mask, D = rowsum(dO*O),
  * transposed per-token images of q and dout, fp32 dK/dV accumulators. */

@@ -53,6 +53,7 @@ SIGNATURES = {
     "infllmv2_fwd_kvcache_scores": [_p] * 8 + [_i, _i, _p, _sz] + [_i] * 5 + [_p] * 4 + [_i, _f],
     "infllmv2_fwd_kvcache_static": [_p] * 10 + [_i] * 7 + [_p] * 6 + [_i, _i, _f, _p, _p, _p, _i64, _i, _p, _p, _i, _i],
     "infllmv2_pack_kv": [_p, _p, _p, _p, _p, _sz, _i, _i64, _i, _i, _i, _p, _p],
+    "infllmv2_pack_kv_and_first": [_p, _p, _p, _p, _p, _sz, _i, _i64, _i, _i, _i, _p, _p, _p, _i64, _i, _i],
     "infllmv2_pack_kv_and_topk": [_p, _p, _p, _p, _p, _sz, _i, _i64, _i, _i, _i, _p, _p, _p, _p, _i64, _i, _i],
 }
 # entry points that exist once per element type: the plain name takes bfloat16, name + "_f16" IEEE half

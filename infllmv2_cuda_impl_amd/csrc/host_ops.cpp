@@ -506,6 +506,21 @@ std::tuple<Tensor, Tensor, OptTensor> select_mask(const Tensor& q, const Tensor&
                                                   int64_t block_size) {
     OptTensor images;
     Tensor mask;
+    const int64_t blocks = (max_len + kBlock - 1) / kBlock;
+    if (max_len > 1 && blocks <= topk && topk <= 2048 && block_size == kBlock && kernel_size > 0 && stride > 0 && block_size / stride == 4 && pack_early(q, k, v, max_len)) {
+        // every row takes all blocks of its sequence: nothing to score
+        check_compress(k, cu);
+        check_qkv(q.stride(-1) == 1 ? q : q.contiguous(), k, v, cu, cu, true);
+        DeviceGuard guard(k.device());
+        const int64_t batch = cu.numel() - 1, n64 = (blocks + 63) / 64;
+        images = image_workspace(k, batch);
+        mask = at::empty({k.size(1), q.size(0), n64}, q.options().dtype(at::kLong));
+        const S2 ks = rows_heads(k), vs = rows_heads(v);
+        check_rc(infllmv2_pack_kv_and_first(stream_of(q), ptr(k), ptr(v), iptr(cu), ptr(*images), static_cast<size_t>(images->numel()), as_int(batch), k.size(0),
+                                            as_int(k.size(1)), as_int(k.size(2)), as_int(max_len), ks.v, vs.v, static_cast<uint64_t*>(ptr(mask)),
+                                            k.size(1) * q.size(0), as_int(blocks), as_int(n64)), "pack_kv_and_first");
+        return {at::empty({k.size(1), 0, topk}, q.options().dtype(at::kInt)), mask, images};
+    }
     const auto [pooled, n64] = block_scores(q, k, cu, cu, max_len, max_len, local_blocks, init_blocks, std::nullopt, 0, scale, true, kernel_size,
                                             stride, block_size, false, &v, &images, topk, &mask);
     if (!mask.defined()) mask = topk_mask(pooled, topk, n64);

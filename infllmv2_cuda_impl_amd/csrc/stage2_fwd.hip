@@ -49,6 +49,27 @@ void pack_kv_and_topk_kernel(const PackParams p, int blocks, const int32_t* __re
     const int wave = threadIdx.x >> 6;
     topk_row_words(idx, mask, wg * kMaskRowsPerWg + wave, rows, k, n64, reinterpret_cast<unsigned long long*>(lds) + wave * n64, threadIdx.x & 63);
 }
+
+// The images, and mask words of rows that all have their first `set` blocks, kWordsPerWg to a workgroup: the front of a prefill whose sequences hold no more blocks than are
+// selected, in place of compressed keys, scores and selection.  Whole prefill in us, 2 KV heads,
+// 64 blocks: 500 tokens 23.8 -> 16.8, 1000 31.2 -> 26.6, 2048 61.1 -> 57.0, 4096 175 -> 169, four of 2000 194 -> 186; 30 of 300, 16 blocks, 98 -> 89.
+constexpr int kWordsPerWg = 2048;
+
+__global__ __launch_bounds__(256)
+void pack_kv_and_first_kernel(const PackParams p, int blocks, uint64_t* __restrict__ mask, int64_t words, int set, int n64) {
+    __shared__ __attribute__((aligned(16))) elem_bits rows[kPackElems];
+    if (static_cast<int>(blockIdx.x) < blocks) {
+        pack_block(p, blockIdx.x, blockIdx.y, blockIdx.z, rows);
+        return;
+    }
+    const int64_t wg = (static_cast<int64_t>(blockIdx.z) * gridDim.y + blockIdx.y) * (gridDim.x - blocks) + (blockIdx.x - blocks);
+    for (int i = threadIdx.x; i < kWordsPerWg; i += 256) {
+        const int64_t at = wg * kWordsPerWg + i;
+        if (at >= words) return;
+        const int from = n64 == 1 ? 0 : 64 * static_cast<int>(at % n64);
+        mask[at] = from + 64 <= set ? ~0ull : from < set ? (1ull << (set - from)) - 1ull : 0ull;
+    }
+}
 #endif
 
 }  // namespace IV2_NS
@@ -115,6 +136,25 @@ extern "C" int infllmv2_pack_kv_and_topk(void* stream, const void* k, const void
     if (lds < kPackElems * sizeof(elem_bits)) lds = kPackElems * sizeof(elem_bits);
     hipLaunchKernelGGL(pack_kv_and_topk_kernel, dim3(static_cast<unsigned>(blocks + mask_wgs), batch, num_heads_k), dim3(256), lds,
                        static_cast<hipStream_t>(stream), pp, blocks, topk_idx, mask, rows, topk, n_uint64_per_row);
+    IV2_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int infllmv2_pack_kv_and_first(void* stream, const void* k, const void* v, const int32_t* cu_seqlens_k, void* workspace, size_t workspace_bytes,
+                                          int batch, int64_t total_k, int num_heads_k, int head_dim, int max_seqlen_k, const int64_t* k_strides,
+                                          const int64_t* v_strides, uint64_t* mask, int64_t rows, int blocks_set, int n_uint64_per_row) {
+    IV2_CHECK(head_dim == kHeadDim, "pack_kv: this build only supports head_dim 128 (got %d)", head_dim);
+    IV2_CHECK(rows >= 0 && blocks_set >= 0 && n_uint64_per_row >= 0, "pack_kv_and_first: bad sizes");
+    IV2_CHECK(rows == 0 || n_uint64_per_row == 0 || mask, "pack_kv_and_first: null pointer");
+    if (int rc = check_pack(k, v, cu_seqlens_k, workspace, workspace_bytes, batch, total_k, num_heads_k, max_seqlen_k, k_strides, v_strides)) return rc;
+    const int blocks = total_k == 0 ? 0 : (max_seqlen_k + kBlockN - 1) / kBlockN;
+    const int64_t pairs = static_cast<int64_t>(batch) * num_heads_k, words = rows * n_uint64_per_row;
+    const int64_t mask_wgs = ((words + kWordsPerWg - 1) / kWordsPerWg + pairs - 1) / pairs;
+    if (blocks + mask_wgs == 0) return 0;
+    IV2_CHECK(blocks + mask_wgs <= max_workgroups(256), "pack_kv_and_first: too many rows");
+    const PackParams pp = pack_params(k, v, cu_seqlens_k, workspace, batch, total_k, num_heads_k, k_strides, v_strides, nullptr);
+    hipLaunchKernelGGL(pack_kv_and_first_kernel, dim3(static_cast<unsigned>(blocks + mask_wgs), batch, num_heads_k), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), pp, blocks, mask, words, blocks_set, n_uint64_per_row);
     IV2_LAUNCH_CHECK();
     return 0;
 }
