@@ -41,8 +41,11 @@ constexpr int kCompressPieces = kCompressMaxLds / 16 / kCompressThreads;      //
 // A workgroup takes rows_per_wg consecutive output rows of one KV head (128 elements of it).  Their windows are one
 // stretch of (rows - 1) * stride + kernel_size K rows: it goes into LDS with every load in flight at once, and then
 // one thread per two output elements adds its columns in window order.  Summing straight from memory, a window walked
-// row by row is a chain of kernel_size round trips: 26 us for the two sets of 2048 tokens where this takes 5.
+// row by row is a chain of kernel_size round trips: 26 us for the two sets of 2048 tokens where this takes 4.3.
 // Windows longer than the LDS holds are added up in several such steps.
+// kColumns (two rows and fewer, the wide windows): a thread adds one element's column instead, so that all four wavefronts add and the chain
+// has half the instructions: 128 keys every 64, two rows to a workgroup, of 2048 tokens 5.04 -> 4.53 us, of 131 072 19.5 -> 18.8.
+template <bool kColumns>
 __device__ __forceinline__ void compress_rows_of_head(const CompressParams& p, int wg, uint4* stage) {
     const int b = blockIdx.y, head = blockIdx.z / ((p.units_per_head + kCompressUnits - 1) / kCompressUnits);
     const int u0 = (blockIdx.z % ((p.units_per_head + kCompressUnits - 1) / kCompressUnits)) * kCompressUnits;
@@ -87,6 +90,18 @@ __device__ __forceinline__ void compress_rows_of_head(const CompressParams& p, i
         for (int t = 0; t < kCompressPieces; ++t)
             if ((tid + t * kCompressThreads) / kCompressUnits < staged) stage[tid + t * kCompressThreads] = piece[t];
         __syncthreads();
+        if constexpr (kColumns) {
+            const int row = tid >> 7;
+            if (row < nrows) {
+                int lo = row * p.stride - base, hi = lo + p.kernel_size;
+                lo = lo < 0 ? 0 : lo;
+                hi = hi < staged ? hi : staged;
+                const elem_bits* column = reinterpret_cast<const elem_bits*>(stage) + (tid & 127);
+#pragma unroll 16
+                for (int i = lo; i < hi; ++i) acc[0][0] += elem_to_f32(column[i * kCompressUnits * 8]);
+            }
+            continue;
+        }
         const uint32_t* words = reinterpret_cast<const uint32_t*>(stage) + lane;
 #pragma unroll
         for (int r = 0; r < kCompressRowsPerWg / 4; ++r) {
@@ -104,8 +119,14 @@ __device__ __forceinline__ void compress_rows_of_head(const CompressParams& p, i
             }
         }
     }
-    if (lane >= nu * 4) return;
     const float n = static_cast<float>(p.kernel_size);
+    if constexpr (kColumns) {
+        const int row = tid >> 7, col = tid & 127;
+        if (row < nrows && col < nu * 8)
+            p.out[((static_cast<int64_t>(before) + j0 + row) * p.num_heads + head) * p.units_per_head * 8 + u0 * 8 + col] = f32_to_elem_hw(acc[0][0] / n);
+        return;
+    }
+    if (lane >= nu * 4) return;
 #pragma unroll
     for (int r = 0; r < kCompressRowsPerWg / 4; ++r) {
         const int row = wave + 4 * r;
@@ -116,27 +137,30 @@ __device__ __forceinline__ void compress_rows_of_head(const CompressParams& p, i
     }
 }
 
+template <bool kColumns>
 __global__ __launch_bounds__(kCompressThreads)
 void compress_keys_kernel(const CompressParams p) {
     extern __shared__ uint4 stage[];
-    compress_rows_of_head(p, blockIdx.x, stage);
+    compress_rows_of_head<kColumns>(p, blockIdx.x, stage);
 }
 // two sets of the same K in one launch: the first wgs_a workgroups of a sequence and head belong to set a
+template <bool kColumnsA, bool kColumnsB>
 __global__ __launch_bounds__(kCompressThreads)
 void compress_keys_pair_kernel(const CompressParams pa, const CompressParams pb, int wgs_a) {
     extern __shared__ uint4 stage[];
-    if (static_cast<int>(blockIdx.x) < wgs_a) compress_rows_of_head(pa, blockIdx.x, stage);
-    else compress_rows_of_head(pb, blockIdx.x - wgs_a, stage);
+    if (static_cast<int>(blockIdx.x) < wgs_a) compress_rows_of_head<kColumnsA>(pa, blockIdx.x, stage);
+    else compress_rows_of_head<kColumnsB>(pb, blockIdx.x - wgs_a, stage);
 }
 
 // ... and the block images of the Stage-2 forward behind them: what prefill needs of K and V before its first scores, in one launch.  Bound by
 // latency like the two it replaces: a whole prefill of 512 tokens 34.9 -> 32.5 us, of 2048 (64 blocks selected) 83.9 -> 80.7, of 16 384 1363 -> 1356.
+template <bool kColumnsA, bool kColumnsB>
 __global__ __launch_bounds__(kCompressThreads)
 void compress_keys_and_pack_kernel(const CompressParams pa, const CompressParams pb, const PackParams pk, int wgs_a, int wgs_ab) {
     extern __shared__ uint4 stage[];
     const int wg = blockIdx.x;
-    if (wg < wgs_a) compress_rows_of_head(pa, wg, stage);
-    else if (wg < wgs_ab) compress_rows_of_head(pb, wg - wgs_a, stage);
+    if (wg < wgs_a) compress_rows_of_head<kColumnsA>(pa, wg, stage);
+    else if (wg < wgs_ab) compress_rows_of_head<kColumnsB>(pb, wg - wgs_a, stage);
     else pack_block(pk, wg - wgs_ab, blockIdx.y, blockIdx.z, reinterpret_cast<elem_bits*>(stage));
 }
 static_assert(kCompressThreads == 256, "the packing part is written for workgroups of 256");
@@ -266,6 +290,11 @@ using namespace IV2_NS;
 
 namespace {
 
+// workgroups per sequence and head; one writes cu_out in any case
+int row_workgroups(const CompressParams& p, int max_seqlen_k) {
+    const int max_rows = max_seqlen_k >= p.kernel_size ? (max_seqlen_k - p.kernel_size) / p.stride + 1 : 0;
+    return max_rows > p.first_row ? (max_rows - p.first_row + p.rows_per_wg - 1) / p.rows_per_wg : 1;
+}
 // checks and parameters of one set of compressed keys of packed sequences; wgs: workgroups per sequence and head
 int packed_params(const char* who, CompressParams& p, int& wgs, const void* k, void* out, const int32_t* cu_seqlens_k,
                   int32_t* cu_seqlens_out, int batch, int max_seqlen_k, int num_heads_k, int head_dim,
@@ -286,17 +315,29 @@ int packed_params(const char* who, CompressParams& p, int& wgs, const void* k, v
     p.kernel_size = kernel_size; p.stride = stride; p.first_row = first_row;
     // as many rows as fit the staging buffer together (8 at 32/16, 2 at 128/64), at least one
     const int lds_rows = kCompressMaxLds / (kCompressUnits * 16);
-    int rows_per_wg = lds_rows > kernel_size ? (lds_rows - kernel_size) / stride + 1 : 1;
+    const int rows_per_wg = lds_rows > kernel_size ? (lds_rows - kernel_size) / stride + 1 : 1;
     p.rows_per_wg = rows_per_wg < kCompressRowsPerWg ? rows_per_wg : kCompressRowsPerWg;
-    const int max_rows = max_seqlen_k >= kernel_size ? (max_seqlen_k - kernel_size) / stride + 1 : 0;
-    wgs = max_rows > first_row ? (max_rows - first_row + p.rows_per_wg - 1) / p.rows_per_wg : 1;   // one writes cu_out in any case
+    wgs = row_workgroups(p, max_seqlen_k);
     return 0;
+}
+// Half the rows to a workgroup where the launch leaves compute units idle: its windows then arrive with fewer loads to a thread, and the K rows
+// that two workgroups both read come from the L2.  A set on its own gains as long as all of
+// its workgroups run at once (kCompressAlone), us: 32 keys every 16 of 2048 tokens and two KV heads 4.18 -> 3.45, of 32 768 5.77 -> 4.36 (1024
+// workgroups), of 131 072 15.1 -> 16.4 (4096, not taken); 128 every 64 4.53 -> 4.15, 6.93 -> 5.50, 18.8 -> 23.5 (not taken).  Two sets share
+// the LDS of the larger (kCompressTogether): 2048 tokens 4.67 -> 4.29, 9000 tokens (560 workgroups) 5.06 -> 4.91, 20 011 (1250) 6.4 -> 6.8
+// (not taken).
+constexpr int64_t kCompressAlone = 1024, kCompressTogether = 640;
+void halve_rows(CompressParams& p, int& wgs, int max_seqlen_k) {
+    if (p.rows_per_wg > 1) p.rows_per_wg /= 2;
+    wgs = row_workgroups(p, max_seqlen_k);
 }
 size_t staging_bytes(const CompressParams& p) {
     const int64_t rows = static_cast<int64_t>(p.rows_per_wg - 1) * p.stride + p.kernel_size;
     const int64_t bytes = rows * kCompressUnits * 16;
     return static_cast<size_t>(bytes < kCompressMaxLds ? bytes : kCompressMaxLds);
 }
+// A column to a thread instead of two to a lane (compress_rows_of_head): with two rows and fewer half of the wavefronts would have no row
+bool by_columns(const CompressParams& p) { return p.rows_per_wg <= 2; }
 unsigned head_parts(const CompressParams& p) {
     return static_cast<unsigned>(p.num_heads * ((p.units_per_head + kCompressUnits - 1) / kCompressUnits));
 }
@@ -312,8 +353,9 @@ extern "C" int IV2_ENTRY(infllmv2_compress_keys)(void* stream, const void* k, vo
     if (int rc = packed_params("compress_keys", p, wgs, k, out, cu_seqlens_k, cu_seqlens_out, batch, max_seqlen_k, num_heads_k,
                                head_dim, k_row_stride, k_head_stride, kernel_size, stride, first_row))
         return rc;
-    hipLaunchKernelGGL(compress_keys_kernel, dim3(wgs, batch, head_parts(p)), dim3(kCompressThreads), staging_bytes(p),
-                       static_cast<hipStream_t>(stream), p);
+    if (2 * static_cast<int64_t>(wgs) * batch * head_parts(p) <= kCompressAlone) halve_rows(p, wgs, max_seqlen_k);
+    auto kernel = by_columns(p) ? compress_keys_kernel<true> : compress_keys_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3(wgs, batch, head_parts(p)), dim3(kCompressThreads), staging_bytes(p), static_cast<hipStream_t>(stream), p);
     IV2_LAUNCH_CHECK();
     return 0;
 }
@@ -330,8 +372,14 @@ extern "C" int IV2_ENTRY(infllmv2_compress_keys_pair)(void* stream, const void* 
     if (int rc = packed_params("compress_keys_pair", pb, wgs_b, k, out_b, cu_seqlens_k, cu_seqlens_out_b, batch, max_seqlen_k,
                                num_heads_k, head_dim, k_row_stride, k_head_stride, kernel_size_b, stride_b, 0))
         return rc;
+    if (2 * (static_cast<int64_t>(wgs_a) + wgs_b) * batch * head_parts(pa) <= kCompressTogether) {
+        halve_rows(pa, wgs_a, max_seqlen_k);
+        halve_rows(pb, wgs_b, max_seqlen_k);
+    }
     const size_t lds = staging_bytes(pa) > staging_bytes(pb) ? staging_bytes(pa) : staging_bytes(pb);
-    hipLaunchKernelGGL(compress_keys_pair_kernel, dim3(wgs_a + wgs_b, batch, head_parts(pa)), dim3(kCompressThreads), lds,
+    auto kernel = by_columns(pa) ? (by_columns(pb) ? compress_keys_pair_kernel<true, true> : compress_keys_pair_kernel<true, false>)
+                                 : (by_columns(pb) ? compress_keys_pair_kernel<false, true> : compress_keys_pair_kernel<false, false>);
+    hipLaunchKernelGGL(kernel, dim3(wgs_a + wgs_b, batch, head_parts(pa)), dim3(kCompressThreads), lds,
                        static_cast<hipStream_t>(stream), pa, pb, wgs_a);
     IV2_LAUNCH_CHECK();
     return 0;
@@ -355,9 +403,15 @@ extern "C" int IV2_ENTRY(infllmv2_compress_keys_and_pack)(void* stream, const vo
         return rc;
     const PackParams pk = pack_params(k, v, cu_seqlens_k, workspace, batch, total_k, num_heads_k, k_strides, v_strides, nullptr);
     const int blocks = total_k == 0 ? 0 : (max_seqlen_k + kBlockN - 1) / kBlockN;
+    if ((2 * (static_cast<int64_t>(wgs_a) + wgs_b) + blocks) * batch * num_heads_k <= kCompressTogether) {
+        halve_rows(pa, wgs_a, max_seqlen_k);
+        halve_rows(pb, wgs_b, max_seqlen_k);
+    }
     size_t lds = staging_bytes(pa) > staging_bytes(pb) ? staging_bytes(pa) : staging_bytes(pb);
     if (lds < kPackElems * sizeof(elem_bits)) lds = kPackElems * sizeof(elem_bits);
-    hipLaunchKernelGGL(compress_keys_and_pack_kernel, dim3(wgs_a + wgs_b + blocks, batch, num_heads_k), dim3(kCompressThreads), lds,
+    auto kernel = by_columns(pa) ? (by_columns(pb) ? compress_keys_and_pack_kernel<true, true> : compress_keys_and_pack_kernel<true, false>)
+                                 : (by_columns(pb) ? compress_keys_and_pack_kernel<false, true> : compress_keys_and_pack_kernel<false, false>);
+    hipLaunchKernelGGL(kernel, dim3(wgs_a + wgs_b + blocks, batch, num_heads_k), dim3(kCompressThreads), lds,
                        static_cast<hipStream_t>(stream), pa, pb, pk, wgs_a, wgs_a + wgs_b);
     IV2_LAUNCH_CHECK();
     return 0;
