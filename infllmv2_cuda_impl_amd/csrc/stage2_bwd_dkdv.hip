@@ -16,7 +16,7 @@
 // pipe the busiest unit of the kernel.
 //
 // Query-side data path.  q and dout of a token pair are gathered straight from the caller's
-// tensors into a two-stage LDS ring by LDS-DMA loads issued one pair ahead (no registers, no
+// tensors into a two-stage LDS ring by LDS-DMA loads issued one pair (a step) ahead (no registers, no
 // transposed copies in memory; wavefront 0 fetches q, wavefront 1 dout, one workgroup barrier per
 // pair): the ring holds them as A-operand fragments of the first two GEMMs, and the transposed
 // operands of dV^T = dO^T P and dK^T = Q^T dS are read from the same bytes with ds_read_b64_tr_b16.
@@ -33,9 +33,10 @@
 namespace IV2_NS {
 
 constexpr int kGroupWords = 32;                                // one mask word per lane of the lower half-wavefront: a group is 2048 tokens
-constexpr int kStage = 16384 + 512 + 512;                      // q a|b, dout a|b (4 KiB each), the pair's 64 row scalars; padded so that two stages are the flush tile
+constexpr int kStage = 16384 + 512 + 512;                      // q a|b, dout a|b (4 KiB each), the step's 64 row scalars; padded so that two stages are the flush tile
 constexpr int kWaveLds = 2 * kStage;                           // = 64 rows x 132 floats: also the flush tile
 constexpr int kFlushPitch = 132;                               // floats per key row of the flush tile
+constexpr int kListTokens = 512 + 16;                           // no item holds more than 512, and the last step is filled up
 constexpr int kWaveTiles = 2;                                  // 16-key tiles per wavefront: a wavefront owns 32 of the block's 64 keys
 
 typedef short short4v __attribute__((ext_vector_type(4)));
@@ -92,9 +93,12 @@ __device__ __forceinline__ uint64_t lowest_set_bits(uint64_t v, int count) {
     return __builtin_popcountll(low) < count ? v : low;
 }
 
+// kPack: query tokens to a tile of 16 rows.  Groups of up to 8 heads put two there (rows 0 to 7 and 8 to 15), so that a step serves four tokens: nothing but
+// the source addresses of the transfers and the rows' key limits depend on it.  Kernel in us with one | two, groups of 8: 2493 tokens (32 blocks selected)
+// 143 | 87, 10179 (64) 1060 | 628, 57466 in four sequences (16) 1342 | 704.
 // kColSlice: query tokens per slice.  kEven: the tokens of a group that selected a block are dealt out evenly; else a slice is a work item, light ones
 // are merged.
-template <bool kCausal, int kColSlice, bool kEven>
+template <bool kCausal, int kColSlice, bool kEven, int kPack>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void bwd_dkdv_wave_kernel(const BwdParams p) {
     constexpr int kSliceWords = kColSlice / 64;                // mask words per slice (a power of two)
@@ -168,7 +172,8 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
     // where a short slice holds 128, and the longest items decided the kernel's time; whole training pass of 12000 tokens, 16
     // blocks selected: 1535 against 1435 us.)  Every workgroup of the group takes the same decision from the
     // group's 32 mask words (lane l < 32 holds word l; a slice is kSliceWords consecutive lanes).
-    unsigned long long* wbuf = reinterpret_cast<unsigned long long*>(ring + kWaveLds);      // [kGroupWords]
+    uint16_t* list = reinterpret_cast<uint16_t*>(ring + kWaveLds);      // the item's tokens, counted from the group's first: [kListTokens]
+    int tokens = 0;                                            // how many
     const int group = slice / kGroupSlices, sub = slice % kGroupSlices;
     const int64_t w0 = static_cast<int64_t>(group) * kGroupWords;
     {
@@ -196,7 +201,6 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
             if (item >= items) return;                         // uniform
             const int each = (total + items - 1) / items, from = item * each - (upto - cnt);
             wv = lowest_set_bits(wv, from + each) & ~lowest_set_bits(wv, from);
-            if (lane < kGroupWords) wbuf[lane] = wv;
         } else {
 #pragma unroll
             for (int off = 1; off < kSliceWords; off <<= 1) cnt += __shfl_xor(cnt, off);   // tokens of this lane's slice that selected the block
@@ -223,10 +227,26 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
                 if (__builtin_ctzll(mates) / kSliceWords != sub) return;                // uniform: another slice collects
                 keep = (mates >> lane) & 1ull;
             }
-            if (lane < kGroupWords) wbuf[lane] = keep ? wv : 0ull;
+            wv = keep ? wv : 0ull;
         }
+        // The item's tokens as a list, so that a step takes the next ones wherever they lie and learns them from one read, made a step ahead.  Walking the
+        // words' bits with scalar instructions between the wait for a step's rows and the request for the next ones, and ending a pair at the end of a word: us with
+        // the walk | the list, whole kernel, 71 552 packed tokens (64 blocks) 8250 | 8100, 6741 in four sequences (16 blocks) 240 | 230.
+        // Both wavefronts write the same list, each for itself: a lane to a token of a word.  What the last step has no tokens for repeats the last.
+        uint64_t words = __ballot(lane < kGroupWords && wv != 0ull);
+        int last = 0;
+        while (words != 0ull) {
+            const int w = __builtin_ctzll(words);
+            words &= words - 1ull;
+            const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(wv), w), hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(wv >> 32), w);
+            const uint64_t v = (static_cast<uint64_t>(hi) << 32) | lo;
+            if ((v >> lane) & 1ull) list[tokens + __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0))] = static_cast<uint16_t>(w * 64 + lane);
+            tokens += __builtin_popcountll(v);
+            last = w * 64 + 63 - __builtin_clzll(v);
+        }
+        if (tokens == 0) return;                               // uniform
+        if (lane < 2 * kPack) list[tokens + lane] = static_cast<uint16_t>(last);
     }
-    __syncthreads();
 
     // ---- K and V of the block: B operands, resident in registers ----
     elem8 kreg[kWaveTiles][4], vreg[kWaveTiles][4];
@@ -250,37 +270,38 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
             dVt[dt][kt] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
 
-    // ---- token-pair cursor over the kept mask words (scalar state) ----
-    int cw = -1;
-    uint64_t bits = 0ull;
-    auto next_pair = [&](int64_t& ta, int64_t& tb, bool& has_b) -> bool {
-        while (bits == 0ull) {
-            if (++cw >= kGroupWords) return false;
-            const uint64_t v = wbuf[cw];
-            const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
-            const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
-            bits = (static_cast<uint64_t>(hi) << 32) | lo;
+    // ---- the tokens of a step: 2 * kPack entries of the list (scalar state) ----
+    struct Step { int tok[2 * kPack]; };
+    const int first_token = static_cast<int>(w0 << 6);         // packed token indices fit 31 bits
+    uint32_t ahead[kPack];                                     // the entries of the step after the next one asked for
+    auto read_ahead = [&](int from) {
+#pragma unroll
+        for (int i = 0; i < kPack; ++i) ahead[i] = reinterpret_cast<const uint32_t*>(list + from)[i];
+    };
+    auto next_step = [&]() {
+        Step step;
+#pragma unroll
+        for (int i = 0; i < kPack; ++i) {
+            const uint32_t two = __builtin_amdgcn_readfirstlane(ahead[i]);
+            step.tok[2 * i] = first_token + static_cast<int>(two & 0xffffu);
+            step.tok[2 * i + 1] = first_token + static_cast<int>(two >> 16);
         }
-        const int64_t base = (w0 + cw) << 6;
-        ta = base + __builtin_ctzll(bits);
-        bits &= bits - 1ull;
-        has_b = bits != 0ull;
-        tb = has_b ? base + __builtin_ctzll(bits) : ta;
-        bits &= bits - 1ull;                                   // no-op on zero
-        return true;
+        return step;
     };
 
-    // ---- LDS-DMA of one pair: per 64-byte chunk c of the 16 head rows, one 1 KiB transfer ----
+    // ---- LDS-DMA of one step: per 64-byte chunk c of a tile's 16 rows, one 1 KiB transfer ----
     const uint32_t ring_lds = __builtin_amdgcn_readfirstlane(lds_addr(ring));
     // Which 16 bytes a lane fetches: the four lanes of a quad take the four 16-byte pieces of one head's 64-byte
     // chunk, so a quad is one contiguous 64-byte request.  LDS unit l = 4 * head + j of a chunk then holds piece
     // (j + head / 4) % 4: the rotation makes the operand reads below bank-conflict free.
     const int dma_piece = ((lane & 3) + (lane >> 4)) & 3;
-    const int dma_head = (lane >> 2) < p.group ? (lane >> 2) : p.group - 1;    // rows beyond the group repeat its last head: their LSE is +inf
+    // rows beyond the group repeat its last head: their LSE is +inf
+    const int dma_row = (lane >> 2) & (16 / kPack - 1), dma_head = dma_row < p.group ? dma_row : p.group - 1;
     // byte offsets inside one token and KV head; wavefront 0 fetches q, wavefront 1 dout
     const uint32_t q_lane = static_cast<uint32_t>((dma_head * (wave == 0 ? p.q_grp : p.do_grp) + 8 * dma_piece) * 2);
-    const uint32_t do_lane = q_lane;
-    const uint32_t stat_lane = static_cast<uint32_t>((lane & 31) * 4);
+    const uint32_t stat_lane = static_cast<uint32_t>(((lane & 16) + (lane & (16 / kPack - 1))) * 4);
+    // kPack == 2: lanes whose row (in the rows' transfers) and whose scalar (in theirs) belong to the second token of a tile
+    const bool row_second = kPack == 2 && (lane & 32), stat_second = kPack == 2 && (lane & 8);
     const elem_bits* q_head = p.q + static_cast<int64_t>(h) * p.q_kvh;
     const elem_bits* do_head = p.dout + static_cast<int64_t>(h) * p.do_kvh;
     const float* stat_head = p.rowstat + static_cast<int64_t>(h) * p.total_q * 32;
@@ -290,27 +311,32 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
     const unsigned char* q_bytes = reinterpret_cast<const unsigned char*>(q_head);
     const unsigned char* do_bytes = reinterpret_cast<const unsigned char*>(do_head);
     const unsigned char* stat_bytes = reinterpret_cast<const unsigned char*>(stat_head);
-    auto issue = [&](int64_t ta, int64_t tb, int stage) {
+    auto issue = [&](const Step& step, int stage) {
         const uint32_t st = ring_lds + stage * kStage;
-        const uint64_t ua = static_cast<uint32_t>(ta), ub = static_cast<uint32_t>(tb);     // packed token indices fit 31 bits
-        const unsigned char* qa = q_bytes + ua * q_tok_bytes;
-        const unsigned char* qb = q_bytes + ub * q_tok_bytes;
-        const unsigned char* da = do_bytes + ua * do_tok_bytes;
-        const unsigned char* db = do_bytes + ub * do_tok_bytes;
-        // the two wavefronts share the pair's transfers: wavefront 0 fetches q, wavefront 1 dout
+        const uint64_t ua = static_cast<uint32_t>(step.tok[0]), ub = static_cast<uint32_t>(step.tok[kPack]);
+        // the second token of a tile lies at most a group of tokens behind the first (the launcher checks that this fits 32 bits)
+        const uint32_t da = kPack == 2 ? static_cast<uint32_t>(step.tok[kPack - 1] - step.tok[0]) : 0u;
+        const uint32_t db = kPack == 2 ? static_cast<uint32_t>(step.tok[2 * kPack - 1] - step.tok[kPack]) : 0u;
+        const uint32_t tok_bytes = wave == 0 ? q_tok_bytes : do_tok_bytes;
+        const uint32_t row_a = q_lane + (row_second ? da * tok_bytes : 0u), row_b = q_lane + (row_second ? db * tok_bytes : 0u);
+        // the two wavefronts share the step's transfers: wavefront 0 fetches q, wavefront 1 dout
         if (wave == 0) {
-            dma16<0, 0>(qa, q_lane, st);        dma16<64, 1024>(qa, q_lane, st);
-            dma16<128, 2048>(qa, q_lane, st);   dma16<192, 3072>(qa, q_lane, st);
-            dma16<0, 4096>(qb, q_lane, st);     dma16<64, 5120>(qb, q_lane, st);
-            dma16<128, 6144>(qb, q_lane, st);   dma16<192, 7168>(qb, q_lane, st);
-            // token a's [lse * log2e (16) | D (16)] (both half-wavefronts fetch the same 128 bytes)
-            dma4<16384>(stat_bytes + (ua << 7), stat_lane, st);
+            const unsigned char* qa = q_bytes + ua * q_tok_bytes;
+            const unsigned char* qb = q_bytes + ub * q_tok_bytes;
+            dma16<0, 0>(qa, row_a, st);        dma16<64, 1024>(qa, row_a, st);
+            dma16<128, 2048>(qa, row_a, st);   dma16<192, 3072>(qa, row_a, st);
+            dma16<0, 4096>(qb, row_b, st);     dma16<64, 5120>(qb, row_b, st);
+            dma16<128, 6144>(qb, row_b, st);   dma16<192, 7168>(qb, row_b, st);
+            // tile a's [lse * log2e (16) | D (16)] (both half-wavefronts fetch the same 128 bytes)
+            dma4<16384>(stat_bytes + (ua << 7), stat_lane + (stat_second ? da << 7 : 0u), st);
         } else {
-            dma16<0, 8192>(da, do_lane, st);    dma16<64, 9216>(da, do_lane, st);
-            dma16<128, 10240>(da, do_lane, st); dma16<192, 11264>(da, do_lane, st);
-            dma16<0, 12288>(db, do_lane, st);   dma16<64, 13312>(db, do_lane, st);
-            dma16<128, 14336>(db, do_lane, st); dma16<192, 15360>(db, do_lane, st);
-            dma4<16384 + 256>(stat_bytes + (ub << 7), stat_lane, st);
+            const unsigned char* oa = do_bytes + ua * do_tok_bytes;
+            const unsigned char* ob = do_bytes + ub * do_tok_bytes;
+            dma16<0, 8192>(oa, row_a, st);    dma16<64, 9216>(oa, row_a, st);
+            dma16<128, 10240>(oa, row_a, st); dma16<192, 11264>(oa, row_a, st);
+            dma16<0, 12288>(ob, row_b, st);   dma16<64, 13312>(ob, row_b, st);
+            dma16<128, 14336>(ob, row_b, st); dma16<192, 15360>(ob, row_b, st);
+            dma4<16384 + 256>(stat_bytes + (ub << 7), stat_lane + (stat_second ? db << 7 : 0u), st);
         }
     };
 
@@ -332,37 +358,37 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
     // operand fragment (head n, piece g) of a chunk: unit 4 n + (g - n / 4) % 4
     const int frag_unit = 4 * n + ((g - (n >> 2)) & 3);
 
-    int64_t ta, tb;
-    bool has_b;
-    bool more = next_pair(ta, tb, has_b);
-    if (more) issue(ta, tb, 0);
+    read_ahead(0);
+    Step now = next_step();
+    read_ahead(2 * kPack);
+    issue(now, 0);
     int stage = 0;
-    while (more) {
-        // This wavefront's half of the pair's transfers has landed (nothing younger is in flight: the next pair goes out
+    for (int done = 0; done < tokens; done += 2 * kPack) {
+        // This wavefront's half of the step's transfers has landed (nothing younger is in flight: the next step goes out
         // below); the barrier adds the other wavefront's half and says that both are done with the other stage.
         __builtin_amdgcn_s_waitcnt(0x0F70);                    // vmcnt(0)
         __syncthreads();
-        int64_t na, nb2;
-        bool nhb;
-        const bool have_next = next_pair(na, nb2, nhb);
-        if (have_next) issue(na, nb2, stage ^ 1);
+        Step next = now;
+        if (done + 2 * kPack < tokens) {
+            next = next_step();
+            issue(next, stage ^ 1);
+            read_ahead(done + 4 * kPack);
+        }
         const unsigned char* st = ring + stage * kStage;
 
-        int lim_a, lim_b;                                      // in-block key index limit (inclusive)
-        {
-            const int valid = Sk - j * kBlockN - 1;
-            lim_a = valid; lim_b = valid;
+        int lim[2 * kPack];                                    // in-block key index limit (inclusive) of each token
+        bool edge = false;
+#pragma unroll
+        for (int i = 0; i < 2 * kPack; ++i) {
+            lim[i] = Sk - j * kBlockN - 1;
             if (kCausal) {
-                const int ca = static_cast<int>(ta - q0) + Sk - Sq - j * kBlockN;
-                const int cb = static_cast<int>(tb - q0) + Sk - Sq - j * kBlockN;
-                lim_a = ca < lim_a ? ca : lim_a;
-                lim_b = cb < lim_b ? cb : lim_b;
+                const int seen = now.tok[i] - q0 + Sk - Sq - j * kBlockN;
+                lim[i] = seen < lim[i] ? seen : lim[i];
             }
-            if (!has_b) lim_b = -1;
+            if (done + i >= tokens) lim[i] = -1;
+            edge |= lim[i] < kBlockN - 1;
         }
-
         const float* scal = reinterpret_cast<const float*>(st + 16384);
-        const bool edge = (lim_a < kBlockN - 1) || (lim_b < kBlockN - 1);
         // Per wavefront 64 MFMAs in four GEMM phases with the softmax backward between them; the other wavefront of the
         // SIMD fills the matrix pipeline while this one does vector work:
         //   A  S = Q K^T                       (both tokens, this wavefront's 32 keys; a fragment read from LDS feeds 2 MFMAs)
@@ -438,6 +464,8 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
 #pragma unroll
             for (int kt = 0; kt < kWaveTiles; ++kt) {
                 const int key0 = 16 * (kWaveTiles * wave + kt);
+                // the lane's rows 4 g .. 4 g + 3 are of the tile's second token where kPack == 2 and g >= 2
+                const int lim_a = kPack == 2 && g >= 2 ? lim[kPack - 1] : lim[0], lim_b = kPack == 2 && g >= 2 ? lim[2 * kPack - 1] : lim[kPack];
                 const bool off_a = n > lim_a - key0, off_b = n > lim_b - key0;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -483,8 +511,7 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        more = have_next;
-        ta = na; tb = nb2; has_b = nhb;
+        now = next;
         stage ^= 1;
     }
 
@@ -592,7 +619,7 @@ static double selected_pairs(int batch, int num_heads_k, int64_t total_q, int64_
 }
 
 template <int kColSlice, bool kEven>
-static int launch_bwd_dkdv_sliced(hipStream_t st, const BwdParams& p_in, int batch, int max_seqlen_q, bool causal, int item_tokens) {
+static int launch_bwd_dkdv_sliced(hipStream_t st, const BwdParams& p_in, int batch, int max_seqlen_q, bool causal, bool pack, int item_tokens) {
     BwdParams p = p_in;
     p.dkdv_item = item_tokens;
     constexpr int kGroupSlices = kGroupWords * 64 / kColSlice;
@@ -626,15 +653,28 @@ static int launch_bwd_dkdv_sliced(hipStream_t st, const BwdParams& p_in, int bat
     IV2_CHECK(p.q_tok >= 0 && p.q_tok < (1ll << 31) && p.do_tok >= 0 && p.do_tok < (1ll << 31) && p.total_q < (1ll << 31),
               "varlen_bwd: token strides of q and dout must lie in [0, 2^31) elements");
     const dim3 grid(static_cast<unsigned>(items), batch, p.num_heads_k);
-    const size_t lds = kWaveLds + kGroupWords * 8;
-    if (causal) hipLaunchKernelGGL((bwd_dkdv_wave_kernel<true, kColSlice, kEven>), grid, dim3(128), lds, st, p);
-    else hipLaunchKernelGGL((bwd_dkdv_wave_kernel<false, kColSlice, kEven>), grid, dim3(128), lds, st, p);
+    const size_t lds = kWaveLds + kListTokens * 2;
+    auto kernel = causal ? bwd_dkdv_wave_kernel<true, kColSlice, kEven, 1> : bwd_dkdv_wave_kernel<false, kColSlice, kEven, 1>;
+    if constexpr (kColSlice >= kDkdvSliceSmall) {              // the shortest items are not asked for with two tokens to a tile
+        if (pack) kernel = causal ? bwd_dkdv_wave_kernel<true, kColSlice, kEven, 2> : bwd_dkdv_wave_kernel<false, kColSlice, kEven, 2>;
+    }
+    hipLaunchKernelGGL(kernel, grid, dim3(128), lds, st, p);
     IV2_LAUNCH_CHECK();
     return 0;
 }
 
+// Two tokens to a tile of 16 rows: groups of up to 8 heads, where the second token of a tile, at most a group of tokens behind the first, is within the
+// transfers' 32-bit byte offsets.  An item's steps are half as many for the same tokens.
+static bool packs_tokens(const BwdParams& p) {
+    auto near = [](int64_t tok, int64_t grp) {
+        return grp >= 0 && grp < (1ll << 31) && (kGroupWords * 64 - 1) * tok + 7 * grp + kHeadDim <= 1ll << 31;
+    };
+    return p.group <= 8 && near(p.q_tok, p.q_grp) && near(p.do_tok, p.do_grp);
+}
+
 int launch_bwd_dkdv_wave(hipStream_t st, const BwdParams& p, int batch, int max_seqlen_q, int max_seqlen_k, bool causal, int most_selected) {
     const int64_t groups = (p.total_q + kGroupWords * 64 - 1) / (kGroupWords * 64);
+    const bool pack = packs_tokens(p);
     if (p.det_slots == nullptr && groups <= kDkdvEvenGroups) {
         // How many tokens to an item.  Where all items can run at once the kernel is fastest with about 600 of them, three to a CU at most: a fourth on some CUs adds
         // 40 us.  So `fit` tokens, 64 at least (a flush costs what 10 tokens do) and 192 at most; past that several rounds of 128, which balance better, and for still
@@ -645,13 +685,21 @@ int launch_bwd_dkdv_wave(hipStream_t st, const BwdParams& p, int batch, int max_
         const double pairs = selected_pairs(batch, p.num_heads_k, p.total_q, p.total_k, max_seqlen_q, max_seqlen_k, causal,
                                             most_selected < 0 ? -most_selected : most_selected);
         const double fit = pairs / 600., many = pairs / 6300.;
-        if (fit < 128.) return launch_bwd_dkdv_sliced<64, true>(st, p, batch, max_seqlen_q, causal, fit > 64. ? static_cast<int>(fit) : 64);
+        if (pack) {
+            // A token costs half as much, a flush as much as before.  Whole training pass in us with 64 / 96 / 128 / 160 / 192 / 224 / 256 / 320 tokens, groups of 8: 2493 tokens,
+            // 32 blocks selected 314 / 294 / 269 / 267 / 275 / 285 / 294 / 316; 1343 + 1562, 16 blocks 241 / 241 / 219 / 221 / 231 / 242 / 252 / 273; 7914, 32 blocks 1237 / 1143 /
+            // 1124 / 1084 / 1077 / 1079 / 1080 / 1085; 10179, 64 blocks 2543 / 2351 / 2253 / 2228 / 2217 / 2204 / 2199 / 2219; 13922, 32 blocks 2359 / 2215 / 2146 / 2148 / 2090 /
+            // 2088 / 2082 / 2095.
+            const int item = fit <= 192. ? (fit > 128. ? static_cast<int>(fit) : 128) : many <= 128. ? 192 : many < 170. ? static_cast<int>(1.5 * many) : 256;
+            return launch_bwd_dkdv_sliced<kDkdvSliceSmall, true>(st, p, batch, max_seqlen_q, causal, pack, item);
+        }
+        if (fit < 128.) return launch_bwd_dkdv_sliced<64, true>(st, p, batch, max_seqlen_q, causal, pack, fit > 64. ? static_cast<int>(fit) : 64);
         const int item = fit <= 192. ? static_cast<int>(fit) : many <= 128. ? 128 : many < 256. ? static_cast<int>(many) : 256;
-        return launch_bwd_dkdv_sliced<kDkdvSliceSmall, true>(st, p, batch, max_seqlen_q, causal, item);
+        return launch_bwd_dkdv_sliced<kDkdvSliceSmall, true>(st, p, batch, max_seqlen_q, causal, pack, item);
     }
     if (dkdv_slice_tokens(max_seqlen_q, p.det_slots != nullptr) == kDkdvSliceSmall)
-        return launch_bwd_dkdv_sliced<kDkdvSliceSmall, false>(st, p, batch, max_seqlen_q, causal, 0);
-    return launch_bwd_dkdv_sliced<kDkdvSlice, false>(st, p, batch, max_seqlen_q, causal, 0);
+        return launch_bwd_dkdv_sliced<kDkdvSliceSmall, false>(st, p, batch, max_seqlen_q, causal, pack, 0);
+    return launch_bwd_dkdv_sliced<kDkdvSlice, false>(st, p, batch, max_seqlen_q, causal, pack, 0);
 }
 
 }  // namespace IV2_NS
