@@ -61,11 +61,14 @@ struct Stage1Params {
 };
 
 // 8 wavefronts x 2 tokens: 112 registers, so four wavefronts share a SIMD and the exp-heavy VALU work of one hides
-// behind the MFMAs of another (4 x 4 at two wavefronts per SIMD measures 6 % slower, 8 x 1 15 % slower where the launch fills the chip; where it does not: launch_stage1)
+// behind the MFMAs of another (4 x 4 at two wavefronts per SIMD measures 6 % slower, 8 x 1 2 to 10 % slower where the launch fills the chip; where it does not: launch_stage1)
 constexpr int kTokPerWave = 2;
 constexpr int kWavesS1 = 8;
 constexpr int kWavesPerSimdS1 = 4;
 constexpr int kTokPerBlock = kTokPerWave * kWavesS1;   // 16
+// 8 x 1 takes 60 registers: eight wavefronts to a SIMD, four workgroups to a CU, or three where LDS ends it (512 blocks of 16 tokens pooled).  Held to four wavefronts
+// like 8 x 2, a third workgroup waited for one of the first two: scores of 2048 | 2049 queries against 20 011 keys 36.2 | 49.3 us, now 36.4 | 42.2.
+constexpr int waves_per_simd(int tok, int items, int pack) { return tok > 1 ? kWavesPerSimdS1 : items * pack >= 16 ? 6 : 8; }
 constexpr int kKeysPerBlock = 4;                       // compressed keys (stride 16) per 64-token key block
 
 __device__ __forceinline__ int trunc_div(int a, int b) { return a / b; }   // C++ semantics on purpose
@@ -184,7 +187,7 @@ __device__ __forceinline__ void pool_quads(float a, float b, float prev_a, float
 // kTok: tiles of 16 rows of a wavefront, a token each: 2 or, in launches of few workgroups (launch_stage1), 1.  kPack == 2: two tokens to a tile, heads 0 to 7 of
 // its rows 0 to 7 and 8 to 15.  The head sums then end where the two halves of the rows would have been added.  A token's row is the same bits in every form.
 template <bool kCausal, bool kPool, int kItems = 0, bool kShared = false, int kTok = kTokPerWave, int kPack = 1>
-__global__ __launch_bounds__(64 * kWavesS1) __attribute__((amdgpu_waves_per_eu(kWavesPerSimdS1, kWavesPerSimdS1)))
+__global__ __launch_bounds__(64 * kWavesS1) __attribute__((amdgpu_waves_per_eu(waves_per_simd(kTok, kItems, kPack), kTok == 1 ? 8 : kWavesPerSimdS1)))
 void stage1_kernel(const Stage1Params p) {
     constexpr int kMine = kTok * kPack, kTokens = kMine * kWavesS1;                 // tokens of a wavefront and of the workgroup
     __shared__ uint4 tile[2][1024];                            // two 16 KiB operand-ordered key tiles
@@ -628,21 +631,27 @@ int launch_stage1(const char* who, void* stream, const void* q, const void* k, c
     const int64_t wgs = static_cast<int64_t>((max_seqlen_q + kTokPerBlock * pack - 1) / (kTokPerBlock * pack)) * batch * num_heads_k;
     const int64_t fill = wgs > 0 ? 256 / wgs : 1, most = max_seqlen_k / 256;
     p.splits = p.mask != nullptr || fill < 2 || most < 2 ? 1 : static_cast<int>(fill < most ? fill : most);
-    // One token to a wavefront (two, where two share the rows), twice the workgroups, up to 384 of the others: fewer than one and a half to a CU that holds two.  The time is then that of the CU with the most, half a
+    // One token to a wavefront (two, where two share the rows), twice the workgroups, up to 384 of the others: three to a CU.  The time is then that of the CU with the most, half a
     // workgroup finer, and of the chain of one tile (one wavefront's products and exponentials behind the other's on a SIMD), which is shorter.  Scores alone, us, two tokens | one, 2 KV heads, 20 011 keys:
-    // 17 queries 18.8 | 12.5, 256 19.3 | 13.3, 512 20.1 | 20.6, 1100 35.1 | 32.9, 2049 54.0 | 49.7, 3000 (376 workgroups) 56.1 | 51.1; 3500 (438) 57.2 | 62.8, 4096 60.3 | 64.1; 60 000
-    // keys, one head, 2049 89.6 | 73.5; selecting prefill of 1000 tokens 15.2 | 12.4, 2048 17.1 | 15.8, 3000 22.4 | 21.5.
+    // 17 queries 18.8 | 12.5, 256 19.3 | 13.3, 512 20.1 | 20.6, 1100 35.1 | 32.9, 2049 54.0 | 42.2, 3000 (376 workgroups) 56.1 | 49.4; 3100 (388) 55.3 | 58.8, 4096 60.0 | 63.6; 131 072
+    // keys, 2049 344 | 244, 3100 313 | 362; selecting prefill of 1000 tokens 15.2 | 12.4.
+    // Selecting, a workgroup walks what its own tokens see, from one tile to all of them, and smaller ones end together: always where two tokens share the rows, else up to 10 240 tokens; longer, the
+    // keys' second trip from L2 costs more.  Selection in us, two tokens | one, 2 KV heads, 16 blocks: 6000 tokens 39.1 | 38.0, 10 000 71.6 | 66.5, 777 + 5003 + 1291 + 9173 92.2 | 83.1, 5000 x 4 80.6 |
+    // 77.5, 8000 x 3 115.8 | 115.9; 12 000 x 4 300 | 317, 16 000 129 | 130.5, 24 000 251.5 | 264.5; groups of 8: 8192 42.1 | 37.9, 20 000 138.6 | 126.8, 24 000 171.5 | 166.2.
     // Workgroups whose rows take every block return at once and do not count (selecting prefill of 5000 tokens, 64 blocks, 22.9 | 19.8, of 8192 with one KV head 26.2 | 23.8).
-    constexpr int64_t kOneTokenWorkgroups = 384;
+    constexpr int64_t kOneTokenWorkgroups = 384, kOneTokenLength = 10240;
     const int64_t scored = p.mask ? static_cast<int64_t>(max_seqlen_q) - static_cast<int64_t>(kBlockN) * p.topk : max_seqlen_q;
-    const bool one = (scored + kTokPerBlock * pack - 1) / (kTokPerBlock * pack) * batch * num_heads_k <= kOneTokenWorkgroups;
+    const bool one = (p.mask && (pack == 2 || max_seqlen_q <= kOneTokenLength)) ||
+                     (scored + kTokPerBlock * pack - 1) / (kTokPerBlock * pack) * batch * num_heads_k <= kOneTokenWorkgroups;
     const int tokens = (one ? kWavesS1 : kTokPerBlock) * pack;
     const dim3 grid((max_seqlen_q + tokens - 1) / tokens * p.splits, batch, num_heads_k);
     hipStream_t st = static_cast<hipStream_t>(stream);
     auto pick = [&](auto tok, auto packed) {
         constexpr int kTok = decltype(tok)::value, kPack = decltype(packed)::value;
-        if (p.mask) return p.pool_len <= 64 ? stage1_kernel<true, true, 1, false, kTok, kPack> : p.pool_len <= 128 ? stage1_kernel<true, true, 2, false, kTok, kPack>
-                         : p.pool_len <= 256 ? stage1_kernel<true, true, 4, false, kTok, kPack> : stage1_kernel<true, true, 8, false, kTok, kPack>;
+        if constexpr (kTok == 1 || kPack == 1) {               // selecting, two tokens that share their rows are all a wavefront takes
+            if (p.mask) return p.pool_len <= 64 ? stage1_kernel<true, true, 1, false, kTok, kPack> : p.pool_len <= 128 ? stage1_kernel<true, true, 2, false, kTok, kPack>
+                             : p.pool_len <= 256 ? stage1_kernel<true, true, 4, false, kTok, kPack> : stage1_kernel<true, true, 8, false, kTok, kPack>;
+        }
         const bool shared = p.splits > 1;
         return pool ? (is_causal ? (shared ? stage1_kernel<true, true, 0, true, kTok, kPack> : stage1_kernel<true, true, 0, false, kTok, kPack>)
                                  : (shared ? stage1_kernel<false, true, 0, true, kTok, kPack> : stage1_kernel<false, true, 0, false, kTok, kPack>))
