@@ -41,6 +41,7 @@ constexpr int kWaveTiles = 2;                                  // 16-key tiles p
 
 typedef short short4v __attribute__((ext_vector_type(4)));
 typedef int int4v __attribute__((ext_vector_type(4)));
+typedef uint32_t __attribute__((may_alias)) two_entries;      // of the list of tokens, written one by one
 
 __device__ __forceinline__ uint32_t lds_addr(const void* ptr) {
     return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)ptr));
@@ -276,7 +277,7 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
     uint32_t ahead[kPack];                                     // the entries of the step after the next one asked for
     auto read_ahead = [&](int from) {
 #pragma unroll
-        for (int i = 0; i < kPack; ++i) ahead[i] = reinterpret_cast<const uint32_t*>(list + from)[i];
+        for (int i = 0; i < kPack; ++i) ahead[i] = reinterpret_cast<const two_entries*>(list + from)[i];
     };
     auto next_step = [&]() {
         Step step;
