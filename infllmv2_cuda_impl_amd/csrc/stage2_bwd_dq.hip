@@ -237,7 +237,10 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
 #pragma unroll
     for (int f = 0; f < 16; ++f) asm volatile("" : "+v"(kreg[f]));
     asm volatile("" : "+v"(lse2));
-    float dsum = 0.f;
+    bool mine0 = false;
+    int j0 = next_common(mine0);
+    if (j0 >= 0) issue(j0, 0);
+    float dsum = 0.f;                                          // formed while the first ring block is on its way (kernel of 3941 tokens 138 -> 136 us)
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
@@ -248,9 +251,6 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
         dsum = 0.f;
     }
     const floatx4 neg_dsum = {-dsum, -dsum, -dsum, -dsum};     // the dP accumulators start here: dS = P (dP - D) is then one product
-    bool mine0 = false;
-    int j0 = next_common(mine0);
-    if (j0 >= 0) issue(j0, 0);
     int tile = 0;
     bool k_ahead = false;                                      // the coming own block's 16 K-fragment loads were issued last turn
     auto own_part = [&]() {
