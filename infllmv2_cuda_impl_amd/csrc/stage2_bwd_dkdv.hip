@@ -233,7 +233,7 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
         // The item's tokens as a list, so that a step takes the next ones wherever they lie and learns them from one read, made a step ahead.  Walking the
         // words' bits with scalar instructions between the wait for a step's rows and the request for the next ones, and ending a pair at the end of a word: us with
         // the walk | the list, whole kernel, 71 552 packed tokens (64 blocks) 8250 | 8100, 6741 in four sequences (16 blocks) 240 | 230.
-        // Both wavefronts write the same list, each for itself: a lane to a token of a word.  What the last step has no tokens for repeats the last.
+        // The first wavefront writes it, a lane to a token of a word; both count, and read it behind a barrier.  What the last step has no tokens for repeats the last.
         uint64_t words = __ballot(lane < kGroupWords && wv != 0ull);
         int last = 0;
         while (words != 0ull) {
@@ -241,12 +241,12 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
             words &= words - 1ull;
             const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(wv), w), hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(wv >> 32), w);
             const uint64_t v = (static_cast<uint64_t>(hi) << 32) | lo;
-            if ((v >> lane) & 1ull) list[tokens + __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0))] = static_cast<uint16_t>(w * 64 + lane);
+            if (wave == 0 && ((v >> lane) & 1ull)) list[tokens + __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0))] = static_cast<uint16_t>(w * 64 + lane);
             tokens += __builtin_popcountll(v);
             last = w * 64 + 63 - __builtin_clzll(v);
         }
         if (tokens == 0) return;                               // uniform
-        if (lane < 2 * kPack) list[tokens + lane] = static_cast<uint16_t>(last);
+        if (wave == 0 && lane < 2 * kPack) list[tokens + lane] = static_cast<uint16_t>(last);
     }
 
     // ---- K and V of the block: B operands, resident in registers ----
@@ -359,6 +359,7 @@ void bwd_dkdv_wave_kernel(const BwdParams p) {
     // operand fragment (head n, piece g) of a chunk: unit 4 n + (g - n / 4) % 4
     const int frag_unit = 4 * n + ((g - (n >> 2)) & 3);
 
+    __syncthreads();                                           // the list, which other lanes and the other wavefront wrote
     read_ahead(0);
     Step now = next_step();
     read_ahead(2 * kPack);
