@@ -96,44 +96,6 @@ __device__ __forceinline__ int own_beside(const unsigned long long* row, const u
     return over > kOwnBeside ? 1 << 30 : over;
 }
 
-// The order of the token groups of a launch of the row-parallel kernels, which take it from the end: one (head, sequence) after the other, its longest prefixes first; or, in
-// launches of up to 4096 groups (16 to a CU), one sequence after the other and in it 16 groups of a head, the same ones of the next head, and so on, so that the longest
-// prefixes of all heads come first and the shortest last.  Head by head the second head's longest groups were begun half-way.  Forward with the images in us, head by head | by turns: 1000 tokens,
-// 4 KV heads, 47.0 | 36.8, 2048, 4 heads, 16 blocks, 98.4 | 87.2, 2 heads 52.3 | 51.5, 4096, 2 heads 182 | 170, 8192 510 | 502, 1500 queries behind 18 511 keys 197 | 185; whole pass of 32 768, 8192 groups,
-// 3275 | 3314, training on 71 552 packed tokens 23.1 | 23.2 ms.
-struct GroupOrder {
-    int batch, heads, groups, chunk_log2;                      // groups: of the longest sequence and a head; chunk_log2 < 0: head by head
-    int64_t per_seq;                                           // by turns, the places of a sequence: heads x its groups rounded up to whole chunks
-    int64_t places() const { return batch * per_seq; }
-};
-constexpr int64_t kGroupsByTurns = 4096;
-inline GroupOrder group_order(int batch, int heads, int groups) {
-    if (static_cast<int64_t>(batch) * heads * groups > kGroupsByTurns) return {batch, heads, groups, -1, static_cast<int64_t>(heads) * groups};
-    int log2 = 0;
-    while (log2 < 4 && (1 << log2) < groups) ++log2;
-    return {batch, heads, groups, log2, static_cast<int64_t>(heads) * (((groups + (1 << log2) - 1) >> log2) << log2)};
-}
-// The group at a place; false: nobody's.
-__device__ __forceinline__ bool group_at(const GroupOrder& o, int at, int& grp, int& h, int& b) {
-    if (o.chunk_log2 < 0) {                                    // uniform
-        const int hb = at / o.groups;
-        grp = at - hb * o.groups;
-        h = hb / o.batch;
-        b = hb - h * o.batch;
-        return true;
-    }
-    b = 0;
-    if (o.batch > 1) {
-        const int per_seq = static_cast<int>(o.per_seq);
-        b = at / per_seq;
-        at -= b * per_seq;
-    }
-    const int chunk = at >> o.chunk_log2, level = chunk / o.heads;
-    h = chunk - level * o.heads;
-    grp = (level << o.chunk_log2) + (at & ((1 << o.chunk_log2) - 1));
-    return grp < o.groups;
-}
-
 // Cross-row exchanges with gfx950's v_permlane16_swap / v_permlane32_swap (VALU speed; a ds_bpermute takes a trip
 // through the LDS crossbar): swapping a register with itself hands every lane its own row's value and the partner
 // row's value.

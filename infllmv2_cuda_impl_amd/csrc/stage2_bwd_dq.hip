@@ -26,13 +26,13 @@
 #include "common.h"
 #include "kv_image.h"
 #include "block_walker.h"
+#include "group_order.h"
 #include "stage2_bwd.h"
 #include <math.h>
 
 namespace IV2_NS {
 
 constexpr int kDqTokens = 8;
-constexpr int kDqChunk = 16;                                   // token groups per XCD chunk
 constexpr int kDqTileBytes = 32768;
 constexpr int kDqMaskWords = 256;                              // LDS copies of the mask rows hold at most this many words each: 16384 key blocks
 constexpr int kDqLdsTiles = 2 * kDqTileBytes + 8 * 8192;       // 2-tile ring + 8 private half K tiles
@@ -110,7 +110,7 @@ void bwd_dq_hybrid_kernel(const BwdParams p, const DqExtra x) {
 
     const int bid = blockIdx.x;
     const int xcd = bid & 7, sidx = bid >> 3;
-    int G = ((sidx / kDqChunk) * 8 + xcd) * kDqChunk + (sidx % kDqChunk);
+    const int G = place_from_end(x.order, xcd, sidx);
     if (G >= x.total_groups) return;                                                // uniform per workgroup
     int grp, h, b;
     if (!group_at(x.order, x.total_groups - 1 - G, grp, h, b)) return;              // uniform per workgroup
@@ -390,7 +390,7 @@ int launch_bwd_dq_hybrid(hipStream_t st, const BwdParams& p, int batch, int max_
     x.order = group_order(batch, p.num_heads_k, (max_seqlen_q + kDqTokens - 1) / kDqTokens);
     const int64_t of_sequence = x.order.per_seq, total = x.order.places();
     IV2_CHECK(p.k_blocks <= kDqMaskWords * 64, "varlen_bwd: more than %d key blocks per sequence", kDqMaskWords * 64);
-    const int64_t most = max_workgroups(512) - 8 * kDqChunk;
+    const int64_t most = max_workgroups(512) - 8 * kLargestShare;
     if (total > most) {                                        // some sequences at a time, as in the forward
         const int fit = static_cast<int>(most / of_sequence);
         IV2_CHECK(fit > 0, "varlen_bwd: too many token groups");
@@ -406,7 +406,7 @@ int launch_bwd_dq_hybrid(hipStream_t st, const BwdParams& p, int batch, int max_
     }
     x.total_groups = static_cast<int>(total);
     x.mask_words = (p.k_blocks + 63) / 64 > 0 ? (p.k_blocks + 63) / 64 : 1;
-    const int64_t per_round = 8 * kDqChunk;
+    const int64_t per_round = 8 << x.order.share_log2;
     const int64_t grid = (total + per_round - 1) / per_round * per_round;
     const size_t lds = kDqLdsTiles + static_cast<size_t>(1 + kDqTokens) * x.mask_words * 8;
     const void* fn = causal ? reinterpret_cast<const void*>(&bwd_dq_hybrid_kernel<true>)

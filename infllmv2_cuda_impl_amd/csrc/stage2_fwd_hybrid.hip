@@ -25,13 +25,14 @@
 // 512 MFMA cycles); the shared walk takes the common half of the work off that path.  Online
 // softmax is order-independent, so the split changes nothing in the result.
 //
-// Workgroups are numbered so that each of the 8 XCDs takes whole chunks of consecutive token
+// Workgroups are numbered so that each of the 8 XCDs takes shares of consecutive token
 // groups of one KV head (their L2 sees one head's images and neighbouring local windows), and
-// the longest causal prefixes are scheduled first (GroupOrder in block_walker.h).
+// the longest causal prefixes are scheduled first (group_order.h).
 // Long sequences are walked in step with the other workgroups of the XCD, at a given pace (in_step.h).
 #include "common.h"
 #include "kv_image.h"
 #include "block_walker.h"
+#include "group_order.h"
 #include "lds_dma.h"
 #include "in_step.h"
 #include "stage2_fwd.h"
@@ -41,7 +42,6 @@
 namespace IV2_NS {
 
 constexpr int kHybTokens = 8;                                  // tokens (= wavefronts) per workgroup
-constexpr int kHybChunk = 16;                                  // token groups per XCD chunk
 constexpr int kRingTiles = 4;
 constexpr int kTileBytes = 32768;                              // K image | V image of one block
 constexpr int kMaxMaskWords = 256;                             // LDS copies of the mask rows hold at most this many words each: 16384 key blocks
@@ -135,11 +135,11 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
     unsigned long long* com = reinterpret_cast<unsigned long long*>(smem_raw + kRingTiles * kTileBytes);   // [mask_words]
     unsigned long long* rows = com + x.mask_words;                                  // [kHybTokens][mask_words]
 
-    // ---- which tokens: XCD-chunked, heaviest first (x.late: but the last group of every sequence at the end) ----
+    // ---- which tokens: in the XCDs' shares, heaviest first (x.late: but the last group of every sequence at the end) ----
     const int bid = blockIdx.x;
     // (few groups are few chunks: two parts to an XCD fill its CUs, the next two go to another)
     const int xcd = (kParts <= 2 ? bid : bid - 16 / kParts * (static_cast<int>(blockIdx.y) >> 1)) & 7, sidx = bid >> 3;
-    int G = ((sidx / kHybChunk) * 8 + xcd) * kHybChunk + (sidx % kHybChunk);
+    const int G = place_from_end(x.order, xcd, sidx);
     if (G >= x.total_groups) return;                                                // uniform per workgroup
     int grp, h, b;
     bool there = true;
@@ -461,10 +461,12 @@ void stage2_fwd_hybrid_kernel(const FwdParams p, const HybridExtra x) {
 static int launch_groups(hipStream_t st, const FwdParams& p, int batch, int num_heads_k, int max_seqlen_q, int max_seqlen_k, bool causal, int most_selected, unsigned* in_step) {
     HybridExtra x{};
     x.groups_per_seq = (max_seqlen_q + kHybTokens - 1) / kHybTokens;
-    x.order = group_order(batch, num_heads_k, x.groups_per_seq);
-    const int64_t of_sequence = x.order.per_seq, groups = static_cast<int64_t>(num_heads_k) * x.groups_per_seq * batch;
+    const int64_t groups = static_cast<int64_t>(num_heads_k) * x.groups_per_seq * batch;
+    const int parts = groups * 2 > 256 ? 1 : groups * 4 > 256 ? 2 : groups * 8 > 256 ? 4 : 8;
+    x.order = group_order(batch, num_heads_k, x.groups_per_seq, parts > 1);
+    const int64_t of_sequence = x.order.per_seq;
     int64_t total = x.order.places();
-    const int64_t most = max_workgroups(512) - 8 * kHybChunk;
+    const int64_t most = max_workgroups(512) - 8 * kLargestShare;
     if (total > most) {                                        // more than a dispatch holds (thousands of sequences beside a long one): some sequences at a time
         const int fit = static_cast<int>(most / of_sequence);
         IV2_CHECK(fit > 0, "varlen_fwd: too many token groups");
@@ -490,7 +492,6 @@ static int launch_groups(hipStream_t st, const FwdParams& p, int batch, int num_
     // and gain nothing: 700 tokens behind 20011, 176 groups, take 102 whole.
     // So few groups run all at once: they neither count nor wait (in_step.h).  They keep the pace: it gives the order in which a row's blocks are added up, which must not
     // depend on the number of parts.
-    const int parts = groups * 2 > 256 ? 1 : groups * 4 > 256 ? 2 : groups * 8 > 256 ? 4 : 8;
     x.finished = parts > 1 ? nullptr : in_step;
     // Heaviest first is also longest prefix first, which puts the one short group of a chunk of queries in front.  Where the chunk's groups are alike, with at least twice as many
     // blocks behind the first of them as a row selects, it holds up a CU that then has as many whole groups to walk as the others, and goes last instead.  Forward with the images in us, first | last, 2 KV heads, 2049
@@ -505,7 +506,7 @@ static int launch_groups(hipStream_t st, const FwdParams& p, int batch, int num_
         total = x.order.places() + x.late;
     }
     x.total_groups = static_cast<int>(total);
-    const int64_t per_round = 8 * kHybChunk;
+    const int64_t per_round = 8 << x.order.share_log2;
     const int64_t grid = (total + per_round - 1) / per_round * per_round;
     auto pick = [&](auto n) {
         constexpr int kParts = decltype(n)::value;
