@@ -831,6 +831,7 @@ std::tuple<Tensor, Tensor> decode_sparse(const Tensor& q, const Tensor& kn, cons
     TORCH_CHECK(topk > 0, "decode_sparse: topk must be positive");
     require_gpu(q, "q");
     TORCH_CHECK(q.dim() == 4 && kc.dim() == 4, "q, k_cache, v_cache must have 4 dimensions");
+    check_step(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, kernel_size, stride, block_size, true);
     DeviceGuard guard(q.device());
     const int64_t batch = q.size(0), hq = q.size(2), hk = kc.size(2);
     const int splits = decode_splits(batch, hk, topk);
@@ -838,7 +839,6 @@ std::tuple<Tensor, Tensor> decode_sparse(const Tensor& q, const Tensor& kn, cons
     const bool all = blocks <= topk;                           // nothing to select: no scores
     if (batch * hk * splits > 256 || max_len > INFLLMV2_DECODE_MAX_SCORES * kBlock) {
         if (all && topk <= INFLLMV2_DECODE_MAX_SCORES) {
-            check_step(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, kernel_size, stride, block_size, true);
             const Tensor new_lens = std::get<0>(decode_front(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, max_len, kernel_size,
                                                              stride, block_size, false, local_blocks, init_blocks, scale));
             return {std::get<0>(fwd_kvcache(q, kc, vc, std::nullopt, std::nullopt, new_lens, scale, 0, std::nullopt, std::nullopt, std::nullopt, std::nullopt,
@@ -849,7 +849,6 @@ std::tuple<Tensor, Tensor> decode_sparse(const Tensor& q, const Tensor& kn, cons
         return {std::get<0>(fwd_kvcache(q, kc, vc, std::nullopt, std::nullopt, new_lens, scale, 0, std::nullopt, mask, std::nullopt, std::nullopt,
                                         std::nullopt, std::nullopt, std::nullopt, false)), new_lens};
     }
-    check_step(q, kn, vn, kc, vc, fine, coarse, lens, host_len, fine_lens, coarse_lens, kernel_size, stride, block_size, true);
     // What lives inside the step shares one allocation, and lengths that the host has get no tensor of their own: a step that the device finishes in 19 to 20 us was
     // bound by the host that issues it (one sequence, seven allocations 22.6 us to issue, two 19.6; six sequences 19.2 and 17.3).
     Tensor new_lens, out = at::empty_like(q);

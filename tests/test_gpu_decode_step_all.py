@@ -32,3 +32,16 @@ def test_step_equals_the_separate_operators(dtype, Hk, G, lens, topk):
                                      32, 16, 64, topk, 2, 1, 128 ** -0.5)
     for a, b in ((got, want), (k, k2), (v, v2), (fine, f2), (coarse, c2)) + (() if one else ((n, n2), (fl, fl2), (cl, cl2))):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("block_size", [0, 32, 128])
+@pytest.mark.parametrize("lens", [[100], [100, 5000]])
+def test_other_block_sizes_are_refused(block_size, lens):
+    """Before anything is divided by them."""
+    import infllmv2_cuda_impl_amd as ops
+    layer, cap, B = ops.InfLLMv2Attention(topk=16, block_size=block_size), 8192, len(lens)
+    rand = lambda *s: torch.randn(*s, device="cuda").to(torch.bfloat16)
+    cache = ops.BatchCache.empty(B, cap, 2, 128, "cuda")
+    layer.fill_cache(cache, rand(sum(lens), 2, 128), rand(sum(lens), 2, 128), lens)
+    with pytest.raises(RuntimeError, match="only 64-token blocks"):
+        layer.decode_batch(rand(B, 1, 32, 128), rand(B, 1, 2, 128), rand(B, 1, 2, 128), cache)
