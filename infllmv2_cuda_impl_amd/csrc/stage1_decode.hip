@@ -635,14 +635,9 @@ void stage1_decode_whole_kernel(const S1DecodeParams p, const Step t) {
             *reinterpret_cast<floatx4*>(records + r * 32 + 16 + 4 * g) = floatx4{ll[0], ll[1], ll[2], ll[3]};
         }
     };
-    for (int r = wave; r < tiles_c; r += 2 * kWholeWaves) {
-        record(ca, r);
-        if (r + 2 * kWholeWaves < tiles_c) s1d_load_tile(ca, sq.cbase, p.c_row_stride, (r + 2 * kWholeWaves) * 64, sq.Lc, n, g);
-        if (r + kWholeWaves < tiles_c) {
-            record(cb, r + kWholeWaves);
-            if (r + 3 * kWholeWaves < tiles_c) s1d_load_tile(cb, sq.cbase, p.c_row_stride, (r + 3 * kWholeWaves) * 64, sq.Lc, n, g);
-        }
-    }
+    static_assert(kWholeRecords <= 2 * kWholeWaves, "two coarse tiles to a wavefront");
+    if (wave < tiles_c) record(ca, wave);
+    if (wave + kWholeWaves < tiles_c) record(cb, wave + kWholeWaves);
     // S of the 16 keys, before the wait for the other records
     auto products = [&](const elem8 (&t4)[4]) {
         floatx4 s = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -706,7 +701,7 @@ void s1d_splits(int batch, int num_heads_k, int max_keys, int max_coarse, int& s
     plan((max_keys + 63) / 64, splits_f, run_f);
     plan((max_coarse + 63) / 64, splits_c, run_c);
 }
-// One launch (stage1_decode_whole_kernel) instead of two: up to five coarse tiles, i.e. 20 543 tokens, and a workgroup per CU.  Every workgroup loads all coarse
+// One launch (stage1_decode_whole_kernel) instead of two: up to five coarse tiles, i.e. 20 607 tokens, and a workgroup per CU.  Every workgroup loads all coarse
 // tiles, 16 KiB each, through its CU's vector memory path and forms their records; that costs 0.4 us a tile, and the launch it saves is worth 1.5 us of the device
 // and 2.5 us of the host that issues it.  A decode step in us, two launches | one: one sequence of 1000 tokens 17.5 | 14.8, 4000 17.6 | 15.1, 8000 17.9 | 15.9, 16 000
 // 18.0 | 16.9, 20 000 18.0 | 18.1, 24 000 18.1 | 18.6, 32 000 18.0 | 19.4; two of up to 8000 17.5 | 15.6, six of up to 20 000 19.2 | 18.1, eight of up to 8000 19.7 | 17.9,

@@ -6,8 +6,8 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# coarse tiles begin at 128 + 64 * 64 k tokens, fine ones at 32 + 16 * 64 k; the rule's five coarse tiles end at 20 543
-LENS = [1, 31, 32, 127, 128, 1039, 1040, 1055, 1056, 1057, 4159, 4160, 4223, 4224, 4287, 8192, 16447, 16448, 20479, 20542]
+# coarse tiles begin at 128 + 64 * 64 k tokens, fine ones at 32 + 16 * 64 k; the rule's five coarse tiles are full from 20 544 to 20 607
+LENS = [1, 31, 32, 127, 128, 1039, 1040, 1055, 1056, 1057, 4159, 4160, 4223, 4224, 4287, 8192, 16447, 16448, 20479, 20542, 20543, 20606, 20607]
 COPIES = 16
 
 
