@@ -652,11 +652,13 @@ int launch_stage1(const char* who, void* stream, const void* q, const void* k, c
             if (p.mask) return p.pool_len <= 64 ? stage1_kernel<true, true, 1, false, kTok, kPack> : p.pool_len <= 128 ? stage1_kernel<true, true, 2, false, kTok, kPack>
                              : p.pool_len <= 256 ? stage1_kernel<true, true, 4, false, kTok, kPack> : stage1_kernel<true, true, 8, false, kTok, kPack>;
         }
-        const bool shared = p.splits > 1;
-        return pool ? (is_causal ? (shared ? stage1_kernel<true, true, 0, true, kTok, kPack> : stage1_kernel<true, true, 0, false, kTok, kPack>)
-                                 : (shared ? stage1_kernel<false, true, 0, true, kTok, kPack> : stage1_kernel<false, true, 0, false, kTok, kPack>))
-                    : (is_causal ? (shared ? stage1_kernel<true, false, 0, true, kTok, kPack> : stage1_kernel<true, false, 0, false, kTok, kPack>)
-                                 : (shared ? stage1_kernel<false, false, 0, true, kTok, kPack> : stage1_kernel<false, false, 0, false, kTok, kPack>));
+        static_assert(kOneTokenWorkgroups >= 128, "launches that share tokens have at most so many workgroups");
+        if constexpr (kTok == 1) {
+            if (p.splits > 1) return pool ? (is_causal ? stage1_kernel<true, true, 0, true, kTok, kPack> : stage1_kernel<false, true, 0, true, kTok, kPack>)
+                                          : (is_causal ? stage1_kernel<true, false, 0, true, kTok, kPack> : stage1_kernel<false, false, 0, true, kTok, kPack>);
+        }
+        return pool ? (is_causal ? stage1_kernel<true, true, 0, false, kTok, kPack> : stage1_kernel<false, true, 0, false, kTok, kPack>)
+                    : (is_causal ? stage1_kernel<true, false, 0, false, kTok, kPack> : stage1_kernel<false, false, 0, false, kTok, kPack>);
     };
     constexpr std::integral_constant<int, 1> k1{};
     constexpr std::integral_constant<int, 2> k2{};
