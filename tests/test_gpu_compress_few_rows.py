@@ -18,9 +18,10 @@ def cu(*lens):
     return torch.tensor([sum(lens[:i]) for i in range(len(lens) + 1)], dtype=torch.int32, device="cuda")
 
 
-# 32 768 and 32 800 tokens of two heads: the last halved launch of either set alone and the first that is not; 10 300: of the pair
+# two heads: 32 799 | 32 800 tokens are the last halved launch of 32 keys every 16 alone and the first that is not, 32 895 | 32 896 of 128 every 64, 10 271 | 10 272 of the pair
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("n,heads,dim", [(127, 2, 128), (128, 2, 128), (257, 1, 64), (1000, 3, 136), (2048, 2, 128), (10300, 2, 128), (32800, 2, 128)])
+@pytest.mark.parametrize("n,heads,dim", [(127, 2, 128), (128, 2, 128), (257, 1, 64), (1000, 3, 136), (2048, 2, 128), (10271, 2, 128), (10272, 2, 128), (10300, 2, 128), (32799, 2, 128), (32800, 2, 128), (32895, 2, 128),
+                                         (32896, 2, 128)])
 @pytest.mark.parametrize("window", [(32, 16), (128, 64), (192, 192), (200, 7), (96, 96), (3, 2)])
 def test_rows_of_short_launches(n, heads, dim, window, dtype):
     size, stride = window

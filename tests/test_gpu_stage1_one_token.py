@@ -1,6 +1,7 @@
-"""Stage 1 in launches of few workgroups, whose wavefronts take one token each (two in groups of 8 heads and fewer): scores, pooled scores and mask words are,
+"""Stage 1 in launches of few workgroups, whose wavefronts take one token each (two in groups of 8 heads and fewer): scores and pooled scores are,
 bit for bit, those of the same sequences among so many copies that the launch takes twice as many tokens to a wavefront.  Lengths around the 8, 16 and
-32 tokens of a workgroup, the 64 keys of a tile and the row lengths of the selection."""
+32 tokens of a workgroup and the 64 keys of a tile.  The mask words, too, are the same among copies; how many tokens a selecting wavefront takes depends on the
+longest sequence alone (test_gpu_stage1_selecting_forms.py)."""
 import numpy as np
 import pytest
 import torch

@@ -1,6 +1,6 @@
 """Rows that take as many blocks as they can score: the selecting Stage 1 forms no scores for them, and its mask words are still those of Stage 1, pooling
 and top-k one after the other, on either side of the line, with forced blocks behind a row's last one, windows wider than
-the selection, scores that are all equal or zero, and one or two tokens to a wavefront."""
+the selection, scores that are all equal or zero, and one token to a wavefront or, beyond 10 240, two."""
 import numpy as np
 import pytest
 import torch
@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("lens, hk", [([2], 1), ([30, 33, 65], 1), ([1023], 1), ([1040, 0, 1025], 2), ([4097], 1), ([4096, 2100, 700], 4)])
+@pytest.mark.parametrize("lens, hk", [([2], 1), ([30, 33, 65], 1), ([1023], 1), ([1040, 0, 1025], 2), ([4097], 1), ([4096, 2100, 700], 4), ([10300, 1100], 1)])
 def test_same_words_as_with_scores(lens, hk, dtype):
     import infllmv2_cuda_impl_amd as ops
     from infllmv2_cuda_impl_amd import _lib

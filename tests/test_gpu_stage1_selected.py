@@ -32,8 +32,9 @@ def test_same_words_as_apart(lens, dtype):
     both(q * 30, k, v, lens, 8, 1, 1)                              # nearly all of them zero
 
 
-@pytest.mark.parametrize("group", [1, 2, 4, 8])
-def test_groups(group):
+@pytest.mark.parametrize("group, lens, hk", [(1, [700, 4300], 3), (2, [700, 4300], 3), (4, [700, 4300], 3), (8, [700, 4300], 3), (8, [16384], 1), (8, [16385], 1), (8, [32768], 1),
+                                             (2, [16385, 300], 1), (4, [32768], 1)])
+def test_groups(group, lens, hk):
     gen = torch.Generator(device="cuda").manual_seed(group)
-    r = lambda heads: torch.randn(5000, heads, 128, generator=gen, device="cuda").to(torch.bfloat16)
-    both(r(3 * group), r(3), r(3), [700, 4300], 12, 3, 1)
+    r = lambda heads: torch.randn(sum(lens), heads, 128, generator=gen, device="cuda").to(torch.bfloat16)
+    both(r(hk * group), r(hk), r(hk), lens, 12, 3, 1)
