@@ -82,13 +82,15 @@ __device__ __forceinline__ uint64_t walked_together(const unsigned long long* wo
     return eights | (fours & (twos | ones));
 }
 
-// How many of the ring's blocks that a row selects have one of its own walked beside them (beside those it does not select there always is one).  A row that has its
-// own blocks beside every ring block until they run out waits, from then on, at ring blocks that are not its own; with so many fewer beside the others it has one for each
-// of those.  That is its blocks less the ring's: negative, none, with few blocks to choose from.  Rows with more than kOwnBeside over take one every time: their own blocks outnumber the ring's that are not theirs, and
-// balanced all the same four packed sequences (71 552 tokens) took 5740 | 7450 us instead of 5625 | 7320, forward and dQ.  Whole passes, every time | balanced: 2048 tokens with 16 blocks
-// 65.0 -> 63.5 us, four ragged prompts 931 -> 922, training on four short samples 588 -> 585; 32 768 tokens and chunks as before.  Two beside a ring block that is not the
-// row's, too, as long as there are enough: 64.1, 942, 584, and 32 768 tokens 3164 -> 3212.  Two over instead of kOwnBeside: forward of 9934 + 3083 tokens, 32 blocks, 591 -> 599 us, of 11 878 + 8202, 64 blocks,
-// 706 -> 711, of 49 other inputs within 1 % on average.  A rule on the group's rows alone, which gives the order in which they are added up.
+// How many of the ring's blocks that a row selects have one of its own walked beside them (beside those it does not select there always is one).
+// A row that has its own blocks beside every ring block until they run out waits, from then on, at ring blocks that are not its own; with so many fewer beside the
+// others it has one for each of those.  That is its blocks less the ring's: negative, none, with few blocks to choose from.  Rows with more than kOwnBeside over take
+// one every time: their own blocks outnumber the ring's that are not theirs.  A rule on the group's rows alone, which gives the order in which they are added up.
+//   all balanced: four packed sequences (71 552 tokens), forward and dQ, 5625 | 7320 -> 5740 | 7450 us
+//   whole passes, every time -> balanced: 2048 tokens with 16 blocks 65.0 -> 63.5, four ragged prompts 931 -> 922, training on four short samples 588 -> 585;
+//   32 768 tokens and chunks as before
+//   two over instead of kOwnBeside: forward of 9934 + 3083 tokens, 32 blocks, 591 -> 599, of 11 878 + 8202, 64 blocks, 706 -> 711, of 49 other inputs within 1 % on average
+//   two beside a ring block that is not the row's, too, as long as there are enough: 64.1, 942, 584, and 32 768 tokens 3164 -> 3212
 constexpr int kOwnBeside = 8;
 __device__ __forceinline__ int own_beside(const unsigned long long* row, const unsigned long long* together, int words, int lane) {
     int over = 0;

@@ -625,20 +625,25 @@ int launch_stage1(const char* who, void* stream, const void* q, const void* k, c
     // give each CU a workgroup, with four tiles each at least.  Kernel alone, us, 2 KV heads, 20 011 keys: 16 queries 34.8 -> 19.3, 256 35.4 -> 20.1, 512 34.8 -> 21.2, 700 35.2 ->
     // 25.6, 1024 35.5 -> 27.2; 60 000 keys, one KV head, 300 queries 90.4 -> 36.1; a whole chunk of 512 queries behind 19 499 keys 154.7 -> 139.9.  Two workgroups to a
     // CU: 700 queries 31.0, 1500 36.1 -> 39.5; two tiles each at least: 256 queries 26.7.
-    // Groups of 8 heads and fewer: two tokens share the 16 rows of a product, of which half were spare.  us, groups of 8, 2 KV heads, one | two tokens: scores of 256 queries against 20 011
-    // keys 13.6 | 13.6, 2049 51.1 | 36.5, 8000 92 | 63; selecting prefill of 2048 tokens 15.7 | 15.0, 32 768 391 | 257; scores of 65 536, one KV head, with the top-k launch 733 | 453.
+    // Groups of 8 heads and fewer: two tokens share the 16 rows of a product, of which half were spare.  us, groups of 8, 2 KV heads, one | two tokens:
+    //   scores of 256 queries against 20 011 keys 13.6 | 13.6, 2049 51.1 | 36.5, 8000 92 | 63; selecting prefill of 2048 tokens 15.7 | 15.0, 32 768 391 | 257;
+    //   scores of 65 536, one KV head, with the top-k launch 733 | 453.
     const int pack = p.group <= 8 ? 2 : 1;
     const int64_t wgs = static_cast<int64_t>((max_seqlen_q + kTokPerBlock * pack - 1) / (kTokPerBlock * pack)) * batch * num_heads_k;
     const int64_t fill = wgs > 0 ? 256 / wgs : 1, most = max_seqlen_k / 256;
     p.splits = p.mask != nullptr || fill < 2 || most < 2 ? 1 : static_cast<int>(fill < most ? fill : most);
-    // One token to a wavefront (two, where two share the rows), twice the workgroups, up to 384 of the others: three to a CU.  The time is then that of the CU with the most, half a
-    // workgroup finer, and of the chain of one tile (one wavefront's products and exponentials behind the other's on a SIMD), which is shorter.  Scores alone, us, two tokens | one, 2 KV heads, 20 011 keys:
-    // 17 queries 18.8 | 12.5, 256 19.3 | 13.3, 512 20.1 | 20.6, 1100 35.1 | 32.9, 2049 54.0 | 42.2, 3000 (376 workgroups) 56.1 | 49.4; 3100 (388) 55.3 | 58.8, 4096 60.0 | 63.6; 131 072
-    // keys, 2049 344 | 244, 3100 313 | 362; selecting prefill of 1000 tokens 15.2 | 12.4.  Whole sequences, whose workgroups walk from one tile to all: 1160 tokens, 4 KV heads, 13.6 | 11.0, 2185, 2 heads, 14.5 |
-    // 11.2, 3849, one head, 12.8 | 10.7, 487 + 1295 + 909, one head, 11.0 | 9.6.
-    // Selecting, a workgroup walks what its own tokens see, from one tile to all of them, and smaller ones end together: always where two tokens share the rows, else up to 10 240 tokens; longer, the
-    // keys' second trip from L2 costs more.  Selection in us, two tokens | one, 2 KV heads, 16 blocks: 6000 tokens 39.1 | 38.0, 10 000 71.6 | 66.5, 777 + 5003 + 1291 + 9173 92.2 | 83.1, 5000 x 4 80.6 |
-    // 77.5, 8000 x 3 115.8 | 115.9; 11 300 79.3 | 74.4, 12 000 82.6 | 77.5, 11 000 with 4 heads and 32 blocks 125 | 120, 11 300 + 11 800 + 11 000 + 10 000 249 | 244 (these four are left to two); 12 000 x 4 300 | 317, 16 000 129 | 130.5, 24 000 251.5 | 264.5; groups of 8: 8192 42.1 | 37.9, 20 000 138.6 | 126.8, 24 000 171.5 | 166.2.
+    // One token to a wavefront (two, where two share the rows), twice the workgroups, up to 384 of the others: three to a CU.  The time is then that of the CU with the
+    // most, half a workgroup finer, and of the chain of one tile (one wavefront's products and exponentials behind the other's on a SIMD), which is shorter.
+    // Scores alone, us, two tokens | one:
+    //   2 KV heads, 20 011 keys: 17 queries 18.8 | 12.5, 256 19.3 | 13.3, 512 20.1 | 20.6, 1100 35.1 | 32.9, 2049 54.0 | 42.2, 3000 (376 workgroups) 56.1 | 49.4;
+    //   3100 (388) 55.3 | 58.8, 4096 60.0 | 63.6; 131 072 keys: 2049 344 | 244, 3100 313 | 362; selecting prefill of 1000 tokens 15.2 | 12.4;
+    //   whole sequences, whose workgroups walk from one tile to all: 1160 tokens, 4 KV heads, 13.6 | 11.0, 2185, 2 heads, 14.5 | 11.2, 3849, one head, 12.8 | 10.7,
+    //   487 + 1295 + 909, one head, 11.0 | 9.6.
+    // Selecting, a workgroup walks what its own tokens see, from one tile to all of them, and smaller ones end together: always where two tokens share the rows, else up to
+    // 10 240 tokens; longer, the keys' second trip from L2 costs more.  Selection in us, two tokens | one, 2 KV heads, 16 blocks:
+    //   6000 tokens 39.1 | 38.0, 10 000 71.6 | 66.5, 777 + 5003 + 1291 + 9173 92.2 | 83.1, 5000 x 4 80.6 | 77.5, 8000 x 3 115.8 | 115.9;
+    //   left to two: 11 300 79.3 | 74.4, 12 000 82.6 | 77.5, 11 000 with 4 heads and 32 blocks 125 | 120, 11 300 + 11 800 + 11 000 + 10 000 249 | 244;
+    //   12 000 x 4 300 | 317, 16 000 129 | 130.5, 24 000 251.5 | 264.5; groups of 8: 8192 42.1 | 37.9, 20 000 138.6 | 126.8, 24 000 171.5 | 166.2.
     // Workgroups whose rows take every block return at once and do not count (selecting prefill of 5000 tokens, 64 blocks, 22.9 | 19.8, of 8192 with one KV head 26.2 | 23.8).
     constexpr int64_t kOneTokenWorkgroups = 384, kOneTokenLength = 10240;
     const int64_t scored = p.mask ? static_cast<int64_t>(max_seqlen_q) - static_cast<int64_t>(kBlockN) * p.topk : max_seqlen_q;

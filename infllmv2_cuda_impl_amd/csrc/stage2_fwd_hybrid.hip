@@ -493,11 +493,13 @@ static int launch_groups(hipStream_t st, const FwdParams& p, int batch, int num_
     // So few groups run all at once: they neither count nor wait (in_step.h).  They keep the pace: it gives the order in which a row's blocks are added up, which must not
     // depend on the number of parts.
     x.finished = parts > 1 ? nullptr : in_step;
-    // Heaviest first is also longest prefix first, which puts the one short group of a chunk of queries in front.  Where the chunk's groups are alike, with at least twice as many
-    // blocks behind the first of them as a row selects, it holds up a CU that then has as many whole groups to walk as the others, and goes last instead.  Forward with the images in us, first | last, 2 KV heads, 2049
-    // queries, 64 blocks: behind 8192 keys 215 | 208, 17 962 234 | 212 (2048 of them 197), 40 960 312 | 238; 32 blocks behind 4096 114 | 114, 12 288 133 | 121; 16 behind 2048 68.6 | 69.0, 10 240 81.2 | 78.0;
-    // 4097 queries, 64 blocks, behind 15 914 432 | 391.  Where the groups do not fill whole rounds, 1412 to 3500 queries, the same within 0.6 %.  With fewer blocks behind them last is slower: 64 blocks
-    // behind 4096 175 | 187, behind none 332 | 359 (6145 queries).
+    // Heaviest first is also longest prefix first, which puts the one short group of a chunk of queries in front.  Where the chunk's groups are alike, with at least
+    // twice as many blocks behind the first of them as a row selects, it holds up a CU that then has as many whole groups to walk as the others, and goes last instead.
+    // Forward with the images in us, first | last, 2 KV heads:
+    //   2049 queries, 64 blocks: behind 8192 keys 215 | 208, 17 962 234 | 212 (2048 of them 197), 40 960 312 | 238; 32 blocks behind 4096 114 | 114, 12 288 133 | 121;
+    //   16 behind 2048 68.6 | 69.0, 10 240 81.2 | 78.0; 4097 queries, 64 blocks, behind 15 914 432 | 391.
+    //   Where the groups do not fill whole rounds, 1412 to 3500 queries, the same within 0.6 %.
+    //   With fewer blocks behind them last is slower: 64 blocks behind 4096 175 | 187, behind none 332 | 359 (6145 queries).
     const int over = max_seqlen_q % kHybTokens;
     const int64_t held = static_cast<int64_t>(max_seqlen_k) - max_seqlen_q, selected = most_selected < 0 ? -static_cast<int64_t>(most_selected) : most_selected;
     if (parts == 1 && over > 0 && over <= 4 && x.groups_per_seq > 1 && selected > 0 && held >= 2 * kBlockN * selected) {
