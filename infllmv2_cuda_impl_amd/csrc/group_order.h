@@ -25,6 +25,8 @@ namespace IV2_NS {
 //   3849, 1, 64                                 83.8 | 82.6 |   72        984 + 3512 + 3164, 2, 64                    251 |  227 |  231
 //   8192, 2, 64                                  514 |  495 |  487        1839 + 584 + 1225, 2, 32                   82.9 | 68.9 | 73.2
 //   8191, 4, 64                                 1009 |  960 |  959        1288 + 1099 + 1098, 4 of 8 heads, 32        104 |  100 |  104
+//   1024, 4, 64                                 47.4 | 34.5 | 32.4        2048, 2, 64                                 59.7 | 52.7 | 46.1
+//   1038, 4, 64 (520 groups: a third round)     46.8 | 35.4 | 38.3        2100, 2, 64 (526)                           60.0 | 52.5 | 55.2
 //   701 queries behind three prompts, 1, 16     65.4 | 73.9 | 75.1        2435 + 1905, 4, 32                          192 |  203 |  196
 // Shares of 4 beyond kGroupsInFour cost L2 hits: 8191 tokens, 4, 16 420 | 441 with them, training on 1023 + 3001 + 517 + 2200, 2, 16, forward 151 | 156.
 // Shares of 16 there instead of 8: that training pass 564 us instead of 570, on 1739 + 1117 + 1273 + 1022 + 2282 606 instead of 579, on 2435 + 1905, 4, 32 897 instead of 885.
